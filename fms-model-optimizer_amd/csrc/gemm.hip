@@ -236,6 +236,12 @@ extern "C" int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspa
     *kernel = FMSMO_PLAN_GENERIC;
     return FMSMO_OK;
   }
+  if (cut_k_tall(M, N, K)) {
+    *kernel = FMSMO_PLAN_TILE_LDS_DMA;
+    *tile_m = TileTallK::BM;
+    *tile_n = TileTallK::BN;
+    return FMSMO_OK;
+  }
   const bool rs = K % 128 == 0 && use_register_staged(MMA_I8);
   const int bm[5] = {256, 128, 128, 256, 256}, bn[5] = {256, 256, 128, 192, 128};
   const int t = pick_tile((int)M, (int)N, rs);

@@ -36,9 +36,9 @@ int check_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const voi
   return FMSMO_OK;
 }
 
-// Tile shapes.  K is consumed in stages of BK bytes; a K that is not a multiple of BK is handled
-// by the caller-visible rule "K % 64 == 0" for the MFMA path (all transformer shapes), anything
-// else goes to the slow generic kernel.
+// Tile shapes.  K is consumed in stages of BK bytes; K that are no multiple of a stage run the KT
+// instances of the LDS-DMA kernel (a last stage that is cut at K), of three shapes: TileBig,
+// TileMidK, TileTallK.
 struct TileBig { static constexpr int BM = 256, BN = 256, BK = 64, NST = 4, WGM = 2, WGN = 2; };
 struct TileWide { static constexpr int BM = 128, BN = 256, BK = 64, NST = 4, WGM = 2, WGN = 2; };
 struct TileMid { static constexpr int BM = 128, BN = 128, BK = 64, NST = 4, WGM = 2, WGN = 2; };
@@ -104,7 +104,7 @@ int pick_tile(int M, int N, bool rs192_ok) {
   return best;
 }
 
-template <class Tile, int OP, bool GROUPED, class Epi>
+template <class Tile, int OP, bool GROUPED, bool KT = false, class Epi>
 void launch_tile(const GemmArgs& g0, const Epi& epi, hipStream_t st) {
   GemmArgs g = g0;
   g.grid_n = div_up(g.N, Tile::BN);
@@ -113,7 +113,7 @@ void launch_tile(const GemmArgs& g0, const Epi& epi, hipStream_t st) {
   dim3 grid((unsigned)(g.grid_m * g.grid_n)), block(Tile::WGM * Tile::WGN * 64);
   hipLaunchKernelGGL(
       (gemm_tile_kernel<Tile::BM, Tile::BN, Tile::BK, Tile::NST, Tile::WGM, Tile::WGN, OP, 1,
-                        GROUPED, Epi>),
+                        GROUPED, Epi, NoChunk, KT>),
       grid, block, 0, st, g, epi, NoChunk{});
 }
 
@@ -179,39 +179,28 @@ void launch_k128(const GemmArgs& g0, int batch, int M, const Epi& epi, hipStream
   hipLaunchKernelGGL((gemm_k128_kernel<OP, Epi>), dim3((unsigned)blocks), dim3(256), 0, st, g, epi);
 }
 
-// Generic fallback (any K % 16 == 0): one thread per output element, 4-byte dot products.
+// K % 128 != 0: the KT instances.  Up to a round of 128 x 64 tiles over the 256 compute units those
+// are taken, then 128 x 128 while they need at most twice the rounds of 256 x 256 tiles, those beyond
+// (us, int8, 128 x 64 / 128 x 128 / 256 x 256, the three tile counts in front):
+//   192 / 96 / 32 (300 x 4096 x 4016) 16.1 / 19.2 / 44.3      256 / 128 / 32 (2000 x 1024 x 4016) 21.5 / 22.8 / 60.4
+//   320 / 160 / 48 (600 x 4096 x 4016) 32.7 / 23.7 / 51.6     512 / 256 / 64 (1000 x 4096 x 4016) 40.0 / 28.5 / 59.3
+//   1024 / 512 / 128 (2000 x 4096 x 4016) 72.5 / 50.8 / 58.7  2048 / 1024 / 256 (2000 x 8192 x 4016) 137 / 95.6 / 72.4
+inline bool cut_k_tall(int64_t M, int64_t N, int64_t K) {
+  return K % 128 && (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN) <= 256;
+}
 template <int OP, class Epi>
-__global__ void gemm_simple_kernel(GemmArgs g, Epi epi) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  const int m = blockIdx.y;
-  if (n >= g.N) return;
-  const uint8_t* ar = g.a + (int64_t)m * g.lda;
-  const uint8_t* br = g.b + (int64_t)n * g.ldb;
-  typename Epi::Col c = epi.col(n, 0, g.N);
-  typename Epi::Row r = epi.row(m);
-  if constexpr (OP == MMA_I8) {
-    int acc = 0;
-    for (int k = 0; k < g.K; k += 4)
-      acc = __builtin_amdgcn_sdot4(*(const int*)(ar + k), *(const int*)(br + k), acc, false);
-    epi.store(m, n, acc, r, c);
-  } else {
-    float acc = 0.f;
-    for (int k = 0; k < g.K; k += 4) {
-      const uint32_t av = *(const uint32_t*)(ar + k), bv = *(const uint32_t*)(br + k);
-      acc = __fmaf_rn(__builtin_amdgcn_cvt_f32_fp8(av, 0), __builtin_amdgcn_cvt_f32_fp8(bv, 0), acc);
-      acc = __fmaf_rn(__builtin_amdgcn_cvt_f32_fp8(av, 1), __builtin_amdgcn_cvt_f32_fp8(bv, 1), acc);
-      acc = __fmaf_rn(__builtin_amdgcn_cvt_f32_fp8(av, 2), __builtin_amdgcn_cvt_f32_fp8(bv, 2), acc);
-      acc = __fmaf_rn(__builtin_amdgcn_cvt_f32_fp8(av, 3), __builtin_amdgcn_cvt_f32_fp8(bv, 3), acc);
-    }
-    epi.store(m, n, acc, r, c);
-  }
+void launch_cut_k(const GemmArgs& g, const Epi& epi, hipStream_t st) {
+  auto rounds = [&](int t) { return div_up((int64_t)div_up(g.M, t) * div_up(g.N, t), 256); };
+  if (cut_k_tall(g.M, g.N, g.K)) launch_tile<TileTallK, OP, false, true>(g, epi, st);
+  else if (rounds(128) <= 2 * rounds(256)) launch_tile<TileMidK, OP, false, true>(g, epi, st);
+  else launch_tile<TileBig, OP, false, true>(g, epi, st);
 }
 
 template <int OP, class Epi>
 void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
   if (use_tall_tiles(g.M, g.N, g.K)) {
     launch_tile<TileTallK, OP, false>(g, epi, st);
-  } else if (g.K % 64 == 0) {
+  } else if (g.K % 64 == 0 && !cut_k_tall(g.M, g.N, g.K)) {
     switch (pick_tile(g.M, g.N, g.K % 128 == 0 && use_register_staged(OP))) {
       case 0:
         if (g.K % 128 == 0 && use_register_staged(OP)) launch_rs<OP>(g, epi, st);
@@ -234,8 +223,7 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
         break;
     }
   } else {
-    dim3 grid(div_up(g.N, 64), (unsigned)g.M), block(64);
-    hipLaunchKernelGGL((gemm_simple_kernel<OP, Epi>), grid, block, 0, st, g, epi);
+    launch_cut_k<OP>(g, epi, st);
   }
 }
 
@@ -333,7 +321,19 @@ struct SplitPlan {
   int64_t k_len, ws_bytes;
   bool rs;  // 256 x 128 tiles of the register-staged kernel instead of 128 x 128 LDS-DMA tiles
   bool tall = false;  // 128 x 64 tiles with 128-byte stages
+  bool cut = false;   // the last slice is shorter than k_len (KT instances of the tall tiles)
 };
+
+// K in `s` slices of whole 128-byte stages of at least 1024 bytes on 128 x 64 tiles, the last one shorter
+inline bool cut_slices(SplitPlan& p, int64_t M, int64_t N, int64_t K, int s) {
+  s = (int)std::min<int64_t>(s, K / 1024);
+  if (s < 2) return false;
+  p.k_len = ((K + s - 1) / s + 127) / 128 * 128;
+  p.splits = (int)((K + p.k_len - 1) / p.k_len);
+  p.ws_bytes = (int64_t)p.splits * M * N * 4;
+  p.tall = p.cut = true;
+  return true;
+}
 
 // `limit` > 0: the workspace at hand; a plan that needs more is passed over for the next one (the
 // register-staged slices need more partial sums than the 128 x 128 ones: more, shorter slices).
@@ -341,7 +341,15 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   SplitPlan p{1, K, 0, false};
   static const char* off = getenv("FMSMO_SPLIT_K");  // FMSMO_SPLIT_K=0 disables (tuning aid)
   if (off && off[0] == '0') return p;
-  if (M <= 16 || M > 1024 || K % 128 || use_tall_tiles(M, N, K)) return p;
+  if (M <= 16 || M > 1024 || use_tall_tiles(M, N, K)) return p;
+  const int64_t tiles_t = (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN);
+  if (K % 128) {
+    // (us, one pass -> slices, M = 40: N = 1024, K = 4016 13.1 -> 8.8; N = 3072 13.6 -> 10.3; M = 100,
+    // N = 3072, K = 8208 26.3 -> 14.4; M = 200, N = 1500, K = 11216 36.7 -> 16.7.  From a quarter of a
+    // round of tiles on these shapes ask for no workspace.)
+    if (tiles_t < 64) cut_slices(p, M, N, K, (int)(256 / tiles_t));
+    return p;
+  }
   // Long reductions under a few hundred rows: 256 x 128 tiles of the register-staged kernel carry
   // the slices (us, 128 x 128 LDS-DMA tiles -> these, N = 4096, K = 14336: M = 384 51.4 -> 49.0,
   // 512 54.6 -> 48.3, 768 84.7 -> 68.2, 1024 87.6 -> 77.8; at K = 4096 they lose, M = 512 25.5 ->
@@ -371,10 +379,13 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   // 19.4 / 17.9 -> 13.8 / 15.5 / 16.3; K = 8192 18.9 / 19.6 / 18.3 -> 17.4 / 18.5 / 17.2; N = 1024,
   // K = 8192 14.3 / 14.6 / 13.1 -> 10.6 / 11.2 / 11.2; K = 14336, N = 4096, M = 33 / 128 / 256 22.7 /
   // 25.1 / 34.1 -> 22.1 / 24.3 / 33.0).  At most 256 blocks of 128 x 64 partial sums: 8 MiB.
-  const int64_t tiles_t = (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN);
   if (tiles_t <= 128) {
     int s = (int)(256 / tiles_t);
+    const int most = (int)std::min<int64_t>(s, K / 1024);
     while (s > 1 && (K % (s * 128) != 0 || K / s < 1024)) --s;
+    // no even split near the one wanted (K = 128 x a prime): slices of whole stages, the last shorter
+    // (us, K = 9344 = 73 x 128: 33 x 250 28.3 -> 10.5, 80 x 768 28.5 -> 11.2)
+    if (most >= 2 && s * 4 < most * 3 && cut_slices(p, M, N, K, most)) return p;
     if (s >= 2) {
       p.splits = s;
       p.k_len = K / s;
@@ -421,8 +432,10 @@ inline int launch_split_k_i32(const SplitPlan& p, const GemmArgs& g0, void* work
   g.M = p.splits * g0.M;
   g.lda_e = p.k_len;
   g.ldb_e = p.k_len;
+  g.k_total = g0.K;
   g.grid_m = p.splits * div_up(g0.M, p.rs ? 256 : TileMid::BM);
   if (p.rs) launch_rs<MMA_I8, true, 128>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
+  else if (p.cut) launch_tile<TileTallK, MMA_I8, true, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
   else if (p.tall) launch_tile<TileTallK, MMA_I8, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
   else launch_tile<TileMid, MMA_I8, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
   dim3 grid(div_up(g0.N, 256), (unsigned)g0.M), block(256);
@@ -444,10 +457,14 @@ int launch_split_k(const SplitPlan& p, const GemmArgs& g0, void* workspace, cons
   g.M = p.splits * g0.M;
   g.lda_e = p.k_len;
   g.ldb_e = p.k_len;
+  g.k_total = g0.K;
   g.grid_m = p.splits * div_up(g0.M, p.rs ? 256 : TileMid::BM);
   if (p.rs) {
     if constexpr (OP == MMA_I8) launch_rs<OP, true, 128>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
     else launch_rs<OP, true, 128>(g, EpiStoreF32{(float*)workspace, g0.N}, st);
+  } else if (p.cut) {
+    if constexpr (OP == MMA_I8) launch_tile<TileTallK, OP, true, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
+    else launch_tile<TileTallK, OP, true, true>(g, EpiStoreF32{(float*)workspace, g0.N}, st);
   } else if (p.tall) {
     if constexpr (OP == MMA_I8) launch_tile<TileTallK, OP, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
     else launch_tile<TileTallK, OP, true>(g, EpiStoreF32{(float*)workspace, g0.N}, st);

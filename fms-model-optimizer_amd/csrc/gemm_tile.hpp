@@ -16,6 +16,13 @@
 // of stage kt, so every stage has NSTAGE-1 full iterations (> 1 us) to arrive from L2/HBM.
 // One barrier per stage; the barrier, the DMA issue and the first operand reads of the next
 // stage are hidden under MFMAs whose operands were read earlier (register double buffering).
+//
+// Reductions that are no multiple of a stage (KT instances; K is a multiple of 16 bytes, i.e. of the
+// 16-byte chunks a lane moves): in the last stage the lanes whose chunk lies past K fetch the row's
+// first chunk of that stage instead, and every wave overwrites what those lanes brought with zeros in
+// LDS before the barrier that publishes the stage.  The rest of the pipeline does not know about it.
+// (One thread per output with 4-byte dot products, which served those K before: 386 x 531 x 11472
+// e4m3 2110 us, now 29; 3868 x 542 x 688 int8 1195 -> 14; 57 x 17694 x 1136 e4m3 1382 -> 14.)
 #pragma once
 #include "common.hpp"
 #include <type_traits>
@@ -39,6 +46,8 @@ struct GemmArgs {
   int rows_per_group;  // > 0: every group owns this many rows (batched matmul, split K), offsets unused
   int64_t lda_e;       // uniform groups: bytes between groups in A (rows * lda for stacked batches,
                        // the K slice length when the groups are slices of one reduction)
+  int k_total;         // KT instances, > 0: the groups are K slices of a reduction of this many bytes,
+                       // the last one may be shorter than K
   int k_rotate;  // register-staged kernel: block b starts its reduction at slab (b * k_rotate) % slabs
   // optional clock probe (register-staged kernel): block 0 stores {core clock counter, 100 MHz
   // wall clock} at its start, after its K loop and after its epilogue; null = off
@@ -217,7 +226,7 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblk, int grid_m, int
 }
 
 template <int BM, int BN, int BK, int NSTAGE, int WGM, int WGN, int OP, int SWZ, bool GROUPED,
-          class Epi, class Chk = NoChunk>
+          class Epi, class Chk = NoChunk, bool KT = false>
 // (two blocks per compute unit for the scheduled chunk hooks; the generic hook keeps a second
 // accumulator set and would spill at 256 registers)
 __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1) void gemm_tile_kernel(GemmArgs g, Epi epi, Chk chk) {
@@ -506,7 +515,34 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
   };
 
   Frag fa[2][FM], fb[2][FN];
-  const int nk = g.K / BK;
+  int k_len = g.K;
+  if constexpr (KT && GROUPED) {
+    if (g.k_total > 0) k_len = min(k_len, g.k_total - expert * k_len);
+  }
+  const int nk = KT ? (k_len + BK - 1) / BK : k_len / BK;
+  // KT: lanes whose chunk of the last stage lies past the end of the reduction
+  [[maybe_unused]] const bool past_end = KT && (nk - 1) * BK + ld_chunk * 16 >= k_len;
+  // before the DMA of stage st: from the last stage on those lanes fetch chunk 0 (in bounds)
+  auto before_issue = [&](int st) __attribute__((always_inline)) {
+    if constexpr (KT) {
+      if (st == nk - 1 && past_end) {
+#pragma unroll
+        for (int j = 0; j < NIA; ++j) a_off[j] -= ld_chunk * 16;
+#pragma unroll
+        for (int j = 0; j < NIB; ++j) b_off[j] -= ld_chunk * 16;
+      }
+    }
+  };
+  // stage st has landed for this wave: replace what those lanes fetched by zeros
+  auto zero_past_end = [&](int st) __attribute__((always_inline)) {
+    if constexpr (KT) {
+      if (st == nk - 1 && past_end) {
+        uint8_t* dst = &lds[0][0] + (st % NSTAGE) * STAGE_BYTES + tid * 16;
+#pragma unroll
+        for (int j = 0; j < NIA + NIB; ++j) *(v4i*)(dst + j * THREADS * 16) = v4i{0, 0, 0, 0};
+      }
+    }
+  };
 
   // One K-stage.  PAR = parity of kt * NKS, so that operand-register buffer indices are static.
   // While stage kt is multiplied, the DMA of stage kt+NSTAGE-1 refills the buffer that stage
@@ -519,6 +555,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
     const int fill = (kt + NSTAGE - 1) % NSTAGE;
     const int fill_k0 = min(kt + NSTAGE - 1, nk - 1) * BK;
     const uint8_t* ls = &lds[0][0] + cur * STAGE_BYTES;
+    before_issue(kt + NSTAGE - 1);
     auto dma = [&](auto s_c) {
       constexpr int S = decltype(s_c)::value;
       issue_part(fill, fill_k0, std::integral_constant<int, NLD * S / NKS>{},
@@ -539,6 +576,10 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
     // stage kt+1 has landed (younger DMA may stay in flight) and until its own LDS reads of
     // stage kt have returned, then barrier: stage kt+1 is now complete for all waves and buffer
     // `cur` may be refilled during the next stage.
+    if constexpr (KT) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 3) * NLD + NLD * (NKS - 1) / NKS) : "memory");
+      zero_past_end(kt + 1);
+    }
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NSTAGE - 3) * NLD + NLD * (NKS - 1) / NKS)
                  : "memory");
     const int nxt = (kt + 1) % NSTAGE;
@@ -550,10 +591,18 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
   };
 
 #pragma unroll
-  for (int st = 0; st < NSTAGE - 1; ++st)
+  for (int st = 0; st < NSTAGE - 1; ++st) {
+    before_issue(st);
     issue_part(st, min(st, nk - 1) * BK, std::integral_constant<int, 0>{},
                std::integral_constant<int, NLD>{});
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NSTAGE - 2) * NLD) : "memory");
+  }
+  if constexpr (KT) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 2) * NLD) : "memory");
+    zero_past_end(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NSTAGE - 2) * NLD) : "memory");
+  }
   if constexpr (Chk::one_stage) {
     // Chunk == stage: the fragments of all k-steps of a chunk are register resident (two sets:
     // the stage being multiplied and the one being read), and the rounding of one 32x32 block is
@@ -567,6 +616,11 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
       constexpr int PAR = decltype(par_c)::value;
       // stage kt + 1 has landed for every wave; its fragments go to the other register set, and
       // the buffer of stage kt - 1 (last read a stage ago) is refilled with stage kt + 3
+      if constexpr (KT) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 3) * NLD) : "memory");
+        zero_past_end(kt + 1);
+        before_issue(kt + NSTAGE - 1);
+      }
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NSTAGE - 3) * NLD) : "memory");
       const uint8_t* ls = &lds[0][0] + ((kt + 1) % NSTAGE) * STAGE_BYTES;
 #pragma unroll

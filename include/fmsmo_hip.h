@@ -374,7 +374,8 @@ enum fmsmo_plan_kernel {
   FMSMO_PLAN_DECODE = 0,                /* skinny-M weight-streaming kernels */
   FMSMO_PLAN_TILE_REGISTER_STAGED = 1,  /* MFMA tiles, 128-byte K slabs staged through registers */
   FMSMO_PLAN_TILE_LDS_DMA = 2,          /* MFMA tiles, 64-byte K stages loaded straight into LDS */
-  FMSMO_PLAN_GENERIC = 3                /* K % 64 != 0: one thread per output element */
+  FMSMO_PLAN_GENERIC = 3                /* K % 64 != 0: MFMA tiles as in 2 with a last stage cut at K
+                                           (the tile shape is not reported) */
 };
 int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
                     int* tile_n, int* splits);

@@ -57,3 +57,32 @@ def test_deploy_module_of_a_bf16_model_rounds_to_fp16_first(dev, M, w_std, kerne
     ref = O.epilogue_ref(acc, s_x, bufs["w_scale"], bufs["bias"], torch.bfloat16)
     assert y.dtype == torch.bfloat16 and bool(torch.isinf(ref).any()) == (w_std > 1)
     assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,Kd", [
+    (1, 5, 16), (3, 64, 48), (17, 65, 80), (128, 63, 112), (129, 130, 144),   # one and two stages, all but empty
+    (16, 301, 1040), (300, 520, 624), (1500, 2400, 688), (257, 4099, 592),     # 128 x 64, 128 x 128, 256 x 256 tiles
+    (2600, 2600, 336), (65, 640, 4160),
+    (40, 100, 2064), (100, 700, 4016), (33, 250, 9344), (200, 130, 11216)])    # K slices, the last one shorter
+def test_reductions_that_are_no_multiple_of_a_stage(dev, M, N, Kd):
+    """K % 128 != 0 (the last stage is cut at K) and slices of unequal length: int8 exact, with and
+    without a workspace; e4m3 exact on small integers.  What lies behind a row's K elements -- here
+    large codes, for e4m3 NaN -- must not enter."""
+    kn = K()
+    g = torch.Generator(device=dev).manual_seed(M + N + Kd)
+    a = torch.randint(-128, 128, (M, Kd + 16), generator=g, dtype=torch.int8, device=dev)[:, :Kd]
+    w = torch.randint(-128, 128, (N, Kd + 32), generator=g, dtype=torch.int8, device=dev)[:, :Kd]
+    acc = (a.double() @ w.double().t()).to(torch.int32)
+    assert torch.equal(kn.gemm_i8_i32(a, w), acc)
+    s_a = (torch.rand(M, 1, generator=gen(61)) * 0.05 + 1e-3).half()
+    s_w = (torch.rand(N, generator=gen(62)) * 1e-3 + 1e-5).float()
+    ref = O.epilogue_ref(acc.cpu(), s_a, s_w, None, torch.float16)
+    y = kn.gemm_i8_dq(a, w, s_a.float().reshape(-1).to(dev), s_w.to(dev), None, out_dtype=torch.float16, exact_ref=True)
+    assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
+    nan = torch.full((), float("nan"), device=dev)
+    a8 = torch.cat((torch.randint(-4, 5, (M, Kd), generator=g, device=dev).float(), nan.expand(M, 16)), 1)
+    w8 = torch.cat((torch.randint(-4, 5, (N, Kd), generator=g, device=dev).float(), nan.expand(N, 16)), 1)
+    one = torch.ones(1, device=dev)
+    y8 = kn.gemm_fp8_dq(a8.to(torch.float8_e4m3fn)[:, :Kd], w8.to(torch.float8_e4m3fn)[:, :Kd], one, one, None,
+                        out_dtype=torch.float32)
+    assert torch.equal(y8.double(), a8[:, :Kd].double() @ w8[:, :Kd].double().t())   # |sums| < 2^24: exact in fp32
