@@ -9,6 +9,7 @@
 // and then rounded to T, which equals the correctly rounded T division torch performs.
 #include "quant_math.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace fmsmo {
@@ -1213,6 +1214,168 @@ __global__ __launch_bounds__(AQ_THREADS) void quant_fp8_pertoken16_kernel(
   }
 }
 
+// ------------------------------------------------------------------ e4m3, one scale per tensor
+// The whole quantizer in two passes over x and two launches (one for small tensors): 256 blocks leave
+// their abs-max in `part`, and every block of the quantizer reduces those 256 words itself while its
+// first elements are on their way.  HBM bound.  (Before: a fill of a [K] vector, column maxima merged
+// with atomics, a one-block kernel over K values for the scale, then the per-token kernel with its row
+// maxima: 4.3 + 7.2 + 13.0 + 10.5 us at 777 x 12800 fp16, now 13.2 for both launches)
+constexpr int TENSOR_PARTS = 256;
+constexpr int TENSOR_SELF_CHUNKS = 8192;  // up to this many 8-element chunks every block reads all of x
+
+// Where the chunks of x lie: a flat index when the rows are contiguous, else row and column.
+__device__ __forceinline__ size_t chunk_elem(int64_t c, int cpr, int64_t ld, bool flat) {
+  if (flat) return (size_t)c * AQ_VEC;
+  const uint32_t row = (uint32_t)c / (uint32_t)cpr;
+  return (size_t)row * ld + (size_t)((uint32_t)c - row * (uint32_t)cpr) * AQ_VEC;
+}
+
+// |x| as fp32 bits (maxima of 16-bit magnitudes keep NaN above infinity, fp32 maxima drop NaN, as the
+// column abs-max kernel has it)
+template <int XT>
+struct AbsMax {
+  us2 best = {0, 0};
+  __device__ __forceinline__ void add(const v4i& w) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t mag = (uint32_t)w[j] & 0x7fff7fffu;
+      us2 m2;
+      __builtin_memcpy(&m2, &mag, 4);
+      best = __builtin_elementwise_max(best, m2);
+    }
+  }
+  __device__ __forceinline__ uint32_t bits() const {
+    return __float_as_uint(cvt16<XT>(best[0] > best[1] ? best[0] : best[1]));
+  }
+};
+template <>
+struct AbsMax<FMSMO_F32> {
+  float best = 0.0f;
+  __device__ __forceinline__ void add(const v4i& w) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) best = fmaxf(best, fabsf(__int_as_float(w[j])));
+  }
+  __device__ __forceinline__ uint32_t bits() const { return __float_as_uint(best); }
+};
+
+// block maximum of an unsigned value, same in every thread; one barrier
+template <int TH>
+__device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* red) {
+  v = wave_max_u32(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  uint32_t r = red[0];
+#pragma unroll
+  for (int w = 1; w < TH / 64; ++w) r = max(r, red[w]);
+  return r;
+}
+
+template <int XT>
+__global__ __launch_bounds__(1024) void absmax_parts_kernel(const void* __restrict__ x, int64_t ldx, int cpr,
+                                                            int64_t nchunks, int flat, uint32_t* __restrict__ part) {
+  __shared__ uint32_t red[16];
+  constexpr int W = XT == FMSMO_F32 ? 2 : 1;  // 16-byte words per chunk
+  constexpr int U = 4;                        // chunks in flight per thread
+  AbsMax<XT> m;
+  const int64_t step = (int64_t)gridDim.x * 1024;
+  for (int64_t c = (int64_t)blockIdx.x * 1024 + threadIdx.x; c < nchunks; c += U * step) {
+    v4i w[U][W];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t e = chunk_elem(min(c + u * step, nchunks - 1), cpr, ldx, flat);  // the tail re-reads the last chunk
+#pragma unroll
+      for (int j = 0; j < W; ++j)
+        w[u][j] = *(const v4i*)((const uint8_t*)x + e * (XT == FMSMO_F32 ? 4 : 2) + j * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < W; ++j) m.add(w[u][j]);
+  }
+  const uint32_t b = block_max_u32<1024>(m.bits(), red);
+  if (threadIdx.x == 0) part[blockIdx.x] = b;
+}
+
+// SELF: every block takes the abs-max of the whole tensor itself (small tensors: one launch); else it is
+// the maximum of the `nparts` words that absmax_parts_kernel left.  Codes as quant_fp8_pertoken16_kernel
+// forms them for a given scale: refined quotients and the hardware conversion while the tensor's
+// maximum is finite and the scale in the quotients' range, IEEE and the software encoder otherwise.
+template <int XT, int VAR, bool SELF>
+__global__ __launch_bounds__(SELF ? 1024 : 256) void quant_fp8_tensor16_kernel(
+    const u16* __restrict__ x, int64_t ldx, int cpr, int64_t nchunks, int flat, const uint32_t* __restrict__ part,
+    int nparts, float scale_floor, int scale_in_xt, uint8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale) {
+  constexpr int TH = SELF ? 1024 : 256;
+  constexpr bool LIN = VAR == FMSMO_FP8_LINEAR;
+  __shared__ uint32_t red[TH / 64];
+  const int64_t step = (int64_t)gridDim.x * TH;
+  int64_t c = (int64_t)blockIdx.x * TH + threadIdx.x;
+  v4i cur = {0, 0, 0, 0};
+  if (c < nchunks) cur = *(const v4i*)(x + chunk_elem(c, cpr, ldx, flat));
+  uint32_t b = 0;
+  if constexpr (SELF) {
+    AbsMax<XT> m;
+    m.add(cur);
+    // every other chunk, once; the block's own ones are in registers (one per thread: SELF grids
+    // cover the tensor)
+    for (int64_t o = threadIdx.x; o < nchunks; o += 4 * 1024) {
+      v4i w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = *(const v4i*)(x + chunk_elem(min(o + u * 1024, nchunks - 1), cpr, ldx, flat));
+#pragma unroll
+      for (int u = 0; u < 4; ++u) m.add(w[u]);
+    }
+    b = m.bits();
+  } else {
+    for (int p = threadIdx.x; p < nparts; p += TH) b = max(b, part[p]);
+  }
+  b = block_max_u32<TH>(b, red);
+  const float amax = __uint_as_float(b);
+  const float s = fp8_dynamic_scale<XT>(amax, scale_floor, scale_in_xt);
+  if (blockIdx.x == 0 && threadIdx.x == 0) scale[0] = s;
+  const bool fast = b < 0x7f800000u && s >= 0x1p-60f && s <= 0x1p60f && amax <= s * 0x1p100f;
+  const float r1 = rcp_refined(s);
+  [[maybe_unused]] const float nz = opaque_neg_zero();
+  while (c < nchunks) {
+    const int64_t next = c + step;
+    v4i nxt = {0, 0, 0, 0};
+    if (next < nchunks) nxt = *(const v4i*)(x + chunk_elem(next, cpr, ldx, flat));
+    uint8_t* dst = q + chunk_elem(c, cpr, ldq, flat && ldq == (int64_t)cpr * AQ_VEC);
+    if (fast) {
+      float t[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float xv = cvt16<XT>((u16)((uint32_t)cur[j >> 1] >> ((j & 1) * 16)));
+        if constexpr (LIN) {
+          if constexpr (XT == FMSMO_F16) t[j] = div32_fast_mix(xv, s, r1, nz);
+          else t[j] = div32_fast(xv, s, r1);
+        } else {
+          t[j] = cvt16<XT>(to16<XT>(div16<XT, false>(xv, s, r1)));
+        }
+        t[j] = __builtin_copysignf(__builtin_amdgcn_fmed3f(t[j], -448.0f, 448.0f), xv);
+        if constexpr (VAR == FMSMO_FP8_FPXACC_DL8) t[j] = fabsf(t[j]) <= 0.0087890625f ? 0.0f : t[j];
+      }
+      int o0 = 0, o1 = 0;
+      o0 = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], o0, false);
+      o0 = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], o0, true);
+      o1 = __builtin_amdgcn_cvt_pk_fp8_f32(t[4], t[5], o1, false);
+      o1 = __builtin_amdgcn_cvt_pk_fp8_f32(t[6], t[7], o1, true);
+      *(uint2*)dst = make_uint2((uint32_t)o0, (uint32_t)o1);
+    } else {
+      uint8_t code[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float xv = cvt16<XT>((u16)((uint32_t)cur[j >> 1] >> ((j & 1) * 16)));
+        const float t = LIN ? fminf(fmaxf(xv / s, -448.0f), 448.0f) : round_to<XT>(xv / s);
+        code[j] = f32_to_e4m3_sw(t);
+        if (VAR == FMSMO_FP8_FPXACC_DL8 && (code[j] & 0x7f) <= 0x04) code[j] = 0x00;
+      }
+      store8(dst, 0, code);
+    }
+    cur = nxt;
+    c = next;
+  }
+}
+
 }  // namespace fmsmo
 
 using namespace fmsmo;
@@ -1562,6 +1725,15 @@ static int check_quant_fp8(const void* x, int x_dtype, int64_t ldx, int variant,
   return FMSMO_OK;
 }
 
+static int check_fp8_floor(float scale_floor, int scale_dtype, int x_dtype) {
+  if (scale_dtype != FMSMO_F32 && scale_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
+  if (!(scale_floor > 0.0f) || !(scale_floor < 0x1p60f)) return FMSMO_ERR_UNSUPPORTED;
+  // a floor that rounds to zero in x's dtype would let a zero row divide by zero
+  if (scale_dtype == FMSMO_F16 && scale_floor <= 0x1p-25f) return FMSMO_ERR_UNSUPPORTED;
+  if (scale_dtype == FMSMO_BF16 && scale_floor < 0x1p-126f) return FMSMO_ERR_UNSUPPORTED;
+  return FMSMO_OK;
+}
+
 extern "C" int fmsmo_quant_act_fp8_pertoken(const void* x, int x_dtype, int64_t ldx, int variant,
                                             int static_scale, uint8_t* q, int64_t ldq,
                                             float* scale, int64_t M, int64_t K,
@@ -1582,11 +1754,7 @@ extern "C" int fmsmo_quant_act_fp8_dynamic(const void* x, int x_dtype, int64_t l
                                            fmsmo_stream_t stream) {
   if (const int e = check_quant_fp8(x, x_dtype, ldx, variant, q, ldq, scale, M, K)) return e;
   if (per_tensor && !col_amax) return FMSMO_ERR_NULL;
-  if (scale_dtype != FMSMO_F32 && scale_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
-  if (!(scale_floor > 0.0f) || !(scale_floor < 0x1p60f)) return FMSMO_ERR_UNSUPPORTED;
-  // a floor that rounds to zero in x's dtype would let a zero row divide by zero
-  if (scale_dtype == FMSMO_F16 && scale_floor <= 0x1p-25f) return FMSMO_ERR_UNSUPPORTED;
-  if (scale_dtype == FMSMO_BF16 && scale_floor < 0x1p-126f) return FMSMO_ERR_UNSUPPORTED;
+  if (const int e = check_fp8_floor(scale_floor, scale_dtype, x_dtype)) return e;
   if (M == 0) return FMSMO_OK;
   hipStream_t st = (hipStream_t)stream;
   const int in_xt = scale_dtype != FMSMO_F32;
@@ -1603,4 +1771,54 @@ extern "C" int fmsmo_quant_act_fp8_dynamic(const void* x, int x_dtype, int64_t l
   }
   return launch_quant_fp8(x, x_dtype, ldx, variant, per_tensor ? 2 : 0, scale_floor, in_xt, q, ldq,
                           scale, M, K, st);
+}
+
+extern "C" int fmsmo_quant_act_fp8_tensor(const void* x, int x_dtype, int64_t ldx, int variant, float scale_floor,
+                                          int scale_dtype, float* scratch, uint8_t* q, int64_t ldq, float* scale,
+                                          int64_t M, int64_t K, fmsmo_stream_t stream) {
+  if (const int e = check_quant_fp8(x, x_dtype, ldx, variant, q, ldq, scale, M, K)) return e;
+  if (!scratch) return FMSMO_ERR_NULL;
+  if (const int e = check_fp8_floor(scale_floor, scale_dtype, x_dtype)) return e;
+  if (M == 0) return FMSMO_OK;
+  const int64_t nchunks = M * (K / AQ_VEC);
+  if (nchunks >= (1ll << 31)) return FMSMO_ERR_UNSUPPORTED;
+  hipStream_t st = (hipStream_t)stream;
+  const int in_xt = scale_dtype != FMSMO_F32, cpr = (int)(K / AQ_VEC), flat = ldx == K;
+  uint32_t* part = (uint32_t*)scratch;
+  const bool self = x_dtype != FMSMO_F32 && nchunks <= TENSOR_SELF_CHUNKS;
+  const int parts = (int)std::min<int64_t>(TENSOR_PARTS, (nchunks + 1023) / 1024);
+  if (!self) {
+#define LAUNCH(XT) \
+  hipLaunchKernelGGL((absmax_parts_kernel<XT>), dim3(parts), dim3(1024), 0, st, x, ldx, cpr, nchunks, flat, part)
+    switch (x_dtype) {
+      case FMSMO_F16: LAUNCH(FMSMO_F16); break;
+      case FMSMO_BF16: LAUNCH(FMSMO_BF16); break;
+      default: LAUNCH(FMSMO_F32); break;
+    }
+#undef LAUNCH
+  }
+  if (x_dtype == FMSMO_F32) {  // the generic quantizer takes a finished scale
+    hipLaunchKernelGGL((fp8_tensor_scale_kernel<FMSMO_F32>), dim3(1), dim3(AQ_THREADS), 0, st, (const float*)part, parts,
+                       scale_floor, in_xt, scale);
+    return launch_quant_fp8(x, x_dtype, ldx, variant, 2, scale_floor, in_xt, q, ldq, scale, M, K, st);
+  }
+#define LAUNCH(XT, VAR)                                                                                               \
+  if (self)                                                                                                           \
+    hipLaunchKernelGGL((quant_fp8_tensor16_kernel<XT, VAR, true>), dim3((unsigned)((nchunks + 1023) / 1024)),         \
+                       dim3(1024), 0, st, (const u16*)x, ldx, cpr, nchunks, flat, part, parts, scale_floor, in_xt, q, \
+                       ldq, scale);                                                                                   \
+  else                                                                                                                \
+    hipLaunchKernelGGL((quant_fp8_tensor16_kernel<XT, VAR, false>),                                                   \
+                       dim3((unsigned)std::min<int64_t>(2048, (nchunks + 255) / 256)), dim3(256), 0, st,              \
+                       (const u16*)x, ldx, cpr, nchunks, flat, part, parts, scale_floor, in_xt, q, ldq, scale)
+#define PICK(XT)                                                          \
+  switch (variant) {                                                      \
+    case FMSMO_FP8_LINEAR: LAUNCH(XT, FMSMO_FP8_LINEAR); break;           \
+    case FMSMO_FP8_FPXACC: LAUNCH(XT, FMSMO_FP8_FPXACC); break;           \
+    default: LAUNCH(XT, FMSMO_FP8_FPXACC_DL8); break;                     \
+  }
+  if (x_dtype == FMSMO_F16) { PICK(FMSMO_F16) } else { PICK(FMSMO_BF16) }
+#undef PICK
+#undef LAUNCH
+  return fmsmo_check_launch();
 }

@@ -189,8 +189,8 @@ def quant_act_fp8_dynamic(x, variant=L.FP8_LINEAR, per_tensor=False, scale_floor
                           scale_in_x_dtype=False):
     """(q e4m3 [M,K], scale fp32 [M] or [1]): the e4m3 quantizer with a dynamic scale
     max(amax / 448, scale_floor) per token or for the whole tensor, the division in fp32 or in
-    x's dtype (see fmsmo_quant_act_fp8_dynamic).  Per tensor it is two passes over x (column
-    abs-max, quantizer) with nothing read back to the host."""
+    x's dtype (see fmsmo_quant_act_fp8_dynamic / _tensor).  Per tensor it is two passes over x
+    (abs-max, quantizer) with nothing read back to the host."""
     _need_gpu(x)
     if x.dim() != 2:
         raise ValueError("expected a 2-D tensor")
@@ -198,12 +198,16 @@ def quant_act_fp8_dynamic(x, variant=L.FP8_LINEAR, per_tensor=False, scale_floor
     M, K = x.shape
     q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=x.device)
     scale = torch.empty((1 if per_tensor else M,), dtype=torch.float32, device=x.device)
-    col_amax = absmax_cols(x) if per_tensor else None
     with _dev(x):
-        L.call("fmsmo_quant_act_fp8_dynamic", x.data_ptr(), _dt(x), _ld(x), int(variant),
-               int(bool(per_tensor)), _ptr(col_amax), float(scale_floor),
-               _dt(x) if scale_in_x_dtype else L.F32, q.data_ptr(), K, scale.data_ptr(), M, K,
-               _stream(x))
+        if per_tensor and M > 0:
+            parts = torch.empty((256,), dtype=torch.float32, device=x.device)
+            L.call("fmsmo_quant_act_fp8_tensor", x.data_ptr(), _dt(x), _ld(x), int(variant), float(scale_floor),
+                   _dt(x) if scale_in_x_dtype else L.F32, parts.data_ptr(), q.data_ptr(), K, scale.data_ptr(),
+                   M, K, _stream(x))
+        else:
+            L.call("fmsmo_quant_act_fp8_dynamic", x.data_ptr(), _dt(x), _ld(x), int(variant), 0, None,
+                   float(scale_floor), _dt(x) if scale_in_x_dtype else L.F32, q.data_ptr(), K,
+                   scale.data_ptr(), M, K, _stream(x))
     return q, scale
 
 

@@ -280,6 +280,14 @@ int fmsmo_quant_act_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, int var
                                 int per_tensor, const float* col_amax, float scale_floor,
                                 int scale_dtype, uint8_t* q, int64_t ldq, float* scale,
                                 int64_t M, int64_t K, fmsmo_stream_t stream);
+/*
+ * The per-tensor form of the above in one call that takes the abs-max itself: two passes over x.
+ * scratch: fp32 [256] on the device, contents undefined before and after (calls that may overlap
+ * need one each).  scale [1] is written.
+ */
+int fmsmo_quant_act_fp8_tensor(const void* x, int x_dtype, int64_t ldx, int variant, float scale_floor,
+                               int scale_dtype, float* scratch, uint8_t* q, int64_t ldq, float* scale,
+                               int64_t M, int64_t K, fmsmo_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------
  * 2. W8A8 GEMMs on MFMA.   C[M,N] = A[M,K] . B[N,K]^T

@@ -86,3 +86,32 @@ def test_reductions_that_are_no_multiple_of_a_stage(dev, M, N, Kd):
     y8 = kn.gemm_fp8_dq(a8.to(torch.float8_e4m3fn)[:, :Kd], w8.to(torch.float8_e4m3fn)[:, :Kd], one, one, None,
                         out_dtype=torch.float32)
     assert torch.equal(y8.double(), a8[:, :Kd].double() @ w8[:, :Kd].double().t())   # |sums| < 2^24: exact in fp32
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,Kd,pad", [(1, 16, 0), (3, 4096, 0), (16, 4096, 8), (17, 3856, 0), (700, 1032, 24), (4096, 512, 0)])
+def test_fp8_per_tensor_quantizer_in_two_passes(dev, dtype, M, Kd, pad):
+    """One scale for the tensor, with the abs-max taken inside the call (one launch up to 8192 groups of
+    eight elements, partial maxima beyond; rows with a stride): bit for bit what the entry point that
+    is handed the column maxima gives, for every recipe, for huge, tiny, infinite and NaN elements."""
+    from fms_mo_amd import _lib as L
+
+    kn, lib = K(), L.load()
+    st = torch.cuda.current_stream().cuda_stream
+    base = (torch.randn(M, Kd + pad, generator=gen(M + Kd)) * 3).to(dtype).to(dev)
+    for special in (None, float("inf"), float("nan"), 0.0, 1e-20):
+        x = base.clone()
+        if special is not None:
+            x = x * 0 if special in (0.0, 1e-20) else x
+            x[M // 2, Kd // 2] = special
+        x = x[:, :Kd]
+        for variant, floor, in_x in ((L.FP8_LINEAR, 1e-12, False), (L.FP8_FPXACC, 1e-5, True), (L.FP8_FPXACC_DL8, 1e-5, True)):
+            q, s = kn.quant_act_fp8_dynamic(x, variant, True, floor, in_x)
+            amax, q2, s2 = kn.absmax_cols(x), torch.empty_like(q), torch.empty_like(s)
+            dt = kn._dt(x)
+            assert lib.fmsmo_quant_act_fp8_dynamic(x.data_ptr(), dt, kn._ld(x), variant, 1, amax.data_ptr(), floor,
+                                                   dt if in_x else L.F32, q2.data_ptr(), Kd, s2.data_ptr(), M, Kd, st) == 0
+            assert torch.equal(s.view(torch.int32), s2.view(torch.int32)), (special, variant)
+            if special is not None and special != special and variant != L.FP8_LINEAR:
+                continue  # a NaN abs-max: every torch code is NaN; both forms keep the floor as scale, only one clamps
+            assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8)), (special, variant)
