@@ -97,9 +97,23 @@ __global__ __launch_bounds__(256, 2) void gemm_k128_kernel(GemmArgs g, Epi epi) 
     }
   };
 
+  // Output through a descriptor that ends with the batch entry's last row: 32-bit offsets; lanes of
+  // columns past N get an offset outside and rows past the end lie outside by themselves, so cut tiles
+  // store like whole ones, without a branch.  (64-bit addresses and per-lane tests, with this epilogue: whole
+  // tiles 67 us for 32 heads of 2048 x 2048, cut ones 20.5 for 12 heads of 335 x 335; so 64 and 7.5.)
+  constexpr int ESZ = Epi::OUT_DT == FMSMO_F32 ? 4 : 2;
+  const int ldy = (int)epi.ldy * ESZ;
+  typename Epi::Col ctx[FN];
+  auto columns = [&](const Where& w) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j) ctx[j] = epi.col(min(w.col_lo + wn * TN + j * 32 + fr, g.N - 1), w.expert, g.N);
+  };
+  const float sc = epi.row(0).sc;
+
   int tile = blockIdx.x;
   if (tile >= total) return;
   Where cur = locate(tile);
+  columns(cur);
   request(cur);
   while (true) {
     // the tile's operands into LDS (waits for its requests)
@@ -110,27 +124,18 @@ __global__ __launch_bounds__(256, 2) void gemm_k128_kernel(GemmArgs g, Epi epi) 
     }
     __syncthreads();
 
-    // epilogue operands of this tile are fetched before the next tile's requests (see above)
-    const int m_base = cur.row_lo + wm * TM + fg * 4;
-    const int n_base = cur.col_lo + wn * TN + fr;
-    typename Epi::Col colctx[FN];
-#pragma unroll
-    for (int j = 0; j < FN; ++j) colctx[j] = epi.col(min(n_base + j * 32, g.N - 1), cur.expert, g.N);
-    constexpr int NROW = Epi::UNIFORM_ROWS ? 1 : FM * 16;  // one scale for all rows: nothing per row
-    typename Epi::Row rowctx[NROW];
-#pragma unroll
-    for (int i = 0; i < NROW; ++i)
-      rowctx[i] = epi.row(min(m_base + (i >> 4) * 32 + ((i & 15) >> 2) * 8 + (i & 3), cur.row_hi - 1));
-    __builtin_amdgcn_sched_barrier(0);
-
     // multiply (one set of fragment registers: the matrix work is a small part of a tile)
+    // the accumulators start from the zero-point correction, an integer per column
     Acc acc[FM][FN];
+    typename Epi::Col done[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) done[j] = ctx[j];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0 - done[j].z;
 #pragma unroll
     for (int s = 0; s < NKS; ++s) {
       Frag fa[FM], fb[FN];
@@ -153,6 +158,7 @@ __global__ __launch_bounds__(256, 2) void gemm_k128_kernel(GemmArgs g, Epi epi) 
     if (has_next) {
       __syncthreads();  // every wave has read its fragments: the slab may be overwritten
       nxt = locate(next);
+      columns(nxt);  // in front of the requests: loads return in order
       request(nxt);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -163,31 +169,32 @@ __global__ __launch_bounds__(256, 2) void gemm_k128_kernel(GemmArgs g, Epi epi) 
     // per lane -- accumulators transposed by swapping the MFMA operands, with or without a pass
     // through LDS to make whole 256-byte runs -- measured slower: 0.27 -> 0.49 / 0.35 ms on 32
     // heads of 4096 x 4096 scores)
-    const bool interior = (cur.row_lo + BM <= cur.row_hi) && (cur.col_lo + BN <= g.N);
+    const __amdgpu_buffer_rsrc_t rsrc_y = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((uint8_t*)epi.y + (int64_t)cur.expert * g.rows_per_group * ldy), 0, g.rows_per_group * ldy, 0x00020000);
+    // (all of an offset is in the vector register: the range check covers it, and 2^31 plus an offset
+    // below 2^31 stays outside)
+    const int row_in = cur.row_lo - cur.expert * g.rows_per_group + wm * TM + fg * 4;
+    unsigned voff[FN];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      if (interior) {
+    for (int j = 0; j < FN; ++j) {
+      const int n = cur.col_lo + wn * TN + j * 32 + fr;
+      voff[j] = n < g.N ? (unsigned)(row_in * ldy + n * ESZ) : 0x80000000u;
+    }
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = m_base + i * 32 + (v >> 2) * 8 + (v & 3);
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
-            epi.store(m, n_base + j * 32, acc[i][j][v], rowctx[Epi::UNIFORM_ROWS ? 0 : i * 16 + v], colctx[j]);
-        }
-      } else {
+      for (int v = 0; v < 16; ++v) {
+        const unsigned step = (unsigned)((i * 32 + (v >> 2) * 8 + (v & 3)) * ldy);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = m_base + i * 32 + (v >> 2) * 8 + (v & 3);
-          if (m < cur.row_hi) {
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-              const int n = n_base + j * 32;
-              if (n < g.N) epi.store(m, n, acc[i][j][v], rowctx[Epi::UNIFORM_ROWS ? 0 : i * 16 + v], colctx[j]);
-            }
-          }
+        for (int j = 0; j < FN; ++j) {
+          const float t = __fmaf_rn((float)acc[i][j][v], sc, done[j].b);
+          if constexpr (Epi::OUT_DT == FMSMO_F32)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(t), rsrc_y, voff[j] + step, 0, 0);
+          else
+            __builtin_amdgcn_raw_buffer_store_b16(Epi::OUT_DT == FMSMO_F16 ? f32_to_f16(t) : f32_to_bf16(t), rsrc_y,
+                                                  voff[j] + step, 0, 0);
         }
       }
-    }
     if (!has_next) break;
     tile = next;
     cur = nxt;

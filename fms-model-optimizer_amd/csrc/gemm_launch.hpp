@@ -505,10 +505,11 @@ namespace {
 template <int OP, class AccT>
 int launch_bmm(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t stride_b,
                const float* a_scale, const float* b_scale, const float* bias, void* y, int y_dtype,
-               int64_t ldy, int64_t batch, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+               int64_t ldy, int64_t batch, int64_t M, int64_t N, int64_t K, hipStream_t st, float sc = 1.0f,
+               const int32_t* sums = nullptr, int parts = 0, int zero = 0) {
   int rc = check_gemm(a, lda, b, ldb, y, ldy, batch * M, N, K);
   if (rc) return rc;
-  if (!a_scale || !b_scale) return FMSMO_ERR_NULL;
+  if (!sums && (!a_scale || !b_scale)) return FMSMO_ERR_NULL;
   if (batch <= 0 || M <= 0 || stride_b < N * ldb) return FMSMO_ERR_SHAPE;
   if (batch * stride_b >= (1ll << 40) || batch >= (1 << 20)) return FMSMO_ERR_UNSUPPORTED;
   if (K % 64 || stride_b % 16) return FMSMO_ERR_ALIGN;
@@ -531,7 +532,7 @@ int launch_bmm(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t s
   g.k_rotate = tall ? 5 : 0;
 #define GO(OUT)                                                                             \
   {                                                                                         \
-    EpiDequant<OUT, FMSMO_F32, false, AccT> epi{y, ldy, a_scale, b_scale, bias, 0, 0};      \
+    const EpiScaleBias<OUT, AccT> epi{y, ldy, a_scale, b_scale, bias, sc, sums, parts, zero, batch * N}; \
     if (tall) {                                                                             \
       g.grid_m = (int)batch * div_up(M, 256);                                               \
       launch_rs<OP, true, 128>(g, epi, st);                                                 \
@@ -540,8 +541,9 @@ int launch_bmm(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t s
       launch_tile<TileMid, OP, true>(g, epi, st);                                           \
     } else {                                                                                \
       g.grid_m = (int)batch * div_up(M, 256);                                               \
-      if (K == 128 && use_register_staged(OP)) {                                            \
-        launch_k128<OP>(g, (int)batch, (int)M, EpiScaleBias<OUT, AccT>{y, ldy, a_scale, b_scale, bias}, st); \
+      /* (its output offsets are 32-bit per batch entry) */                                 \
+      if (K == 128 && use_register_staged(OP) && ldy == N && M * N * 4 < (1ll << 31)) {     \
+        launch_k128<OP>(g, (int)batch, (int)M, epi, st);                                    \
       }                                                                                     \
       else if (K % 128 == 0 && use_register_staged(OP)) launch_rs<OP, true>(g, epi, st);    \
       else launch_tile<TileBig, OP, true>(g, epi, st);                                      \

@@ -977,8 +977,25 @@ struct EpiDequant {
   }
 };
 
-// y = acc * (a_scale[0] * w_scale[0]) + bias[n]: the batched matmuls' epilogue, one scale for the
-// whole batch (EpiDequant's fp32-scale arithmetic with nothing to fetch per row).
+// Sum of `parts` partial sums, `stride` apart: eight loads in flight (one after the other, 24 parts took
+// 15 us of a product of one query row; so 9).
+__device__ __forceinline__ int sum_parts(const int32_t* p, int64_t stride, int parts) {
+  int sum = 0;
+  for (int i = 0; i < parts; i += 8) {
+    int v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[min(i + u, parts - 1) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum += i + u < parts ? v[u] : 0;
+  }
+  return sum;
+}
+
+// y = (acc - zero * sum[n]) * (a_scale * w_scale) + bias[n]: the batched matmuls' epilogue, one scale for
+// the whole batch (EpiDequant's fp32-scale arithmetic with nothing to fetch per row).  sums: `parts`
+// partial sums over the reduction of the second operand's codes, [parts][batch * N] (int32 operands
+// only: the zero-point correction of the first one, exact in integers), or NULL.  The scale product
+// is that of two device scalars, or `sc` itself where they are NULL.
 template <int OUT, class AccT>
 struct EpiScaleBias {
   static constexpr bool UNIFORM_ROWS = true;
@@ -988,17 +1005,32 @@ struct EpiScaleBias {
   const float* a_scale;
   const float* w_scale;
   const float* bias;
+  float sc = 1.0f;
+  const int32_t* sums = nullptr;
+  int parts = 0, zero = 0;
+  int64_t part_stride = 0;
   struct Col {
     float b;
+    AccT z;
   };
   struct Row {
     float sc;
   };
   __device__ __forceinline__ Col col(int n, int expert, int N) const {
-    return Col{bias ? bias[(int64_t)expert * N + n] : -0.0f};
+    const int64_t o = (int64_t)expert * N + n;
+    Col c{bias ? bias[o] : -0.0f, 0};
+    if constexpr (std::is_same<AccT, int>::value) {
+      if (sums) {
+        c.z = zero * sum_parts(sums + o, part_stride, parts);
+      }
+    }
+    return c;
   }
-  __device__ __forceinline__ Row row(int) const { return Row{__fmul_rn(a_scale[0], w_scale[0])}; }
-  __device__ __forceinline__ float value(AccT v, Row r, Col c) const { return __fmaf_rn((float)v, r.sc, c.b); }
+  __device__ __forceinline__ Row row(int) const { return Row{a_scale ? __fmul_rn(a_scale[0], w_scale[0]) : sc}; }
+  __device__ __forceinline__ float value(AccT v, Row r, Col c) const {
+    if constexpr (std::is_same<AccT, int>::value) v -= c.z;
+    return __fmaf_rn((float)v, r.sc, c.b);
+  }
   __device__ __forceinline__ void store(int m, int n, AccT v, Row r, Col c) const {
     store_from_f32<OUT>(y, (int64_t)m * ldy + n, value(v, r, c));
   }

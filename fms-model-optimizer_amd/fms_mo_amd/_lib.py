@@ -62,6 +62,9 @@ SIGNATURES = {
     "fmsmo_quant_weight_i8": [_P, _I, _L, _P, _I, _P, _I, _L, _I, _P, _L, _P, _L, _L, _P],
     "fmsmo_absmax_cols": [_P, _I, _L, _L, _L, _P, _P],
     "fmsmo_quant_i8_affine": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _L, _L, _L, _P],
+    "fmsmo_quant_i8_affine_sums": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _P, _L, _L, _L, _P],
+    "fmsmo_bmm_i8_zp": [_P, _L, _P, _L, _L, _F, _I, _P, _I, _P, _I, _L, _L, _L, _L, _L, _P],
+    "fmsmo_bmm_qa_i8": [_P, _I, _L, _L, _F, _F, _I, _P, _L, _L, _F, _P, _I, _P, _L, _L, _L, _L, _L, _P],
     "fmsmo_bmm_i8_dq": [_P, _L, _P, _L, _L, _P, _P, _P, _P, _I, _L, _L, _L, _L, _L, _P],
     "fmsmo_bmm_fp8_dq": [_P, _L, _P, _L, _L, _P, _P, _P, _P, _I, _L, _L, _L, _L, _L, _P],
     "fmsmo_zero_shift_bias": [_P, _L, _P, _L, _P, _F, _P, _I, _P, _L, _L, _P],
@@ -74,6 +77,8 @@ OTHER = {
     "fmsmo_abi_version": ([], c_int),
     "fmsmo_status_str": ([c_int], c_char_p),
     "fmsmo_last_error": ([], c_char_p),
+    "fmsmo_affine_sum_parts": ([c_int64, c_int64, c_int64, c_int], c_int),
+    "fmsmo_bmm_qa_ok": ([c_int, c_int, c_float, c_float, c_int64, c_int64, c_int64, c_int64], c_int),
     "fmsmo_gemm_workspace_bytes": ([c_int64, c_int64, c_int64], c_int64),
     "fmsmo_decode_linear_ok": ([c_int64, c_int64], c_int),
     "fmsmo_decode_linear_f32s_ok": ([c_int64, c_int64], c_int),

@@ -597,21 +597,27 @@ def _batched3(t: torch.Tensor) -> torch.Tensor:
     return t3
 
 
-def quant_i8_affine(x, scale: float, offset: float, compute_dtype=None, transpose=False, pad_to=64):
+def quant_i8_affine(x, scale: float, offset: float, compute_dtype=None, transpose=False, pad_to=64, want_sums=False):
     """int8 codes of x [..., R, C] (see fmsmo_quant_i8_affine) as [batch, R, Cp] or, transposed,
-    [batch, C, Rp]; the last dimension is zero-padded to a multiple of ``pad_to``."""
+    [batch, C, Rp]; the last dimension is zero-padded to a multiple of ``pad_to``.  want_sums: also
+    the int32 sums of the codes along that dimension, [parts, batch, rows] to be added over the parts."""
     _need_gpu(x)
     x3 = _batched3(x)
     B, R, C = x3.shape
     compute_dtype = compute_dtype or x.dtype
     inner = R if transpose else C
     ldq = (inner + pad_to - 1) // pad_to * pad_to
-    q = torch.empty((B, C if transpose else R, ldq), dtype=torch.int8, device=x.device)
+    rows = C if transpose else R
+    q = torch.empty((B, rows, ldq), dtype=torch.int8, device=x.device)
+    sums = None
+    if want_sums:
+        parts = L.load().fmsmo_affine_sum_parts(B, R, C, int(bool(transpose)))
+        sums = torch.empty((parts, B, rows), dtype=torch.int32, device=x.device)
     with _dev(x):
-        L.call("fmsmo_quant_i8_affine", x3.data_ptr(), _dt(x3), x3.stride(1) if R > 1 else C,
+        L.call("fmsmo_quant_i8_affine_sums", x3.data_ptr(), _dt(x3), x3.stride(1) if R > 1 else C,
                x3.stride(0) if B > 1 else R * C, float(scale), float(offset), _DT[compute_dtype],
-               int(bool(transpose)), q.data_ptr(), ldq, q.stride(0), B, R, C, _stream(x))
-    return q
+               int(bool(transpose)), q.data_ptr(), ldq, q.stride(0), _ptr(sums), B, R, C, _stream(x))
+    return (q, sums) if want_sums else q
 
 
 def _bmm(fn, dtype, a, b, a_scale, b_scale, bias, out_dtype):
@@ -642,6 +648,46 @@ def _bmm(fn, dtype, a, b, a_scale, b_scale, bias, out_dtype):
 def bmm_i8_dq(a, b, a_scale, b_scale, bias=None, out_dtype=torch.float16):
     """y [batch,M,N] = (a [batch,M,K] . b [batch,N,K]^T) * a_scale * b_scale + bias [batch,N]."""
     return _bmm("fmsmo_bmm_i8_dq", torch.int8, a, b, a_scale, b_scale, bias, out_dtype)
+
+
+def bmm_i8_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype):
+    """y [batch, M, N] of m1's dtype = dequant(quant(m1) . quant(m2)): both operands quantized with their
+    static parameters (see quant_i8_affine), the zero-point correction of m1 made from the column
+    sums of m2's codes.  m1 [..., M, K], m2 [..., K, N] with equal leading dimensions.  Probabilities x
+    values quantize m1 inside the product (fmsmo_bmm_qa_i8)."""
+    _need_gpu(m1, m2)
+    M, K = m1.shape[-2:]
+    N = m2.shape[-1]
+    a3 = _batched3(m1)
+    B = a3.shape[0]
+    qa = m1.dtype in (torch.float16, torch.bfloat16) and bool(L.load().fmsmo_bmm_qa_ok(
+        _dt(m1), _DT[compute_dtype], scale1, zero1, B, M, N, K))
+    # scores of a head dimension up to 128 run on the kernel for a reduction of exactly 128
+    pad = 128 if K <= 128 and M > 128 and N > 128 else 64
+    if m2.stride(-2) == 1 and m2.shape[-2] > 1:  # a transposed view of a [n, k] tensor
+        q2, sums = quant_i8_affine(m2.transpose(-1, -2), scale2, zero2, compute_dtype, False, pad, want_sums=True)
+    else:
+        q2, sums = quant_i8_affine(m2, scale2, zero2, compute_dtype, True, pad, want_sums=True)
+    y = torch.empty((B, M, N), dtype=m1.dtype, device=m1.device)
+    with _dev(m1):
+        if qa:
+            L.call("fmsmo_bmm_qa_i8", a3.data_ptr(), _dt(a3), a3.stride(1), a3.stride(0) if B > 1 else M * K,
+                   float(scale1), float(zero1), _DT[compute_dtype], q2.data_ptr(), q2.stride(1), q2.stride(0),
+                   float(scale2), sums.data_ptr(), sums.shape[0], y.data_ptr(), N, B, M, N, K, _stream(m1))
+        else:
+            q1 = quant_i8_affine(m1, scale1, zero1, compute_dtype, False, pad)
+            Kp = q1.shape[2]
+            L.call("fmsmo_bmm_i8_zp", q1.data_ptr(), Kp, q2.data_ptr(), Kp, q2.stride(0),
+                   _f32_product(scale1, scale2), int(zero1), sums.data_ptr(), sums.shape[0], y.data_ptr(),
+                   _DT[m1.dtype], N, B, M, N, Kp, _stream(m1))
+    return y
+
+
+def _f32_product(a, b):
+    """a * b rounded to fp32 (the factors are fp32 values)."""
+    import struct
+
+    return struct.unpack("f", struct.pack("f", a * b))[0]
 
 
 def bmm_fp8_dq(a, b, a_scale, b_scale, bias=None, out_dtype=torch.bfloat16):

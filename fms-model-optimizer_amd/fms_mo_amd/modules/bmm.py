@@ -4,8 +4,9 @@ class name, ``from_fms_mo`` signature and buffers (fms_mo/modules/bmm.py:607-748
 The reference's forward still *simulates* the integer product (``torch.matmul`` on the int8 codes
 cast to fp16, "haven't implemented any batched CUTLASS matmul").  Here both operands are quantized
 by one HIP kernel each (m2, stored ``[k, n]``, is written transposed so that its reduction
-dimension becomes contiguous), multiplied on the MFMA units with exact int32 accumulation, and
-dequantized in the GEMM epilogue together with the zero-point correction of the asymmetric m1.
+dimension becomes contiguous; a large m1 -- probabilities x values -- on its way into the product),
+multiplied on the MFMA units with exact int32 accumulation, and dequantized in the GEMM epilogue
+together with the zero-point correction of the asymmetric m1, made in integers.
 The correction is summed over the reduction dimension of every batch entry; the reference's
 ``m2_i8.sum(dim=0)`` is that sum only for a 2-D m2.
 """
@@ -55,18 +56,14 @@ class QBmmINT8Deploy(nn.Module):
             qbmm_int.register_buffer("m2_clip_valn", -Qw.clip_val.detach() * cvn_ext_ratio)
         return qbmm_int.to(target_device)
 
-    # host copies of the four scalars and the device metadata of the correction kernel are made
-    # once (and again when the buffers change dtype or device), so forward never synchronizes
+    # host copies of the four scalars are made once (and again when the buffers change dtype or
+    # device), so forward never synchronizes
     def _scalars(self):
         key = (self.m1_scale.dtype, self.m1_scale.device)
         if getattr(self, "_cache_key", None) != key:
             s1, s2 = float(self.m1_scale), float(self.m2_scale)
             z1, z2 = int(self.m1_zp) - 128, int(self.m2_zp)
-            dev = self.m1_scale.device
             self._host = (s1, z1, s2, z2)
-            self._s1 = torch.tensor([s1], dtype=torch.float32, device=dev)
-            self._s2 = torch.tensor([s2], dtype=torch.float32, device=dev)
-            self._meta = torch.tensor([s1, -float(z1)], dtype=torch.float32, device=dev)
             self._cache_key = key
         return self._host
 
@@ -77,12 +74,15 @@ class QBmmINT8Deploy(nn.Module):
         return (f"nbits_m1,m2={self.num_bits_m1},{self.num_bits_m2}, "
                 f"use_int_kernel={self.use_int_kernel}")
 
+    def _compute_dtype(self, m1):
+        sc = self.m1_scale
+        return torch.promote_types(m1.dtype, sc.dtype) if sc.dim() > 0 else m1.dtype
+
     def quantize_operands(self, m1, m2):
         """int8 codes ready for the batched kernel: m1 as [batch, M, Kp], m2 as [batch, N, Kp]
         (Kp = K rounded up to 64, zero-filled)."""
         s1, z1, s2, z2 = self._scalars()
-        sc = self.m1_scale
-        T = torch.promote_types(m1.dtype, sc.dtype) if sc.dim() > 0 else m1.dtype
+        T = self._compute_dtype(m1)
         q1 = kernels.quant_i8_affine(m1, s1, z1, T, transpose=False)
         if m2.stride(-2) == 1 and m2.shape[-2] > 1:  # a transposed view of a [n, k] tensor
             q2 = kernels.quant_i8_affine(m2.transpose(-1, -2), s2, z2, T, transpose=False)
@@ -97,11 +97,8 @@ class QBmmINT8Deploy(nn.Module):
         if m1.shape[:-2] != m2.shape[:-2] or m1.shape[-1] != m2.shape[-2]:
             raise ValueError(f"incompatible operands {tuple(m1.shape)} @ {tuple(m2.shape)}")
         with torch.no_grad():
-            q1, q2 = self.quantize_operands(m1, m2)
-            B, N, Kp = q2.shape
-            corr = kernels.zero_shift_bias(q2.view(B * N, Kp), self._s2, self._meta, bias=None,
-                                           offset=0.0)
-            y = kernels.bmm_i8_dq(q1, q2, self._s1, self._s2, bias=corr, out_dtype=m1.dtype)
+            s1, z1, s2, z2 = self._scalars()
+            y = kernels.bmm_i8_quantized(m1, m2, s1, z1, s2, z2, self._compute_dtype(m1))
         return y.reshape(*m1.shape[:-1], m2.shape[-1])
 
 

@@ -639,6 +639,17 @@ int fmsmo_quant_i8_affine(const void* x, int x_dtype, int64_t ldx, int64_t strid
                           float offset, int compute_dtype, int transpose, int8_t* q, int64_t ldq,
                           int64_t stride_q, int64_t batch, int64_t R, int64_t C,
                           fmsmo_stream_t stream);
+/*
+ * The same with the sums of the codes along the last dimension of q, for the zero-point correction of
+ * the matmul: sums int32 [parts][batch][rows of q] (NULL: not wanted), the correction uses the sum over
+ * the parts.  parts = fmsmo_affine_sum_parts(batch, R, C, transpose) (host only).  x only needs the
+ * alignment of its elements.
+ */
+int fmsmo_affine_sum_parts(int64_t batch, int64_t R, int64_t C, int transpose);
+int fmsmo_quant_i8_affine_sums(const void* x, int x_dtype, int64_t ldx, int64_t stride_x, float scale,
+                               float offset, int compute_dtype, int transpose, int8_t* q, int64_t ldq,
+                               int64_t stride_q, int32_t* sums, int64_t batch, int64_t R, int64_t C,
+                               fmsmo_stream_t stream);
 
 /*
  * y[b] = ( a[b] . b[b]^T ) * (a_scale[0] * b_scale[0]) + bias[b][n]      for b in [0, batch)
@@ -660,6 +671,27 @@ int fmsmo_bmm_fp8_dq(const uint8_t* a, int64_t lda, const uint8_t* b, int64_t ld
                      int64_t stride_b, const float* a_scale, const float* b_scale,
                      const float* bias, void* y, int y_dtype, int64_t ldy, int64_t batch,
                      int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream);
+/*
+ * y[b] = ( a[b] . b[b]^T - zero * sums[b][n] ) * scale: the int8 product with the zero-point correction of
+ * an asymmetric first operand made in integers from the sums that fmsmo_quant_i8_affine_sums left
+ * (operands as for fmsmo_bmm_i8_dq).
+ */
+int fmsmo_bmm_i8_zp(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, int64_t stride_b,
+                    float scale, int zero, const int32_t* sums, int parts, void* y, int y_dtype,
+                    int64_t ldy, int64_t batch, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream);
+/*
+ * The same product with the first operand quantized on its way into the kernel (probabilities x
+ * values: x is read once and its codes never reach memory): x [batch][M][K] fp16 / bf16 with row stride
+ * ldx and batch stride stride_x in elements, quantized like fmsmo_quant_i8_affine with (scale, offset),
+ * b the codes of the second operand, [batch][N][ldb] zero-padded past K (stride_b = N * ldb or more);
+ * y [batch * M][N] of x's dtype.  fmsmo_bmm_qa_ok tells the shapes and scales it serves.
+ */
+int fmsmo_bmm_qa_ok(int x_dtype, int compute_dtype, float scale, float offset, int64_t batch, int64_t M,
+                    int64_t N, int64_t K);
+int fmsmo_bmm_qa_i8(const void* x, int x_dtype, int64_t ldx, int64_t stride_x, float scale, float offset,
+                    int compute_dtype, const int8_t* b, int64_t ldb, int64_t stride_b, float b_scale,
+                    const int32_t* sums, int parts, void* y, int64_t ldy, int64_t batch, int64_t M,
+                    int64_t N, int64_t K, fmsmo_stream_t stream);
 
 #ifdef __cplusplus
 }

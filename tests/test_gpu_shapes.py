@@ -115,3 +115,46 @@ def test_fp8_per_tensor_quantizer_in_two_passes(dev, dtype, M, Kd, pad):
             if special is not None and special != special and variant != L.FP8_LINEAR:
                 continue  # a NaN abs-max: every torch code is NaN; both forms keep the floor as scale, only one clamps
             assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8)), (special, variant)
+
+
+def make_qbmm(dev, lo, hi, other, dtype):
+    import types
+
+    from fms_mo_amd.modules.bmm import QBmmINT8Deploy
+
+    one = lambda v: torch.tensor([v], dtype=dtype)
+    src = types.SimpleNamespace(num_bits_m1=8, num_bits_m2=8, qm1_mode="max",
+                                quantize_m1=types.SimpleNamespace(clip_val=one(hi), clip_valn=one(lo), num_bits=8),
+                                quantize_m2=types.SimpleNamespace(clip_val=one(other), num_bits=8))
+    return QBmmINT8Deploy.from_fms_mo(src, target_device=dev)
+
+
+@pytest.mark.parametrize("xdt,sdt", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
+                                     (torch.float16, torch.float32), (torch.bfloat16, torch.float32),
+                                     (torch.float32, torch.float32)])
+@pytest.mark.parametrize("B,M,Kd,N,view", [
+    (32, 64, 256, 64, False),     # the smallest product that quantizes m1 on the way
+    (33, 130, 300, 80, False), (32, 129, 1001, 128, False), (40, 100, 383, 1, False),   # ragged rows, slabs, columns
+    (2, 70, 513, 128, False), (3, 1, 77, 96, False),                                    # two launches
+    (5, 200, 64, 300, True), (2, 131, 80, 129, True), (4, 1, 128, 500, True)])          # scores
+def test_attention_products(dev, xdt, sdt, B, M, Kd, N, view):
+    """QBmmINT8Deploy against the exact product of its own codes: integers (sums with the zero-point
+    correction) times the fp32 scale product, one fp32 rounding each of sum and product, then the
+    output's: at most the output's half ulp plus 2^-23.  Infinite and NaN elements of m1 quantize as in the
+    stand-alone quantizer."""
+    m = make_qbmm(dev, -0.7 if view else 0.0, 1.0, 3.0, sdt)
+    m1 = torch.randn(B, M, Kd, generator=gen(B + M)).to(xdt)
+    if not view:
+        m1 = torch.softmax(m1.float() * 2, -1).to(xdt)
+    m1[0, 0, 0], m1[-1, -1, -1], m1[B // 2, M // 2, Kd // 2] = float("inf"), float("nan"), -float("inf")
+    m2 = torch.randn(B, N, Kd, generator=gen(N)).to(xdt).to(dev).transpose(-1, -2) if view else \
+        torch.randn(B, Kd, N, generator=gen(N)).to(xdt).to(dev)
+    m1 = m1.to(dev)
+    y = m(m1, m2)
+    q1, q2 = m.quantize_operands(m1, m2)
+    s1, z1, s2, _ = m._scalars()
+    exact = torch.matmul(q1[..., :Kd].double() - z1, q2[..., :Kd].double().transpose(1, 2).contiguous())
+    exact = exact * float(torch.tensor(s1) * torch.tensor(s2))
+    assert y.shape == exact.shape and y.dtype == xdt
+    ulp = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}[xdt]
+    assert ((y.double() - exact).abs() <= exact.abs() * (ulp + 2.0 ** -22) + 2.0 ** -25).all()
