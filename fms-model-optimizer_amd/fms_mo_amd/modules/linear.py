@@ -79,6 +79,16 @@ def _quantize_weight_rows(weight, smoothq_scale, w_scale):
     return w.to(torch.int).to(torch.int8)
 
 
+def _weight_column_max(w):
+    """max_n |W| as [1, K] in the weights' dtype.  16-bit weights on the GPU take the column abs-max
+    kernel (one pass over W; a magnitude is exact in fp32 and back, NaN stays), others the torch
+    expression."""
+    if (w.is_cuda and w.dtype in (torch.float16, torch.bfloat16) and w.is_contiguous() and w.numel()
+            and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0):
+        return kernels.absmax_cols(w.detach()).to(w.dtype).unsqueeze(0)
+    return w.abs().max(dim=0, keepdim=True)[0]
+
+
 def _compute_dtype(x_dtype, smooth):
     return x_dtype if smooth is None else torch.promote_types(x_dtype, smooth.dtype)
 
@@ -360,27 +370,31 @@ class QLinearINT8Deploy(nn.Linear):
         with torch.no_grad():
             Qa, Qw = fms_mo_qlinear.quantize_feature, fms_mo_qlinear.quantize_weight
             if kwargs.get("recalc_clipvals", True):
-                Qw(fms_mo_qlinear.weight)
+                if isinstance(Qw, Qmax):
+                    Qw.observe(fms_mo_qlinear.weight)
+                else:
+                    Qw(fms_mo_qlinear.weight)
             w_cv = Qw.clip_val
-            a_cv = getattr(Qa, "clip_val", torch.tensor(8.0, device=src_dev))
-            a_cvn = getattr(Qa, "clip_valn", torch.tensor(-8.0, device=src_dev))
+            # (constants by fill kernels: torch.tensor(..., device=...) copies from the host and waits)
+            a_cv = Qa.clip_val if hasattr(Qa, "clip_val") else torch.full((), 8.0, device=src_dev)
+            a_cvn = Qa.clip_valn if hasattr(Qa, "clip_valn") else torch.full((), -8.0, device=src_dev)
             m.cvs = [a_cv, a_cvn, w_cv]
-            smoothq_scale = torch.tensor([1.0], device=src_dev, dtype=w_dtype)
+            smoothq_scale = torch.ones(1, device=src_dev, dtype=w_dtype)
             if getattr(fms_mo_qlinear, "smoothq", False):
                 a_s = fms_mo_qlinear.smoothq_act_scale
-                w_s = fms_mo_qlinear.weight.abs().max(dim=0, keepdim=True)[0].clamp(min=1e-5)
                 alpha = fms_mo_qlinear.smoothq_alpha
                 if torch.all(a_s != 0).item():
+                    w_s = _weight_column_max(fms_mo_qlinear.weight).clamp(min=1e-5)
                     smoothq_scale = (a_s**alpha / w_s ** (1.0 - alpha)).clamp(min=1e-5).to(a_s.dtype)
-            input_scale = torch.tensor(1.0, device=src_dev)
+            input_scale = torch.ones((), device=src_dev)
             # tensor divisor: keeps the IEEE quotient on the GPU as well (see prepare_deploy_weights)
-            w_scale = w_cv * 2 / torch.tensor(float(w_levels), device=w_cv.device, dtype=w_cv.dtype)
+            w_scale = w_cv * 2 / torch.full((), float(w_levels), device=w_cv.device, dtype=w_cv.dtype)
             m.use_fake_zero_shift = False
             if m.useDynMaxQfunc in [-1, -2]:
-                input_zero_point = torch.tensor(128 - m.useSymAct, device=src_dev)
+                input_zero_point = torch.full((), 128 - m.useSymAct, device=src_dev, dtype=torch.int)
             elif 0 < m.useDynMaxQfunc < 65:
                 m.use_fake_zero_shift = True
-                input_zero_point = torch.tensor(m.useDynMaxQfunc, device=src_dev)
+                input_zero_point = torch.full((), m.useDynMaxQfunc, device=src_dev)
             elif m.usePTnativeQfunc:
                 input_scale = torch.tensor([(a_cv - a_cvn) / a_levels], device=src_dev)
                 input_zero_point = torch.round(-a_cvn / input_scale)
@@ -406,7 +420,7 @@ class QLinearINT8Deploy(nn.Linear):
                 Qw.dequantize = False
                 w_int8 = Qw(fms_mo_qlinear.weight.float() * smoothq_scale).to(torch.int)
             else:
-                w_int8 = _quantize_weight_rows(fms_mo_qlinear.weight, smoothq_scale, w_scale).to(torch.int)
+                w_int8 = _quantize_weight_rows(fms_mo_qlinear.weight, smoothq_scale, w_scale)
             m.weight = nn.Parameter(w_int8.to(torch.int8), requires_grad=False)
             if m.useSymAct:
                 corr_term_int = 0

@@ -158,3 +158,53 @@ def test_attention_products(dev, xdt, sdt, B, M, Kd, N, view):
     assert y.shape == exact.shape and y.dtype == xdt
     ulp = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}[xdt]
     assert ((y.double() - exact).abs() <= exact.abs() * (ulp + 2.0 ** -22) + 2.0 ** -25).all()
+
+
+@pytest.mark.parametrize("wdt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("smooth", [False, True])
+@pytest.mark.parametrize("N,Kd", [(1, 8), (3, 16), (4, 2040), (5, 2048), (130, 2056), (7, 4104)])
+def test_weight_quantizer_with_fp32_divisors(dev, wdt, smooth, N, Kd):
+    """The short exact quotient against the IEEE one: ties (integers and halves times the divisor), codes
+    past the range, infinities, NaN (code -127), zeros, and rows whose divisor leaves the range it serves."""
+    g = gen(N * Kd)
+    w = 0.05 * torch.randn(N, Kd, generator=g)
+    c = 2.0 ** torch.randint(-12, 3, (N,), generator=g).float() * (1 + (torch.rand(N, generator=g) > 0.5) * torch.rand(N, generator=g))
+    half = torch.arange(Kd) % 300 - 150
+    w[::2] = 0.5 * half * c[::2, None]
+    w[-1, :8] = torch.tensor([float("inf"), -float("inf"), float("nan"), 0.0, -0.0, 6e4, -6e4, 1e-7])
+    if N > 4:
+        c[0], c[1], c[2], c[3] = 1e-38, 0.0, -0.01, float("inf")
+    w = w.to(wdt)
+    s = 0.25 + 4 * torch.rand(Kd, generator=g) if smooth else None
+    t = w.float() * s if smooth else w.float()
+    ref = torch.nan_to_num((t / c[:, None]).round().clamp(-127, 127), nan=-127.0).to(torch.int8)
+    q, rows = K().quant_weight_i8(w.to(dev), c.to(dev), s.to(dev) if smooth else None, mode="div", want_row_sum=True)
+    assert torch.equal(q.cpu(), ref)
+    assert torch.equal(rows.cpu(), ref.int().sum(1, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_conversion_in_eval_and_training_mode(dev, dtype):
+    """from_fms_mo leaves the weight quantizer as a forward on the weights would, and its buffers equal those of
+    the torch expressions evaluated on the same GPU."""
+    import copy
+
+    from fms_mo_amd.modules.linear import QLinearINT8Deploy
+
+    for train in (False, True):
+        m = make_qlinear(264, 37, dtype).to(dev)
+        m.smoothq, m.smoothq_alpha = True, torch.full((1,), 0.5, device=dev)
+        m.smoothq_act_scale = 0.5 + torch.rand(264, generator=gen(3)).to(dev)
+        m.quantize_weight.train(train)
+        other = copy.deepcopy(m)
+        dep = QLinearINT8Deploy.from_fms_mo(m, use_dynamic_max_act_Qfunc=-1)
+        with torch.no_grad():
+            other.quantize_weight(other.weight)
+        a, b = m.quantize_weight, other.quantize_weight
+        assert a.Niter == b.Niter and torch.equal(a.clip_val, b.clip_val) and torch.equal(a.clip_valn, b.clip_valn)
+        ws = b.clip_val * 2 / torch.tensor(254.0, device=dev)
+        wm = other.weight.detach().abs().max(dim=0, keepdim=True)[0].clamp(min=1e-5)
+        sq = (m.smoothq_act_scale ** m.smoothq_alpha / wm ** (1.0 - m.smoothq_alpha)).clamp(min=1e-5)
+        codes = ((other.weight.detach() * sq).t() / ws).round().clamp(-127, 127).t().to(torch.int8)
+        assert torch.equal(dep.w_scale, ws) and torch.equal(dep.smoothq_scale, sq) and torch.equal(dep.weight, codes)
+        assert dep.input_zp.dtype == torch.int32 and int(dep.input_zp) == 127 and dep.corr_term.abs().max() == 0
