@@ -198,16 +198,19 @@ def quant_act_fp8_dynamic(x, variant=L.FP8_LINEAR, per_tensor=False, scale_floor
     M, K = x.shape
     q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=x.device)
     scale = torch.empty((1 if per_tensor else M,), dtype=torch.float32, device=x.device)
+    # (fmsmo_quant_act_fp8_tensor counts 8-element chunks in 31 bits; larger tensors take column maxima)
+    tensor_call = per_tensor and 0 < M * K < 1 << 34
+    col_amax = absmax_cols(x) if per_tensor and not tensor_call else None
     with _dev(x):
-        if per_tensor and M > 0:
+        if tensor_call:
             parts = torch.empty((256,), dtype=torch.float32, device=x.device)
             L.call("fmsmo_quant_act_fp8_tensor", x.data_ptr(), _dt(x), _ld(x), int(variant), float(scale_floor),
                    _dt(x) if scale_in_x_dtype else L.F32, parts.data_ptr(), q.data_ptr(), K, scale.data_ptr(),
                    M, K, _stream(x))
         else:
-            L.call("fmsmo_quant_act_fp8_dynamic", x.data_ptr(), _dt(x), _ld(x), int(variant), 0, None,
-                   float(scale_floor), _dt(x) if scale_in_x_dtype else L.F32, q.data_ptr(), K,
-                   scale.data_ptr(), M, K, _stream(x))
+            L.call("fmsmo_quant_act_fp8_dynamic", x.data_ptr(), _dt(x), _ld(x), int(variant),
+                   int(bool(per_tensor)), _ptr(col_amax), float(scale_floor),
+                   _dt(x) if scale_in_x_dtype else L.F32, q.data_ptr(), K, scale.data_ptr(), M, K, _stream(x))
     return q, scale
 
 
