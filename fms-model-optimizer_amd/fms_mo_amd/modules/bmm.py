@@ -98,7 +98,15 @@ class QBmmINT8Deploy(nn.Module):
             raise ValueError(f"incompatible operands {tuple(m1.shape)} @ {tuple(m2.shape)}")
         with torch.no_grad():
             s1, z1, s2, z2 = self._scalars()
-            y = kernels.bmm_i8_quantized(m1, m2, s1, z1, s2, z2, self._compute_dtype(m1))
+            if (abs(z1) + 128) * 128 * m1.shape[-1] < 1 << 31:
+                y = kernels.bmm_i8_quantized(m1, m2, s1, z1, s2, z2, self._compute_dtype(m1))
+            else:  # the corrected sum might leave 32 bits: corrected in fp32 behind the product
+                q1, q2 = self.quantize_operands(m1, m2)
+                B, N, Kp = q2.shape
+                one = lambda v: torch.full((1,), v, dtype=torch.float32, device=m1.device)  # noqa: E731
+                corr = kernels.zero_shift_bias(q2.view(B * N, Kp), one(s2), torch.cat((one(s1), one(-float(z1)))),
+                                               bias=None, offset=0.0)
+                y = kernels.bmm_i8_dq(q1, q2, one(s1), one(s2), bias=corr, out_dtype=m1.dtype)
         return y.reshape(*m1.shape[:-1], m2.shape[-1])
 
 

@@ -173,6 +173,15 @@ def test_attention_products(dev, xdt, sdt, B, M, Kd, N, view):
     assert ((y.double() - exact).abs() <= exact.abs() * (ulp + 2.0 ** -22) + 2.0 ** -25).all()
 
 
+@pytest.mark.parametrize("Kd", [65664, 70016])  # 256 * 128 * K on either side of 2^31: 65536
+def test_attention_product_whose_corrected_sum_leaves_32_bits(dev, Kd):
+    """Codes 127 with zero point -128 against codes 127: 255 * 127 * K is beyond 2^31 from K = 66311 on.
+    The correction in fp32 costs two roundings of terms twice the result."""
+    m = make_qbmm(dev, 0.0, 1.0, 3.0, torch.float32)
+    m1, m2 = torch.ones(1, 3, Kd, device=dev), torch.full((1, Kd, 5), 3.0, device=dev)
+    assert ((m(m1, m2).double() / (3.0 * Kd) - 1).abs() < 2e-6).all()
+
+
 @pytest.mark.parametrize("wdt", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("smooth", [False, True])
 @pytest.mark.parametrize("N,Kd", [(1, 8), (3, 16), (4, 2040), (5, 2048), (130, 2056), (7, 4104)])
