@@ -337,7 +337,7 @@ inline bool cut_slices(SplitPlan& p, int64_t M, int64_t N, int64_t K, int s) {
 
 // `limit` > 0: the workspace at hand; a plan that needs more is passed over for the next one (the
 // register-staged slices need more partial sums than the 128 x 128 ones: more, shorter slices).
-inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0) {
+inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0, bool fp8 = false) {
   SplitPlan p{1, K, 0, false};
   static const char* off = getenv("FMSMO_SPLIT_K");  // FMSMO_SPLIT_K=0 disables (tuning aid)
   if (off && off[0] == '0') return p;
@@ -356,10 +356,17 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   // 27.7, and below 384 rows their 256-row tiles are half empty)
   if (K >= 8192 && M >= 384 && use_register_staged(0)) {
     const int64_t t = (int64_t)div_up(M, 256) * div_up(N, 128);
-    // a full round of 128 x 128 tiles runs faster in one pass with 128-byte stages than as two
-    // slices (1024 x 4096, us: K = 8192 53.4 -> 42.6, K = 14336 80.0 -> 72.5)
-    const bool full_round = (int64_t)div_up(M, TileMidK::BM) * div_up(N, TileMidK::BN) == 256;
-    if (t <= 128 && !full_round) {
+    // 129 .. 256 tiles of 128 x 128 fill most of a round of the compute units in one pass with 128-byte
+    // stages, without partial sums.  e4m3 is faster so throughout; int8 where the round is nearly full
+    // or K short, else only with the weights in the last-level cache (us with weights from HBM, slices ->
+    // one pass, int8 | e4m3: 777 x 4096 x 12800, 224 tiles, 64.1 -> 52.5 | 74.3 -> 53.0; 896 x 4096 x 14336,
+    // 224, 68.0 -> 65.0 | 81.2 -> 65.1; 700 x 4096 x 8192, 192, 40.5 -> 32.8 | 48.8 -> 33.0; 1000 x 2304 x
+    // 9216, 144, 36.3 -> 30.2 | 42.1 -> 31.8; 640 x 4096 x 14336, 160, 60.1 -> 64.4 | 73.5 -> 67.5; 640 x 5120
+    // x 13824, 200, 63.6 -> 68.2 | 76.1 -> 68.4; 600 x 4352 x 11008, 170, 48.5 -> 52.1 | 58.8 -> 51.3;
+    // 1024 x 4096 x 14336, 256, 80.0 -> 72.5)
+    const int64_t t128 = (int64_t)div_up(M, TileMidK::BM) * div_up(N, TileMidK::BN);
+    if (t128 > 128 && t128 <= 256 && (fp8 || t128 >= 224 || K <= 9216)) return p;
+    if (t <= 128) {
       int s = (int)(256 / t);
       while (s > 1 && (K % (s * 128) != 0 || K / s < 512)) --s;
       if (s >= 2 && (limit <= 0 || (int64_t)s * M * N * 4 <= limit)) {

@@ -91,7 +91,7 @@ class FP8Linear(nn.Module):
                     raise NotImplementedError("static activation scales are per tensor")
                 q, s = kernels.quant_act_fp8_pertoken(x2, L.FP8_LINEAR, static_scale=self.input_scale.float())
             elif act["strategy"] == "tensor":
-                # column abs-max and quantizer: two passes over x, the scale never leaves the device
+                # abs-max and quantizer: two passes over x, the scale never leaves the device
                 q, s = kernels.quant_act_fp8_dynamic(x2, L.FP8_LINEAR, True, self.dynamic_scale_floor,
                                                      self.dynamic_scale_in_input_dtype)
             elif self.dynamic_scale_floor != 1e-12 or self.dynamic_scale_in_input_dtype:

@@ -230,3 +230,19 @@ def test_conversion_in_eval_and_training_mode(dev, dtype):
         codes = ((other.weight.detach() * sq).t() / ws).round().clamp(-127, 127).t().to(torch.int8)
         assert torch.equal(dep.w_scale, ws) and torch.equal(dep.smoothq_scale, sq) and torch.equal(dep.weight, codes)
         assert dep.input_zp.dtype == torch.int32 and int(dep.input_zp) == 127 and dep.corr_term.abs().max() == 0
+
+
+@pytest.mark.parametrize("M,N,Kd", [(385, 4100, 8192), (769, 4090, 12800), (1024, 2176, 9216), (641, 5000, 8320)])
+def test_most_of_a_round_of_tiles_in_one_pass(dev, M, N, Kd):
+    """129 .. 256 tiles of 128 x 128 and a long reduction, ragged edges included: int8 exact, e4m3 exact on
+    small integers (sums below 2^24)."""
+    kn = K()
+    assert kn.gemm_plan(M, N, Kd, with_workspace=True)[1:] == (128, 128, 1)
+    g = torch.Generator(device=dev).manual_seed(M)
+    a = torch.randint(-128, 128, (M, Kd), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-128, 128, (N, Kd), generator=g, dtype=torch.int8, device=dev)
+    assert torch.equal(kn.gemm_i8_i32(a, w), (a.double() @ w.double().t()).to(torch.int32))
+    a, w = a.float().div(32).round(), w.float().div(32).round()
+    one = torch.ones(1, device=dev)
+    y = kn.gemm_fp8_dq(a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn), one, one, None, out_dtype=torch.float32)
+    assert torch.equal(y, (a.double() @ w.double().t()).float())
