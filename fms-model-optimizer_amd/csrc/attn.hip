@@ -244,7 +244,8 @@ __global__ __launch_bounds__(256) void quant_i8_affine_kernel(const void* __rest
 // `tiles` tiles of 64 x 64 in LDS, the next one in flight; a thread owns 4 x 4 elements, turns them in
 // registers and writes four words (rows of 76 bytes in LDS: at most two lanes per bank).
 // sums[part][b][c]: the block's share of the column sums (added up where they are used: no atomics,
-// nothing to clear).
+// nothing to clear).  A block whose rows all lie past R (ldq may be padded beyond the last 64 rows of data)
+// has no part: fmsmo_affine_sum_parts counts the blocks that begin inside R.
 template <int XT>
 struct Raw4 {
   uint32_t w[XT == FMSMO_F32 ? 4 : 2];
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(256) void quant_i8_affine_t_kernel(const void* __re
 #pragma unroll
     for (int i = 0; i < 4; ++i) cur[i] = nxt[i];
   }
-  if (sums) {
+  if (sums && t0 * 64 < R) {
     sum += __shfl_xor(sum, 1, 64);
     sum += __shfl_xor(sum, 2, 64);
     if (chunk == 0 && c0 + oc < C) sums[((size_t)blockIdx.x * gridDim.z + blockIdx.z) * C + c0 + oc] = sum;

@@ -642,8 +642,8 @@ int fmsmo_quant_i8_affine(const void* x, int x_dtype, int64_t ldx, int64_t strid
 /*
  * The same with the sums of the codes along the last dimension of q, for the zero-point correction of
  * the matmul: sums int32 [parts][batch][rows of q] (NULL: not wanted), the correction uses the sum over
- * the parts.  parts = fmsmo_affine_sum_parts(batch, R, C, transpose) (host only).  x only needs the
- * alignment of its elements.
+ * the parts.  parts = fmsmo_affine_sum_parts(batch, R, C, transpose) (host only), whatever ldq is: what pads a
+ * row of q adds nothing to its sum and no part to the sums.  x only needs the alignment of its elements.
  */
 int fmsmo_affine_sum_parts(int64_t batch, int64_t R, int64_t C, int transpose);
 int fmsmo_quant_i8_affine_sums(const void* x, int x_dtype, int64_t ldx, int64_t stride_x, float scale,

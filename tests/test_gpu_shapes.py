@@ -246,3 +246,45 @@ def test_most_of_a_round_of_tiles_in_one_pass(dev, M, N, Kd):
     one = torch.ones(1, device=dev)
     y = kn.gemm_fp8_dq(a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn), one, one, None, out_dtype=torch.float32)
     assert torch.equal(y, (a.double() @ w.double().t()).float())
+
+
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,R,C,ldq", [
+    (5, 64, 300, 128), (32, 64, 2048, 128), (3, 40, 131, 128), (2, 1, 5, 64), (1, 65, 64, 128),
+    (2, 130, 70, 512),            # several blocks past the data
+    (32, 300, 2048, 320), (32, 250, 2048, 448), (24, 700, 2100, 1024)])   # several tiles per block
+def test_column_sums_of_a_padded_transposed_operand(dev, xdt, B, R, C, ldq):
+    """The sums of the transposing quantizer fill fmsmo_affine_sum_parts parts and nothing behind them, however
+    far ldq is padded; rows of q past R are zero."""
+    from fms_mo_amd import _lib as L
+
+    kn, lib = K(), L.load()
+    x = (2 * torch.randn(B, R, C, generator=gen(R + C))).to(xdt).to(dev)
+    parts = lib.fmsmo_affine_sum_parts(B, R, C, 1)
+    guard = 4 * B * C
+    sums = torch.full((parts * B * C + guard,), 0x5a5a5a5a, dtype=torch.int32, device=dev)
+    q = torch.full((B, C, ldq), 99, dtype=torch.int8, device=dev)
+    dt = kn._dt(x)
+    assert lib.fmsmo_quant_i8_affine_sums(x.data_ptr(), dt, C, R * C, 0.03125, 3.0, dt, 1, q.data_ptr(), ldq, C * ldq,
+                                          sums.data_ptr(), B, R, C, torch.cuda.current_stream().cuda_stream) == 0
+    ref = (x / 0.03125 + 3.0).round().clamp(-128, 127).to(torch.int8).transpose(1, 2)
+    assert torch.equal(q[..., :R], ref) and not q[..., R:].any()
+    assert torch.equal(sums[:parts * B * C].view(parts, B, C).sum(0), ref.sum(-1, dtype=torch.int32))
+    assert (sums[parts * B * C:] == 0x5a5a5a5a).all()
+
+
+@pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Kd", [16, 40, 64, 72, 128])
+def test_attention_scores_of_a_stored_second_operand(dev, xdt, Kd):
+    """Scores whose second operand is stored [k, n]: its codes are padded to the 128 of the kernel for short
+    reductions, beyond the data's last 64 rows for head dimensions up to 64."""
+    m = make_qbmm(dev, -0.7, 1.0, 3.0, xdt)
+    m1 = torch.randn(3, 140, Kd, generator=gen(Kd)).to(xdt).to(dev)
+    m2 = torch.randn(3, Kd, 300, generator=gen(Kd + 1)).to(xdt).to(dev)
+    y = m(m1, m2)
+    assert torch.equal(y, m(m1, m2.transpose(1, 2).contiguous().transpose(1, 2)))
+    q1, q2 = m.quantize_operands(m1, m2)
+    s1, z1, s2, _ = m._scalars()
+    exact = torch.matmul(q1[..., :Kd].double() - z1, q2[..., :Kd].double().transpose(1, 2).contiguous()) * (s1 * s2)
+    ulp = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[xdt]
+    assert ((y.double() - exact).abs() <= exact.abs() * (ulp + 2.0 ** -22) + 2.0 ** -25).all()
