@@ -355,6 +355,12 @@ __global__ __launch_bounds__(256) void quant_i8_affine_t_kernel(const void* __re
   }
 }
 
+// sums[0][i] += sums[1 .. parts - 1][i]
+__global__ __launch_bounds__(256) void add_parts_kernel(int32_t* sums, int parts, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) sums[i] = sum_parts(sums + i, n, parts);
+}
+
 // ------------------------------------------------- product with the first operand quantized on the way
 // y[b] = dequant( quant(x[b]) . q2[b]^T ): probabilities x values.  x [M, K] is 16-bit and by far the largest
 // operand; quantized by a kernel of its own it is read once, its codes written and read again (2 + 1 + 1
@@ -511,6 +517,15 @@ extern "C" int fmsmo_affine_sum_parts(int64_t batch, int64_t R, int64_t C, int t
   if (!transpose || R <= 0 || C <= 0 || batch <= 0) return 1;
   const int64_t total = (R + 63) / 64, tiles = affine_t_tiles(batch, R, C);
   return (int)((total + tiles - 1) / tiles);
+}
+
+extern "C" int fmsmo_affine_add_parts(int32_t* sums, int parts, int64_t n, fmsmo_stream_t stream) {
+  if (!sums) return FMSMO_ERR_NULL;
+  if (parts < 1 || n <= 0 || n > (1ll << 38)) return FMSMO_ERR_SHAPE;
+  if (parts > 1)
+    hipLaunchKernelGGL(add_parts_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, sums,
+                       parts, n);
+  return fmsmo_check_launch();
 }
 
 extern "C" int fmsmo_quant_i8_affine_sums(const void* x, int x_dtype, int64_t ldx, int64_t stride_x, float scale,

@@ -537,24 +537,34 @@ int launch_bmm(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t s
   // they sweep K together (K = 14336: 205 -> 255 us when staggered).
   const bool tall = N > 64 && N <= 128 && M >= 256 && K % 128 == 0 && K >= 512 && use_register_staged(OP);
   g.k_rotate = tall ? 5 : 0;
-#define GO(OUT)                                                                             \
-  {                                                                                         \
-    const EpiScaleBias<OUT, AccT> epi{y, ldy, a_scale, b_scale, bias, sc, sums, parts, zero, batch * N}; \
-    if (tall) {                                                                             \
-      g.grid_m = (int)batch * div_up(M, 256);                                               \
-      launch_rs<OP, true, 128>(g, epi, st);                                                 \
-    } else if (mid) {                                                                       \
-      g.grid_m = (int)batch * div_up(M, TileMid::BM);                                       \
-      launch_tile<TileMid, OP, true>(g, epi, st);                                           \
-    } else {                                                                                \
-      g.grid_m = (int)batch * div_up(M, 256);                                               \
-      /* (its output offsets are 32-bit per batch entry) */                                 \
-      if (K == 128 && use_register_staged(OP) && ldy == N && M * N * 4 < (1ll << 31)) {     \
-        launch_k128<OP>(g, (int)batch, (int)M, epi, st);                                    \
-      }                                                                                     \
-      else if (K % 128 == 0 && use_register_staged(OP)) launch_rs<OP, true>(g, epi, st);    \
-      else launch_tile<TileBig, OP, true>(g, epi, st);                                      \
-    }                                                                                       \
+  // (the kernel for a reduction of 128 has 32-bit output offsets per batch entry)
+  const bool k128 = !tall && !mid && K == 128 && use_register_staged(OP) && M * ldy * 4 < (1ll << 31);
+  auto run = [&](const auto& epi) {
+    if (tall) {
+      g.grid_m = (int)batch * div_up(M, 256);
+      launch_rs<OP, true, 128>(g, epi, st);
+    } else if (mid) {
+      g.grid_m = (int)batch * div_up(M, TileMid::BM);
+      launch_tile<TileMid, OP, true>(g, epi, st);
+    } else {
+      g.grid_m = (int)batch * div_up(M, 256);
+      if (K % 128 == 0 && use_register_staged(OP)) launch_rs<OP, true>(g, epi, st);
+      else launch_tile<TileBig, OP, true>(g, epi, st);
+    }
+  };
+#define GO(OUT)                                                                                          \
+  {                                                                                                      \
+    const EpiScaleBias<OUT, AccT> sb{y, ldy, a_scale, b_scale, bias, sc, sums, parts, zero, batch * N};  \
+    if (k128) {                                                                                          \
+      g.grid_m = (int)batch * div_up(M, 256);                                                            \
+      launch_k128<OP>(g, (int)batch, (int)M, sb, st);                                                    \
+    } else if constexpr (OP == MMA_I8) {                                                                 \
+      if (sums && parts > 1) run(sb);                                                                    \
+      else if (sums) run(EpiZeroPoint<OUT>{y, ldy, sc, sums, zero});                                     \
+      else run(EpiDequant<OUT, FMSMO_F32, false, AccT>{y, ldy, a_scale, b_scale, bias, 0, 0});           \
+    } else {                                                                                             \
+      run(EpiDequant<OUT, FMSMO_F32, false, AccT>{y, ldy, a_scale, b_scale, bias, 0, 0});                \
+    }                                                                                                    \
   }
   switch (y_dtype) {
     case FMSMO_F16: GO(FMSMO_F16) break;

@@ -991,11 +991,34 @@ __device__ __forceinline__ int sum_parts(const int32_t* p, int64_t stride, int p
   return sum;
 }
 
-// y = (acc - zero * sum[n]) * (a_scale * w_scale) + bias[n]: the batched matmuls' epilogue, one scale for
-// the whole batch (EpiDequant's fp32-scale arithmetic with nothing to fetch per row).  sums: `parts`
-// partial sums over the reduction of the second operand's codes, [parts][batch * N] (int32 operands
-// only: the zero-point correction of the first one, exact in integers), or NULL.  The scale product
-// is that of two device scalars, or `sc` itself where they are NULL.
+// y = (acc - zero * sum[n]) * scale: the int8 batched matmul whose first operand has a zero point, in
+// kernels that keep all their accumulators until the end.  sum: of the second operand's codes over the
+// reduction, [batch * N].  One load per column, like EpiDequant: adding up partial sums here (EpiScaleBias
+// below) cost the register-staged 256 x 256 tile 17 us of 44 (12 heads of 129 x 129 x 512: 27.5) and
+// the 128 x 128 tile 14 of 47 (64 x 64 x 8192), more than the launch that adds them up first.
+template <int OUT>
+struct EpiZeroPoint {
+  void* y;
+  int64_t ldy;
+  float sc;
+  const int32_t* sums;
+  int zero;
+  struct Col {
+    int z;
+  };
+  struct Row {};
+  __device__ __forceinline__ Col col(int n, int expert, int N) const { return Col{zero * sums[(int64_t)expert * N + n]}; }
+  __device__ __forceinline__ Row row(int) const { return Row{}; }
+  __device__ __forceinline__ void store(int m, int n, int v, Row, Col c) const {
+    store_from_f32<OUT>(y, (int64_t)m * ldy + n, __fmul_rn((float)(v - c.z), sc));
+  }
+};
+
+// y = (acc - zero * sum[n]) * (a_scale * w_scale) + bias[n]: the epilogue of the batched matmul with a
+// reduction of 128, one scale for the whole batch (EpiDequant's fp32-scale arithmetic with nothing to
+// fetch per row).  sums: `parts` partial sums over the reduction of the second operand's codes,
+// [parts][batch * N] (int32 operands only: the zero-point correction of the first one, exact in
+// integers), or NULL.  The scale product is that of two device scalars, or `sc` itself where they are NULL.
 template <int OUT, class AccT>
 struct EpiScaleBias {
   static constexpr bool UNIFORM_ROWS = true;

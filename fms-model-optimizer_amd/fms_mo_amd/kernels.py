@@ -679,9 +679,13 @@ def bmm_i8_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype):
                    float(scale2), sums.data_ptr(), sums.shape[0], y.data_ptr(), N, B, M, N, K, _stream(m1))
         else:
             q1 = quant_i8_affine(m1, scale1, zero1, compute_dtype, False, pad)
-            Kp = q1.shape[2]
+            Kp, parts = q1.shape[2], sums.shape[0]
+            if parts > 1 and (Kp != 128 or M <= 128 or N <= 128):
+                # (the kernel for a reduction of 128 adds its two parts itself)
+                L.call("fmsmo_affine_add_parts", sums.data_ptr(), parts, B * N, _stream(m1))
+                parts = 1
             L.call("fmsmo_bmm_i8_zp", q1.data_ptr(), Kp, q2.data_ptr(), Kp, q2.stride(0),
-                   _f32_product(scale1, scale2), int(zero1), sums.data_ptr(), sums.shape[0], y.data_ptr(),
+                   _f32_product(scale1, scale2), int(zero1), sums.data_ptr(), parts, y.data_ptr(),
                    _DT[m1.dtype], N, B, M, N, Kp, _stream(m1))
     return y
 

@@ -288,3 +288,34 @@ def test_attention_scores_of_a_stored_second_operand(dev, xdt, Kd):
     exact = torch.matmul(q1[..., :Kd].double() - z1, q2[..., :Kd].double().transpose(1, 2).contiguous()) * (s1 * s2)
     ulp = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[xdt]
     assert ((y.double() - exact).abs() <= exact.abs() * (ulp + 2.0 ** -22) + 2.0 ** -25).all()
+
+
+@pytest.mark.parametrize("odt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,M,Kd,N,ldy", [
+    (3, 1, 640, 100, 100), (2, 130, 1024, 64, 70), (2, 300, 1024, 100, 100), (2, 129, 512, 129, 129),
+    (2, 140, 192, 300, 300), (2, 140, 128, 300, 300), (2, 140, 128, 300, 312)])
+def test_zero_point_product_with_one_or_several_parts(dev, odt, B, M, Kd, N, ldy):
+    """fmsmo_bmm_i8_zp with the sums of the second operand in parts and added up first: the same bits, and the
+    exact integer times the scale rounded twice (fp32, output).  Output rows may be further apart than N."""
+    from fms_mo_amd import _lib as L
+
+    lib, st = L.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    a = torch.randint(-128, 128, (B, M, Kd), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-128, 128, (B, N, Kd), generator=g, dtype=torch.int8, device=dev)
+    whole = w.sum(-1, dtype=torch.int32)
+    parts = torch.randint(-9999, 9999, (11, B, N), generator=g, dtype=torch.int32, device=dev)
+    parts[4] += whole - parts.sum(0, dtype=torch.int32)
+    scale, zero, ys = 0.0371, -77, []
+    for add in (False, True):
+        if add:
+            assert lib.fmsmo_affine_add_parts(parts.data_ptr(), 11, B * N, st) == 0
+            assert torch.equal(parts[0], whole)
+        y = torch.full((B, M, ldy), 7.0, dtype=odt, device=dev)
+        assert lib.fmsmo_bmm_i8_zp(a.data_ptr(), Kd, w.data_ptr(), Kd, N * Kd, scale, zero, parts.data_ptr(),
+                                   1 if add else 11, y.data_ptr(), K()._DT[odt], ldy, B, M, N, Kd, st) == 0
+        assert (y[..., N:] == 7.0).all()
+        ys.append(y[..., :N])
+    acc = torch.matmul(a.double() - zero, w.double().transpose(1, 2).contiguous())
+    ref = (acc.float() * torch.tensor(scale, dtype=torch.float32, device=dev)).to(odt)   # |acc| < 2^31, one rounding each
+    assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ref)
