@@ -56,16 +56,18 @@ class QBmmINT8Deploy(nn.Module):
             qbmm_int.register_buffer("m2_clip_valn", -Qw.clip_val.detach() * cvn_ext_ratio)
         return qbmm_int.to(target_device)
 
-    # host copies of the four scalars are made once (and again when the buffers change dtype or
-    # device), so forward never synchronizes
+    # host copies of the four scalars, read again when a buffer is replaced or written to (load_state_dict,
+    # copy_, .to(), .half()), so that forward does not synchronize.  (The buffers are kept beside the copies: an
+    # id or address alone could come back with other contents.  Tensors made in inference mode count no
+    # versions, and writes through .data are not counted either.)
     def _scalars(self):
-        key = (self.m1_scale.dtype, self.m1_scale.device)
-        if getattr(self, "_cache_key", None) != key:
-            s1, s2 = float(self.m1_scale), float(self.m2_scale)
-            z1, z2 = int(self.m1_zp) - 128, int(self.m2_zp)
-            self._host = (s1, z1, s2, z2)
-            self._cache_key = key
-        return self._host
+        bufs = (self.m1_scale, self.m1_zp, self.m2_scale, self.m2_zp)
+        state = tuple((t.data_ptr(), -1 if t.is_inference() else t._version) for t in bufs)
+        kept = self.__dict__.get("_kept")
+        if kept is None or kept[1] != state or any(a is not b for a, b in zip(kept[0], bufs)):
+            host = (float(bufs[0]), int(bufs[1]) - 128, float(bufs[2]), int(bufs[3]))
+            kept = self._kept = (bufs, state, host)
+        return kept[2]
 
     def _get_name(self):
         return "QBmmINT8Deploy"
