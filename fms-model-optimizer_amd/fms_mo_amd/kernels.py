@@ -678,7 +678,7 @@ def bmm_i8_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype):
                    float(scale1), float(zero1), _DT[compute_dtype], q2.data_ptr(), q2.stride(1), q2.stride(0),
                    float(scale2), sums.data_ptr(), sums.shape[0], y.data_ptr(), N, B, M, N, K, _stream(m1))
         else:
-            q1 = quant_i8_affine(m1, scale1, zero1, compute_dtype, False, pad)
+            q1 = quant_i8_affine(a3, scale1, zero1, compute_dtype, False, pad)
             Kp, parts = q1.shape[2], sums.shape[0]
             if parts > 1 and (Kp != 128 or M <= 128 or N <= 128):
                 # (the kernel for a reduction of 128 adds its two parts itself)

@@ -319,3 +319,23 @@ def test_zero_point_product_with_one_or_several_parts(dev, odt, B, M, Kd, N, ldy
     acc = torch.matmul(a.double() - zero, w.double().transpose(1, 2).contiguous())
     ref = (acc.float() * torch.tensor(scale, dtype=torch.float32, device=dev)).to(odt)   # |acc| < 2^31, one rounding each
     assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ref)
+
+
+@pytest.mark.parametrize("M,Kd,N", [(70, 130, 140), (140, 80, 200)])
+def test_attention_operands_are_copied_once(dev, monkeypatch, M, Kd, N):
+    """m1 [batch, heads, rows, k] that lies as [batch, rows, heads, k] is made contiguous once."""
+    kn = K()
+    m = make_qbmm(dev, -1.0, 1.0, 3.0, torch.float32)
+    m1 = torch.randn(2, M, 3, Kd, generator=gen(M)).to(dev).transpose(1, 2)
+    m2 = torch.randn(2, 3, Kd, N, generator=gen(N)).to(dev)
+    ref = m(m1.contiguous(), m2)
+    copies, batched3 = [], kn._batched3
+
+    def spy(t):
+        out = batched3(t)
+        copies.extend([t.shape] if out.data_ptr() != t.data_ptr() else [])
+        return out
+
+    monkeypatch.setattr(kn, "_batched3", spy)
+    assert torch.equal(m(m1, m2), ref)
+    assert copies == [m1.shape]
