@@ -598,7 +598,8 @@ static bool is_value_of(float v, int dtype) {
   return a * 0x1p24f == (float)(int)(a * 0x1p24f);  // subnormal (or zero): a multiple of 2^-24
 }
 
-// Which products quantize their first operand on the way: all columns in one tile (nothing is
+// Which products quantize their first operand on the way: corrected sums that stay in 32 bits
+// (zero_sums_fit), all columns in one tile (nothing is
 // quantized twice), whole row tiles, a reduction of two slabs or more and an eighth of the compute
 // units busy (12 heads of 335 x 335 x 96, 72 tiles: 18.2 -> 11.3 us; 8 of 1501 x 1501 x 80 53 -> 29); and a
 // scale and offset that the packed quotient serves.
@@ -611,7 +612,7 @@ extern "C" int fmsmo_bmm_qa_ok(int x_dtype, int compute_dtype, float scale, floa
                                     !is_value_of(offset, compute_dtype) ||
                                     (compute_dtype == FMSMO_F16 && (a > 64.0f || offset > 512.0f || offset < -512.0f))))
     return 0;
-  return N <= 128 && K >= 256 && M >= QA_BM && batch * ((M + QA_BM - 1) / QA_BM) >= 32;
+  return zero_sums_fit((int)offset, K) && N <= 128 && K >= 256 && M >= QA_BM && batch * ((M + QA_BM - 1) / QA_BM) >= 32;
 }
 
 extern "C" int fmsmo_bmm_qa_i8(const void* x, int x_dtype, int64_t ldx, int64_t stride_x, float scale, float offset,

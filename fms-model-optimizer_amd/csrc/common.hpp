@@ -125,6 +125,12 @@ __device__ __forceinline__ uint8_t f32_to_e4m3_sw(float f) {
   return sign | (uint8_t)((e << 3) | (r & 7));
 }
 
+// The corrected sum of an int8 product, sum over k of (q1 - zero) q2, fits 32 bits whatever the codes are.
+inline bool zero_sums_fit(int zero, int64_t K) {
+  const int64_t z = zero < 0 ? -(int64_t)zero : zero;
+  return K <= ((1ll << 31) - 1) / ((z + 128) * 128);
+}
+
 inline int div_up(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
 }  // namespace fmsmo

@@ -294,6 +294,7 @@ extern "C" int fmsmo_bmm_i8_zp(const int8_t* a, int64_t lda, const int8_t* b, in
                                int64_t ldy, int64_t batch, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream) {
   if (!sums) return FMSMO_ERR_NULL;
   if (parts < 1) return FMSMO_ERR_SHAPE;
+  if (!zero_sums_fit(zero, K)) return FMSMO_ERR_UNSUPPORTED;
   return launch_bmm<MMA_I8, int>(a, lda, b, ldb, stride_b, nullptr, nullptr, nullptr, y, y_dtype, ldy, batch, M, N, K,
                                  (hipStream_t)stream, scale, sums, parts, zero);
 }

@@ -653,13 +653,21 @@ def bmm_i8_dq(a, b, a_scale, b_scale, bias=None, out_dtype=torch.float16):
     return _bmm("fmsmo_bmm_i8_dq", torch.int8, a, b, a_scale, b_scale, bias, out_dtype)
 
 
+def zero_sums_fit(zero, K):
+    """Whether the int32 sums of bmm_i8_quantized hold (q1 - zero) . q2 whatever the codes are (K as the kernels
+    see it, padded to at most 128)."""
+    return (abs(int(zero)) + 128) * 128 * (-(-K // 128) * 128) < 1 << 31
+
+
 def bmm_i8_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype):
     """y [batch, M, N] of m1's dtype = dequant(quant(m1) . quant(m2)): both operands quantized with their
     static parameters (see quant_i8_affine), the zero-point correction of m1 made from the column
     sums of m2's codes.  m1 [..., M, K], m2 [..., K, N] with equal leading dimensions.  Probabilities x
-    values quantize m1 inside the product (fmsmo_bmm_qa_i8)."""
+    values quantize m1 inside the product (fmsmo_bmm_qa_i8).  zero_sums_fit(zero1, K) must hold."""
     _need_gpu(m1, m2)
     M, K = m1.shape[-2:]
+    if not zero_sums_fit(zero1, K):
+        raise ValueError(f"the zero-point correction of K = {K} codes with zero point {zero1} may leave 32 bits")
     N = m2.shape[-1]
     a3 = _batched3(m1)
     B = a3.shape[0]

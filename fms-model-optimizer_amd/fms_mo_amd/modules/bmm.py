@@ -100,7 +100,7 @@ class QBmmINT8Deploy(nn.Module):
             raise ValueError(f"incompatible operands {tuple(m1.shape)} @ {tuple(m2.shape)}")
         with torch.no_grad():
             s1, z1, s2, z2 = self._scalars()
-            if (abs(z1) + 128) * 128 * m1.shape[-1] < 1 << 31:
+            if kernels.zero_sums_fit(z1, m1.shape[-1]):
                 y = kernels.bmm_i8_quantized(m1, m2, s1, z1, s2, z2, self._compute_dtype(m1))
             else:  # the corrected sum might leave 32 bits: corrected in fp32 behind the product
                 q1, q2 = self.quantize_operands(m1, m2)

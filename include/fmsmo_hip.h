@@ -676,7 +676,9 @@ int fmsmo_bmm_fp8_dq(const uint8_t* a, int64_t lda, const uint8_t* b, int64_t ld
 /*
  * y[b] = ( a[b] . b[b]^T - zero * sums[b][n] ) * scale: the int8 product with the zero-point correction of
  * an asymmetric first operand made in integers from the sums that fmsmo_quant_i8_affine_sums left
- * (operands as for fmsmo_bmm_i8_dq).
+ * (operands as for fmsmo_bmm_i8_dq).  The corrected sum is formed in 32 bits: a (zero, K) with
+ * (|zero| + 128) * 128 * K >= 2^31, where it could leave them, returns FMSMO_ERR_UNSUPPORTED
+ * (fmsmo_zero_shift_bias and fmsmo_bmm_i8_dq correct in fp32).
  */
 int fmsmo_bmm_i8_zp(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, int64_t stride_b,
                     float scale, int zero, const int32_t* sums, int parts, void* y, int y_dtype,
@@ -686,7 +688,8 @@ int fmsmo_bmm_i8_zp(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, 
  * values: x is read once and its codes never reach memory): x [batch][M][K] fp16 / bf16 with row stride
  * ldx and batch stride stride_x in elements, quantized like fmsmo_quant_i8_affine with (scale, offset),
  * b the codes of the second operand, [batch][N][ldb] zero-padded past K (stride_b = N * ldb or more);
- * y [batch * M][N] of x's dtype.  fmsmo_bmm_qa_ok tells the shapes and scales it serves.
+ * y [batch * M][N] of x's dtype.  fmsmo_bmm_qa_ok tells the shapes, scales and zero
+ * points it serves (the bound of fmsmo_bmm_i8_zp among them); others return FMSMO_ERR_UNSUPPORTED.
  */
 int fmsmo_bmm_qa_ok(int x_dtype, int compute_dtype, float scale, float offset, int64_t batch, int64_t M,
                     int64_t N, int64_t K);
