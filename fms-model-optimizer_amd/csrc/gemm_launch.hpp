@@ -198,7 +198,10 @@ void launch_cut_k(const GemmArgs& g, const Epi& epi, hipStream_t st) {
 
 template <int OP, class Epi>
 void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
-  if (use_tall_tiles(g.M, g.N, g.K)) {
+  if constexpr (OP == MMA_FP8_F16) {  // K % 64 != 0
+    if (cut_k_tall(g.M, g.N, g.K)) launch_tile<TileTallK, OP, false, true>(g, epi, st);
+    else launch_tile<TileMidK, OP, false, true>(g, epi, st);
+  } else if (use_tall_tiles(g.M, g.N, g.K)) {
     launch_tile<TileTallK, OP, false>(g, epi, st);
   } else if (g.K % 64 == 0 && !cut_k_tall(g.M, g.N, g.K)) {
     switch (pick_tile(g.M, g.N, g.K % 128 == 0 && use_register_staged(OP))) {
@@ -222,6 +225,8 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
           launch_tile<TileMid, OP, false>(g, epi, st);
         break;
     }
+  } else if constexpr (OP == MMA_FP8) {
+    launch_tile<TileTallK, OP, false, true>(g, epi, st);  // (K % 64 == 0: MMA_FP8_F16 takes the others)
   } else {
     launch_cut_k<OP>(g, epi, st);
   }
@@ -466,7 +471,9 @@ int launch_split_k(const SplitPlan& p, const GemmArgs& g0, void* workspace, cons
   g.ldb_e = p.k_len;
   g.k_total = g0.K;
   g.grid_m = p.splits * div_up(g0.M, p.rs ? 256 : TileMid::BM);
-  if (p.rs) {
+  if constexpr (OP == MMA_FP8_F16) {  // K % 64 != 0: such plans are cut ones
+    launch_tile<TileTallK, OP, true, true>(g, EpiStoreF32{(float*)workspace, g0.N}, st);
+  } else if (p.rs) {
     if constexpr (OP == MMA_I8) launch_rs<OP, true, 128>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
     else launch_rs<OP, true, 128>(g, EpiStoreF32{(float*)workspace, g0.N}, st);
   } else if (p.cut) {

@@ -21,8 +21,8 @@
 // 16-byte chunks a lane moves): in the last stage the lanes whose chunk lies past K fetch the row's
 // first chunk of that stage instead, and every wave overwrites what those lanes brought with zeros in
 // LDS before the barrier that publishes the stage.  The rest of the pipeline does not know about it.
-// (One thread per output with 4-byte dot products, which served those K before: 386 x 531 x 11472
-// e4m3 2110 us, now 29; 3868 x 542 x 688 int8 1195 -> 14; 57 x 17694 x 1136 e4m3 1382 -> 14.)
+// (One thread per output with 4-byte dot products, which served those K before: 3868 x 542 x 688 int8
+// 1195 us, now 14; e4m3, see MMA_FP8_F16, 386 x 531 x 11472 2110 -> 19, 57 x 17694 x 1136 1382 -> 13.)
 #pragma once
 #include "common.hpp"
 #include <type_traits>
@@ -30,7 +30,7 @@
 
 namespace fmsmo {
 
-enum { MMA_I8 = 0, MMA_FP8 = 1, MMA_FP8_K32 = 2, MMA_F16 = 3, MMA_BF16 = 4, MMA_F32 = 5 };
+enum { MMA_I8 = 0, MMA_FP8 = 1, MMA_FP8_K32 = 2, MMA_F16 = 3, MMA_BF16 = 4, MMA_F32 = 5, MMA_FP8_F16 = 6 };
 
 struct GemmArgs {
   const uint8_t* a;
@@ -121,6 +121,31 @@ struct Mma<MMA_F16> {
   __device__ static __forceinline__ Acc mma(const Frag& a, const Frag& b, const Acc& c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a),
                                                   __builtin_bit_cast(v8h, b), c, 0, 0, 0);
+  }
+};
+// e4m3 operands widened to fp16 (exact) on their way from LDS into the fp16 matrix instruction, which adds
+// their products as accurately as fp32 additions one after the other do (2-norm error of the sum against
+// 64 bits at K = 544 / 1136 / 11472: 4.5e-9 / 1.4e-8 / 5.7e-8, the additions 4.7e-9 / 1.4e-8 / 8.6e-8; the
+// e4m3 instruction, which keeps fewer bits while it adds, 1.3e-5).  Half the matrix rate and four
+// conversions per instruction; us from a HIP graph, e4m3 instruction / this: 386 x 531 x 11472 15.7 / 18.8,
+// 1000 x 4096 x 4016 27.8 / 36.0, 4096 x 4096 x 4016 73.9 / 146.
+template <>
+struct Mma<MMA_FP8_F16> {
+  typedef v4i Frag;
+  typedef v16f Acc;
+  typedef float Elem;
+  static constexpr int KSTEP = 32;
+  typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+  __device__ static __forceinline__ v8h widen(int lo, int hi) {
+    const uint32_t w[4] = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, false)),
+                           __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, true)),
+                           __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, false)),
+                           __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, true))};
+    return __builtin_bit_cast(v8h, v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]});
+  }
+  __device__ static __forceinline__ Acc mma(const Frag& a, const Frag& b, const Acc& c) {
+    const Acc t = __builtin_amdgcn_mfma_f32_32x32x16_f16(widen(a[0], a[1]), widen(b[0], b[1]), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(widen(a[2], a[3]), widen(b[2], b[3]), t, 0, 0, 0);
   }
 };
 template <>

@@ -335,6 +335,9 @@ int fmsmo_gemm_i8_dq(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
 
 /*
  * e4m3 x e4m3 -> fp32 accumulate, y = out( acc * a_scale[m] * w_scale[n] + bias[n] ).
+ * With K % 64 == 0 the e4m3 matrix instruction adds the products (2-norm error of the sum against 64 bits
+ * about 1.5e-5); other K run on the fp16 one (exactly widened operands; no more error than fp32 additions
+ * one after the other, 1.1e-8 at K = 1136).
  * Reference: the torch._scaled_mm call made through addmm_float8_unwrapped_inference in
  * FP8Linear.forward (fms_mo/aiu_addons/fp8/fp8_linear.py:275-283); CPU semantics
  * _scaled_mm_cpu_out (fms_mo/aiu_addons/fp8/fp8_spyre_op.py:35-60).

@@ -88,8 +88,35 @@ def test_reductions_that_are_no_multiple_of_a_stage(dev, M, N, Kd):
     assert torch.equal(y8.double(), a8[:, :Kd].double() @ w8[:, :Kd].double().t())   # |sums| < 2^24: exact in fp32
 
 
+@pytest.mark.parametrize("M,N,Kd", [(1, 5, 16), (17, 33, 48), (32, 64, 544), (65, 31, 1136), (96, 160, 11472)])
+@pytest.mark.parametrize("odt", [torch.float32, torch.float16])
+def test_e4m3_reductions_that_are_no_multiple_of_64_add_in_fp32(dev, M, N, Kd, odt):
+    """2-norm error against 64 bits no larger than that of one fp32 addition after the other (products of e4m3
+    elements are exact in fp32); the e4m3 matrix instruction, which keeps fewer bits, misses it by a hundred."""
+    g = torch.Generator(device=dev).manual_seed(M + Kd)
+    a = torch.randn(M, Kd, generator=g, device=dev).to(torch.float8_e4m3fn)
+    w = torch.randn(N, Kd, generator=g, device=dev).to(torch.float8_e4m3fn)
+    s_a, s_w = torch.rand(M, generator=g, device=dev) + 0.5, torch.rand(N, generator=g, device=dev) + 0.5
+    bias = torch.randn(N, generator=g, device=dev)
+    af, wf = a.float(), w.float()
+    chain = torch.zeros(M, N, device=dev)
+    for k in range(Kd):
+        chain += af[:, k, None] * wf[:, k]
+    exact = af.double() @ wf.double().t()
+    one = torch.ones(1, device=dev)
+    err = lambda y, ref: float((y.double() - ref).norm() / ref.norm())  # noqa: E731
+    if odt == torch.float32:
+        y = K().gemm_fp8_dq(a, w, one, one, None, out_dtype=odt)
+        assert err(y, exact) <= max(err(chain, exact), 2.0 ** -25)
+    ref = exact * (s_a[:, None] * s_w).double() + bias.double()
+    y = K().gemm_fp8_dq(a, w, s_a, s_w, bias, out_dtype=odt)
+    # (one rounding each of scale product, fma and output beyond the sum's)
+    assert err(y, ref) <= 4 * err(chain, exact) + 2.0 ** (-22 if odt == torch.float32 else -11)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("M,Kd,pad", [(1, 16, 0), (3, 4096, 0), (16, 4096, 8), (17, 3856, 0), (700, 1032, 24), (4096, 512, 0)])
+@pytest.mark.parametrize("M,Kd,pad", [(1, 16, 0), (3, 4096, 0), (16, 4096, 8), (17, 3856, 0), (700, 1032, 24), (4096, 512, 0), (3, 16384, 8),
+                                      (5, 16392, 0), (900, 4096, 0)])
 def test_fp8_per_tensor_quantizer_in_two_passes(dev, dtype, M, Kd, pad):
     """One scale for the tensor, with the abs-max taken inside the call (one launch up to 8192 groups of
     eight elements, partial maxima beyond; rows with a stride): bit for bit what the entry point that
