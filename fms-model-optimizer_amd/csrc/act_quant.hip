@@ -1232,16 +1232,12 @@ __global__ __launch_bounds__(SELF ? 1024 : 256) void quant_fp8_tensor16_kernel(
   const bool fast = b < 0x7f800000u && s >= 0x1p-60f && s <= 0x1p60f && amax <= s * 0x1p100f;
   const float r1 = rcp_refined(s);
   [[maybe_unused]] const float nz = opaque_neg_zero();
-  while (c < nchunks) {
-    const int64_t next = c + step;
-    v4i nxt = {0, 0, 0, 0};
-    if (next < nchunks) nxt = *(const v4i*)(x + chunk_elem(next, cpr, ldx, flat));
-    uint8_t* dst = q + chunk_elem(c, cpr, ldq, flat && ldq == (int64_t)cpr * AQ_VEC);
-    if (fast) {
+  auto emit = [&](const v4i& w, uint8_t* dst, bool fast_codes) __attribute__((always_inline)) {
+    if (fast_codes) {
       float t[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float xv = cvt16<XT>((u16)((uint32_t)cur[j >> 1] >> ((j & 1) * 16)));
+        const float xv = cvt16<XT>((u16)((uint32_t)w[j >> 1] >> ((j & 1) * 16)));
         if constexpr (LIN) {
           if constexpr (XT == FMSMO_F16) t[j] = div32_fast_mix(xv, s, r1, nz);
           else t[j] = div32_fast(xv, s, r1);
@@ -1261,13 +1257,38 @@ __global__ __launch_bounds__(SELF ? 1024 : 256) void quant_fp8_tensor16_kernel(
       uint8_t code[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float xv = cvt16<XT>((u16)((uint32_t)cur[j >> 1] >> ((j & 1) * 16)));
+        const float xv = cvt16<XT>((u16)((uint32_t)w[j >> 1] >> ((j & 1) * 16)));
         const float t = LIN ? fminf(fmaxf(xv / s, -448.0f), 448.0f) : round_to<XT>(xv / s);
         code[j] = f32_to_e4m3_sw(t);
         if (VAR == FMSMO_FP8_FPXACC_DL8 && (code[j] & 0x7f) <= 0x04) code[j] = 0x00;
       }
       store8(dst, 0, code);
     }
+  };
+  if constexpr (!LIN) {
+    // A NaN in the tensor leaves the floor as scale, whose quotients leave the e4m3 range: as in the row kernel,
+    // rows that are finite themselves saturate and the others keep unclamped quotients.
+    if (b > 0x7f800000u && cpr <= AQ_MAXCHUNK * AQ_THREADS) {  // the row kernel's longest row
+      const int64_t rows = nchunks / cpr;
+      for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        AbsMax<XT> m;
+        for (int i = threadIdx.x; i < cpr; i += TH) m.add(*(const v4i*)(x + (size_t)row * ldx + (size_t)i * AQ_VEC));
+        __syncthreads();  // every thread has read the last maximum
+        const uint32_t rb = block_max_u32<TH>(m.bits(), red);
+        const bool row_fast =
+            rb < 0x7f800000u && s >= 0x1p-60f && s <= 0x1p60f && __uint_as_float(rb) <= s * 0x1p100f;
+        for (int i = threadIdx.x; i < cpr; i += TH)
+          emit(*(const v4i*)(x + (size_t)row * ldx + (size_t)i * AQ_VEC),
+               q + (size_t)row * ldq + (size_t)i * AQ_VEC, row_fast);
+      }
+      return;
+    }
+  }
+  while (c < nchunks) {
+    const int64_t next = c + step;
+    v4i nxt = {0, 0, 0, 0};
+    if (next < nchunks) nxt = *(const v4i*)(x + chunk_elem(next, cpr, ldx, flat));
+    emit(cur, q + chunk_elem(c, cpr, ldq, flat && ldq == (int64_t)cpr * AQ_VEC), fast);
     cur = nxt;
     c = next;
   }
