@@ -762,7 +762,8 @@ class QLinearINT8Deploy(nn.Linear):
         sq = self.smoothq_scale.reshape(-1) if use_sq else None
         # A bf16 model: the epilogues round to fp16 (acc_dtype) and then to bf16 before they store, where a
         # cast of the fp16 result would be one more pass over [M, N] (16 us of 56 at 1000 x 6144 outputs).
-        out16 = torch.bfloat16 if org_dtype == torch.bfloat16 and self.acc_dtype == torch.float16 else torch.float16
+        to_bf16 = org_dtype == torch.bfloat16 and self.acc_dtype == torch.float16
+        out16 = torch.bfloat16 if to_bf16 else torch.float16
         if plain and (sq is None or sq.numel() == K) and kernels.decode_linear_ok(x2, sq, K):
             # decode step of a few tokens: quantizer and weight-streaming matmul in one launch
             y, s = kernels.decode_linear_i8(x2, self.weight, self._w_scale_f32(), self.bias, sq,
@@ -778,11 +779,11 @@ class QLinearINT8Deploy(nn.Linear):
             with torch.no_grad():
                 if use_sq:
                     x2 = x2 / self.smoothq_scale
-                if self.use_int_kernel and out16 == torch.bfloat16:
-                    y = self.iaddmm(self.bias, x2, self.weight.t(), out_dtype=out16)
-                else:
-                    y = self.iaddmm(self.bias, x2, self.weight.t())
-        if y.dtype != self.acc_dtype and not (self.use_int_kernel and y.dtype == out16 == torch.bfloat16):
+                # (an iaddmm of the user's own takes three arguments and returns acc_dtype)
+                to_bf16 = to_bf16 and getattr(self.iaddmm, "__func__", None) is QLinearINT8Deploy.iaddmm_int
+                kw = {"out_dtype": out16} if to_bf16 else {}
+                y = self.iaddmm(self.bias, x2, self.weight.t(), **kw)
+        if y.dtype != self.acc_dtype and not (to_bf16 and y.dtype == torch.bfloat16):
             y = y.to(self.acc_dtype)
         if not two_d:
             y = y.reshape(tuple(x.shape[:-1]) + (y.shape[-1],))

@@ -59,6 +59,28 @@ def test_deploy_module_of_a_bf16_model_rounds_to_fp16_first(dev, M, w_std, kerne
     assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
 
 
+@pytest.mark.parametrize("how", ["assigned", "subclass"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_an_iaddmm_of_the_users_own_keeps_its_three_arguments(dev, how, dtype):
+    """What it returns is cast to acc_dtype and then to the model's dtype."""
+    from fms_mo_amd.modules.linear import QLinearINT8Deploy
+
+    class Own(QLinearINT8Deploy):
+        def iaddmm_int(self, bias, m1, m2):
+            return 2 * super().iaddmm_int(bias, m1, m2).float()
+
+    cls = Own if how == "subclass" else QLinearINT8Deploy
+    dep = cls.from_fms_mo(make_qlinear(256, 40, dtype), use_int_kernel="triton", use_dynamic_max_act_Qfunc=-1,
+                          recalc_clipvals=False, target_device=dev, truncate_lsb=4, chunk_size=64)
+    x = torch.randn(7, 256, generator=gen(7)).to(dtype).to(dev)
+    plain = QLinearINT8Deploy.iaddmm_int
+    if how == "assigned":
+        dep.iaddmm = lambda bias, m1, m2: 2 * plain(dep, bias, m1, m2).float()
+    y = dep(x)
+    ref = (2 * plain(dep, dep.bias, x, dep.weight.t()).float()).half().to(dtype)
+    assert y.dtype == dtype and torch.equal(y, ref)
+
+
 @pytest.mark.parametrize("M,N,Kd", [
     (1, 5, 16), (3, 64, 48), (17, 65, 80), (128, 63, 112), (129, 130, 144),   # one and two stages, all but empty
     (16, 301, 1040), (300, 520, 624), (1500, 2400, 688), (257, 4099, 592),     # 128 x 64, 128 x 128, 256 x 256 tiles
