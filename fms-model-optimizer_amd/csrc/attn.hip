@@ -34,8 +34,10 @@ __device__ __forceinline__ AffineDiv affine_div(float scale, float offset) {
   } else {
     d.fast = d.fast && XT == T && round_to<T>(scale) == scale;
     d.r = __builtin_amdgcn_rcpf(scale);
-    // (fp16: |scale| <= 64 and |offset| <= 512 keep 65504 / scale + offset outside the codes)
-    d.packed = d.fast && round_to<T>(offset) == offset && (T != FMSMO_F16 || (m <= 64.0f && fabsf(offset) <= 512.0f));
+    // (fp16: scale <= 64 and |offset| <= 512 keep 65504 / scale + offset outside the codes; the sign of a
+    // negative scale would turn the stand-in of a NaN over)
+    d.packed = d.fast && round_to<T>(offset) == offset &&
+               (T != FMSMO_F16 || (scale > 0.0f && scale <= 64.0f && fabsf(offset) <= 512.0f));
   }
   return d;
 }
@@ -61,12 +63,13 @@ __device__ __forceinline__ float affine_code(float e, const AffineDiv& d) {
 template <int XT, int T>
 __device__ __forceinline__ uint32_t affine_codes_packed(uint32_t w, const AffineDiv& d, float nz) {
   if constexpr (T == FMSMO_F16) {
-    // infinite and NaN elements become +-65504 (NaN the lower bound, as the later clamp would have it):
+    // infinite and NaN elements become +-65504 (NaN the lower bound, as the later clamp would have it: the
+    // minimum hands a NaN on quieted, of which the maximum takes the other operand):
     // with |65504 / scale| beyond any code their quotient clamps to the code of the infinite one, and
     // no v_div_fixup is needed behind a finite dividend.  (As instructions of their own: the compiler
     // puts a quieting v_pk_max in front of a max of loaded values.)
+    asm("v_pk_minimum3_f16 %0, %1, %2, %2" : "=v"(w) : "v"(w), "s"(0x7bff7bffu));
     asm("v_pk_max_f16 %0, %1, %2" : "=v"(w) : "v"(w), "s"(0xfbfffbffu));
-    asm("v_pk_min_f16 %0, %1, %2" : "=v"(w) : "v"(w), "s"(0x7bff7bffu));
   }
   const float el = cvt16<XT>((u16)(w & 0xffff)), eh = cvt16<XT>((u16)(w >> 16));
   if constexpr (T == FMSMO_F32) {
@@ -610,7 +613,7 @@ extern "C" int fmsmo_bmm_qa_ok(int x_dtype, int compute_dtype, float scale, floa
   if (compute_dtype == FMSMO_F32 ? x_dtype != FMSMO_F16
                                  : (x_dtype != compute_dtype || !is_value_of(scale, compute_dtype) ||
                                     !is_value_of(offset, compute_dtype) ||
-                                    (compute_dtype == FMSMO_F16 && (a > 64.0f || offset > 512.0f || offset < -512.0f))))
+                                    (compute_dtype == FMSMO_F16 && (scale < 0.0f || a > 64.0f || offset > 512.0f || offset < -512.0f))))
     return 0;
   return zero_sums_fit((int)offset, K) && N <= 128 && K >= 256 && M >= QA_BM && batch * ((M + QA_BM - 1) / QA_BM) >= 32;
 }

@@ -190,6 +190,20 @@ def make_qbmm(dev, lo, hi, other, dtype):
     return QBmmINT8Deploy.from_fms_mo(src, target_device=dev)
 
 
+@pytest.mark.parametrize("xdt,cdt", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
+                                     (torch.float16, torch.float32), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_affine_codes_of_nan_are_the_lower_bound(dev, xdt, cdt, transpose):
+    """Every NaN pattern, quiet and signalling, for scales of both signs (exact in 16 bits)."""
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(xdt)
+    x = x[torch.isnan(x)][:248].repeat(64).reshape(1, -1, 62).to(dev) if xdt == torch.bfloat16 else \
+        x[torch.isnan(x)].reshape(1, -1, 62).to(dev)
+    for scale in (0.03125, -0.03125, 64.0, -640.0):
+        for zero in (0.0, -128.0, 100.0):
+            q = K().quant_i8_affine(x, scale, zero, cdt, transpose)
+            assert (q[..., :x.shape[1] if transpose else 62] == -128).all(), (scale, zero)
+
+
 @pytest.mark.parametrize("xdt,sdt", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
                                      (torch.float16, torch.float32), (torch.bfloat16, torch.float32),
                                      (torch.float32, torch.float32)])
