@@ -341,18 +341,20 @@ inline bool cut_slices(SplitPlan& p, int64_t M, int64_t N, int64_t K, int s) {
 }
 
 // `limit` > 0: the workspace at hand; a plan that needs more is passed over for the next one (the
-// register-staged slices need more partial sums than the 128 x 128 ones: more, shorter slices).
+// register-staged slices need more partial sums than the 128 x 128 ones: more, shorter slices) or
+// takes as many slices as there is room for.
 inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0, bool fp8 = false) {
   SplitPlan p{1, K, 0, false};
   static const char* off = getenv("FMSMO_SPLIT_K");  // FMSMO_SPLIT_K=0 disables (tuning aid)
   if (off && off[0] == '0') return p;
   if (M <= 16 || M > 1024 || use_tall_tiles(M, N, K)) return p;
   const int64_t tiles_t = (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN);
+  const int64_t room = limit > 0 ? limit / (M * N * 4) : 256;
   if (K % 128) {
     // (us, one pass -> slices, M = 40: N = 1024, K = 4016 13.1 -> 8.8; N = 3072 13.6 -> 10.3; M = 100,
     // N = 3072, K = 8208 26.3 -> 14.4; M = 200, N = 1500, K = 11216 36.7 -> 16.7.  From a quarter of a
     // round of tiles on these shapes ask for no workspace.)
-    if (tiles_t < 64) cut_slices(p, M, N, K, (int)(256 / tiles_t));
+    if (tiles_t < 64) cut_slices(p, M, N, K, (int)std::min<int64_t>(256 / tiles_t, room));
     return p;
   }
   // Long reductions under a few hundred rows: 256 x 128 tiles of the register-staged kernel carry
@@ -368,7 +370,9 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
     // 224, 68.0 -> 65.0 | 81.2 -> 65.1; 700 x 4096 x 8192, 192, 40.5 -> 32.8 | 48.8 -> 33.0; 1000 x 2304 x
     // 9216, 144, 36.3 -> 30.2 | 42.1 -> 31.8; 640 x 4096 x 14336, 160, 60.1 -> 64.4 | 73.5 -> 67.5; 640 x 5120
     // x 13824, 200, 63.6 -> 68.2 | 76.1 -> 68.4; 600 x 4352 x 11008, 170, 48.5 -> 52.1 | 58.8 -> 51.3;
-    // 1024 x 4096 x 14336, 256, 80.0 -> 72.5)
+    // 1024 x 4096 x 14336, 256, 80.0 -> 72.5; 512 x 7168, 224: K = 10240 63.8 -> 57.5, 12288 66.5 -> 67.3,
+    // 14336 78.7 -> 75.2, 16384 83.1 -> 80.2; of 58 shapes with 224 .. 256 tiles and K = 10240 .. 16384 56 gained
+    // up to 17 %, two lost 1 %)
     const int64_t t128 = (int64_t)div_up(M, TileMidK::BM) * div_up(N, TileMidK::BN);
     if (t128 > 128 && t128 <= 256 && (fp8 || t128 >= 224 || K <= 9216)) return p;
     if (t <= 128) {
@@ -392,7 +396,7 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   // K = 8192 14.3 / 14.6 / 13.1 -> 10.6 / 11.2 / 11.2; K = 14336, N = 4096, M = 33 / 128 / 256 22.7 /
   // 25.1 / 34.1 -> 22.1 / 24.3 / 33.0).  At most 256 blocks of 128 x 64 partial sums: 8 MiB.
   if (tiles_t <= 128) {
-    int s = (int)(256 / tiles_t);
+    int s = (int)std::min<int64_t>(256 / tiles_t, room);
     const int most = (int)std::min<int64_t>(s, K / 1024);
     while (s > 1 && (K % (s * 128) != 0 || K / s < 1024)) --s;
     // no even split near the one wanted (K = 128 x a prime): slices of whole stages, the last shorter
@@ -409,7 +413,8 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   // shorter reductions: 128 x 128 tiles, slices of at least 512
   const int64_t tiles = (int64_t)div_up(M, TileMid::BM) * div_up(N, TileMid::BN);
   if (tiles > 128) return p;
-  int s = (int)(256 / tiles);  // one block per compute unit; 512 and 1024 blocks measured slower
+  // one block per compute unit; 512 and 1024 blocks measured slower
+  int s = (int)std::min<int64_t>(256 / tiles, room);
   while (s > 1 && (K % (s * 128) != 0 || K / s < 512)) --s;
   // Slices of 512 are mostly prologue and partial-sum traffic (as many bytes as the weights at
   // 128 rows): from K = 4096 on, half as many slices of 1024 are faster while 64 blocks remain

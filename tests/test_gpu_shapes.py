@@ -401,3 +401,26 @@ def test_attention_operands_are_copied_once(dev, monkeypatch, M, Kd, N):
     monkeypatch.setattr(kn, "_batched3", spy)
     assert torch.equal(m(m1, m2), ref)
     assert copies == [m1.shape]
+
+
+@pytest.mark.parametrize("M,N,Kd", [(33, 250, 9472), (40, 100, 4016), (65, 1000, 4096), (200, 1024, 1536)])
+def test_a_workspace_with_room_for_fewer_slices_is_used(dev, M, N, Kd):
+    """Slices of unequal length (K = 74 x 128 and K % 128 != 0) and of equal length: with room for fewer slices than
+    the plan would take the call makes fewer, within the room; with room for one it leaves the workspace alone."""
+    from fms_mo_amd import _lib as L
+
+    st = torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(M)
+    a = torch.randint(-128, 128, (M, Kd), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-128, 128, (N, Kd), generator=g, dtype=torch.int8, device=dev)
+    ref = (a.double() @ w.double().t()).to(torch.int32)
+    full = L.load().fmsmo_gemm_workspace_bytes(M, N, Kd) // (M * N * 4)
+    assert full > 2
+    for room in (1, 2, full - 1, full):
+        ws = torch.full((room * M * N + 64,), 0x55555555, dtype=torch.int32, device=dev)
+        c = torch.empty((M, N), dtype=torch.int32, device=dev)
+        L.call("fmsmo_gemm_i8_i32_ws", a.data_ptr(), Kd, w.data_ptr(), Kd, c.data_ptr(), N, M, N, Kd,
+               ws.data_ptr(), room * M * N * 4 + 16, st)
+        assert torch.equal(c, ref)
+        assert bool((ws[:2 * M * N] != 0x55555555).any()) == (room > 1), room
+        assert (ws[room * M * N:] == 0x55555555).all()
