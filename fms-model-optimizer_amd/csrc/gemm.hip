@@ -196,6 +196,9 @@ extern "C" int fmsmo_gemm_i8_dq_noalloc(const int8_t* a, int64_t lda, const int8
 extern "C" int64_t fmsmo_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return plan_split_k(M, N, K).ws_bytes;
 }
+extern "C" int64_t fmsmo_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  return plan_split_k(M, N, K, 0, true).ws_bytes;
+}
 
 extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
@@ -203,8 +206,8 @@ extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) {
   return tail_split_columns((int)M, (int)N, (int)K);
 }
 
-extern "C" int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel,
-                               int* tile_m, int* tile_n, int* splits) {
+static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
+                     int* tile_n, int* splits) {
   if (!kernel || !tile_m || !tile_n || !splits) return FMSMO_ERR_NULL;
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff)
     return FMSMO_ERR_SHAPE;
@@ -221,8 +224,8 @@ extern "C" int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspa
     *tile_n = TileTallK::BN;
     return FMSMO_OK;
   }
-  const SplitPlan plan = with_workspace == 2 ? plan_split_k(M, N, K, (int64_t)FMSMO_STATIC_SCRATCH_BYTES)
-                                             : plan_split_k(M, N, K);
+  const SplitPlan plan = with_workspace == 2 ? plan_split_k(M, N, K, (int64_t)FMSMO_STATIC_SCRATCH_BYTES, fp8)
+                                             : plan_split_k(M, N, K, 0, fp8);
   if (with_workspace == 2 && plan.ws_bytes > (int64_t)FMSMO_STATIC_SCRATCH_BYTES)
     return FMSMO_ERR_SCRATCH;  // what the noalloc entry point returns for this shape
   if (with_workspace && plan.splits > 1) {
@@ -249,6 +252,16 @@ extern "C" int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspa
   *tile_m = bm[t];
   *tile_n = (t == 3 && !rs) ? 256 : bn[t];
   return FMSMO_OK;
+}
+
+extern "C" int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
+                               int* tile_n, int* splits) {
+  return gemm_plan(false, M, N, K, with_workspace, kernel, tile_m, tile_n, splits);
+}
+extern "C" int fmsmo_gemm_fp8_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
+                                   int* tile_n, int* splits) {
+  if (with_workspace == 2) return FMSMO_ERR_UNSUPPORTED;  // there is no e4m3 call on the static scratch
+  return gemm_plan(true, M, N, K, with_workspace, kernel, tile_m, tile_n, splits);
 }
 
 extern "C" int fmsmo_grouped_gemm_i8_dq(const int8_t* a, int64_t lda, const int8_t* b,

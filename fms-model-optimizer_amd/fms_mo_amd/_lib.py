@@ -73,6 +73,7 @@ SIGNATURES = {
     "fmsmo_debug_stream_read": [_P, _L, _P, _P],
     "fmsmo_debug_mfma_loop": [_I, _P, _L, _I, _P, _P, _P],
     "fmsmo_gemm_plan": [_L, _L, _L, _I, _P, _P, _P, _P],
+    "fmsmo_gemm_fp8_plan": [_L, _L, _L, _I, _P, _P, _P, _P],
 }
 OTHER = {
     "fmsmo_abi_version": ([], c_int),
@@ -81,6 +82,7 @@ OTHER = {
     "fmsmo_affine_sum_parts": ([c_int64, c_int64, c_int64, c_int], c_int),
     "fmsmo_bmm_qa_ok": ([c_int, c_int, c_float, c_float, c_int64, c_int64, c_int64, c_int64], c_int),
     "fmsmo_gemm_workspace_bytes": ([c_int64, c_int64, c_int64], c_int64),
+    "fmsmo_gemm_fp8_workspace_bytes": ([c_int64, c_int64, c_int64], c_int64),
     "fmsmo_decode_linear_ok": ([c_int64, c_int64], c_int),
     "fmsmo_decode_linear_f32s_ok": ([c_int64, c_int64], c_int),
     "fmsmo_gemm_tail_columns": ([c_int64, c_int64, c_int64], c_int64),

@@ -267,27 +267,30 @@ def fake_quant_fp8(x, mode, want_values=True, want_codes=False):
 
 
 # ------------------------------------------------------------------------------------ GEMMs
-_WS_BYTES: dict = {}
+_WS_BYTES: dict = {}      # int8
+_WS_BYTES_FP8: dict = {}  # e4m3
 
 
-def _workspace(M, N, K, device):
+def _workspace(M, N, K, device, fp8=False):
     """Scratch for the split-K form of the *_dq GEMMs (None when the shape does not use one).  It
     comes from torch's caching allocator like every output, so it is also valid under graph
     capture; the library itself never allocates."""
-    key = (M, N, K)
-    nbytes = _WS_BYTES.get(key)
+    known, key = _WS_BYTES_FP8 if fp8 else _WS_BYTES, (M, N, K)
+    nbytes = known.get(key)
     if nbytes is None:  # the policy is fixed for the life of the process: ask the library once per shape
-        nbytes = _WS_BYTES[key] = L.load().fmsmo_gemm_workspace_bytes(M, N, K)
+        lib = L.load()
+        nbytes = known[key] = (lib.fmsmo_gemm_fp8_workspace_bytes if fp8 else lib.fmsmo_gemm_workspace_bytes)(M, N, K)
     return torch.empty((nbytes,), dtype=torch.uint8, device=device) if nbytes > 0 else None
 
 
-def gemm_plan(M, N, K, with_workspace=False):
-    """(kernel, tile_m, tile_n, splits) the *_dq GEMMs use for a shape; no GPU needed
-    (kernel is one of L.PLAN_*; see fmsmo_gemm_plan)."""
+def gemm_plan(M, N, K, with_workspace=False, fp8=False):
+    """(kernel, tile_m, tile_n, splits) the *_dq GEMMs of int8 (e4m3) operands use for a shape; no GPU
+    needed (kernel is one of L.PLAN_*; see fmsmo_gemm_plan)."""
     import ctypes
 
     out = [ctypes.c_int(0) for _ in range(4)]
-    L.call("fmsmo_gemm_plan", M, N, K, int(bool(with_workspace)), *[ctypes.byref(o) for o in out])
+    L.call("fmsmo_gemm_fp8_plan" if fp8 else "fmsmo_gemm_plan", M, N, K, int(bool(with_workspace)),
+           *[ctypes.byref(o) for o in out])
     return tuple(o.value for o in out)
 
 
@@ -405,7 +408,7 @@ def gemm_fp8_dq(a, w, a_scale, w_scale, bias=None, out_dtype=torch.bfloat16, for
     args = (a.data_ptr(), _ld(a), w.data_ptr(), _ld(w), a_scale.data_ptr(),
             a_scale.numel(), w_scale.data_ptr(), w_scale.numel(), _ptr(bias),
             _dt(bias) if bias is not None else 0, y.data_ptr(), _DT[out_dtype], N, M, N, K)
-    ws = None if force_gemv else _workspace(M, N, K, a.device)
+    ws = None if force_gemv else _workspace(M, N, K, a.device, True)
     with _dev(a):
         if ws is not None:
             L.call("fmsmo_gemm_fp8_dq_ws", *args, ws.data_ptr(), ws.numel(), _stream(a))
@@ -964,9 +967,9 @@ def _gemm_fp8_dq_lean(a, w, a_scale, w_scale, bias, out_dtype):
     if _CUR_DEVICE() != idx or out_dtype not in _DT:
         return None
     y = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    nbytes = _WS_BYTES.get((M, N, K))
+    nbytes = _WS_BYTES_FP8.get((M, N, K))
     if nbytes is None:
-        nbytes = _WS_BYTES[(M, N, K)] = L.load().fmsmo_gemm_workspace_bytes(M, N, K)
+        nbytes = _WS_BYTES_FP8[(M, N, K)] = L.load().fmsmo_gemm_fp8_workspace_bytes(M, N, K)
     if nbytes > 0:
         ws = torch.empty((nbytes,), dtype=torch.uint8, device=a.device)
         rc = _fn("fmsmo_gemm_fp8_dq_ws")(a.data_ptr(), lda, w.data_ptr(), ldw, a_scale.data_ptr(), a_scale.numel(),

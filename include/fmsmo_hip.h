@@ -307,7 +307,8 @@ int fmsmo_gemm_i8_i32(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb
  * The same with an optional scratch buffer, as for fmsmo_gemm_i8_dq_ws below: shapes with few
  * output tiles and a long reduction run as K slices whose int32 partial sums are added in a fixed
  * order (exact, so the result is the single-pass one bit for bit); fmsmo_gemm_workspace_bytes
- * tells the bytes a shape can use, workspace == NULL or fewer bytes runs the single pass.
+ * tells the bytes a shape can use, with fewer bytes the call takes the split that fits them, with
+ * workspace == NULL it runs the single pass.
  * Up to 16 rows (and the batches of up to 64 rows that fmsmo_gemm_i8_dq sends there) run on the
  * weight-streaming kernels with either call.
  * Same reference interfaces as fmsmo_gemm_i8_i32; the workspace has no counterpart there.
@@ -349,29 +350,33 @@ int fmsmo_gemm_fp8_dq(const uint8_t* a, int64_t lda, const uint8_t* b, int64_t l
 
 /*
  * The two *_dq GEMMs with a caller-provided workspace (the library allocates nothing).  When the
- * output has few tiles and the reduction is long (16 < M <= 1024, at most 128 tiles of 128 x 128,
- * K % 128 == 0: a batch of tens to hundreds of tokens through a projection with few output
+ * output has few tiles and the reduction is long (16 < M <= 1024, at most 128 tiles of 128 x 128:
+ * a batch of tens to hundreds of tokens through a projection with few output
  * columns) the reduction is split into slices that run side by side and a second kernel adds the
  * slices in a fixed order and applies the epilogue: 17 x 4096 x 14336 runs on 256 compute units
  * instead of 32.  int32 partial sums are exact, so the int8 result is bit-identical to
  * fmsmo_gemm_i8_dq's; the e4m3 result differs from fmsmo_gemm_fp8_dq's only by the order of the
  * fp32 additions.  From 384 rows and K >= 8192 the slices run on 256 x 128 tiles of the
- * register-staged kernel (more, shorter slices: more partial sums).  Shapes whose 128 x 64 tiles
+ * register-staged kernel (more, shorter slices: more partial sums); K that no number of equal slices
+ * of whole 128-byte stages divides (128 x a prime, K % 128 != 0) is cut into slices of which the last
+ * one is shorter.  In one pass, asking for no workspace, run instead: shapes whose 128 x 64 tiles
  * fill half a round of the compute units or more with a short reduction (192-256 tiles and
- * K <= 8192, or M > 128, 96-191 tiles and K <= 4096), and a full round of 128 x 128 tiles, run in
- * one pass instead and ask for no workspace.  fmsmo_gemm_workspace_bytes
- * returns the bytes a shape can use at most (0: no split); with fewer bytes the call takes the
+ * K <= 8192, or M > 128, 96-191 tiles and K <= 4096); from 384 rows and K >= 8192, shapes of 129-256 tiles of
+ * 128 x 128 (e4m3 all of them, int8 from 224 tiles on or with K <= 9216); K % 128 != 0 with 64 tiles of 128 x 64 or more.
+ * fmsmo_gemm_workspace_bytes (int8) and fmsmo_gemm_fp8_workspace_bytes (e4m3)
+ * return the bytes a shape can use at most (0: no split); with fewer bytes the call takes the
  * split that fits them (the 128 x 128 tiles' never needs more than 16 MiB), with none or
  * workspace == NULL it is fmsmo_gemm_*_dq.  workspace: 16-byte aligned
  * device memory, contents undefined before and after, private to the call while it runs.
  * No counterpart in the reference (its GEMMs are single launches of CUTLASS / cuBLASLt kernels).
  */
 int64_t fmsmo_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int64_t fmsmo_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
- * Which kernel the *_dq GEMMs run for a shape, without launching anything (host-only; for tests,
- * tuning and capacity planning).  with_workspace = 1 describes the *_dq_ws calls given a
- * sufficient workspace, with_workspace = 2 what fmsmo_gemm_i8_dq_noalloc runs (the split that
+ * Which kernel the *_dq GEMMs (int8; fmsmo_gemm_fp8_plan: e4m3) run for a shape, without launching anything
+ * (host-only; for tests, tuning and capacity planning).  with_workspace = 1 describes the *_dq_ws calls given a
+ * sufficient workspace, with_workspace = 2 what fmsmo_gemm_i8_dq_noalloc runs (int8 only; the split that
  * fits its static scratch; FMSMO_ERR_SCRATCH where that call returns it).  tile_m / tile_n are 0 for the decode and generic kernels; splits is the
  * number of K slices (1 = single pass).  The choice weighs the measured efficiency of each tile
  * shape against how full the last round of tiles leaves the 256 compute units, e.g.
@@ -390,6 +395,8 @@ enum fmsmo_plan_kernel {
 };
 int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
                     int* tile_n, int* splits);
+int fmsmo_gemm_fp8_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
+                        int* tile_n, int* splits);
 /* Columns that the single-pass *_dq GEMMs cut off the end of N and run as a second GEMM behind
    the first (0: the GEMM runs whole; fmsmo_gemm_plan describes the first, main part).  Host-only. */
 int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K);

@@ -1,5 +1,6 @@
 """Rules that the host evaluates for a launch, without a GPU."""
 import ctypes
+import os
 
 import pytest
 
@@ -26,3 +27,24 @@ def test_zero_point_products_refuse_what_leaves_32_bits(zero):
     if abs(zero) <= 512:
         assert lib.fmsmo_bmm_qa_ok(L.F16, L.F16, 0.5, float(zero), 32, 64, 64, last) == 1
     assert lib.fmsmo_bmm_qa_ok(L.F16, L.F32, 0.5, float(zero), 32, 64, 64, max(256, last + 1)) == 0
+
+
+def test_e4m3_plan_and_workspace_are_those_of_the_e4m3_calls():
+    """129 .. 256 tiles of 128 x 128 and a long reduction: e4m3 runs in one pass throughout, int8 from 224 tiles on; the
+    workspace that is asked for (and allocated) is that of the operand type."""
+    if any(os.environ.get(k) for k in ("FMSMO_TILE", "FMSMO_RS", "FMSMO_SPLIT_K", "FMSMO_TALL")):
+        pytest.skip("tuning overrides are set")
+    lib, rs, dma = L.load(), L.PLAN_TILE_REGISTER_STAGED, L.PLAN_TILE_LDS_DMA
+    for M, N, K, i8, fp8 in ((640, 4096, 14336, (rs, 256, 128, 2), (dma, 128, 128, 1)),      # 160 tiles
+                             (640, 5120, 13824, (rs, 256, 128, 2), (dma, 128, 128, 1)),      # 200
+                             (777, 4096, 12800, (dma, 128, 128, 1), (dma, 128, 128, 1)),     # 224
+                             (512, 4096, 14336, (rs, 256, 128, 4), (rs, 256, 128, 4)),       # 128: slices for both
+                             (40, 100, 4016, (dma, 128, 64, 3), (dma, 128, 64, 3))):         # the last slice shorter
+        for fp8_call, want, size in ((False, i8, lib.fmsmo_gemm_workspace_bytes),
+                                     (True, fp8, lib.fmsmo_gemm_fp8_workspace_bytes)):
+            plan = kernels.gemm_plan(M, N, K, with_workspace=True, fp8=fp8_call)
+            nbytes = want[3] * M * N * 4 if want[3] > 1 else 0
+            ws = kernels._workspace(M, N, K, "cpu", fp8_call)
+            assert plan == want and size(M, N, K) == nbytes and (ws.numel() if ws is not None else 0) == nbytes, (M, N, K)
+    out = [ctypes.byref(ctypes.c_int()) for _ in range(4)]
+    assert lib.fmsmo_gemm_fp8_plan(640, 4096, 14336, 2, *out) == 4   # no e4m3 call on the static scratch: refused
