@@ -1210,10 +1210,7 @@ __global__ __launch_bounds__(SELF ? 1024 : 256) void quant_fp8_tensor16_kernel(
   if (c < nchunks) cur = *(const v4i*)(x + chunk_elem(c, cpr, ldx, flat));
   uint32_t b = 0;
   if constexpr (SELF) {
-    AbsMax<XT> m;
-    m.add(cur);
-    // every other chunk, once; the block's own ones are in registers (one per thread: SELF grids
-    // cover the tensor)
+    AbsMax<XT> m;  // of every chunk, the block's own ones (one per thread: SELF grids cover the tensor) included
     for (int64_t o = threadIdx.x; o < nchunks; o += 4 * 1024) {
       v4i w[4];
 #pragma unroll

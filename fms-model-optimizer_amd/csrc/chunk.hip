@@ -45,7 +45,6 @@ struct ChunkArgs {
 enum { CHUNK_EPI_RAW = -1 };
 template <class AccT>
 struct EpiChunk {
-  static constexpr bool UNIFORM_ROWS = false;
   void* y;
   int64_t ldy;
   const float* a_scale;

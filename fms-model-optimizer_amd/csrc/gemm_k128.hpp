@@ -9,9 +9,9 @@
 // blockIdx.x + gridDim.x, ...:  the operands of its next tile are requested (into registers) before
 // the current tile is converted and written (after its MFMAs, when the fragment registers are
 // free: two blocks per compute unit leave 256 registers per lane), so the next tile's memory
-// latency runs under the current tile's epilogue; the row / column operands of the epilogue are
-// fetched before those requests (loads return in order: fetched after them, the epilogue would
-// wait for the whole next tile first).
+// latency runs under the current tile's epilogue; the next tile's column operands (bias, zero-point sums; one
+// scale serves all rows) are fetched ahead of its requests (loads return in order: fetched after them, the
+// accumulators that start from them would wait for the whole tile first).
 //
 // LDS layout, operand fragments and accumulator layout are those of gemm_rs.hpp (rows of 128
 // bytes, 16-byte chunk c of row r at position c ^ swz(r); 32 x 32 MFMA blocks).

@@ -252,7 +252,7 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblk, int grid_m, int
 
 template <int BM, int BN, int BK, int NSTAGE, int WGM, int WGN, int OP, int SWZ, bool GROUPED,
           class Epi, class Chk = NoChunk, bool KT = false>
-// (two blocks per compute unit for the scheduled chunk hooks; the generic hook keeps a second
+// (KT: without chunk hooks only.  Two blocks per compute unit for the scheduled chunk hooks; the generic hook keeps a second
 // accumulator set and would spill at 256 registers)
 __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1) void gemm_tile_kernel(GemmArgs g, Epi epi, Chk chk) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
@@ -269,6 +269,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
   constexpr int CL = MM::KSTEP / 32;           // 16-byte chunks per lane per k-step
   static_assert(RPI % 16 == 0 && BM % RPI == 0 && BN % RPI == 0, "loader shape");
   static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile");
+  static_assert(!KT || !Chk::enabled, "chunks end with whole stages");
 
   constexpr int STAGE_BYTES = (BM + BN) * BK;
   __shared__ __attribute__((aligned(16))) uint8_t lds[NSTAGE][STAGE_BYTES];
@@ -641,11 +642,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
       constexpr int PAR = decltype(par_c)::value;
       // stage kt + 1 has landed for every wave; its fragments go to the other register set, and
       // the buffer of stage kt - 1 (last read a stage ago) is refilled with stage kt + 3
-      if constexpr (KT) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 3) * NLD) : "memory");
-        zero_past_end(kt + 1);
-        before_issue(kt + NSTAGE - 1);
-      }
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NSTAGE - 3) * NLD) : "memory");
       const uint8_t* ls = &lds[0][0] + ((kt + 1) % NSTAGE) * STAGE_BYTES;
 #pragma unroll
@@ -961,7 +957,6 @@ struct EpiStoreF32 {
 // tile came out four registers short.
 template <int OUT, int BIAS, bool REF_F16, class AccT, bool MULADD_SWITCH = true>
 struct EpiDequant {
-  static constexpr bool UNIFORM_ROWS = false;
   void* y;
   int64_t ldy;
   const float* a_scale;
@@ -1046,7 +1041,6 @@ struct EpiZeroPoint {
 // integers), or NULL.  The scale product is that of two device scalars, or `sc` itself where they are NULL.
 template <int OUT, class AccT>
 struct EpiScaleBias {
-  static constexpr bool UNIFORM_ROWS = true;
   static constexpr int OUT_DT = OUT;
   void* y;
   int64_t ldy;
