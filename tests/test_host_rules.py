@@ -1,8 +1,10 @@
 """Rules that the host evaluates for a launch, without a GPU."""
+import contextlib
 import ctypes
 import os
 
 import pytest
+import torch
 
 from fms_mo_amd import _lib as L
 from fms_mo_amd import kernels
@@ -48,3 +50,19 @@ def test_e4m3_plan_and_workspace_are_those_of_the_e4m3_calls():
             assert plan == want and size(M, N, K) == nbytes and (ws.numel() if ws is not None else 0) == nbytes, (M, N, K)
     out = [ctypes.byref(ctypes.c_int()) for _ in range(4)]
     assert lib.fmsmo_gemm_fp8_plan(640, 4096, 14336, 2, *out) == 4   # no e4m3 call on the static scratch: refused
+
+
+def test_fp8_per_tensor_quantizer_of_a_huge_tensor(monkeypatch):
+    """From 2^31 groups of eight elements on, more than the two-pass call counts, the column maxima serve as
+    before.  (The calls are recorded, not made, and the 32 GiB have no storage.)"""
+    names = []
+    monkeypatch.setattr(kernels.L, "call", lambda name, *args: names.append((name, args)))
+    monkeypatch.setattr(kernels, "_need_gpu", lambda *t: None)
+    monkeypatch.setattr(kernels, "_dev", lambda t: contextlib.nullcontext())
+    monkeypatch.setattr(kernels, "_stream", lambda t: None)
+    for rows, want in ((1 << 20, ["fmsmo_absmax_cols", "fmsmo_quant_act_fp8_dynamic"]),
+                       ((1 << 20) - 1, ["fmsmo_quant_act_fp8_tensor"])):
+        kernels._quant_act_fp8_dynamic_impl(torch.empty(rows, 1 << 14, dtype=torch.float16, device="meta"), per_tensor=True)
+        assert [n for n, _ in names] == want
+        assert want[-1] != "fmsmo_quant_act_fp8_dynamic" or (names[-1][1][4] == 1 and names[-1][1][5] is not None)
+        names.clear()
