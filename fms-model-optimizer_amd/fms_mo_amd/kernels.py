@@ -597,7 +597,7 @@ def zero_shift_bias(w, w_scale, a_meta, bias=None, offset=128.0):
 def _batched3(t: torch.Tensor) -> torch.Tensor:
     """[..., R, C] -> [batch, R, C] with unit inner stride and one batch stride (a view when the
     leading dimensions collapse, a copy otherwise)."""
-    t3 = t.reshape(-1, t.shape[-2], t.shape[-1])
+    t3 = t if t.dim() == 3 else t.reshape(-1, t.shape[-2], t.shape[-1])
     if t3.stride(2) != 1 or (t3.shape[1] > 1 and t3.stride(1) < t3.shape[2]):
         t3 = t3.contiguous()
     return t3

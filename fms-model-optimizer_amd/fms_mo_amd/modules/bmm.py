@@ -61,13 +61,21 @@ class QBmmINT8Deploy(nn.Module):
     # id or address alone could come back with other contents.  Tensors made in inference mode count no
     # versions, and writes through .data are not counted either.)
     def _scalars(self):
-        bufs = (self.m1_scale, self.m1_zp, self.m2_scale, self.m2_zp)
-        state = tuple((t.data_ptr(), -1 if t.is_inference() else t._version) for t in bufs)
+        b = self._buffers
+        s1, z1, s2, z2 = bufs = b["m1_scale"], b["m1_zp"], b["m2_scale"], b["m2_zp"]
+        try:
+            state = (s1._version, z1._version, s2._version, z2._version,
+                     s1.data_ptr(), z1.data_ptr(), s2.data_ptr(), z2.data_ptr())
+        except RuntimeError:  # an inference tensor
+            state = tuple((t.data_ptr(), -1 if t.is_inference() else t._version) for t in bufs)
         kept = self.__dict__.get("_kept")
-        if kept is None or kept[1] != state or any(a is not b for a, b in zip(kept[0], bufs)):
-            host = (float(bufs[0]), int(bufs[1]) - 128, float(bufs[2]), int(bufs[3]))
-            kept = self._kept = (bufs, state, host)
-        return kept[2]
+        if kept is not None and kept[1] == state:
+            k = kept[0]
+            if k[0] is s1 and k[1] is z1 and k[2] is s2 and k[3] is z2:
+                return kept[2]
+        host = (float(s1), int(z1) - 128, float(s2), int(z2))
+        self._kept = (bufs, state, host)
+        return host
 
     def _get_name(self):
         return "QBmmINT8Deploy"
@@ -77,7 +85,7 @@ class QBmmINT8Deploy(nn.Module):
                 f"use_int_kernel={self.use_int_kernel}")
 
     def _compute_dtype(self, m1):
-        sc = self.m1_scale
+        sc = self._buffers["m1_scale"]
         return torch.promote_types(m1.dtype, sc.dtype) if sc.dim() > 0 else m1.dtype
 
     def quantize_operands(self, m1, m2):
