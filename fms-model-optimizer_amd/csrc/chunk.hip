@@ -6,15 +6,15 @@
 // and only then added to the running accumulator -- the same order of operations as the
 // reference's Triton kernels, whose BLOCK_SIZE_K equals the chunk size.
 //
-// Two kernels.  K (in bytes) a multiple of 64: the pipelined tile kernel of gemm_tile.hpp
-// (128x128 block, 4-stage DMA ring) with its chunk hook.  Any other K: the simple kernel below.
+// Two kernels.  Operands within 2^31 bytes each: the pipelined tile kernel of chunk_tile.hpp.
+// Larger ones: the simple kernel below, which addresses its rows with 64 bits.
 //
 // Simple kernel tiling: 128x128 block, 4 waves of 64x64 (2x2 MFMA 32x32 blocks each); K advances in 64-byte
 // stages through two LDS buffers filled with bounds-checked 16-byte loads (zero fill past M, N
 // and K, which is what "the K tail is masked to 0" means).  One MFMA k-step is 32 bytes of K
 // for every operand type, so chunk boundaries (multiples of 32 bytes) always fall between
 // k-steps.
-#include "gemm_tile.hpp"
+#include "chunk_tile.hpp"
 
 namespace fmsmo {
 
@@ -30,74 +30,6 @@ struct ChunkArgs {
   int trun_bits, max_acc_bits, dl16, tta;
   const void* c_in;
   int64_t ldc;  // row stride of c_in (elements)
-};
-
-// What happens to a finished accumulator element.  One functor type per accumulator type with the
-// mode, the output dtype and the bias dtype as run-time fields: the switch is on wave-uniform
-// values in a 64-element epilogue behind a K loop of thousands of MFMAs, and it keeps the number
-// of instantiations of the pipelined kernel (operand types x interleaving schedules) unchanged.
-//   CHUNK_EPI_RAW        d[m,n] = acc                                  (int32 / fp32 out)
-//   FMSMO_EPI_REF_F16    f16( f32(acc) * f16(as ws) + b )              (iaddmm_int's plain branch)
-//   FMSMO_EPI_F32        fma( f32(acc), as ws, b )
-//   FMSMO_EPI_F32_MULADD ( f32(acc) * (as ws) ) + b, every step rounded (iaddmm_int's chunk loop)
-//   FMSMO_EPI_SEQ_OUT    T( T( (f32(acc) * as) * ws ) + T(b) ), T = output dtype
-//                        (LinearFuncFPxFwdBwd / LinearFuncINT8FwdFP32Bwd: descale, cast, add bias)
-enum { CHUNK_EPI_RAW = -1 };
-template <class AccT>
-struct EpiChunk {
-  void* y;
-  int64_t ldy;
-  const float* a_scale;
-  const float* w_scale;
-  const void* bias;
-  int a_stride, w_stride;
-  int mode, out_dt, bias_dt;
-  struct Col {
-    float ws, b;
-  };
-  struct Row {
-    float as;
-  };
-  __device__ __forceinline__ float to_out_grid(float v) const {
-    return out_dt == FMSMO_F16 ? round_to<FMSMO_F16>(v) : out_dt == FMSMO_BF16 ? round_to<FMSMO_BF16>(v) : v;
-  }
-  __device__ __forceinline__ Col col(int n, int, int) const {
-    Col c{1.0f, -0.0f};
-    if (mode == CHUNK_EPI_RAW) return c;
-    c.ws = w_scale[w_stride ? n : 0];
-    if (bias) {
-      c.b = bias_dt == FMSMO_F16 ? load_as_f32<FMSMO_F16>(bias, n)
-            : bias_dt == FMSMO_BF16 ? load_as_f32<FMSMO_BF16>(bias, n) : load_as_f32<FMSMO_F32>(bias, n);
-      if (mode == FMSMO_EPI_SEQ_OUT) c.b = to_out_grid(c.b);
-    }
-    return c;
-  }
-  __device__ __forceinline__ Row row(int m) const {
-    return Row{mode == CHUNK_EPI_RAW ? 1.0f : a_scale[a_stride ? m : 0]};
-  }
-  __device__ __forceinline__ void store(int m, int n, AccT v, Row r, Col c) const {
-    const int64_t idx = (int64_t)m * ldy + n;
-    if (mode == CHUNK_EPI_RAW) {
-      ((AccT*)y)[idx] = v;
-      return;
-    }
-    float t;
-    if (mode == FMSMO_EPI_REF_F16) {
-      const float sc = round_to<FMSMO_F16>(__fmul_rn(r.as, c.ws));
-      t = __fadd_rn(__fmul_rn((float)v, sc), c.b);
-      if (out_dt != FMSMO_F32) t = round_to<FMSMO_F16>(t);  // the fp16 accumulator dtype, then the output dtype
-    } else if (mode == FMSMO_EPI_F32) {
-      t = __fmaf_rn((float)v, __fmul_rn(r.as, c.ws), c.b);
-    } else if (mode == FMSMO_EPI_F32_MULADD) {
-      t = __fadd_rn(__fmul_rn((float)v, __fmul_rn(r.as, c.ws)), c.b);
-    } else {
-      t = to_out_grid(__fmul_rn(__fmul_rn((float)v, r.as), c.ws));
-      if (bias) t = __fadd_rn(t, c.b);
-    }
-    if (out_dt == FMSMO_F16) store_from_f32<FMSMO_F16>(y, idx, t);
-    else if (out_dt == FMSMO_BF16) store_from_f32<FMSMO_BF16>(y, idx, t);
-    else ((float*)y)[idx] = t;
-  }
 };
 
 template <int OP>
@@ -281,20 +213,18 @@ __global__ __launch_bounds__(256) void chunk_matmul_kernel(ChunkArgs g, EpiChunk
   }
   if (in_chunk != 0) finish_chunk();  // zero-padded K tail
 
+  // finished half a wave tile (32 rows) at a time in the wave's quarter of the stage buffers
+  Elem* const mine = (Elem*)&lds[0][0] + wave * (32 * 64);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 2; ++i) {
+    __syncthreads();
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = row0 + wm * 64 + i * 32 + (v >> 2) * 8 + fg * 4 + (v & 3);
-      if (m < g.M) {
-        const auto rowctx = epi.row(m);
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int n = col0 + wn * 64 + j * 32 + fr;
-          if (n < g.N) epi.store(m, n, acc[i][j][v], rowctx, epi.col(n, 0, g.N));
-        }
-      }
-    }
+      for (int v = 0; v < 16; ++v) mine[((v >> 2) * 8 + fg * 4 + (v & 3)) * 64 + j * 32 + fr] = acc[i][j][v];
+    __syncthreads();
+    chunk_finish(epi, mine, 32, row0 + wm * 64 + i * 32, col0 + wn * 64, g.M, g.N, lane);
+  }
 }
 
 }  // namespace fmsmo
@@ -302,59 +232,38 @@ __global__ __launch_bounds__(256) void chunk_matmul_kernel(ChunkArgs g, EpiChunk
 using namespace fmsmo;
 int fmsmo_check_launch();
 
-// Pipelined path: the tile GEMM kernel with the chunk hook.  Needs whole 64-byte K stages and
-// 32-bit row offsets; the K tail inside the last chunk (K not a multiple of the chunk) is
-// finished after the loop like any chunk.
+// Pipelined path.  Needs 32-bit row offsets (chunks are whole 32-byte k-steps: a power of two of at
+// least 32 bytes).
 template <int MMA, class Epi>
 static bool launch_chunk_tile(const ChunkArgs& c, const Epi& epi, hipStream_t st) {
-  if (c.Kb % 64 || c.chunk_bytes % 32 || (int64_t)c.M * c.lda >= (1ll << 31) ||
-      (int64_t)c.N * c.ldb >= (1ll << 31))
+  if (c.chunk_bytes % 32 || (int64_t)c.M * c.lda >= (1ll << 31) || (int64_t)c.N * c.ldb >= (1ll << 31))
     return false;
-  GemmArgs g{};
+  ChunkTileArgs g{};
   g.a = c.a; g.b = c.b; g.lda = c.lda; g.ldb = c.ldb;
   g.M = c.M; g.N = c.N; g.K = c.Kb;
-  g.grid_m = div_up(c.M, 128); g.grid_n = div_up(c.N, 128); g.group_m = 8;
+  g.grid_m = div_up(c.M, 128); g.grid_n = div_up(c.N, 128);
+  g.chunk_ks = c.chunk_bytes / 32;
+  g.t = c.dl16 ? 14 : c.trun_bits;
+  g.round_bit = g.t > 0 ? 1u << (g.t - 1) : 0u;
+  g.mask = ~((1u << g.t) - 1u);
+  g.lo = c.max_acc_bits < 32 ? -(1 << (c.max_acc_bits - 1)) : (int)0x80000000;
+  g.hi = c.max_acc_bits < 32 ? (1 << (c.max_acc_bits - 1)) - 1 : 0x7fffffff;
+  g.post = c.dl16 || g.t > 0 || c.max_acc_bits < 32;
+  g.dl16 = c.dl16; g.tta = c.tta; g.c_in = c.c_in; g.ldc = c.ldc;
   const bool fast = c.tta && !c.dl16 && c.max_acc_bits >= 32;
-  ChunkTrunc<false> k{};
-  k.chunk_ks = c.chunk_bytes / 32;
-  k.t = c.dl16 ? 14 : c.trun_bits;
-  k.round_bit = k.t > 0 ? 1u << (k.t - 1) : 0u;
-  k.mask = ~((1u << k.t) - 1u);
-  k.lo = c.max_acc_bits < 32 ? -(1 << (c.max_acc_bits - 1)) : (int)0x80000000;
-  k.hi = c.max_acc_bits < 32 ? (1 << (c.max_acc_bits - 1)) - 1 : 0x7fffffff;
-  k.post = c.dl16 || k.t > 0 || c.max_acc_bits < 32;
-  k.dl16 = c.dl16; k.tta = c.tta; k.c_in = c.c_in; k.ldc = c.ldc;
-  dim3 grid((unsigned)(g.grid_m * g.grid_n)), block(256);
-  // the schedules that round one block while the matrix unit multiplies the others: a chunk of one
-  // 64-byte stage (every operand type), of several stages or of one 32-byte k-step (int8)
-  const int sched = !fast ? 0 : c.chunk_bytes == 64 ? 1 : MMA != MMA_I8 ? 0 : c.chunk_bytes == 32 ? 3
-                    : c.chunk_bytes % 64 == 0 ? 2 : 0;
-#define LAUNCH_SCHED(SV)                                                                             \
-  {                                                                                                  \
-    ChunkTrunc<true, SV> kf{};                                                                       \
-    kf.chunk_ks = k.chunk_ks; kf.t = k.t; kf.round_bit = k.round_bit; kf.mask = k.mask;              \
-    kf.lo = k.lo; kf.hi = k.hi; kf.post = k.post; kf.dl16 = 0; kf.tta = 1;                           \
-    kf.c_in = k.c_in; kf.ldc = k.ldc;                                                                \
-    hipLaunchKernelGGL((gemm_tile_kernel<128, 128, 64, 4, 2, 2, MMA, 1, false, Epi, ChunkTrunc<true, SV>>), \
-                       grid, block, 0, st, g, epi, kf);                                              \
-  }
-  if (sched == 1) {
-    LAUNCH_SCHED(1)
-  } else if (sched == 2) {
-    if constexpr (MMA == MMA_I8) LAUNCH_SCHED(2)
-  } else if (sched == 3) {
-    if constexpr (MMA == MMA_I8) LAUNCH_SCHED(3)
-  } else if (fast) {
-    ChunkTrunc<true> kf{};
-    kf.chunk_ks = k.chunk_ks; kf.t = k.t; kf.round_bit = k.round_bit; kf.mask = k.mask;
-    kf.lo = k.lo; kf.hi = k.hi; kf.post = k.post; kf.dl16 = 0; kf.tta = 1;
-    kf.c_in = k.c_in; kf.ldc = k.ldc;
-    hipLaunchKernelGGL((gemm_tile_kernel<128, 128, 64, 4, 2, 2, MMA, 1, false, Epi, ChunkTrunc<true>>),
-                       grid, block, 0, st, g, epi, kf);
-  } else {
-    hipLaunchKernelGGL((gemm_tile_kernel<128, 128, 64, 4, 2, 2, MMA, 1, false, Epi, ChunkTrunc<false>>),
-                       grid, block, 0, st, g, epi, k);
-  }
+  const dim3 grid((unsigned)(g.grid_m * g.grid_n)), block(256);
+  auto go = [&](auto kt_c) {
+    constexpr bool KT = decltype(kt_c)::value;
+    // the schedules that round one block while the matrix unit multiplies the others: a chunk of one
+    // 64-byte stage (every operand type), of several stages or of one 32-byte k-step (int8)
+    if (!fast) hipLaunchKernelGGL((chunk_tile_kernel<MMA, false, 0, KT>), grid, block, 0, st, g, epi);
+    else if (c.chunk_bytes == 64) hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 1, KT>), grid, block, 0, st, g, epi);
+    else if constexpr (MMA != MMA_I8) hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 0, KT>), grid, block, 0, st, g, epi);
+    else if (c.chunk_bytes == 32) hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 3, KT>), grid, block, 0, st, g, epi);
+    else hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 2, KT>), grid, block, 0, st, g, epi);
+  };
+  if (g.K % 64) go(std::true_type{});
+  else go(std::false_type{});
   return true;
 }
 
@@ -379,6 +288,21 @@ static int check_chunk_dq(const float* a_scale, int64_t a_scale_n, const float* 
   if (y_dtype < 0 || y_dtype > 2 || (bias && (bias_dtype < 0 || bias_dtype > 2))) return FMSMO_ERR_UNSUPPORTED;
   if (epilogue < FMSMO_EPI_REF_F16 || epilogue > FMSMO_EPI_SEQ_OUT) return FMSMO_ERR_UNSUPPORTED;
   return FMSMO_OK;
+}
+
+template <class AccT>
+static EpiChunk<AccT> epi_raw(void* d, int64_t ldd) {
+  EpiChunk<AccT> e{};
+  e.y = d; e.ldy = ldd; e.mode = CHUNK_EPI_RAW;
+  e.vec4 = ldd % 4 == 0 && ((uintptr_t)d & 15) == 0;
+  return e;
+}
+template <class AccT>
+static EpiChunk<AccT> epi_dq(const float* a_scale, int64_t a_scale_n, const float* w_scale, int64_t w_scale_n,
+                             const void* bias, int bias_dtype, int epilogue, void* y, int y_dtype, int64_t ldy) {
+  return EpiChunk<AccT>{y, ldy, a_scale, w_scale, bias, a_scale_n == 1 ? 0 : 1, w_scale_n == 1 ? 0 : 1, epilogue,
+                        y_dtype, bias ? bias_dtype : FMSMO_F32,
+                        ldy % 4 == 0 && ((uintptr_t)y & (y_dtype == FMSMO_F32 ? 15 : 7)) == 0};
 }
 
 static int run_chunk_i8(const ChunkArgs& g, const EpiChunk<int>& epi, hipStream_t st) {
@@ -433,9 +357,7 @@ extern "C" int fmsmo_matmul_chunk_i8(const int8_t* a, int64_t lda, const int8_t*
     return fmsmo_gemm_i8_i32(a, lda, b, ldb, d, ldd, M, N, K, stream);
   const ChunkArgs g = chunk_args_i8(a, lda, b, ldb, M, N, K, chunk_size, chunk_trun_bits, max_acc_bits,
                                     truncate_then_accumulate, c_in, ldd);
-  EpiChunk<int> epi{};
-  epi.y = d; epi.ldy = ldd; epi.mode = CHUNK_EPI_RAW;
-  return run_chunk_i8(g, epi, (hipStream_t)stream);
+  return run_chunk_i8(g, epi_raw<int>(d, ldd), (hipStream_t)stream);
 }
 
 extern "C" int fmsmo_matmul_chunk_i8_dq(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
@@ -458,8 +380,7 @@ extern "C" int fmsmo_matmul_chunk_i8_dq(const int8_t* a, int64_t lda, const int8
                             epilogue, y, y_dtype, ldy, M, N, K, stream);
   const ChunkArgs g = chunk_args_i8(a, lda, b, ldb, M, N, K, chunk_size, chunk_trun_bits, max_acc_bits,
                                     truncate_then_accumulate, nullptr, 0);
-  EpiChunk<int> epi{y, ldy, a_scale, w_scale, bias, a_scale_n == 1 ? 0 : 1, w_scale_n == 1 ? 0 : 1,
-                    epilogue, y_dtype, bias ? bias_dtype : FMSMO_F32};
+  const EpiChunk<int> epi = epi_dq<int>(a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype, epilogue, y, y_dtype, ldy);
   return run_chunk_i8(g, epi, (hipStream_t)stream);
 }
 
@@ -493,9 +414,7 @@ extern "C" int fmsmo_matmul_chunk_fp(const void* a, int64_t lda, const void* b, 
                          clamp_dl16, truncate_then_accumulate, c_in, ldd, &g);
   if (rc) return rc;
   if (M == 0) return FMSMO_OK;
-  EpiChunk<float> epi{};
-  epi.y = d; epi.ldy = ldd; epi.mode = CHUNK_EPI_RAW;
-  return run_chunk_fp(op_dtype, g, epi, (hipStream_t)stream);
+  return run_chunk_fp(op_dtype, g, epi_raw<float>(d, ldd), (hipStream_t)stream);
 }
 
 extern "C" int fmsmo_matmul_chunk_fp_dq(const void* a, int64_t lda, const void* b, int64_t ldb,
@@ -512,7 +431,6 @@ extern "C" int fmsmo_matmul_chunk_fp_dq(const void* a, int64_t lda, const void* 
   rc = check_chunk_dq(a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype, epilogue, y_dtype, M, N);
   if (rc) return rc;
   if (M == 0) return FMSMO_OK;
-  EpiChunk<float> epi{y, ldy, a_scale, w_scale, bias, a_scale_n == 1 ? 0 : 1, w_scale_n == 1 ? 0 : 1,
-                      epilogue, y_dtype, bias ? bias_dtype : FMSMO_F32};
+  const EpiChunk<float> epi = epi_dq<float>(a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype, epilogue, y, y_dtype, ldy);
   return run_chunk_fp(op_dtype, g, epi, (hipStream_t)stream);
 }

@@ -113,8 +113,8 @@ void launch_tile(const GemmArgs& g0, const Epi& epi, hipStream_t st) {
   dim3 grid((unsigned)(g.grid_m * g.grid_n)), block(Tile::WGM * Tile::WGN * 64);
   hipLaunchKernelGGL(
       (gemm_tile_kernel<Tile::BM, Tile::BN, Tile::BK, Tile::NST, Tile::WGM, Tile::WGN, OP, 1,
-                        GROUPED, Epi, NoChunk, KT>),
-      grid, block, 0, st, g, epi, NoChunk{});
+                        GROUPED, Epi, KT>),
+      grid, block, 0, st, g, epi);
 }
 
 // 256x256 tiles with K a multiple of 128 run the register-staged pipeline (gemm_rs.hpp: whole

@@ -93,36 +93,6 @@ struct Mma<MMA_FP8> {
   }
 };
 
-// 32-byte k-steps for the chunked-accumulation kernels (chunk boundaries are multiples of 32
-// bytes of K for every operand type): two legacy K=16 e4m3 MFMAs, one K=16 f16 / bf16 MFMA, four
-// K=2 fp32 MFMAs per 16-byte lane operand.
-template <>
-struct Mma<MMA_FP8_K32> {
-  typedef v4i Frag;
-  typedef v16f Acc;
-  typedef float Elem;
-  static constexpr int KSTEP = 32;
-  __device__ static __forceinline__ Acc mma(const Frag& a, const Frag& b, const Acc& c) {
-    const long a0 = ((long)(unsigned)a[1] << 32) | (unsigned)a[0];
-    const long a1 = ((long)(unsigned)a[3] << 32) | (unsigned)a[2];
-    const long b0 = ((long)(unsigned)b[1] << 32) | (unsigned)b[0];
-    const long b1 = ((long)(unsigned)b[3] << 32) | (unsigned)b[2];
-    Acc t = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(a0, b0, c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(a1, b1, t, 0, 0, 0);
-  }
-};
-template <>
-struct Mma<MMA_F16> {
-  typedef v4i Frag;
-  typedef v16f Acc;
-  typedef float Elem;
-  static constexpr int KSTEP = 32;
-  typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-  __device__ static __forceinline__ Acc mma(const Frag& a, const Frag& b, const Acc& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a),
-                                                  __builtin_bit_cast(v8h, b), c, 0, 0, 0);
-  }
-};
 // e4m3 operands widened to fp16 (exact) on their way from LDS into the fp16 matrix instruction, which adds
 // their products as accurately as fp32 additions one after the other do (2-norm error of the sum against
 // 64 bits at K = 544 / 1136 / 11472: 4.5e-9 / 1.4e-8 / 5.7e-8, the additions 4.7e-9 / 1.4e-8 / 8.6e-8; the
@@ -148,78 +118,6 @@ struct Mma<MMA_FP8_F16> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(widen(a[2], a[3]), widen(b[2], b[3]), t, 0, 0, 0);
   }
 };
-template <>
-struct Mma<MMA_BF16> {
-  typedef v4i Frag;
-  typedef v16f Acc;
-  typedef float Elem;
-  static constexpr int KSTEP = 32;
-  typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-  __device__ static __forceinline__ Acc mma(const Frag& a, const Frag& b, const Acc& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a),
-                                                   __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-  }
-};
-template <>
-struct Mma<MMA_F32> {
-  typedef v4i Frag;
-  typedef v16f Acc;
-  typedef float Elem;
-  static constexpr int KSTEP = 32;
-  __device__ static __forceinline__ Acc mma(const Frag& a, const Frag& b, const Acc& c) {
-    Acc t = c;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      t = __builtin_amdgcn_mfma_f32_32x32x2f32(__int_as_float(a[e]), __int_as_float(b[e]), t, 0, 0, 0);
-    return t;
-  }
-};
-
-// ---- chunked accumulation: every `chunk_ks` MFMA k-steps the partial product is range-clamped /
-// LSB-rounded and folded into the running accumulator (or the running accumulator itself is
-// rounded when tta == 0).
-struct NoChunk {
-  static constexpr bool enabled = false;
-  static constexpr bool fast = false;
-  static constexpr bool one_stage = false;
-};
-// FAST = the common configuration (truncate-then-accumulate, no integer clamp, no DL16 clamp):
-// three vector ALU operations per accumulator element and chunk.
-// ONE_STAGE (with FAST) = the schedules that interleave the rounding of one 32x32 block with the
-// MFMAs of the others inside one wave (see the loop in gemm_tile_kernel): integers with any chunk
-// of one k-step or of whole LDS stages, floating point with a chunk of exactly one stage.
-// SCHED: 1 = a chunk is one stage, 2 = several whole stages, 3 = one k-step (integers only); each is
-// a kernel of its own (one kernel holding all three loops runs out of registers).
-template <bool FAST, int SCHED = 0>
-struct ChunkTrunc {
-  static_assert(FAST || SCHED == 0, "the interleaved schedules exist for the fast configuration only");
-  static constexpr bool enabled = true;
-  static constexpr bool fast = FAST;
-  static constexpr bool one_stage = SCHED != 0;
-  static constexpr int sched = SCHED;
-  int chunk_ks;           // MFMA k-steps (32 bytes of K) per chunk
-  int t, lo, hi;          // LSBs to round away; integer clamp range
-  unsigned round_bit, mask;
-  int post, dl16, tta;
-  const void* c_in;       // optional initial accumulator [M, N], same element type as the output
-  int64_t ldc;
-};
-__device__ __forceinline__ int trunc_i32(int p, int lo, int hi, int round_bit, int t) {
-  p = max(min(p, hi), lo);
-  // (p + 2^(t-1)) >> t << t with two's-complement wrap on the add, arithmetic right shift
-  p = (int)((unsigned)p + (unsigned)round_bit);
-  return (int)((unsigned)(p >> t) << t);
-}
-__device__ __forceinline__ float trunc_f32(float p, unsigned round_bit, unsigned mask, int dl16) {
-  float x = __uint_as_float((__float_as_uint(p) + round_bit) & mask);
-  if (dl16) {
-    x = x >= 8581545984.0f ? __builtin_inff() : x;
-    x = x <= -8581545984.0f ? -__builtin_inff() : x;
-    x = fabsf(x) < 4.665707820095122e-10f ? 0.0f : x;
-  }
-  return x;
-}
-
 // Position `pid` of the tile sequence: column-major inside groups of `group_m` tile rows (the
 // second half of tile_of_block below, for blocks that walk the sequence themselves).
 __device__ __forceinline__ void tile_of_pid(int pid, int grid_m, int grid_n, int group_m, int& tm, int& tn) {
@@ -251,10 +149,8 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblk, int grid_m, int
 }
 
 template <int BM, int BN, int BK, int NSTAGE, int WGM, int WGN, int OP, int SWZ, bool GROUPED,
-          class Epi, class Chk = NoChunk, bool KT = false>
-// (KT: without chunk hooks only.  Two blocks per compute unit for the scheduled chunk hooks; the generic hook keeps a second
-// accumulator set and would spill at 256 registers)
-__global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1) void gemm_tile_kernel(GemmArgs g, Epi epi, Chk chk) {
+          class Epi, bool KT = false>
+__global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_tile_kernel(GemmArgs g, Epi epi) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
   typedef Mma<OP> MM;
   typedef typename MM::Frag Frag;
@@ -269,7 +165,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
   constexpr int CL = MM::KSTEP / 32;           // 16-byte chunks per lane per k-step
   static_assert(RPI % 16 == 0 && BM % RPI == 0 && BN % RPI == 0, "loader shape");
   static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile");
-  static_assert(!KT || !Chk::enabled, "chunks end with whole stages");
 
   constexpr int STAGE_BYTES = (BM + BN) * BK;
   __shared__ __attribute__((aligned(16))) uint8_t lds[NSTAGE][STAGE_BYTES];
@@ -381,85 +276,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
 
-  // chunked accumulation: MFMAs run into `work`, finished chunks are folded into `acc`
-  typedef typename MM::Elem Elem;
-  Acc work[Chk::enabled ? FM : 1][Chk::enabled ? FN : 1];
-  int ks_cnt = 0;
-  if constexpr (Chk::enabled) {
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          Elem init = 0;
-          if (chk.c_in) {
-            const int m = row_lo + wm * TM + i * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-            const int n = col_lo + wn * TN + j * 32 + (lane & 31);
-            if (m < row_hi && n < g.N) init = ((const Elem*)chk.c_in)[(int64_t)m * chk.ldc + n];
-          }
-          acc[i][j][v] = chk.tta ? init : (Elem)0;
-          work[i][j][v] = chk.tta ? (Elem)0 : init;
-        }
-  }
-  auto finish_chunk = [&](auto post_c, auto tta_c) __attribute__((always_inline)) {
-    constexpr bool POST = decltype(post_c)::value, TTA = decltype(tta_c)::value;
-    if constexpr (Chk::enabled) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            Elem p = work[i][j][v];
-            if constexpr (POST) {
-              if constexpr (std::is_same<Elem, int>::value) p = trunc_i32(p, chk.lo, chk.hi, (int)chk.round_bit, chk.t);
-              else p = trunc_f32(p, chk.round_bit, chk.mask, chk.dl16);
-            }
-            if constexpr (TTA) {
-              if constexpr (std::is_same<Elem, int>::value) acc[i][j][v] = (int)((unsigned)acc[i][j][v] + (unsigned)p);
-              else acc[i][j][v] += p;
-              work[i][j][v] = 0;
-            } else {
-              work[i][j][v] = p;  // the running accumulator itself is rounded
-            }
-          }
-    }
-  };
-  auto finish_any = [&]() __attribute__((always_inline)) {
-    if constexpr (Chk::fast) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            // (p + 2^(t-1)) with the low t bits cleared: same bits for two's-complement integers
-            // ((p + r) >> t << t) and for fp32 patterns; work is overwritten by the next chunk
-            if constexpr (std::is_same<Elem, int>::value) {
-              acc[i][j][v] = (int)((unsigned)acc[i][j][v] + (((unsigned)work[i][j][v] + chk.round_bit) & chk.mask));
-            } else {
-              acc[i][j][v] += __uint_as_float((__float_as_uint(work[i][j][v]) + chk.round_bit) & chk.mask);
-            }
-          }
-    } else if constexpr (Chk::enabled) {
-      if (chk.tta) {
-        if (chk.post) finish_chunk(std::true_type{}, std::true_type{});
-        else finish_chunk(std::false_type{}, std::true_type{});
-      } else if (chk.post) {
-        finish_chunk(std::true_type{}, std::false_type{});
-      }
-    }
-  };
-  auto chunk_tick = [&]() __attribute__((always_inline)) {
-    if constexpr (Chk::enabled) {
-      if (++ks_cnt == chk.chunk_ks) {
-        finish_any();
-        ks_cnt = 0;
-      }
-    }
-  };
-
   auto read_frags = [&](const uint8_t* ls, int s, Frag* af, Frag* bf) {
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
@@ -486,29 +302,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        if constexpr (Chk::enabled) work[i][j] = MM::mma(af[i], bf[j], work[i][j]);
-        else acc[i][j] = MM::mma(af[i], bf[j], acc[i][j]);
-      }
-  };
-  // first k-step of a chunk in FAST mode: the MFMA's C operand is the constant 0, so `work` needs
-  // no clearing between chunks
-  auto mma_step_fresh = [&](const Frag* af, const Frag* bf) {
-    Acc zero;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) zero[v] = 0;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) work[i][j] = MM::mma(af[i], bf[j], zero);
-  };
-  auto mma_any = [&](const Frag* af, const Frag* bf) __attribute__((always_inline)) {
-    if constexpr (Chk::fast) {
-      if (ks_cnt == 0) mma_step_fresh(af, bf);
-      else mma_step(af, bf);
-    } else {
-      mma_step(af, bf);
-    }
+      for (int j = 0; j < FN; ++j) acc[i][j] = MM::mma(af[i], bf[j], acc[i][j]);
   };
   // Instruction-order hints (DS read = 0x100, MFMA = 0x008, VMEM = 0x020): the operand reads of
   // the next k-step go between the first MFMAs of the current one, so their latency is covered
@@ -592,9 +386,8 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
           [&] {
             read_frags(ls, S + 1, fa[(PAR + S + 1) & 1], fb[(PAR + S + 1) & 1]);
             dma(std::integral_constant<int, S>{});
-            mma_any(fa[(PAR + S) & 1], fb[(PAR + S) & 1]);
+            mma_step(fa[(PAR + S) & 1], fb[(PAR + S) & 1]);
             interleave(std::integral_constant<int, NLD * (S + 1) / NKS - NLD * S / NKS>{});
-            chunk_tick();
           }(),
           ...);
     }(std::make_integer_sequence<int, NKS - 1>{});
@@ -611,9 +404,8 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
     const int nxt = (kt + 1) % NSTAGE;
     read_frags(&lds[0][0] + nxt * STAGE_BYTES, 0, fa[(PAR + NKS) & 1], fb[(PAR + NKS) & 1]);
     dma(std::integral_constant<int, NKS - 1>{});
-    mma_any(fa[(PAR + NKS - 1) & 1], fb[(PAR + NKS - 1) & 1]);
+    mma_step(fa[(PAR + NKS - 1) & 1], fb[(PAR + NKS - 1) & 1]);
     interleave(std::integral_constant<int, NLD - NLD * (NKS - 1) / NKS>{});
-    chunk_tick();
   };
 
 #pragma unroll
@@ -629,209 +421,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
   } else {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NSTAGE - 2) * NLD) : "memory");
   }
-  if constexpr (Chk::one_stage) {
-    // Chunk == stage: the fragments of all k-steps of a chunk are register resident (two sets:
-    // the stage being multiplied and the one being read), and the rounding of one 32x32 block is
-    // issued between the MFMAs of the others, so that one wave keeps both units busy.  With all
-    // MFMAs of a chunk issued before any rounding (the generic schedule) the units take turns, and
-    // only a second resident wave overlaps them -- which a problem with about one tile per compute
-    // unit does not have.
-    Frag ca[2][NKS][FM], cb[2][NKS][FN];
-    constexpr bool INT = std::is_same<Elem, int>::value;
-    auto stage_top = [&](int kt, auto par_c) {
-      constexpr int PAR = decltype(par_c)::value;
-      // stage kt + 1 has landed for every wave; its fragments go to the other register set, and
-      // the buffer of stage kt - 1 (last read a stage ago) is refilled with stage kt + 3
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NSTAGE - 3) * NLD) : "memory");
-      const uint8_t* ls = &lds[0][0] + ((kt + 1) % NSTAGE) * STAGE_BYTES;
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) read_frags(ls, ks, ca[PAR ^ 1][ks], cb[PAR ^ 1][ks]);
-      issue_part((kt + NSTAGE - 1) % NSTAGE, min(kt + NSTAGE - 1, nk - 1) * BK,
-                 std::integral_constant<int, 0>{}, std::integral_constant<int, NLD>{});
-      __builtin_amdgcn_sched_barrier(0);
-    };
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) read_frags(&lds[0][0], ks, ca[0][ks], cb[0][ks]);
-    if constexpr (INT) {
-      // Integers: with R the running sum (a multiple of 2^t) and r the rounding bit, a chunk's
-      // MFMAs started from C = R + r leave W = R + p + r, and (W & mask) = R + ((p + r) & mask) is
-      // the new running sum: ONE operation per element and chunk, W <- (W & mask) | r, turns the
-      // accumulator into the next chunk's C operand (low bits are zero, so OR adds r), and the
-      // matrix unit does the accumulation.  8 such operations take as long as one MFMA, and a
-      // chunk has 8 MFMAs and 64 elements per lane: the steady state below issues 8 operations in
-      // front of every MFMA.  Block b's k-steps are two MFMA slots apart, its 16 operations follow
-      // its second MFMA by a slot or more and are complete before its next first MFMA:
-      //   slot       0       1       2       3       4       5       6       7
-      //   rounding   b1 hi'  b2 lo'  b2 hi'  b3 lo'  b3 hi'  b0 lo   b0 hi   b1 lo    (' = previous chunk)
-      //   MFMA       b0 k0   b1 k0   b0 k1   b1 k1   b2 k0   b3 k0   b2 k1   b3 k1
-      // (a chunk of several stages rounds behind its last stage only; a chunk of one k-step has a
-      // table of its own below)
-      // Rounding an accumulator that holds C = R + r changes nothing, so the first chunk runs the
-      // same code.  An initial accumulator enters as its multiple of 2^t; its low bits are added
-      // at the end (adding a multiple of 2^t commutes with clearing the low bits).
-      static_assert(NKS == 2 && FM == 2 && FN == 2, "the slot table is written for 2 k-steps x 4 blocks");
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int jj = 0; jj < FN; ++jj)
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            work[i][jj][v] = (int)(((unsigned)acc[i][jj][v] & chk.mask) | chk.round_bit);
-      // (one v_and_or_b32: the instruction takes a single scalar operand, so the rounding bit
-      // lives in a vector register)
-      unsigned rbv = chk.round_bit;
-      asm volatile("" : "+v"(rbv));
-      auto rnd = [&](auto b_c, auto h_c) {
-        constexpr int I = decltype(b_c)::value / FN, J = decltype(b_c)::value % FN, H = decltype(h_c)::value;
-#pragma unroll
-        for (int v = H * 8; v < H * 8 + 8; ++v)
-          work[I][J][v] = (int)(((unsigned)work[I][J][v] & chk.mask) | rbv);
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      auto mm = [&](auto par_c, auto b_c, auto ks_c) {
-        constexpr int PAR = decltype(par_c)::value, KS = decltype(ks_c)::value;
-        constexpr int I = decltype(b_c)::value / FN, J = decltype(b_c)::value % FN;
-        work[I][J] = MM::mma(ca[PAR][KS][I], cb[PAR][KS][J], work[I][J]);
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      typedef std::integral_constant<int, 0> I0;
-      typedef std::integral_constant<int, 1> I1;
-      typedef std::integral_constant<int, 2> I2;
-      typedef std::integral_constant<int, 3> I3;
-      if constexpr (Chk::sched == 1) {
-        // a chunk is one stage: the table as it stands
-        auto chunk_stage = [&](int kt, auto par_c) {
-          stage_top(kt, par_c);
-          rnd(I1{}, I1{}); mm(par_c, I0{}, I0{});
-          rnd(I2{}, I0{}); mm(par_c, I1{}, I0{});
-          rnd(I2{}, I1{}); mm(par_c, I0{}, I1{});
-          rnd(I3{}, I0{}); mm(par_c, I1{}, I1{});
-          rnd(I3{}, I1{}); mm(par_c, I2{}, I0{});
-          rnd(I0{}, I0{}); mm(par_c, I3{}, I0{});
-          rnd(I0{}, I1{}); mm(par_c, I2{}, I1{});
-          rnd(I1{}, I0{}); mm(par_c, I3{}, I1{});
-        };
-        int kt = 0;
-        for (; kt + 1 < nk; kt += 2) {
-          chunk_stage(kt, I0{});
-          chunk_stage(kt + 1, I1{});
-        }
-        if (kt < nk) chunk_stage(kt, I0{});
-      } else if constexpr (Chk::sched == 2) {
-        // a chunk is several whole stages: the roundings run only behind a chunk's last stage
-        // (slots 5 - 7 of that stage, slots 0 - 4 of the following one)
-        const int spc = chk.chunk_ks / NKS;
-        int phase = 0;  // stage index inside the chunk
-        auto chunk_stage = [&](int kt, auto par_c) {
-          stage_top(kt, par_c);
-          const bool prev_end = phase == 0, this_end = phase + 1 == spc;
-          phase = this_end ? 0 : phase + 1;
-          if (prev_end) rnd(I1{}, I1{});
-          mm(par_c, I0{}, I0{});
-          if (prev_end) rnd(I2{}, I0{});
-          mm(par_c, I1{}, I0{});
-          if (prev_end) rnd(I2{}, I1{});
-          mm(par_c, I0{}, I1{});
-          if (prev_end) rnd(I3{}, I0{});
-          mm(par_c, I1{}, I1{});
-          if (prev_end) rnd(I3{}, I1{});
-          mm(par_c, I2{}, I0{});
-          if (this_end) rnd(I0{}, I0{});
-          mm(par_c, I3{}, I0{});
-          if (this_end) rnd(I0{}, I1{});
-          mm(par_c, I2{}, I1{});
-          if (this_end) rnd(I1{}, I0{});
-          mm(par_c, I3{}, I1{});
-        };
-        int kt = 0;
-        for (; kt + 1 < nk; kt += 2) {
-          chunk_stage(kt, I0{});
-          chunk_stage(kt + 1, I1{});
-        }
-        if (kt < nk) chunk_stage(kt, I0{});
-      } else {
-        // a chunk is one k-step (32 bytes of K): 16 roundings per MFMA, the vector ALU is the
-        // bound (half the MFMA rate at best).  Per k-step: MFMA b0, round b2', MFMA b1, round b3',
-        // MFMA b2, round b0, MFMA b3, round b1 (' = of the previous k-step).
-        auto chunk_stage = [&](int kt, auto par_c) {
-          stage_top(kt, par_c);
-          [&]<int... KS>(std::integer_sequence<int, KS...>) {
-            (
-                [&] {
-                  typedef std::integral_constant<int, KS> CK;
-                  mm(par_c, I0{}, CK{}); rnd(I2{}, I0{}); rnd(I2{}, I1{});
-                  mm(par_c, I1{}, CK{}); rnd(I3{}, I0{}); rnd(I3{}, I1{});
-                  mm(par_c, I2{}, CK{}); rnd(I0{}, I0{}); rnd(I0{}, I1{});
-                  mm(par_c, I3{}, CK{}); rnd(I1{}, I0{}); rnd(I1{}, I1{});
-                }(),
-                ...);
-          }(std::make_integer_sequence<int, NKS>{});
-        };
-        int kt = 0;
-        for (; kt + 1 < nk; kt += 2) {
-          chunk_stage(kt, I0{});
-          chunk_stage(kt + 1, I1{});
-        }
-        if (kt < nk) chunk_stage(kt, I0{});
-      }
-      // the sum of the rounded chunks, plus the low bits of the initial accumulator (read again
-      // here: holding it in registers through the loop would cost 64 of them)
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int jj = 0; jj < FN; ++jj)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            unsigned low = 0;
-            if (chk.c_in) {
-              const int m = row_lo + wm * TM + i * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-              const int n = col_lo + wn * TN + jj * 32 + (lane & 31);
-              if (m < row_hi && n < g.N) low = (unsigned)((const int*)chk.c_in)[(int64_t)m * chk.ldc + n] & ~chk.mask;
-            }
-            acc[i][jj][v] = (int)(((unsigned)work[i][jj][v] & chk.mask) + low);
-          }
-    } else {
-      // Floating point: the rounding works on the bits of the chunk's own sum, which is then added
-      // in fp32 -- three operations per element (integer add, and, float add).  Block b's MFMAs
-      // start from C = 0; block b - 1 is folded into `acc` while they run.
-      Acc zero;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) zero[v] = 0;
-      auto fold = [&](auto b_c) {
-        constexpr int I = decltype(b_c)::value / FN, J = decltype(b_c)::value % FN;
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          acc[I][J][v] += __uint_as_float((__float_as_uint(work[I][J][v]) + chk.round_bit) & chk.mask);
-      };
-      auto chunk_stage = [&](int kt, auto par_c) {
-        constexpr int PAR = decltype(par_c)::value;
-        stage_top(kt, par_c);
-        [&]<int... B>(std::integer_sequence<int, B...>) {
-          (
-              [&] {
-                constexpr int I = B / FN, J = B % FN;
-                work[I][J] = MM::mma(ca[PAR][0][I], cb[PAR][0][J], zero);
-#pragma unroll
-                for (int ks = 1; ks < NKS; ++ks)
-                  work[I][J] = MM::mma(ca[PAR][ks][I], cb[PAR][ks][J], work[I][J]);
-                __builtin_amdgcn_sched_barrier(0);
-                // block B - 1 of this chunk, or the last block of the previous one (zeros before
-                // the first chunk: a zero block folds to zero)
-                fold(std::integral_constant<int, (B + NMMA - 1) % NMMA>{});
-                __builtin_amdgcn_sched_barrier(0);
-              }(),
-              ...);
-        }(std::make_integer_sequence<int, NMMA>{});
-      };
-      int kt = 0;
-      for (; kt + 1 < nk; kt += 2) {
-        chunk_stage(kt, std::integral_constant<int, 0>{});
-        chunk_stage(kt + 1, std::integral_constant<int, 1>{});
-      }
-      if (kt < nk) chunk_stage(kt, std::integral_constant<int, 0>{});
-      fold(std::integral_constant<int, NMMA - 1>{});
-    }
-  } else {
   read_frags(&lds[0][0], 0, fa[0], fb[0]);
   {
     int kt = 0;
@@ -845,18 +434,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, (Chk::enabled && Chk::fast) ? 2 : 1)
       if (kt < nk) stage(kt, std::integral_constant<int, 0>{});
     }
   }
-  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA may be in flight when LDS is released
-  if constexpr (Chk::enabled && !Chk::one_stage) {
-    if (ks_cnt != 0) finish_any();  // K ended inside a chunk
-    if (!chk.tta) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = work[i][j];
-    }
-  }
-
   // ---- epilogue: acc[i][j][v] is C(row, col) with
   //      row = 32 i + 8 (v / 4) + 4 (lane / 32) + v % 4,   col = 32 j + lane % 32
   const int m_base = row_lo + wm * TM + fg * 4;

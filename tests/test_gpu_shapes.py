@@ -411,3 +411,27 @@ def test_a_workspace_with_room_for_fewer_slices_is_used(dev, M, N, Kd):
         assert torch.equal(c, ref)
         assert bool((ws[:2 * M * N] != 0x55555555).any()) == (room > 1), room
         assert (ws[room * M * N:] == 0x55555555).all()
+
+
+@pytest.mark.parametrize("Kd", [16, 64, 272, 1000])          # shorter than a stage, one stage, cut last stages
+@pytest.mark.parametrize("M,N", [(1, 1), (65, 131), (128, 128), (130, 260)])
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn, torch.float16, torch.float32])
+def test_chunked_products_at_the_edges_of_tiles_and_of_the_reduction(dev, M, N, Kd, dtype):
+    """Integer-valued operands whose partial sums stay below 2^24: every chunk sum and every sum of rounded
+    chunks is exact in fp32 whatever its order, so the result is bit-pinned for all operand types."""
+    if dtype == torch.float32:
+        Kd = Kd // 4 * 4
+    elif Kd % 16:
+        Kd = Kd // 16 * 16
+    a = torch.randint(-6, 7, (M, Kd), generator=gen(M + Kd)).float().to(dtype)
+    w = torch.randint(-6, 7, (N, Kd), generator=gen(N + Kd + 1)).float().to(dtype)
+    for cs, t in ((32, 3), (64, 5), (128, 4)):
+        if dtype == torch.int8:
+            ref = O.chunk_matmul_i8(a, w, None, cs, t, 32)
+        else:
+            ref = O.chunk_matmul_fp(a.float(), w.float(), None, cs, t)
+        d = K().matmul_chunk(a.to(dev), w.to(dev), None, chunk_size=cs, chunk_trun_bits=t)
+        assert torch.equal(d.cpu(), ref), (cs, t)
+        one = torch.ones(1, device=dev)
+        y = K().matmul_chunk_dq(a.to(dev), w.to(dev), one, one, None, 1, torch.float32, chunk_size=cs, chunk_trun_bits=t)
+        assert torch.equal(y.cpu(), ref.float()), (cs, t)
