@@ -15,6 +15,7 @@
 // for every operand type, so chunk boundaries (multiples of 32 bytes) always fall between
 // k-steps.
 #include "chunk_tile.hpp"
+#include <algorithm>
 
 namespace fmsmo {
 
@@ -232,12 +233,48 @@ __global__ __launch_bounds__(256) void chunk_matmul_kernel(ChunkArgs g, EpiChunk
 using namespace fmsmo;
 int fmsmo_check_launch();
 
+// How the tiles of the pipelined kernel are laid over the 256 compute units: the tiles past the last whole
+// round of 256 are cut along K into `slices` pieces of whole chunks, where that is estimated to be faster.
+// (us, uncut -> cut as planned here, int8 chunk 64: 16 x 4096 x 14336 70.1 -> 17.2 in 8 slices, 512 rows 73.8 ->
+// 49.8 in 2, 1069 rows 126.4 -> 95.1 (32 of 288 tiles in 8), 100 x 700 x 8192 44.2 -> 12.2 in 16, 100 x 1024 x 2048
+// 16.5 -> 9.5 in 8; left whole: 300 x 4096 x 4096 26.7 with 96 tiles of 64 stages; fp16 chunk 32 100 x 4096 x 4096
+// 75.6 -> 20.4 in 8, 600 rows 77.0 -> 52.3 in 3; e4m3 chunk 64 1024 x 700 x 8192 84.6 -> 28.0 in 5)
+struct ChunkPlan {
+  int full, slices, slice_len;
+  int64_t ws_bytes;
+};
+static ChunkPlan plan_chunk(int mma, int64_t M, int64_t N, int64_t Kb, int64_t chunk_bytes, bool may_cut, int64_t limit) {
+  const int64_t tiles = (int64_t)div_up(M, 128) * div_up(N, 128), rest = tiles % 256;
+  ChunkPlan p{(int)tiles, 1, (int)Kb, 0};
+  if (!may_cut || rest == 0) return p;
+  const int64_t unit = std::max<int64_t>(64, chunk_bytes), units = (Kb + unit - 1) / unit;
+  // us: a round of one tile per compute unit takes `stage` per 64 bytes of K; a slice costs its first loads and
+  // its accumulators written and read again, the second launch 4
+  const double stage = mma == MMA_I8 ? 0.34 : mma == MMA_F32 ? 1.2 : 0.6;
+  const double rows = std::min<double>(1.0, (double)M / 128);
+  double best = stage * (Kb / 64.0);
+  for (int64_t s = 2; s <= std::min<int64_t>(units, 64); ++s) {
+    const int64_t len = (units + s - 1) / s;  // in units; the slices that are left
+    const int64_t n = (units + len - 1) / len, bytes = rest * n * 65536;
+    if (n != s || len * unit < 256) continue;
+    if (limit >= 0 && bytes > limit) break;
+    const double t = (double)((rest * n + 255) / 256) * (stage * (len * unit / 64.0) + 2.0) + 4.0 + bytes * rows / 2.5e6;
+    if (t < best) {
+      best = t;
+      p = ChunkPlan{(int)(tiles - rest), (int)n, (int)(len * unit), bytes};
+    }
+  }
+  return p;
+}
+
 // Pipelined path.  Needs 32-bit row offsets (chunks are whole 32-byte k-steps: a power of two of at
 // least 32 bytes).
-template <int MMA, class Epi>
-static bool launch_chunk_tile(const ChunkArgs& c, const Epi& epi, hipStream_t st) {
-  if (c.chunk_bytes % 32 || (int64_t)c.M * c.lda >= (1ll << 31) || (int64_t)c.N * c.ldb >= (1ll << 31))
-    return false;
+static bool chunk_tile_ok(const ChunkArgs& c) {
+  return c.chunk_bytes % 32 == 0 && (int64_t)c.M * c.lda < (1ll << 31) && (int64_t)c.N * c.ldb < (1ll << 31);
+}
+template <int MMA, class AccT>
+static bool launch_chunk_tile(const ChunkArgs& c, const EpiChunk<AccT>& epi, void* ws, int64_t ws_bytes, hipStream_t st) {
+  if (!chunk_tile_ok(c)) return false;
   ChunkTileArgs g{};
   g.a = c.a; g.b = c.b; g.lda = c.lda; g.ldb = c.ldb;
   g.M = c.M; g.N = c.N; g.K = c.Kb;
@@ -250,8 +287,11 @@ static bool launch_chunk_tile(const ChunkArgs& c, const Epi& epi, hipStream_t st
   g.hi = c.max_acc_bits < 32 ? (1 << (c.max_acc_bits - 1)) - 1 : 0x7fffffff;
   g.post = c.dl16 || g.t > 0 || c.max_acc_bits < 32;
   g.dl16 = c.dl16; g.tta = c.tta; g.c_in = c.c_in; g.ldc = c.ldc;
+  const ChunkPlan p = plan_chunk(MMA, c.M, c.N, c.Kb, c.chunk_bytes, c.tta && !c.c_in && ws, ws_bytes);
+  g.full = p.full; g.slices = p.slices; g.slice_len = p.slice_len; g.ws = ws;
   const bool fast = c.tta && !c.dl16 && c.max_acc_bits >= 32;
-  const dim3 grid((unsigned)(g.grid_m * g.grid_n)), block(256);
+  const int tiles = g.grid_m * g.grid_n, cut = tiles - p.full;
+  const dim3 grid((unsigned)(p.full + cut * p.slices)), block(256);
   auto go = [&](auto kt_c) {
     constexpr bool KT = decltype(kt_c)::value;
     // the schedules that round one block while the matrix unit multiplies the others: a chunk of one
@@ -264,6 +304,8 @@ static bool launch_chunk_tile(const ChunkArgs& c, const Epi& epi, hipStream_t st
   };
   if (g.K % 64) go(std::true_type{});
   else go(std::false_type{});
+  if (cut > 0)
+    hipLaunchKernelGGL((chunk_reduce_kernel<AccT>), dim3((unsigned)cut, 16), block, 0, st, g, epi);
   return true;
 }
 
@@ -305,18 +347,21 @@ static EpiChunk<AccT> epi_dq(const float* a_scale, int64_t a_scale_n, const floa
                         ldy % 4 == 0 && ((uintptr_t)y & (y_dtype == FMSMO_F32 ? 15 : 7)) == 0};
 }
 
-static int run_chunk_i8(const ChunkArgs& g, const EpiChunk<int>& epi, hipStream_t st) {
-  if (launch_chunk_tile<MMA_I8>(g, epi, st)) return fmsmo_check_launch();
+static int run_chunk_i8(const ChunkArgs& g, const EpiChunk<int>& epi, void* ws, int64_t ws_bytes, hipStream_t st) {
+  if ((uintptr_t)ws & 15) return FMSMO_ERR_ALIGN;
+  if (launch_chunk_tile<MMA_I8>(g, epi, ws, ws_bytes, st)) return fmsmo_check_launch();
   dim3 grid(div_up(g.N, 128), div_up(g.M, 128));
   hipLaunchKernelGGL((chunk_matmul_kernel<FMSMO_OP_I8>), grid, dim3(256), 0, st, g, epi);
   return fmsmo_check_launch();
 }
 
-static int run_chunk_fp(int op_dtype, const ChunkArgs& g, const EpiChunk<float>& epi, hipStream_t st) {
-  const bool done = op_dtype == FMSMO_OP_E4M3 ? launch_chunk_tile<MMA_FP8_K32>(g, epi, st)
-                    : op_dtype == FMSMO_OP_F16 ? launch_chunk_tile<MMA_F16>(g, epi, st)
-                    : op_dtype == FMSMO_OP_BF16 ? launch_chunk_tile<MMA_BF16>(g, epi, st)
-                                                : launch_chunk_tile<MMA_F32>(g, epi, st);
+static int run_chunk_fp(int op_dtype, const ChunkArgs& g, const EpiChunk<float>& epi, void* ws, int64_t ws_bytes,
+                        hipStream_t st) {
+  if ((uintptr_t)ws & 15) return FMSMO_ERR_ALIGN;
+  const bool done = op_dtype == FMSMO_OP_E4M3 ? launch_chunk_tile<MMA_FP8_K32>(g, epi, ws, ws_bytes, st)
+                    : op_dtype == FMSMO_OP_F16 ? launch_chunk_tile<MMA_F16>(g, epi, ws, ws_bytes, st)
+                    : op_dtype == FMSMO_OP_BF16 ? launch_chunk_tile<MMA_BF16>(g, epi, ws, ws_bytes, st)
+                                                : launch_chunk_tile<MMA_F32>(g, epi, ws, ws_bytes, st);
   if (done) return fmsmo_check_launch();
   dim3 grid(div_up(g.N, 128), div_up(g.M, 128));
   if (op_dtype == FMSMO_OP_E4M3)
@@ -341,11 +386,33 @@ static ChunkArgs chunk_args_i8(const int8_t* a, int64_t lda, const int8_t* b, in
   return g;
 }
 
-extern "C" int fmsmo_matmul_chunk_i8(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
+// (the mma code of an operand type and its element size, or -1)
+static int chunk_mma(int op_dtype, int* esz) {
+  *esz = op_dtype == FMSMO_OP_I8 || op_dtype == FMSMO_OP_E4M3 ? 1 : op_dtype == FMSMO_OP_F32 ? 4 : 2;
+  switch (op_dtype) {
+    case FMSMO_OP_I8: return MMA_I8;
+    case FMSMO_OP_E4M3: return MMA_FP8_K32;
+    case FMSMO_OP_F16: return MMA_F16;
+    case FMSMO_OP_BF16: return MMA_BF16;
+    case FMSMO_OP_F32: return MMA_F32;
+    default: return -1;
+  }
+}
+extern "C" int64_t fmsmo_matmul_chunk_workspace_bytes(int op_dtype, int64_t M, int64_t N, int64_t K, int chunk_size,
+                                                      int truncate_then_accumulate) {
+  int esz;
+  const int mma = chunk_mma(op_dtype, &esz);
+  if (mma < 0 || M <= 0 || N <= 0 || K <= 0 || M >= (1 << 30) || N >= (1 << 30) || K * esz >= (1ll << 31) ||
+      chunk_size * esz < 32 || chunk_size > (1 << 28))
+    return 0;
+  return plan_chunk(mma, M, N, K * esz, (int64_t)chunk_size * esz, truncate_then_accumulate != 0, -1).ws_bytes;
+}
+
+extern "C" int fmsmo_matmul_chunk_i8_ws(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
                                      const int32_t* c_in, int32_t* d, int64_t ldd, int64_t M,
                                      int64_t N, int64_t K, int chunk_size, int chunk_trun_bits,
                                      int max_acc_bits, int truncate_then_accumulate,
-                                     fmsmo_stream_t stream) {
+                                     void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream) {
   int rc = check_chunk(a, lda, b, ldb, d, ldd, M, N, K, 1, chunk_size, 32);
   if (rc) return rc;
   if (chunk_trun_bits < 0 || chunk_trun_bits > 31 || max_acc_bits < 2 || max_acc_bits > 32)
@@ -357,16 +424,24 @@ extern "C" int fmsmo_matmul_chunk_i8(const int8_t* a, int64_t lda, const int8_t*
     return fmsmo_gemm_i8_i32(a, lda, b, ldb, d, ldd, M, N, K, stream);
   const ChunkArgs g = chunk_args_i8(a, lda, b, ldb, M, N, K, chunk_size, chunk_trun_bits, max_acc_bits,
                                     truncate_then_accumulate, c_in, ldd);
-  return run_chunk_i8(g, epi_raw<int>(d, ldd), (hipStream_t)stream);
+  return run_chunk_i8(g, epi_raw<int>(d, ldd), workspace, workspace_bytes, (hipStream_t)stream);
+}
+extern "C" int fmsmo_matmul_chunk_i8(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
+                                     const int32_t* c_in, int32_t* d, int64_t ldd, int64_t M,
+                                     int64_t N, int64_t K, int chunk_size, int chunk_trun_bits,
+                                     int max_acc_bits, int truncate_then_accumulate, fmsmo_stream_t stream) {
+  return fmsmo_matmul_chunk_i8_ws(a, lda, b, ldb, c_in, d, ldd, M, N, K, chunk_size, chunk_trun_bits, max_acc_bits,
+                                  truncate_then_accumulate, nullptr, 0, stream);
 }
 
-extern "C" int fmsmo_matmul_chunk_i8_dq(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
+extern "C" int fmsmo_matmul_chunk_i8_dq_ws(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
                                         const float* a_scale, int64_t a_scale_n,
                                         const float* w_scale, int64_t w_scale_n, const void* bias,
                                         int bias_dtype, int epilogue, void* y, int y_dtype,
                                         int64_t ldy, int64_t M, int64_t N, int64_t K,
                                         int chunk_size, int chunk_trun_bits, int max_acc_bits,
-                                        int truncate_then_accumulate, fmsmo_stream_t stream) {
+                                        int truncate_then_accumulate,
+                                     void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream) {
   int rc = check_chunk(a, lda, b, ldb, y, ldy, M, N, K, 1, chunk_size, 32);
   if (rc) return rc;
   rc = check_chunk_dq(a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype, epilogue, y_dtype, M, N);
@@ -381,7 +456,18 @@ extern "C" int fmsmo_matmul_chunk_i8_dq(const int8_t* a, int64_t lda, const int8
   const ChunkArgs g = chunk_args_i8(a, lda, b, ldb, M, N, K, chunk_size, chunk_trun_bits, max_acc_bits,
                                     truncate_then_accumulate, nullptr, 0);
   const EpiChunk<int> epi = epi_dq<int>(a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype, epilogue, y, y_dtype, ldy);
-  return run_chunk_i8(g, epi, (hipStream_t)stream);
+  return run_chunk_i8(g, epi, workspace, workspace_bytes, (hipStream_t)stream);
+}
+extern "C" int fmsmo_matmul_chunk_i8_dq(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
+                                        const float* a_scale, int64_t a_scale_n,
+                                        const float* w_scale, int64_t w_scale_n, const void* bias,
+                                        int bias_dtype, int epilogue, void* y, int y_dtype,
+                                        int64_t ldy, int64_t M, int64_t N, int64_t K,
+                                        int chunk_size, int chunk_trun_bits, int max_acc_bits,
+                                        int truncate_then_accumulate, fmsmo_stream_t stream) {
+  return fmsmo_matmul_chunk_i8_dq_ws(a, lda, b, ldb, a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype,
+                                     epilogue, y, y_dtype, ldy, M, N, K, chunk_size, chunk_trun_bits, max_acc_bits,
+                                     truncate_then_accumulate, nullptr, 0, stream);
 }
 
 static int chunk_args_fp(const void* a, int64_t lda, const void* b, int64_t ldb, int op_dtype,
@@ -404,26 +490,36 @@ static int chunk_args_fp(const void* a, int64_t lda, const void* b, int64_t ldb,
   return FMSMO_OK;
 }
 
-extern "C" int fmsmo_matmul_chunk_fp(const void* a, int64_t lda, const void* b, int64_t ldb,
+extern "C" int fmsmo_matmul_chunk_fp_ws(const void* a, int64_t lda, const void* b, int64_t ldb,
                                      int op_dtype, const float* c_in, float* d, int64_t ldd,
                                      int64_t M, int64_t N, int64_t K, int chunk_size,
                                      int chunk_trun_bits, int clamp_dl16,
-                                     int truncate_then_accumulate, fmsmo_stream_t stream) {
+                                     int truncate_then_accumulate,
+                                     void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream) {
   ChunkArgs g{};
   int rc = chunk_args_fp(a, lda, b, ldb, op_dtype, d, ldd, M, N, K, chunk_size, chunk_trun_bits,
                          clamp_dl16, truncate_then_accumulate, c_in, ldd, &g);
   if (rc) return rc;
   if (M == 0) return FMSMO_OK;
-  return run_chunk_fp(op_dtype, g, epi_raw<float>(d, ldd), (hipStream_t)stream);
+  return run_chunk_fp(op_dtype, g, epi_raw<float>(d, ldd), workspace, workspace_bytes, (hipStream_t)stream);
+}
+extern "C" int fmsmo_matmul_chunk_fp(const void* a, int64_t lda, const void* b, int64_t ldb,
+                                     int op_dtype, const float* c_in, float* d, int64_t ldd,
+                                     int64_t M, int64_t N, int64_t K, int chunk_size,
+                                     int chunk_trun_bits, int clamp_dl16,
+                                     int truncate_then_accumulate, fmsmo_stream_t stream) {
+  return fmsmo_matmul_chunk_fp_ws(a, lda, b, ldb, op_dtype, c_in, d, ldd, M, N, K, chunk_size, chunk_trun_bits,
+                                  clamp_dl16, truncate_then_accumulate, nullptr, 0, stream);
 }
 
-extern "C" int fmsmo_matmul_chunk_fp_dq(const void* a, int64_t lda, const void* b, int64_t ldb,
+extern "C" int fmsmo_matmul_chunk_fp_dq_ws(const void* a, int64_t lda, const void* b, int64_t ldb,
                                         int op_dtype, const float* a_scale, int64_t a_scale_n,
                                         const float* w_scale, int64_t w_scale_n, const void* bias,
                                         int bias_dtype, int epilogue, void* y, int y_dtype,
                                         int64_t ldy, int64_t M, int64_t N, int64_t K,
                                         int chunk_size, int chunk_trun_bits, int clamp_dl16,
-                                        int truncate_then_accumulate, fmsmo_stream_t stream) {
+                                        int truncate_then_accumulate,
+                                     void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream) {
   ChunkArgs g{};
   int rc = chunk_args_fp(a, lda, b, ldb, op_dtype, y, ldy, M, N, K, chunk_size, chunk_trun_bits,
                          clamp_dl16, truncate_then_accumulate, nullptr, 0, &g);
@@ -432,5 +528,16 @@ extern "C" int fmsmo_matmul_chunk_fp_dq(const void* a, int64_t lda, const void* 
   if (rc) return rc;
   if (M == 0) return FMSMO_OK;
   const EpiChunk<float> epi = epi_dq<float>(a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype, epilogue, y, y_dtype, ldy);
-  return run_chunk_fp(op_dtype, g, epi, (hipStream_t)stream);
+  return run_chunk_fp(op_dtype, g, epi, workspace, workspace_bytes, (hipStream_t)stream);
+}
+extern "C" int fmsmo_matmul_chunk_fp_dq(const void* a, int64_t lda, const void* b, int64_t ldb,
+                                        int op_dtype, const float* a_scale, int64_t a_scale_n,
+                                        const float* w_scale, int64_t w_scale_n, const void* bias,
+                                        int bias_dtype, int epilogue, void* y, int y_dtype,
+                                        int64_t ldy, int64_t M, int64_t N, int64_t K,
+                                        int chunk_size, int chunk_trun_bits, int clamp_dl16,
+                                        int truncate_then_accumulate, fmsmo_stream_t stream) {
+  return fmsmo_matmul_chunk_fp_dq_ws(a, lda, b, ldb, op_dtype, a_scale, a_scale_n, w_scale, w_scale_n, bias,
+                                     bias_dtype, epilogue, y, y_dtype, ldy, M, N, K, chunk_size, chunk_trun_bits,
+                                     clamp_dl16, truncate_then_accumulate, nullptr, 0, stream);
 }

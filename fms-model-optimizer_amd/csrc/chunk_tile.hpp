@@ -229,7 +229,14 @@ struct ChunkTileArgs {
   int post, dl16, tta;
   const void* c_in;    // optional initial accumulator [M, N], same element type as the accumulator
   int64_t ldc;
+  // Tiles [0, full) of the tile sequence are whole; of the others every block takes one of `slices` pieces of
+  // the reduction of slice_len bytes (whole chunks; the last one shorter) and leaves its accumulators in `ws`
+  // for chunk_reduce_kernel.  Rounded chunks are added, so slices of whole chunks may be added in any grouping
+  // (int32 exactly; not with a running accumulator that is itself rounded, nor with c_in).
+  int full, slices, slice_len;
+  void* ws;
 };
+constexpr int CHUNK_GROUP_M = 8;  // tile order: column-major in groups of as many tile rows
 
 // KT: K is no multiple of a stage.
 template <int OP, bool FAST, int SCHED, bool KT>
@@ -258,8 +265,21 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
   const int wm = wave >> 1, wn = wave & 1;
 
   int tile_m, tile_n;
-  tile_of_block(blockIdx.x, gridDim.x, g.grid_m, g.grid_n, 8, tile_m, tile_n);
-  const int k_len = g.K;
+  int k_len = g.K, unit = -1;
+  int64_t k_lo = 0;
+  if ((int)blockIdx.x < g.full) {
+    tile_of_block(blockIdx.x, g.full, g.grid_m, g.grid_n, CHUNK_GROUP_M, tile_m, tile_n);
+  } else {
+    // slice by slice, and an XCD's blocks are neighbours in that order: they share rows of A and B
+    const int cut = g.grid_m * g.grid_n - g.full;
+    const int idx = blockIdx.x - g.full, nblk = cut * g.slices, per = nblk >> 3, rem = nblk & 7;
+    const int xcd = idx & 7;
+    unit = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (idx >> 3);
+    const int slice = unit / cut;
+    tile_of_pid(g.full + unit - slice * cut, g.grid_m, g.grid_n, CHUNK_GROUP_M, tile_m, tile_n);
+    k_lo = (int64_t)slice * g.slice_len;
+    k_len = min(g.slice_len, g.K - (int)k_lo);
+  }
   const int row_lo = tile_m * BM, col_lo = tile_n * BN;
 
   // ---- global -> LDS loader addressing (per thread, constant over the K loop)
@@ -276,8 +296,8 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
     const int r = min(col_lo + ld_row + j * RPI, g.N - 1);
     b_off[j] = (uint32_t)r * (uint32_t)g.ldb + ld_chunk * 16;
   }
-  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)g.a, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)g.b, 0, -1, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)(g.a + k_lo), 0, -1, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)(g.b + k_lo), 0, -1, 0x00020000);
   auto issue_part = [&](int stage, int k0, auto j0_c, auto j1_c) {
     constexpr int J0 = decltype(j0_c)::value, J1 = decltype(j1_c)::value;
     uint8_t* la = lds + stage * STAGE_BYTES + wave * 1024;
@@ -655,6 +675,22 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
 
   // ---- epilogue: acc[i][j][v] is C(row, col) with
   //      row = 32 i + 8 (v / 4) + 4 (lane / 32) + v % 4,   col = 32 j + lane % 32
+  if (unit >= 0) {
+    // a slice: the accumulators as the lanes hold them, 16 bytes each, rows past the end left out
+    int* dst = (int*)g.ws + (int64_t)unit * (BM * BN) + tid * 4;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (row_lo + wm * TM + i * 32 + q * 8 < g.M) {
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            Elem e[4] = {acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
+            *(v4i*)(dst + ((i * FN + j) * 4 + q) * 1024) = *(const v4i*)e;
+          }
+        }
+    return;
+  }
   // The wave's 64 x 64 results pass through its quarter of the LDS ring and are finished in a rolled
   // loop, four neighbours of a row per lane.
   __syncthreads();
@@ -668,6 +704,46 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
   __syncthreads();
   chunk_finish(epi, mine, TM, row_lo + wm * TM, col_lo + wn * TN, g.M, g.N, lane);
 #endif  // __HIP_DEVICE_COMPILE__
+}
+
+// Adds the slices' accumulators up, slice by slice, and finishes them: block (tile, piece) takes four rows per
+// half wave of one 32-column block (the layout of the accumulators).
+template <class AccT>
+__global__ __launch_bounds__(256) void chunk_reduce_kernel(ChunkTileArgs g, EpiChunk<AccT> epi) {
+  const int cut = gridDim.x, piece = blockIdx.y;
+  const int i = piece >> 3, j = (piece >> 2) & 1, q = piece & 3;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int tile_m, tile_n;
+  tile_of_pid(g.full + blockIdx.x, g.grid_m, g.grid_n, CHUNK_GROUP_M, tile_m, tile_n);
+  const int m = tile_m * 128 + (wave >> 1) * 64 + i * 32 + q * 8 + (lane >> 5) * 4;
+  const int n = tile_n * 128 + (wave & 1) * 64 + j * 32 + (lane & 31);
+  if (m >= g.M || n >= g.N) return;
+  const AccT* p = (const AccT*)g.ws + ((int64_t)blockIdx.x * 16 + piece) * 1024 + threadIdx.x * 4;
+  const int64_t step = (int64_t)cut * 16384;
+  AccT sum[4];
+  *(v4i*)sum = *(const v4i*)p;
+  for (int s = 1; s < g.slices; s += 4) {
+    AccT v[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) *(v4i*)v[u] = *(const v4i*)(p + min(s + u, g.slices - 1) * step);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (s + u < g.slices) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (std::is_same<AccT, int>::value) sum[e] = (int)((unsigned)sum[e] + (unsigned)v[u][e]);
+          else sum[e] += v[u][e];
+        }
+      }
+  }
+  const typename EpiChunk<AccT>::Col c = epi.col(n);
+  epi.dispatch([&](auto mode_c, auto out_c) __attribute__((always_inline)) {
+    constexpr int MODE = decltype(mode_c)::value, OUT = decltype(out_c)::value;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (m + e < g.M)
+        epi.template put<MODE, OUT>((int64_t)(m + e) * epi.ldy + n, epi.template bits<MODE, OUT>(sum[e], epi.row(m + e), c));
+  });
 }
 
 }  // namespace fmsmo

@@ -52,11 +52,21 @@ SIGNATURES = {
     "fmsmo_decode_linear_i8": [_P, _I, _L, _P, _I, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_decode_linear_fp8": [_P, _I, _L, _P, _L, _P, _L, _P, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_matmul_chunk_i8": [_P, _L, _P, _L, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I, _P],
+    "fmsmo_matmul_chunk_i8_ws": [_P, _L, _P, _L, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I,
+                                 _P, _L, _P],
     "fmsmo_matmul_chunk_fp": [_P, _L, _P, _L, _I, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I, _P],
+    "fmsmo_matmul_chunk_fp_ws": [_P, _L, _P, _L, _I, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I,
+                                 _P, _L, _P],
     "fmsmo_matmul_chunk_i8_dq": [_P, _L, _P, _L, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _L, _L, _L,
                                  _I, _I, _I, _I, _P],
+    "fmsmo_matmul_chunk_i8_dq_ws": [_P, _L, _P, _L, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _L, _L, _L,
+                                 _I, _I, _I, _I,
+                                    _P, _L, _P],
     "fmsmo_matmul_chunk_fp_dq": [_P, _L, _P, _L, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _L, _L, _L,
                                  _I, _I, _I, _I, _P],
+    "fmsmo_matmul_chunk_fp_dq_ws": [_P, _L, _P, _L, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _L, _L, _L,
+                                 _I, _I, _I, _I,
+                                    _P, _L, _P],
     "fmsmo_grouped_gemm_i8_dq": [_P, _L, _P, _L, _L, _P, _I, _L, _P, _P, _P, _I, _I, _P, _I, _L,
                                  _L, _L, _P],
     "fmsmo_quant_weight_i8": [_P, _I, _L, _P, _I, _P, _I, _L, _I, _P, _L, _P, _L, _L, _P],
@@ -83,6 +93,7 @@ OTHER = {
     "fmsmo_bmm_qa_ok": ([c_int, c_int, c_float, c_float, c_int64, c_int64, c_int64, c_int64], c_int),
     "fmsmo_gemm_workspace_bytes": ([c_int64, c_int64, c_int64], c_int64),
     "fmsmo_gemm_fp8_workspace_bytes": ([c_int64, c_int64, c_int64], c_int64),
+    "fmsmo_matmul_chunk_workspace_bytes": ([c_int, c_int64, c_int64, c_int64, c_int, c_int], c_int64),
     "fmsmo_decode_linear_ok": ([c_int64, c_int64], c_int),
     "fmsmo_decode_linear_f32s_ok": ([c_int64, c_int64], c_int),
     "fmsmo_gemm_tail_columns": ([c_int64, c_int64, c_int64], c_int64),

@@ -565,6 +565,40 @@ int fmsmo_matmul_chunk_fp_dq(const void* a, int64_t lda, const void* b, int64_t 
                              int chunk_size, int chunk_trun_bits, int clamp_dl16,
                              int truncate_then_accumulate, fmsmo_stream_t stream);
 
+/*
+ * The chunked matmuls with a caller's workspace (16-byte aligned device memory, written and read within the
+ * call's work on the stream): tiles past the last whole round of the compute units are cut along K and their
+ * partial accumulators added in it.  int8 results are the same bits, floating-point ones sums of the same
+ * rounded chunks in another grouping.  fmsmo_matmul_chunk_workspace_bytes (host only): what the calls of a shape
+ * use, 0 where they use none; a smaller workspace cuts into fewer slices, NULL into none.  chunk_size in elements.
+ */
+int64_t fmsmo_matmul_chunk_workspace_bytes(int op_dtype, int64_t M, int64_t N, int64_t K, int chunk_size,
+                                           int truncate_then_accumulate);
+int fmsmo_matmul_chunk_i8_ws(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
+                          const int32_t* c_in, int32_t* d, int64_t ldd, int64_t M, int64_t N,
+                          int64_t K, int chunk_size, int chunk_trun_bits, int max_acc_bits,
+                          int truncate_then_accumulate,
+    void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream);
+int fmsmo_matmul_chunk_fp_ws(const void* a, int64_t lda, const void* b, int64_t ldb, int op_dtype,
+                          const float* c_in, float* d, int64_t ldd, int64_t M, int64_t N,
+                          int64_t K, int chunk_size, int chunk_trun_bits, int clamp_dl16,
+                          int truncate_then_accumulate,
+    void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream);
+int fmsmo_matmul_chunk_i8_dq_ws(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
+                             const float* a_scale, int64_t a_scale_n, const float* w_scale,
+                             int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
+                             void* y, int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K,
+                             int chunk_size, int chunk_trun_bits, int max_acc_bits,
+                             int truncate_then_accumulate,
+    void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream);
+int fmsmo_matmul_chunk_fp_dq_ws(const void* a, int64_t lda, const void* b, int64_t ldb, int op_dtype,
+                             const float* a_scale, int64_t a_scale_n, const float* w_scale,
+                             int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
+                             void* y, int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K,
+                             int chunk_size, int chunk_trun_bits, int clamp_dl16,
+                             int truncate_then_accumulate,
+    void* workspace, int64_t workspace_bytes, fmsmo_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------
  * 5. Grouped int8 GEMM for mixture-of-experts FFNs (uneven rows per expert, one launch).
  *    Rows of A are sorted by expert; expert e owns rows [offsets[e], offsets[e+1]).

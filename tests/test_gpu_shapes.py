@@ -435,3 +435,40 @@ def test_chunked_products_at_the_edges_of_tiles_and_of_the_reduction(dev, M, N, 
         one = torch.ones(1, device=dev)
         y = K().matmul_chunk_dq(a.to(dev), w.to(dev), one, one, None, 1, torch.float32, chunk_size=cs, chunk_trun_bits=t)
         assert torch.equal(y.cpu(), ref.float()), (cs, t)
+
+
+@pytest.mark.parametrize("M,N,Kd,cs", [(16, 130, 8192, 64), (129, 100, 4112, 128), (40, 600, 4096 + 48, 32),
+                                       (1100, 4096, 6144, 64),     # 288 tiles: whole ones and cut ones in one launch
+                                       (70, 260, 6000, 4096)])     # few, long chunks
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn, torch.float16])
+def test_chunked_products_whose_reduction_is_cut(dev, M, N, Kd, cs, dtype):
+    """The sums of the slices against the uncut launch (no workspace) and, where it is quick, the oracle: integer-valued
+    operands, whose rounded chunks add up exactly in fp32 in any grouping (as in the test above)."""
+    from fms_mo_amd import _lib as L
+
+    lib = L.load()
+    a = torch.randint(-6, 7, (M, Kd), generator=gen(M + Kd)).float().to(dtype).to(dev)
+    w = torch.randint(-6, 7, (N, Kd), generator=gen(N + Kd + 1)).float().to(dtype).to(dev)
+    op, esz, t = K()._OPDT[dtype], a.element_size(), 5
+    nbytes = lib.fmsmo_matmul_chunk_workspace_bytes(op, M, N, Kd, cs, 1)
+    if cs < 4096:
+        assert nbytes > 0
+    acc = torch.int32 if dtype == torch.int8 else torch.float32
+
+    def run(limit):
+        d = torch.full((M, N), -7, dtype=acc, device=dev)
+        ws = torch.full((max(limit, 16),), 0x5a, dtype=torch.uint8, device=dev)
+        tail = (32, 1) if dtype == torch.int8 else (0, 1)
+        head = (a.data_ptr(), Kd, w.data_ptr(), Kd) + (() if dtype == torch.int8 else (op,))
+        L.call("fmsmo_matmul_chunk_i8_ws" if dtype == torch.int8 else "fmsmo_matmul_chunk_fp_ws", *head, None, d.data_ptr(), N,
+               M, N, Kd, cs, t, *tail, ws.data_ptr() if limit else None, limit, torch.cuda.current_stream().cuda_stream)
+        return d
+
+    whole = run(0)
+    for limit in {nbytes, nbytes // 2, nbytes - 16}:
+        if limit > 0:
+            assert torch.equal(run(limit), whole), limit
+    if N < 1000:
+        ref = (O.chunk_matmul_i8(a.cpu(), w.cpu(), None, cs, t, 32) if dtype == torch.int8
+               else O.chunk_matmul_fp(a.cpu().float(), w.cpu().float(), None, cs, t))
+        assert torch.equal(whole.cpu(), ref)

@@ -66,3 +66,15 @@ def test_fp8_per_tensor_quantizer_of_a_huge_tensor(monkeypatch):
         assert [n for n, _ in names] == want
         assert want[-1] != "fmsmo_quant_act_fp8_dynamic" or (names[-1][1][4] == 1 and names[-1][1][5] is not None)
         names.clear()
+
+
+def test_chunked_products_ask_for_a_workspace_only_where_they_may_be_cut():
+    lib = L.load()
+    need = lib.fmsmo_matmul_chunk_workspace_bytes
+    assert need(L.OP_I8, 16, 4096, 14336, 64, 1) == 256 * 65536      # 32 tiles, eight slices each
+    assert need(L.OP_I8, 1069, 4096, 14336, 64, 1) == 256 * 65536    # 256 whole tiles and 32 cut ones
+    assert need(L.OP_I8, 16, 4096, 14336, 64, 0) == 0                # the running accumulator itself is rounded
+    assert need(L.OP_I8, 1024, 4096, 14336, 64, 1) == 0              # one whole round
+    assert need(L.OP_I8, 16, 4096, 14336, 16384, 1) == 0             # one chunk
+    assert need(L.OP_F16, 16, 4096, 4096, 8, 1) == 0 and need(9, 16, 4096, 4096, 64, 1) == 0
+    assert need(L.OP_I8, 0, 4096, 4096, 64, 1) == 0 and need(L.OP_I8, 1 << 30, 4096, 4096, 64, 1) == 0
