@@ -275,6 +275,54 @@ __global__ __launch_bounds__(256) void absmax_cols_kernel(const void* __restrict
   }
 }
 
+// The vectors of a deployed linear in one launch: the SmoothQuant scale of every input channel, the weight
+// scale, zero point, correction term and bias of every output channel, and the scalars.  As torch operators
+// these were some twenty launches of 1 ... 5 us, 5 us of the host each, which is what a conversion took.
+// Block b < kb takes 256 input channels and tells in zero_seen[b] whether one of their statistics is 0 (the
+// caller then leaves SmoothQuant out), the others 256 output channels each.
+template <int WT>
+__global__ __launch_bounds__(256) void deploy_vectors_kernel(
+    const float* __restrict__ act, const float* __restrict__ w_absmax, const float* __restrict__ alpha,
+    float* __restrict__ smooth, int32_t* __restrict__ zero_seen, int K, int kb, const float* __restrict__ clip,
+    float levels, const void* __restrict__ bias, int bias_dtype, float* __restrict__ w_scale,
+    int32_t* __restrict__ w_zp, float* __restrict__ corr, void* __restrict__ new_bias, int N,
+    float* __restrict__ input_scale, int32_t* __restrict__ input_zp, int zp, float* __restrict__ clips, float clip_val) {
+  const int b = blockIdx.x;
+  if (b < kb) {
+    const int k = b * 256 + threadIdx.x;
+    const bool live = k < K;
+    const float a = act[min(k, K - 1)];
+    if (live) {
+      // clamp(a^alpha / clamp(max|W|, 1e-5)^(1 - alpha), 1e-5), the inner clamp in the weights' dtype; a NaN stays
+      const float al = alpha[0], wm = w_absmax[k];
+      const float wc = round_to<WT>(wm < 1e-5f ? 1e-5f : wm);
+      const float v = powf(a, al) / powf(wc, 1.0f - al);
+      smooth[k] = v < 1e-5f ? 1e-5f : v;
+    }
+    const int any = __syncthreads_or(live && a == 0.0f);
+    if (threadIdx.x == 0) zero_seen[b] = any;
+    return;
+  }
+  const int n = (b - kb) * 256 + threadIdx.x;
+  if (n < N) {
+    const float ws = clip[n] * 2.0f / levels;
+    const float c = 0.0f * ws;  // (NaN for a scale that is no finite number, as 0 * w_scale * input_scale is)
+    w_scale[n] = ws;
+    w_zp[n] = 0;
+    corr[n] = c;
+    const float nb = bias ? load_dyn(bias, bias_dtype, n) - c : -c;
+    store_from_f32<WT>(new_bias, n, nb);
+  }
+  if (b == kb && threadIdx.x == 0) {
+    input_scale[0] = 1.0f;
+    input_zp[0] = zp;
+    if (clips) {
+      clips[0] = clip_val;
+      clips[1] = -clip_val;
+    }
+  }
+}
+
 // Bias with the zero-point correction of asymmetric activations folded in:
 //   out_n = bias_n + (offset + a_meta[1]) * (sum_k w_nk) * a_meta[0] * w_scale_n
 // a_meta = { 1 / activation scale, activation zero point } as left on the device by the
@@ -351,6 +399,31 @@ extern "C" int fmsmo_quant_weight_i8(const void* w, int w_dtype, int64_t ldw, co
   hipLaunchKernelGGL((quant_weight_i8_kernel<WT>), grid, block, 0, st, w, ldw, smooth,          \
                      smooth_dtype, coef, coef_dtype, coef_n == 1 ? 0 : 1, t1, t2, mode, q, ldq, \
                      row_sum, (int)K)
+  switch (w_dtype) {
+    case FMSMO_F16: LAUNCH(FMSMO_F16); break;
+    case FMSMO_BF16: LAUNCH(FMSMO_BF16); break;
+    default: LAUNCH(FMSMO_F32); break;
+  }
+#undef LAUNCH
+  return fmsmo_check_launch();
+}
+
+extern "C" int fmsmo_deploy_vectors(const float* act, const float* w_absmax, const float* alpha, float* smooth,
+                                    int32_t* zero_seen, int64_t K, const float* clip, float levels, const void* bias,
+                                    int bias_dtype, float* w_scale, int32_t* w_zp, float* corr, void* new_bias,
+                                    int w_dtype, int64_t N, float* input_scale, int32_t* input_zp, int zp, float* clips,
+                                    float clip_val, fmsmo_stream_t stream) {
+  if (!clip || !w_scale || !w_zp || !corr || !new_bias || !input_scale || !input_zp) return FMSMO_ERR_NULL;
+  if (act && (!w_absmax || !alpha || !smooth || !zero_seen)) return FMSMO_ERR_NULL;
+  if (N <= 0 || N > 0x7fffff00 || (act && (K <= 0 || K > 0x3fffffff))) return FMSMO_ERR_SHAPE;
+  if (w_dtype < 0 || w_dtype > 2 || (bias && (bias_dtype < 0 || bias_dtype > 2))) return FMSMO_ERR_UNSUPPORTED;
+  const int kb = act ? div_up(K, 256) : 0;
+  const dim3 grid((unsigned)(kb + div_up(N, 256))), block(256);
+  hipStream_t st = (hipStream_t)stream;
+#define LAUNCH(WT)                                                                                                 \
+  hipLaunchKernelGGL((deploy_vectors_kernel<WT>), grid, block, 0, st, act, w_absmax, alpha, smooth, zero_seen, (int)K, \
+                     kb, clip, levels, bias, bias_dtype, w_scale, w_zp, corr, new_bias, (int)N, input_scale, input_zp, \
+                     zp, clips, clip_val)
   switch (w_dtype) {
     case FMSMO_F16: LAUNCH(FMSMO_F16); break;
     case FMSMO_BF16: LAUNCH(FMSMO_BF16); break;

@@ -70,6 +70,7 @@ SIGNATURES = {
     "fmsmo_grouped_gemm_i8_dq": [_P, _L, _P, _L, _L, _P, _I, _L, _P, _P, _P, _I, _I, _P, _I, _L,
                                  _L, _L, _P],
     "fmsmo_quant_weight_i8": [_P, _I, _L, _P, _I, _P, _I, _L, _I, _P, _L, _P, _L, _L, _P],
+    "fmsmo_deploy_vectors": [_P, _P, _P, _P, _P, _L, _P, _F, _P, _I, _P, _P, _P, _P, _I, _L, _P, _P, _I, _P, _F, _P],
     "fmsmo_absmax_cols": [_P, _I, _L, _L, _L, _P, _P],
     "fmsmo_quant_i8_affine": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _L, _L, _L, _P],
     "fmsmo_quant_i8_affine_sums": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _P, _L, _L, _L, _P],

@@ -582,6 +582,32 @@ def absmax_cols(x, running=None):
     return running
 
 
+def deploy_vectors(clip, levels, bias, w_dtype, zp, clip_val=None, act=None, w_absmax=None, alpha=None):
+    """The vectors and scalars of a deployed linear in one launch (see fmsmo_deploy_vectors): a dict with
+    smooth [K] and zero_seen (None without act), w_scale, w_zp, corr, bias [N], input_scale, input_zp and the
+    two clip values (None without clip_val)."""
+    _need_gpu(clip, bias, act, w_absmax, alpha)
+    dev, N = clip.device, clip.numel()
+    f32 = dict(dtype=torch.float32, device=dev)
+    i32 = dict(dtype=torch.int32, device=dev)
+    o = {"w_scale": torch.empty((N,), **f32), "w_zp": torch.empty((N,), **i32), "corr": torch.empty((N,), **f32),
+         "bias": torch.empty((N,), dtype=w_dtype, device=dev), "input_scale": torch.empty((), **f32),
+         "input_zp": torch.empty((), **i32), "clips": None if clip_val is None else torch.empty((2,), **f32),
+         "smooth": None, "zero_seen": None}
+    K = 0
+    if act is not None:
+        K = act.numel()
+        o["smooth"] = torch.empty((1, K), **f32)
+        o["zero_seen"] = torch.empty(((K + 255) // 256,), **i32)
+    with _dev(clip):
+        L.call("fmsmo_deploy_vectors", _ptr(act), _ptr(w_absmax), _ptr(alpha), _ptr(o["smooth"]), _ptr(o["zero_seen"]), K,
+               clip.data_ptr(), float(levels), _ptr(bias), _dt(bias) if bias is not None else 0,
+               o["w_scale"].data_ptr(), o["w_zp"].data_ptr(), o["corr"].data_ptr(), o["bias"].data_ptr(), _DT[w_dtype], N,
+               o["input_scale"].data_ptr(), o["input_zp"].data_ptr(), int(zp), _ptr(o["clips"]),
+               0.0 if clip_val is None else float(clip_val), _stream(clip))
+    return o
+
+
 def zero_shift_bias(w, w_scale, a_meta, bias=None, offset=128.0):
     """fp32 [N] bias with the zero-point correction of asymmetric activations folded in
     (see fmsmo_zero_shift_bias).  w int8 [N,K]; w_scale fp32 [N] or [1]; a_meta fp32 [2]."""

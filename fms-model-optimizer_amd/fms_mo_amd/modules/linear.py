@@ -89,6 +89,65 @@ def _weight_column_max(w):
     return w.abs().max(dim=0, keepdim=True)[0]
 
 
+def _plain_f32(t, n):
+    return (type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == torch.float32 and t.numel() == n
+            and t.is_contiguous())
+
+
+def _dynamic_operands(q):
+    """What _convert_dynamic takes: None, or (activation statistics, alpha, column maximum of the weights) where
+    SmoothQuant is on and (None, None, None) where it is not.  The maximum is one pass over the weights,
+    launched here, ahead of everything the host does for the conversion."""
+    w, bias = q.weight, q.bias
+    if not (w.is_cuda and w.dtype in (torch.float16, torch.bfloat16) and w.is_contiguous() and w.shape[1] % 8 == 0
+            and w.numel() and w.data_ptr() % 16 == 0
+            and (bias is None or (bias.is_contiguous() and bias.dtype in (torch.float16, torch.bfloat16, torch.float32)
+                                  and bias.device == w.device))):
+        return None
+    if not getattr(q, "smoothq", False):
+        return None, None, None
+    act, alpha = q.smoothq_act_scale, q.smoothq_alpha
+    if not (torch.is_tensor(act) and torch.is_tensor(alpha) and _plain_f32(act, w.shape[1]) and act.dim() == 1
+            and _plain_f32(alpha, 1) and alpha.dim() == 1 and act.device == w.device == alpha.device):
+        return None
+    return act, alpha, kernels.absmax_cols(w.detach())
+
+
+def _convert_dynamic(m, q, w_levels, operands):
+    """The offline part of QLinearINT8Deploy.from_fms_mo for a dynamic activation scale, on the device, in
+    three launches: column maximum of the weights (`operands`), every vector and scalar, weight quantizer --
+    nothing waits for the host until the module is built.  Fills `m` and returns True; False for what it does
+    not take (an activation statistic of 0 among it), which from_fms_mo does with torch operators."""
+    w, Qa, Qw, bias = q.weight, q.quantize_feature, q.quantize_weight, q.bias
+    N, Kd = w.shape
+    w_cv = Qw.clip_val
+    if not (_plain_f32(w_cv, N) and w_cv.dim() == 1 and w_cv.device == w.device):
+        return False
+    act, alpha, w_absmax = operands
+    own_clips = hasattr(Qa, "clip_val")
+    if own_clips != hasattr(Qa, "clip_valn"):
+        return False
+    v = kernels.deploy_vectors(w_cv.detach(), w_levels, None if bias is None else bias.detach(), w.dtype,
+                               128 - m.useSymAct, None if own_clips else 8.0, act, w_absmax, alpha)
+    sq = v["smooth"]
+    w_int8 = kernels.quant_weight_i8(w.detach(), v["w_scale"], None if sq is None else sq.view(Kd), mode="div")
+    a_cv, a_cvn = (Qa.clip_val, Qa.clip_valn) if own_clips else v["clips"].unbind(0)
+    m.cvs = [a_cv, a_cvn, w_cv]
+    m.use_fake_zero_shift = False
+    m.org_model_has_bias = bias is not None
+    m._parameters["weight"] = nn.Parameter(w_int8, requires_grad=False)
+    del m._parameters["bias"]
+    if sq is None:
+        sq = torch.ones(1, device=w.device, dtype=w.dtype)
+    m._buffers.update(input_scale=v["input_scale"], input_zp=v["input_zp"], w_scale=v["w_scale"], w_zp=v["w_zp"],
+                      smoothq_scale=sq, corr_term=v["corr"], bias=v["bias"])
+    if act is not None and any(v["zero_seen"].tolist()):
+        m._buffers.clear()
+        m.register_parameter("bias", None)
+        return False
+    return True
+
+
 def _compute_dtype(x_dtype, smooth):
     return x_dtype if smooth is None else torch.promote_types(x_dtype, smooth.dtype)
 
@@ -337,6 +396,10 @@ class QLinearINT8Deploy(nn.Linear):
     ``smoothq_scale``, ``corr_term``, ``bias`` -- the names the reference registers
     (linear.py:843-911)."""
 
+    def reset_parameters(self):
+        if not self.weight.is_meta:  # (the conversions start from meta tensors: nothing to initialise)
+            super().reset_parameters()
+
     @classmethod
     def from_fms_mo(cls, fms_mo_qlinear, **kwargs):
         """Convert a QLinear.  Keyword arguments as in the reference: use_int_kernel
@@ -351,6 +414,10 @@ class QLinearINT8Deploy(nn.Linear):
         # and target on one device; converting a CPU module for a GPU target also works here and
         # gives the CPU roundings of pow / division for the offline scales).
         src_dev = fms_mo_qlinear.weight.device
+        operands = None
+        if kwargs.get("use_dynamic_max_act_Qfunc", False) in [-1, -2] and not isinstance(fms_mo_qlinear.quantize_weight, SAWB):
+            with torch.no_grad():
+                operands = _dynamic_operands(fms_mo_qlinear)
         m = cls(fms_mo_qlinear.in_features, fms_mo_qlinear.out_features,
                 bias=fms_mo_qlinear.bias is not None, device="meta")
         qcfg = getattr(fms_mo_qlinear, "qcfg", {})
@@ -374,6 +441,9 @@ class QLinearINT8Deploy(nn.Linear):
                     Qw.observe(fms_mo_qlinear.weight)
                 else:
                     Qw(fms_mo_qlinear.weight)
+            if operands is not None and m.useSymAct and _convert_dynamic(m, fms_mo_qlinear, w_levels, operands):
+                m.set_matmul_op()
+                return m if torch.device(tar_dev) == m.weight.device else m.to(tar_dev)
             w_cv = Qw.clip_val
             # (constants by fill kernels: torch.tensor(..., device=...) copies from the host and waits)
             a_cv = Qa.clip_val if hasattr(Qa, "clip_val") else torch.full((), 8.0, device=src_dev)

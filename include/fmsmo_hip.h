@@ -649,6 +649,21 @@ int fmsmo_absmax_cols(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_
                       fmsmo_stream_t stream);
 
 /*
+ * The vectors of a deployed linear with dynamic activation scales, in one launch:
+ *   smooth[k]   = max(act[k]^alpha / max(w_absmax[k], 1e-5)^(1 - alpha), 1e-5)   (act NULL: no SmoothQuant)
+ *   zero_seen[b]  whether one of act[256 b .. 256 b + 255] is 0, ceil(K / 256) flags
+ *   w_scale[n]  = clip[n] * 2 / levels,  w_zp[n] = 0,  corr[n] = 0 * w_scale[n],  new_bias[n] = bias[n] - corr[n]
+ *   input_scale[0] = 1,  input_zp[0] = zp,  clips = {clip_val, -clip_val} (clips NULL: not wanted)
+ * w_dtype: of the weights (the inner maximum is taken in it) and of new_bias; bias may be NULL.
+ * Reference: the offline arithmetic of QLinearINT8Deploy.from_fms_mo (fms_mo/modules/linear.py:800-911).
+ */
+int fmsmo_deploy_vectors(const float* act, const float* w_absmax, const float* alpha, float* smooth,
+                         int32_t* zero_seen, int64_t K, const float* clip, float levels, const void* bias,
+                         int bias_dtype, float* w_scale, int32_t* w_zp, float* corr, void* new_bias,
+                         int w_dtype, int64_t N, float* input_scale, int32_t* input_zp, int zp, float* clips,
+                         float clip_val, fmsmo_stream_t stream);
+
+/*
  * Bias with the zero-point correction of asymmetric per-tensor activations folded in, for use
  * as the bias of fmsmo_gemm_i8_dq when the activation codes are stored minus `offset`:
  *   out[n] = bias[n] + (offset + a_meta[1]) * (sum_k w[n,k]) * a_meta[0] * w_scale[n]

@@ -472,3 +472,41 @@ def test_chunked_products_whose_reduction_is_cut(dev, M, N, Kd, cs, dtype):
         ref = (O.chunk_matmul_i8(a.cpu(), w.cpu(), None, cs, t, 32) if dtype == torch.int8
                else O.chunk_matmul_fp(a.cpu().float(), w.cpu().float(), None, cs, t))
         assert torch.equal(whole.cpu(), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Kd,N,bias,stats", [(264, 37, True, "some"), (256, 256, False, "some"), (520, 300, True, "zero"),
+                                             (8, 1, False, "none"), (512, 257, True, "extreme")])
+def test_vectors_of_a_converted_linear(dev, dtype, Kd, N, bias, stats):
+    """One launch for the vectors against the torch expressions on the same GPU: ends of 256-channel groups, a
+    statistic of zero (SmoothQuant is left out), no statistics at all, statistics and weights at both ends of the range."""
+    from fms_mo_amd.modules.linear import QLinearINT8Deploy
+
+    m = make_qlinear(Kd, N, dtype, bias=bias).to(dev)
+    if stats != "none":
+        m.smoothq, m.smoothq_alpha = True, torch.full((1,), 0.4, device=dev)
+        m.smoothq_act_scale = 0.5 + torch.rand(Kd, generator=gen(3)).to(dev)
+    if stats == "zero":
+        m.smoothq_act_scale[Kd - 1] = 0
+    if stats == "extreme":
+        with torch.no_grad():
+            m.weight[:, :4] = 0
+            m.weight[:, 4:8] = 6e4
+        m.smoothq_act_scale[2], m.smoothq_act_scale[3] = 1e-30, 1e30
+        m.smoothq_act_scale[6], m.smoothq_act_scale[7] = 1e-30, float("nan")
+    dep = QLinearINT8Deploy.from_fms_mo(m, use_dynamic_max_act_Qfunc=-1, recalc_clipvals=False)
+    cv, w = m.quantize_weight.clip_val, m.weight.detach()
+    ws = cv * 2 / torch.tensor(254.0, device=dev)
+    if stats in ("none", "zero"):
+        sq = torch.ones(1, device=dev, dtype=dtype)
+    else:
+        wm = w.abs().max(dim=0, keepdim=True)[0].clamp(min=1e-5)
+        sq = (m.smoothq_act_scale ** m.smoothq_alpha / wm ** (1.0 - m.smoothq_alpha)).clamp(min=1e-5)
+    codes = torch.nan_to_num(((w * sq).t() / ws).round().clamp(-127, 127).t(), nan=-127.0).to(torch.int8)
+    assert dep.smoothq_scale.dtype == sq.dtype and torch.equal(torch.nan_to_num(dep.smoothq_scale), torch.nan_to_num(sq))
+    assert torch.equal(dep.w_scale, ws) and torch.equal(dep.weight, codes)
+    b = m.bias.detach().float() if bias else torch.zeros(N, device=dev)
+    assert dep.bias.dtype == dtype and torch.equal(dep.bias, b.to(dtype)) and torch.equal(dep.corr_term, torch.zeros_like(ws))
+    assert torch.equal(dep.w_zp, torch.zeros(N, dtype=torch.int32, device=dev)) and int(dep.input_zp) == 127
+    assert list(dep.state_dict()) == ["weight", "input_scale", "input_zp", "w_scale", "w_zp", "smoothq_scale", "corr_term", "bias"]
+    assert float(dep.input_scale) == 1 and [float(v) for v in dep.cvs[:2]] == [8.0, -8.0]
