@@ -13,6 +13,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # FMSMO_LIB names another build of the library (A/B measurements of kernel variants)
 LIB_PATH = os.environ.get("FMSMO_LIB") or os.path.normpath(os.path.join(_HERE, "..", "lib", "libfmsmo_hip.so"))
+HOST_PATH = os.path.normpath(os.path.join(_HERE, "..", "lib", "_fmsmo_host.so"))
 
 # dtype / enum codes of include/fmsmo_hip.h
 F16, BF16, F32 = 0, 1, 2
@@ -71,6 +72,7 @@ SIGNATURES = {
                                  _L, _L, _P],
     "fmsmo_quant_weight_i8": [_P, _I, _L, _P, _I, _P, _I, _L, _I, _P, _L, _P, _L, _L, _P],
     "fmsmo_deploy_vectors": [_P, _P, _P, _P, _P, _L, _P, _F, _P, _I, _P, _P, _P, _P, _I, _L, _P, _P, _I, _P, _F, _P],
+    "fmsmo_clip_values": [_P, _P, _L, _P],
     "fmsmo_absmax_cols": [_P, _I, _L, _L, _L, _P, _P],
     "fmsmo_quant_i8_affine": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _L, _L, _L, _P],
     "fmsmo_quant_i8_affine_sums": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _P, _L, _L, _L, _P],
@@ -131,6 +133,28 @@ def load() -> ctypes.CDLL:
         raise FmsMoHipError("libfmsmo_hip.so ABI version mismatch; rebuild the library")
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The extension module that checks, allocates and launches the hot calls (csrc/host_calls.cpp), bound to the
+    entry points of the library on first use.  Missing like the library: an error, no fallback."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    if not os.path.exists(HOST_PATH):
+        raise FmsMoHipError(f"{HOST_PATH} is missing: build it first (make -C fms-model-optimizer_amd/csrc)")
+    from importlib import machinery, util
+
+    loader = machinery.ExtensionFileLoader("_fmsmo_host", HOST_PATH)
+    mod = util.module_from_spec(util.spec_from_file_location("_fmsmo_host", HOST_PATH, loader=loader))
+    loader.exec_module(mod)
+    mod.bind({n: ctypes.cast(getattr(lib, n), c_void_p).value for n in mod.entries()}, raise_status)
+    _host = mod
+    return mod
 
 
 def raise_status(name: str, rc: int) -> None:

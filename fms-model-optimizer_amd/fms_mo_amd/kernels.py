@@ -217,6 +217,10 @@ def quant_act_fp8_dynamic(x, variant=L.FP8_LINEAR, per_tensor=False, scale_floor
 def quant_act_i8_static_t(x, mode, compute_dtype, scale, zp, sym=0, clip_lo=0.0, clip_hi=0.0):
     """int8 [M,K]: the static per-tensor formulas evaluated in ``compute_dtype`` (see
     fmsmo_quant_act_i8_static_t; mode is one of L.SQ_*).  All parameters are host numbers."""
+    if not _COMPILING():
+        q = (_H or _host()).quant_i8_static_t(x, mode, compute_dtype, scale, zp, sym, clip_lo, clip_hi)
+        if q is not None:
+            return q
     _need_gpu(x)
     x = _rows(x)
     M, K = x.shape
@@ -421,6 +425,11 @@ def grouped_gemm_i8_dq(a, w, offsets, a_scale, w_scale, bias=None, out_dtype=tor
                        exact_ref=True):
     """a int8 [T,K] rows sorted by expert, w int8 [E,N,K], offsets int32 [E+1] (device),
     a_scale fp32 [T], w_scale fp32 [E,N], bias [E,N] or None -> [T,N]."""
+    if not _COMPILING():
+        y = (_H or _host()).grouped_i8(a, w, offsets, a_scale, w_scale, bias, out_dtype,
+                                       L.EPI_REF_F16 if exact_ref else L.EPI_F32)
+        if y is not None:
+            return y
     _need_gpu(a, w, offsets)
     if a.dtype != torch.int8 or w.dtype != torch.int8 or w.dim() != 3:
         raise TypeError("a must be int8 [T,K], w int8 [E,N,K]")
@@ -503,6 +512,11 @@ def matmul_chunk_dq(a, w, a_scale, w_scale, bias=None, epilogue=L.EPI_SEQ_OUT, o
     """y [M,N] = epilogue(chunked accumulator of a [M,K] . w [N,K]^T): the chunk-truncate matmul and
     its dequantization in one launch (see fmsmo_matmul_chunk_i8_dq / _fp_dq).  a_scale fp32 [M] or
     [1], w_scale fp32 [N] or [1], bias [N] (fp16 / bf16 / fp32) or None, epilogue one of L.EPI_*."""
+    if not _COMPILING():
+        y = (_H or _host()).chunk_dq(a, w, a_scale, w_scale, bias, epilogue, out_dtype, chunk_size, chunk_trun_bits, max_acc_bits,
+                                     truncate_then_accumulate, clamp_acc_to_dl16)
+        if y is not None:
+            return y
     _need_gpu(a, w, a_scale, w_scale, bias)
     if a.dtype != w.dtype or a.dtype not in _OPDT:
         raise TypeError(f"unsupported operand dtypes {a.dtype}, {w.dtype}")
@@ -709,6 +723,10 @@ def bmm_i8_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype):
     M, K = m1.shape[-2:]
     if not zero_sums_fit(zero1, K):
         raise ValueError(f"the zero-point correction of K = {K} codes with zero point {zero1} may leave 32 bits")
+    if not _COMPILING():
+        y = (_H or _host()).bmm_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype)
+        if y is not None:
+            return y
     N = m2.shape[-1]
     a3 = _batched3(m1)
     B = a3.shape[0]
@@ -833,227 +851,26 @@ def _as_scale(s, device):
     return torch.tensor([float(s)], dtype=torch.float32, device=device)
 
 
-# Lean forms of the three calls a decode step makes.  An eager call of a 5 us kernel is bound by
-# what the host does per launch; the general wrappers above spend about 60 Python-level calls on
-# argument handling.  These take the common case only -- plain, well-formed tensors on the current
-# GPU, outside a compiler trace -- with the checks written inline, and return None for anything
-# else, which then goes through the general path (and gets its error messages there).
-_T, _P = torch.Tensor, torch.nn.Parameter
+# An eager call of a 5 us kernel is bound by what the host does per launch: the common case -- plain,
+# well-formed tensors on the current GPU, outside a compiler trace -- is checked, allocated and launched by
+# the native module (csrc/host_calls.cpp), which returns None for anything else; that then goes through
+# the general path (and gets its error messages there).
 _COMPILING = torch.compiler.is_compiling
-_F32, _I8 = torch.float32, torch.int8
-_FN = {}
+_H = None
 
 
-def _fn(name):
-    f = _FN.get(name)
-    if f is None:
-        f = _FN[name] = L.entry(name)
-    return f
-
-
-def _mat(t, dtype):
-    """(rows, cols, row stride) of a plain 2-D CUDA tensor of `dtype` with unit inner stride on
-    the current GPU, else None."""
-    tt = type(t)
-    if (tt is not _T and tt is not _P) or t.dtype is not dtype or not t.is_cuda or t.dim() != 2:
-        return None
-    r, c = t.shape
-    s0, s1 = t.stride()
-    if s1 != 1 or (r > 1 and s0 < c):
-        return None
-    return r, c, (s0 if r > 1 else max(c, s0))
-
-
-def _vec32(t, n):
-    return (type(t) is _T and t.dtype is _F32 and t.is_cuda and t.dim() == 1 and t.is_contiguous()
-            and (t.numel() == n or t.numel() == 1) and not t.requires_grad)
-
-
-def _gemm_i8_dq_lean(a, w, a_scale, w_scale, bias, out_dtype, epilogue):
-    if _COMPILING() or _RAW_STREAM is None:
-        return None
-    ma, mw = _mat(a, _I8), _mat(w, _I8)
-    if ma is None or mw is None or ma[1] != mw[1] or not _vec32(a_scale, ma[0]) or not _vec32(w_scale, mw[0]):
-        return None
-    M, K, lda = ma
-    N, _, ldw = mw
-    if bias is not None:
-        tb = type(bias)
-        if ((tb is not _T and tb is not _P) or not bias.is_cuda or bias.dim() != 1 or bias.numel() != N
-                or not bias.is_contiguous() or bias.dtype not in _DT):
-            return None
-        bptr, bdt = bias.data_ptr(), _DT[bias.dtype]
-    else:
-        bptr, bdt = None, 0
-    idx = a.get_device()
-    if _CUR_DEVICE() != idx or out_dtype not in _DT:
-        return None
-    y = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    nbytes = _WS_BYTES.get((M, N, K))
-    if nbytes is None:
-        nbytes = _WS_BYTES[(M, N, K)] = L.load().fmsmo_gemm_workspace_bytes(M, N, K)
-    if nbytes > 0:
-        ws = torch.empty((nbytes,), dtype=torch.uint8, device=a.device)
-        rc = _fn("fmsmo_gemm_i8_dq_ws")(a.data_ptr(), lda, w.data_ptr(), ldw, a_scale.data_ptr(), a_scale.numel(),
-                                        w_scale.data_ptr(), w_scale.numel(), bptr, bdt, epilogue, y.data_ptr(),
-                                        _DT[out_dtype], N, M, N, K, ws.data_ptr(), nbytes, _RAW_STREAM(idx))
-    else:
-        rc = _fn("fmsmo_gemm_i8_dq")(a.data_ptr(), lda, w.data_ptr(), ldw, a_scale.data_ptr(), a_scale.numel(),
-                                     w_scale.data_ptr(), w_scale.numel(), bptr, bdt, epilogue, y.data_ptr(),
-                                     _DT[out_dtype], N, M, N, K, _RAW_STREAM(idx))
-    if rc:
-        L.raise_status("fmsmo_gemm_i8_dq", rc)
-    return y
-
-
-def _smooth_ok(smooth, K):
-    ts = type(smooth)
-    return ((ts is _T or ts is _P) and smooth.is_cuda and smooth.dim() == 1 and smooth.numel() == K
-            and smooth.is_contiguous() and smooth.dtype in _DT and smooth.data_ptr() % 16 == 0)
-
-
-def _quant_act_i8_pertoken_lean(x, smooth, compute_dtype, saturate):
-    if _COMPILING() or _RAW_STREAM is None or x.dtype not in _DT:
-        return None
-    mx = _mat(x, x.dtype)
-    if mx is None:
-        return None
-    M, K, ldx = mx
-    if smooth is not None:
-        if not _smooth_ok(smooth, K):
-            return None
-        sptr, sdt = smooth.data_ptr(), _DT[smooth.dtype]
-        if compute_dtype is None:
-            compute_dtype = x.dtype if smooth.dtype is x.dtype else torch.promote_types(x.dtype, smooth.dtype)
-    else:
-        sptr, sdt = None, 0
-        if compute_dtype is None:
-            compute_dtype = x.dtype
-    idx = x.get_device()
-    if _CUR_DEVICE() != idx or compute_dtype not in _DT:
-        return None
-    q = torch.empty((M, K), dtype=_I8, device=x.device)
-    scale = torch.empty((M,), dtype=_F32, device=x.device)
-    rc = _fn("fmsmo_quant_act_i8_pertoken")(x.data_ptr(), _DT[x.dtype], ldx, sptr, sdt, _DT[compute_dtype],
-                                            1 if saturate else 0, q.data_ptr(), K, scale.data_ptr(), M, K,
-                                            _RAW_STREAM(idx))
-    if rc:
-        L.raise_status("fmsmo_quant_act_i8_pertoken", rc)
-    return q, scale
-
-
-def _decode_linear_i8_lean(x, w, w_scale, bias, smooth, out_dtype, exact_ref, saturate):
-    if _COMPILING() or _RAW_STREAM is None or x.dtype not in _DT:
-        return None
-    mx, mw = _mat(x, x.dtype), _mat(w, _I8)
-    if mx is None or mw is None or mx[1] != mw[1] or not _vec32(w_scale, mw[0]):
-        return None
-    M, K, ldx = mx
-    N, _, ldw = mw
-    if smooth is not None:
-        if not _smooth_ok(smooth, K):
-            return None
-        sptr, sdt = smooth.data_ptr(), _DT[smooth.dtype]
-    else:
-        sptr, sdt = None, 0
-    if bias is not None:
-        tb = type(bias)
-        if ((tb is not _T and tb is not _P) or not bias.is_cuda or bias.dim() != 1 or bias.numel() != N
-                or not bias.is_contiguous() or bias.dtype not in _DT):
-            return None
-        bptr, bdt = bias.data_ptr(), _DT[bias.dtype]
-    else:
-        bptr, bdt = None, 0
-    idx = x.get_device()
-    if _CUR_DEVICE() != idx or out_dtype not in _DT:
-        return None
-    y = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    a_scale = torch.empty((M,), dtype=_F32, device=x.device)
-    rc = _fn("fmsmo_decode_linear_i8")(x.data_ptr(), _DT[x.dtype], ldx, sptr, sdt, 1 if saturate else 0, w.data_ptr(),
-                                       ldw, w_scale.data_ptr(), w_scale.numel(), bptr, bdt,
-                                       L.EPI_REF_F16 if exact_ref else L.EPI_F32, y.data_ptr(), _DT[out_dtype], N,
-                                       a_scale.data_ptr(), M, N, K, _RAW_STREAM(idx))
-    if rc:
-        L.raise_status("fmsmo_decode_linear_i8", rc)
-    return y, a_scale
-
-
-_E4M3 = torch.float8_e4m3fn
-
-
-def _bias_ok(bias, N):
-    tb = type(bias)
-    return ((tb is _T or tb is _P) and bias.is_cuda and bias.dim() == 1 and bias.numel() == N
-            and bias.is_contiguous() and bias.dtype in _DT)
-
-
-def _gemm_fp8_dq_lean(a, w, a_scale, w_scale, bias, out_dtype):
-    if _COMPILING() or _RAW_STREAM is None:
-        return None
-    ma, mw = _mat(a, _E4M3), _mat(w, _E4M3)
-    if ma is None or mw is None or ma[1] != mw[1] or not _vec32(a_scale, ma[0]) or not _vec32(w_scale, mw[0]):
-        return None
-    M, K, lda = ma
-    N, _, ldw = mw
-    if bias is not None:
-        if not _bias_ok(bias, N):
-            return None
-        bptr, bdt = bias.data_ptr(), _DT[bias.dtype]
-    else:
-        bptr, bdt = None, 0
-    idx = a.get_device()
-    if _CUR_DEVICE() != idx or out_dtype not in _DT:
-        return None
-    y = torch.empty((M, N), dtype=out_dtype, device=a.device)
-    nbytes = _WS_BYTES_FP8.get((M, N, K))
-    if nbytes is None:
-        nbytes = _WS_BYTES_FP8[(M, N, K)] = L.load().fmsmo_gemm_fp8_workspace_bytes(M, N, K)
-    if nbytes > 0:
-        ws = torch.empty((nbytes,), dtype=torch.uint8, device=a.device)
-        rc = _fn("fmsmo_gemm_fp8_dq_ws")(a.data_ptr(), lda, w.data_ptr(), ldw, a_scale.data_ptr(), a_scale.numel(),
-                                         w_scale.data_ptr(), w_scale.numel(), bptr, bdt, y.data_ptr(),
-                                         _DT[out_dtype], N, M, N, K, ws.data_ptr(), nbytes, _RAW_STREAM(idx))
-    else:
-        rc = _fn("fmsmo_gemm_fp8_dq")(a.data_ptr(), lda, w.data_ptr(), ldw, a_scale.data_ptr(), a_scale.numel(),
-                                      w_scale.data_ptr(), w_scale.numel(), bptr, bdt, y.data_ptr(),
-                                      _DT[out_dtype], N, M, N, K, _RAW_STREAM(idx))
-    if rc:
-        L.raise_status("fmsmo_gemm_fp8_dq", rc)
-    return y
-
-
-def _decode_linear_fp8_lean(x, w, w_scale, bias, out_dtype):
-    if _COMPILING() or _RAW_STREAM is None or x.dtype not in _DT:
-        return None
-    mx, mw = _mat(x, x.dtype), _mat(w, _E4M3)
-    if mx is None or mw is None or mx[1] != mw[1] or not _vec32(w_scale, mw[0]):
-        return None
-    M, K, ldx = mx
-    N, _, ldw = mw
-    if bias is not None:
-        if not _bias_ok(bias, N):
-            return None
-        bptr, bdt = bias.data_ptr(), _DT[bias.dtype]
-    else:
-        bptr, bdt = None, 0
-    idx = x.get_device()
-    if _CUR_DEVICE() != idx or out_dtype not in _DT:
-        return None
-    y = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    a_scale = torch.empty((M,), dtype=_F32, device=x.device)
-    rc = _fn("fmsmo_decode_linear_fp8")(x.data_ptr(), _DT[x.dtype], ldx, w.data_ptr(), ldw, w_scale.data_ptr(),
-                                        w_scale.numel(), bptr, bdt, y.data_ptr(), _DT[out_dtype], N,
-                                        a_scale.data_ptr(), M, N, K, _RAW_STREAM(idx))
-    if rc:
-        L.raise_status("fmsmo_decode_linear_fp8", rc)
-    return y, a_scale
+def _host():
+    global _H
+    _H = L.host()
+    return _H
 
 
 def quant_act_i8_pertoken(x, smooth=None, compute_dtype=None, saturate=False):  # noqa: F811
     """(q int8 [M,K], scale fp32 [M]) -- see fmsmo_quant_act_i8_pertoken."""
-    r = _quant_act_i8_pertoken_lean(x, smooth, compute_dtype, saturate)
-    if r is not None:
-        return r
+    if not _COMPILING():
+        r = (_H or _host()).quant_i8(x, smooth, compute_dtype, saturate)
+        if r is not None:
+            return r
     _need_gpu(x, smooth)
     if x.dim() != 2:
         raise ValueError("expected a 2-D tensor")
@@ -1063,6 +880,10 @@ def quant_act_i8_pertoken(x, smooth=None, compute_dtype=None, saturate=False):  
 
 
 def quant_act_i8_static(x, scale: float, zp: int, sym: int):  # noqa: F811
+    if not _COMPILING():
+        q = (_H or _host()).quant_i8_static(x, scale, zp, sym)
+        if q is not None:
+            return q
     _need_gpu(x)
     if x.dim() != 2:
         raise ValueError("expected a 2-D tensor")
@@ -1073,6 +894,10 @@ def quant_act_i8_static(x, scale: float, zp: int, sym: int):  # noqa: F811
 
 def quant_act_fp8_pertoken(x, variant=L.FP8_LINEAR, static_scale=None):  # noqa: F811
     """(q e4m3 [M,K], scale fp32 [M] or the [1] static scale)."""
+    if static_scale is None and not _COMPILING():
+        r = (_H or _host()).quant_fp8(x, variant, False, 1e-12, False)
+        if r is not None:
+            return r
     _need_gpu(x)
     if x.dim() != 2:
         raise ValueError("expected a 2-D tensor")
@@ -1086,6 +911,10 @@ def quant_act_fp8_pertoken(x, variant=L.FP8_LINEAR, static_scale=None):  # noqa:
 def quant_act_fp8_dynamic(x, variant=L.FP8_LINEAR, per_tensor=False, scale_floor=1e-12,  # noqa: F811
                           scale_in_x_dtype=False):
     """(q e4m3 [M,K], scale fp32 [M] or [1]), see fmsmo_quant_act_fp8_dynamic."""
+    if not _COMPILING() and (per_tensor or scale_floor != 1e-12 or scale_in_x_dtype):
+        r = (_H or _host()).quant_fp8(x, variant, per_tensor, scale_floor, scale_in_x_dtype)
+        if r is not None:
+            return r
     _need_gpu(x)
     if x.dim() != 2:
         raise ValueError("expected a 2-D tensor")
@@ -1102,8 +931,8 @@ def gemm_i8_dq(a, w, a_scale, w_scale, bias=None, out_dtype=torch.float16, exact
     L.EPI_*) overrides ``exact_ref`` (True = L.EPI_REF_F16, False = L.EPI_F32)."""
     if epilogue is None:
         epilogue = L.EPI_REF_F16 if exact_ref else L.EPI_F32
-    if not force_gemv:
-        y = _gemm_i8_dq_lean(a, w, a_scale, w_scale, bias, out_dtype, int(epilogue))
+    if not force_gemv and not _COMPILING():
+        y = (_H or _host()).gemm_dq(a, w, a_scale, w_scale, bias, out_dtype, int(epilogue))
         if y is not None:
             return y
     _need_gpu(a, w, bias)
@@ -1115,8 +944,8 @@ def gemm_i8_dq(a, w, a_scale, w_scale, bias=None, out_dtype=torch.float16, exact
 
 
 def gemm_fp8_dq(a, w, a_scale, w_scale, bias=None, out_dtype=torch.bfloat16, force_gemv=False):  # noqa: F811
-    if not force_gemv:
-        y = _gemm_fp8_dq_lean(a, w, a_scale, w_scale, bias, out_dtype)
+    if not force_gemv and not _COMPILING():
+        y = (_H or _host()).gemm_dq(a, w, a_scale, w_scale, bias, out_dtype, 0)
         if y is not None:
             return y
     _need_gpu(a, w, bias)
@@ -1200,9 +1029,10 @@ def decode_linear_i8(x, w, w_scale, bias=None, smooth=None, out_dtype=torch.floa
                      saturate=False):
     """(y [M,N], per-token scales fp32 [M]) = quantize x per token (see quant_act_i8_pertoken) and
     multiply with the int8 weights w [N,K], in one launch; check ``decode_linear_ok`` first."""
-    r = _decode_linear_i8_lean(x, w, w_scale, bias, smooth, out_dtype, exact_ref, saturate)
-    if r is not None:
-        return r
+    if not _COMPILING():
+        r = (_H or _host()).decode_i8(x, w, w_scale, bias, smooth, out_dtype, L.EPI_REF_F16 if exact_ref else L.EPI_F32, saturate)
+        if r is not None:
+            return r
     _need_gpu(x, w, bias, smooth)
     if _eager(x, w, bias, smooth) and (not torch.is_tensor(w_scale) or _eager(w_scale)):
         return _decode_linear_i8_impl(x, w, w_scale, bias, smooth, out_dtype, bool(exact_ref), bool(saturate))
@@ -1245,9 +1075,10 @@ _register(
 def decode_linear_fp8(x, w, w_scale, bias=None, out_dtype=torch.bfloat16):
     """(y [M,N], token scales fp32 [M]): dynamic per-token e4m3 quantizer (the FP8Linear recipe) and
     the e4m3 weight-streaming matmul in one launch; check ``decode_linear_ok(x, None, K)`` first."""
-    r = _decode_linear_fp8_lean(x, w, w_scale, bias, out_dtype)
-    if r is not None:
-        return r
+    if not _COMPILING():
+        r = (_H or _host()).decode_fp8(x, w, w_scale, bias, out_dtype)
+        if r is not None:
+            return r
     _need_gpu(x, w, bias)
     if _eager(x, w, bias) and (not torch.is_tensor(w_scale) or _eager(w_scale)):
         return _decode_linear_fp8_impl(x, w, w_scale, bias, out_dtype)

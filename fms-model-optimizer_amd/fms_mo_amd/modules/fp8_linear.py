@@ -74,9 +74,15 @@ class FP8Linear(nn.Module):
         return m
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        act = self.linear_config["input_activations"]
+        if act is not None and act["dynamic"] and not torch.compiler.is_compiling():
+            # the dynamic forms, natively; None: something here is less common
+            y = L.host().fp8_linear(self._parameters, self.has_bias, x, act["strategy"] == "tensor",
+                                    self.dynamic_scale_floor, self.dynamic_scale_in_input_dtype)
+            if y is not None:
+                return y
         if not x.is_cuda:
             raise RuntimeError("fms_mo_amd.FP8Linear runs on an AMD GPU only; there is no CPU path")
-        act = self.linear_config["input_activations"]
         out_shape = tuple(x.shape[:-1]) + (self.out_features,)
         x2 = x.reshape(-1, x.shape[-1])
         with torch.no_grad():

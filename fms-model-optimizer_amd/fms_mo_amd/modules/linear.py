@@ -819,6 +819,11 @@ class QLinearINT8Deploy(nn.Linear):
         # (the reference runs this forward under torch.no_grad; the kernel paths below create their
         # outputs outside autograd anyway, and the torch-op branch enters no_grad itself -- an eager
         # decode step is bound by what the host does per call, so nothing is done twice here)
+        if type(self) is QLinearINT8Deploy and not torch.compiler.is_compiling():
+            # the dynamic per-token forms, natively; None: something here is less common
+            y = L.host().deploy_i8(self.__dict__, x, _IADDMM_INT)
+            if y is not None:
+                return y
         org_dtype = x.dtype
         K = x.shape[-1]
         two_d = x.dim() == 2
@@ -858,6 +863,10 @@ class QLinearINT8Deploy(nn.Linear):
         if not two_d:
             y = y.reshape(tuple(x.shape[:-1]) + (y.shape[-1],))
         return y if y.dtype == org_dtype else y.to(org_dtype)
+
+
+# deploy_i8 knows what a module's iaddmm does only where it is the class's own
+_IADDMM_INT = QLinearINT8Deploy.iaddmm_int
 
 
 class LinearFPxAcc(torch.nn.Linear):

@@ -649,6 +649,12 @@ int fmsmo_absmax_cols(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_
                       fmsmo_stream_t stream);
 
 /*
+ * out[m] = scale[m] * 127 and out[M + m] = -out[m]: the clip values a dynamic per-token scale stands for
+ * (cvs[0:2] of QLinearINT8Deploy, fms_mo/modules/linear.py:1085-1100).
+ */
+int fmsmo_clip_values(const float* scale, float* out, int64_t M, fmsmo_stream_t stream);
+
+/*
  * The vectors of a deployed linear with dynamic activation scales, in one launch:
  *   smooth[k]   = max(act[k]^alpha / max(w_absmax[k], 1e-5)^(1 - alpha), 1e-5)   (act NULL: no SmoothQuant)
  *   zero_seen[b]  whether one of act[256 b .. 256 b + 255] is 0, ceil(K / 256) flags
