@@ -97,9 +97,9 @@ static int gemm_i8_dq_impl(const int8_t* a, int64_t lda, const int8_t* b, int64_
                                               epilogue == FMSMO_EPI_F32_MULADD);
   }
   if (epilogue == FMSMO_EPI_REF_F16)
-    return launch_dq<MMA_I8, true, int, false>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y,
+    return launch_dq<MMA_I8, true, int>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y,
                                                y_dtype, ldy, (hipStream_t)stream);
-  return launch_dq<MMA_I8, false, int, false>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y,
+  return launch_dq<MMA_I8, false, int>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y,
                                               y_dtype, ldy, (hipStream_t)stream, true,
                                               epilogue == FMSMO_EPI_F32_MULADD);
 }
@@ -263,35 +263,6 @@ extern "C" int fmsmo_gemm_fp8_plan(int64_t M, int64_t N, int64_t K, int with_wor
   if (with_workspace == 2) return FMSMO_ERR_UNSUPPORTED;  // there is no e4m3 call on the static scratch
   return gemm_plan(true, M, N, K, with_workspace, kernel, tile_m, tile_n, splits);
 }
-
-extern "C" int fmsmo_grouped_gemm_i8_dq(const int8_t* a, int64_t lda, const int8_t* b,
-                                        int64_t ldb, int64_t ldb_e, const int32_t* offsets,
-                                        int num_experts, int64_t total_rows, const float* a_scale,
-                                        const float* w_scale, const void* bias, int bias_dtype,
-                                        int epilogue, void* y, int y_dtype, int64_t ldy, int64_t N,
-                                        int64_t K, fmsmo_stream_t stream) {
-  int rc = check_gemm(a, lda, b, ldb, y, ldy, total_rows, N, K);
-  if (rc) return rc;
-  if (!offsets || !a_scale || !w_scale) return FMSMO_ERR_NULL;
-  if (num_experts <= 0 || ldb_e < N * ldb) return FMSMO_ERR_SHAPE;
-  if ((int64_t)num_experts * ldb_e >= (1ll << 40)) return FMSMO_ERR_UNSUPPORTED;
-  if (K % 64 || ldb_e % 16) return FMSMO_ERR_ALIGN;
-  if (y_dtype < 0 || y_dtype > 2 || (bias && (bias_dtype < 0 || bias_dtype > 2))) return FMSMO_ERR_UNSUPPORTED;
-  if (epilogue < FMSMO_EPI_REF_F16 || epilogue > FMSMO_EPI_F32_MULADD) return FMSMO_ERR_UNSUPPORTED;
-  if (total_rows == 0) return FMSMO_OK;
-  GemmArgs g{};
-  g.a = (const uint8_t*)a; g.b = (const uint8_t*)b; g.lda = lda; g.ldb = ldb;
-  g.M = (int)total_rows; g.N = (int)N; g.K = (int)K;
-  g.offsets = offsets; g.num_experts = num_experts; g.ldb_e = ldb_e;
-  g.grid_m = div_up(total_rows, TileBig::BM) + num_experts;  // upper bound on row tiles
-  if (epilogue == FMSMO_EPI_REF_F16)
-    return launch_dq<MMA_I8, true, int, true>(g, a_scale, 1, w_scale, 1, bias, bias_dtype, y,
-                                              y_dtype, ldy, (hipStream_t)stream);
-  return launch_dq<MMA_I8, false, int, true>(g, a_scale, 1, w_scale, 1, bias, bias_dtype, y,
-                                             y_dtype, ldy, (hipStream_t)stream, true,
-                                             epilogue == FMSMO_EPI_F32_MULADD);
-}
-
 
 extern "C" int fmsmo_bmm_i8_dq(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
                                int64_t stride_b, const float* a_scale, const float* b_scale,

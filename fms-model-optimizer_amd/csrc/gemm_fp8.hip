@@ -34,9 +34,9 @@ static int gemm_fp8_dq_impl(const uint8_t* a, int64_t lda, const uint8_t* b, int
   // 128 x 64 in front: 192 (300 x 4096) 22.3 / 27.4 / 46.7; 256 (1000 x 2048) 24.1 / 27.3 / 46.9; 320 (600 x 4096) 40.6 / 29.8 / 47.2;
   // 512 (1000 x 4096) 45.1 / 35.3 / 47.9; 2048 (4000 x 4096) 163.6 / 131.2 / 121.8: 7 % for one more instance, left out).
   if (K % 64)
-    return launch_dq<MMA_FP8_F16, false, float, false>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y, y_dtype, ldy,
+    return launch_dq<MMA_FP8_F16, false, float>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y, y_dtype, ldy,
                                                        (hipStream_t)stream);
-  return launch_dq<MMA_FP8, false, float, false>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y,
+  return launch_dq<MMA_FP8, false, float>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y,
                                                  y_dtype, ldy, (hipStream_t)stream);
 }
 

@@ -252,37 +252,31 @@ inline int tail_split_columns(int M, int N, int K) {
   return (int)(N - (gn - cut) * 256);
 }
 
-template <int OP, bool REF, class AccT, bool GROUPED>
+template <int OP, bool REF, class AccT>
 int launch_dq(const GemmArgs& g, const float* a_scale, int a_stride, const float* w_scale,
               int w_stride, const void* bias, int bias_dtype, void* y, int y_dtype, int64_t ldy,
               hipStream_t st, bool may_split = true, int muladd = 0) {
   if (!bias) bias_dtype = FMSMO_F32;
-  if constexpr (!GROUPED) {
-    const int tail = may_split ? tail_split_columns(g.M, g.N, g.K) : 0;
-    if (tail > 0) {
-      const int64_t n0 = g.N - tail;
-      GemmArgs g1 = g, g2 = g;
-      g1.N = (int)n0;
-      g2.N = tail;
-      g2.b = g.b + n0 * g.ldb;
-      const int64_t ysz = y_dtype == FMSMO_F32 ? 4 : 2, bsz = bias_dtype == FMSMO_F32 ? 4 : 2;
-      int rc = launch_dq<OP, REF, AccT, false>(g1, a_scale, a_stride, w_scale, w_stride, bias, bias_dtype,
-                                               y, y_dtype, ldy, st, false, muladd);
-      if (rc) return rc;
-      return launch_dq<OP, REF, AccT, false>(
-          g2, a_scale, a_stride, w_scale + (w_stride ? n0 : 0), w_stride,
-          bias ? (const void*)((const char*)bias + n0 * bsz) : nullptr, bias_dtype,
-          (void*)((char*)y + n0 * ysz), y_dtype, ldy, st, false, muladd);
-    }
+  const int tail = may_split ? tail_split_columns(g.M, g.N, g.K) : 0;
+  if (tail > 0) {
+    const int64_t n0 = g.N - tail;
+    GemmArgs g1 = g, g2 = g;
+    g1.N = (int)n0;
+    g2.N = tail;
+    g2.b = g.b + n0 * g.ldb;
+    const int64_t ysz = y_dtype == FMSMO_F32 ? 4 : 2, bsz = bias_dtype == FMSMO_F32 ? 4 : 2;
+    int rc = launch_dq<OP, REF, AccT>(g1, a_scale, a_stride, w_scale, w_stride, bias, bias_dtype,
+                                             y, y_dtype, ldy, st, false, muladd);
+    if (rc) return rc;
+    return launch_dq<OP, REF, AccT>(
+        g2, a_scale, a_stride, w_scale + (w_stride ? n0 : 0), w_stride,
+        bias ? (const void*)((const char*)bias + n0 * bsz) : nullptr, bias_dtype,
+        (void*)((char*)y + n0 * ysz), y_dtype, ldy, st, false, muladd);
   }
 #define GO(OUT, BIAS)                                                                         \
   {                                                                                           \
     EpiDequant<OUT, BIAS, REF, AccT, OP == MMA_I8 || OUT == FMSMO_F32> epi{y, ldy, a_scale, w_scale, bias, a_stride, w_stride, muladd}; \
-    if constexpr (GROUPED) {                                                                  \
-      if (g.K % 128 == 0 && use_register_staged(OP)) launch_rs<OP, true>(g, epi, st);         \
-      else launch_tile<TileBig, OP, true>(g, epi, st);                                        \
-    } else                                                                                    \
-      launch_any<OP>(g, epi, st);                                                             \
+    launch_any<OP>(g, epi, st);                                                               \
   }
 #define GO_BIAS(OUT)                            \
   switch (bias_dtype) {                         \

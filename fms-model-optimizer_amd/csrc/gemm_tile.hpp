@@ -148,6 +148,46 @@ __device__ __forceinline__ void tile_of_block(int bid, int nblk, int grid_m, int
   tn = r / gsz;
 }
 
+// Row tiles of `bm` rows over all groups (rows offsets[e] .. offsets[e + 1]), and the group that owns row tile
+// `tile`: 64 groups at a time, one per lane (one after the other, each waiting for its offsets, 16 groups took
+// 2 us of every block).
+__device__ __forceinline__ int wave_scan_add(int v, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(v, o, 64);
+    v += lane >= o ? u : 0;
+  }
+  return v;
+}
+__device__ __forceinline__ int group_tiles(const int32_t* offsets, int groups, int bm, int lane) {
+  int sum = 0;
+  for (int e0 = 0; e0 < groups; e0 += 64) {
+    const int e = e0 + lane;
+    sum += e < groups ? (offsets[e + 1] - offsets[e] + bm - 1) / bm : 0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  return __builtin_amdgcn_readfirstlane(sum);
+}
+__device__ __forceinline__ void group_of_tile(const int32_t* offsets, int groups, int bm, int lane, int tile,
+                                              int& group, int& row_lo, int& row_hi) {
+  for (int e0 = 0, before = 0; e0 < groups; e0 += 64) {
+    const int e = min(e0 + lane, groups - 1);
+    const int lo = offsets[e], hi = offsets[e + 1];
+    const int n = e0 + lane < groups ? (hi - lo + bm - 1) / bm : 0;
+    const int incl = before + wave_scan_add(n, lane);
+    const unsigned long long after = __ballot(incl > tile);  // the first such lane owns it
+    if (after) {
+      const int l = __builtin_ctzll(after);
+      group = e0 + l;
+      row_lo = __builtin_amdgcn_readlane(lo, l) + (tile - __builtin_amdgcn_readlane(incl - n, l)) * bm;
+      row_hi = __builtin_amdgcn_readlane(hi, l);
+      return;
+    }
+    before = __builtin_amdgcn_readlane(incl, 63);
+  }
+}
+
 template <int BM, int BN, int BK, int NSTAGE, int WGM, int WGN, int OP, int SWZ, bool GROUPED,
           class Epi, bool KT = false>
 __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_tile_kernel(GemmArgs g, Epi epi) {
@@ -193,23 +233,10 @@ __global__ __launch_bounds__(WGM* WGN * 64, 1) void gemm_tile_kernel(GemmArgs g,
       // real row tiles and map only the first real_tiles block ids, so that every XCD gets an
       // equal share of real work; the surplus blocks are the last to be dispatched and exit at
       // once.
-      int real_m = 0;
-      for (int e = 0; e < g.num_experts; ++e) real_m += (g.offsets[e + 1] - g.offsets[e] + BM - 1) / BM;
-      const int real_tiles = real_m * g.grid_n;
+      const int real_tiles = group_tiles(g.offsets, g.num_experts, BM, lane) * g.grid_n;
       if ((int)blockIdx.x >= real_tiles) return;  // uniform for the whole block
-      tile_of_block(blockIdx.x, real_tiles, real_m, g.grid_n, g.group_m, tile_m, tile_n);
-      int t = tile_m;
-      for (int e = 0; e < g.num_experts; ++e) {
-        const int lo = g.offsets[e], hi = g.offsets[e + 1];
-        const int nt = (hi - lo + BM - 1) / BM;
-        if (t < nt) {
-          row_lo = lo + t * BM;
-          row_hi = hi;
-          expert = e;
-          break;
-        }
-        t -= nt;
-      }
+      tile_of_block(blockIdx.x, real_tiles, real_tiles / g.grid_n, g.grid_n, g.group_m, tile_m, tile_n);
+      group_of_tile(g.offsets, g.num_experts, BM, lane, tile_m, expert, row_lo, row_hi);
     }
   } else {
     tile_of_block(blockIdx.x, gridDim.x, g.grid_m, g.grid_n, g.group_m, tile_m, tile_n);

@@ -510,3 +510,31 @@ def test_vectors_of_a_converted_linear(dev, dtype, Kd, N, bias, stats):
     assert torch.equal(dep.w_zp, torch.zeros(N, dtype=torch.int32, device=dev)) and int(dep.input_zp) == 127
     assert list(dep.state_dict()) == ["weight", "input_scale", "input_zp", "w_scale", "w_zp", "smoothq_scale", "corr_term", "bias"]
     assert float(dep.input_scale) == 1 and [float(v) for v in dep.cvs[:2]] == [8.0, -8.0]
+
+
+@pytest.mark.parametrize("counts,N,Kd", [
+    ([3, 0, 1, 5], 130, 256),                       # a few rows per expert: 32 x 128 tiles
+    ([0] * 40 + [1, 2, 33] + [0] * 30 + [64, 1], 72, 384),   # more groups than lanes, most of them empty
+    ([43, 64, 65, 0], 200, 1024),                   # 64 x 64
+    ([180, 256, 100, 129, 181], 1100, 640),         # 128 x 128, 64-byte stages
+    ([350, 300, 257, 384, 1], 2500, 4096),          # 128 x 128, 128-byte stages
+    ([513, 0, 700, 2000], 8200, 512),               # 256 x 256
+    ([10, 200, 127], 300, 192)])                    # reduction of whole 64-byte stages only
+@pytest.mark.parametrize("exact_ref,out_dtype", [(True, torch.float16), (False, torch.float32)])
+def test_grouped_products_in_every_tile(dev, counts, N, Kd, exact_ref, out_dtype):
+    """Bit-identical to one product per expert (integer sums, the same epilogue), rows of no expert untouched."""
+    kn = K()
+    E, T = len(counts), sum(counts)
+    g = torch.Generator(device=dev).manual_seed(N)
+    a = torch.randint(-128, 128, (T, Kd), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-128, 128, (E, N, Kd), generator=g, dtype=torch.int8, device=dev)
+    sa, sw = torch.rand(T, generator=g, device=dev) * 1e-3, torch.rand(E, N, generator=g, device=dev) * 1e-2
+    b = torch.randn(E, N, generator=g, device=dev)
+    off = torch.tensor([0] + counts, device=dev).cumsum(0).to(torch.int32)
+    y = kn.grouped_gemm_i8_dq(a, w, off, sa, sw, b, out_dtype=out_dtype, exact_ref=exact_ref)
+    lo = 0
+    for e, c in enumerate(counts):
+        if c:
+            ref = kn.gemm_i8_dq(a[lo:lo + c], w[e], sa[lo:lo + c], sw[e], b[e], out_dtype=out_dtype, exact_ref=exact_ref)
+            assert torch.equal(y[lo:lo + c], ref), e
+        lo += c
