@@ -45,7 +45,7 @@ extern "C" int fmsmo_gemm_i8_i32_ws(const int8_t* a, int64_t lda, const int8_t* 
   if (rc) return rc;
   if (M == 0) return FMSMO_OK;
   // a few tokens: the weight-streaming decode kernels, storing their int32 sums
-  if ((M <= 16 && K % 128 == 0) || fmsmo_gemv_batch_ok(M, K))
+  if (use_decode(M, N, K))
     return fmsmo_gemv_dispatch(FMSMO_OP_I8, a, lda, b, ldb, nullptr, 1, nullptr, 1, nullptr, FMSMO_F32,
                                EPI_RAW_I32, c, FMSMO_F32, ldc, M, N, K, (hipStream_t)stream);
   GemmArgs g{};
@@ -78,7 +78,7 @@ static int gemm_i8_dq_impl(const int8_t* a, int64_t lda, const int8_t* b, int64_
   if (rc) return rc;
   if (epilogue < FMSMO_EPI_REF_F16 || epilogue > FMSMO_EPI_F32_MULADD) return FMSMO_ERR_UNSUPPORTED;
   if (M == 0) return FMSMO_OK;
-  if ((M <= 16 && K % 128 == 0) || fmsmo_gemv_batch_ok(M, K))
+  if (use_decode(M, N, K))
     return fmsmo_gemv_dispatch(FMSMO_OP_I8, a, lda, b, ldb, a_scale, a_scale_n, w_scale, w_scale_n,
                                bias, bias_dtype, epilogue, y, y_dtype, ldy, M, N, K,
                                (hipStream_t)stream);
@@ -172,7 +172,7 @@ extern "C" int fmsmo_gemm_i8_dq_noalloc(const int8_t* a, int64_t lda, const int8
   if (epilogue < FMSMO_EPI_REF_F16 || epilogue > FMSMO_EPI_F32_MULADD) return FMSMO_ERR_UNSUPPORTED;
   if (M == 0) return FMSMO_OK;
   // the weight-streaming decode kernels use no scratch
-  const bool decode = (M <= 16 && K % 128 == 0) || fmsmo_gemv_batch_ok(M, K);
+  const bool decode = use_decode(M, N, K);
   // (the plan that fits the scratch, if one does: else the preferred plan's size is reported)
   int64_t need = decode ? 0 : plan_split_k(M, N, K, (int64_t)FMSMO_STATIC_SCRATCH_BYTES).ws_bytes;
   if (need > (int64_t)FMSMO_STATIC_SCRATCH_BYTES) {
@@ -202,7 +202,7 @@ extern "C" int64_t fmsmo_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t 
 
 extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
-  if ((M <= 16 && K % 128 == 0) || fmsmo_gemv_batch_ok(M, K)) return 0;
+  if (use_decode(M, N, K)) return 0;
   return tail_split_columns((int)M, (int)N, (int)K);
 }
 
@@ -214,13 +214,14 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
   if (K % 16) return FMSMO_ERR_ALIGN;
   *tile_m = *tile_n = 0;
   *splits = 1;
-  if ((M <= 16 && K % 128 == 0) || fmsmo_gemv_batch_ok(M, K)) {
+  if (use_decode(M, N, K)) {
     *kernel = FMSMO_PLAN_DECODE;
     return FMSMO_OK;
   }
-  if (use_tall_tiles(M, N, K)) {  // one pass of 128 x 64 tiles, with or without a workspace
+  // one pass of 64 x 64 or 128 x 64 tiles, with or without a workspace
+  if (use_small_tiles(M, N, K) || use_tall_tiles(M, N, K)) {
     *kernel = FMSMO_PLAN_TILE_LDS_DMA;
-    *tile_m = TileTallK::BM;
+    *tile_m = use_small_tiles(M, N, K) ? TileSmallK::BM : TileTallK::BM;
     *tile_n = TileTallK::BN;
     return FMSMO_OK;
   }
@@ -230,8 +231,8 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
     return FMSMO_ERR_SCRATCH;  // what the noalloc entry point returns for this shape
   if (with_workspace && plan.splits > 1) {
     *kernel = plan.rs ? FMSMO_PLAN_TILE_REGISTER_STAGED : FMSMO_PLAN_TILE_LDS_DMA;
-    *tile_m = plan.rs ? 256 : TileMid::BM;
-    *tile_n = plan.rs ? 128 : plan.tall ? TileTallK::BN : TileMid::BN;
+    *tile_m = plan.rs ? 256 : plan.small ? TileSmallK::BM : TileMid::BM;
+    *tile_n = plan.rs ? 128 : plan.tall || plan.small ? TileTallK::BN : TileMid::BN;
     *splits = plan.splits;
     return FMSMO_OK;
   }

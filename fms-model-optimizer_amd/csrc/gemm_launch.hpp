@@ -48,6 +48,37 @@ struct TileMid { static constexpr int BM = 128, BN = 128, BK = 64, NST = 4, WGM 
 struct TileMidK { static constexpr int BM = 128, BN = 128, BK = 128, NST = 4, WGM = 2, WGN = 2; };
 struct TileTallK { static constexpr int BM = 128, BN = 64, BK = 128, NST = 5, WGM = 2, WGN = 2; };
 
+// 64 x 64 tiles, two blocks per compute unit, for launches that would leave most compute units idle or take
+// K slices and a second kernel.
+struct TileSmallK { static constexpr int BM = 64, BN = 64, BK = 128, NST = 4, WGM = 2, WGN = 2; };
+
+// Which launches they take: up to one block per compute unit on reductions under 2048 (one pass takes 3.3 us + 1.6
+// per 1024 of K, less than a pass of any other tile; from there on slices of two or four come close), up to 3072
+// above 128 rows and under 8192 above 256 rows, whose partial sums cost more than they save; up to two per compute
+// unit on short ones.  (33 .. 64 tiles, and the reductions these bounds leave out, keep the plans they had, some of
+// which callers and tests rely on.)  Up to 64 tokens the decode kernels re-read the activations for every 16 weight
+// rows and win until there are many of those.  us from a HIP graph, int8 | e4m3, before -> these:
+//   N = 6144, K = 1024: M = 100 10.4 -> 5.3; N = 2432, K = 2048: 200 10.4 -> 6.8, 400 9.0 -> 8.1; N = 4096, K = 3072:
+//   200 11.6 -> 8.9 | 10.7 -> 7.5; N = 1024: K = 4096, M = 800 13.5 -> 10.6, 1000 13.6 -> 10.9; K = 5120 / 6144, M = 1000
+//   16.8 / 17.9 -> 12.3 / 14.0 | 16.5 / 17.0 -> 11.0 / 13.8; N = 2048, M = 500 17.7 / 18.6 -> 12.4 / 14.5; N = 512, K = 1024:
+//   800 8.9 -> 5.1, 1500 8.3 -> 5.4, 2500 8.8 -> 6.3, 4000 8.6 -> 6.8 (504 tiles).
+//   Up to 64 tokens: N = 12288, K = 1024: M = 17 5.1 -> 4.9 | 5.8 -> 4.6, 40 7.4 -> 5.2, 64 8.7 -> 5.1; N = 28672: 17 9.8 ->
+//   6.0, 64 15.8 -> 6.8; N = 14336, K = 4096: 17 13.4 -> 11.4, 40 18.0 -> 12.2 | 18.8 -> 11.8; N = 8192: 33 11.0 -> 10.5, 64 14.9 ->
+//   10.5; kept: N = 4096, K = 4096, 33 8.9 against 9.7; N = 8192, 32 9.6 against 10.5
+inline bool use_small_tiles(int64_t M, int64_t N, int64_t K) {
+  if (M <= 16 || K % 128 || K >= 8192) return false;
+  const int64_t tiles = (int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN);
+  if (tiles > 512) return false;
+  if (fmsmo_gemv_batch_ok(M, K)) return K <= (tiles > 256 ? 2048 : 4096) && tiles >= (M > 32 ? 128 : 192);
+  if (tiles > 256) return K <= 1536;
+  if (tiles > 64) return K < 2048 || (M > 128 && K <= 3072) || M > 256;
+  return tiles <= 32 && K < 2048;
+}
+// The decode kernels take the launch.
+inline bool use_decode(int64_t M, int64_t N, int64_t K) {
+  return (M <= 16 && K % 128 == 0) || (fmsmo_gemv_batch_ok(M, K) && !use_small_tiles(M, N, K));
+}
+
 // A few hundred rows through a projection whose 128 x 64 tiles fill half a round of the 256
 // compute units or more run as ONE pass of those tiles rather than as K slices with a second
 // kernel: no partial sums to write and read back.  A block walks K in ~0.41 us per 128-byte stage (one
@@ -201,6 +232,8 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
   if constexpr (OP == MMA_FP8_F16) {  // K % 64 != 0
     if (cut_k_tall(g.M, g.N, g.K)) launch_tile<TileTallK, OP, false, true>(g, epi, st);
     else launch_tile<TileMidK, OP, false, true>(g, epi, st);
+  } else if (use_small_tiles(g.M, g.N, g.K)) {
+    launch_tile<TileSmallK, OP, false>(g, epi, st);
   } else if (use_tall_tiles(g.M, g.N, g.K)) {
     launch_tile<TileTallK, OP, false>(g, epi, st);
   } else if (g.K % 64 == 0 && !cut_k_tall(g.M, g.N, g.K)) {
@@ -320,7 +353,8 @@ struct SplitPlan {
   int64_t k_len, ws_bytes;
   bool rs;  // 256 x 128 tiles of the register-staged kernel instead of 128 x 128 LDS-DMA tiles
   bool tall = false;  // 128 x 64 tiles with 128-byte stages
-  bool cut = false;   // the last slice is shorter than k_len (KT instances of the tall tiles)
+  bool cut = false;   // the last slice is shorter than k_len (KT instances of the tall and the small tiles)
+  bool small = false; // 64 x 64 tiles with 128-byte stages
 };
 
 // K in `s` slices of whole 128-byte stages of at least 1024 bytes on 128 x 64 tiles, the last one shorter
@@ -341,9 +375,25 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   SplitPlan p{1, K, 0, false};
   static const char* off = getenv("FMSMO_SPLIT_K");  // FMSMO_SPLIT_K=0 disables (tuning aid)
   if (off && off[0] == '0') return p;
-  if (M <= 16 || M > 1024 || use_tall_tiles(M, N, K)) return p;
+  if (M <= 16 || M > 1024 || use_small_tiles(M, N, K) || use_tall_tiles(M, N, K)) return p;
   const int64_t tiles_t = (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN);
   const int64_t room = limit > 0 ? limit / (M * N * 4) : 256;
+  const int64_t tiles_s = (int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN);
+  if (K % 128 == 0 && tiles_s <= 32 && K > 2048) {
+    // Few tiles: slices on 64 x 64 ones, four (eight of a long reduction: from then on the partial sums cost more
+    // than a shorter pass saves).  us, slices of 128 x 64 tiles -> these, M = 100, N = 1024: K = 3072 8.7 -> 6.9, 4096 9.2 ->
+    // 7.2, 6144 9.9 -> 8.0, 8192 9.8 -> 8.8, 14336 13.7 -> 10.8 (four: 11.2); N = 256, K = 4096 8.2 -> 6.9; 40 x 512 x 9344
+    // 10.3 -> 9.3; e4m3 within 3 % of these
+    const int want = (int)std::min<int64_t>(K >= 12288 ? 8 : 4, room);
+    if (want >= 2) {
+      p.k_len = ((K + want - 1) / want + 127) / 128 * 128;
+      p.splits = (int)((K + p.k_len - 1) / p.k_len);
+      p.ws_bytes = (int64_t)p.splits * M * N * 4;
+      p.small = true;
+      p.cut = K % p.k_len != 0;
+      return p;
+    }
+  }
   if (K % 128) {
     // (us, one pass -> slices, M = 40: N = 1024, K = 4016 13.1 -> 8.8; N = 3072 13.6 -> 10.3; M = 100,
     // N = 3072, K = 8208 26.3 -> 14.4; M = 200, N = 1500, K = 11216 36.7 -> 16.7.  From a quarter of a
@@ -444,8 +494,10 @@ inline int launch_split_k_i32(const SplitPlan& p, const GemmArgs& g0, void* work
   g.lda_e = p.k_len;
   g.ldb_e = p.k_len;
   g.k_total = g0.K;
-  g.grid_m = p.splits * div_up(g0.M, p.rs ? 256 : TileMid::BM);
-  if (p.rs) launch_rs<MMA_I8, true, 128>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
+  g.grid_m = p.splits * div_up(g0.M, p.rs ? 256 : p.small ? TileSmallK::BM : TileMid::BM);
+  if (p.small && p.cut) launch_tile<TileSmallK, MMA_I8, true, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
+  else if (p.small) launch_tile<TileSmallK, MMA_I8, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
+  else if (p.rs) launch_rs<MMA_I8, true, 128>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
   else if (p.cut) launch_tile<TileTallK, MMA_I8, true, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
   else if (p.tall) launch_tile<TileTallK, MMA_I8, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
   else launch_tile<TileMid, MMA_I8, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
@@ -469,9 +521,15 @@ int launch_split_k(const SplitPlan& p, const GemmArgs& g0, void* workspace, cons
   g.lda_e = p.k_len;
   g.ldb_e = p.k_len;
   g.k_total = g0.K;
-  g.grid_m = p.splits * div_up(g0.M, p.rs ? 256 : TileMid::BM);
+  g.grid_m = p.splits * div_up(g0.M, p.rs ? 256 : p.small ? TileSmallK::BM : TileMid::BM);
   if constexpr (OP == MMA_FP8_F16) {  // K % 64 != 0: such plans are cut ones
     launch_tile<TileTallK, OP, true, true>(g, EpiStoreF32{(float*)workspace, g0.N}, st);
+  } else if (p.small && p.cut) {
+    if constexpr (OP == MMA_I8) launch_tile<TileSmallK, OP, true, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
+    else launch_tile<TileSmallK, OP, true, true>(g, EpiStoreF32{(float*)workspace, g0.N}, st);
+  } else if (p.small) {
+    if constexpr (OP == MMA_I8) launch_tile<TileSmallK, OP, true>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
+    else launch_tile<TileSmallK, OP, true>(g, EpiStoreF32{(float*)workspace, g0.N}, st);
   } else if (p.rs) {
     if constexpr (OP == MMA_I8) launch_rs<OP, true, 128>(g, EpiStoreI32{(int32_t*)workspace, g0.N}, st);
     else launch_rs<OP, true, 128>(g, EpiStoreF32{(float*)workspace, g0.N}, st);

@@ -538,3 +538,30 @@ def test_grouped_products_in_every_tile(dev, counts, N, Kd, exact_ref, out_dtype
             ref = kn.gemm_i8_dq(a[lo:lo + c], w[e], sa[lo:lo + c], sw[e], b[e], out_dtype=out_dtype, exact_ref=exact_ref)
             assert torch.equal(y[lo:lo + c], ref), e
         lo += c
+
+
+@pytest.mark.parametrize("M,N,Kd,slices", [
+    (17, 12290, 1024, 1), (33, 8200, 4096, 1), (64, 28600, 2048, 1),       # up to 64 tokens, many columns
+    (65, 1000, 1920, 1), (100, 5000, 128, 1), (129, 2050, 3072, 1), (257, 1030, 8064, 1),   # up to one block per unit
+    (700, 1500, 1536, 1), (4033, 500, 1024, 1), (1, 64, 256, 0),           # up to two; (a decode launch beside them)
+    (100, 1000, 2176, 4), (70, 300, 4736, 4), (128, 1024, 14336, 8), (90, 60, 12416, 8)])   # slices, the last one shorter
+def test_small_tiles(dev, M, N, Kd, slices):
+    """64 x 64 tiles at the ends of the ranges that take them, ragged edges included: int8 exact, e4m3 exact on small
+    integers (sums below 2^24), rows and columns past the end untouched."""
+    kn = K()
+    for fp8 in (False, True):
+        plan = kn.gemm_plan(M, N, Kd, with_workspace=True, fp8=fp8)
+        if slices:
+            assert plan[1:3] == (64, 64) and plan[3] == slices, plan
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    a = torch.randint(-128, 128, (M, Kd), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-128, 128, (N, Kd), generator=g, dtype=torch.int8, device=dev)
+    assert torch.equal(kn.gemm_i8_i32(a, w), (a.double() @ w.double().t()).to(torch.int32))
+    a, w = a.float().div(32).round(), w.float().div(32).round()
+    ref = (a.double() @ w.double().t()).float()
+    one = torch.ones(1, device=dev)
+    y = kn.gemm_fp8_dq(a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn), one, one, None, out_dtype=torch.float32)
+    assert torch.equal(y, ref)
+    sa, sw = torch.rand(M, generator=g, device=dev), torch.rand(N, generator=g, device=dev)
+    y = kn.gemm_i8_dq(a.to(torch.int8), w.to(torch.int8), sa, sw, None, out_dtype=torch.float32, exact_ref=False)
+    torch.testing.assert_close(y, ref * (sa[:, None] * sw[None, :]), rtol=1e-6, atol=0)
