@@ -29,11 +29,20 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   return r;
 }
 
+// The clip values a dynamic scale stands for, +- scale * 127, as [2][M] (written with the scale: as two vector
+// operators behind the quantizer they were two launches of 5 us)
+__device__ __forceinline__ void put_clips(float* clips, int row, int M, float s) {
+  const float a = s * 127.0f;
+  clips[row] = a;
+  clips[(size_t)M + row] = -a;
+}
+
 // ------------------------------------------------------------------ int8, dynamic per token
 template <int XT, int T>
 __global__ __launch_bounds__(AQ_THREADS) void quant_i8_pertoken_kernel(
     const void* __restrict__ x, int64_t ldx, const void* __restrict__ smooth, int smooth_dtype,
-    int saturate, int8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale, int K) {
+    int saturate, int8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale,
+    float* __restrict__ clips, int K) {
   __shared__ float red[AQ_THREADS / 64];
   const int row = blockIdx.x;
   const size_t xrow = (size_t)row * ldx;
@@ -72,7 +81,10 @@ __global__ __launch_bounds__(AQ_THREADS) void quant_i8_pertoken_kernel(
 
   // s = rnd_T( max(amax, rnd_T(1e-5)) / 127 )
   const float s = round_to<T>(fmaxf(amax, round_to<T>(1e-5f)) / 127.0f);
-  if (threadIdx.x == 0) scale[row] = s;
+  if (threadIdx.x == 0) {
+    scale[row] = s;
+    if (clips) put_clips(clips, row, gridDim.x, s);
+  }
 
   auto emit = [&](int c, const float (&e)[8]) {
     uint8_t b[8];
@@ -120,7 +132,7 @@ __global__ __launch_bounds__(AQ_THREADS) void quant_i8_pertoken_kernel(
 template <int T, int NCH, bool SMOOTH, int TH = AQ_THREADS, bool KEEP = true>
 __global__ __launch_bounds__(TH) void quant_i8_pertoken16_kernel(
     const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ smooth, int saturate,
-    int8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale, int M, int K) {
+    int8_t* __restrict__ q, int64_t ldq, float* __restrict__ scale, float* __restrict__ clips, int M, int K) {
   // reciprocals of the divisors stay in registers across rows while the row is short enough
   constexpr bool KEEP_RCP = SMOOTH && KEEP;
   __shared__ float red[2][TH / 64];
@@ -254,6 +266,7 @@ __global__ __launch_bounds__(TH) void quant_i8_pertoken16_kernel(
       // row: IEEE divisions, straight from memory (block-uniform branch)
       quant_i8_row_ieee16<T, TH>(x + (size_t)row * ldx, SMOOTH ? smooth : nullptr, saturate,
                                  q + (size_t)row * ldq, scale + row, K, red[0]);
+      if (clips && threadIdx.x == 0) put_clips(clips, row, M, scale[row]);  // (this thread wrote the scale)
 #pragma unroll
       for (int i = 0; i < NCH; ++i) cur[i] = nxt[i];
       continue;
@@ -264,7 +277,10 @@ __global__ __launch_bounds__(TH) void quant_i8_pertoken16_kernel(
     // need no special-case fix-up unless the row overflowed the 16-bit range (amax = inf)
     const float s = cvt16<T>(to16<T>(fmaxf(amax, floor_T) / 127.0f));
     const float rs = __builtin_amdgcn_rcpf(s);
-    if (threadIdx.x == 0) scale[row] = s;
+    if (threadIdx.x == 0) {
+      scale[row] = s;
+      if (clips) put_clips(clips, row, M, s);
+    }
     int8_t* qr = q + (size_t)row * ldq;
     {
 #pragma unroll
@@ -1329,11 +1345,10 @@ static int64_t row_walk_grid(int64_t M, int64_t resident, bool one_row_per_block
   return one_row_per_block || M < resident ? M : resident;
 }
 
-extern "C" int fmsmo_quant_act_i8_pertoken(const void* x, int x_dtype, int64_t ldx,
-                                           const void* smooth, int smooth_dtype,
-                                           int compute_dtype, int saturate, int8_t* q, int64_t ldq,
-                                           float* scale, int64_t M, int64_t K,
-                                           fmsmo_stream_t stream) {
+// clips: NULL, or [2][M] for the clip values (without SmoothQuant divisors only)
+static int quant_act_i8_pertoken(const void* x, int x_dtype, int64_t ldx, const void* smooth, int smooth_dtype,
+                                 int compute_dtype, int saturate, int8_t* q, int64_t ldq, float* scale, float* clips,
+                                 int64_t M, int64_t K, fmsmo_stream_t stream) {
   if (!x || !q || !scale) return FMSMO_ERR_NULL;
   if (M < 0 || K <= 0 || ldx < K || ldq < K || M > 0x7fffffff || K > 0x7fffffff) return FMSMO_ERR_SHAPE;
   if (x_dtype < 0 || x_dtype > 2 || compute_dtype < 0 || compute_dtype > 2) return FMSMO_ERR_UNSUPPORTED;
@@ -1357,7 +1372,7 @@ extern "C" int fmsmo_quant_act_i8_pertoken(const void* x, int x_dtype, int64_t l
     dim3 grid16((unsigned)row_walk_grid(M, resident, !(SM) || (T == FMSMO_F16 && NCH <= 4))),    \
         block16(TH);                                                                             \
     hipLaunchKernelGGL((quant_i8_pertoken16_kernel<T, NCH, SM, TH, KEEP>), grid16, block16, 0,   \
-                       st, (const u16*)x, ldx, (const u16*)smooth, saturate, q, ldq, scale,      \
+                       st, (const u16*)x, ldx, (const u16*)smooth, saturate, q, ldq, scale, clips, \
                        (int)M, (int)K);                                                          \
   }
     // divisors with rows of up to 8192 elements: fp16 blocks run one row each and keep nothing;
@@ -1416,7 +1431,7 @@ extern "C" int fmsmo_quant_act_i8_pertoken(const void* x, int x_dtype, int64_t l
   dim3 grid((unsigned)M), block(AQ_THREADS);
 #define LAUNCH(XT, T)                                                                          \
   hipLaunchKernelGGL((quant_i8_pertoken_kernel<XT, T>), grid, block, 0, st, x, ldx, smooth,    \
-                     smooth_dtype, saturate, q, ldq, scale, (int)K)
+                     smooth_dtype, saturate, q, ldq, scale, clips, (int)K)
 #define DISPATCH_T(XT)                                                      \
   switch (compute_dtype) {                                                  \
     case FMSMO_F16: LAUNCH(XT, FMSMO_F16); break;                           \
@@ -1431,6 +1446,21 @@ extern "C" int fmsmo_quant_act_i8_pertoken(const void* x, int x_dtype, int64_t l
 #undef LAUNCH
 #undef DISPATCH_T
   return fmsmo_check_launch();
+}
+extern "C" int fmsmo_quant_act_i8_pertoken(const void* x, int x_dtype, int64_t ldx,
+                                           const void* smooth, int smooth_dtype,
+                                           int compute_dtype, int saturate, int8_t* q, int64_t ldq,
+                                           float* scale, int64_t M, int64_t K,
+                                           fmsmo_stream_t stream) {
+  return quant_act_i8_pertoken(x, x_dtype, ldx, smooth, smooth_dtype, compute_dtype, saturate, q, ldq, scale, nullptr, M, K,
+                               stream);
+}
+extern "C" int fmsmo_quant_act_i8_pertoken_clips(const void* x, int x_dtype, int64_t ldx, int compute_dtype, int saturate,
+                                                 int8_t* q, int64_t ldq, float* scale, float* clips, int64_t M, int64_t K,
+                                                 fmsmo_stream_t stream) {
+  if (!clips) return FMSMO_ERR_NULL;
+  return quant_act_i8_pertoken(x, x_dtype, ldx, nullptr, FMSMO_F32, compute_dtype, saturate, q, ldq, scale, clips, M, K,
+                               stream);
 }
 
 extern "C" int fmsmo_quant_act_i8_static(const void* x, int x_dtype, int64_t ldx, float scale,

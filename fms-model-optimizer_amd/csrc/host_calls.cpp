@@ -24,7 +24,7 @@ namespace {
 #define ENTRIES(X)                                                                                       \
   X(fmsmo_quant_act_i8_pertoken) X(fmsmo_quant_act_i8_static) X(fmsmo_quant_act_i8_static_t)             \
   X(fmsmo_quant_act_fp8_pertoken) X(fmsmo_quant_act_fp8_dynamic) X(fmsmo_quant_act_fp8_tensor)           \
-  X(fmsmo_clip_values) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
+  X(fmsmo_quant_act_i8_pertoken_clips) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
   X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_grouped_gemm_i8_dq)                   \
   X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq_ws) X(fmsmo_matmul_chunk_workspace_bytes)    \
@@ -169,6 +169,31 @@ PyObject* quant_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
               (int8_t*)q.data_ptr(), x.cols, (float*)s.data_ptr(), x.rows, x.cols, stream_of(*x.t)))
     return nullptr;
   return wrap2(q, s);
+  END_HANDLE_TH_ERRORS
+}
+// int8 codes per token without divisors, scale [M,1] and the clip values [2,M,1]
+bool codes_and_clips(const Mat& x, at::Tensor* q, at::Tensor* s, at::Tensor* c) {
+  const int dt = code_of(x.t->scalar_type());
+  *q = empty({x.rows, x.cols}, at::kChar, *x.t);
+  *s = empty({x.rows, 1}, at::kFloat, *x.t);
+  *c = empty({2, x.rows, 1}, at::kFloat, *x.t);
+  return LAUNCH(fmsmo_quant_act_i8_pertoken_clips, x.p, dt, x.ld, dt, 0, (int8_t*)q->data_ptr(), x.cols,
+                (float*)s->data_ptr(), (float*)c->data_ptr(), x.rows, x.cols, stream_of(*x.t));
+}
+// x -> (q int8 [M,K], scale fp32 [M,1], clip value [M,1], its negative)
+PyObject* quant_i8_clips(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  WANT(1);
+  const Mat x = mat(args[0]);
+  if (!x || code_of(x.t->scalar_type()) < 0 || !here(*x.t)) return none();
+  at::Tensor q, s, c;
+  if (!codes_and_clips(x, &q, &s, &c)) return nullptr;
+  PyObject* t = PyTuple_New(4);
+  PyTuple_SET_ITEM(t, 0, wrap(q));
+  PyTuple_SET_ITEM(t, 1, wrap(s));
+  PyTuple_SET_ITEM(t, 2, wrap(c.select(0, 0)));
+  PyTuple_SET_ITEM(t, 3, wrap(c.select(0, 1)));
+  return t;
   END_HANDLE_TH_ERRORS
 }
 // (x, scale, zp, sym) -> q
@@ -540,10 +565,11 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   // the epilogues round to the fp16 accumulator dtype and then to bf16 for a bf16 model
   const at::ScalarType ot = xt == at::kBFloat16 ? at::kBFloat16 : at::kHalf;
   if (xt == at::kFloat) return none();  // (the fp16 result is cast behind the product)
-  at::Tensor y = out_like(*x.t, w.rows, ot), s = empty({x.rows, 1}, at::kFloat, *x.t);
+  at::Tensor y = out_like(*x.t, w.rows, ot), s;
   const bool f32s = smooth && sm.st == at::kFloat;
   const bool one = (!smooth || sm.st == xt || f32s) &&
                    (f32s ? p_fmsmo_decode_linear_f32s_ok(x.rows, x.cols) : p_fmsmo_decode_linear_ok(x.rows, x.cols));
+  if (one || smooth) s = empty({x.rows, 1}, at::kFloat, *x.t);
   if (one) {
     // decode step of a few tokens: quantizer and weight-streaming matmul in one launch
     if (!run_decode_i8(x, sm, 0, w, *ws, b, FMSMO_EPI_REF_F16, y, s)) return nullptr;
@@ -556,19 +582,19 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
           PyList_GET_SIZE(cvs) < 2)
         return none();
     }
-    const at::ScalarType ct = smooth ? promoted(xt, sm.st) : xt;
-    at::Tensor q = empty({x.rows, x.cols}, at::kChar, *x.t);
-    if (!LAUNCH(fmsmo_quant_act_i8_pertoken, x.p, code_of(xt), x.ld, sm.p, sm.dt, code_of(ct), 0, (int8_t*)q.data_ptr(),
-                x.cols, (float*)s.data_ptr(), x.rows, x.cols, stream_of(*x.t)))
+    at::Tensor q, c;
+    if (smooth) {
+      q = empty({x.rows, x.cols}, at::kChar, *x.t);
+      if (!LAUNCH(fmsmo_quant_act_i8_pertoken, x.p, code_of(xt), x.ld, sm.p, sm.dt, code_of(promoted(xt, sm.st)), 0,
+                  (int8_t*)q.data_ptr(), x.cols, (float*)s.data_ptr(), x.rows, x.cols, stream_of(*x.t)))
+        return nullptr;
+    } else if (!codes_and_clips(x, &q, &s, &c)) {
       return nullptr;
+    }
     if (!run_gemm_i8((const char*)q.data_ptr(), x.cols, w, (const float*)s.data_ptr(), x.rows, *ws, b, FMSMO_EPI_REF_F16,
                      y, x.rows, x.cols))
       return nullptr;
     if (!smooth) {
-      // the clip values the quantizer implies, +- scale * 127
-      at::Tensor c = empty({2, x.rows, 1}, at::kFloat, *x.t);
-      if (!LAUNCH(fmsmo_clip_values, (const float*)s.data_ptr(), (float*)c.data_ptr(), x.rows, stream_of(*x.t)))
-        return nullptr;
       PyObject* cvs = item(self, k_cvs);
       PyList_SetItem(cvs, 0, wrap(c.select(0, 0)));
       PyList_SetItem(cvs, 1, wrap(c.select(0, 1)));
@@ -654,7 +680,7 @@ PyObject* entries(PyObject*, PyObject*) {
   return l;
 }
 #define FAST(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FAST(quant_i8), FAST(quant_i8_static), FAST(quant_i8_static_t), FAST(quant_fp8), FAST(gemm_dq),
+PyMethodDef methods[] = {FAST(quant_i8), FAST(quant_i8_clips), FAST(quant_i8_static), FAST(quant_i8_static_t), FAST(quant_fp8), FAST(gemm_dq),
                          FAST(decode_i8), FAST(decode_fp8), FAST(grouped_i8), FAST(chunk_dq), FAST(bmm_quantized),
                          FAST(deploy_i8), FAST(fp8_linear), FAST(bind), {"entries", entries, METH_NOARGS, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

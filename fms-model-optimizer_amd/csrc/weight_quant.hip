@@ -351,15 +351,6 @@ __global__ __launch_bounds__(256) void zero_shift_bias_kernel(
   }
 }
 
-// out[m] = scale[m] * 127, out[M + m] = -out[m]: the clip values a dynamic per-token scale stands for
-__global__ __launch_bounds__(256) void clip_values_kernel(const float* __restrict__ scale, float* __restrict__ out, int64_t M) {
-  const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (m >= M) return;
-  const float a = scale[m] * 127.0f;
-  out[m] = a;
-  out[M + m] = -a;
-}
-
 }  // namespace fmsmo
 
 using namespace fmsmo;
@@ -414,14 +405,6 @@ extern "C" int fmsmo_quant_weight_i8(const void* w, int w_dtype, int64_t ldw, co
     default: LAUNCH(FMSMO_F32); break;
   }
 #undef LAUNCH
-  return fmsmo_check_launch();
-}
-
-extern "C" int fmsmo_clip_values(const float* scale, float* out, int64_t M, fmsmo_stream_t stream) {
-  if (!scale || !out) return FMSMO_ERR_NULL;
-  if (M < 0 || M > (1ll << 38)) return FMSMO_ERR_SHAPE;
-  if (M == 0) return FMSMO_OK;
-  hipLaunchKernelGGL(clip_values_kernel, dim3((unsigned)div_up(M, 256)), dim3(256), 0, (hipStream_t)stream, scale, out, M);
   return fmsmo_check_launch();
 }
 

@@ -33,6 +33,7 @@ _P, _I, _L, _F = c_void_p, c_int, c_int64, c_float
 # name -> argument types (all functions return int except the three below)
 SIGNATURES = {
     "fmsmo_quant_act_i8_pertoken": [_P, _I, _L, _P, _I, _I, _I, _P, _L, _P, _L, _L, _P],
+    "fmsmo_quant_act_i8_pertoken_clips": [_P, _I, _L, _I, _I, _P, _L, _P, _P, _L, _L, _P],
     "fmsmo_quant_act_i8_static": [_P, _I, _L, _F, _I, _I, _P, _L, _L, _L, _P],
     "fmsmo_quant_act_i8_static_t": [_P, _I, _L, _I, _I, _F, _F, _I, _F, _F, _P, _L, _L, _L, _P],
     "fmsmo_quant_act_i8_dynamic": [_P, _I, _L, _P, _I, _I, _I, _P, _L, _P, _L, _L, _P],
@@ -72,7 +73,6 @@ SIGNATURES = {
                                  _L, _L, _P],
     "fmsmo_quant_weight_i8": [_P, _I, _L, _P, _I, _P, _I, _L, _I, _P, _L, _P, _L, _L, _P],
     "fmsmo_deploy_vectors": [_P, _P, _P, _P, _P, _L, _P, _F, _P, _I, _P, _P, _P, _P, _I, _L, _P, _P, _I, _P, _F, _P],
-    "fmsmo_clip_values": [_P, _P, _L, _P],
     "fmsmo_absmax_cols": [_P, _I, _L, _L, _L, _P, _P],
     "fmsmo_quant_i8_affine": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _L, _L, _L, _P],
     "fmsmo_quant_i8_affine_sums": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _P, _L, _L, _L, _P],

@@ -620,6 +620,11 @@ class QLinearINT8Deploy(nn.Linear):
             s = s.reshape(1, -1).to(x.dtype)
             amax = col_amax.reshape(1, -1).to(x.dtype)      # the abs-max itself, as the reference stores
         else:
+            r = None if torch.compiler.is_compiling() else L.host().quant_i8_clips(x)
+            if r is not None:   # the clip values from the quantizer's own launch
+                self._set_input_scale(r[1])
+                self.cvs[0], self.cvs[1] = r[2], r[3]
+                return r[0]
             q, s = kernels.quant_act_i8_pertoken(x, None, compute_dtype=x.dtype)
             s = s.reshape(-1, 1)
             # the per-token kernel hands over scales only: scale * 127 is the row maximum up to the

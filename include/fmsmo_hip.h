@@ -136,6 +136,13 @@ int fmsmo_quant_act_i8_pertoken(const void* x, int x_dtype, int64_t ldx, const v
                                 int smooth_dtype, int compute_dtype, int saturate, int8_t* q,
                                 int64_t ldq, float* scale, int64_t M, int64_t K,
                                 fmsmo_stream_t stream);
+/*
+ * The same without divisors, and with the clip values that the scales stand for: clips [2][M] =
+ * { scale[m] * 127, -scale[m] * 127 } (cvs[0:2] of qa_dynamic_max_qfunc).
+ */
+int fmsmo_quant_act_i8_pertoken_clips(const void* x, int x_dtype, int64_t ldx, int compute_dtype, int saturate,
+                                      int8_t* q, int64_t ldq, float* scale, float* clips, int64_t M, int64_t K,
+                                      fmsmo_stream_t stream);
 
 /*
  * Static per-tensor int8 quantizer:  q = clamp( rint( x/scale + zp - 128 + sym ), -128, 127 )
@@ -647,12 +654,6 @@ int fmsmo_quant_weight_i8(const void* w, int w_dtype, int64_t ldw, const void* s
  */
 int fmsmo_absmax_cols(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, float* out,
                       fmsmo_stream_t stream);
-
-/*
- * out[m] = scale[m] * 127 and out[M + m] = -out[m]: the clip values a dynamic per-token scale stands for
- * (cvs[0:2] of QLinearINT8Deploy, fms_mo/modules/linear.py:1085-1100).
- */
-int fmsmo_clip_values(const float* scale, float* out, int64_t M, fmsmo_stream_t stream);
 
 /*
  * The vectors of a deployed linear with dynamic activation scales, in one launch:

@@ -197,6 +197,25 @@ def test_wrappers_take_and_refuse_what_they_did(dev, general):
         assert type(here.value) is type(there.value) and str(here.value) == str(there.value), i
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Kd", [8, 4096, 40000])
+def test_clip_values_come_with_the_scales(dev, general, dtype, Kd):
+    """+- scale * 127 of every row, also of rows that take the quantizer's IEEE branch (infinite, NaN, zero)."""
+    from fms_mo_amd import _lib as L
+
+    x = torch.randn(70, Kd, device=dev).to(dtype)
+    x[3], x[5, 0], x[6, Kd - 1] = 0, float("inf"), float("nan")
+    q, s, c0, c1 = L.host().quant_i8_clips(x)
+    with general():
+        from fms_mo_amd import kernels
+
+        q2, s2 = kernels.quant_act_i8_pertoken(x)
+    rows = torch.ones(70, dtype=torch.bool)
+    rows[6] = False   # (codes of a row with a NaN are not specified)
+    assert torch.equal(q[rows], q2[rows]) and same(s.reshape(-1)[rows], s2[rows])
+    assert same(c0[rows], (s2.reshape(-1, 1) * 127)[rows]) and same(c1[rows], -(s2.reshape(-1, 1) * 127)[rows])
+
+
 def test_graph_capture_and_streams(dev):
     """The calls of a forward on a side stream, captured and replayed several times, against the eager result."""
     from fms_mo_amd.modules.linear import QLinearINT8Deploy
