@@ -8,6 +8,7 @@
 #include "quant_math.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace fmsmo {
 
@@ -180,6 +181,20 @@ __device__ __forceinline__ int sum_codes(uint2 o, int acc) {
   return __builtin_amdgcn_sdot4((int)o.y, 0x01010101, acc, false);
 }
 
+// Sum over aligned groups of 2^lg lanes, the same in each of them: within 16 lanes by DPP modifiers of the additions
+// (four rows of sums through LDS shuffles took 1.1 us of a launch of a few heads)
+__device__ __forceinline__ int group_sum(int v, int lg) {
+#define STEP(ctrl) v += __builtin_amdgcn_update_dpp(0, v, ctrl, 0xf, 0xf, true)
+  if (lg > 0) STEP(0xb1);   // quad_perm [1,0,3,2]
+  if (lg > 1) STEP(0x4e);   // quad_perm [2,3,0,1]
+  if (lg > 2) STEP(0x141);  // row_half_mirror
+  if (lg > 3) STEP(0x140);  // row_mirror
+#undef STEP
+  if (lg > 4) v += __shfl_xor(v, 16, 64);
+  if (lg > 5) v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
 template <int XT>
 __device__ __forceinline__ const void* elem_ptr(const void* x, size_t i) {
   return (const uint8_t*)x + i * (XT == FMSMO_F32 ? 4 : 2);
@@ -190,29 +205,40 @@ __device__ __forceinline__ const void* elem_ptr(const void* x, size_t i) {
 // keep four groups in flight each: of four rows where the lanes hold a whole row (ROWS), else of one row.
 // HBM bound.  (One 256-thread block per row, 16 threads of it with work, took 34 us for
 // 32 x 2048 x 128 where this takes 8.)
+struct AffineOp {
+  const void* x;
+  int64_t ldx, stride_x;  // elements
+  float scale, offset;
+  int8_t* q;
+  int64_t ldq, stride_q;
+  int32_t* sums;
+  int R, C;
+  int lg, tiles;  // row form: 2^lg lanes per row; transposing form: tiles per block
+  int gx, gy;     // blocks along the rows (row form) / tile groups, column tiles (transposing form)
+};
 template <int XT, int T, bool ROWS>
-__global__ __launch_bounds__(256) void quant_i8_affine_kernel(const void* __restrict__ x, int64_t ldx,
-                                                              int64_t stride_x, float scale, float offset,
-                                                              int8_t* __restrict__ q, int64_t ldq, int64_t stride_q,
-                                                              int32_t* __restrict__ sums, int R, int C, int lg) {
+__device__ __forceinline__ void affine_rows(const AffineOp& g, int bx, int bat) {
   constexpr int U = 4;
-  const int lanes = 1 << lg, l = threadIdx.x & (lanes - 1), rows = 256 >> lg;
-  const int row0 = (ROWS ? U : 1) * blockIdx.x * rows + (threadIdx.x >> lg);
+  const int64_t ldq = g.ldq;
+  const int R = g.R, C = g.C;
+  int32_t* const sums = g.sums;
+  const int lanes = 1 << g.lg, l = threadIdx.x & (lanes - 1), rows = 256 >> g.lg;
+  const int row0 = (ROWS ? U : 1) * bx * rows + (threadIdx.x >> g.lg);
   if (row0 >= R) return;  // whole groups of lanes
-  const AffineDiv d = affine_div<XT, T>(scale, offset);
+  const AffineDiv d = affine_div<XT, T>(g.scale, g.offset);
   const float nz = opaque_neg_zero();
-  auto xrow = [&](int r) { return (size_t)blockIdx.y * stride_x + (size_t)min(r, R - 1) * ldx; };
-  auto qrow = [&](int r) { return q + (size_t)blockIdx.y * stride_q + (size_t)r * ldq; };
+  auto xrow = [&](int r) { return (size_t)bat * g.stride_x + (size_t)min(r, R - 1) * g.ldx; };
+  auto qrow = [&](int r) { return g.q + (size_t)bat * g.stride_q + (size_t)r * ldq; };
   auto put_sum = [&](int r, int sum) {
-    for (int o = lanes >> 1; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    if (l == 0 && r < R) sums[(size_t)blockIdx.y * R + r] = sum;
+    sum = group_sum(sum, g.lg);
+    if (l == 0 && r < R) sums[(size_t)bat * R + r] = sum;
   };
   if constexpr (ROWS) {
     const int c = l * 8;
     Raw8<XT> w[U];
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      w[u] = load_raw8<XT>(elem_ptr<XT>(x, xrow(row0 + u * rows) + min(c, C - 1)), C - c);
+      w[u] = load_raw8<XT>(elem_ptr<XT>(g.x, xrow(row0 + u * rows) + min(c, C - 1)), C - c);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int r = row0 + u * rows;
@@ -227,7 +253,7 @@ __global__ __launch_bounds__(256) void quant_i8_affine_kernel(const void* __rest
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int c = c0 + u * lanes * 8;
-        w[u] = load_raw8<XT>(elem_ptr<XT>(x, xrow(row0) + min(c, C - 1)), C - c);
+        w[u] = load_raw8<XT>(elem_ptr<XT>(g.x, xrow(row0) + min(c, C - 1)), C - c);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -241,6 +267,10 @@ __global__ __launch_bounds__(256) void quant_i8_affine_kernel(const void* __rest
     }
     if (sums) put_sum(row0, sum);
   }
+}
+template <int XT, int T, bool ROWS>
+__global__ __launch_bounds__(256) void quant_i8_affine_kernel(AffineOp g) {
+  affine_rows<XT, T, ROWS>(g, blockIdx.x, blockIdx.y);
 }
 
 // The transposing form: q [batch][C][ldq], q[c][r] = code of x[r][c], rows past R zero.  A block turns
@@ -303,17 +333,16 @@ __device__ __forceinline__ uint32_t affine_codes4(const Raw4<XT>& x, int n, cons
 }
 
 template <int XT, int T>
-__global__ __launch_bounds__(256) void quant_i8_affine_t_kernel(const void* __restrict__ x, int64_t ldx,
-                                                                int64_t stride_x, float scale, float offset,
-                                                                int8_t* __restrict__ q, int64_t ldq, int64_t stride_q,
-                                                                int32_t* __restrict__ sums, int R, int C, int tiles) {
+__device__ __forceinline__ void affine_turned(const AffineOp& g, int bx, int by, int bat, int batch) {
   constexpr int LDW = 19;  // words per LDS row [c][r]
   __shared__ uint32_t tile[64 * LDW];
-  const int c0 = blockIdx.y * 64, total = (int)(ldq / 64);
-  const int t0 = blockIdx.x * tiles, t1 = min(t0 + tiles, total);
-  const size_t xb = (size_t)blockIdx.z * stride_x;
+  const int64_t ldq = g.ldq;
+  const int R = g.R, C = g.C;
+  const int c0 = by * 64, total = (int)(ldq / 64);
+  const int t0 = bx * g.tiles, t1 = min(t0 + g.tiles, total);
+  const size_t xb = (size_t)bat * g.stride_x;
   const int cl = (threadIdx.x & 15) * 4, rl = (threadIdx.x >> 4) * 4;  // this thread's 4 x 4 of a tile
-  const AffineDiv d = affine_div<XT, T>(scale, offset);
+  const AffineDiv d = affine_div<XT, T>(g.scale, g.offset);
   const float nz = opaque_neg_zero();
   const int oc = threadIdx.x >> 2, chunk = threadIdx.x & 3;
   const int nc = C - (c0 + cl);  // columns left from this thread's first one
@@ -321,7 +350,7 @@ __global__ __launch_bounds__(256) void quant_i8_affine_t_kernel(const void* __re
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = t * 64 + rl + i;
-      w[i] = load_raw4<XT>(elem_ptr<XT>(x, xb + (size_t)min(r, R - 1) * ldx + min(c0 + cl, C - 1)), nc);
+      w[i] = load_raw4<XT>(elem_ptr<XT>(g.x, xb + (size_t)min(r, R - 1) * g.ldx + min(c0 + cl, C - 1)), nc);
     }
   };
   Raw4<XT> cur[4], nxt[4];
@@ -344,17 +373,44 @@ __global__ __launch_bounds__(256) void quant_i8_affine_t_kernel(const void* __re
     const uint32_t* src = tile + oc * LDW + chunk * 4;
     const uint4 v = make_uint4(src[0], src[1], src[2], src[3]);
     if (c0 + oc < C)
-      *(uint4*)((uint8_t*)q + (size_t)blockIdx.z * stride_q + (size_t)(c0 + oc) * ldq + t * 64 + chunk * 16) = v;
+      *(uint4*)((uint8_t*)g.q + (size_t)bat * g.stride_q + (size_t)(c0 + oc) * ldq + t * 64 + chunk * 16) = v;
     sum = sum_codes(make_uint2(v.x, v.y), sum);
     sum = sum_codes(make_uint2(v.z, v.w), sum);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i) cur[i] = nxt[i];
   }
-  if (sums && t0 * 64 < R) {
+  if (g.sums && t0 * 64 < R) {
     sum += __shfl_xor(sum, 1, 64);
     sum += __shfl_xor(sum, 2, 64);
-    if (chunk == 0 && c0 + oc < C) sums[((size_t)blockIdx.x * gridDim.z + blockIdx.z) * C + c0 + oc] = sum;
+    if (chunk == 0 && c0 + oc < C) g.sums[((size_t)bx * batch + bat) * C + c0 + oc] = sum;
+  }
+}
+template <int XT, int T>
+__global__ __launch_bounds__(256) void quant_i8_affine_t_kernel(AffineOp g) {
+  affine_turned<XT, T>(g, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
+}
+
+// Both operands of a product in one launch: blocks [0, split) take the first, row by row, the others the second,
+// row by row or transposing it.  A quantizer of 17 MB takes 10 us for 5 us of traffic (one burst of loads, one
+// of stores and the launch); two of them behind each other, and for a few heads mostly two launches.
+// us, fp16: scores of 32 heads of 2048 x 2048 x 128 (both quantizers and the product) 90 -> 83, 8 heads of 155 x 155 x 80
+// 18.7 -> 12.3 (5.3 + 5.6 for the two alone).
+template <int XT, int T, bool ROWS, bool TURN>
+__global__ __launch_bounds__(256) void quant_i8_affine_pair_kernel(AffineOp a, AffineOp b, int split, int batch) {
+  int id = blockIdx.x;
+  if (id < split) {  // uniform for the whole block
+    const int bat = id / a.gx;
+    affine_rows<XT, T, ROWS>(a, id - bat * a.gx, bat);
+    return;
+  }
+  id -= split;
+  if constexpr (TURN) {
+    const int per = b.gx * b.gy, bat = id / per, r = id - bat * per, by = r / b.gx;
+    affine_turned<XT, T>(b, r - by * b.gx, by, bat, batch);
+  } else {
+    const int bat = id / b.gx;
+    affine_rows<XT, T, ROWS>(b, id - bat * b.gx, bat);
   }
 }
 
@@ -531,55 +587,106 @@ extern "C" int fmsmo_affine_add_parts(int32_t* sums, int parts, int64_t n, fmsmo
   return fmsmo_check_launch();
 }
 
+static int check_affine(int x_dtype, int compute_dtype, int transpose, const AffineOp& g) {
+  if (g.ldx < g.C || g.stride_x < 0 || g.stride_q < 0) return FMSMO_ERR_SHAPE;
+  if (x_dtype < 0 || x_dtype > 2 || compute_dtype < 0 || compute_dtype > 2) return FMSMO_ERR_UNSUPPORTED;
+  if (compute_dtype != FMSMO_F32 && compute_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
+  if (transpose) {
+    if (g.ldq < g.R || g.ldq % 64 || g.stride_q % 16 || !aligned16(g.q)) return FMSMO_ERR_ALIGN;
+    if (g.C > 65535 * 64ll || g.ldq > 0x7fffffff) return FMSMO_ERR_SHAPE;
+  } else {
+    if (g.ldq < g.C || g.ldq % 8 || g.stride_q % 8 || (((uintptr_t)g.q) & 7)) return FMSMO_ERR_ALIGN;
+    if (g.ldq > 0x7fffffff) return FMSMO_ERR_SHAPE;
+  }
+  return (((uintptr_t)g.x) & (x_dtype == FMSMO_F32 ? 3 : 1)) ? FMSMO_ERR_ALIGN : FMSMO_OK;
+}
+// how an operand is laid over blocks; true: every lane group of the row form holds a whole row
+static bool lay_affine(AffineOp& g, int transpose, int64_t batch) {
+  if (transpose) {
+    g.tiles = affine_t_tiles(batch, g.R, g.C);
+    g.gx = div_up(g.ldq / 64, g.tiles);
+    g.gy = div_up(g.C, 64);
+    return false;
+  }
+  // lanes per row: one group of eight codes each, at most a wave
+  g.lg = 0;
+  while (g.lg < 6 && ((int64_t)8 << g.lg) < g.ldq) ++g.lg;
+  const bool rows = ((int64_t)8 << g.lg) >= g.ldq;
+  g.gx = div_up(g.R, (rows ? 4 : 1) * (256 >> g.lg));
+  g.gy = 1;
+  return rows;
+}
+// f<XT, T>() for the dtypes of a call (checked)
+template <class F>
+static void affine_dtypes(int x_dtype, int compute_dtype, F&& f) {
+  typedef std::integral_constant<int, FMSMO_F16> H;
+  typedef std::integral_constant<int, FMSMO_BF16> B;
+  typedef std::integral_constant<int, FMSMO_F32> S;
+  if (compute_dtype == FMSMO_F32) {
+    if (x_dtype == FMSMO_F16) f(H{}, S{});
+    else if (x_dtype == FMSMO_BF16) f(B{}, S{});
+    else f(S{}, S{});
+  } else if (x_dtype == FMSMO_F16) {
+    f(H{}, H{});
+  } else {
+    f(B{}, B{});
+  }
+}
+
 extern "C" int fmsmo_quant_i8_affine_sums(const void* x, int x_dtype, int64_t ldx, int64_t stride_x, float scale,
                                           float offset, int compute_dtype, int transpose, int8_t* q, int64_t ldq,
                                           int64_t stride_q, int32_t* sums, int64_t batch, int64_t R, int64_t C,
                                           fmsmo_stream_t stream) {
   if (!x || !q) return FMSMO_ERR_NULL;
-  if (batch <= 0 || R <= 0 || C <= 0 || ldx < C || batch > 65535 || R > 0x7fffffff ||
-      C > 0x7fffffff || stride_x < 0 || stride_q < 0)
-    return FMSMO_ERR_SHAPE;
-  if (x_dtype < 0 || x_dtype > 2 || compute_dtype < 0 || compute_dtype > 2) return FMSMO_ERR_UNSUPPORTED;
-  if (compute_dtype != FMSMO_F32 && compute_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
-  if (transpose) {
-    if (ldq < R || ldq % 64 || stride_q % 16 || !aligned16(q)) return FMSMO_ERR_ALIGN;
-    if (C > 65535 * 64ll || ldq > 0x7fffffff) return FMSMO_ERR_SHAPE;
-  } else {
-    if (ldq < C || ldq % 8 || stride_q % 8 || (((uintptr_t)q) & 7)) return FMSMO_ERR_ALIGN;
-    if (ldq > 0x7fffffff) return FMSMO_ERR_SHAPE;
-  }
-  if (((uintptr_t)x) & (x_dtype == FMSMO_F32 ? 3 : 1)) return FMSMO_ERR_ALIGN;
+  if (batch <= 0 || R <= 0 || C <= 0 || batch > 65535 || R > 0x7fffffff || C > 0x7fffffff) return FMSMO_ERR_SHAPE;
+  AffineOp g{x, ldx, stride_x, scale, offset, q, ldq, stride_q, sums, (int)R, (int)C, 0, 0, 0, 0};
+  const int rc = check_affine(x_dtype, compute_dtype, transpose, g);
+  if (rc) return rc;
+  const bool rows = lay_affine(g, transpose, batch);
   hipStream_t st = (hipStream_t)stream;
-  const int tiles = affine_t_tiles(batch, R, C);
-  // lanes per row: one group of eight codes each, at most a wave
-  int lg = 0;
-  while (lg < 6 && ((int64_t)8 << lg) < ldq) ++lg;
-#define LAUNCH(XT, T)                                                                                      \
-  if (transpose)                                                                                           \
-    hipLaunchKernelGGL((quant_i8_affine_t_kernel<XT, T>),                                                  \
-                       dim3((unsigned)div_up(ldq / 64, tiles), (unsigned)div_up(C, 64), (unsigned)batch),  \
-                       dim3(256), 0, st, x, ldx, stride_x, scale, offset, q, ldq, stride_q, sums, (int)R,  \
-                       (int)C, tiles);                                                                     \
-  else if (((int64_t)8 << lg) >= ldq)                                                                      \
-    hipLaunchKernelGGL((quant_i8_affine_kernel<XT, T, true>),                                              \
-                       dim3((unsigned)div_up(R, 4 * (256 >> lg)), (unsigned)batch), dim3(256), 0, st, x,   \
-                       ldx, stride_x, scale, offset, q, ldq, stride_q, sums, (int)R, (int)C, lg);          \
-  else                                                                                                     \
-    hipLaunchKernelGGL((quant_i8_affine_kernel<XT, T, false>),                                             \
-                       dim3((unsigned)div_up(R, 256 >> lg), (unsigned)batch), dim3(256), 0, st, x, ldx,    \
-                       stride_x, scale, offset, q, ldq, stride_q, sums, (int)R, (int)C, lg)
-  if (compute_dtype == FMSMO_F32) {
-    switch (x_dtype) {
-      case FMSMO_F16: LAUNCH(FMSMO_F16, FMSMO_F32); break;
-      case FMSMO_BF16: LAUNCH(FMSMO_BF16, FMSMO_F32); break;
-      default: LAUNCH(FMSMO_F32, FMSMO_F32); break;
-    }
-  } else if (x_dtype == FMSMO_F16) {
-    LAUNCH(FMSMO_F16, FMSMO_F16);
-  } else {
-    LAUNCH(FMSMO_BF16, FMSMO_BF16);
-  }
-#undef LAUNCH
+  affine_dtypes(x_dtype, compute_dtype, [&](auto xt, auto t) {
+    constexpr int XT = decltype(xt)::value, T = decltype(t)::value;
+    if (transpose)
+      hipLaunchKernelGGL((quant_i8_affine_t_kernel<XT, T>), dim3((unsigned)g.gx, (unsigned)g.gy, (unsigned)batch), dim3(256),
+                         0, st, g);
+    else if (rows)
+      hipLaunchKernelGGL((quant_i8_affine_kernel<XT, T, true>), dim3((unsigned)g.gx, (unsigned)batch), dim3(256), 0, st, g);
+    else
+      hipLaunchKernelGGL((quant_i8_affine_kernel<XT, T, false>), dim3((unsigned)g.gx, (unsigned)batch), dim3(256), 0, st, g);
+  });
+  return fmsmo_check_launch();
+}
+
+extern "C" int fmsmo_quant_i8_affine_pair(int x_dtype, int compute_dtype, int64_t batch, const void* a, int64_t lda,
+                                          int64_t stride_a, float scale_a, float offset_a, int8_t* qa, int64_t stride_qa,
+                                          int64_t M, const void* b, int64_t ldb, int64_t stride_b, float scale_b,
+                                          float offset_b, int transpose_b, int8_t* qb, int64_t stride_qb, int32_t* sums_b,
+                                          int64_t N, int64_t K, int64_t ldq, fmsmo_stream_t stream) {
+  if (!a || !b || !qa || !qb) return FMSMO_ERR_NULL;
+  if (batch <= 0 || M <= 0 || N <= 0 || K <= 0 || batch > 65535 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff)
+    return FMSMO_ERR_SHAPE;
+  AffineOp ga{a, lda, stride_a, scale_a, offset_a, qa, ldq, stride_qa, nullptr, (int)M, (int)K, 0, 0, 0, 0};
+  AffineOp gb{b, ldb, stride_b, scale_b, offset_b, qb, ldq, stride_qb, sums_b, (int)(transpose_b ? K : N),
+              (int)(transpose_b ? N : K), 0, 0, 0, 0};
+  int rc = check_affine(x_dtype, compute_dtype, 0, ga);
+  if (!rc) rc = check_affine(x_dtype, compute_dtype, transpose_b, gb);
+  if (rc) return rc;
+  const bool rows = lay_affine(ga, 0, batch);  // (the second operand's rows, not transposed, have the same length)
+  lay_affine(gb, transpose_b, batch);
+  const int64_t na = ga.gx * batch, nb = (int64_t)gb.gx * gb.gy * batch;
+  if (na + nb >= (1ll << 31)) return FMSMO_ERR_UNSUPPORTED;
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((unsigned)(na + nb)), block(256);
+  affine_dtypes(x_dtype, compute_dtype, [&](auto xt, auto t) {
+    constexpr int XT = decltype(xt)::value, T = decltype(t)::value;
+#define GO(ROWS, TURN) \
+  hipLaunchKernelGGL((quant_i8_affine_pair_kernel<XT, T, ROWS, TURN>), grid, block, 0, st, ga, gb, (int)na, (int)batch)
+    if (rows && transpose_b) GO(true, true);
+    else if (rows) GO(true, false);
+    else if (transpose_b) GO(false, true);
+    else GO(false, false);
+#undef GO
+  });
   return fmsmo_check_launch();
 }
 

@@ -28,7 +28,7 @@ namespace {
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
   X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_grouped_gemm_i8_dq)                   \
   X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq_ws) X(fmsmo_matmul_chunk_workspace_bytes)    \
-  X(fmsmo_quant_i8_affine_sums) X(fmsmo_affine_sum_parts) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
+  X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
   X(fmsmo_bmm_qa_i8) X(fmsmo_bmm_i8_zp)
 #define DECLARE(f) decltype(&::f) p_##f = nullptr;
 ENTRIES(DECLARE)
@@ -439,6 +439,10 @@ bool affine(const at::Tensor& like, const void* x, int64_t ldx, int64_t stride, 
                 (int8_t*)c->q.data_ptr(), c->ld, rows * c->ld, want_sums ? (int32_t*)c->sums.data_ptr() : nullptr, B, R, C,
                 stream_of(like));
 }
+// The parts of the column sums are added up by a launch of their own, except where the product adds them: the kernel
+// for a reduction of 128, and a few query rows (us, launch of their own / inside: 1 row, 8 heads of 194 x 64 6.3 / 5.5, 32 of
+// 2048 x 128 11.3 / 10.9; 93 rows, 16 heads of 93 x 64 9.4 / 12.4)
+bool sums_added_first(int64_t M, int64_t N, int64_t K) { return M > 64 && (K != 128 || M <= 128 || N <= 128); }
 // (m1 [.., M, K], m2 [.., K, N], scale1, zero1, scale2, zero2, compute dtype) -> y [B, M, N]
 PyObject* bmm_quantized(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -464,28 +468,33 @@ PyObject* bmm_quantized(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool qa = xt != FMSMO_F32 && p_fmsmo_bmm_qa_ok(xt, ct, s1, z1, B, M, N, K);
   // scores of a head dimension up to 128 run on the kernel for a reduction of exactly 128
   const int64_t pad = K <= 128 && M > 128 && N > 128 ? 128 : 64;
-  Codes c2;
-  if (!(by_rows ? affine(*m2, m2->data_ptr(), K, N * K, s2, z2, ct, false, pad, true, B, N, K, &c2)
-                : affine(*m2, m2->data_ptr(), N, K * N, s2, z2, ct, true, pad, true, B, K, N, &c2)))
-    return nullptr;
   at::Tensor y = empty({B, M, N}, m1->scalar_type(), *m1);
-  int32_t* sums = (int32_t*)c2.sums.data_ptr();
   if (qa) {
+    Codes c2;
+    if (!(by_rows ? affine(*m2, m2->data_ptr(), K, N * K, s2, z2, ct, false, pad, true, B, N, K, &c2)
+                  : affine(*m2, m2->data_ptr(), N, K * N, s2, z2, ct, true, pad, true, B, K, N, &c2)))
+      return nullptr;
     if (!LAUNCH(fmsmo_bmm_qa_i8, m1->data_ptr(), xt, K, M * K, s1, z1, ct, (const int8_t*)c2.q.data_ptr(), c2.ld, N * c2.ld,
-                s2, sums, c2.parts, y.data_ptr(), N, B, M, N, K, stream_of(*m1)))
+                s2, (int32_t*)c2.sums.data_ptr(), c2.parts, y.data_ptr(), N, B, M, N, K, stream_of(*m1)))
       return nullptr;
     return wrap(y);
   }
-  Codes c1;
-  if (!affine(*m1, m1->data_ptr(), K, M * K, s1, z1, ct, false, pad, false, B, M, K, &c1)) return nullptr;
-  int parts = c2.parts;
-  if (parts > 1 && (c1.ld != 128 || M <= 128 || N <= 128)) {
-    // (the kernel for a reduction of 128 adds its two parts itself)
+  // both operands' codes and the second one's sums in one launch
+  const int64_t ld = (K + pad - 1) / pad * pad;
+  int parts = by_rows ? 1 : p_fmsmo_affine_sum_parts(B, K, N, 1);
+  at::Tensor q1 = empty({B, M, ld}, at::kChar, *m1), q2 = empty({B, N, ld}, at::kChar, *m1),
+             sum = empty({parts, B, N}, at::kInt, *m1);
+  int32_t* sums = (int32_t*)sum.data_ptr();
+  if (!LAUNCH(fmsmo_quant_i8_affine_pair, xt, ct, B, m1->data_ptr(), K, M * K, s1, z1, (int8_t*)q1.data_ptr(), M * ld, M,
+              m2->data_ptr(), by_rows ? K : N, N * K, s2, z2, by_rows ? 0 : 1, (int8_t*)q2.data_ptr(), N * ld, sums, N, K,
+              ld, stream_of(*m1)))
+    return nullptr;
+  if (parts > 1 && sums_added_first(M, N, ld)) {
     if (!LAUNCH(fmsmo_affine_add_parts, sums, parts, B * N, stream_of(*m1))) return nullptr;
     parts = 1;
   }
-  if (!LAUNCH(fmsmo_bmm_i8_zp, (const int8_t*)c1.q.data_ptr(), c1.ld, (const int8_t*)c2.q.data_ptr(), c1.ld, N * c2.ld,
-              product, (int)z1, sums, parts, y.data_ptr(), xt, N, B, M, N, c1.ld, stream_of(*m1)))
+  if (!LAUNCH(fmsmo_bmm_i8_zp, (const int8_t*)q1.data_ptr(), ld, (const int8_t*)q2.data_ptr(), ld, N * ld, product, (int)z1,
+              sums, parts, y.data_ptr(), xt, N, B, M, N, ld, stream_of(*m1)))
     return nullptr;
   return wrap(y);
   END_HANDLE_TH_ERRORS

@@ -76,6 +76,8 @@ SIGNATURES = {
     "fmsmo_absmax_cols": [_P, _I, _L, _L, _L, _P, _P],
     "fmsmo_quant_i8_affine": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _L, _L, _L, _P],
     "fmsmo_quant_i8_affine_sums": [_P, _I, _L, _L, _F, _F, _I, _I, _P, _L, _L, _P, _L, _L, _L, _P],
+    "fmsmo_quant_i8_affine_pair": [_I, _I, _L, _P, _L, _L, _F, _F, _P, _L, _L, _P, _L, _L, _F, _F, _I, _P, _L, _P, _L, _L, _L,
+                                   _P],
     "fmsmo_affine_add_parts": [_P, _I, _L, _P],
     "fmsmo_bmm_i8_zp": [_P, _L, _P, _L, _L, _F, _I, _P, _I, _P, _I, _L, _L, _L, _L, _L, _P],
     "fmsmo_bmm_qa_i8": [_P, _I, _L, _L, _F, _F, _I, _P, _L, _L, _F, _P, _I, _P, _L, _L, _L, _L, _L, _P],

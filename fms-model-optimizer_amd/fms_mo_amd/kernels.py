@@ -734,26 +734,43 @@ def bmm_i8_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype):
         _dt(m1), _DT[compute_dtype], scale1, zero1, B, M, N, K))
     # scores of a head dimension up to 128 run on the kernel for a reduction of exactly 128
     pad = 128 if K <= 128 and M > 128 and N > 128 else 64
-    if m2.stride(-2) == 1 and m2.shape[-2] > 1:  # a transposed view of a [n, k] tensor
-        q2, sums = quant_i8_affine(m2.transpose(-1, -2), scale2, zero2, compute_dtype, False, pad, want_sums=True)
-    else:
-        q2, sums = quant_i8_affine(m2, scale2, zero2, compute_dtype, True, pad, want_sums=True)
+    by_rows = m2.stride(-2) == 1 and m2.shape[-2] > 1  # a transposed view of a [n, k] tensor
     y = torch.empty((B, M, N), dtype=m1.dtype, device=m1.device)
-    with _dev(m1):
-        if qa:
+    if qa:
+        q2, sums = quant_i8_affine(m2.transpose(-1, -2) if by_rows else m2, scale2, zero2, compute_dtype, not by_rows, pad,
+                                   want_sums=True)
+        with _dev(m1):
             L.call("fmsmo_bmm_qa_i8", a3.data_ptr(), _dt(a3), a3.stride(1), a3.stride(0) if B > 1 else M * K,
                    float(scale1), float(zero1), _DT[compute_dtype], q2.data_ptr(), q2.stride(1), q2.stride(0),
                    float(scale2), sums.data_ptr(), sums.shape[0], y.data_ptr(), N, B, M, N, K, _stream(m1))
-        else:
-            q1 = quant_i8_affine(a3, scale1, zero1, compute_dtype, False, pad)
-            Kp, parts = q1.shape[2], sums.shape[0]
-            if parts > 1 and (Kp != 128 or M <= 128 or N <= 128):
-                # (the kernel for a reduction of 128 adds its two parts itself)
-                L.call("fmsmo_affine_add_parts", sums.data_ptr(), parts, B * N, _stream(m1))
-                parts = 1
-            L.call("fmsmo_bmm_i8_zp", q1.data_ptr(), Kp, q2.data_ptr(), Kp, q2.stride(0),
-                   _f32_product(scale1, scale2), int(zero1), sums.data_ptr(), parts, y.data_ptr(),
-                   _DT[m1.dtype], N, B, M, N, Kp, _stream(m1))
+        return y
+    if m1.dtype == m2.dtype and m2.numel() == B * K * N:
+        # both operands' codes and the second one's sums in one launch
+        b3 = _batched3(m2.transpose(-1, -2) if by_rows else m2)
+        R, C = b3.shape[1:]
+        Kp = (K + pad - 1) // pad * pad
+        parts = L.load().fmsmo_affine_sum_parts(B, R, C, int(not by_rows))
+        q1 = torch.empty((B, M, Kp), dtype=torch.int8, device=m1.device)
+        q2 = torch.empty((B, N, Kp), dtype=torch.int8, device=m1.device)
+        sums = torch.empty((parts, B, N), dtype=torch.int32, device=m1.device)
+        with _dev(m1):
+            L.call("fmsmo_quant_i8_affine_pair", _dt(a3), _DT[compute_dtype], B, a3.data_ptr(), a3.stride(1) if M > 1 else K,
+                   a3.stride(0) if B > 1 else M * K, float(scale1), float(zero1), q1.data_ptr(), M * Kp, M, b3.data_ptr(),
+                   b3.stride(1) if R > 1 else C, b3.stride(0) if B > 1 else R * C, float(scale2), float(zero2),
+                   int(not by_rows), q2.data_ptr(), N * Kp, sums.data_ptr(), N, K, Kp, _stream(m1))
+    else:
+        q2, sums = quant_i8_affine(m2.transpose(-1, -2) if by_rows else m2, scale2, zero2, compute_dtype, not by_rows, pad,
+                                   want_sums=True)
+        q1 = quant_i8_affine(a3, scale1, zero1, compute_dtype, False, pad)
+    Kp, parts = q1.shape[2], sums.shape[0]
+    with _dev(m1):
+        if parts > 1 and M > 64 and (Kp != 128 or M <= 128 or N <= 128):
+            # (a product of a few rows and the kernel for a reduction of 128 add the parts themselves)
+            L.call("fmsmo_affine_add_parts", sums.data_ptr(), parts, B * N, _stream(m1))
+            parts = 1
+        L.call("fmsmo_bmm_i8_zp", q1.data_ptr(), Kp, q2.data_ptr(), Kp, q2.stride(0),
+               _f32_product(scale1, scale2), int(zero1), sums.data_ptr(), parts, y.data_ptr(),
+               _DT[m1.dtype], N, B, M, N, Kp, _stream(m1))
     return y
 
 

@@ -720,6 +720,17 @@ int fmsmo_quant_i8_affine_sums(const void* x, int x_dtype, int64_t ldx, int64_t 
                                fmsmo_stream_t stream);
 
 /*
+ * Both operands of a product in one launch: qa [batch][M][ldq] from a [batch][M][K] and qb [batch][N][ldq] from b
+ * [batch][N][K], or with transpose_b [batch][K][N], each as fmsmo_quant_i8_affine_sums has it (sums_b: of the
+ * second one's codes, or NULL; fmsmo_affine_sum_parts(batch, K, N, 1) parts when transposing, else one).
+ */
+int fmsmo_quant_i8_affine_pair(int x_dtype, int compute_dtype, int64_t batch, const void* a, int64_t lda,
+                               int64_t stride_a, float scale_a, float offset_a, int8_t* qa, int64_t stride_qa,
+                               int64_t M, const void* b, int64_t ldb, int64_t stride_b, float scale_b,
+                               float offset_b, int transpose_b, int8_t* qb, int64_t stride_qb, int32_t* sums_b,
+                               int64_t N, int64_t K, int64_t ldq, fmsmo_stream_t stream);
+
+/*
  * y[b] = ( a[b] . b[b]^T ) * (a_scale[0] * b_scale[0]) + bias[b][n]      for b in [0, batch)
  * a: [batch * M][K] (the batches stacked, row stride lda), b: [batch][N][K] (row stride ldb, batch
  * stride stride_b), y: [batch * M][N] (row stride ldy); a_scale, b_scale: device fp32 scalars;

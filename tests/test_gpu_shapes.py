@@ -565,3 +565,28 @@ def test_small_tiles(dev, M, N, Kd, slices):
     sa, sw = torch.rand(M, generator=g, device=dev), torch.rand(N, generator=g, device=dev)
     y = kn.gemm_i8_dq(a.to(torch.int8), w.to(torch.int8), sa, sw, None, out_dtype=torch.float32, exact_ref=False)
     torch.testing.assert_close(y, ref * (sa[:, None] * sw[None, :]), rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("dtype,compute", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
+                                           (torch.float16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("M,N,Kd,pad", [(1, 1, 1, 64), (5, 63, 8, 64), (130, 129, 128, 128), (64, 200, 65, 64), (3, 70, 1030, 64),
+                                        (257, 80, 512, 64)])
+@pytest.mark.parametrize("turned", [False, True])
+def test_both_operands_of_a_product_quantized_in_one_launch(dev, dtype, compute, M, N, Kd, pad, turned):
+    """Codes and sums of the pair against the two launches it stands for, rows of a wider tensor included."""
+    from fms_mo_amd import _lib as L
+
+    kn, B = K(), 3
+    a = torch.randn(B, M, Kd + 3, generator=gen(M)).to(dtype).to(dev)[:, :, :Kd]
+    b = torch.randn(B, Kd if turned else N, (N if turned else Kd) + 5, generator=gen(N)).to(dtype).to(dev)
+    b = b[:, :, :N if turned else Kd]
+    b[0, 0, 0] = float("inf")
+    q1 = kn.quant_i8_affine(a, 0.03125, 3, compute, False, pad)
+    q2, sums = kn.quant_i8_affine(b, 0.02, -7, compute, turned, pad, want_sums=True)
+    ld = q1.shape[2]
+    p1, p2, s2 = torch.full_like(q1, 99), torch.full_like(q2, 99), torch.full_like(sums, 99)
+    L.call("fmsmo_quant_i8_affine_pair", kn._DT[dtype], kn._DT[compute], B, a.data_ptr(), a.stride(1), a.stride(0), 0.03125, 3.0,
+           p1.data_ptr(), p1.stride(0), M, b.data_ptr(), b.stride(1), b.stride(0), 0.02, -7.0, int(turned), p2.data_ptr(),
+           p2.stride(0), s2.data_ptr(), N, Kd, ld, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(p1, q1) and torch.equal(p2, q2) and torch.equal(s2, sums)
+    assert torch.equal(sums.sum(0, dtype=torch.int32), q2.sum(2, dtype=torch.int32))
