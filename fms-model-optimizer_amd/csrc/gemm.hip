@@ -203,7 +203,7 @@ extern "C" int64_t fmsmo_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t 
 extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
   if (use_decode(M, N, K)) return 0;
-  return tail_split_columns((int)M, (int)N, (int)K);
+  return tail_split_columns((int)M, (int)N, (int)K, false);
 }
 
 static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
@@ -248,7 +248,7 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
   }
   const bool rs = K % 128 == 0 && use_register_staged(MMA_I8);
   const int bm[5] = {256, 128, 128, 256, 256}, bn[5] = {256, 256, 128, 192, 128};
-  const int t = pick_tile((int)M, (int)N, rs);
+  const int t = pick_tile((int)M, (int)N, (int)K, rs, fp8);
   *kernel = (rs && (t == 0 || t >= 3)) ? FMSMO_PLAN_TILE_REGISTER_STAGED : FMSMO_PLAN_TILE_LDS_DMA;
   *tile_m = bm[t];
   *tile_n = (t == 3 && !rs) ? 256 : bn[t];

@@ -54,25 +54,26 @@ struct TileSmallK { static constexpr int BM = 64, BN = 64, BK = 128, NST = 4, WG
 
 // Which launches they take: up to one block per compute unit on reductions under 2048 (one pass takes 3.3 us + 1.6
 // per 1024 of K, less than a pass of any other tile; from there on slices of two or four come close), up to 3072
-// above 128 rows and under 8192 above 256 rows, whose partial sums cost more than they save; up to two per compute
-// unit on short ones.  (33 .. 64 tiles, and the reductions these bounds leave out, keep the plans they had, some of
+// above 128 rows, under 8192 above 256 rows, whose partial sums cost more than they save, and any length above 1024
+// rows, which take no slices; up to two per compute unit on short ones.  (33 .. 64 tiles, and the reductions these bounds leave out, keep the plans they had, some of
 // which callers and tests rely on.)  Up to 64 tokens the decode kernels re-read the activations for every 16 weight
 // rows and win until there are many of those.  us from a HIP graph, int8 | e4m3, before -> these:
 //   N = 6144, K = 1024: M = 100 10.4 -> 5.3; N = 2432, K = 2048: 200 10.4 -> 6.8, 400 9.0 -> 8.1; N = 4096, K = 3072:
 //   200 11.6 -> 8.9 | 10.7 -> 7.5; N = 1024: K = 4096, M = 800 13.5 -> 10.6, 1000 13.6 -> 10.9; K = 5120 / 6144, M = 1000
 //   16.8 / 17.9 -> 12.3 / 14.0 | 16.5 / 17.0 -> 11.0 / 13.8; N = 2048, M = 500 17.7 / 18.6 -> 12.4 / 14.5; N = 512, K = 1024:
 //   800 8.9 -> 5.1, 1500 8.3 -> 5.4, 2500 8.8 -> 6.3, 4000 8.6 -> 6.8 (504 tiles).
+//   N = 640, M = 1400: K = 8192 27.2 -> 18.4 | 28.8 -> 17.7, 14336 43.2 -> 28.5 | 46.3 -> 28.0.
 //   Up to 64 tokens: N = 12288, K = 1024: M = 17 5.1 -> 4.9 | 5.8 -> 4.6, 40 7.4 -> 5.2, 64 8.7 -> 5.1; N = 28672: 17 9.8 ->
 //   6.0, 64 15.8 -> 6.8; N = 14336, K = 4096: 17 13.4 -> 11.4, 40 18.0 -> 12.2 | 18.8 -> 11.8; N = 8192: 33 11.0 -> 10.5, 64 14.9 ->
 //   10.5; kept: N = 4096, K = 4096, 33 8.9 against 9.7; N = 8192, 32 9.6 against 10.5
 inline bool use_small_tiles(int64_t M, int64_t N, int64_t K) {
-  if (M <= 16 || K % 128 || K >= 8192) return false;
+  if (M <= 16 || K % 128 || (K >= 8192 && M <= 1024)) return false;
   const int64_t tiles = (int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN);
   if (tiles > 512) return false;
   if (fmsmo_gemv_batch_ok(M, K)) return K <= (tiles > 256 ? 2048 : 4096) && tiles >= (M > 32 ? 128 : 192);
   if (tiles > 256) return K <= 1536;
   if (tiles > 64) return K < 2048 || (M > 128 && K <= 3072) || M > 256;
-  return tiles <= 32 && K < 2048;
+  return M > 1024 || (tiles <= 32 && K < 2048);
 }
 // The decode kernels take the launch.
 inline bool use_decode(int64_t M, int64_t N, int64_t K) {
@@ -89,12 +90,16 @@ inline bool use_decode(int64_t M, int64_t N, int64_t K) {
 //   17.5; N = 1024: 1024 21.9 -> 15.6; K = 2048, N = 4096: 129 / 256 / 512 14.4 / 18.2 / 22.9 -> 9.5 /
 //   10.7 / 11.3; K = 8192: 512 36.4 -> 31.6; half a round at K = 5120 / 8192 loses (256 rows: 21.1 ->
 //   22.8, 24.5 -> 29.1) and so does K = 14336 (512 rows 48.2 -> 51.3): those keep the slices.
+// Above 1024 rows there are no slices and up to a round of these tiles beats what else would run (128 x 128 tiles on at
+// most half the compute units) at every K: us, int8 | e4m3, N = 1280, M = 1400: K = 2048 11.6 -> 9.8 | 11.9 -> 9.5, 4096
+//   17.5 -> 14.9 | 17.9 -> 14.4, 14336 46.0 -> 38.2 | 47.2 -> 35.0; N = 640, M = 2800: 11.4 -> 9.8, 17.4 -> 15.0, 45.6 -> 38.2.
 inline bool use_tall_tiles(int64_t M, int64_t N, int64_t K) {
   static const char* off = getenv("FMSMO_TALL");  // FMSMO_TALL=0 disables (tuning aid)
   if (off && off[0] == '0') return false;
-  if (M <= 16 || M > 1024 || K % 128) return false;
+  if (M <= 16 || K % 128) return false;
   const int64_t tiles = (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN);
   if (tiles > 256) return false;
+  if (M > 1024) return true;
   // three quarters of a round or more: also for a single row of tiles (batches of 17 .. 128 tokens
   // that the decode kernels do not take, through a wide projection; us, M = 33 / 64 / 128: N = 14336,
   // K = 8192 39.4 / 39.6 / 42.5 -> 32.2 / 33.8 / 38.3; N = 13824, K = 5120 26.2 / 28.1 -> 20.7 / 23.2;
@@ -112,8 +117,15 @@ inline bool use_tall_tiles(int64_t M, int64_t N, int64_t K) {
 // matmul): 0.85 of the 256x256 rate where both fill their rounds (4096 x 4096 x 4096: 73 -> 85 us),
 // but 2048 rows x 4096 columns make 256 tiles instead of 128 (us, int8 / e4m3: K = 4096 45.8 ->
 // 43.4 / 42.2 -> 38.7, K = 12800 141 -> 123 / 130 -> 114).
+// A round also costs what does not depend on K (launch, first loads, epilogue): about as much as 400 / 250 / 500 / 400 of K
+// for the four other shapes over the 128 x 128 one, whose two blocks per compute unit cover it for each other.  Short
+// reductions take that one where this puts it well ahead (12 %, e4m3 18 %: nearer than that the faster one is hard to
+// tell), up to the K where it no longer pays (int8 1280, e4m3 640; not measured below 512).  Of 412 launches of 130 .. 4096 rows
+// and 640 .. 28672 columns up to there 107 changed, by 4 % in the mean of all 412 and none more than 3.3 % slower, e4m3 61 of
+// 125, 5 %, 1.7 %.  us, int8 | e4m3, K = 512: 2000 x 2560 13.7 -> 9.8 | 11.2 -> 10.1, 4000 x 2560 22.3 -> 15.4 | 19.8 -> 16.2, 1400 x
+// 25600 51.1 -> 41.9 | 51.1 -> 40.6.
 constexpr double EFF_RS128 = 0.85;
-int pick_tile(int M, int N, bool rs192_ok) {
+int pick_tile(int M, int N, int K, bool rs192_ok, bool fp8) {
   static const char* force = getenv("FMSMO_TILE");  // tuning aid: 0 = 256x256, 1 = 128x256, 2 = 128x128, 3 = 256x192, 4 = 256x128
   if (force && force[0] >= '0' && force[0] <= '4') return (force[0] == '4' && !rs192_ok) ? 2 : force[0] - '0';
   // Fitted to measurements on the Llama / Granite shapes: relative loop efficiency of the three
@@ -121,6 +133,8 @@ int pick_tile(int M, int N, bool rs192_ok) {
   // power, hence clock, to the busy ones).
   const double eff[5] = {1.0, 0.76, 0.70, 0.92, EFF_RS128};
   const int bm[5] = {256, 128, 128, 256, 256}, bn[5] = {256, 256, 128, 192, 128};
+  const double fixed[5] = {400, 250, 0, 500, 400};
+  double scores[5];
   int best = 0;
   double best_score = -1;
   for (int t = 0; t < (rs192_ok ? 5 : 3); ++t) {
@@ -129,9 +143,12 @@ int pick_tile(int M, int N, bool rs192_ok) {
     const long rounds = (tiles + slots - 1) / slots;
     const double fill = (double)tiles / (double)(rounds * slots);
     const double pad = ((double)M * N) / ((double)div_up(M, bm[t]) * bm[t] * (double)div_up(N, bn[t]) * bn[t]);
-    const double score = eff[t] * pow(fill, 0.6) * pad;
+    const double score = scores[t] = eff[t] * pow(fill, 0.6) * pad;
     if (score > best_score) { best_score = score; best = t; }
   }
+  if (rs192_ok && K >= 512 && K <= (fp8 ? 640 : 1280) &&
+      scores[2] > (fp8 ? 1.18 : 1.12) * best_score * (1 + fixed[best] / 4096) * K / (K + fixed[best]))
+    best = 2;
   return best;
 }
 
@@ -237,7 +254,7 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
   } else if (use_tall_tiles(g.M, g.N, g.K)) {
     launch_tile<TileTallK, OP, false>(g, epi, st);
   } else if (g.K % 64 == 0 && !cut_k_tall(g.M, g.N, g.K)) {
-    switch (pick_tile(g.M, g.N, g.K % 128 == 0 && use_register_staged(OP))) {
+    switch (pick_tile(g.M, g.N, g.K, g.K % 128 == 0 && use_register_staged(OP), OP != MMA_I8)) {
       case 0:
         if (g.K % 128 == 0 && use_register_staged(OP)) launch_rs<OP>(g, epi, st);
         else launch_tile<TileBig, OP, false>(g, epi, st);
@@ -272,10 +289,10 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
 // that costs as much as the sparse round it replaces (us, whole -> cut: 2048 x 25600 x 4096, 32
 // tiles over 3 rounds, int8 263 -> 248, e4m3 224 -> 204; 4096 x 8448 x 8192, 16 tiles over 2
 // rounds, one column tile cut: 316 -> 321).  FMSMO_TAIL_SPLIT=0 switches this off (tuning aid).
-inline int tail_split_columns(int M, int N, int K) {
+inline int tail_split_columns(int M, int N, int K, bool fp8) {
   static const char* off = getenv("FMSMO_TAIL_SPLIT");
   if (off && off[0] == '0') return 0;
-  if (K % 128 || !use_register_staged(0) || pick_tile(M, N, true) != 0) return 0;
+  if (K % 128 || !use_register_staged(0) || pick_tile(M, N, K, true, fp8) != 0) return 0;
   const long gm = div_up(M, 256), gn = div_up(N, 256), tiles = gm * gn;
   if (tiles <= 256) return 0;
   const long last = tiles % 256;
@@ -290,7 +307,7 @@ int launch_dq(const GemmArgs& g, const float* a_scale, int a_stride, const float
               int w_stride, const void* bias, int bias_dtype, void* y, int y_dtype, int64_t ldy,
               hipStream_t st, bool may_split = true, int muladd = 0) {
   if (!bias) bias_dtype = FMSMO_F32;
-  const int tail = may_split ? tail_split_columns(g.M, g.N, g.K) : 0;
+  const int tail = may_split ? tail_split_columns(g.M, g.N, g.K, OP != MMA_I8) : 0;
   if (tail > 0) {
     const int64_t n0 = g.N - tail;
     GemmArgs g1 = g, g2 = g;

@@ -567,6 +567,24 @@ def test_small_tiles(dev, M, N, Kd, slices):
     torch.testing.assert_close(y, ref * (sa[:, None] * sw[None, :]), rtol=1e-6, atol=0)
 
 
+@pytest.mark.parametrize("M,N,Kd,tile", [
+    (1025, 900, 8192, (64, 64)), (1030, 70, 8320, (64, 64)),            # above 1024 rows: up to a round of 64 x 64 tiles,
+    (1300, 1279, 2176, (128, 64)), (2700, 641, 14336, (128, 64)),       # then of 128 x 64 ones, however long the reduction
+    (2000, 2559, 512, (128, 128)), (1400, 25590, 640, (128, 128))])                      # short ones
+def test_tiles_of_many_rows_and_of_short_reductions(dev, M, N, Kd, tile):
+    """Ragged edges of the tiles that such launches take: int8 exact, e4m3 exact on small integers (sums below 2^24)."""
+    kn = K()
+    assert kn.gemm_plan(M, N, Kd, with_workspace=True)[1:] == (*tile, 1)
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    a = torch.randint(-128, 128, (M, Kd), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-128, 128, (N, Kd), generator=g, dtype=torch.int8, device=dev)
+    assert torch.equal(kn.gemm_i8_i32(a, w), (a.double() @ w.double().t()).to(torch.int32))
+    a, w = a.float().div(32).round(), w.float().div(32).round()
+    one = torch.ones(1, device=dev)
+    y = kn.gemm_fp8_dq(a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn), one, one, None, out_dtype=torch.float32)
+    assert torch.equal(y, (a.double() @ w.double().t()).float())
+
+
 @pytest.mark.parametrize("dtype,compute", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
                                            (torch.float16, torch.float32), (torch.float32, torch.float32)])
 @pytest.mark.parametrize("M,N,Kd,pad", [(1, 1, 1, 64), (5, 63, 8, 64), (130, 129, 128, 128), (64, 200, 65, 64), (3, 70, 1030, 64),
