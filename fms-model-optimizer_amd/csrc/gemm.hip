@@ -247,9 +247,9 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
     return FMSMO_OK;
   }
   const bool rs = K % 128 == 0 && use_register_staged(MMA_I8);
-  const int bm[5] = {256, 128, 128, 256, 256}, bn[5] = {256, 256, 128, 192, 128};
+  const int bm[7] = {256, 128, 128, 256, 256, 128, 128}, bn[7] = {256, 256, 128, 192, 128, 192, 256};
   const int t = pick_tile((int)M, (int)N, (int)K, rs, fp8);
-  *kernel = (rs && (t == 0 || t >= 3)) ? FMSMO_PLAN_TILE_REGISTER_STAGED : FMSMO_PLAN_TILE_LDS_DMA;
+  *kernel = (rs && (t == 0 || t == 3 || t == 4)) ? FMSMO_PLAN_TILE_REGISTER_STAGED : FMSMO_PLAN_TILE_LDS_DMA;
   *tile_m = bm[t];
   *tile_n = (t == 3 && !rs) ? 256 : bn[t];
   return FMSMO_OK;

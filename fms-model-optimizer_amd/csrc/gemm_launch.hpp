@@ -47,6 +47,10 @@ struct TileMid { static constexpr int BM = 128, BN = 128, BK = 64, NST = 4, WGM 
 // three stages lose a third against five; six (tall) and five (square) change nothing.
 struct TileMidK { static constexpr int BM = 128, BN = 128, BK = 128, NST = 4, WGM = 2, WGN = 2; };
 struct TileTallK { static constexpr int BM = 128, BN = 64, BK = 128, NST = 5, WGM = 2, WGN = 2; };
+// One round of 128 x 192 or 128 x 256 tiles: eight waves (two per SIMD hide each other's LDS reads and barriers), 128-byte
+// stages, 160 / 144 KiB of LDS.  Three stages suffice the wider one; four waves take 1 ... 4 % longer.
+struct Tile192K { static constexpr int BM = 128, BN = 192, BK = 128, NST = 4, WGM = 4, WGN = 2; };
+struct TileWideK { static constexpr int BM = 128, BN = 256, BK = 128, NST = 3, WGM = 2, WGN = 4; };
 
 // 64 x 64 tiles, two blocks per compute unit, for launches that would leave most compute units idle or take
 // K slices and a second kernel.
@@ -146,9 +150,22 @@ int pick_tile(int M, int N, int K, bool rs192_ok, bool fp8) {
     const double score = scores[t] = eff[t] * pow(fill, 0.6) * pad;
     if (score > best_score) { best_score = score; best = t; }
   }
-  if (rs192_ok && K >= 512 && K <= (fp8 ? 640 : 1280) &&
-      scores[2] > (fp8 ? 1.18 : 1.12) * best_score * (1 + fixed[best] / 4096) * K / (K + fixed[best]))
-    best = 2;
+  if (!rs192_ok || K < 512) return best;
+  if (K <= (fp8 ? 640 : 1280)) {
+    if (scores[2] > (fp8 ? 1.18 : 1.12) * best_score * (1 + fixed[best] / 4096) * K / (K + fixed[best])) best = 2;
+    if (best == 2) return best;
+  }
+  // One round of the compute units instead of an emptier one of bigger tiles or two of smaller ones: 128 x 192 where 128 x 128
+  // needs more than a round, then 128 x 256, up to (not including) the full round that 256 x 128 tiles then make too.  The
+  // smaller the tile that still fits a round the shorter the round.  Of 1384 launches with more than a round of 128 x 64
+  // tiles (130 .. 4096 rows, 512 .. 28672 columns, K = 512 .. 16384) 323 changed, by 20 % in the mean, one more than 2 % slower.
+  // us, int8 | e4m3, 256 x 128 or two rounds of 128 x 128 -> these: K = 4096: 1000 x 6144 36.2 -> 29.6 | 33.8 -> 29.2, 500 x 12288
+  // 36.4 -> 29.6 | 33.9 -> 29.2, 2000 x 3072 36.2 -> 29.3 | 33.4 -> 29.2, 700 x 8192 36.1 -> 30.6 | 31.7 -> 29.8, 1500 x 4096 36.3 -> 30.7
+  // | 33.4 -> 29.5.
+  if ((long)div_up(M, 128) * div_up(N, 128) > 256) {
+    if ((long)div_up(M, Tile192K::BM) * div_up(N, Tile192K::BN) <= 256) return 5;
+    if ((long)div_up(M, TileWideK::BM) * div_up(N, TileWideK::BN) < 256) return 6;
+  }
   return best;
 }
 
@@ -264,7 +281,9 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
         if (g.K % 128 == 0 && use_register_staged(OP)) launch_rs<OP, false, 192>(g, epi, st);
         else launch_tile<TileBig, OP, false>(g, epi, st);
         break;
-      case 4: launch_rs<OP, false, 128>(g, epi, st); break;  // only offered when K % 128 == 0
+      case 4: launch_rs<OP, false, 128>(g, epi, st); break;  // 4 .. 6 only offered when K % 128 == 0
+      case 5: launch_tile<Tile192K, OP, false>(g, epi, st); break;
+      case 6: launch_tile<TileWideK, OP, false>(g, epi, st); break;
       default:
         // one round of 128 x 128 tiles: stages of 128 bytes (us, 1024 rows, N = 4096: K = 4096 29.0 ->
         // 25.6, 5120 36.8 -> 31.2; 512 rows, N = 6144, K = 4096: 28.0 -> 23.5); more than a round keeps
