@@ -47,10 +47,17 @@ struct TileMid { static constexpr int BM = 128, BN = 128, BK = 64, NST = 4, WGM 
 // three stages lose a third against five; six (tall) and five (square) change nothing.
 struct TileMidK { static constexpr int BM = 128, BN = 128, BK = 128, NST = 4, WGM = 2, WGN = 2; };
 struct TileTallK { static constexpr int BM = 128, BN = 64, BK = 128, NST = 5, WGM = 2, WGN = 2; };
-// TileMidK with eight waves instead of four, two per SIMD, where they measured faster: e4m3 and int8 under 4096 (mean of
-// 40 .. 55 launches of 100 .. 256 tiles each, against four, int8 | e4m3: K < 1024 -10 | -11 %, < 2048 -8 | -11, < 4096 -2 | -7, < 8192
-// +2 | -4, beyond +1 | -6).
-struct TileMidK8 { static constexpr int BM = 128, BN = 128, BK = 128, NST = 4, WGM = 2, WGN = 4; };
+// The two with eight waves, two per SIMD, which fill each other's waits at barriers and for fragments: e4m3 and, below this K,
+// int8, whose longer loops four waves run 1 ... 3 % faster.  us, weights in the cache | from HBM, four waves -> eight:
+//   128 x 128, e4m3: 777 x 4096 x 12800 47.9 -> 45.0 | 51.0 -> 49.2, 777 x 4096 x 4096 18.9 -> 17.0 | 20.5 -> 19.9, 1400 x 2560 x 1024 8.7 -> 7.0 |
+//   9.7 -> 9.0; int8: 1400 x 2560 x 1024 8.2 -> 7.2 | 9.6 -> 8.7, 777 x 4096 x 4096 18.4 -> 18.2 | 20.7 -> 20.2, K = 7168 32.4 -> 32.7 | 34.2 -> 34.0,
+//   12800 49.5 -> 50.0 | 51.9 -> 52.1 (2 x 4 waves instead of 4 x 2: up to 5 % behind four)
+//   128 x 64, e4m3: 100 x 13824 x 5120 17.0 -> 16.4 | 27.0 -> 24.9, 1000 x 2048 x 2048 8.5 -> 7.5 | 10.4 -> 9.8; int8: 100 x 13824 x 5120 17.3 ->
+//   16.9 | 25.1 -> 24.5, 2000 x 640 x 1024 6.6 -> 6.1 | 7.4 -> 7.0, 200 x 8192 x 6144 19.9 -> 20.1 | 22.6 -> 22.5, 1300 x 1280 x 8192 22.7 -> 23.3 |
+//   24.5 -> 25.2
+constexpr int I8_EIGHT_WAVES_BELOW = 6144;
+struct TileMidK8 { static constexpr int BM = 128, BN = 128, BK = 128, NST = 4, WGM = 4, WGN = 2; };
+struct TileTallK8 { static constexpr int BM = 128, BN = 64, BK = 128, NST = 5, WGM = 4, WGN = 2; };
 // One round of 128 x 192 or 128 x 256 tiles: eight waves (two per SIMD hide each other's LDS reads and barriers), 128-byte
 // stages, 160 / 144 KiB of LDS.  Three stages suffice the wider one; four waves take 1 ... 4 % longer.
 struct Tile192K { static constexpr int BM = 128, BN = 192, BK = 128, NST = 4, WGM = 4, WGN = 2; };
@@ -273,7 +280,8 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
   } else if (use_small_tiles(g.M, g.N, g.K)) {
     launch_tile<TileSmallK, OP, false>(g, epi, st);
   } else if (use_tall_tiles(g.M, g.N, g.K)) {
-    launch_tile<TileTallK, OP, false>(g, epi, st);
+    if (OP != MMA_I8 || g.K < I8_EIGHT_WAVES_BELOW) launch_tile<TileTallK8, OP, false>(g, epi, st);
+    else if constexpr (OP == MMA_I8) launch_tile<TileTallK, OP, false>(g, epi, st);
   } else if (g.K % 64 == 0 && !cut_k_tall(g.M, g.N, g.K)) {
     switch (pick_tile(g.M, g.N, g.K, g.K % 128 == 0 && use_register_staged(OP), OP != MMA_I8)) {
       case 0:
@@ -293,7 +301,7 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
         // 25.6, 5120 36.8 -> 31.2; 512 rows, N = 6144, K = 4096: 28.0 -> 23.5); more than a round keeps
         // the 64-byte stages, whose blocks fit two to a compute unit
         if (g.K % 128 == 0 && (long)div_up(g.M, TileMidK::BM) * div_up(g.N, TileMidK::BN) <= 256) {
-          if (OP != MMA_I8 || g.K < 4096) launch_tile<TileMidK8, OP, false>(g, epi, st);
+          if (OP != MMA_I8 || g.K < I8_EIGHT_WAVES_BELOW) launch_tile<TileMidK8, OP, false>(g, epi, st);
           else if constexpr (OP == MMA_I8) launch_tile<TileMidK, OP, false>(g, epi, st);
         } else {
           launch_tile<TileMid, OP, false>(g, epi, st);

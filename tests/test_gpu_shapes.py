@@ -572,7 +572,8 @@ def test_small_tiles(dev, M, N, Kd, slices):
     (1300, 1279, 2176, (128, 64)), (2700, 641, 14336, (128, 64)),       # then of 128 x 64 ones, however long the reduction
     (2000, 2559, 512, (128, 128)), (1400, 25590, 640, (128, 128)),                      # short ones
     (1000, 6143, 2048, (128, 192)), (385, 8193, 1408, (128, 192)), (3900, 1930, 1536, (128, 256)),  # one round, more than of
-    (1200, 2999, 3968, (128, 128)), (1200, 2999, 4096, (128, 128))])    # 128 x 128; eight waves, int8 from 4096 on four
+    (1200, 2999, 6016, (128, 128)), (1200, 2999, 6144, (128, 128)),     # 128 x 128; eight waves, int8 from 6144 on four
+    (1100, 1601, 6016, (128, 64)), (1100, 1601, 6144, (128, 64))])
 def test_tiles_of_many_rows_and_of_short_reductions(dev, M, N, Kd, tile):
     """Ragged edges of the tiles that such launches take: int8 exact, e4m3 exact on small integers (sums below 2^24)."""
     kn = K()
