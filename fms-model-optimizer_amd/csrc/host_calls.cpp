@@ -506,28 +506,34 @@ PyObject* item(PyObject* dict, PyObject* key) {  // borrowed, or null
 }
 #define NAMES(X)                                                                                                \
   X(_buffers) X(_parameters) X(weight) X(bias) X(w_scale) X(smoothq_scale) X(input_scale) X(useDynMaxQfunc)      \
-  X(use_int_kernel) X(chunk_size) X(truncate_lsb) X(use_fake_zero_shift) X(acc_dtype) X(_sq_key) X(_sq_on)       \
-  X(_ws_key) X(_ws_f32) X(iaddmm) X(cvs) X(weight_scale) X(_quantize) X(qa_dynamic_max_qfunc)
+  X(use_int_kernel) X(chunk_size) X(truncate_lsb) X(use_fake_zero_shift) X(acc_dtype) X(_sq_kept) X(_ws_kept)    \
+  X(iaddmm) X(cvs) X(weight_scale) X(_quantize) X(qa_dynamic_max_qfunc)
 #define DECLARE(n) PyObject* k_##n = nullptr;
 NAMES(DECLARE)
 #undef DECLARE
 
-// (data pointer, version, ..) as the Python side wrote it down when it read the buffer
-bool same_buffer(PyObject* key, const at::Tensor& t) {
-  if (!key || !PyTuple_Check(key) || PyTuple_GET_SIZE(key) < 2 || t.is_inference()) return false;
-  const unsigned long long p = PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(key, 0));
-  const long long v = PyLong_AsLongLong(PyTuple_GET_ITEM(key, 1));
+// What the Python side found out about buffer t, kept as ((data pointer, version, dtype), finding, alias of the
+// buffer): the finding (borrowed), or null where the buffer is another one or was written to since.  (The alias keeps
+// the memory, so the address is the buffer's own.)
+PyObject* kept_for(PyObject* kept, const at::Tensor& t) {
+  if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3 || t.is_inference()) return nullptr;
+  PyObject* stamp = PyTuple_GET_ITEM(kept, 0);
+  if (!PyTuple_Check(stamp) || PyTuple_GET_SIZE(stamp) != 3 || !THPDtype_Check(PyTuple_GET_ITEM(stamp, 2))) return nullptr;
+  const unsigned long long p = PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(stamp, 0));
+  const long long v = PyLong_AsLongLong(PyTuple_GET_ITEM(stamp, 1));
   if (PyErr_Occurred()) {
     PyErr_Clear();
-    return false;
+    return nullptr;
   }
-  return p == (unsigned long long)(uintptr_t)t.data_ptr() && v == (long long)t._version();
+  const bool same = p == (unsigned long long)(uintptr_t)t.data_ptr() && v == (long long)t._version() &&
+                    ((THPDtype*)PyTuple_GET_ITEM(stamp, 2))->scalar_type == t.scalar_type();
+  return same ? PyTuple_GET_ITEM(kept, 1) : nullptr;
 }
 
 // QLinearINT8Deploy.forward with dynamic per-token scales and a plain integer product: (instance dict, x, the
 // class's own iaddmm_int) -> y.
 // The scales' host-side facts (does SmoothQuant apply, the fp32 copy of w_scale) are those the Python side
-// keeps with the buffers' addresses and versions; where they are stale it is asked (None).
+// keeps beside the buffers; where they are stale it is asked (None).
 PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   WANT(3);
@@ -549,14 +555,9 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!dtype_arg(acc, &acct) || acct != at::kHalf || !w || w.t->scalar_type() != at::kChar || w.cols != x.cols)
     return none();
   const at::Tensor *sq = plain(osq), *wsrc = plain(ows);
-  if (!sq || !wsrc || !same_buffer(item(self, k__sq_key), *sq)) return none();
-  PyObject* wkey = item(self, k__ws_key);
-  if (!same_buffer(wkey, *wsrc) || PyTuple_GET_SIZE(wkey) != 3 || !THPDtype_Check(PyTuple_GET_ITEM(wkey, 2)) ||
-      ((THPDtype*)PyTuple_GET_ITEM(wkey, 2))->scalar_type != wsrc->scalar_type())
-    return none();
-  PyObject* own = item(self, k__ws_f32);
+  if (!sq || !wsrc) return none();
+  PyObject *on = kept_for(item(self, k__sq_kept), *sq), *own = kept_for(item(self, k__ws_kept), *wsrc);
   const at::Tensor* ws = own ? vec32(own, w.rows) : nullptr;
-  PyObject* on = item(self, k__sq_on);
   const bool smooth = on == Py_True;
   if (!ws || (!smooth && on != Py_False)) return none();
   Opt sm;

@@ -89,6 +89,22 @@ def _weight_column_max(w):
     return w.abs().max(dim=0, keepdim=True)[0]
 
 
+class _Kept(tuple):
+    """What a module has found out about small tensors of its own: (stamp, finding, aliases).  The aliases keep the
+    tensors' memory, without which a stamp could come back with other contents: a buffer that is freed and one that
+    is allocated in its place share address, type and version.  Copies and pickles of a module start without."""
+
+    def __deepcopy__(self, memo):
+        return _Kept()
+
+    def __reduce__(self):
+        return _Kept, ()
+
+
+def _stamp(t):
+    return t.data_ptr(), t._version, t.dtype
+
+
 def _plain_f32(t, n):
     return (type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == torch.float32 and t.numel() == n
             and t.is_contiguous())
@@ -571,8 +587,9 @@ class QLinearINT8Deploy(nn.Linear):
         if fmo:
             tensors += [self.quant_stepsize, self.quant_zero_point]
             tensors += [t for t in self.cvs[:2] if torch.is_tensor(t)]
-        key = (x_dtype,) + tuple((t.data_ptr(), t._version, t.dtype) for t in tensors)
-        if getattr(self, "_sp_key", None) != key:
+        stamp = (x_dtype,) + tuple(_stamp(t) for t in tensors)
+        kept = getattr(self, "_sp_kept", None)
+        if not kept or kept[0] != stamp:
             probe = torch.empty((1, 1), dtype=x_dtype)
             p = {"scale": float(self.input_scale.reshape(-1)[0]), "zp": int(self.input_zp.reshape(-1)[0]),
                  "T": torch.result_type(probe, self.input_scale.cpu())}
@@ -585,8 +602,8 @@ class QLinearINT8Deploy(nn.Linear):
                          hi=float(cv.to(clamped.dtype).reshape(-1)[0]),
                          step=float(self.quant_stepsize.reshape(-1)[0]),
                          qzp=float(self.quant_zero_point.reshape(-1)[0]))
-            self._sp_key, self._sp = key, p
-        return self._sp
+            self._sp_kept = kept = _Kept((stamp, p, [t.detach() for t in tensors]))
+        return kept[1]
 
     def qa_raw_qfunc(self, x):
         """clamp(round(x / input_scale + input_zp - 128 + sym), -128, 127) in the dtype torch
@@ -638,11 +655,12 @@ class QLinearINT8Deploy(nn.Linear):
         """One dynamic scale amax / (127 - zp) for the whole tensor, codes shifted by zp
         (linear.py:1102-1113).  The zero point is a construction-time constant."""
         zp = self.input_zp
-        key = (zp.data_ptr(), zp._version)
-        if getattr(self, "_fzs_key", None) != key:      # reading the buffer costs a host sync
-            self._fzs_key, self._fzs_zp = key, int(zp)
-        levels = 2 ** (self.nbits_a - 1) - 1 - self._fzs_zp
-        q, s, col_amax = kernels.quant_act_i8_dynamic(x, False, levels, self._fzs_zp, want_amax=True)
+        stamp = _stamp(zp)
+        kept = getattr(self, "_fzs_kept", None)
+        if not kept or kept[0] != stamp:      # reading the buffer costs a host sync
+            self._fzs_kept = kept = _Kept((stamp, int(zp), zp.detach()))
+        levels = 2 ** (self.nbits_a - 1) - 1 - kept[1]
+        q, s, col_amax = kernels.quant_act_i8_dynamic(x, False, levels, kept[1], want_amax=True)
         self.input_scale = s.reshape(()).to(x.dtype)
         amax = col_amax.max().to(x.dtype)
         self.cvs[0], self.cvs[1] = amax, -amax
@@ -792,11 +810,12 @@ class QLinearINT8Deploy(nn.Linear):
             # the answer of the last eager call (the module has to run eagerly once before it is
             # compiled, as it has to before it is captured in a graph)
             return self._sq_on
-        key = (sq.data_ptr(), sq._version)
-        if getattr(self, "_sq_key", None) != key:
-            self._sq_key = key
+        stamp = _stamp(sq)
+        kept = getattr(self, "_sq_kept", None)
+        if not kept or kept[0] != stamp:
             self._sq_on = bool(torch.all(sq != 1).item())
-        return self._sq_on
+            self._sq_kept = kept = _Kept((stamp, self._sq_on, sq.detach()))
+        return kept[1]
 
     def _w_scale_f32(self):
         """``w_scale`` as the contiguous fp32 vector the kernels read, converted once (the buffer
@@ -804,11 +823,11 @@ class QLinearINT8Deploy(nn.Linear):
         ws = self.w_scale
         if torch.compiler.is_compiling():
             return ws.float().reshape(-1)
-        key = (ws.data_ptr(), ws._version, ws.dtype)
-        if getattr(self, "_ws_key", None) != key:
-            self._ws_key = key
-            self._ws_f32 = ws.detach().float().reshape(-1).contiguous()
-        return self._ws_f32
+        stamp = _stamp(ws)
+        kept = getattr(self, "_ws_kept", None)
+        if not kept or kept[0] != stamp:
+            self._ws_kept = kept = _Kept((stamp, ws.detach().float().reshape(-1).contiguous(), ws.detach()))
+        return kept[1]
 
     def _set_input_scale(self, s):
         """Replace the ``input_scale`` buffer (the reference assigns it in every dynamic forward,
@@ -1064,14 +1083,14 @@ class QLinearCublasI8I32NT(nn.Linear):
 
     def _params(self, x_dtype):
         """Host copies of scale and zero point and the dtype torch evaluates the quantizer in."""
-        key = (x_dtype, self.input_scale.data_ptr(), self.input_scale._version, self.input_scale.dtype,
-               self.input_zp.data_ptr(), self.input_zp._version)
-        if getattr(self, "_p_key", None) != key:
+        stamp = (x_dtype, _stamp(self.input_scale), _stamp(self.input_zp))
+        kept = getattr(self, "_p_kept", None)
+        if not kept or kept[0] != stamp:
             probe = torch.empty((1, 1), dtype=x_dtype)
             T = (probe / self.input_scale.cpu() + self.input_zp.cpu()).dtype
-            self._p_key = key
-            self._p = (float(self.input_scale.reshape(-1)[0]), float(self.input_zp.reshape(-1)[0]), T)
-        return self._p
+            p = (float(self.input_scale.reshape(-1)[0]), float(self.input_zp.reshape(-1)[0]), T)
+            self._p_kept = kept = _Kept((stamp, p, (self.input_scale.detach(), self.input_zp.detach())))
+        return kept[1]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         with torch.no_grad():

@@ -238,3 +238,22 @@ def test_graph_capture_and_streams(dev):
         g.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(out, want)), i
+
+
+def test_scales_in_the_memory_of_the_ones_before(dev, general):
+    """A 16-bit weight scale and a SmoothQuant divisor dropped and allocated anew, with other values and no forward in
+    between, as a trip through host memory leaves them: the address and the version may be those of the old ones."""
+    from fms_mo_amd.modules.linear import QLinearINT8Deploy
+
+    x = torch.randn(50, 512, device=dev).half()
+    m = QLinearINT8Deploy.from_fms_mo(qlinear(512, 64, torch.float16, True, dev, True), use_dynamic_max_act_Qfunc=-1).half()
+    m(x)
+    for i, factor in enumerate((2.0, 0.5, 4.0)):
+        y0 = m(x)
+        m = m.cpu()
+        m.w_scale.mul_(factor)
+        m.smoothq_scale = m.smoothq_scale.mul(2) if i != 1 else torch.ones_like(m.smoothq_scale)
+        m = m.to(dev)
+        y = m(x)
+        with general():
+            assert same(y, m(x)) and not torch.equal(y, y0), i
