@@ -15,6 +15,7 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include "../../include/fmsmo_hip.h"
 
@@ -103,6 +104,7 @@ struct Opt {
   void* p = nullptr;
   int dt = 0;
   at::ScalarType st = at::kFloat;
+  const at::Tensor* t = nullptr;
 };
 Opt opt_vec(PyObject* o, int64_t n, int align = 1) {
   Opt r;
@@ -114,7 +116,7 @@ Opt opt_vec(PyObject* o, int64_t n, int align = 1) {
   if (!t || t->dim() != 1 || t->numel() != n || !t->is_contiguous() || code_of(t->scalar_type()) < 0 ||
       (uintptr_t)t->data_ptr() % align)
     return r;
-  return Opt{true, t->data_ptr(), code_of(t->scalar_type()), t->scalar_type()};
+  return Opt{true, t->data_ptr(), code_of(t->scalar_type()), t->scalar_type(), t};
 }
 bool dtype_arg(PyObject* o, at::ScalarType* st) {
   if (!THPDtype_Check(o)) return false;
@@ -501,6 +503,9 @@ PyObject* bmm_quantized(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // ------------------------------------------------------------------ whole forwards
+// Their operands are the module's.  A launch lets go of the interpreter lock, and another thread may then replace
+// what the module's dicts hold: these forwards own what they go on using (the arguments of a call are its caller's).
+at::Tensor owned(const at::Tensor* t) { return t ? *t : at::Tensor(); }
 PyObject* item(PyObject* dict, PyObject* key) {  // borrowed, or null
   return dict && PyDict_Check(dict) ? PyDict_GetItemWithError(dict, key) : nullptr;
 }
@@ -551,7 +556,7 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return none();
   }
   at::ScalarType acct;
-  const Mat w = mat(ow);
+  Mat w = mat(ow);
   if (!dtype_arg(acc, &acct) || acct != at::kHalf || !w || w.t->scalar_type() != at::kChar || w.cols != x.cols)
     return none();
   const at::Tensor *sq = plain(osq), *wsrc = plain(ows);
@@ -564,7 +569,7 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (smooth) {
     const at::ScalarType st = sq->scalar_type();
     if (sq->numel() != x.cols || !sq->is_contiguous() || code_of(st) < 0 || (uintptr_t)sq->data_ptr() % 16) return none();
-    sm = Opt{true, sq->data_ptr(), code_of(st), st};
+    sm = Opt{true, sq->data_ptr(), code_of(st), st, sq};
   }
   PyObject* ob = item(buffers, k_bias);
   if (!ob) ob = item(params, k_bias);
@@ -575,6 +580,10 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   // the epilogues round to the fp16 accumulator dtype and then to bf16 for a bf16 model
   const at::ScalarType ot = xt == at::kBFloat16 ? at::kBFloat16 : at::kHalf;
   if (xt == at::kFloat) return none();  // (the fp16 result is cast behind the product)
+  const at::Tensor own_w = *w.t, own_ws = *ws, own_sm = owned(sm.t), own_b = owned(b.t);
+  const THPObjectPtr own_buffers(Py_NewRef(buffers));
+  w.t = &own_w;
+  ws = &own_ws;
   at::Tensor y = out_like(*x.t, w.rows, ot), s;
   const bool f32s = smooth && sm.st == at::kFloat;
   const bool one = (!smooth || sm.st == xt || f32s) &&
@@ -604,8 +613,8 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!run_gemm_i8((const char*)q.data_ptr(), x.cols, w, (const float*)s.data_ptr(), x.rows, *ws, b, FMSMO_EPI_REF_F16,
                      y, x.rows, x.cols))
       return nullptr;
-    if (!smooth) {
-      PyObject* cvs = item(self, k_cvs);
+    PyObject* cvs = smooth ? nullptr : item(self, k_cvs);
+    if (cvs && PyList_CheckExact(cvs) && PyList_GET_SIZE(cvs) >= 2) {
       PyList_SetItem(cvs, 0, wrap(c.select(0, 0)));
       PyList_SetItem(cvs, 1, wrap(c.select(0, 1)));
     }
@@ -624,7 +633,7 @@ PyObject* fp8_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Mat x = rows_of(args[2]);
   PyObject *ow = item(args[0], k_weight), *ows = item(args[0], k_weight_scale);
   if (!x || x.rows == 0 || code_of(x.t->scalar_type()) < 0 || !ow || !ows) return none();
-  const Mat w = mat(ow);
+  Mat w = mat(ow);
   const at::Tensor* ws = plain(ows);
   if (!w || w.t->scalar_type() != at::kFloat8_e4m3fn || w.cols != x.cols || !ws || ws->scalar_type() != at::kFloat ||
       !ws->is_contiguous() || (ws->numel() != 1 && ws->numel() != w.rows))
@@ -641,6 +650,9 @@ PyObject* fp8_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   NUMBERS_OK;
   if (!b.ok || !here(*x.t) || w.t->get_device() != x.t->get_device() || (per_tensor && !fp8_tensor_ok(x))) return none();
   const at::ScalarType xt = x.t->scalar_type();
+  const at::Tensor own_w = *w.t, own_ws = *ws, own_b = owned(b.t);
+  w.t = &own_w;
+  ws = &own_ws;
   const float* wp = (const float*)ws->data_ptr();
   at::Tensor y = out_like(*x.t, w.rows, xt);
   if (!per_tensor && floor == 1e-12 && !in_x && xt != at::kFloat && p_fmsmo_decode_linear_ok(x.rows, x.cols)) {

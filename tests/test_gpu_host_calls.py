@@ -257,3 +257,45 @@ def test_scales_in_the_memory_of_the_ones_before(dev, general):
         y = m(x)
         with general():
             assert same(y, m(x)) and not torch.equal(y, y0), i
+
+
+@pytest.mark.parametrize("kind", ["smooth", "plain", "e4m3"])
+def test_operands_replaced_while_a_launch_runs(dev, kind):
+    """Another thread may replace a module's tensors between the two launches of its forward: here the quantizer's entry
+    point does so itself, drops them and writes over memory of their sizes.  The forward ends with those it began with."""
+    import ctypes
+
+    from fms_mo_amd import _lib as L
+    from fms_mo_amd.modules.fp8_linear import FP8Linear
+    from fms_mo_amd.modules.linear import QLinearINT8Deploy
+
+    x = torch.randn(50, 512, device=dev).half()
+    if kind == "e4m3":
+        m = FP8Linear.from_float(0.02 * torch.randn(128, 512, device=dev), torch.randn(128, device=dev).half(), per_channel=True)
+        name = "fmsmo_quant_act_fp8_pertoken"
+    else:
+        m = QLinearINT8Deploy.from_fms_mo(qlinear(512, 128, torch.float16, True, dev, kind == "smooth"),
+                                          use_dynamic_max_act_Qfunc=-1).half()
+        name = "fmsmo_quant_act_i8_pertoken" + ("" if kind == "smooth" else "_clips")
+    want, host, lib, seen, junk = m(x), L.host(), L.load(), [], []
+    addresses = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in host.entries()}
+
+    def replace(*args):
+        rc = getattr(lib, name)(*args)
+        for held in (m._parameters, m._buffers):
+            for n in [n for n, t in held.items() if t is not None and t.dim() > 0]:
+                sizes, dtype = held[n].shape, held[n].dtype
+                held[n] = None
+                junk.extend(torch.full(sizes, 3.0, device=dev).to(dtype) for _ in range(2))
+        m.__dict__.pop("_ws_kept", None), m.__dict__.pop("_sq_kept", None)
+        junk.extend(torch.full((128,), 7.0, device=dev) for _ in range(2))
+        seen.append(rc)
+        return rc
+
+    call = ctypes.CFUNCTYPE(ctypes.c_int, *L.SIGNATURES[name])(replace)
+    host.bind({**addresses, name: ctypes.cast(call, ctypes.c_void_p).value}, L.raise_status)
+    try:
+        y = m(x)
+    finally:
+        host.bind(addresses, L.raise_status)
+    assert seen == [0] and same(y, want)
