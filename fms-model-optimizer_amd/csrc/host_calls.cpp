@@ -123,9 +123,12 @@ bool dtype_arg(PyObject* o, at::ScalarType* st) {
   *st = ((THPDtype*)o)->scalar_type;
   return code_of(*st) >= 0;
 }
-// the call can be made here: tensors on the current device, no mode that wants to see the allocations
-bool here(const at::Tensor& t) {
-  return !c10::impl::TorchDispatchModeTLS::any_modes_set() && c10::hip::current_device() == t.get_device();
+// the call can be made here: every tensor of it (null: an operand left out) on the current device -- a scale on another
+// one is the general path's to move -- and no mode that wants to see the allocations
+template <class... T>
+bool here(const T*... t) {
+  const auto d = c10::hip::current_device();
+  return !c10::impl::TorchDispatchModeTLS::any_modes_set() && ((!t || t->get_device() == d) && ...);
 }
 void* stream_of(const at::Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 at::Tensor empty(at::IntArrayRef sizes, at::ScalarType st, const at::Tensor& like) {
@@ -162,7 +165,7 @@ PyObject* quant_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Mat x = mat(args[0]);
   if (!x || code_of(x.t->scalar_type()) < 0) return none();
   const Opt sm = opt_vec(args[1], x.cols, 16);
-  if (!sm.ok || !here(*x.t)) return none();
+  if (!sm.ok || !here(x.t, sm.t)) return none();
   at::ScalarType ct = sm.p ? promoted(x.t->scalar_type(), sm.st) : x.t->scalar_type();
   if (args[2] != Py_None && !dtype_arg(args[2], &ct)) return none();
   const int sat = PyObject_IsTrue(args[3]);
@@ -187,7 +190,7 @@ PyObject* quant_i8_clips(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   WANT(1);
   const Mat x = mat(args[0]);
-  if (!x || code_of(x.t->scalar_type()) < 0 || !here(*x.t)) return none();
+  if (!x || code_of(x.t->scalar_type()) < 0 || !here(x.t)) return none();
   at::Tensor q, s, c;
   if (!codes_and_clips(x, &q, &s, &c)) return nullptr;
   PyObject* t = PyTuple_New(4);
@@ -203,7 +206,7 @@ PyObject* quant_i8_static(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   WANT(4);
   const Mat x = mat(args[0]);
-  if (!x || code_of(x.t->scalar_type()) < 0 || !here(*x.t)) return none();
+  if (!x || code_of(x.t->scalar_type()) < 0 || !here(x.t)) return none();
   const float scale = (float)REAL(1);
   const int zp = (int)WHOLE(2), sym = (int)WHOLE(3);
   NUMBERS_OK;
@@ -220,7 +223,7 @@ PyObject* quant_i8_static_t(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   WANT(8);
   const Mat x = mat(args[0]);
   at::ScalarType ct;
-  if (!x || code_of(x.t->scalar_type()) < 0 || !dtype_arg(args[2], &ct) || !here(*x.t)) return none();
+  if (!x || code_of(x.t->scalar_type()) < 0 || !dtype_arg(args[2], &ct) || !here(x.t)) return none();
   const int mode = (int)WHOLE(1), sym = (int)WHOLE(5);
   const float scale = (float)REAL(3), zp = (float)REAL(4), lo = (float)REAL(6), hi = (float)REAL(7);
   NUMBERS_OK;
@@ -257,7 +260,7 @@ PyObject* quant_fp8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   WANT(5);
   const Mat x = mat(args[0]);
-  if (!x || code_of(x.t->scalar_type()) < 0 || !here(*x.t)) return none();
+  if (!x || code_of(x.t->scalar_type()) < 0 || !here(x.t)) return none();
   const int variant = (int)WHOLE(1);
   const bool per_tensor = PyObject_IsTrue(args[2]) == 1, in_x = PyObject_IsTrue(args[4]) == 1;
   const double floor = REAL(3);
@@ -297,7 +300,7 @@ PyObject* gemm_dq(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!i8 && a.t->scalar_type() != at::kFloat8_e4m3fn) return none();
   const at::Tensor *as = vec32(args[2], a.rows), *ws = vec32(args[3], w.rows);
   const Opt b = opt_vec(args[4], w.rows);
-  if (!as || !ws || !b.ok || !here(*a.t)) return none();
+  if (!as || !ws || !b.ok || !here(a.t, w.t, as, ws, b.t)) return none();
   const int epi = (int)WHOLE(6);
   NUMBERS_OK;
   at::Tensor y = empty({a.rows, w.rows}, ot, *a.t);
@@ -324,7 +327,7 @@ PyObject* decode_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return none();
   const at::Tensor* ws = vec32(args[2], w.rows);
   const Opt b = opt_vec(args[3], w.rows), sm = opt_vec(args[4], x.cols, 16);
-  if (!ws || !b.ok || !sm.ok || !here(*x.t)) return none();
+  if (!ws || !b.ok || !sm.ok || !here(x.t, w.t, ws, b.t, sm.t)) return none();
   const int epi = (int)WHOLE(6), sat = PyObject_IsTrue(args[7]);
   NUMBERS_OK;
   at::Tensor y = empty({x.rows, w.rows}, ot, *x.t), s = empty({x.rows}, at::kFloat, *x.t);
@@ -343,7 +346,7 @@ PyObject* decode_fp8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return none();
   const at::Tensor* ws = vec32(args[2], w.rows);
   const Opt b = opt_vec(args[3], w.rows);
-  if (!ws || !b.ok || !here(*x.t)) return none();
+  if (!ws || !b.ok || !here(x.t, w.t, ws, b.t)) return none();
   at::Tensor y = empty({x.rows, w.rows}, ot, *x.t), s = empty({x.rows}, at::kFloat, *x.t);
   if (!LAUNCH(fmsmo_decode_linear_fp8, x.p, code_of(x.t->scalar_type()), x.ld, (const uint8_t*)w.p, w.ld,
               (const float*)ws->data_ptr(), ws->numel(), b.p, b.dt, y.data_ptr(), code_of(ot), w.rows,
@@ -372,9 +375,9 @@ PyObject* grouped_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!b.ok) {
     const at::Tensor* t = plain(args[5]);
     if (!t || !t->is_contiguous() || t->numel() != E * N || code_of(t->scalar_type()) < 0) return none();
-    b = Opt{true, t->data_ptr(), code_of(t->scalar_type()), t->scalar_type()};
+    b = Opt{true, t->data_ptr(), code_of(t->scalar_type()), t->scalar_type(), t};
   }
-  if (!here(*a.t)) return none();
+  if (!here(a.t, w, off, as, ws, b.t)) return none();
   const int epi = (int)WHOLE(7);
   NUMBERS_OK;
   at::Tensor y = empty({a.rows, N}, ot, *a.t);
@@ -400,7 +403,7 @@ PyObject* chunk_dq(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t per16 = 16 / (int64_t)a.t->element_size(), M = a.rows, N = w.rows, K = a.cols;
   const at::Tensor *as = vec32(args[2], M), *ws = vec32(args[3], N);
   const Opt b = opt_vec(args[4], N);
-  if (K % per16 || a.ld % per16 || w.ld % per16 || !as || !ws || !b.ok || !here(*a.t)) return none();
+  if (K % per16 || a.ld % per16 || w.ld % per16 || !as || !ws || !b.ok || !here(a.t, w.t, as, ws, b.t)) return none();
   const int epi = (int)WHOLE(5), chunk = (int)WHOLE(7), trun = (int)WHOLE(8), bits = (int)WHOLE(9);
   NUMBERS_OK;
   const int tta = PyObject_IsTrue(args[10]) == 1, dl16 = PyObject_IsTrue(args[11]) == 1;
@@ -461,7 +464,7 @@ PyObject* bmm_quantized(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   // m2 as it lies in memory: [.., K, N], or the transposed view of [.., N, K]
   const bool by_rows = m2->stride(d - 2) == 1 && K > 1;
   if (by_rows ? !m2->transpose(d - 2, d - 1).is_contiguous() : !m2->is_contiguous()) return none();
-  if (!here(*m1) || m2->get_device() != m1->get_device()) return none();
+  if (!here(m1, m2)) return none();
   const float s1 = (float)REAL(2), z1 = (float)REAL(3), s2 = (float)REAL(4), z2 = (float)REAL(5);
   const float product = (float)(REAL(2) * REAL(4));
   NUMBERS_OK;
@@ -576,7 +579,7 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!ob) return none();
   const Opt b = opt_vec(ob, w.rows);
   const at::ScalarType xt = x.t->scalar_type();
-  if (!b.ok || !here(*x.t) || w.t->get_device() != x.t->get_device() || x.t->dim() == 0) return none();
+  if (!b.ok || !here(x.t, w.t, ws, sm.t, b.t)) return none();
   // the epilogues round to the fp16 accumulator dtype and then to bf16 for a bf16 model
   const at::ScalarType ot = xt == at::kBFloat16 ? at::kBFloat16 : at::kHalf;
   if (xt == at::kFloat) return none();  // (the fp16 result is cast behind the product)
@@ -648,7 +651,7 @@ PyObject* fp8_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool per_tensor = PyObject_IsTrue(args[3]) == 1, in_x = PyObject_IsTrue(args[5]) == 1;
   const double floor = REAL(4);
   NUMBERS_OK;
-  if (!b.ok || !here(*x.t) || w.t->get_device() != x.t->get_device() || (per_tensor && !fp8_tensor_ok(x))) return none();
+  if (!b.ok || !here(x.t, w.t, ws, b.t) || (per_tensor && !fp8_tensor_ok(x))) return none();
   const at::ScalarType xt = x.t->scalar_type();
   const at::Tensor own_w = *w.t, own_ws = *ws, own_b = owned(b.t);
   w.t = &own_w;

@@ -252,7 +252,7 @@ def test_scales_in_the_memory_of_the_ones_before(dev, general):
         y0 = m(x)
         m = m.cpu()
         m.w_scale.mul_(factor)
-        m.smoothq_scale = m.smoothq_scale.mul(2) if i != 1 else torch.ones_like(m.smoothq_scale)
+        m.smoothq_scale = m.smoothq_scale.mul(3) if i != 1 else torch.ones_like(m.smoothq_scale)
         m = m.to(dev)
         y = m(x)
         with general():
@@ -299,3 +299,52 @@ def test_operands_replaced_while_a_launch_runs(dev, kind):
     finally:
         host.bind(addresses, L.raise_status)
     assert seen == [0] and same(y, want)
+
+
+def on_another_gpu(t):
+    """A tensor that says it lies on the next GPU (its memory is that of `t`: it is for checks, not for launches)."""
+    import ctypes
+
+    class Exchange(ctypes.Structure):   # DLManagedTensor
+        _fields_ = [("data", ctypes.c_void_p), ("device_type", ctypes.c_int32), ("device", ctypes.c_int32), ("ndim", ctypes.c_int32),
+                    ("code", ctypes.c_uint8), ("bits", ctypes.c_uint8), ("lanes", ctypes.c_uint16), ("shape", ctypes.c_void_p),
+                    ("strides", ctypes.c_void_p), ("offset", ctypes.c_uint64), ("context", ctypes.c_void_p), ("deleter", ctypes.c_void_p)]
+
+    raw = t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t
+    sizes = (ctypes.c_int64 * t.dim())(*t.shape)
+    steps = (ctypes.c_int64 * t.dim())(*t.stride())
+    code = 0 if raw.dtype in (torch.int8, torch.int32) else 1 if raw.dtype == torch.uint8 else 4 if raw.dtype == torch.bfloat16 else 2
+    x = Exchange(t.data_ptr(), 10, t.get_device() + 1, t.dim(), code, 8 * t.element_size(), 1, ctypes.addressof(sizes),
+                 ctypes.addressof(steps), 0, None, None)
+    new = ctypes.pythonapi.PyCapsule_New
+    new.restype, new.argtypes = ctypes.py_object, [ctypes.c_void_p, ctypes.c_char_p, ctypes.c_void_p]
+    out = torch.utils.dlpack.from_dlpack(new(ctypes.addressof(x), b"dltensor", None)).view(t.dtype)
+    out._keep = (t, x, sizes, steps)
+    assert out.get_device() == t.get_device() + 1 and out.shape == t.shape
+    return out
+
+
+def test_native_calls_leave_tensors_of_another_gpu_to_the_general_path(dev):
+    from fms_mo_amd import _lib as L
+
+    h, half = L.host(), torch.float16
+    x, xb = torch.randn(4, 128, device=dev).half(), torch.randn(1, 2, 8, 64, device=dev).half()
+    q, w = torch.ones(4, 128, device=dev, dtype=torch.int8), torch.ones(32, 128, device=dev, dtype=torch.int8)
+    qf, wf = q.half().to(torch.float8_e4m3fn), w.half().to(torch.float8_e4m3fn)
+    s, ws, b, sm = torch.ones(4, device=dev), torch.ones(32, device=dev), torch.ones(32, device=dev).half(), torch.ones(128, device=dev).half()
+    off, w3 = torch.tensor([0, 4], device=dev, dtype=torch.int32), w[None].contiguous()
+    calls = [(h.quant_i8, x, sm, None, False), (h.quant_i8_clips, x), (h.quant_i8_static, x, 0.1, 3, 0),
+             (h.quant_i8_static_t, x, L.SQ_RAW, half, 0.1, 3, 1, 0.0, 0.0), (h.quant_fp8, x, L.FP8_LINEAR, False, 1e-12, False),
+             (h.gemm_dq, q, w, s, ws, b, half, L.EPI_F32), (h.gemm_dq, qf, wf, s, ws, b, half, 0),
+             (h.decode_i8, x, w, ws, b, sm, half, L.EPI_F32, False), (h.decode_fp8, x, wf, ws, b, half),
+             (h.grouped_i8, q, w3, off, s, ws[None], b[None], half, L.EPI_F32),
+             (h.chunk_dq, q, w, s, ws, b, L.EPI_SEQ_OUT, half, 64, 4, 32, True, False),
+             (h.bmm_quantized, xb, xb.transpose(-1, -2), 0.1, 0, 0.1, 0, half),
+             (h.fp8_linear, {"weight": wf, "weight_scale": ws, "bias": b}, True, x, False, 1e-12, False)]
+    for f, *args in calls:
+        for i, a in enumerate(args):
+            if torch.is_tensor(a):
+                assert f(*args[:i], on_another_gpu(a), *args[i + 1:]) is None, (f.__name__, i)
+            elif isinstance(a, dict):
+                for k in a:
+                    assert f(*args[:i], {**a, k: on_another_gpu(a[k])}, *args[i + 1:]) is None, (f.__name__, k)
