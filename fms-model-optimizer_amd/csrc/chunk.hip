@@ -4,7 +4,9 @@
 // multiplied into a FRESH MFMA accumulator (the C operand is the inline constant 0 for the
 // first MFMA of the chunk), the chunk result is range-clamped / LSB-rounded on the vector ALU,
 // and only then added to the running accumulator -- the same order of operations as the
-// reference's Triton kernels, whose BLOCK_SIZE_K equals the chunk size.
+// reference's Triton kernels, whose BLOCK_SIZE_K equals the chunk size.  A caller who passes a workspace lets
+// reductions be cut into slices of whole chunks whose sums are added behind (plan_chunk): the same int32 sums, but
+// another grouping of fp32 ones, whose last bits then depend on the tile a row falls into.
 //
 // Two kernels.  Operands within 2^31 bytes each: the pipelined tile kernel of chunk_tile.hpp.
 // Larger ones: the simple kernel below, which addresses its rows with 64 bits.

@@ -231,8 +231,9 @@ struct ChunkTileArgs {
   int64_t ldc;
   // Tiles [0, full) of the tile sequence are whole; of the others every block takes one of `slices` pieces of
   // the reduction of slice_len bytes (whole chunks; the last one shorter) and leaves its accumulators in `ws`
-  // for chunk_reduce_kernel.  Rounded chunks are added, so slices of whole chunks may be added in any grouping
-  // (int32 exactly; not with a running accumulator that is itself rounded, nor with c_in).
+  // for chunk_reduce_kernel.  Rounded chunks are added, so slices of whole chunks give the same int32 sums and fp32
+  // ones in another grouping, which is the caller's choice (a workspace or none).  Not with a running accumulator
+  // that is itself rounded, nor with c_in.
   int full, slices, slice_len;
   void* ws;
 };

@@ -28,7 +28,7 @@ namespace {
   X(fmsmo_quant_act_i8_pertoken_clips) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
   X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_grouped_gemm_i8_dq)                   \
-  X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq_ws) X(fmsmo_matmul_chunk_workspace_bytes)    \
+  X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq) X(fmsmo_matmul_chunk_workspace_bytes)    \
   X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
   X(fmsmo_bmm_qa_i8) X(fmsmo_bmm_i8_zp)
 #define DECLARE(f) decltype(&::f) p_##f = nullptr;
@@ -408,7 +408,9 @@ PyObject* chunk_dq(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   NUMBERS_OK;
   const int tta = PyObject_IsTrue(args[10]) == 1, dl16 = PyObject_IsTrue(args[11]) == 1;
   at::Tensor y = empty({M, N}, ot, *a.t);
-  const at::Tensor scratch = workspace(p_fmsmo_matmul_chunk_workspace_bytes(op, M, N, K, chunk, tta), *a.t);
+  // (in floating point no workspace: the rounded chunks are to be added one after the other, see matmul_chunk)
+  const at::Tensor scratch =
+      workspace(op == FMSMO_OP_I8 ? p_fmsmo_matmul_chunk_workspace_bytes(op, M, N, K, chunk, tta) : 0, *a.t);
   void* wp = scratch.defined() ? scratch.data_ptr() : nullptr;
   const int64_t wb = scratch.defined() ? scratch.numel() : 0;
   const float *ap = (const float*)as->data_ptr(), *sp = (const float*)ws->data_ptr();
@@ -418,8 +420,8 @@ PyObject* chunk_dq(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
           ? LAUNCH(fmsmo_matmul_chunk_i8_dq_ws, (const int8_t*)a.p, a.ld, (const int8_t*)w.p, w.ld, ap, as->numel(), sp,
                    ws->numel(), b.p, bdt, epi, y.data_ptr(), code_of(ot), N, M, N, K, chunk, trun, bits, tta, wp, wb,
                    stream_of(*a.t))
-          : LAUNCH(fmsmo_matmul_chunk_fp_dq_ws, a.p, a.ld, w.p, w.ld, op, ap, as->numel(), sp, ws->numel(), b.p, bdt, epi,
-                   y.data_ptr(), code_of(ot), N, M, N, K, chunk, trun, dl16, tta, wp, wb, stream_of(*a.t));
+          : LAUNCH(fmsmo_matmul_chunk_fp_dq, a.p, a.ld, w.p, w.ld, op, ap, as->numel(), sp, ws->numel(), b.p, bdt, epi,
+                   y.data_ptr(), code_of(ot), N, M, N, K, chunk, trun, dl16, tta, stream_of(*a.t));
   return ok ? wrap(y) : nullptr;
   END_HANDLE_TH_ERRORS
 }

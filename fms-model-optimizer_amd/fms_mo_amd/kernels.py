@@ -459,7 +459,7 @@ def grouped_gemm_i8_dq(a, w, offsets, a_scale, w_scale, bias=None, out_dtype=tor
 
 # ----------------------------------------------------------------------- chunked accumulation
 def _chunk_workspace(a, N, chunk_size, tta):
-    """(pointer, bytes, the tensor itself) of the scratch in which the slices of a cut reduction are added."""
+    """(pointer, bytes, the tensor itself) of the scratch in which the slices of a cut int8 reduction are added."""
     M, K = a.shape
     nbytes = L.load().fmsmo_matmul_chunk_workspace_bytes(_OPDT[a.dtype], M, N, K, int(chunk_size), int(bool(tta)))
     if nbytes == 0:
@@ -470,7 +470,9 @@ def _chunk_workspace(a, N, chunk_size, tta):
 
 def matmul_chunk(a, w, c=None, chunk_size=64, chunk_trun_bits=0, max_acc_bits=32,
                  truncate_then_accumulate=True, clamp_acc_to_dl16=False):
-    """a [M,K], w [N,K] (int8 | float8_e4m3fn | float16 | bfloat16 | float32) -> int32 / fp32 [M,N]."""
+    """a [M,K], w [N,K] (int8 | float8_e4m3fn | float16 | bfloat16 | float32) -> int32 / fp32 [M,N].  Floating-point
+    accumulators add the rounded chunks one after the other, so a row's result does not depend on the rows beside it
+    (an int32 accumulator adds them in any grouping: the entry points cut its reduction where there is a workspace)."""
     _need_gpu(a, w, c)
     if a.dtype != w.dtype or a.dtype not in _OPDT:
         raise TypeError(f"unsupported operand dtypes {a.dtype}, {w.dtype}")
@@ -492,17 +494,17 @@ def matmul_chunk(a, w, c=None, chunk_size=64, chunk_trun_bits=0, max_acc_bits=32
         if c.shape != (M, N):
             raise ValueError("C shape is inconsistent with A B.")
         c = c.to(acc_dtype).contiguous()
-    wptr, wbytes, _ws = _chunk_workspace(a, N, chunk_size, truncate_then_accumulate and c is None)
     with _dev(a):
         if a.dtype == torch.int8:
+            wptr, wbytes, _ws = _chunk_workspace(a, N, chunk_size, truncate_then_accumulate and c is None)
             L.call("fmsmo_matmul_chunk_i8_ws", a.data_ptr(), _ld(a), w.data_ptr(), _ld(w), _ptr(c),
                    d.data_ptr(), N, M, N, K, int(chunk_size), int(chunk_trun_bits),
                    int(max_acc_bits), int(bool(truncate_then_accumulate)), wptr, wbytes, _stream(a))
         else:
-            L.call("fmsmo_matmul_chunk_fp_ws", a.data_ptr(), _ld(a), w.data_ptr(), _ld(w),
+            L.call("fmsmo_matmul_chunk_fp", a.data_ptr(), _ld(a), w.data_ptr(), _ld(w),
                    _OPDT[a.dtype], _ptr(c), d.data_ptr(), N, M, N, K, int(chunk_size),
                    int(chunk_trun_bits), int(bool(clamp_acc_to_dl16)),
-                   int(bool(truncate_then_accumulate)), wptr, wbytes, _stream(a))
+                   int(bool(truncate_then_accumulate)), _stream(a))
     return d
 
 
@@ -542,14 +544,14 @@ def matmul_chunk_dq(a, w, a_scale, w_scale, bias=None, epilogue=L.EPI_SEQ_OUT, o
     common = (a_scale.data_ptr(), a_scale.numel(), w_scale.data_ptr(), w_scale.numel(), _ptr(bias),
               _DT[bias.dtype] if bias is not None else L.F32, int(epilogue), y.data_ptr(), _DT[out_dtype],
               N, M, N, K, int(chunk_size), int(chunk_trun_bits))
-    wptr, wbytes, _ws = _chunk_workspace(a, N, chunk_size, truncate_then_accumulate)
     with _dev(a):
         if a.dtype == torch.int8:
+            wptr, wbytes, _ws = _chunk_workspace(a, N, chunk_size, truncate_then_accumulate)
             L.call("fmsmo_matmul_chunk_i8_dq_ws", a.data_ptr(), _ld(a), w.data_ptr(), _ld(w), *common,
                    int(max_acc_bits), int(bool(truncate_then_accumulate)), wptr, wbytes, _stream(a))
         else:
-            L.call("fmsmo_matmul_chunk_fp_dq_ws", a.data_ptr(), _ld(a), w.data_ptr(), _ld(w), _OPDT[a.dtype],
-                   *common, int(bool(clamp_acc_to_dl16)), int(bool(truncate_then_accumulate)), wptr, wbytes, _stream(a))
+            L.call("fmsmo_matmul_chunk_fp_dq", a.data_ptr(), _ld(a), w.data_ptr(), _ld(w), _OPDT[a.dtype],
+                   *common, int(bool(clamp_acc_to_dl16)), int(bool(truncate_then_accumulate)), _stream(a))
     return y
 
 

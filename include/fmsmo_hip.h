@@ -576,7 +576,8 @@ int fmsmo_matmul_chunk_fp_dq(const void* a, int64_t lda, const void* b, int64_t 
  * The chunked matmuls with a caller's workspace (16-byte aligned device memory, written and read within the
  * call's work on the stream): tiles past the last whole round of the compute units are cut along K and their
  * partial accumulators added in it.  int8 results are the same bits, floating-point ones sums of the same
- * rounded chunks in another grouping.  fmsmo_matmul_chunk_workspace_bytes (host only): what the calls of a shape
+ * rounded chunks in another grouping, so that their last bits depend on the number of rows in the call: pass a
+ * workspace to the _fp forms where that does not matter (the Python wrappers pass none).  fmsmo_matmul_chunk_workspace_bytes (host only): what the calls of a shape
  * use, 0 where they use none; a smaller workspace cuts into fewer slices, NULL into none.  chunk_size in elements.
  */
 int64_t fmsmo_matmul_chunk_workspace_bytes(int op_dtype, int64_t M, int64_t N, int64_t K, int chunk_size,

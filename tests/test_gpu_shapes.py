@@ -474,6 +474,26 @@ def test_chunked_products_whose_reduction_is_cut(dev, M, N, Kd, cs, dtype):
         assert torch.equal(whole.cpu(), ref)
 
 
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,Kd,cs", [(130, 8192, 64), (600, 4096 + 48, 32)])
+def test_chunked_rows_do_not_depend_on_the_rows_beside_them(dev, dtype, N, Kd, cs):
+    """Real-valued operands, whose rounded chunks do not add up exactly: every row has the bits of the launch without a
+    workspace, which adds its chunks one after the other, whatever the number of rows."""
+    from fms_mo_amd import _lib as L
+
+    a = torch.randn(300, Kd, generator=gen(Kd)).to(dtype).to(dev)
+    w = torch.randn(N, Kd, generator=gen(N)).to(dtype).to(dev)
+    d = torch.empty((300, N), device=dev)
+    L.call("fmsmo_matmul_chunk_fp", a.data_ptr(), Kd, w.data_ptr(), Kd, K()._OPDT[dtype], None, d.data_ptr(), N, 300, N, Kd,
+           cs, 5, 0, 1, torch.cuda.current_stream().cuda_stream)
+    one = torch.ones(1, device=dev)
+    for M in (1, 16, 129, 300):
+        assert torch.equal(K().matmul_chunk(a[:M], w, None, chunk_size=cs, chunk_trun_bits=5), d[:M]), M
+        for a_scale in (one, 1.0 * one.expand(M).contiguous(), one.reshape(1, 1)):   # native call (twice), general path
+            y = K().matmul_chunk_dq(a[:M], w, a_scale, one, None, 1, torch.float32, chunk_size=cs, chunk_trun_bits=5)
+            assert torch.equal(y, d[:M]), M
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Kd,N,bias,stats", [(264, 37, True, "some"), (256, 256, False, "some"), (520, 300, True, "zero"),
                                              (8, 1, False, "none"), (512, 257, True, "extreme")])
