@@ -517,7 +517,8 @@ PyObject* item(PyObject* dict, PyObject* key) {  // borrowed, or null
 #define NAMES(X)                                                                                                \
   X(_buffers) X(_parameters) X(weight) X(bias) X(w_scale) X(smoothq_scale) X(input_scale) X(useDynMaxQfunc)      \
   X(use_int_kernel) X(chunk_size) X(truncate_lsb) X(use_fake_zero_shift) X(acc_dtype) X(_sq_kept) X(_ws_kept)    \
-  X(iaddmm) X(cvs) X(weight_scale) X(_quantize) X(qa_dynamic_max_qfunc)
+  X(iaddmm) X(cvs) X(weight_scale) X(_quantize) X(qa_dynamic_max_qfunc) X(_smoothq_active) X(_w_scale_f32)         \
+  X(_set_input_scale)
 #define DECLARE(n) PyObject* k_##n = nullptr;
 NAMES(DECLARE)
 #undef DECLARE
@@ -540,14 +541,24 @@ PyObject* kept_for(PyObject* kept, const at::Tensor& t) {
   return same ? PyTuple_GET_ITEM(kept, 1) : nullptr;
 }
 
-// QLinearINT8Deploy.forward with dynamic per-token scales and a plain integer product: (instance dict, x, the
-// class's own iaddmm_int) -> y.
+// Is a method of the class, or of this instance, another function than the one that came with it?
+bool replaced(PyObject* self, PyTypeObject* cls, PyObject* name, PyObject* own) {
+  return item(self, name) || _PyType_Lookup(cls, name) != own;
+}
+// QLinearINT8Deploy.forward with dynamic per-token scales and a plain integer product: (instance dict, x, the class,
+// (iaddmm_int, _smoothq_active, _w_scale_f32, _set_input_scale, _quantize, qa_dynamic_max_qfunc) as it came) -> y.
 // The scales' host-side facts (does SmoothQuant apply, the fp32 copy of w_scale) are those the Python side
 // keeps beside the buffers; where they are stale it is asked (None).
 PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  WANT(3);
-  PyObject* self = args[0];
+  WANT(4);
+  PyObject *self = args[0], *own_f = args[3];
+  if (!PyType_Check(args[2]) || !PyTuple_CheckExact(own_f) || PyTuple_GET_SIZE(own_f) != 6) return none();
+  // the methods that the forward in Python goes through
+  PyTypeObject* cls = (PyTypeObject*)args[2];
+  PyObject* const names[] = {k__smoothq_active, k__w_scale_f32, k__set_input_scale, k__quantize, k_qa_dynamic_max_qfunc};
+  for (int i = 0; i < 5; ++i)
+    if (replaced(self, cls, names[i], PyTuple_GET_ITEM(own_f, i + 1))) return none();
   const Mat x = rows_of(args[1]);
   if (!x || x.rows == 0 || code_of(x.t->scalar_type()) < 0) return none();
   PyObject *buffers = item(self, k__buffers), *params = item(self, k__parameters);
@@ -581,7 +592,7 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!ob) return none();
   const Opt b = opt_vec(ob, w.rows);
   const at::ScalarType xt = x.t->scalar_type();
-  if (!b.ok || !here(x.t, w.t, ws, sm.t, b.t)) return none();
+  if (!b.ok || !here(x.t, w.t, wsrc, ws, sq, b.t)) return none();
   // the epilogues round to the fp16 accumulator dtype and then to bf16 for a bf16 model
   const at::ScalarType ot = xt == at::kBFloat16 ? at::kBFloat16 : at::kHalf;
   if (xt == at::kFloat) return none();  // (the fp16 result is cast behind the product)
@@ -601,9 +612,8 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!smooth) {  // this branch ends in the module's iaddmm: only the class's own one is known here
       PyObject* f = item(self, k_iaddmm);
       PyObject* cvs = item(self, k_cvs);
-      if (!f || !PyMethod_Check(f) || PyMethod_GET_FUNCTION(f) != args[2] || item(self, k__quantize) ||
-          item(self, k_qa_dynamic_max_qfunc) || !cvs || !PyList_CheckExact(cvs) ||
-          PyList_GET_SIZE(cvs) < 2)
+      if (!f || !PyMethod_Check(f) || PyMethod_GET_FUNCTION(f) != PyTuple_GET_ITEM(own_f, 0) || !cvs ||
+          !PyList_CheckExact(cvs) || PyList_GET_SIZE(cvs) < 2)
         return none();
     }
     at::Tensor q, c;

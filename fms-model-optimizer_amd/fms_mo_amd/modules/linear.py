@@ -845,7 +845,7 @@ class QLinearINT8Deploy(nn.Linear):
         # decode step is bound by what the host does per call, so nothing is done twice here)
         if type(self) is QLinearINT8Deploy and not torch.compiler.is_compiling():
             # the dynamic per-token forms, natively; None: something here is less common
-            y = L.host().deploy_i8(self.__dict__, x, _IADDMM_INT)
+            y = L.host().deploy_i8(self.__dict__, x, QLinearINT8Deploy, _OWN_METHODS)
             if y is not None:
                 return y
         org_dtype = x.dtype
@@ -889,8 +889,9 @@ class QLinearINT8Deploy(nn.Linear):
         return y if y.dtype == org_dtype else y.to(org_dtype)
 
 
-# deploy_i8 knows what a module's iaddmm does only where it is the class's own
-_IADDMM_INT = QLinearINT8Deploy.iaddmm_int
+# deploy_i8 knows what the methods of a forward do only where they are these
+_OWN_METHODS = tuple(getattr(QLinearINT8Deploy, n) for n in ("iaddmm_int", "_smoothq_active", "_w_scale_f32", "_set_input_scale",
+                                                             "_quantize", "qa_dynamic_max_qfunc"))
 
 
 class LinearFPxAcc(torch.nn.Linear):

@@ -247,15 +247,26 @@ def test_scales_in_the_memory_of_the_ones_before(dev, general):
 
     x = torch.randn(50, 512, device=dev).half()
     m = QLinearINT8Deploy.from_fms_mo(qlinear(512, 64, torch.float16, True, dev, True), use_dynamic_max_act_Qfunc=-1).half()
-    m(x)
-    for i, factor in enumerate((2.0, 0.5, 4.0)):
+
+    def replace(name, values):
+        old = m._buffers[name].data_ptr()
+        m._buffers[name] = None
+        tried = []
+        while not tried or (tried[-1].data_ptr() != old and len(tried) < 64):
+            tried.append(values.to(dev))
+        m._buffers[name] = tried[-1]
+
+    scale, divisors = m.w_scale.cpu(), m.smoothq_scale.cpu()
+    replace("w_scale", scale)
+    replace("smoothq_scale", divisors)
+    for i in range(1, 4):
         y0 = m(x)
-        m = m.cpu()
-        m.w_scale.mul_(factor)
-        m.smoothq_scale = m.smoothq_scale.mul(3) if i != 1 else torch.ones_like(m.smoothq_scale)
-        m = m.to(dev)
+        replace("w_scale", scale * 2**i)
+        replace("smoothq_scale", divisors * 3 if i != 2 else torch.ones_like(divisors))
         y = m(x)
         with general():
+            for k in [k for k in m.__dict__ if k.startswith(("_ws_", "_sq_"))]:   # nothing kept
+                del m.__dict__[k]
             assert same(y, m(x)) and not torch.equal(y, y0), i
 
 
@@ -348,3 +359,41 @@ def test_native_calls_leave_tensors_of_another_gpu_to_the_general_path(dev):
             elif isinstance(a, dict):
                 for k in a:
                     assert f(*args[:i], {**a, k: on_another_gpu(a[k])}, *args[i + 1:]) is None, (f.__name__, k)
+    from fms_mo_amd.modules import linear
+
+    x = torch.randn(50, 512, device=dev).half()
+    m = linear.QLinearINT8Deploy.from_fms_mo(qlinear(512, 64, half, True, dev, True), use_dynamic_max_act_Qfunc=-1)
+    m(x)
+    call = lambda: h.deploy_i8(m.__dict__, x, type(m), linear._OWN_METHODS)  # noqa: E731
+    for held, n in ((m._parameters, "weight"), (m._buffers, "w_scale"), (m._buffers, "smoothq_scale"), (m._buffers, "bias")):
+        assert call() is not None
+        own, held[n] = held[n], on_another_gpu(held[n].detach())
+        assert call() is None, n
+        held[n] = own
+
+
+@pytest.mark.parametrize("smooth,tokens", [(False, 50), (True, 50), (True, 1)])
+def test_methods_replaced_on_the_class_or_the_module_are_called(dev, monkeypatch, smooth, tokens):
+    """Every method that the forward in Python goes through, replaced where a user would: on the class, on one module."""
+    from fms_mo_amd.modules.linear import QLinearINT8Deploy
+
+    x = torch.randn(tokens, 4096, device=dev).half()
+    m = QLinearINT8Deploy.from_fms_mo(qlinear(4096, 64, torch.float16, True, dev, smooth), use_dynamic_max_act_Qfunc=-1)
+    want = m(x)
+    names = ["_smoothq_active", "_w_scale_f32", "_set_input_scale"] + ["_quantize", "qa_dynamic_max_qfunc"] * (not smooth)
+    for name in names:
+        own, calls = getattr(QLinearINT8Deploy, name), []
+
+        def spy(self, *args):
+            calls.append(name)
+            return own(self, *args)
+
+        with monkeypatch.context() as p:
+            p.setattr(QLinearINT8Deploy, name, spy)
+            assert same(m(x), want) and calls, name
+        calls.clear()
+        m.__dict__[name] = lambda *args: spy(m, *args)
+        assert same(m(x), want) and calls, name
+        del m.__dict__[name]
+        calls.clear()
+        assert same(m(x), want) and not calls
