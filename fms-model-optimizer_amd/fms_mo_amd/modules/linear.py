@@ -117,7 +117,8 @@ def _dynamic_operands(q):
     w, bias = q.weight, q.bias
     if not (w.is_cuda and w.dtype in (torch.float16, torch.bfloat16) and w.is_contiguous() and w.shape[1] % 8 == 0
             and w.numel() and w.data_ptr() % 16 == 0
-            and (bias is None or (bias.is_contiguous() and bias.dtype in (torch.float16, torch.bfloat16, torch.float32)
+            and (bias is None or (bias.dim() == 1 and bias.numel() == w.shape[0] and bias.is_contiguous()
+                                  and bias.dtype in (torch.float16, torch.bfloat16, torch.float32)
                                   and bias.device == w.device))):
         return None
     if not getattr(q, "smoothq", False):

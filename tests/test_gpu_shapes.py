@@ -532,6 +532,21 @@ def test_vectors_of_a_converted_linear(dev, dtype, Kd, N, bias, stats):
     assert float(dep.input_scale) == 1 and [float(v) for v in dep.cvs[:2]] == [8.0, -8.0]
 
 
+def test_conversion_broadcasts_a_bias_of_one_element_and_refuses_another_length(dev):
+    """The kernel for the vectors reads one bias per output channel: other lengths are left to the torch expressions."""
+    from fms_mo_amd.modules.linear import QLinearINT8Deploy
+
+    m = make_qlinear(256, 96, torch.float16, bias=True).to(dev)
+    for n in (1, 7, 95, 97):
+        m.bias = torch.nn.Parameter(torch.full((n,), 0.25, device=dev).half())
+        if n == 1:
+            dep = QLinearINT8Deploy.from_fms_mo(m, use_dynamic_max_act_Qfunc=-1, recalc_clipvals=False)
+            assert torch.equal(dep.bias, torch.full((96,), 0.25, device=dev).half())
+        else:
+            with pytest.raises(RuntimeError):
+                QLinearINT8Deploy.from_fms_mo(m, use_dynamic_max_act_Qfunc=-1, recalc_clipvals=False)
+
+
 @pytest.mark.parametrize("counts,N,Kd", [
     ([3, 0, 1, 5], 130, 256),                       # a few rows per expert: 32 x 128 tiles
     ([0] * 40 + [1, 2, 33] + [0] * 30 + [64, 1], 72, 384),   # more groups than lanes, most of them empty
