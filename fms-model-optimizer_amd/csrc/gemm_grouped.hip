@@ -41,6 +41,8 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
   return pick;
 }
 
+bool big_is_persistent(int64_t K) { return K % 128 == 0 && use_register_staged(MMA_I8); }
+
 template <bool REF>
 int launch_grouped(const GemmArgs& g0, const float* a_scale, const float* w_scale, const void* bias, int bias_dtype,
                    int muladd, void* y, int y_dtype, int64_t ldy, hipStream_t st) {
@@ -56,7 +58,7 @@ int launch_grouped(const GemmArgs& g0, const float* a_scale, const float* w_scal
       case G_32: g.grid_m = rows_of(Tile32::BM); launch_tile<Tile32, MMA_I8, true>(g, epi, st); break;
       default:
         g.grid_m = rows_of(256);
-        if (g.K % 128 == 0 && use_register_staged(MMA_I8)) launch_rs<MMA_I8, true>(g, epi, st);
+        if (big_is_persistent(g.K)) launch_rs<MMA_I8, true>(g, epi, st);
         else launch_tile<TileBig, MMA_I8, true>(g, epi, st);
     }
   };
@@ -102,4 +104,18 @@ extern "C" int fmsmo_grouped_gemm_i8_dq(const int8_t* a, int64_t lda, const int8
     return launch_grouped<true>(g, a_scale, w_scale, bias, bias_dtype, 0, y, y_dtype, ldy, (hipStream_t)stream);
   return launch_grouped<false>(g, a_scale, w_scale, bias, bias_dtype, epilogue == FMSMO_EPI_F32_MULADD, y, y_dtype, ldy,
                                (hipStream_t)stream);
+}
+
+extern "C" int fmsmo_grouped_gemm_plan(int num_experts, int64_t total_rows, int64_t N, int64_t K, int* kernel, int* tile_m,
+                                       int* tile_n, int* stage) {
+  if (!kernel || !tile_m || !tile_n || !stage) return FMSMO_ERR_NULL;
+  if (num_experts <= 0 || total_rows <= 0 || N <= 0 || K <= 0 || total_rows >= (1 << 30) || N >= (1 << 30) || K >= (1ll << 31))
+    return FMSMO_ERR_SHAPE;
+  if (K % 64) return FMSMO_ERR_ALIGN;
+  const GroupedTile t = pick_grouped_tile(num_experts, total_rows, N, K);
+  *kernel = t == G_BIG && big_is_persistent(K) ? FMSMO_PLAN_TILE_REGISTER_STAGED : FMSMO_PLAN_TILE_LDS_DMA;
+  *tile_m = t == G_BIG ? 256 : t == G_64 ? Tile64::BM : t == G_32 ? Tile32::BM : TileMid::BM;
+  *tile_n = t == G_BIG ? 256 : t == G_64 ? Tile64::BN : t == G_32 ? Tile32::BN : TileMid::BN;
+  *stage = t == G_MID || (t == G_BIG && *kernel == FMSMO_PLAN_TILE_LDS_DMA) ? 64 : 128;
+  return FMSMO_OK;
 }

@@ -298,6 +298,15 @@ def gemm_plan(M, N, K, with_workspace=False, fp8=False):
     return tuple(o.value for o in out)
 
 
+def grouped_gemm_plan(experts, rows, N, K):
+    """(kernel, tile_m, tile_n, bytes of K per stage) grouped_gemm_i8_dq uses for a shape; no GPU needed."""
+    import ctypes
+
+    out = [ctypes.c_int(0) for _ in range(4)]
+    L.call("fmsmo_grouped_gemm_plan", experts, rows, N, K, *[ctypes.byref(o) for o in out])
+    return tuple(o.value for o in out)
+
+
 def clock_probe(buf):
     """Diagnostic: have block 0 of the following 256-row-tile GEMM launches store its clock
     readings into `buf` (int64 [6] on the GPU), or switch the probe off with None.  See

@@ -624,6 +624,9 @@ int fmsmo_grouped_gemm_i8_dq(const int8_t* a, int64_t lda, const int8_t* b, int6
                              const void* bias, int bias_dtype, int epilogue, void* y,
                              int y_dtype, int64_t ldy, int64_t N, int64_t K,
                              fmsmo_stream_t stream);
+/* Which kernel (enum fmsmo_plan_kernel), tile and bytes of K per stage it runs for a shape.  Host-only. */
+int fmsmo_grouped_gemm_plan(int num_experts, int64_t total_rows, int64_t N, int64_t K, int* kernel, int* tile_m,
+                            int* tile_n, int* stage);
 
 /* ------------------------------------------------------------------------------------------
  * 6. Offline weight path: float weights -> int8 rows (+ integer row sums), one pass over W.

@@ -547,27 +547,42 @@ def test_conversion_broadcasts_a_bias_of_one_element_and_refuses_another_length(
                 QLinearINT8Deploy.from_fms_mo(m, use_dynamic_max_act_Qfunc=-1, recalc_clipvals=False)
 
 
-@pytest.mark.parametrize("counts,N,Kd", [
-    ([3, 0, 1, 5], 130, 256),                       # a few rows per expert: 32 x 128 tiles
-    ([0] * 40 + [1, 2, 33] + [0] * 30 + [64, 1], 72, 384),   # more groups than lanes, most of them empty
-    ([43, 64, 65, 0], 200, 1024),                   # 64 x 64
-    ([180, 256, 100, 129, 181], 1100, 640),         # 128 x 128, 64-byte stages
-    ([350, 300, 257, 384, 1], 2500, 4096),          # 128 x 128, 128-byte stages
-    ([513, 0, 700, 2000], 8200, 512),               # 256 x 256
-    ([10, 200, 127], 300, 192)])                    # reduction of whole 64-byte stages only
+@pytest.mark.parametrize("counts,N,Kd,tile", [
+    ([3, 0, 1, 5], 130, 256, (256, 256, 128)),                                   # a few rows per expert
+    ([0] * 40 + [1, 2, 33] + [0] * 30 + [64, 1], 72, 384, (64, 64, 128)),        # more groups than lanes, most of them empty
+    ([43, 64, 65, 0], 200, 1024, (64, 64, 128)),
+    ([180, 256, 100, 129, 181], 1100, 640, (64, 64, 128)),
+    ([41, 0, 60, 63], 8203, 256, (32, 128, 128)),                                # whole and ragged tiles of 32 rows
+    ([1, 31, 32, 33, 2, 0, 9, 10, 64, 65, 1, 7, 8, 0, 0, 12], 8190, 384, (32, 128, 128)),
+    ([20] * 69 + [65], 4097, 384, (32, 128, 128)),                               # more groups than lanes
+    ([40] * 64 + [0, 7, 128, 1, 1, 3], 4100, 384, (128, 128, 64)),
+    ([0, 40, 60], 1100, 192, (128, 128, 64)),                                    # reduction of whole 64-byte stages only
+    ([350, 300, 257, 384, 1], 2500, 4096, (128, 128, 128)),
+    ([1, 128, 129, 42], 8200, 256, (128, 128, 64)),
+    ([513, 0, 700, 2000], 8200, 512, (256, 256, 128)),
+    ([10, 200, 127], 300, 192, (256, 256, 64))])
 @pytest.mark.parametrize("exact_ref,out_dtype", [(True, torch.float16), (False, torch.float32)])
-def test_grouped_products_in_every_tile(dev, counts, N, Kd, exact_ref, out_dtype):
+def test_grouped_products_in_every_tile(dev, counts, N, Kd, tile, exact_ref, out_dtype):
     """Bit-identical to one product per expert (integer sums, the same epilogue), rows of no expert untouched."""
+    from fms_mo_amd import _lib as L
+
     kn = K()
-    E, T = len(counts), sum(counts)
+    E, lead, T = len(counts), 3, sum(counts) + 5     # three rows in front of the first expert's, two behind the last one's
+    for rows in (T - 5, T):
+        assert kn.grouped_gemm_plan(E, rows, N, Kd)[1:] == tile
     g = torch.Generator(device=dev).manual_seed(N)
     a = torch.randint(-128, 128, (T, Kd), generator=g, dtype=torch.int8, device=dev)
     w = torch.randint(-128, 128, (E, N, Kd), generator=g, dtype=torch.int8, device=dev)
     sa, sw = torch.rand(T, generator=g, device=dev) * 1e-3, torch.rand(E, N, generator=g, device=dev) * 1e-2
     b = torch.randn(E, N, generator=g, device=dev)
-    off = torch.tensor([0] + counts, device=dev).cumsum(0).to(torch.int32)
-    y = kn.grouped_gemm_i8_dq(a, w, off, sa, sw, b, out_dtype=out_dtype, exact_ref=exact_ref)
-    lo = 0
+    off = torch.tensor([lead] + counts, device=dev).cumsum(0).to(torch.int32)
+    y = torch.full((T + 1, N), -7.0, device=dev, dtype=out_dtype)
+    L.call("fmsmo_grouped_gemm_i8_dq", a.data_ptr(), Kd, w.data_ptr(), Kd, N * Kd, off.data_ptr(), E, T, sa.data_ptr(), sw.data_ptr(),
+           b.data_ptr(), L.F32, L.EPI_REF_F16 if exact_ref else L.EPI_F32, y.data_ptr(), kn._DT[out_dtype], N, N, Kd,
+           torch.cuda.current_stream().cuda_stream)
+    inner = kn.grouped_gemm_i8_dq(a[lead:-2], w, off - lead, sa[lead:-2], sw, b, out_dtype=out_dtype, exact_ref=exact_ref)
+    assert torch.equal(inner, y[lead:-3]) and (y[:lead] == -7).all() and (y[-3:] == -7).all()
+    lo = lead
     for e, c in enumerate(counts):
         if c:
             ref = kn.gemm_i8_dq(a[lo:lo + c], w[e], sa[lo:lo + c], sw[e], b[e], out_dtype=out_dtype, exact_ref=exact_ref)
