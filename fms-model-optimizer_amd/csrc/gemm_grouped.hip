@@ -19,6 +19,8 @@ struct Tile32 { static constexpr int BM = 32, BN = 128, BK = 128, NST = 4, WGM =
 //   16, 1336, 1664, 5632 67.6 | 29.3 | 30.3 | 39.1 | 43.2    8, 2652, 4352, 2176  69.1 | 48.2 | 49.4 | 59.7 | 63.6
 //   16, 1992, 1280, 11136 106.7 | 54.1 | 61.5 | 58.3 | 72.4  4, 1387, 8192, 3968  61.2 | 64.1 | 67.9 | 85.5 | 102.9
 //   8, 4772, 2560, 12672 175 | 234 | 254 | 325 | 377         8, 8192, 4096, 14336 537 | 636 | 724 | 1012 | 1331
+// A launch takes a round at least, however few its tiles (taken as half a one, up to a dozen tiles went to 256 x 256; us,
+// -> as now: 4, 9, 130, 256 8.8 -> 3.9; 7, 949, 59, 448 24.7 -> 9.0; of 60 such launches all faster, 13.8 -> 6.2 in the mean).
 enum GroupedTile { G_BIG, G_MIDK, G_MID, G_64, G_32 };
 GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t K) {
   const double slabs = (double)K / 128;
@@ -27,7 +29,7 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
     return (rows < experts ? (double)rows : experts * per) * div_up(N, bn);
   };
   const double t256 = tiles(256, 256) / 256, t128 = tiles(128, 128);
-  const double big = 0.5 * (std::ceil(std::max(0.0, t256 - 0.05)) + std::ceil(t256 + 0.05)) * (1.6 * slabs + 9);
+  const double big = 0.5 * (std::max(1.0, std::ceil(t256 - 0.05)) + std::ceil(t256 + 0.05)) * (1.6 * slabs + 9);
   double best = 0.95 * big;
   GroupedTile pick = G_BIG;
   auto offer = [&](GroupedTile t, double cost) {

@@ -548,7 +548,7 @@ def test_conversion_broadcasts_a_bias_of_one_element_and_refuses_another_length(
 
 
 @pytest.mark.parametrize("counts,N,Kd,tile", [
-    ([3, 0, 1, 5], 130, 256, (256, 256, 128)),                                   # a few rows per expert
+    ([3, 0, 1, 5], 130, 256, (64, 64, 128)),                                     # a few rows per expert
     ([0] * 40 + [1, 2, 33] + [0] * 30 + [64, 1], 72, 384, (64, 64, 128)),        # more groups than lanes, most of them empty
     ([43, 64, 65, 0], 200, 1024, (64, 64, 128)),
     ([180, 256, 100, 129, 181], 1100, 640, (64, 64, 128)),
@@ -560,7 +560,8 @@ def test_conversion_broadcasts_a_bias_of_one_element_and_refuses_another_length(
     ([350, 300, 257, 384, 1], 2500, 4096, (128, 128, 128)),
     ([1, 128, 129, 42], 8200, 256, (128, 128, 64)),
     ([513, 0, 700, 2000], 8200, 512, (256, 256, 128)),
-    ([10, 200, 127], 300, 192, (256, 256, 64))])
+    ([10, 200, 127], 300, 192, (128, 128, 64)),
+    ([2049, 0, 1800, 255], 8200, 1216, (256, 256, 64))])
 @pytest.mark.parametrize("exact_ref,out_dtype", [(True, torch.float16), (False, torch.float32)])
 def test_grouped_products_in_every_tile(dev, counts, N, Kd, tile, exact_ref, out_dtype):
     """Bit-identical to one product per expert (integer sums, the same epilogue), rows of no expert untouched."""

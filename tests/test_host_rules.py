@@ -78,3 +78,18 @@ def test_chunked_products_ask_for_a_workspace_only_where_they_may_be_cut():
     assert need(L.OP_I8, 16, 4096, 14336, 16384, 1) == 0             # one chunk
     assert need(L.OP_F16, 16, 4096, 4096, 8, 1) == 0 and need(9, 16, 4096, 4096, 64, 1) == 0
     assert need(L.OP_I8, 0, 4096, 4096, 64, 1) == 0 and need(L.OP_I8, 1 << 30, 4096, 4096, 64, 1) == 0
+
+
+def test_a_grouped_launch_of_a_few_tiles_takes_small_ones():
+    """Never 256 x 256, which leave all but a dozen compute units idle, nor anything that is no whole number of stages."""
+    for E in (1, 4, 7, 64):
+        for rows in (1, 9, 164, 949):
+            for N in (1, 59, 256, 300):
+                for Kd in (64, 128, 192, 256, 448, 1472, 4096):
+                    _, tm, tn, stage = kernels.grouped_gemm_plan(E, rows, N, Kd)
+                    assert (tm, tn) != (256, 256) and Kd % stage == 0, (E, rows, N, Kd)
+    assert kernels.grouped_gemm_plan(8, 8192, 28672, 4096) == (L.PLAN_TILE_REGISTER_STAGED, 256, 256, 128)
+    assert kernels.grouped_gemm_plan(4, 4104, 8200, 1216) == (L.PLAN_TILE_LDS_DMA, 256, 256, 64)
+    for bad in ((0, 8, 8, 64), (1, 0, 8, 64), (1, 8, 8, 96)):
+        with pytest.raises(L.FmsMoHipError):
+            kernels.grouped_gemm_plan(*bad)
