@@ -725,9 +725,16 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fmsmo_host", nullptr, -1, methods
 
 }  // namespace
 
+#define TEXT_(x) #x
+#define TEXT(x) TEXT_(x)
 PyMODINIT_FUNC PyInit__fmsmo_host() {
 #define INTERN(n) k_##n = PyUnicode_InternFromString(#n);
   NAMES(INTERN)
 #undef INTERN
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  // what this file was compiled against: neither torch's nor Python's ABI is in the file's name
+  if (m && PyModule_AddStringConstant(m, "built_for", "torch " FMSMO_TORCH_VERSION ", Python " TEXT(PY_MAJOR_VERSION) "." TEXT(
+                                                          PY_MINOR_VERSION)))
+    return nullptr;
+  return m;
 }

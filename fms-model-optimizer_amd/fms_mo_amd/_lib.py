@@ -150,11 +150,17 @@ def host():
     lib = load()
     if not os.path.exists(HOST_PATH):
         raise FmsMoHipError(f"{HOST_PATH} is missing: build it first (make -C fms-model-optimizer_amd/csrc)")
+    import sys
     from importlib import machinery, util
+
+    import torch
 
     loader = machinery.ExtensionFileLoader("_fmsmo_host", HOST_PATH)
     mod = util.module_from_spec(util.spec_from_file_location("_fmsmo_host", HOST_PATH, loader=loader))
     loader.exec_module(mod)
+    here = f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"
+    if mod.built_for != here:
+        raise FmsMoHipError(f"{HOST_PATH} was built for {mod.built_for}, this is {here}: build it again")
     mod.bind({n: ctypes.cast(getattr(lib, n), c_void_p).value for n in mod.entries()}, raise_status)
     _host = mod
     return mod

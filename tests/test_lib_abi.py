@@ -234,3 +234,15 @@ def test_plan_of_the_entry_point_that_allocates_nothing():
     for mode in (0, 1, 2):
         assert lib.fmsmo_gemm_plan(4, 4096, 4096, mode, ctypes.byref(k), ctypes.byref(tm), ctypes.byref(tn), ctypes.byref(sp)) == 0
         assert k.value == _lib.PLAN_DECODE
+
+
+def test_the_host_module_is_refused_under_another_torch(monkeypatch):
+    import torch
+
+    from fms_mo_amd import _lib
+
+    assert _lib.host().built_for.startswith(f"torch {torch.__version__}, ")
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    with pytest.raises(_lib.FmsMoHipError, match="was built for torch"):
+        _lib.host()
