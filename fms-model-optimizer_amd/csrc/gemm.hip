@@ -200,11 +200,13 @@ extern "C" int64_t fmsmo_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t 
   return plan_split_k(M, N, K, 0, true).ws_bytes;
 }
 
-extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) {
+static int64_t gemm_tail_columns(bool fp8, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
   if (use_decode(M, N, K)) return 0;
-  return tail_split_columns((int)M, (int)N, (int)K, false);
+  return tail_split_columns((int)M, (int)N, (int)K, fp8);
 }
+extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) { return gemm_tail_columns(false, M, N, K); }
+extern "C" int64_t fmsmo_gemm_fp8_tail_columns(int64_t M, int64_t N, int64_t K) { return gemm_tail_columns(true, M, N, K); }
 
 static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
                      int* tile_n, int* splits) {

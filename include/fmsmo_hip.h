@@ -405,8 +405,9 @@ int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* ke
 int fmsmo_gemm_fp8_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
                         int* tile_n, int* splits);
 /* Columns that the single-pass *_dq GEMMs cut off the end of N and run as a second GEMM behind
-   the first (0: the GEMM runs whole; fmsmo_gemm_plan describes the first, main part).  Host-only. */
+   the first (0: the GEMM runs whole; fmsmo_gemm_plan describes the first, main part).  int8, e4m3.  Host-only. */
 int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K);
+int64_t fmsmo_gemm_fp8_tail_columns(int64_t M, int64_t N, int64_t K);
 int fmsmo_gemm_i8_dq_ws(const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
                         const float* a_scale, int64_t a_scale_n, const float* w_scale,
                         int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue, void* y,

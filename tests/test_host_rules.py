@@ -93,3 +93,15 @@ def test_a_grouped_launch_of_a_few_tiles_takes_small_ones():
     for bad in ((0, 8, 8, 64), (1, 0, 8, 64), (1, 8, 8, 96)):
         with pytest.raises(L.FmsMoHipError):
             kernels.grouped_gemm_plan(*bad)
+
+
+def test_the_columns_cut_off_a_last_round_are_those_of_the_operand_type():
+    """int8 takes 128 x 128 tiles up to K = 1280 where that pays, e4m3 up to 640 and by another margin: a launch that does
+    has no round of 256 x 256 tiles to cut."""
+    if any(os.environ.get(k) for k in ("FMSMO_TILE", "FMSMO_RS", "FMSMO_TAIL_SPLIT")):
+        pytest.skip("tuning overrides are set")
+    i8, fp8 = L.load().fmsmo_gemm_tail_columns, L.load().fmsmo_gemm_fp8_tail_columns
+    assert (i8(1700, 20992, 640), fp8(1700, 20992, 640)) == (0, 2304)
+    assert kernels.gemm_plan(1700, 20992, 640)[1:3] == (128, 128) and kernels.gemm_plan(1700, 20992, 640, fp8=True)[1:3] == (256, 256)
+    assert i8(2048, 25600, 4096) == fp8(2048, 25600, 4096) == 1024
+    assert fp8(4096, 28672, 4096) == fp8(16, 25600, 4096) == fp8(0, 25600, 4096) == 0
