@@ -554,11 +554,10 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   WANT(4);
   PyObject *self = args[0], *own_f = args[3];
   if (!PyType_Check(args[2]) || !PyTuple_CheckExact(own_f) || PyTuple_GET_SIZE(own_f) != 6) return none();
-  // the methods that the forward in Python goes through
+  // the methods that the forward in Python goes through: these always, its quantizer's and iaddmm on one branch below
   PyTypeObject* cls = (PyTypeObject*)args[2];
-  PyObject* const names[] = {k__smoothq_active, k__w_scale_f32, k__set_input_scale, k__quantize, k_qa_dynamic_max_qfunc};
-  for (int i = 0; i < 5; ++i)
-    if (replaced(self, cls, names[i], PyTuple_GET_ITEM(own_f, i + 1))) return none();
+  auto other = [&](PyObject* name, int i) { return replaced(self, cls, name, PyTuple_GET_ITEM(own_f, i)); };
+  if (other(k__smoothq_active, 1) || other(k__w_scale_f32, 2) || other(k__set_input_scale, 3)) return none();
   const Mat x = rows_of(args[1]);
   if (!x || x.rows == 0 || code_of(x.t->scalar_type()) < 0) return none();
   PyObject *buffers = item(self, k__buffers), *params = item(self, k__parameters);
@@ -613,7 +612,7 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       PyObject* f = item(self, k_iaddmm);
       PyObject* cvs = item(self, k_cvs);
       if (!f || !PyMethod_Check(f) || PyMethod_GET_FUNCTION(f) != PyTuple_GET_ITEM(own_f, 0) || !cvs ||
-          !PyList_CheckExact(cvs) || PyList_GET_SIZE(cvs) < 2)
+          !PyList_CheckExact(cvs) || PyList_GET_SIZE(cvs) < 2 || other(k__quantize, 4) || other(k_qa_dynamic_max_qfunc, 5))
         return none();
     }
     at::Tensor q, c;
