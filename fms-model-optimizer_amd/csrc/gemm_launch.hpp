@@ -70,8 +70,10 @@ struct TileSmallK { static constexpr int BM = 64, BN = 64, BK = 128, NST = 4, WG
 // Which launches they take: up to one block per compute unit on reductions under 2048 (one pass takes 3.3 us + 1.6
 // per 1024 of K, less than a pass of any other tile; from there on slices of two or four come close), up to 3072
 // above 128 rows, under 8192 above 256 rows, whose partial sums cost more than they save, and any length above 1024
-// rows, which take no slices; up to two per compute unit on short ones.  (33 .. 64 tiles, and the reductions these bounds leave out, keep the plans they had, some of
-// which callers and tests rely on.)  Up to 64 tokens the decode kernels re-read the activations for every 16 weight
+// rows, which take no slices; up to two per compute unit on short ones.  33 .. 64 tiles up to 1024 rows keep the plans they
+// had, two of which the tests pin (200 x 1024 x 1536 in three slices, 300 x 520 x 1024 on 128 x 128 tiles), and not for their speed: with K < 2048
+// these tiles take 0.50 ... 0.78 of the time (33 launches, int8 8.2 -> 5.4 and 9.2 -> 5.1 in those two), above 256 rows with K = 2048 .. 7680
+// 1.04 (int8) and 0.87 (e4m3) in the mean of 38.  Up to 64 tokens the decode kernels re-read the activations for every 16 weight
 // rows and win until there are many of those.  us from a HIP graph, int8 | e4m3, before -> these:
 //   N = 6144, K = 1024: M = 100 10.4 -> 5.3; N = 2432, K = 2048: 200 10.4 -> 6.8, 400 9.0 -> 8.1; N = 4096, K = 3072:
 //   200 11.6 -> 8.9 | 10.7 -> 7.5; N = 1024: K = 4096, M = 800 13.5 -> 10.6, 1000 13.6 -> 10.9; K = 5120 / 6144, M = 1000

@@ -180,8 +180,3 @@ def call(name: str, *args) -> None:
     rc = getattr(load(), name)(*args)
     if rc != 0:
         raise_status(name, rc)
-
-
-def entry(name: str):
-    """The bound entry point itself (returns the status), for callers that keep it."""
-    return getattr(load(), name)

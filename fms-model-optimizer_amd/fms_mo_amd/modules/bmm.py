@@ -3,8 +3,8 @@ class name, ``from_fms_mo`` signature and buffers (fms_mo/modules/bmm.py:607-748
 
 The reference's forward still *simulates* the integer product (``torch.matmul`` on the int8 codes
 cast to fp16, "haven't implemented any batched CUTLASS matmul").  Here both operands are quantized
-by one HIP kernel each (m2, stored ``[k, n]``, is written transposed so that its reduction
-dimension becomes contiguous; a large m1 -- probabilities x values -- on its way into the product),
+in one HIP launch (m2, stored ``[k, n]``, is written transposed so that its reduction
+dimension becomes contiguous; a large m1 -- probabilities x values -- instead on its way into the product),
 multiplied on the MFMA units with exact int32 accumulation, and dequantized in the GEMM epilogue
 together with the zero-point correction of the asymmetric m1, made in integers.
 The correction is summed over the reduction dimension of every batch entry; the reference's
