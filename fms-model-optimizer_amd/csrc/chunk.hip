@@ -289,7 +289,9 @@ static bool launch_chunk_tile(const ChunkArgs& c, const EpiChunk<AccT>& epi, voi
   g.hi = c.max_acc_bits < 32 ? (1 << (c.max_acc_bits - 1)) - 1 : 0x7fffffff;
   g.post = c.dl16 || g.t > 0 || c.max_acc_bits < 32;
   g.dl16 = c.dl16; g.tta = c.tta; g.c_in = c.c_in; g.ldc = c.ldc;
-  const ChunkPlan p = plan_chunk(MMA, c.M, c.N, c.Kb, c.chunk_bytes, c.tta && !c.c_in && ws, ws_bytes);
+  // (a size below zero is no room, not the query's "as much as it takes")
+  const ChunkPlan p =
+      plan_chunk(MMA, c.M, c.N, c.Kb, c.chunk_bytes, c.tta && !c.c_in && ws, std::max<int64_t>(0, ws_bytes));
   g.full = p.full; g.slices = p.slices; g.slice_len = p.slice_len; g.ws = ws;
   const bool fast = c.tta && !c.dl16 && c.max_acc_bits >= 32;
   const int tiles = g.grid_m * g.grid_n, cut = tiles - p.full;

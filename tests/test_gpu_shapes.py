@@ -468,6 +468,11 @@ def test_chunked_products_whose_reduction_is_cut(dev, M, N, Kd, cs, dtype):
     for limit in {nbytes, nbytes // 2, nbytes - 16}:
         if limit > 0:
             assert torch.equal(run(limit), whole), limit
+    if dtype == torch.int8 and nbytes:   # a size below zero is no room
+        d, ws = torch.empty((M, N), dtype=acc, device=dev), torch.full((nbytes,), 0x5a, dtype=torch.uint8, device=dev)
+        L.call("fmsmo_matmul_chunk_i8_ws", a.data_ptr(), Kd, w.data_ptr(), Kd, None, d.data_ptr(), N, M, N, Kd, cs, t, 32, 1,
+               ws.data_ptr(), -1, torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(d, whole) and bool((ws == 0x5a).all())
     if N < 1000:
         ref = (O.chunk_matmul_i8(a.cpu(), w.cpu(), None, cs, t, 32) if dtype == torch.int8
                else O.chunk_matmul_fp(a.cpu().float(), w.cpu().float(), None, cs, t))
