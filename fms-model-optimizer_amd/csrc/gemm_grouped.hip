@@ -32,14 +32,16 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
   const double big = 0.5 * (std::max(1.0, std::ceil(t256 - 0.05)) + std::ceil(t256 + 0.05)) * (1.6 * slabs + 9);
   double best = 0.95 * big;
   GroupedTile pick = G_BIG;
-  auto offer = [&](GroupedTile t, double cost) {
+  auto offer = [&](GroupedTile t, int bm, int bn, double cost) {
+    // one block per possible tile, 256 threads each: a launch holds less than 2^32 threads (the persistent blocks do not grow)
+    if (((rows + bm - 1) / bm + experts) * div_up(N, bn) >= (1 << 24)) return;
     if (cost < best) best = cost, pick = t;
   };
-  offer(G_MID, std::max(1.0, t128 / 512) * (1.2 * slabs + 6));
+  offer(G_MID, 128, 128, std::max(1.0, t128 / 512) * (1.2 * slabs + 6));
   if (K % 128) return pick;  // (the others take whole 128-byte stages)
-  offer(G_MIDK, std::ceil(t128 / 256) * ((t128 <= 512 ? 0.5 : 0.6) * slabs + 5));
-  offer(G_64, std::max(1.0, tiles(64, 64) / 512) * (0.4 * slabs + 5));
-  offer(G_32, std::max(1.0, tiles(32, 128) / 512) * (0.45 * slabs + 5));
+  offer(G_MIDK, 128, 128, std::ceil(t128 / 256) * ((t128 <= 512 ? 0.5 : 0.6) * slabs + 5));
+  offer(G_64, 64, 64, std::max(1.0, tiles(64, 64) / 512) * (0.4 * slabs + 5));
+  offer(G_32, 32, 128, std::max(1.0, tiles(32, 128) / 512) * (0.45 * slabs + 5));
   return pick;
 }
 

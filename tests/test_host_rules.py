@@ -90,6 +90,10 @@ def test_a_grouped_launch_of_a_few_tiles_takes_small_ones():
                     assert (tm, tn) != (256, 256) and Kd % stage == 0, (E, rows, N, Kd)
     assert kernels.grouped_gemm_plan(8, 8192, 28672, 4096) == (L.PLAN_TILE_REGISTER_STAGED, 256, 256, 128)
     assert kernels.grouped_gemm_plan(4, 4104, 8200, 1216) == (L.PLAN_TILE_LDS_DMA, 256, 256, 64)
+    # tens of thousands of experts: no launch of more than 2^32 threads (one block per possible tile)
+    for E, rows, N, Kd in ((1 << 16, 1 << 16, 16384, 128), (1 << 18, 100, 8192, 128), (1 << 20, 1 << 20, 2048, 128)):
+        kernel, tm, tn, _ = kernels.grouped_gemm_plan(E, rows, N, Kd)
+        assert kernel == L.PLAN_TILE_REGISTER_STAGED or (-(-rows // tm) + E) * -(-N // tn) * 256 < 1 << 32, (E, rows, N)
     for bad in ((0, 8, 8, 64), (1, 0, 8, 64), (1, 8, 8, 96)):
         with pytest.raises(L.FmsMoHipError):
             kernels.grouped_gemm_plan(*bad)
