@@ -288,7 +288,7 @@ static bool launch_chunk_tile(const ChunkArgs& c, const EpiChunk<AccT>& epi, voi
   g.lo = c.max_acc_bits < 32 ? -(1 << (c.max_acc_bits - 1)) : (int)0x80000000;
   g.hi = c.max_acc_bits < 32 ? (1 << (c.max_acc_bits - 1)) - 1 : 0x7fffffff;
   g.post = c.dl16 || g.t > 0 || c.max_acc_bits < 32;
-  g.dl16 = c.dl16; g.tta = c.tta; g.c_in = c.c_in; g.ldc = c.ldc;
+  g.c_in = c.c_in; g.ldc = c.ldc;
   // (a size below zero is no room, not the query's "as much as it takes")
   const ChunkPlan p =
       plan_chunk(MMA, c.M, c.N, c.Kb, c.chunk_bytes, c.tta && !c.c_in && ws, std::max<int64_t>(0, ws_bytes));
@@ -300,11 +300,19 @@ static bool launch_chunk_tile(const ChunkArgs& c, const EpiChunk<AccT>& epi, voi
     constexpr bool KT = decltype(kt_c)::value;
     // the schedules that round one block while the matrix unit multiplies the others: a chunk of one
     // 64-byte stage (every operand type), of several stages or of one 32-byte k-step (int8)
-    if (!fast) hipLaunchKernelGGL((chunk_tile_kernel<MMA, false, 0, KT>), grid, block, 0, st, g, epi);
-    else if (c.chunk_bytes == 64) hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 1, KT>), grid, block, 0, st, g, epi);
-    else if constexpr (MMA != MMA_I8) hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 0, KT>), grid, block, 0, st, g, epi);
-    else if (c.chunk_bytes == 32) hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 3, KT>), grid, block, 0, st, g, epi);
-    else hipLaunchKernelGGL((chunk_tile_kernel<MMA, true, 2, KT>), grid, block, 0, st, g, epi);
+    auto run = [&](auto hook_c, auto sched_c) {
+      hipLaunchKernelGGL((chunk_tile_kernel<MMA, decltype(hook_c)::value, decltype(sched_c)::value, KT>), grid, block, 0, st, g, epi);
+    };
+    typedef std::integral_constant<int, CHUNK_FAST> Fast;
+    typedef std::integral_constant<int, 0> S0;
+    if (!c.tta && c.dl16 && MMA != MMA_I8) {
+      if constexpr (MMA != MMA_I8) run(std::integral_constant<int, CHUNK_RUNNING_DL16>{}, S0{});
+    } else if (!c.tta) run(std::integral_constant<int, CHUNK_RUNNING>{}, S0{});
+    else if (!fast) run(std::integral_constant<int, CHUNK_CLAMP>{}, S0{});
+    else if (c.chunk_bytes == 64) run(Fast{}, std::integral_constant<int, 1>{});
+    else if constexpr (MMA != MMA_I8) run(Fast{}, S0{});
+    else if (c.chunk_bytes == 32) run(Fast{}, std::integral_constant<int, 3>{});
+    else run(Fast{}, std::integral_constant<int, 2>{});
   };
   if (g.K % 64) go(std::true_type{});
   else go(std::false_type{});

@@ -4,8 +4,8 @@
 //
 // Every `chunk_ks` MFMA k-steps (32 bytes of K) the partial product is range-clamped / LSB-rounded on
 // the vector ALU and folded into the running accumulator (or the running accumulator itself is rounded
-// when tta == 0).  FAST = the common configuration (truncate-then-accumulate, no integer clamp, no DL16
-// clamp).  SCHED (with FAST): the schedules that round one block while the matrix unit multiplies the
+// when tta == 0).  HOOK says how: CHUNK_FAST = the common configuration (truncate-then-accumulate, no integer
+// clamp, no DL16 clamp), the others are below.  SCHED (with CHUNK_FAST): the schedules that round one block while the matrix unit multiplies the
 // others inside one wave; 1 = a chunk is one stage, 2 = several whole stages (integers), 3 = one k-step
 // (integers), 0 = the generic hook.  Each is a kernel of its own (one kernel with all three loops spills).
 //
@@ -226,7 +226,7 @@ struct ChunkTileArgs {
   int chunk_ks;        // MFMA k-steps (32 bytes of K) per chunk
   int t, lo, hi;       // LSBs to round away; integer clamp range
   unsigned round_bit, mask;
-  int post, dl16, tta;
+  int post;            // something to round or clamp
   const void* c_in;    // optional initial accumulator [M, N], same element type as the accumulator
   int64_t ldc;
   // Tiles [0, full) of the tile sequence are whole; of the others every block takes one of `slices` pieces of
@@ -239,12 +239,20 @@ struct ChunkTileArgs {
 };
 constexpr int CHUNK_GROUP_M = 8;  // tile order: column-major in groups of as many tile rows
 
+// What happens at the end of a chunk, beside the common configuration: a clamped chunk is folded (integers: to
+// fewer bits, floating point: to DL16), or the running accumulator itself is rounded, in floating point without or
+// with the DL16 clamp.  As constants: tested per element, and with the other form's accumulators in registers, these
+// kernels took 1.1 to 4 times as long (us, before -> after, chunk 64: fp16 running sum 435 x 857 x 1472 51.8 -> 17.4,
+// e4m3 333 x 56 x 7296 349 -> 100; chunk 32: int8 clamped to 20 bits 5 x 25 x 6720 277 -> 169, fp16 running sum with
+// DL16 33 x 315 x 1568 149 -> 83).
+enum { CHUNK_FAST, CHUNK_CLAMP, CHUNK_RUNNING, CHUNK_RUNNING_DL16 };
 // KT: K is no multiple of a stage.
-template <int OP, bool FAST, int SCHED, bool KT>
-// (two blocks per compute unit for the fast configuration; the generic hook keeps a second
-// accumulator set and would spill at 256 registers)
-__global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTileArgs g, EpiChunk<typename Mma<OP>::Elem> epi) {
+template <int OP, int HOOK, int SCHED, bool KT>
+// (two blocks per compute unit for the fast configuration; the others would spill at 256 registers)
+__global__ __launch_bounds__(256, HOOK == CHUNK_FAST ? 2 : 1) void chunk_tile_kernel(ChunkTileArgs g, EpiChunk<typename Mma<OP>::Elem> epi) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
+  constexpr bool FAST = HOOK == CHUNK_FAST;
+  constexpr bool TTA = HOOK <= CHUNK_CLAMP;  // the rounded chunk is added; else the running accumulator is rounded
   static_assert(FAST || SCHED == 0, "the interleaved schedules exist for the fast configuration only");
   typedef Mma<OP> MM;
   typedef typename MM::Frag Frag;
@@ -356,8 +364,7 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const Elem init = initial(i, j, v);
-            acc[i][j][v] = g.tta ? init : (Elem)0;
-            work[i][j][v] = g.tta ? (Elem)0 : init;
+            (TTA ? acc : work)[i][j][v] = init;
           }
   }
 
@@ -589,6 +596,7 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
     }
   } else {
     auto finish_chunk = [&]() __attribute__((always_inline)) {
+      if (!TTA && !g.post) return;
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -604,17 +612,11 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
                 acc[i][j][v] += __uint_as_float((__float_as_uint(work[i][j][v]) + g.round_bit) & g.mask);
             } else {
               Elem p = work[i][j][v];
-              if (g.post) {
-                if constexpr (std::is_same<Elem, int>::value) p = trunc_i32(p, g.lo, g.hi, (int)g.round_bit, g.t);
-                else p = trunc_f32(p, g.round_bit, g.mask, g.dl16);
-              }
-              if (g.tta) {
-                if constexpr (std::is_same<Elem, int>::value) acc[i][j][v] = (int)((unsigned)acc[i][j][v] + (unsigned)p);
-                else acc[i][j][v] += p;
-                work[i][j][v] = 0;
-              } else {
-                work[i][j][v] = p;  // the running accumulator itself is rounded
-              }
+              if constexpr (std::is_same<Elem, int>::value) p = trunc_i32(p, g.lo, g.hi, (int)g.round_bit, g.t);
+              else p = trunc_f32(p, g.round_bit, g.mask, HOOK != CHUNK_RUNNING);
+              if constexpr (!TTA) work[i][j][v] = p;
+              else if constexpr (std::is_same<Elem, int>::value) acc[i][j][v] = (int)((unsigned)acc[i][j][v] + (unsigned)p);
+              else acc[i][j][v] += p;
             }
           }
     };
@@ -625,9 +627,9 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
       }
     };
     auto mma_any = [&](const Frag* af, const Frag* bf) __attribute__((always_inline)) {
-      // first k-step of a chunk in FAST mode: the MFMA's C operand is the constant 0, so `work` needs
+      // first k-step of a chunk that is added: the MFMA's C operand is the constant 0, so `work` needs
       // no clearing between chunks
-      if (FAST && ks_cnt == 0) {
+      if (TTA && ks_cnt == 0) {
         Acc zero;
 #pragma unroll
         for (int v = 0; v < 16; ++v) zero[v] = 0;
@@ -665,7 +667,7 @@ __global__ __launch_bounds__(256, FAST ? 2 : 1) void chunk_tile_kernel(ChunkTile
       chunk_tick();
     }
     if (ks_cnt != 0) finish_chunk();  // K ended inside a chunk
-    if (!FAST && !g.tta) {
+    if constexpr (!TTA) {
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll

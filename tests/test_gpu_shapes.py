@@ -437,6 +437,26 @@ def test_chunked_products_at_the_edges_of_tiles_and_of_the_reduction(dev, M, N, 
         assert torch.equal(y.cpu(), ref.float()), (cs, t)
 
 
+@pytest.mark.parametrize("tta,dl16,bits", [(True, False, 14), (True, True, 32), (False, False, 32), (False, True, 32), (False, False, 14)])
+@pytest.mark.parametrize("M,N,Kd", [(1, 1, 16), (65, 131, 272), (130, 260, 1024)])   # K below, past and at the end of a stage
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn, torch.float16, torch.float32])
+def test_chunked_products_clamped_or_with_a_rounded_running_sum(dev, M, N, Kd, dtype, tta, dl16, bits):
+    """What is done at the end of a chunk beside the common configuration, with and without an initial accumulator, bits to
+    round or none: integer-valued operands whose sums stay below 2^24, exact in fp32 in any order (as in the test above)."""
+    a = torch.randint(-6, 7, (M, Kd), generator=gen(M + Kd)).float().to(dtype)
+    w = torch.randint(-6, 7, (N, Kd), generator=gen(N + Kd + 1)).float().to(dtype)
+    c0 = torch.randint(-999, 999, (M, N), generator=gen(5)).to(torch.int32 if dtype == torch.int8 else torch.float32)
+    for cs, t in ((32, 3), (64, 0), (256, 5)):
+        for c in (None, c0):
+            if dtype == torch.int8:
+                ref = O.chunk_matmul_i8(a, w, c, cs, t, bits, tta)
+            else:
+                ref = O.chunk_matmul_fp(a.float(), w.float(), c, cs, t, dl16, tta)
+            d = K().matmul_chunk(a.to(dev), w.to(dev), None if c is None else c.to(dev), chunk_size=cs, chunk_trun_bits=t,
+                                 max_acc_bits=bits, truncate_then_accumulate=tta, clamp_acc_to_dl16=dl16)
+            assert torch.equal(d.cpu(), ref), (cs, t, c is not None)
+
+
 @pytest.mark.parametrize("M,N,Kd,cs", [(16, 130, 8192, 64), (129, 100, 4112, 128), (40, 600, 4096 + 48, 32),
                                        (1100, 4096, 6144, 64),     # 288 tiles: whole ones and cut ones in one launch
                                        (70, 260, 6000, 4096)])     # few, long chunks
