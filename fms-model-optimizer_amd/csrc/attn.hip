@@ -578,6 +578,15 @@ extern "C" int fmsmo_affine_sum_parts(int64_t batch, int64_t R, int64_t C, int t
   return (int)((total + tiles - 1) / tiles);
 }
 
+// A product adds the parts itself where that is its kernel for a reduction of 128, and for a few query rows of a few
+// parts: every block adds them for its columns again (us from a HIP graph, launch of their own / inside, fp16, 8 heads:
+// 1 row, 4 parts 10.0 / 9.6, 8 parts 10.7 / 10.4, 23 parts 14.5 / 14.6, 32 parts 18.4 / 19.6; 4 parts, 8 rows 10.5 / 10.4,
+// 16 rows 10.8 / 11.3, 32 rows 11.8 / 13.2, 64 rows 13.5 / 16.9; 8 parts of 128 columns, 16 ... 64 rows within 2 %)
+extern "C" int fmsmo_affine_parts_first(int parts, int64_t M, int64_t N, int64_t K) {
+  const bool inside = (K == 128 && M > 128 && N > 128) || (M <= 8 && parts <= 8);
+  return parts > 1 && !inside;
+}
+
 extern "C" int fmsmo_affine_add_parts(int32_t* sums, int parts, int64_t n, fmsmo_stream_t stream) {
   if (!sums) return FMSMO_ERR_NULL;
   if (parts < 1 || n <= 0 || n > (1ll << 38)) return FMSMO_ERR_SHAPE;

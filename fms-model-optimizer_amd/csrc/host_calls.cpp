@@ -30,7 +30,7 @@ namespace {
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
   X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_grouped_gemm_i8_dq)                   \
   X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq) X(fmsmo_matmul_chunk_workspace_bytes)    \
-  X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
+  X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_parts_first) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
   X(fmsmo_bmm_qa_i8) X(fmsmo_bmm_i8_zp)
 #define DECLARE(f) decltype(&::f) p_##f = nullptr;
 ENTRIES(DECLARE)
@@ -447,10 +447,6 @@ bool affine(const at::Tensor& like, const void* x, int64_t ldx, int64_t stride, 
                 (int8_t*)c->q.data_ptr(), c->ld, rows * c->ld, want_sums ? (int32_t*)c->sums.data_ptr() : nullptr, B, R, C,
                 stream_of(like));
 }
-// The parts of the column sums are added up by a launch of their own, except where the product adds them: the kernel
-// for a reduction of 128, and a few query rows (us, launch of their own / inside: 1 row, 8 heads of 194 x 64 6.3 / 5.5, 32 of
-// 2048 x 128 11.3 / 10.9; 93 rows, 16 heads of 93 x 64 9.4 / 12.4)
-bool sums_added_first(int64_t M, int64_t N, int64_t K) { return M > 64 && (K != 128 || M <= 128 || N <= 128); }
 // (m1 [.., M, K], m2 [.., K, N], scale1, zero1, scale2, zero2, compute dtype) -> y [B, M, N]
 PyObject* bmm_quantized(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -497,7 +493,7 @@ PyObject* bmm_quantized(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
               m2->data_ptr(), by_rows ? K : N, N * K, s2, z2, by_rows ? 0 : 1, (int8_t*)q2.data_ptr(), N * ld, sums, N, K,
               ld, stream_of(*m1)))
     return nullptr;
-  if (parts > 1 && sums_added_first(M, N, ld)) {
+  if (p_fmsmo_affine_parts_first(parts, M, N, ld)) {
     if (!LAUNCH(fmsmo_affine_add_parts, sums, parts, B * N, stream_of(*m1))) return nullptr;
     parts = 1;
   }

@@ -96,6 +96,7 @@ OTHER = {
     "fmsmo_status_str": ([c_int], c_char_p),
     "fmsmo_last_error": ([], c_char_p),
     "fmsmo_affine_sum_parts": ([c_int64, c_int64, c_int64, c_int], c_int),
+    "fmsmo_affine_parts_first": ([c_int, c_int64, c_int64, c_int64], c_int),
     "fmsmo_bmm_qa_ok": ([c_int, c_int, c_float, c_float, c_int64, c_int64, c_int64, c_int64], c_int),
     "fmsmo_gemm_workspace_bytes": ([c_int64, c_int64, c_int64], c_int64),
     "fmsmo_gemm_fp8_workspace_bytes": ([c_int64, c_int64, c_int64], c_int64),

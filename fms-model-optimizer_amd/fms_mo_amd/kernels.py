@@ -775,8 +775,7 @@ def bmm_i8_quantized(m1, m2, scale1, zero1, scale2, zero2, compute_dtype):
         q1 = quant_i8_affine(a3, scale1, zero1, compute_dtype, False, pad)
     Kp, parts = q1.shape[2], sums.shape[0]
     with _dev(m1):
-        if parts > 1 and M > 64 and (Kp != 128 or M <= 128 or N <= 128):
-            # (a product of a few rows and the kernel for a reduction of 128 add the parts themselves)
+        if L.load().fmsmo_affine_parts_first(parts, M, N, Kp):   # (else the product adds the parts itself)
             L.call("fmsmo_affine_add_parts", sums.data_ptr(), parts, B * N, _stream(m1))
             parts = 1
         L.call("fmsmo_bmm_i8_zp", q1.data_ptr(), Kp, q2.data_ptr(), Kp, q2.stride(0),

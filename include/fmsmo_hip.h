@@ -717,8 +717,10 @@ int fmsmo_quant_i8_affine(const void* x, int x_dtype, int64_t ldx, int64_t strid
  * row of q adds nothing to its sum and no part to the sums.  x only needs the alignment of its elements.
  */
 int fmsmo_affine_sum_parts(int64_t batch, int64_t R, int64_t C, int transpose);
-/* Adds the parts up in the first one (n = batch * rows of q): fmsmo_bmm_i8_zp with parts = 1 is the faster. */
+/* Adds the parts up in the first one (n = batch * rows of q); fmsmo_affine_parts_first (host only): whether this and
+   fmsmo_bmm_i8_zp with parts = 1 take less time than fmsmo_bmm_i8_zp with all of them. */
 int fmsmo_affine_add_parts(int32_t* sums, int parts, int64_t n, fmsmo_stream_t stream);
+int fmsmo_affine_parts_first(int parts, int64_t M, int64_t N, int64_t K);
 int fmsmo_quant_i8_affine_sums(const void* x, int x_dtype, int64_t ldx, int64_t stride_x, float scale,
                                float offset, int compute_dtype, int transpose, int8_t* q, int64_t ldq,
                                int64_t stride_q, int32_t* sums, int64_t batch, int64_t R, int64_t C,

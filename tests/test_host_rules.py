@@ -109,3 +109,10 @@ def test_the_columns_cut_off_a_last_round_are_those_of_the_operand_type():
     assert kernels.gemm_plan(1700, 20992, 640)[1:3] == (128, 128) and kernels.gemm_plan(1700, 20992, 640, fp8=True)[1:3] == (256, 256)
     assert i8(2048, 25600, 4096) == fp8(2048, 25600, 4096) == 1024
     assert fp8(4096, 28672, 4096) == fp8(16, 25600, 4096) == fp8(0, 25600, 4096) == 0
+
+
+def test_parts_of_column_sums_are_added_first_but_for_a_few_rows_and_the_kernel_of_128():
+    first = L.load().fmsmo_affine_parts_first
+    assert not first(1, 1000, 64, 256) and not first(4, 1, 64, 256) and not first(8, 8, 64, 256)
+    assert first(4, 9, 64, 256) and first(9, 1, 64, 576) and first(32, 64, 128, 2048) and first(2, 128, 300, 128)
+    assert not first(2, 129, 129, 128) and first(2, 129, 128, 128) and first(2, 300, 300, 192)
