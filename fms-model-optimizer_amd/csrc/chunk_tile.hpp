@@ -243,7 +243,7 @@ constexpr int CHUNK_GROUP_M = 8;  // tile order: column-major in groups of as ma
 // fewer bits, floating point: to DL16), or the running accumulator itself is rounded, in floating point without or
 // with the DL16 clamp.  As constants: tested per element, and with the other form's accumulators in registers, these
 // kernels took 1.1 to 4 times as long (us, before -> after, chunk 64: fp16 running sum 435 x 857 x 1472 51.8 -> 17.4,
-// e4m3 333 x 56 x 7296 349 -> 100; chunk 32: int8 clamped to 20 bits 5 x 25 x 6720 277 -> 169, fp16 running sum with
+// e4m3 333 x 56 x 7296 349 -> 100; chunk 32: int8 clamped to 20 bits 5 x 25 x 6720 277 -> 192, fp16 running sum with
 // DL16 33 x 315 x 1568 149 -> 83).
 enum { CHUNK_FAST, CHUNK_CLAMP, CHUNK_RUNNING, CHUNK_RUNNING_DL16 };
 // KT: K is no multiple of a stage.
@@ -617,6 +617,7 @@ __global__ __launch_bounds__(256, HOOK == CHUNK_FAST ? 2 : 1) void chunk_tile_ke
               if constexpr (!TTA) work[i][j][v] = p;
               else if constexpr (std::is_same<Elem, int>::value) acc[i][j][v] = (int)((unsigned)acc[i][j][v] + (unsigned)p);
               else acc[i][j][v] += p;
+              if constexpr (TTA) work[i][j][v] = 0;
             }
           }
     };
@@ -627,9 +628,9 @@ __global__ __launch_bounds__(256, HOOK == CHUNK_FAST ? 2 : 1) void chunk_tile_ke
       }
     };
     auto mma_any = [&](const Frag* af, const Frag* bf) __attribute__((always_inline)) {
-      // first k-step of a chunk that is added: the MFMA's C operand is the constant 0, so `work` needs
+      // first k-step of a chunk in FAST mode: the MFMA's C operand is the constant 0, so `work` needs
       // no clearing between chunks
-      if (TTA && ks_cnt == 0) {
+      if (FAST && ks_cnt == 0) {
         Acc zero;
 #pragma unroll
         for (int v = 0; v < 16; ++v) zero[v] = 0;
