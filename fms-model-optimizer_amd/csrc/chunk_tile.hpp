@@ -242,14 +242,14 @@ constexpr int CHUNK_GROUP_M = 8;  // tile order: column-major in groups of as ma
 // What happens at the end of a chunk, beside the common configuration: a clamped chunk is folded (integers: to
 // fewer bits, floating point: to DL16), or the running accumulator itself is rounded, in floating point without or
 // with the DL16 clamp.  As constants: tested per element, and with the other form's accumulators in registers, these
-// kernels took 1.1 to 4 times as long (us, before -> after, chunk 64: fp16 running sum 435 x 857 x 1472 51.8 -> 17.4,
-// e4m3 333 x 56 x 7296 349 -> 100; chunk 32: int8 clamped to 20 bits 5 x 25 x 6720 277 -> 192, fp16 running sum with
-// DL16 33 x 315 x 1568 149 -> 83).
+// kernels needed more than 256 registers, ran one block per compute unit and copied their accumulators between the two
+// halves of the register file at every stage (us, before -> after, chunk 64: fp16 running sum 435 x 857 x 1472 51.8 ->
+// 16.9, e4m3 333 x 56 x 7296 349 -> 65; chunk 32: int8 clamped to 20 bits 5 x 25 x 6720 277 -> 164, fp16 running sum
+// with DL16 33 x 315 x 1568 149 -> 78).  Now 106 ... 178 registers.
 enum { CHUNK_FAST, CHUNK_CLAMP, CHUNK_RUNNING, CHUNK_RUNNING_DL16 };
 // KT: K is no multiple of a stage.
 template <int OP, int HOOK, int SCHED, bool KT>
-// (two blocks per compute unit for the fast configuration; the others would spill at 256 registers)
-__global__ __launch_bounds__(256, HOOK == CHUNK_FAST ? 2 : 1) void chunk_tile_kernel(ChunkTileArgs g, EpiChunk<typename Mma<OP>::Elem> epi) {
+__global__ __launch_bounds__(256, 2) void chunk_tile_kernel(ChunkTileArgs g, EpiChunk<typename Mma<OP>::Elem> epi) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
   constexpr bool FAST = HOOK == CHUNK_FAST;
   constexpr bool TTA = HOOK <= CHUNK_CLAMP;  // the rounded chunk is added; else the running accumulator is rounded
