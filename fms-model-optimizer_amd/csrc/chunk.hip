@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void chunk_matmul_kernel(ChunkArgs g, EpiChunk
 #pragma unroll
       for (int v = 0; v < 16; ++v) mine[((v >> 2) * 8 + fg * 4 + (v & 3)) * 64 + j * 32 + fr] = acc[i][j][v];
     __syncthreads();
-    chunk_finish(epi, mine, 32, row0 + wm * 64 + i * 32, col0 + wn * 64, g.M, g.N, lane);
+    chunk_finish<64>(epi, mine, 32, row0 + wm * 64 + i * 32, col0 + wn * 64, g.M, g.N, lane);
   }
 }
 
@@ -269,6 +269,17 @@ static ChunkPlan plan_chunk(int mma, int64_t M, int64_t N, int64_t Kb, int64_t c
   return p;
 }
 
+// fp32 accumulators add their chunks one after the other, so a reduction is not to be cut where the caller has not said
+// that it may be.  Up to two 64 x 64 tiles per compute unit take those instead: a wave then rounds and adds a quarter
+// as many elements per stage (us, 128 x 128 -> 64 x 64, the tiles of 64 in front, chunks one after the other, bits the
+// same: fp16 4, 47 x 231 x 6992 94.8 -> 48.6; 94, 107 x 2992 x 3584 55.0 -> 28.1; bf16 333, 151 x 7093 x 5760 71.7 -> 44.8;
+// e4m3 414, 1096 x 1439 x 4224 77.4 -> 35.5; fp32 152, 203 x 2372 x 3392 227 -> 74; with the DL16 clamp fp16 490, 632 x 3080
+// x 4432 267 -> 104; beyond: fp16 680, 603 x 4326 x 6848 103 -> 107, 837, 561 x 5895 x 5888 82 -> 113; of 105 launches up to
+// 490 tiles all faster, 0.43 in the mean).  int32 sums are cut (or take the interleaved schedules of the big tiles).
+static bool small_chunk_tiles(int64_t M, int64_t N) {
+  return (int64_t)div_up(M, 64) * div_up(N, 64) <= 512;
+}
+
 // Pipelined path.  Needs 32-bit row offsets (chunks are whole 32-byte k-steps: a power of two of at
 // least 32 bytes).
 static bool chunk_tile_ok(const ChunkArgs& c) {
@@ -280,7 +291,12 @@ static bool launch_chunk_tile(const ChunkArgs& c, const EpiChunk<AccT>& epi, voi
   ChunkTileArgs g{};
   g.a = c.a; g.b = c.b; g.lda = c.lda; g.ldb = c.ldb;
   g.M = c.M; g.N = c.N; g.K = c.Kb;
-  g.grid_m = div_up(c.M, 128); g.grid_n = div_up(c.N, 128);
+  const bool fast = c.tta && !c.dl16 && c.max_acc_bits >= 32;
+  const ChunkPlan p =
+      plan_chunk(MMA, c.M, c.N, c.Kb, c.chunk_bytes, c.tta && !c.c_in && ws, std::max<int64_t>(0, ws_bytes));
+  // (a size below zero is no room, not the query's "as much as it takes")
+  const int tile = MMA != MMA_I8 && c.tta && p.slices == 1 && small_chunk_tiles(c.M, c.N) ? 64 : 128;
+  g.grid_m = div_up(c.M, tile); g.grid_n = div_up(c.N, tile);
   g.chunk_ks = c.chunk_bytes / 32;
   g.t = c.dl16 ? 14 : c.trun_bits;
   g.round_bit = g.t > 0 ? 1u << (g.t - 1) : 0u;
@@ -289,13 +305,9 @@ static bool launch_chunk_tile(const ChunkArgs& c, const EpiChunk<AccT>& epi, voi
   g.hi = c.max_acc_bits < 32 ? (1 << (c.max_acc_bits - 1)) - 1 : 0x7fffffff;
   g.post = c.dl16 || g.t > 0 || c.max_acc_bits < 32;
   g.c_in = c.c_in; g.ldc = c.ldc;
-  // (a size below zero is no room, not the query's "as much as it takes")
-  const ChunkPlan p =
-      plan_chunk(MMA, c.M, c.N, c.Kb, c.chunk_bytes, c.tta && !c.c_in && ws, std::max<int64_t>(0, ws_bytes));
-  g.full = p.full; g.slices = p.slices; g.slice_len = p.slice_len; g.ws = ws;
-  const bool fast = c.tta && !c.dl16 && c.max_acc_bits >= 32;
-  const int tiles = g.grid_m * g.grid_n, cut = tiles - p.full;
-  const dim3 grid((unsigned)(p.full + cut * p.slices)), block(256);
+  g.full = tile == 64 ? g.grid_m * g.grid_n : p.full; g.slices = p.slices; g.slice_len = p.slice_len; g.ws = ws;
+  const int cut = g.grid_m * g.grid_n - g.full;
+  const dim3 grid((unsigned)(g.full + cut * p.slices)), block(256);
   auto go = [&](auto kt_c) {
     constexpr bool KT = decltype(kt_c)::value;
     // the schedules that round one block while the matrix unit multiplies the others: a chunk of one
@@ -305,6 +317,12 @@ static bool launch_chunk_tile(const ChunkArgs& c, const EpiChunk<AccT>& epi, voi
     };
     typedef std::integral_constant<int, CHUNK_FAST> Fast;
     typedef std::integral_constant<int, 0> S0;
+    if constexpr (MMA != MMA_I8)
+      if (tile == 64) {
+        if (fast) hipLaunchKernelGGL((chunk_tile_kernel<MMA, CHUNK_FAST, 0, KT, 64>), grid, block, 0, st, g, epi);
+        else hipLaunchKernelGGL((chunk_tile_kernel<MMA, CHUNK_CLAMP, 0, KT, 64>), grid, block, 0, st, g, epi);
+        return;
+      }
     if (!c.tta && c.dl16 && MMA != MMA_I8) {
       if constexpr (MMA != MMA_I8) run(std::integral_constant<int, CHUNK_RUNNING_DL16>{}, S0{});
     } else if (!c.tta) run(std::integral_constant<int, CHUNK_RUNNING>{}, S0{});

@@ -1,5 +1,5 @@
-// Pipelined kernel of the chunked reduced-precision-accumulation matmuls (see chunk.hip): 128 x 128
-// tiles, four waves of 64 x 64 (2 x 2 MFMA blocks of 32 x 32), K in stages of 64 bytes through a ring
+// Pipelined kernel of the chunked reduced-precision-accumulation matmuls (see chunk.hip): tiles of 128 x 128 or
+// 64 x 64, four waves (of 2 x 2 MFMA blocks of 32 x 32, or of one), K in stages of 64 bytes through a ring
 // of four LDS buffers that DMA loads fill three stages ahead, two blocks per compute unit.
 //
 // Every `chunk_ks` MFMA k-steps (32 bytes of K) the partial product is range-clamped / LSB-rounded on
@@ -178,12 +178,13 @@ struct EpiChunk {
 // dtypes were tested per element in a fully unrolled epilogue (us, before -> after, chunk 64: 1069 x 4096 x
 // 14336 139.6 -> 128.2, 300 x 4096 x 4096 39.3 -> 27.7, 1024 x 12000 x 2048 69.5 -> 46.0).
 //
-// A wave finishes `height` rows of 64 accumulators that lie in LDS row by row (rows m0 .., columns n0 ..
+// A wave finishes `height` rows of W accumulators that lie in LDS row by row (rows m0 .., columns n0 ..
 // of the result): a rolled loop, four neighbours of a row per lane, whole 128-byte lines of 16-bit results.
-template <class AccT>
+template <int W, class AccT>
 __device__ __forceinline__ void chunk_finish(const EpiChunk<AccT>& epi, const AccT* acc, int height, int m0, int n0,
                                              int M, int N, int lane) {
-  const int n = n0 + (lane & 15) * 4;
+  constexpr int LPR = W / 4;  // lanes per row
+  const int n = n0 + lane % LPR * 4;
   const int rows = min(height, M - m0);
   if (rows <= 0) return;
   const float as_all = epi.row(min(m0 + lane, M - 1));  // lane r holds the scale of row r
@@ -194,11 +195,11 @@ __device__ __forceinline__ void chunk_finish(const EpiChunk<AccT>& epi, const Ac
   epi.dispatch([&](auto mode_c, auto out_c) __attribute__((always_inline)) {
     constexpr int MODE = decltype(mode_c)::value, OUT = decltype(out_c)::value;
 #pragma unroll 1
-    for (int r0 = 0; r0 < rows; r0 += 4) {
-      const int r = r0 + (lane >> 4);
+    for (int r0 = 0; r0 < rows; r0 += 64 / LPR) {
+      const int r = r0 + lane / LPR;
       const float as = __shfl(as_all, r);
       AccT val[4];
-      *(v4i*)val = *(const v4i*)(acc + r * 64 + (lane & 15) * 4);
+      *(v4i*)val = *(const v4i*)(acc + r * W + lane % LPR * 4);
       uint32_t u[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) u[e] = epi.template bits<MODE, OUT>(val[e], as, cc[e]);
@@ -247,8 +248,8 @@ constexpr int CHUNK_GROUP_M = 8;  // tile order: column-major in groups of as ma
 // 16.9, e4m3 333 x 56 x 7296 349 -> 65; chunk 32: int8 clamped to 20 bits 5 x 25 x 6720 277 -> 164, fp16 running sum
 // with DL16 33 x 315 x 1568 149 -> 78).  Now 106 ... 178 registers.
 enum { CHUNK_FAST, CHUNK_CLAMP, CHUNK_RUNNING, CHUNK_RUNNING_DL16 };
-// KT: K is no multiple of a stage.
-template <int OP, int HOOK, int SCHED, bool KT>
+// KT: K is no multiple of a stage.  TILE: rows and columns of a block's tile.
+template <int OP, int HOOK, int SCHED, bool KT, int TILE = 128>
 __global__ __launch_bounds__(256, 2) void chunk_tile_kernel(ChunkTileArgs g, EpiChunk<typename Mma<OP>::Elem> epi) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
   constexpr bool FAST = HOOK == CHUNK_FAST;
@@ -259,14 +260,15 @@ __global__ __launch_bounds__(256, 2) void chunk_tile_kernel(ChunkTileArgs g, Epi
   typedef typename MM::Acc Acc;
   typedef typename MM::Elem Elem;
   static_assert(MM::KSTEP == 32, "a lane's operand of a k-step is one 16-byte chunk");
-  constexpr int BM = 128, BN = 128, BK = 64, NSTAGE = 4;
+  static_assert(TILE == 128 || SCHED == 0, "the interleaved schedules take four blocks per wave");
+  constexpr int BM = TILE, BN = TILE, BK = 64, NSTAGE = 4;
   constexpr int CPR = BK / 16, RPI = 256 / CPR;  // chunks per tile row, rows per block-wide load
   constexpr int NIA = BM / RPI, NIB = BN / RPI;
-  constexpr int TM = 64, TN = 64, FM = 2, FN = 2, NKS = 2;
+  constexpr int TM = BM / 2, TN = BN / 2, FM = TM / 32, FN = TN / 32, NKS = 2;
   constexpr int NMMA = FM * FN, NLD = NIA + NIB;
   constexpr int STAGE_BYTES = (BM + BN) * BK;
   __shared__ __attribute__((aligned(16))) uint8_t lds[NSTAGE * STAGE_BYTES];
-  static_assert(NSTAGE * STAGE_BYTES == BM * BN * 4, "the finished tile passes through the ring's buffers");
+  static_assert(NSTAGE * STAGE_BYTES >= BM * BN * 4, "the finished tile passes through the ring's buffers");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -706,7 +708,7 @@ __global__ __launch_bounds__(256, 2) void chunk_tile_kernel(ChunkTileArgs g, Epi
 #pragma unroll
       for (int v = 0; v < 16; ++v) mine[(i * 32 + (v >> 2) * 8 + fg * 4 + (v & 3)) * TN + j * 32 + fr] = acc[i][j][v];
   __syncthreads();
-  chunk_finish(epi, mine, TM, row_lo + wm * TM, col_lo + wn * TN, g.M, g.N, lane);
+  chunk_finish<TN>(epi, mine, TM, row_lo + wm * TM, col_lo + wn * TN, g.M, g.N, lane);
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

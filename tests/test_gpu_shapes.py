@@ -457,6 +457,29 @@ def test_chunked_products_clamped_or_with_a_rounded_running_sum(dev, M, N, Kd, d
             assert torch.equal(d.cpu(), ref), (cs, t, c is not None)
 
 
+@pytest.mark.parametrize("M,N", [(1030, 2050), (1024, 2048), (65, 129)])   # 561 and 512 tiles of 64 x 64, ragged ones
+@pytest.mark.parametrize("Kd", [272, 256])
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, torch.float16, torch.bfloat16, torch.float32])
+def test_chunked_products_in_floating_point_on_either_tile(dev, M, N, Kd, dtype):
+    """Both sides of the line between 64 x 64 and 128 x 128 tiles, every schedule and the DL16 clamp, an initial accumulator:
+    integer-valued operands, exact in fp32 in any order (as in the test above).  On real values a row has the same bits on
+    either tile."""
+    a = torch.randint(-6, 7, (M, Kd), generator=gen(M + Kd)).float().to(dtype)
+    w = torch.randint(-6, 7, (N, Kd), generator=gen(N + Kd + 1)).float().to(dtype)
+    c = torch.randint(-999, 999, (M, N), generator=gen(5)).float()
+    esz = a.element_size()
+    for cs, t, dl16, c0 in ((64 // esz, 4, False, None), (128 // esz, 0, False, c), (256 // esz, 5, True, None), (64 // esz, 3, True, c)):
+        cs = max(cs, 32 if esz == 1 else 16)
+        ref = O.chunk_matmul_fp(a.float(), w.float(), c0, cs, t, dl16)
+        d = K().matmul_chunk(a.to(dev), w.to(dev), None if c0 is None else c0.to(dev), chunk_size=cs, chunk_trun_bits=t,
+                             clamp_acc_to_dl16=dl16)
+        assert torch.equal(d.cpu(), ref), (cs, t, dl16)
+    a, w = (torch.randn(s, Kd, generator=gen(s)).to(dtype).to(dev) for s in (1030, 2050))
+    for dl16 in (False, True):
+        big = K().matmul_chunk(a, w, None, chunk_size=64, chunk_trun_bits=5, clamp_acc_to_dl16=dl16)
+        assert torch.equal(K().matmul_chunk(a[:M], w[:N], None, chunk_size=64, chunk_trun_bits=5, clamp_acc_to_dl16=dl16), big[:M, :N])
+
+
 @pytest.mark.parametrize("M,N,Kd,cs", [(16, 130, 8192, 64), (129, 100, 4112, 128), (40, 600, 4096 + 48, 32),
                                        (1100, 4096, 6144, 64),     # 288 tiles: whole ones and cut ones in one launch
                                        (70, 260, 6000, 4096)])     # few, long chunks
