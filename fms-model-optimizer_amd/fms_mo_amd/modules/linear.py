@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import json
 import logging
+import weakref
 
 import torch
 import torch.nn.functional as F
@@ -99,6 +100,12 @@ class _Kept(tuple):
 
     def __reduce__(self):
         return _Kept, ()
+
+
+def _kept_of(kept, key, weight):
+    """Is this the finding for `key` and this very weight tensor?  (Weights are held weakly, beside the aliases: their
+    memory is not to be kept for a finding.)"""
+    return type(kept) is _Kept and len(kept) > 0 and kept[0] == key and kept[-1][0]() is weight
 
 
 def _stamp(t):
@@ -230,8 +237,8 @@ class QLinear(nn.Linear):
             self.register_buffer("smoothq_act_scale", torch.zeros(self.weight.shape[1]))
             self.register_buffer("smoothq_alpha",
                                  torch.tensor([qcfg.get("smoothq_alpha", 0.5)], dtype=torch.float32))
-        self._wcache = None   # (key, quantized weights, weight scales) of the eval-mode kernel paths
-        self._sqcache = None  # (key, SmoothQuant scale or None)
+        self._wcache = _Kept()   # key, quantized weights, weight scales of the eval-mode kernel paths, what they are of
+        self._sqcache = _Kept()  # key, SmoothQuant scale or None, what it is of
         self._sq_gen = 0
 
     # -- SmoothQuant ------------------------------------------------------------------------
@@ -255,15 +262,17 @@ class QLinear(nn.Linear):
         a, al, w = self.smoothq_act_scale, self.smoothq_alpha, self.weight
         key = (a.data_ptr(), a._version, w.data_ptr(), w._version, x.dtype, x.device,
                (al.data_ptr(), al._version) if torch.is_tensor(al) else al)
-        if self._sqcache is None or self._sqcache[0] != key:
+        kept = self._sqcache
+        if not _kept_of(kept, key, w):
             # detached and built outside autograd: the cached tensor serves the kernel paths and
             # no-grad evaluation only (forward() recomputes the scale inside the graph whenever a
             # gradient can flow through it, as the reference does on every call)
             with torch.no_grad():
                 scale = self.get_smoothq_scale(x).detach()
             self._sq_gen += 1  # names this scale in the keys of the weight caches
-            self._sqcache = (key, scale if scale.numel() > 1 else None)
-        return self._sqcache[1]
+            small = [t.detach() for t in (a, al) if torch.is_tensor(t)]
+            self._sqcache = kept = _Kept((key, scale if scale.numel() > 1 else None, (weakref.ref(w), small)))
+        return kept[1]
 
     # -- forward ----------------------------------------------------------------------------
     def _eval_path_ok(self, x):
@@ -302,8 +311,9 @@ class QLinear(nn.Linear):
         quantizer defines the grid (eval-mode semantics)."""
         qw = self.quantize_weight
         key = self._weights_key(scale) + (qw.clip_val._version, qw.clip_val.data_ptr())
-        if self._wcache is not None and self._wcache[0] == key:
-            return self._wcache[1], self._wcache[2]
+        kept = self._wcache
+        if _kept_of(kept, key, self.weight):
+            return kept[1], kept[2]
         with torch.no_grad():
             cv = qw.clip_val.to(self.weight.device).float()
             w_scale = cv * 2 / 254
@@ -320,8 +330,9 @@ class QLinear(nn.Linear):
                 ws = self.weight if scale is None else self.weight * scale
                 u = ws.mul(1 / cv.to(ws.dtype)).clamp(-1, 1).mul(0.5).add(0.5)
                 w_int8 = (torch.round(254 * u) - 127).to(torch.int8).contiguous()
-        self._wcache = (key, w_int8, w_scale.float().reshape(-1))
-        return w_int8, self._wcache[2]
+        w_scale = w_scale.float().reshape(-1)
+        self._wcache = _Kept((key, w_int8, w_scale, (weakref.ref(self.weight), qw.clip_val.detach())))
+        return w_int8, w_scale
 
     @staticmethod
     def _fp8_mode(q):
@@ -333,15 +344,16 @@ class QLinear(nn.Linear):
         """e4m3 codes of the emulation quantizer's W*scale and their dequantizing factors, cached
         like the integer weights."""
         key = self._weights_key(scale) + ("fp8", self.quantize_weight.q_mode)
-        if self._wcache is not None and self._wcache[0] == key:
-            return self._wcache[1], self._wcache[2]
+        kept = self._wcache
+        if _kept_of(kept, key, self.weight):
+            return kept[1], kept[2]
         with torch.no_grad():
             ws = self.weight.detach() if scale is None else self.weight.detach() * scale
             _, q, _, inv = kernels.fake_quant_fp8(ws, self._fp8_mode(self.quantize_weight),
                                                   want_values=False, want_codes=True)
             if inv is None:
                 inv = torch.ones(1, dtype=torch.float32, device=ws.device)
-        self._wcache = (key, q, inv)
+        self._wcache = _Kept((key, q, inv, (weakref.ref(self.weight),)))
         return q, inv
 
     def forward(self, x):

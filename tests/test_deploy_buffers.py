@@ -1,4 +1,4 @@
-"""What a deployed linear finds out about its buffers is asked again when another buffer takes their place."""
+"""What a linear finds out about its tensors is asked again when another one takes their place."""
 import copy
 import io
 
@@ -72,3 +72,44 @@ def test_copies_and_pickles_ask_for_themselves():
         c.w_scale.mul_(2)
         assert c._w_scale_f32().tolist() == c.w_scale.float().tolist() != m._w_scale_f32().tolist()
         assert c._smoothq_active() is m._smoothq_active() is True
+
+
+def test_quantized_weights_and_smoothquant_scale_of_a_weight_in_the_memory_of_the_one_before():
+    """The eval-mode caches of a QLinear: another weight, another statistic, another clip value of version 0 where the old
+    one lay; what was quantized for the old weight is not kept for the new one."""
+    m = QLinear(64, 48, bias=False, num_bits_feature=8, qa_mode="pertokenmax", num_bits_weight=8, qw_mode="max",
+                qcfg={"smoothq": True}, device="cpu").eval()
+    with torch.no_grad():
+        m.weight.normal_(0, 0.02)
+        m.quantize_weight.clip_val.fill_(0.1)
+        m.smoothq_act_scale.copy_(torch.rand(64) + 0.5)
+    x = torch.zeros(1, 64)
+
+    def check():
+        scale = m._cached_smoothq_scale(x)
+        q, s = m._int_weights(scale)
+        fresh = copy.deepcopy(m)
+        assert not fresh._wcache and not fresh._sqcache
+        scale2 = fresh._cached_smoothq_scale(x)
+        q2, s2 = fresh._int_weights(scale2)
+        assert torch.equal(scale, scale2) and torch.equal(q, q2) and torch.equal(s, s2)
+        assert m._int_weights(m._cached_smoothq_scale(x))[0] is q      # asked once
+        return q
+
+    def replace(held, name, values, wrap=lambda t: t):
+        address, held[name] = held[name].data_ptr(), None
+        tried = [torch.empty(values.shape)]
+        while tried[-1].data_ptr() != address and len(tried) < 64:
+            tried.append(torch.empty(values.shape))
+        tried[-1].numpy()[...] = values.numpy()
+        held[name] = wrap(tried[-1])
+
+    for i in range(6):
+        q = check()
+        replace(m._parameters, "weight", torch.randn(48, 64) * 0.02, lambda t: torch.nn.Parameter(t))
+        assert not torch.equal(check(), q)
+        replace(m._buffers, "smoothq_act_scale", torch.rand(64) + 0.5)
+        check()
+        with torch.no_grad():
+            m.weight.mul_(0.5)
+        check()
