@@ -57,8 +57,8 @@ class QBmmINT8Deploy(nn.Module):
         return qbmm_int.to(target_device)
 
     # host copies of the four scalars, read again when a buffer is replaced or written to (load_state_dict,
-    # copy_, .to(), .half()), so that forward does not synchronize.  (The buffers are kept beside the copies: an
-    # id or address alone could come back with other contents.  Tensors made in inference mode count no
+    # copy_, .to(), .half()), so that forward does not synchronize.  (The buffers and aliases of their memory are kept
+    # beside the copies: an id or address alone could come back with other contents.  Tensors made in inference mode count no
     # versions, and writes through .data are not counted either.)
     def _scalars(self):
         b = self._buffers
@@ -74,7 +74,7 @@ class QBmmINT8Deploy(nn.Module):
             if k[0] is s1 and k[1] is z1 and k[2] is s2 and k[3] is z2:
                 return kept[2]
         host = (float(s1), int(z1) - 128, float(s2), int(z2))
-        self._kept = (bufs, state, host)
+        self._kept = (bufs, state, host, [t.detach() for t in bufs])
         return host
 
     def _get_name(self):

@@ -1,6 +1,7 @@
 """What a linear finds out about its tensors is asked again when another one takes their place."""
 import copy
 import io
+import types
 
 import pytest
 import torch
@@ -113,3 +114,26 @@ def test_quantized_weights_and_smoothquant_scale_of_a_weight_in_the_memory_of_th
         with torch.no_grad():
             m.weight.mul_(0.5)
         check()
+
+
+def test_attention_scalars_assigned_twice_through_data():
+    """Two assignments with no forward in between: the second may lie where the first buffer lay, in the same tensor."""
+    from fms_mo_amd.modules.bmm import QBmmINT8Deploy
+
+    one = lambda v: torch.tensor([v])  # noqa: E731
+    src = types.SimpleNamespace(num_bits_m1=8, num_bits_m2=8, qm1_mode="max",
+                                quantize_m1=types.SimpleNamespace(clip_val=one(4.0), clip_valn=one(-4.0), num_bits=8),
+                                quantize_m2=types.SimpleNamespace(clip_val=one(4.0), num_bits=8))
+    m = QBmmINT8Deploy.from_fms_mo(src, target_device="cpu")
+    m.m2_scale.data = one(1.0)
+    for i in range(100):
+        assert m._scalars()[2] == float(m.m2_scale)
+        address = m.m2_scale.data_ptr()
+        m.m2_scale.data = torch.empty(1)
+        tried = []
+        while not tried or (tried[-1].data_ptr() != address and len(tried) < 200):
+            tried.append(torch.empty(1))
+        tried[-1].numpy()[...] = 20.0 + i
+        m.m2_scale.data = tried[-1]
+        del tried
+        assert m._scalars()[2] == 20.0 + i
