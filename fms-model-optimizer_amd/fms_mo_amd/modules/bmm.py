@@ -16,6 +16,7 @@ import torch
 from torch import nn
 
 from .. import kernels
+from .linear import _Kept
 
 
 class QBmmINT8Deploy(nn.Module):
@@ -59,7 +60,7 @@ class QBmmINT8Deploy(nn.Module):
     # host copies of the four scalars, read again when a buffer is replaced or written to (load_state_dict,
     # copy_, .to(), .half()), so that forward does not synchronize.  (The buffers and aliases of their memory are kept
     # beside the copies: an id or address alone could come back with other contents.  Tensors made in inference mode count no
-    # versions, and writes through .data are not counted either.)
+    # versions, and writes through .data are not counted either.  Copies and pickles start without.)
     def _scalars(self):
         b = self._buffers
         s1, z1, s2, z2 = bufs = b["m1_scale"], b["m1_zp"], b["m2_scale"], b["m2_zp"]
@@ -69,12 +70,12 @@ class QBmmINT8Deploy(nn.Module):
         except RuntimeError:  # an inference tensor
             state = tuple((t.data_ptr(), -1 if t.is_inference() else t._version) for t in bufs)
         kept = self.__dict__.get("_kept")
-        if kept is not None and kept[1] == state:
+        if kept and kept[1] == state:
             k = kept[0]
             if k[0] is s1 and k[1] is z1 and k[2] is s2 and k[3] is z2:
                 return kept[2]
         host = (float(s1), int(z1) - 128, float(s2), int(z2))
-        self._kept = (bufs, state, host, [t.detach() for t in bufs])
+        self._kept = _Kept((bufs, state, host, [t.detach() for t in bufs]))
         return host
 
     def _get_name(self):

@@ -91,7 +91,7 @@ def _weight_column_max(w):
 
 
 class _Kept(tuple):
-    """What a module has found out about small tensors of its own: (stamp, finding, aliases).  The aliases keep the
+    """What a module has found out about small tensors of its own: a stamp, the finding, aliases.  The aliases keep the
     tensors' memory, without which a stamp could come back with other contents: a buffer that is freed and one that
     is allocated in its place share address, type and version.  Copies and pickles of a module start without."""
 

@@ -58,3 +58,15 @@ def test_scalars_of_copies_and_of_inference_tensors():
     with torch.inference_mode():
         i = make()
         assert i._scalars() == want(i)
+
+
+def test_copies_do_not_take_the_scalars_of_the_module_they_came_from():
+    """Its buffers' memory, written to and given to the copy, has the addresses and versions of its finding."""
+    m = copy.deepcopy(make())   # (a copy's buffers begin at version 1, those of a copy of it too)
+    m._scalars()
+    memory = [m._buffers[n].detach() for n in ("m1_scale", "m1_zp", "m2_scale", "m2_zp")]
+    c = copy.deepcopy(m)
+    memory[2].fill_(9.0)
+    for n, t in zip(("m1_scale", "m1_zp", "m2_scale", "m2_zp"), memory):
+        c._buffers[n].data = t
+    assert c._scalars() == want(c) and c._scalars()[2] == 9.0
