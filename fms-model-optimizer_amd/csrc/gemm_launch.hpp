@@ -48,13 +48,15 @@ struct TileMid { static constexpr int BM = 128, BN = 128, BK = 64, NST = 4, WGM 
 struct TileMidK { static constexpr int BM = 128, BN = 128, BK = 128, NST = 4, WGM = 2, WGN = 2; };
 struct TileTallK { static constexpr int BM = 128, BN = 64, BK = 128, NST = 5, WGM = 2, WGN = 2; };
 // The two with eight waves, two per SIMD, which fill each other's waits at barriers and for fragments: e4m3 and, below this K,
-// int8, whose longer loops four waves run 1 ... 3 % faster.  us, weights in the cache | from HBM, four waves -> eight:
+// int8, whose longer loops four waves run up to 3 % faster.  us, weights in the cache | from HBM, four waves -> eight:
 //   128 x 128, e4m3: 777 x 4096 x 12800 47.9 -> 45.0 | 51.0 -> 49.2, 777 x 4096 x 4096 18.9 -> 17.0 | 20.5 -> 19.9, 1400 x 2560 x 1024 8.7 -> 7.0 |
 //   9.7 -> 9.0; int8: 1400 x 2560 x 1024 8.2 -> 7.2 | 9.6 -> 8.7, 777 x 4096 x 4096 18.4 -> 18.2 | 20.7 -> 20.2, K = 7168 32.4 -> 32.7 | 34.2 -> 34.0,
 //   12800 49.5 -> 50.0 | 51.9 -> 52.1 (2 x 4 waves instead of 4 x 2: up to 5 % behind four)
 //   128 x 64, e4m3: 100 x 13824 x 5120 17.0 -> 16.4 | 27.0 -> 24.9, 1000 x 2048 x 2048 8.5 -> 7.5 | 10.4 -> 9.8; int8: 100 x 13824 x 5120 17.3 ->
 //   16.9 | 25.1 -> 24.5, 2000 x 640 x 1024 6.6 -> 6.1 | 7.4 -> 7.0, 200 x 8192 x 6144 19.9 -> 20.1 | 22.6 -> 22.5, 1300 x 1280 x 8192 22.7 -> 23.3 |
 //   24.5 -> 25.2
+//   int8, eight waves' time over four's, in the mean of 150 launches of one round and at most, K below 1536 | 2304 | 4096 | 6144: 128 x 128
+//   0.84 | 0.87 | 0.91 | 0.95, at most 1.001; 128 x 64 (from 1536 on) 0.96 | 0.98 | 1.00, at most 1.016
 constexpr int I8_EIGHT_WAVES_BELOW = 6144;
 struct TileMidK8 { static constexpr int BM = 128, BN = 128, BK = 128, NST = 4, WGM = 4, WGN = 2; };
 struct TileTallK8 { static constexpr int BM = 128, BN = 64, BK = 128, NST = 5, WGM = 4, WGN = 2; };
