@@ -578,12 +578,15 @@ extern "C" int fmsmo_affine_sum_parts(int64_t batch, int64_t R, int64_t C, int t
   return (int)((total + tiles - 1) / tiles);
 }
 
-// A product adds the parts itself where that is its kernel for a reduction of 128, and for a few query rows of a few
-// parts: every block adds them for its columns again (us from a HIP graph, launch of their own / inside, fp16, 8 heads:
-// 1 row, 4 parts 10.0 / 9.6, 8 parts 10.7 / 10.4, 23 parts 14.5 / 14.6, 32 parts 18.4 / 19.6; 4 parts, 8 rows 10.5 / 10.4,
-// 16 rows 10.8 / 11.3, 32 rows 11.8 / 13.2, 64 rows 13.5 / 16.9; 8 parts of 128 columns, 16 ... 64 rows within 2 %)
+// A product adds the parts itself where that is its kernel for a reduction of 128, and for a few query rows: every block
+// adds them for its columns again, which takes longer with the rows and the parts, and a launch of their own takes the host 3 us,
+// by which an eager call of a few rows is bound: one query, 12 heads, scores and values, launch of their own / inside: 864 x 128
+// 37.0 / 33.8 us, 587 x 80 38.6 / 34.7.  Device alone (us from a HIP graph, fp16, 8 heads, one product; 64 columns of values
+// where not said): 1 row, 4 parts 10.3 / 9.8, 8 parts 11.0 / 10.6, 21 parts 14.6 / 14.5, 32 parts 17.4 / 17.7, of 128 columns 18.8 / 20.0;
+// 8 rows, 4 parts 10.5 / 10.4, 32 parts 17.8 / 18.6; 16 rows, 4 parts 10.8 / 11.5, 32 parts 18.1 / 19.6; 32 rows 11.8 / 13.2,
+// 19.2 / 21.4; 64 rows, 4 parts 13.5 / 16.9
 extern "C" int fmsmo_affine_parts_first(int parts, int64_t M, int64_t N, int64_t K) {
-  const bool inside = (K == 128 && M > 128 && N > 128) || (M <= 8 && parts <= 8);
+  const bool inside = (K == 128 && M > 128 && N > 128) || (M <= 8 && parts <= 32);
   return parts > 1 && !inside;
 }
 

@@ -113,6 +113,6 @@ def test_the_columns_cut_off_a_last_round_are_those_of_the_operand_type():
 
 def test_parts_of_column_sums_are_added_first_but_for_a_few_rows_and_the_kernel_of_128():
     first = L.load().fmsmo_affine_parts_first
-    assert not first(1, 1000, 64, 256) and not first(4, 1, 64, 256) and not first(8, 8, 64, 256)
-    assert first(4, 9, 64, 256) and first(9, 1, 64, 576) and first(32, 64, 128, 2048) and first(2, 128, 300, 128)
+    assert not first(1, 1000, 64, 256) and not first(4, 1, 64, 256) and not first(8, 8, 64, 256) and not first(32, 8, 128, 2048)
+    assert first(4, 9, 64, 256) and first(33, 1, 64, 2112) and first(32, 64, 128, 2048) and first(2, 128, 300, 128)
     assert not first(2, 129, 129, 128) and first(2, 129, 128, 128) and first(2, 300, 300, 192)
