@@ -193,11 +193,12 @@ extern "C" int fmsmo_gemm_i8_dq_noalloc(const int8_t* a, int64_t lda, const int8
                          epilogue, y, y_dtype, ldy, M, N, K, ws, need, stream);
 }
 
+static bool any_takes(int64_t M, int64_t N, int64_t K) { return !fmsmo_gemv_batch_ok(M, K) && fmsmo_gemv_any_ok(M, N, K); }
 extern "C" int64_t fmsmo_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  return plan_split_k(M, N, K).ws_bytes;
+  return any_takes(M, N, K) ? 0 : plan_split_k(M, N, K).ws_bytes;
 }
 extern "C" int64_t fmsmo_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  return plan_split_k(M, N, K, 0, true).ws_bytes;
+  return any_takes(M, N, K) ? 0 : plan_split_k(M, N, K, 0, true).ws_bytes;
 }
 
 static int64_t gemm_tail_columns(bool fp8, int64_t M, int64_t N, int64_t K) {

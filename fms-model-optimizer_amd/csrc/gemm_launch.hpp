@@ -14,6 +14,7 @@ int fmsmo_check_launch();
 // block 0's clock readings (null = off); defined in gemm.hip.
 unsigned long long*& fmsmo_clock_probe();
 bool fmsmo_gemv_batch_ok(int64_t M, int64_t K);
+bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K);
 int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64_t ldb,
                         const float* a_scale, int64_t a_scale_n, const float* w_scale,
                         int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
@@ -96,7 +97,7 @@ inline bool use_small_tiles(int64_t M, int64_t N, int64_t K) {
 }
 // The decode kernels take the launch.
 inline bool use_decode(int64_t M, int64_t N, int64_t K) {
-  return (M <= 16 && K % 128 == 0) || (fmsmo_gemv_batch_ok(M, K) && !use_small_tiles(M, N, K));
+  return fmsmo_gemv_batch_ok(M, K) ? !use_small_tiles(M, N, K) : fmsmo_gemv_any_ok(M, N, K);
 }
 
 // A few hundred rows through a projection whose 128 x 64 tiles fill half a round of the 256

@@ -28,7 +28,7 @@ namespace {
   X(fmsmo_quant_act_fp8_pertoken) X(fmsmo_quant_act_fp8_dynamic) X(fmsmo_quant_act_fp8_tensor)           \
   X(fmsmo_quant_act_i8_pertoken_clips) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
-  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_grouped_gemm_i8_dq)                   \
+  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_small_linear_ok) X(fmsmo_small_linear_i8) X(fmsmo_small_linear_fp8) X(fmsmo_grouped_gemm_i8_dq)                   \
   X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq) X(fmsmo_matmul_chunk_workspace_bytes)    \
   X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_parts_first) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
   X(fmsmo_bmm_qa_i8) X(fmsmo_bmm_i8_zp)
@@ -600,7 +600,9 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool f32s = smooth && sm.st == at::kFloat;
   const bool one = (!smooth || sm.st == xt || f32s) &&
                    (f32s ? p_fmsmo_decode_linear_f32s_ok(x.rows, x.cols) : p_fmsmo_decode_linear_ok(x.rows, x.cols));
-  if (one || smooth) s = empty({x.rows, 1}, at::kFloat, *x.t);
+  const bool small = !one && (!smooth || sm.st == xt || f32s) && w.rows * w.ld < (1ll << 31) &&
+                     p_fmsmo_small_linear_ok(x.rows, w.rows, x.cols, f32s);
+  if (one || smooth || small) s = empty({x.rows, 1}, at::kFloat, *x.t);
   if (one) {
     // decode step of a few tokens: quantizer and weight-streaming matmul in one launch
     if (!run_decode_i8(x, sm, 0, w, *ws, b, FMSMO_EPI_REF_F16, y, s)) return nullptr;
@@ -613,7 +615,14 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         return none();
     }
     at::Tensor q, c;
-    if (smooth) {
+    if (small) {  // quantizer and product in one launch, the clip values from it too
+      if (!smooth) c = empty({2, x.rows, 1}, at::kFloat, *x.t);
+      if (!LAUNCH(fmsmo_small_linear_i8, x.p, code_of(xt), x.ld, sm.p, sm.dt, (const int8_t*)w.p, w.ld,
+                  (const float*)ws->data_ptr(), ws->numel(), b.p, b.dt, FMSMO_EPI_REF_F16, y.data_ptr(),
+                  code_of(y.scalar_type()), w.rows, (float*)s.data_ptr(), smooth ? nullptr : (float*)c.data_ptr(), x.rows,
+                  w.rows, x.cols, stream_of(*x.t)))
+        return nullptr;
+    } else if (smooth) {
       q = empty({x.rows, x.cols}, at::kChar, *x.t);
       if (!LAUNCH(fmsmo_quant_act_i8_pertoken, x.p, code_of(xt), x.ld, sm.p, sm.dt, code_of(promoted(xt, sm.st)), 0,
                   (int8_t*)q.data_ptr(), x.cols, (float*)s.data_ptr(), x.rows, x.cols, stream_of(*x.t)))
@@ -621,8 +630,8 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     } else if (!codes_and_clips(x, &q, &s, &c)) {
       return nullptr;
     }
-    if (!run_gemm_i8((const char*)q.data_ptr(), x.cols, w, (const float*)s.data_ptr(), x.rows, *ws, b, FMSMO_EPI_REF_F16,
-                     y, x.rows, x.cols))
+    if (!small && !run_gemm_i8((const char*)q.data_ptr(), x.cols, w, (const float*)s.data_ptr(), x.rows, *ws, b,
+                               FMSMO_EPI_REF_F16, y, x.rows, x.cols))
       return nullptr;
     PyObject* cvs = smooth ? nullptr : item(self, k_cvs);
     if (cvs && PyList_CheckExact(cvs) && PyList_GET_SIZE(cvs) >= 2) {
@@ -666,10 +675,11 @@ PyObject* fp8_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   ws = &own_ws;
   const float* wp = (const float*)ws->data_ptr();
   at::Tensor y = out_like(*x.t, w.rows, xt);
-  if (!per_tensor && floor == 1e-12 && !in_x && xt != at::kFloat && p_fmsmo_decode_linear_ok(x.rows, x.cols)) {
-    at::Tensor s = empty({x.rows}, at::kFloat, *x.t);
-    if (!LAUNCH(fmsmo_decode_linear_fp8, x.p, code_of(xt), x.ld, (const uint8_t*)w.p, w.ld, wp, ws->numel(), b.p, b.dt,
-                y.data_ptr(), code_of(xt), w.rows, (float*)s.data_ptr(), x.rows, w.rows, x.cols, stream_of(*x.t)))
+  if (!per_tensor && floor == 1e-12 && !in_x && xt != at::kFloat &&
+      (p_fmsmo_decode_linear_ok(x.rows, x.cols) ||
+       (w.rows * w.ld < (1ll << 31) && p_fmsmo_small_linear_ok(x.rows, w.rows, x.cols, 0)))) {
+    if (!LAUNCH(fmsmo_small_linear_fp8, x.p, code_of(xt), x.ld, (const uint8_t*)w.p, w.ld, wp, ws->numel(), b.p, b.dt,
+                y.data_ptr(), code_of(xt), w.rows, (float*)nullptr, x.rows, w.rows, x.cols, stream_of(*x.t)))
       return nullptr;
     return wrap(y);
   }

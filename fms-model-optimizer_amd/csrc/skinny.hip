@@ -12,33 +12,9 @@
 //     do the dot products, so the vector ALUs stay free and the loop is pure load + MFMA;
 //   * the NW partial 16x16 blocks are reduced through LDS and dequantized by the first 256
 //     threads.
-#include "quant_math.hpp"
+#include "gemv_args.hpp"
 
 namespace fmsmo {
-
-struct GemvArgs {
-  const uint8_t* a;  // [M,K] quantized activations
-  const uint8_t* b;  // [N,K] quantized weights
-  int64_t lda, ldb;
-  int M, N, K;
-  const float* a_scale;
-  const float* w_scale;
-  int a_stride, w_stride;
-  const void* bias;
-  int bias_dtype;
-  int epi;  // FMSMO_EPI_*
-  void* y;
-  int y_dtype;
-  int64_t ldy;
-  // fused decode linear: the activations arrive unquantized (fp16 / bf16) and every block
-  // quantizes them itself
-  const u16* x16;       // [M,K]
-  int64_t ldx;
-  const u16* smooth;    // [K] SmoothQuant divisors of x's dtype (fp32 when smooth_f32), or NULL
-  int smooth_f32;
-  int saturate;
-  float* a_scale_out;   // [M] per-token scales (written by block 0), or NULL
-};
 
 // Per-token int8 quantization of up to MAXM token rows by all NT threads of a block, into LDS:
 // the arithmetic of the stand-alone quantizer for a 16-bit compute dtype T (divide by the
@@ -128,7 +104,7 @@ __device__ __forceinline__ void quantize_rows_to_lds(const GemvArgs& g, uint8_t 
     }
   }
   __syncthreads();
-  if (blockIdx.x == 0 && g.a_scale_out && threadIdx.x < g.M) g.a_scale_out[threadIdx.x] = sc[threadIdx.x];
+  gemv_put_scales(g, sc);
 }
 
 // The FP8Linear recipe for one token row by all NT threads of a block, into LDS:
@@ -193,7 +169,7 @@ __device__ __forceinline__ void quantize_row_fp8_to_lds(const GemvArgs& g, uint8
     }
   }
   __syncthreads();
-  if (blockIdx.x == 0 && g.a_scale_out && threadIdx.x == 0) g.a_scale_out[0] = sc[0];
+  gemv_put_scales(g, sc);
 }
 
 // The two quantizers above for up to MAXM token rows of KROW elements, split in two so that the
@@ -339,7 +315,7 @@ __device__ __forceinline__ void rows_finish_i8(const GemvArgs& g, v4i (&cur)[P::
     }
   }
   __syncthreads();
-  if (blockIdx.x == 0 && g.a_scale_out && (int)threadIdx.x < g.M) g.a_scale_out[threadIdx.x] = sc[threadIdx.x];
+  gemv_put_scales(g, sc);
 }
 
 // fp32 SmoothQuant divisors: torch promotes x / smooth to fp32 and the whole quantizer then runs in
@@ -500,7 +476,7 @@ __device__ __forceinline__ void rows_finish_i8_f32s(const GemvArgs& g, const v4i
     }
   }
   __syncthreads();
-  if (blockIdx.x == 0 && g.a_scale_out && (int)threadIdx.x < g.M) g.a_scale_out[threadIdx.x] = sc[threadIdx.x];
+  gemv_put_scales(g, sc);
 }
 
 template <int XT, class P>
@@ -568,97 +544,54 @@ __device__ __forceinline__ void rows_finish_fp8(const GemvArgs& g, const v4i (&c
     }
   }
   __syncthreads();
-  if (blockIdx.x == 0 && g.a_scale_out && (int)threadIdx.x < g.M) g.a_scale_out[threadIdx.x] = sc[threadIdx.x];
+  gemv_put_scales(g, sc);
 }
 
-template <int OP, int RG, int NW>
+// Any K that is a multiple of 128 NW, 64-bit addresses: for operands past the 32-bit offsets of the other kernels.
+template <int OP, int NW>
 __global__ __launch_bounds__(NW * 64) void gemv_kernel(GemvArgs g) {
   typedef typename std::conditional<OP == FMSMO_OP_I8, int, float>::type AccT;
   typedef AccT Acc4 __attribute__((ext_vector_type(4)));
-  __shared__ AccT red[NW][RG][256];
+  __shared__ AccT red[NW][256];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int r = lane & 15, kg = lane >> 4;
-  const int n0 = blockIdx.x * (RG * 16);
+  const int n0 = blockIdx.x * 16;
   const int kslice = g.K / NW;  // multiple of 128 (checked on the host)
   const int kbeg = wave * kslice;
 
   const uint8_t* xp = g.a + (int64_t)min(r, g.M - 1) * g.lda + kbeg + kg * 16;
-  const uint8_t* wp[RG];
-#pragma unroll
-  for (int i = 0; i < RG; ++i)
-    wp[i] = g.b + (int64_t)min(n0 + i * 16 + r, g.N - 1) * g.ldb + kbeg + kg * 16;
-
-  Acc4 acc[RG];
-#pragma unroll
-  for (int i = 0; i < RG; ++i) acc[i] = Acc4{0, 0, 0, 0};
-
-  constexpr int UNROLL = 4 / RG > 0 ? 4 / RG : 1;  // ~8 x 16 B weight loads in flight per lane
-  int k = 0;
-  auto step = [&](int kk) {
-    const v4i x0 = *(const v4i*)(xp + kk);
-    const v4i x1 = *(const v4i*)(xp + kk + 64);
-#pragma unroll
-    for (int i = 0; i < RG; ++i) {
-      const v4i w0 = __builtin_nontemporal_load((const v4i*)(wp[i] + kk));
-      const v4i w1 = __builtin_nontemporal_load((const v4i*)(wp[i] + kk + 64));
-      if constexpr (OP == FMSMO_OP_I8) {
-        acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, x0, acc[i], 0, 0, 0);
-        acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, x1, acc[i], 0, 0, 0);
-      } else {
-        const v8i w = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
-        const v8i x = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-        acc[i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, x, acc[i], 0, 0, 0, 0, 0, 0);
-      }
+  const uint8_t* wp = g.b + (int64_t)min(n0 + r, g.N - 1) * g.ldb + kbeg + kg * 16;
+  Acc4 acc = {0, 0, 0, 0};
+  for (int k = 0; k < kslice; k += 128) {
+    const v4i x0 = *(const v4i*)(xp + k), x1 = *(const v4i*)(xp + k + 64);
+    const v4i w0 = __builtin_nontemporal_load((const v4i*)(wp + k));
+    const v4i w1 = __builtin_nontemporal_load((const v4i*)(wp + k + 64));
+    if constexpr (OP == FMSMO_OP_I8) {
+      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, x0, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, x1, acc, 0, 0, 0);
+    } else {
+      const v8i w = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
+      const v8i x = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+      acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, x, acc, 0, 0, 0, 0, 0, 0);
     }
-  };
-  for (; k + 128 * UNROLL <= kslice; k += 128 * UNROLL) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) step(k + u * 128);
   }
-  for (; k < kslice; k += 128) step(k);
 
-  // acc[i][v] = partial C(n = n0 + 16 i + 4 (lane / 16) + v, m = lane % 16)
+  // acc[v] = partial C(n = n0 + 4 (lane / 16) + v, m = lane % 16)
 #pragma unroll
-  for (int i = 0; i < RG; ++i)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) red[wave][i][(kg * 4 + v) * 16 + r] = acc[i][v];
+  for (int v = 0; v < 4; ++v) red[wave][(kg * 4 + v) * 16 + r] = acc[v];
   __syncthreads();
-
-  for (int o = threadIdx.x; o < RG * 256; o += NW * 64) {
-    const int i = o >> 8, e = o & 255;
-    AccT s = red[0][i][e];
+  for (int e = threadIdx.x; e < 256; e += NW * 64) {
+    AccT s = red[0][e];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) s += red[w][i][e];
-    const int n = n0 + i * 16 + (e >> 4), m = e & 15;
-    if (n < g.N && m < g.M) {
-      const float as = g.a_scale ? g.a_scale[g.a_stride ? m : 0] : 1.f, ws = g.w_scale ? g.w_scale[g.w_stride ? n : 0] : 1.f;
-      float b = -0.f;  // no bias: adding -0 changes nothing, not even the sign of a zero product
-      if (g.bias) {
-        b = g.bias_dtype == FMSMO_F16 ? f16_to_f32(((const u16*)g.bias)[n])
-            : g.bias_dtype == FMSMO_BF16 ? bf16_to_f32(((const u16*)g.bias)[n])
-                                         : ((const float*)g.bias)[n];
-      }
-      float out;
-      if (g.epi == FMSMO_EPI_REF_F16) {
-        const float sc = round_to<FMSMO_F16>(__fmul_rn(as, ws));
-        out = __fadd_rn(__fmul_rn((float)s, sc), b);
-        if (g.y_dtype != FMSMO_F32) out = round_to<FMSMO_F16>(out);
-      } else if (g.epi == FMSMO_EPI_F32_MULADD) {
-        out = __fadd_rn(__fmul_rn((float)s, __fmul_rn(as, ws)), b);
-      } else {
-        out = __fmaf_rn((float)s, __fmul_rn(as, ws), b);
-      }
-      const int64_t idx = (int64_t)m * g.ldy + n;
-      if (g.epi == EPI_RAW_I32) ((int*)g.y)[idx] = (int)s;
-      else if (g.y_dtype == FMSMO_F16) ((u16*)g.y)[idx] = f32_to_f16(out);
-      else if (g.y_dtype == FMSMO_BF16) ((u16*)g.y)[idx] = f32_to_bf16(out);
-      else ((float*)g.y)[idx] = out;
-    }
+    for (int w = 1; w < NW; ++w) s += red[w][e];
+    const int n = n0 + (e >> 4), m = e & 15;
+    if (n < g.N && m < g.M)
+      gemv_store(g, m, n, s, g.a_scale ? g.a_scale[g.a_stride ? m : 0] : 1.f, g.w_scale ? g.w_scale[g.w_stride ? n : 0] : 1.f,
+                 gemv_bias(g, n));
   }
 }
-
 
 // Streaming variant (K = 128 * STEPS * NW).  Weight rows must be fetched as whole 128-byte
 // lines: a wave load that touches 16 rows x 64 B tops out near 4.4 TB/s on this part, 8 rows x
@@ -1088,16 +1021,33 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvArgs g) {
 using namespace fmsmo;
 
 int fmsmo_check_launch();
+// gemv_any.hip: any K, up to 64 tokens; the form with the quantizer inside
+int fmsmo_gemv_any(int op, const GemvArgs& g, hipStream_t st);
+int fmsmo_gemv_any_fused(int op, int x_dtype, const GemvArgs& g, hipStream_t st);
 
-template <int OP, int RG>
-static void launch_gemv(const GemvArgs& g, int nw, hipStream_t st) {
-  dim3 grid(div_up(g.N, RG * 16));
-  switch (nw) {
-    case 8: hipLaunchKernelGGL((gemv_kernel<OP, RG, 8>), grid, dim3(512), 0, st, g); break;
-    case 4: hipLaunchKernelGGL((gemv_kernel<OP, RG, 4>), grid, dim3(256), 0, st, g); break;
-    case 2: hipLaunchKernelGGL((gemv_kernel<OP, RG, 2>), grid, dim3(128), 0, st, g); break;
-    default: hipLaunchKernelGGL((gemv_kernel<OP, RG, 1>), grid, dim3(64), 0, st, g); break;
-  }
+template <int OP>
+static void launch_gemv(const GemvArgs& g, hipStream_t st) {
+  const dim3 grid(div_up(g.N, 16));
+  if (g.K % 1024 == 0) hipLaunchKernelGGL((gemv_kernel<OP, 8>), grid, dim3(512), 0, st, g);
+  else hipLaunchKernelGGL((gemv_kernel<OP, 1>), grid, dim3(64), 0, st, g);
+}
+
+// One and two tokens by whole rows (gemv_rows_kernel).  us, rows | gemv_any_kernel, N = 1024 / 3072 / 8192:
+//   int8, one token: K = 2048 3.5 / 3.8 / 5.2 | 4.0 / 4.2 / 5.9, 5376 3.9 / 5.6 / 9.4 | 5.5 / 6.5 / 10.0, 10240 4.4 / 7.4 / 14.8 | 7.4 / 8.8 / 15.1;
+//     up to 1024 3.4 / 4.1 / - | 3.0 / 3.4 / -, but 20000 columns 6.4 | 7.2
+//   two tokens: 2048 4.1 / 4.4 / 6.0 | 4.0 / 4.2 / 5.9, 3072 3.6 / 4.7 / 6.5 | 4.4 / 4.9 / 7.3, 7168 4.5 / 6.5 / 12.9 | 6.1 / 7.0 / 11.8, 10240 4.7 / 8.3 / 17.6
+//     | 7.4 / 8.7 / 15.1
+//   e4m3 (twice the instructions per byte), one token: 7168 4.3 / 6.5 / 12.9 | 6.0 / 7.0 / 11.8, 10240 4.7 / 7.6 / 17.3 | 7.4 / 8.6 / 15.3, up to
+//     1024 3.7 / 4.5 / - | 3.1 / 3.4 / -; two: 3072 3.8 / 4.8 / 6.9 | 4.4 / 4.9 / 7.2, 7168 4.6 / 6.8 / 14.0 | 6.0 / 6.9 / 11.8, 10240 5.6 / 13.6 / 26.2 |
+//     7.5 / 8.7 / 15.3
+static bool rows_take(int op, int64_t M, int64_t N, int64_t K) {
+  const int64_t kch = (K + 1023) / 1024;
+  if (M > 2 || kch > 16) return false;
+  const bool i8 = op == FMSMO_OP_I8;
+  if (kch == 1) return i8 && M == 1 && N > 8192;
+  if (M == 1) return i8 || kch <= 8 || N <= 2048;
+  if (kch == 2) return false;
+  return kch <= 8 ? i8 || N <= 4096 : N <= (i8 ? 2048 : 1024);
 }
 
 // Batches of 17 .. 64 tokens that the weight-streaming kernel takes in one pass (their
@@ -1123,8 +1073,8 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
   g.a_stride = a_scale_n == 1 ? 0 : 1; g.w_stride = w_scale_n == 1 ? 0 : 1;
   g.bias = bias; g.bias_dtype = bias_dtype; g.epi = epilogue;
   g.y = y; g.y_dtype = y_dtype; g.ldy = ldy;
-  // M <= 2: whole-row streaming on the vector ALUs (at M = 4 its register use halves the
-  // occupancy and the MFMA streaming kernel below is faster) (FMSMO_GEMV_KIND=1 disables it for tuning)
+  // M <= 2: whole-row streaming on the vector ALUs (at M = 4 its register use halves the occupancy)
+  // (FMSMO_GEMV_KIND=1 disables it for tuning)
   {
     static const int env_kind = getenv("FMSMO_GEMV_KIND") ? atoi(getenv("FMSMO_GEMV_KIND")) : 0;
     const int kch = (int)((K + 1023) / 1024);
@@ -1132,7 +1082,7 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
     // Where the MFMA streaming kernel below has an instantiation for K it is the faster one for
     // two e4m3 tokens (twice the widening work per weight byte; us at N = 4096, rows -> streaming:
     // K = 4096 6.2 -> 5.4, 14336 22.3 -> 12.6), for two int8 tokens from K = 8192 (7.9 -> 7.4;
-    // 14336: 13.7 -> 12.1; 5120: 5.7 against 5.9), for one e4m3 token from K = 12800 (12.6 ->
+    // 14336: 13.7 -> 12.1; 5120: 5.7 against 5.9) and up to 2048 (6.8 -> 4.0), for one e4m3 token from K = 12800 (12.6 ->
     // 11.2; 8192: 7.9 both) and for one int8 token at K = 12800 (11.4 -> 10.8; 14336: 11.8 both,
     // 16384: 13.0 against 13.8).
     const int steps128 = K % 128 ? 0 : (int)(K / 128);
@@ -1145,8 +1095,7 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
     const bool prefer_stream =
         stream_ok && (op == FMSMO_OP_I8 ? (M == 2 ? kch >= 8 : (kch == 13 || (kch == 14 && one_group)))
                                         : (M == 2 || kch >= 11));
-    bool handled = env_kind != 1 && M <= 2 && K >= 1024 && !prefer_stream;
-    if (handled) {
+    if (env_kind != 1 && !prefer_stream && rows_take(op, M, N, K)) {
       // 16 waves per CU resident (register use allows it), rows dealt round-robin to waves
       const int64_t waves_needed = N;  // at U = 1
       dim3 block(256);
@@ -1159,24 +1108,31 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
 #define GEMV_ROWS_M(OPV, KCHV, UV)                                   \
   if (mr == 1) GEMV_ROWS(OPV, 1, KCHV, UV)                           \
   else GEMV_ROWS(OPV, 2, KCHV, UV)
+// (one token, K = 2048: four rows in flight 3.5 us, eight 4.4 at N = 1024, 5.2 against 5.8 at 8192)
 #define GEMV_ROWS_K(OPV)                                        \
   switch (kch) {                                                \
-    case 1: GEMV_ROWS_M(OPV, 1, 8) break;                       \
-    case 2: GEMV_ROWS_M(OPV, 2, 8) break;                       \
+    case 1: GEMV_ROWS(OPV, 1, 1, 8) break;                      \
+    case 2: GEMV_ROWS(OPV, 1, 2, 4) break;                      \
+    case 3: GEMV_ROWS_M(OPV, 3, 2) break;                       \
     case 4: GEMV_ROWS_M(OPV, 4, 4) break;                       \
     case 5: GEMV_ROWS_M(OPV, 5, 2) break;                       \
+    case 6: GEMV_ROWS_M(OPV, 6, 2) break;                       \
+    case 7: GEMV_ROWS_M(OPV, 7, 2) break;                       \
     case 8: GEMV_ROWS_M(OPV, 8, 2) break;                       \
+    case 9: GEMV_ROWS_M(OPV, 9, 1) break;                       \
+    case 10: GEMV_ROWS_M(OPV, 10, 1) break;                     \
     case 11: GEMV_ROWS_M(OPV, 11, 1) break;                     \
+    case 12: GEMV_ROWS_M(OPV, 12, 1) break;                     \
     case 13: GEMV_ROWS_M(OPV, 13, 1) break;                     \
     case 14: GEMV_ROWS_M(OPV, 14, 1) break;                     \
-    case 16: GEMV_ROWS_M(OPV, 16, 1) break;                     \
-    default: handled = false; break;                            \
+    case 15: GEMV_ROWS_M(OPV, 15, 1) break;                     \
+    default: GEMV_ROWS_M(OPV, 16, 1) break;                     \
   }
       if (op == FMSMO_OP_I8) { GEMV_ROWS_K(FMSMO_OP_I8) } else { GEMV_ROWS_K(FMSMO_OP_E4M3) }
 #undef GEMV_ROWS_K
 #undef GEMV_ROWS_M
 #undef GEMV_ROWS
-      if (handled) return fmsmo_check_launch();
+      return fmsmo_check_launch();
     }
   }
   // Streaming variant when the K steps of 128 split evenly over the waves of a block in one of
@@ -1187,11 +1143,11 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
   // G = 7).  FMSMO_GEMV_G overrides G for tuning.
   {
     static const int env_g = getenv("FMSMO_GEMV_G") ? atoi(getenv("FMSMO_GEMV_G")) : 0;
-    const int steps_total = (int)(K / 128);
+    const int steps_total = K % 128 ? 0 : (int)(K / 128);
     const int64_t groups = (N + 15) / 16;
     int NW = 0;
-    if (steps_total % 8 == 0) NW = 8;
-    else if (steps_total % 10 == 0) NW = 10;
+    if (steps_total && steps_total % 8 == 0) NW = 8;
+    else if (steps_total && steps_total % 10 == 0) NW = 10;
     // K = 4096 and at most 16 tokens: 16 waves of 2 steps each instead of 8 of 4 (us at M = 4 / 16:
     // o 5.8 -> 5.5 / 6.6 -> 6.0, qkv 7.0 -> 7.0 / 8.2 -> 7.7, gate+up 21.8 -> 20.9 / 22.8 -> 21.8).
     if (M <= 16 && steps_total == 32) NW = 16;
@@ -1247,22 +1203,10 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
 #undef GEMV_STREAM_H
     if (handled) return fmsmo_check_launch();
   }
-  if (M > 16) return FMSMO_ERR_UNSUPPORTED;  // callers ask fmsmo_gemv_batch_ok first
-  int nw = 8;
-  while (nw > 1 && K % (128 * nw)) nw >>= 1;
-  // enough row groups per block to amortise the activation re-reads, while keeping >= 2 blocks
-  // per compute unit (256 CUs)
-  const int64_t groups = (N + 15) / 16;
-  const int rg = groups >= 4 * 512 ? 4 : groups >= 2 * 512 ? 2 : 1;
-  if (op == FMSMO_OP_I8) {
-    if (rg == 4) launch_gemv<FMSMO_OP_I8, 4>(g, nw, st);
-    else if (rg == 2) launch_gemv<FMSMO_OP_I8, 2>(g, nw, st);
-    else launch_gemv<FMSMO_OP_I8, 1>(g, nw, st);
-  } else {
-    if (rg == 4) launch_gemv<FMSMO_OP_E4M3, 4>(g, nw, st);
-    else if (rg == 2) launch_gemv<FMSMO_OP_E4M3, 2>(g, nw, st);
-    else launch_gemv<FMSMO_OP_E4M3, 1>(g, nw, st);
-  }
+  const int rc = fmsmo_gemv_any(op, g, st);
+  if (rc != FMSMO_ERR_UNSUPPORTED || M > 16 || K % 128) return rc;
+  if (op == FMSMO_OP_I8) launch_gemv<FMSMO_OP_I8>(g, st);
+  else launch_gemv<FMSMO_OP_E4M3>(g, st);
   return fmsmo_check_launch();
 }
 
@@ -1295,6 +1239,30 @@ extern "C" int fmsmo_decode_linear_f32s_ok(int64_t M, int64_t K) {
   return K == 4096 || (M == 1 && (K == 14336 || K == 12800));
 }
 
+// One token, K <= 8192: the row kernel's fused form.  (us with SmoothQuant, two launches -> one, N = 1024 / 4096: K = 3072 7.1 / 7.5 ->
+// 4.2 / 5.9, 5376 13.3 / 14.2 -> 5.3 / 8.3, 7168 11.0 / 11.7 -> 5.9 / 9.3; K = 2048, eight rows in flight -> four: 5.0 / 5.4 -> 4.1 / 4.6)
+template <int OP, int XT>
+static int decode_rows_fused(const GemvArgs& g, hipStream_t st) {
+#define ROWS(KCHV, UV)                                                                            \
+  {                                                                                                \
+    const int64_t blocks = ((int64_t)g.N + 4 * UV - 1) / (4 * UV);                                 \
+    dim3 grid((unsigned)(blocks < 1024 ? blocks : 1024));                                          \
+    hipLaunchKernelGGL((gemv_rows_kernel<OP, 1, KCHV, UV, XT>), grid, dim3(256), 0, st, g);         \
+  }
+  switch ((g.K + 1023) / 1024) {
+    case 1: ROWS(1, 8) break;
+    case 2: ROWS(2, 4) break;
+    case 3: ROWS(3, 2) break;
+    case 4: ROWS(4, 4) break;
+    case 5: ROWS(5, 2) break;
+    case 6: ROWS(6, 2) break;
+    case 7: ROWS(7, 2) break;
+    case 8: ROWS(8, 2) break;
+    default: return FMSMO_ERR_UNSUPPORTED;
+  }
+#undef ROWS
+  return fmsmo_check_launch();
+}
 template <int OP, int XT>
 static int decode_fused_launch(const GemvArgs& g, hipStream_t st) {
   // the streaming kernel's fused form: (waves, steps per wave, loads in flight, most tokens)
@@ -1307,7 +1275,7 @@ static int decode_fused_launch(const GemvArgs& g, hipStream_t st) {
   // the row kernel's, us at N = 4096 / 1024 from bf16 with SmoothQuant: 6.6 -> 6.3 / 5.3 -> 4.6;
   // e4m3 stays with the row kernel there, whose fp32 sums are those of the two-call path)
   else if (g.K == 4096 && OP == FMSMO_OP_I8 && g.N <= 4096) shape = 1602;
-  if (sf32 && (!shape || OP != FMSMO_OP_I8)) return FMSMO_ERR_UNSUPPORTED;
+  if (sf32 && OP != FMSMO_OP_I8) return FMSMO_ERR_UNSUPPORTED;
   if (shape) {
     const int halves = (g.N + 7) / 8;
     const int nblocks = halves < 256 ? halves : 256;
@@ -1341,22 +1309,18 @@ static int decode_fused_launch(const GemvArgs& g, hipStream_t st) {
 #undef STREAM_G
     return fmsmo_check_launch();
   }
-  const int kch = (int)((g.K + 1023) / 1024);
-#define ROWS(KCHV, UV)                                                                            \
-  {                                                                                                \
-    const int64_t blocks = ((int64_t)g.N + 4 * UV - 1) / (4 * UV);                                 \
-    dim3 grid((unsigned)(blocks < 1024 ? blocks : 1024));                                          \
-    hipLaunchKernelGGL((gemv_rows_kernel<OP, 1, KCHV, UV, XT>), grid, dim3(256), 0, st, g);         \
-  }
-  switch (kch) {
-    case 1: ROWS(1, 8) break;
-    case 2: ROWS(2, 8) break;
-    case 4: ROWS(4, 4) break;
-    case 8: ROWS(8, 2) break;
-    default: return FMSMO_ERR_UNSUPPORTED;
-  }
-#undef ROWS
-  return fmsmo_check_launch();
+  // (up to 1024 elements without divisors the weights' rows are too short for a wave each: us, e4m3, N = 1024 / 4096, rows -> these:
+  // K = 512 4.6 / 4.8 -> 3.6 / 3.7, 1024 4.5 / 4.7 -> 3.8 / 3.9; int8 4.5 -> 4.1, 4.5 -> 4.3)
+  const bool rows = g.M == 1 && !sf32 && g.K <= 8192 && (g.K > 1024 || g.smooth || (OP == FMSMO_OP_I8 && g.N > 8192));
+  const int rc = rows ? FMSMO_ERR_UNSUPPORTED : fmsmo_gemv_any_fused(OP, XT, g, st);
+  return rc == FMSMO_ERR_UNSUPPORTED && g.M == 1 && !sf32 ? decode_rows_fused<OP, XT>(g, st) : rc;
+}
+int fmsmo_decode_fused(int op, int x_dtype, const GemvArgs& g, hipStream_t st) {
+  if (op == FMSMO_OP_I8)
+    return x_dtype == FMSMO_F16 ? decode_fused_launch<FMSMO_OP_I8, FMSMO_F16>(g, st)
+                                : decode_fused_launch<FMSMO_OP_I8, FMSMO_BF16>(g, st);
+  return x_dtype == FMSMO_F16 ? decode_fused_launch<FMSMO_OP_E4M3, FMSMO_F16>(g, st)
+                              : decode_fused_launch<FMSMO_OP_E4M3, FMSMO_BF16>(g, st);
 }
 
 extern "C" int fmsmo_decode_linear_i8(const void* x, int x_dtype, int64_t ldx, const void* smooth,
@@ -1387,8 +1351,7 @@ extern "C" int fmsmo_decode_linear_i8(const void* x, int x_dtype, int64_t ldx, c
   g.x16 = (const u16*)x; g.ldx = ldx; g.smooth = (const u16*)smooth; g.saturate = saturate;
   g.smooth_f32 = sf32 ? 1 : 0;
   g.a_scale_out = a_scale_out;
-  return x_dtype == FMSMO_F16 ? decode_fused_launch<FMSMO_OP_I8, FMSMO_F16>(g, (hipStream_t)stream)
-                              : decode_fused_launch<FMSMO_OP_I8, FMSMO_BF16>(g, (hipStream_t)stream);
+  return fmsmo_decode_fused(FMSMO_OP_I8, x_dtype, g, (hipStream_t)stream);
 }
 
 extern "C" int fmsmo_decode_linear_fp8(const void* x, int x_dtype, int64_t ldx, const uint8_t* w,
@@ -1411,8 +1374,7 @@ extern "C" int fmsmo_decode_linear_fp8(const void* x, int x_dtype, int64_t ldx, 
   g.y = y; g.y_dtype = y_dtype; g.ldy = ldy;
   g.x16 = (const u16*)x; g.ldx = ldx;
   g.a_scale_out = a_scale_out;
-  return x_dtype == FMSMO_F16 ? decode_fused_launch<FMSMO_OP_E4M3, FMSMO_F16>(g, (hipStream_t)stream)
-                              : decode_fused_launch<FMSMO_OP_E4M3, FMSMO_BF16>(g, (hipStream_t)stream);
+  return fmsmo_decode_fused(FMSMO_OP_E4M3, x_dtype, g, (hipStream_t)stream);
 }
 
 namespace fmsmo {
