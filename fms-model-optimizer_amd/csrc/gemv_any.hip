@@ -17,6 +17,8 @@ namespace fmsmo {
 // K % 64 != 0, e4m3: codes widened to fp16 (exact), products on the fp16 instruction, whose sums keep what fp32
 // additions keep (the e4m3 instruction, which takes 64 elements and more at a time, does not)
 constexpr int GEMV_FP8_F16 = 6;
+// per token (int8: with divisors of the 16-bit dtype, or none), with fp32 divisors, static per tensor
+enum { QUANT_TOKEN, QUANT_TOKEN_F32S, QUANT_STATIC };
 constexpr unsigned GEMV_OUTSIDE = 0x80000000u;  // past the end of every descriptor made here
 constexpr int UNIT = 512;                       // elements of a token row that a wave quantizes at a time
 
@@ -264,6 +266,25 @@ __device__ __forceinline__ void units_fp8(const GemvArgs& g, const Units<NW, UPW
   }
 }
 
+// Static per-tensor int8 (FMSMO_SQ_FMO in fp32): no maxima, no scales to hand over.
+template <int XT, int NW, int UPW>
+__device__ __forceinline__ void units_static(const GemvArgs& g, const Units<NW, UPW>& U, const v4i (&cur)[UPW], uint8_t* xq,
+                                             int xs) {
+  const float nz = opaque_neg_zero();
+#pragma unroll
+  for (int i = 0; i < UPW; ++i) {
+    if (!U.has(i)) continue;
+    const int c = U.chunk(i);
+    uint32_t code[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      code[q] = static_fmo32_codes<XT>((uint32_t)cur[i][q], g.q_lo, g.q_hi, g.q_step, g.q_rcp, g.q_zp, g.q_shift, nz);
+    const uint2 o = make_uint2(__builtin_amdgcn_perm(code[1], code[0], 0x06040200u),
+                               __builtin_amdgcn_perm(code[3], code[2], 0x06040200u));
+    *(uint2*)(xq + (size_t)U.row(i) * xs + (size_t)c * AQ_VEC) = c < U.nchunk ? o : make_uint2(0, 0);
+  }
+}
+
 // ------------------------------------------------------------------ the product
 __device__ __forceinline__ h8 widen_fp8(int a, int b) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -289,10 +310,10 @@ __device__ __forceinline__ Acc4 gemv_mma(v4i w0, v4i w1, v4i x0, v4i x1, Acc4 ac
 }
 
 // XT >= 0: the activations are x16 (of that dtype), UPW units of them per wave quantized by every block for itself, in
-// LDS, while the head of its weight stream is in flight.  SF32: with fp32 SmoothQuant divisors.
-template <int OP, int NW, int MT = 1, int XT = -1, int UPW = 1, bool SF32 = false>
+// LDS, while the head of its weight stream is in flight, by the quantizer QUANT.
+template <int OP, int NW, int MT = 1, int XT = -1, int UPW = 1, int QUANT = QUANT_TOKEN>
 __global__ __launch_bounds__(NW * 64) void gemv_any_kernel(GemvArgs g, int halves) {
-  constexpr bool FUSED = XT >= 0;
+  constexpr bool FUSED = XT >= 0, SF32 = QUANT == QUANT_TOKEN_F32S, STATIC = QUANT == QUANT_STATIC;
   static_assert(!FUSED || MT == 1, "the fused form serves one tile of tokens");
   typedef typename std::conditional<OP == FMSMO_OP_I8, int, float>::type AccT;
   typedef AccT Acc4 __attribute__((ext_vector_type(4)));
@@ -348,7 +369,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_any_kernel(GemvArgs g, int halve
   v4i wb[2], xb[MT][2];
   const Units<NW, UPW> U(g);
   const int xs = U.nseg * UNIT + 16;
-  v4i qcur[FUSED ? UPW : 1], qsm[FUSED && !SF32 ? UPW : 1];
+  v4i qcur[FUSED ? UPW : 1], qsm[FUSED && !SF32 && !STATIC ? UPW : 1];
   float qsd[SF32 ? UPW : 1][8];
   if constexpr (FUSED) {
 #pragma unroll
@@ -358,7 +379,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_any_kernel(GemvArgs g, int halve
 #pragma unroll
         for (int q = 0; q < 8; ++q) qsd[i][q] = 1.0f;
         if (in) load8<FMSMO_F32>(g.smooth, (size_t)U.chunk(i) * AQ_VEC, qsd[i]);
-      } else {
+      } else if constexpr (!STATIC) {
         qsm[i] = v4i{0, 0, 0, 0};
         if (in && g.smooth) qsm[i] = *(const v4i*)(g.smooth + (size_t)U.chunk(i) * AQ_VEC);
       }
@@ -373,12 +394,13 @@ __global__ __launch_bounds__(NW * 64) void gemv_any_kernel(GemvArgs g, int halve
   const int em = min((int)(threadIdx.x & 15), g.M - 1);
   float as;
   if constexpr (FUSED) {
-    if constexpr (SF32) units_i8_f32s<XT, NW, UPW>(g, U, qcur, qsd, xq, xs, xsc, xred);
+    if constexpr (STATIC) units_static<XT, NW, UPW>(g, U, qcur, xq, xs);
+    else if constexpr (SF32) units_i8_f32s<XT, NW, UPW>(g, U, qcur, qsd, xq, xs, xsc, xred);
     else if constexpr (OP == FMSMO_OP_I8) units_i8<XT, NW, UPW>(g, U, qcur, qsm, xq, xs, xsc, xred);
     else units_fp8<XT, NW, UPW>(g, U, qcur, xq, xs, xsc, xred);
     __syncthreads();
-    gemv_put_scales(g, xsc);
-    as = xsc[em];
+    if constexpr (!STATIC) gemv_put_scales(g, xsc);
+    as = STATIC ? g.a_value : xsc[em];
   } else {
     as = g.a_scale ? g.a_scale[g.a_stride ? em : 0] : 1.f;
   }
@@ -484,7 +506,7 @@ static bool any_offsets_ok(const GemvArgs& g) {
   return (std::min(g.N, 16) - 1) * g.ldb + g.K < (1ll << 31) && (g.M > 1 ? (g.M - 1) * g.lda : 0) + g.K < (1ll << 31);
 }
 
-template <int OP, int MT, int XT = -1, bool SF32 = false>
+template <int OP, int MT, int XT = -1, int QUANT = QUANT_TOKEN>
 static int any_launch(const GemvArgs& g, hipStream_t st) {
   const AnyPlan p = any_plan(g.M, g.N, g.K);
   const int halves = (g.N + 7) / 8;
@@ -494,18 +516,18 @@ static int any_launch(const GemvArgs& g, hipStream_t st) {
   const int units = g.M * ((g.K + UNIT - 1) / UNIT);
   if constexpr (MT == 1) {
     if (p.nw == 4 && units <= 4 * UPW) {
-      hipLaunchKernelGGL((gemv_any_kernel<OP, 4, MT, XT, UPW, SF32>), grid, dim3(256), 0, st, g, halves);
+      hipLaunchKernelGGL((gemv_any_kernel<OP, 4, MT, XT, UPW, QUANT>), grid, dim3(256), 0, st, g, halves);
       return fmsmo_check_launch();
     }
   }
   if constexpr (MT <= 2) {
     if (p.nw == 16 || (XT >= 0 && units > 8 * UPW)) {
       if (XT >= 0 && units > 16 * UPW) return FMSMO_ERR_UNSUPPORTED;
-      hipLaunchKernelGGL((gemv_any_kernel<OP, 16, MT, XT, UPW, SF32>), grid, dim3(1024), 0, st, g, halves);
+      hipLaunchKernelGGL((gemv_any_kernel<OP, 16, MT, XT, UPW, QUANT>), grid, dim3(1024), 0, st, g, halves);
       return fmsmo_check_launch();
     }
   }
-  hipLaunchKernelGGL((gemv_any_kernel<OP, 8, MT, XT, UPW, SF32>), grid, dim3(512), 0, st, g, halves);
+  hipLaunchKernelGGL((gemv_any_kernel<OP, 8, MT, XT, UPW, QUANT>), grid, dim3(512), 0, st, g, halves);
   return fmsmo_check_launch();
 }
 
@@ -525,7 +547,7 @@ int fmsmo_gemv_any(int op, const GemvArgs& g, hipStream_t st) {
 template <int XT>
 static int any_fused(int op, const GemvArgs& g, hipStream_t st) {
   if (op == FMSMO_OP_I8) {
-    if (g.smooth && g.smooth_f32) return any_launch<FMSMO_OP_I8, 1, XT, true>(g, st);
+    if (g.smooth && g.smooth_f32) return any_launch<FMSMO_OP_I8, 1, XT, QUANT_TOKEN_F32S>(g, st);
     return any_launch<FMSMO_OP_I8, 1, XT>(g, st);
   }
   if (g.K % 64) return any_launch<GEMV_FP8_F16, 1, XT>(g, st);
@@ -595,4 +617,40 @@ extern "C" int fmsmo_small_linear_fp8(const void* x, int x_dtype, int64_t ldx, c
                                       fmsmo_stream_t stream) {
   return small_linear(FMSMO_OP_E4M3, x, x_dtype, ldx, nullptr, x_dtype, w, ldw, w_scale, w_scale_n, bias, bias_dtype,
                       FMSMO_EPI_F32, y, y_dtype, ldy, a_scale_out, nullptr, M, N, K, stream);
+}
+
+// Static activations: no reduction in front of the codes, so more of them than per token, but no form of the row kernel for one long
+// token.  us, quantizer + product -> one launch, N = 1024 / 4096: 1 x 2048 5.9 / 6.1 -> 4.4 / 5.0, 3072 5.9 / 6.6 -> 5.0 / 5.7, 5376 5.9 / 8.1 -> 6.3 / 7.6; 4 x 3072
+// 6.5 / 7.1 -> 6.0 / 6.5, 4096 6.6 / 8.4 -> 6.9 / 8.6; 8 x 2048 6.6 / 6.6 -> 6.0 / 6.3, 3072 6.6 / 7.2 -> 7.6 / 7.8; 16 x 640 6.4 / 6.4 -> 6.0 / 6.2, 2048 6.5 / 6.5 -> 8.2 / 8.3; N =
+// 12000: 4 x 1024 7.7 -> 6.9, 2048 9.3 -> 9.5, 12 x 640 7.7 -> 11.2.
+extern "C" int fmsmo_small_linear_static_ok(int64_t M, int64_t N, int64_t K, float step, float zp, float clip_lo, float clip_hi) {
+  if (M < 1 || M > 16 || N < 1 || K < 16 || K % 16 || N >= (1 << 30)) return 0;
+  return K <= 3072 && M * ((K + UNIT - 1) / UNIT) <= 32 && (N <= 8192 || (M <= 4 && K <= 1024)) &&
+         static_fmo32_ok(clip_lo, clip_hi, step, zp);
+}
+extern "C" int fmsmo_small_linear_i8_static(const void* x, int x_dtype, int64_t ldx, float step, float zp, int sym, float clip_lo,
+                                            float clip_hi, float a_scale, const int8_t* w, int64_t ldw, const float* w_scale,
+                                            int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue, void* y,
+                                            int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream) {
+  if (!x || !w || !w_scale || !y) return FMSMO_ERR_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || (M > 1 && ldx < K) || ldw < K || ldy < N) return FMSMO_ERR_SHAPE;
+  if (w_scale_n != 1 && w_scale_n != N) return FMSMO_ERR_SHAPE;
+  if (x_dtype != FMSMO_F16 && x_dtype != FMSMO_BF16) return FMSMO_ERR_UNSUPPORTED;
+  if (!fmsmo_small_linear_static_ok(M, N, K, step, zp, clip_lo, clip_hi)) return FMSMO_ERR_UNSUPPORTED;
+  if (N * ldw >= (1ll << 31)) return FMSMO_ERR_UNSUPPORTED;
+  if (y_dtype < 0 || y_dtype > 2 || (bias && (bias_dtype < 0 || bias_dtype > 2))) return FMSMO_ERR_UNSUPPORTED;
+  if (epilogue < FMSMO_EPI_REF_F16 || epilogue > FMSMO_EPI_F32_MULADD) return FMSMO_ERR_UNSUPPORTED;
+  if ((M > 1 && ldx % 8) || ldw % 16 || (((uintptr_t)x) & 15) || (((uintptr_t)w) & 15)) return FMSMO_ERR_ALIGN;
+  GemvArgs g{};
+  g.b = (const uint8_t*)w; g.ldb = ldw;
+  g.M = (int)M; g.N = (int)N; g.K = (int)K;
+  g.w_scale = w_scale; g.w_stride = w_scale_n == 1 ? 0 : 1;
+  g.bias = bias; g.bias_dtype = bias_dtype; g.epi = epilogue;
+  g.y = y; g.y_dtype = y_dtype; g.ldy = ldy;
+  g.x16 = (const u16*)x; g.ldx = ldx;
+  g.q_lo = clip_lo; g.q_hi = clip_hi; g.q_step = step; g.q_rcp = 1.0f / step; g.q_zp = zp; g.q_shift = 128 - (sym ? 1 : 0);
+  g.a_value = a_scale;
+  if (!any_offsets_ok(g)) return FMSMO_ERR_UNSUPPORTED;
+  return x_dtype == FMSMO_F16 ? any_launch<FMSMO_OP_I8, 1, FMSMO_F16, QUANT_STATIC>(g, (hipStream_t)stream)
+                              : any_launch<FMSMO_OP_I8, 1, FMSMO_BF16, QUANT_STATIC>(g, (hipStream_t)stream);
 }

@@ -26,6 +26,10 @@ struct GemvArgs {
   int smooth_f32;
   int saturate;
   float* a_scale_out;   // [M] per-token scales (written by block 0), or NULL
+  // static per-tensor quantizer (see fmsmo_quant_act_i8_static_t, FMSMO_SQ_FMO in fp32): clip values, step and its
+  // reciprocal, zero point, 128 - sym, and the scale that the sums are dequantized with
+  float q_lo, q_hi, q_step, q_rcp, q_zp, a_value;
+  int q_shift;
   float* clips;         // [2][M] the clip values they stand for, scale * 127 and its negative, or NULL
 };
 

@@ -28,7 +28,7 @@ namespace {
   X(fmsmo_quant_act_fp8_pertoken) X(fmsmo_quant_act_fp8_dynamic) X(fmsmo_quant_act_fp8_tensor)           \
   X(fmsmo_quant_act_i8_pertoken_clips) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
-  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_small_linear_ok) X(fmsmo_small_linear_i8) X(fmsmo_small_linear_fp8) X(fmsmo_grouped_gemm_i8_dq)                   \
+  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_small_linear_ok) X(fmsmo_small_linear_i8) X(fmsmo_small_linear_fp8) X(fmsmo_small_linear_static_ok) X(fmsmo_small_linear_i8_static) X(fmsmo_grouped_gemm_i8_dq)                   \
   X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq) X(fmsmo_matmul_chunk_workspace_bytes)    \
   X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_parts_first) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
   X(fmsmo_bmm_qa_i8) X(fmsmo_bmm_i8_zp)
@@ -515,42 +515,80 @@ PyObject* item(PyObject* dict, PyObject* key) {  // borrowed, or null
   X(_buffers) X(_parameters) X(weight) X(bias) X(w_scale) X(smoothq_scale) X(input_scale) X(useDynMaxQfunc)      \
   X(use_int_kernel) X(chunk_size) X(truncate_lsb) X(use_fake_zero_shift) X(acc_dtype) X(_sq_kept) X(_ws_kept)    \
   X(iaddmm) X(cvs) X(weight_scale) X(_quantize) X(qa_dynamic_max_qfunc) X(_smoothq_active) X(_w_scale_f32)         \
-  X(_set_input_scale)
+  X(_set_input_scale) X(_sp_kept) X(usePTnativeQfunc) X(useSymAct) X(input_zp) X(quant_stepsize) X(quant_zero_point)     \
+  X(qa_fmo_mo_qfunc) X(_static_params)
 #define DECLARE(n) PyObject* k_##n = nullptr;
 NAMES(DECLARE)
 #undef DECLARE
 
-// What the Python side found out about buffer t, kept as ((data pointer, version, dtype), finding, alias of the
-// buffer): the finding (borrowed), or null where the buffer is another one or was written to since.  (The alias keeps
-// the memory, so the address is the buffer's own.)
-PyObject* kept_for(PyObject* kept, const at::Tensor& t) {
-  if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3 || t.is_inference()) return nullptr;
-  PyObject* stamp = PyTuple_GET_ITEM(kept, 0);
-  if (!PyTuple_Check(stamp) || PyTuple_GET_SIZE(stamp) != 3 || !THPDtype_Check(PyTuple_GET_ITEM(stamp, 2))) return nullptr;
+// Is this (data pointer, version, dtype) the stamp of t as it is now?
+bool same_stamp(PyObject* stamp, const at::Tensor& t) {
+  if (t.is_inference() || !PyTuple_Check(stamp) || PyTuple_GET_SIZE(stamp) != 3 || !THPDtype_Check(PyTuple_GET_ITEM(stamp, 2)))
+    return false;
   const unsigned long long p = PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(stamp, 0));
   const long long v = PyLong_AsLongLong(PyTuple_GET_ITEM(stamp, 1));
   if (PyErr_Occurred()) {
     PyErr_Clear();
-    return nullptr;
+    return false;
   }
-  const bool same = p == (unsigned long long)(uintptr_t)t.data_ptr() && v == (long long)t._version() &&
-                    ((THPDtype*)PyTuple_GET_ITEM(stamp, 2))->scalar_type == t.scalar_type();
-  return same ? PyTuple_GET_ITEM(kept, 1) : nullptr;
+  return p == (unsigned long long)(uintptr_t)t.data_ptr() && v == (long long)t._version() &&
+         ((THPDtype*)PyTuple_GET_ITEM(stamp, 2))->scalar_type == t.scalar_type();
+}
+// What the Python side found out about buffer t, kept as ((data pointer, version, dtype), finding, alias of the
+// buffer): the finding (borrowed), or null where the buffer is another one or was written to since.  (The alias keeps
+// the memory, so the address is the buffer's own.)
+PyObject* kept_for(PyObject* kept, const at::Tensor& t) {
+  if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3) return nullptr;
+  return same_stamp(PyTuple_GET_ITEM(kept, 0), t) ? PyTuple_GET_ITEM(kept, 1) : nullptr;
+}
+// The parameters of the static quantizer that the Python side keeps for activations of dtype xt beside the buffers they were read from
+// (QLinearINT8Deploy._static_params); false where one of those is another tensor or was written to since.
+struct StaticParams {
+  double scale = 0, step = 0, qzp = 0, lo = 0, hi = 0;
+  at::ScalarType T = at::kFloat;
+  const at::Tensor* scale_t = nullptr;  // the scale as fp32 on the device
+};
+bool static_params(PyObject* self, PyObject* buffers, at::ScalarType xt, StaticParams* p) {
+  PyObject *kept = item(self, k__sp_kept), *cvs = item(self, k_cvs);
+  if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3 || !cvs || !PyList_CheckExact(cvs) || PyList_GET_SIZE(cvs) < 2)
+    return false;
+  PyObject *stamps = PyTuple_GET_ITEM(kept, 0), *found = PyTuple_GET_ITEM(kept, 1);
+  if (!PyTuple_Check(stamps) || PyTuple_GET_SIZE(stamps) != 7 || !PyDict_Check(found)) return false;
+  if (!THPDtype_Check(PyTuple_GET_ITEM(stamps, 0)) || ((THPDtype*)PyTuple_GET_ITEM(stamps, 0))->scalar_type != xt) return false;
+  PyObject* of[6] = {item(buffers, k_input_scale), item(buffers, k_input_zp), item(buffers, k_quant_stepsize),
+                     item(buffers, k_quant_zero_point), PyList_GET_ITEM(cvs, 0), PyList_GET_ITEM(cvs, 1)};
+  for (int i = 0; i < 6; ++i) {
+    const at::Tensor* t = of[i] ? plain(of[i]) : nullptr;
+    if (!t || !same_stamp(PyTuple_GET_ITEM(stamps, i + 1), *t)) return false;
+    if (i == 0 && t->numel() != 1) return false;
+  }
+  const char* names[5] = {"scale", "step", "qzp", "lo", "hi"};
+  double* to[5] = {&p->scale, &p->step, &p->qzp, &p->lo, &p->hi};
+  for (int i = 0; i < 5; ++i) {
+    PyObject* v = PyDict_GetItemString(found, names[i]);
+    if (!v || !PyFloat_Check(v)) return false;
+    *to[i] = PyFloat_AS_DOUBLE(v);
+  }
+  PyObject *T = PyDict_GetItemString(found, "T"), *st = PyDict_GetItemString(found, "scale_t");
+  if (!T || !dtype_arg(T, &p->T) || !st) return false;
+  p->scale_t = vec32(st, 1);
+  return p->scale_t != nullptr;
 }
 
 // Is a method of the class, or of this instance, another function than the one that came with it?
 bool replaced(PyObject* self, PyTypeObject* cls, PyObject* name, PyObject* own) {
   return item(self, name) || _PyType_Lookup(cls, name) != own;
 }
-// QLinearINT8Deploy.forward with dynamic per-token scales and a plain integer product: (instance dict, x, the class,
-// (iaddmm_int, _smoothq_active, _w_scale_f32, _set_input_scale, _quantize, qa_dynamic_max_qfunc) as it came) -> y.
+// QLinearINT8Deploy.forward with dynamic per-token scales, or static ones by the fms_mo formula, and a plain integer product: (instance
+// dict, x, the class, (iaddmm_int, _smoothq_active, _w_scale_f32, _set_input_scale, _quantize, qa_dynamic_max_qfunc, qa_fmo_mo_qfunc,
+// _static_params) as it came) -> y.
 // The scales' host-side facts (does SmoothQuant apply, the fp32 copy of w_scale) are those the Python side
 // keeps beside the buffers; where they are stale it is asked (None).
 PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   WANT(4);
   PyObject *self = args[0], *own_f = args[3];
-  if (!PyType_Check(args[2]) || !PyTuple_CheckExact(own_f) || PyTuple_GET_SIZE(own_f) != 6) return none();
+  if (!PyType_Check(args[2]) || !PyTuple_CheckExact(own_f) || PyTuple_GET_SIZE(own_f) != 8) return none();
   // the methods that the forward in Python goes through: these always, its quantizer's and iaddmm on one branch below
   PyTypeObject* cls = (PyTypeObject*)args[2];
   auto other = [&](PyObject* name, int i) { return replaced(self, cls, name, PyTuple_GET_ITEM(own_f, i)); };
@@ -561,8 +599,9 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   PyObject *dyn = item(self, k_useDynMaxQfunc), *kern = item(self, k_use_int_kernel), *acc = item(self, k_acc_dtype);
   PyObject *chunk = item(self, k_chunk_size), *lsb = item(self, k_truncate_lsb), *fzs = item(self, k_use_fake_zero_shift);
   PyObject *ow = item(params, k_weight), *osq = item(buffers, k_smoothq_scale), *ows = item(buffers, k_w_scale);
-  if (!dyn || !PyLong_CheckExact(dyn) || !kern || !acc || !chunk || !PyLong_Check(chunk) || !lsb || !PyLong_Check(lsb) ||
-      !ow || !osq || !ows || !item(buffers, k_input_scale) || PyLong_AsLong(dyn) != -1 || PyObject_IsTrue(kern) != 1 ||
+  const bool stat = dyn == Py_False;
+  if (!dyn || (!stat && (!PyLong_CheckExact(dyn) || PyLong_AsLong(dyn) != -1)) || !kern || !acc || !chunk || !PyLong_Check(chunk) || !lsb || !PyLong_Check(lsb) ||
+      !ow || !osq || !ows || !item(buffers, k_input_scale) || PyObject_IsTrue(kern) != 1 ||
       PyLong_AsLong(lsb) > 0 || x.cols > PyLong_AsLong(chunk) || (fzs && PyObject_IsTrue(fzs) != 0)) {
     PyErr_Clear();
     return none();
@@ -596,6 +635,37 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const THPObjectPtr own_buffers(Py_NewRef(buffers));
   w.t = &own_w;
   ws = &own_ws;
+  auto plain_product = [&]() {  // the branch that ends in the module's iaddmm: only the class's own one is known here
+    PyObject* f = item(self, k_iaddmm);
+    return f && PyMethod_Check(f) && PyMethod_GET_FUNCTION(f) == PyTuple_GET_ITEM(own_f, 0) && !other(k__quantize, 4);
+  };
+  if (stat) {
+    PyObject* native = item(self, k_usePTnativeQfunc);
+    PyObject* sym = item(self, k_useSymAct);
+    StaticParams p;
+    if (smooth || native != Py_False || !sym || !plain_product() || other(k_qa_fmo_mo_qfunc, 6) || other(k__static_params, 7) ||
+        !static_params(self, buffers, xt, &p) || !here(x.t, p.scale_t))
+      return none();
+    const at::Tensor own_scale = *p.scale_t;
+    const int sy = PyObject_IsTrue(sym) == 1;
+    at::Tensor y = out_like(*x.t, w.rows, ot);
+    if (p.T == at::kFloat && w.rows * w.ld < (1ll << 31) &&
+        p_fmsmo_small_linear_static_ok(x.rows, w.rows, x.cols, (float)p.step, (float)p.qzp, (float)p.lo, (float)p.hi)) {
+      if (!LAUNCH(fmsmo_small_linear_i8_static, x.p, code_of(xt), x.ld, (float)p.step, (float)p.qzp, sy, (float)p.lo, (float)p.hi,
+                  (float)p.scale, (const int8_t*)w.p, w.ld, (const float*)ws->data_ptr(), ws->numel(), b.p, b.dt,
+                  FMSMO_EPI_REF_F16, y.data_ptr(), code_of(ot), w.rows, x.rows, w.rows, x.cols, stream_of(*x.t)))
+        return nullptr;
+      return wrap(y);
+    }
+    at::Tensor q = empty({x.rows, x.cols}, at::kChar, *x.t);
+    if (!LAUNCH(fmsmo_quant_act_i8_static_t, x.p, code_of(xt), x.ld, FMSMO_SQ_FMO, code_of(p.T), (float)p.step, (float)p.qzp, sy,
+                (float)p.lo, (float)p.hi, (int8_t*)q.data_ptr(), x.cols, x.rows, x.cols, stream_of(*x.t)))
+      return nullptr;
+    if (!run_gemm_i8((const char*)q.data_ptr(), x.cols, w, (const float*)own_scale.data_ptr(), 1, *ws, b, FMSMO_EPI_REF_F16, y,
+                     x.rows, x.cols))
+      return nullptr;
+    return wrap(y);
+  }
   at::Tensor y = out_like(*x.t, w.rows, ot), s;
   const bool f32s = smooth && sm.st == at::kFloat;
   const bool one = (!smooth || sm.st == xt || f32s) &&
@@ -607,11 +677,9 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // decode step of a few tokens: quantizer and weight-streaming matmul in one launch
     if (!run_decode_i8(x, sm, 0, w, *ws, b, FMSMO_EPI_REF_F16, y, s)) return nullptr;
   } else {
-    if (!smooth) {  // this branch ends in the module's iaddmm: only the class's own one is known here
-      PyObject* f = item(self, k_iaddmm);
+    if (!smooth) {
       PyObject* cvs = item(self, k_cvs);
-      if (!f || !PyMethod_Check(f) || PyMethod_GET_FUNCTION(f) != PyTuple_GET_ITEM(own_f, 0) || !cvs ||
-          !PyList_CheckExact(cvs) || PyList_GET_SIZE(cvs) < 2 || other(k__quantize, 4) || other(k_qa_dynamic_max_qfunc, 5))
+      if (!plain_product() || !cvs || !PyList_CheckExact(cvs) || PyList_GET_SIZE(cvs) < 2 || other(k_qa_dynamic_max_qfunc, 5))
         return none();
     }
     at::Tensor q, c;

@@ -3,6 +3,7 @@
 // fallback routine for one row.
 #pragma once
 #include "common.hpp"
+#include <cmath>
 
 namespace fmsmo {
 
@@ -164,6 +165,24 @@ __device__ __forceinline__ uint32_t rint_codes(u16 lo, u16 hi) {
     const uint32_t c = __float_as_uint(bf16_to_f32(hi) + 12582912.0f) & 0xffu;
     return a | (c << 16);
   }
+}
+
+// code = int8( rint( clamp(x, lo, hi) / step - zp ) - shift ) of a packed pair of XT in the low byte of each half, every step in fp32
+// (the static quantizer FMSMO_SQ_FMO).  The division by its short sequence, which the host allows where |step| lies in
+// 2^-20 .. 2^20, the clip values are finite and no |quotient| + |zp| reaches 10^6 (static_fmo32_ok): exact, but for quotients under 2^-80, which
+// the zero point or the rounding to an integer swallows whichever way their last bit goes.  rint by the addition
+// of 1.5 * 2^23, which leaves the integer in two's complement in the low mantissa bits.
+template <int XT>
+__device__ __forceinline__ uint32_t static_fmo32_codes(uint32_t w, float lo, float hi, float step, float rcp, float zp,
+                                                       int shift, float nz) {
+  const float e0 = fminf(fmaxf(cvt16<XT>((u16)(w & 0xffff)), lo), hi), e1 = fminf(fmaxf(cvt16<XT>((u16)(w >> 16)), lo), hi);
+  const float t0 = __fsub_rn(div32_fast_mix(e0, step, rcp, nz), zp), t1 = __fsub_rn(div32_fast_mix(e1, step, rcp, nz), zp);
+  const uint32_t c0 = __float_as_uint(t0 + 12582912.0f) - (uint32_t)shift, c1 = __float_as_uint(t1 + 12582912.0f) - (uint32_t)shift;
+  return (c0 & 0xffu) | (c1 << 16);
+}
+inline bool static_fmo32_ok(float lo, float hi, float step, float zp) {
+  const float s = fabsf(step), m = fmaxf(fabsf(lo), fabsf(hi));
+  return s >= 9.5367431640625e-07f && s <= 1048576.0f && m < INFINITY && fabsf(zp) < 1.0e6f && m / s + fabsf(zp) < 1.0e6f;
 }
 
 // One row with plain IEEE divisions, chunk by chunk from memory (no register cache, so that this

@@ -126,6 +126,24 @@ __global__ __launch_bounds__(256) void quant_i8_static16_kernel(const u16* __res
   }
 }
 
+// FMSMO_SQ_FMO with 16-bit x and fp32 arithmetic (a 16-bit model whose clip values stayed fp32) on contiguous x.  The generic
+// kernel's IEEE division and 64-bit index division kept it at half the memory rate: us, bf16, 1000 x 4096 5.4 -> 4.0,
+// 3149 x 4096 12.2 -> 8.6, 4096 x 14336 40.8 -> 29.5 (6.0 TB/s), 18 x 1280 3.0 -> 2.1.
+template <int XT>
+__global__ __launch_bounds__(256) void quant_i8_static_fmo32_kernel(const u16* __restrict__ x, StaticArgs p, float rcp,
+                                                                    int8_t* __restrict__ q, int64_t nchunks) {
+  const float nz = opaque_neg_zero();
+  const int shift = 128 - (int)p.sym;
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)gridDim.x * 256) {
+    const v4i raw = __builtin_nontemporal_load((const v4i*)(x + c * AQ_VEC));
+    uint32_t code[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) code[j] = static_fmo32_codes<XT>((uint32_t)raw[j], p.lo, p.hi, p.scale, rcp, p.zp, shift, nz);
+    *(uint2*)(q + c * AQ_VEC) = make_uint2(__builtin_amdgcn_perm(code[1], code[0], 0x06040200u),
+                                           __builtin_amdgcn_perm(code[3], code[2], 0x06040200u));
+  }
+}
+
 // scale[k] = rnd_T( max(amax_k, rnd_T(1e-5)) / levels ) per column, or the same of the maximum
 // over all columns into scale[0] (one block).
 template <int T>
@@ -408,6 +426,16 @@ extern "C" int fmsmo_quant_act_i8_static_t(const void* x, int x_dtype, int64_t l
     if (x_dtype == FMSMO_F16) { FAST_T(FMSMO_F16) } else { FAST_T(FMSMO_BF16) }
 #undef FAST_T
 #undef FAST
+    return fmsmo_check_launch();
+  }
+  if (compute_dtype == FMSMO_F32 && x_dtype != FMSMO_F32 && mode == FMSMO_SQ_FMO && ldx == K && ldq == K &&
+      static_fmo32_ok(clip_lo, clip_hi, scale, zp)) {
+    const int64_t nchunks = M * (K / AQ_VEC);
+    const float rcp = 1.0f / scale;
+    if (x_dtype == FMSMO_F16)
+      hipLaunchKernelGGL((quant_i8_static_fmo32_kernel<FMSMO_F16>), grid, block, 0, st, (const u16*)x, p, rcp, q, nchunks);
+    else
+      hipLaunchKernelGGL((quant_i8_static_fmo32_kernel<FMSMO_BF16>), grid, block, 0, st, (const u16*)x, p, rcp, q, nchunks);
     return fmsmo_check_launch();
   }
 #define LAUNCH(XT, T) \

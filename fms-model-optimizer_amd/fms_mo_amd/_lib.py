@@ -53,6 +53,7 @@ SIGNATURES = {
     "fmsmo_gemv_fp8_dq": [_P, _L, _P, _L, _P, _L, _P, _L, _P, _I, _P, _I, _L, _L, _L, _L, _P],
     "fmsmo_decode_linear_i8": [_P, _I, _L, _P, _I, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_small_linear_i8": [_P, _I, _L, _P, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _P, _P, _L, _L, _L, _P],
+    "fmsmo_small_linear_i8_static": [_P, _I, _L, _F, _F, _I, _F, _F, _F, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _L, _L, _L, _P],
     "fmsmo_small_linear_fp8": [_P, _I, _L, _P, _L, _P, _L, _P, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_decode_linear_fp8": [_P, _I, _L, _P, _L, _P, _L, _P, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_matmul_chunk_i8": [_P, _L, _P, _L, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I, _P],
@@ -105,6 +106,7 @@ OTHER = {
     "fmsmo_matmul_chunk_workspace_bytes": ([c_int, c_int64, c_int64, c_int64, c_int, c_int], c_int64),
     "fmsmo_decode_linear_ok": ([c_int64, c_int64], c_int),
     "fmsmo_decode_linear_f32s_ok": ([c_int64, c_int64], c_int),
+    "fmsmo_small_linear_static_ok": ([c_int64, c_int64, c_int64, _F, _F, _F, _F], c_int),
     "fmsmo_small_linear_ok": ([c_int64, c_int64, c_int64, c_int], c_int),
     "fmsmo_gemm_tail_columns": ([c_int64, c_int64, c_int64], c_int64),
     "fmsmo_gemm_fp8_tail_columns": ([c_int64, c_int64, c_int64], c_int64),

@@ -614,7 +614,8 @@ class QLinearINT8Deploy(nn.Linear):
                 p.update(T=quot.dtype, lo=float(cvn.to(clamped.dtype).reshape(-1)[0]),
                          hi=float(cv.to(clamped.dtype).reshape(-1)[0]),
                          step=float(self.quant_stepsize.reshape(-1)[0]),
-                         qzp=float(self.quant_zero_point.reshape(-1)[0]))
+                         qzp=float(self.quant_zero_point.reshape(-1)[0]),
+                         scale_t=self.input_scale.detach().float().reshape(-1).contiguous())
             self._sp_kept = kept = _Kept((stamp, p, [t.detach() for t in tensors]))
         return kept[1]
 
@@ -857,7 +858,7 @@ class QLinearINT8Deploy(nn.Linear):
         # outputs outside autograd anyway, and the torch-op branch enters no_grad itself -- an eager
         # decode step is bound by what the host does per call, so nothing is done twice here)
         if type(self) is QLinearINT8Deploy and not torch.compiler.is_compiling():
-            # the dynamic per-token forms, natively; None: something here is less common
+            # the dynamic per-token forms and the static one, natively; None: something here is less common
             y = L.host().deploy_i8(self.__dict__, x, QLinearINT8Deploy, _OWN_METHODS)
             if y is not None:
                 return y
@@ -904,7 +905,8 @@ class QLinearINT8Deploy(nn.Linear):
 
 # deploy_i8 knows what the methods of a forward do only where they are these
 _OWN_METHODS = tuple(getattr(QLinearINT8Deploy, n) for n in ("iaddmm_int", "_smoothq_active", "_w_scale_f32", "_set_input_scale",
-                                                             "_quantize", "qa_dynamic_max_qfunc"))
+                                                             "_quantize", "qa_dynamic_max_qfunc", "qa_fmo_mo_qfunc",
+                                                             "_static_params"))
 
 
 class LinearFPxAcc(torch.nn.Linear):

@@ -521,6 +521,17 @@ int fmsmo_small_linear_i8(const void* x, int x_dtype, int64_t ldx, const void* s
 int fmsmo_small_linear_fp8(const void* x, int x_dtype, int64_t ldx, const uint8_t* w, int64_t ldw, const float* w_scale,
                            int64_t w_scale_n, const void* bias, int bias_dtype, void* y, int y_dtype, int64_t ldy,
                            float* a_scale_out, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream);
+/*
+ * The same with the static quantizer FMSMO_SQ_FMO in fp32 (step = quant_stepsize, zp = quant_zero_point, see
+ * fmsmo_quant_act_i8_static_t) and one dequantizing scale a_scale, where fmsmo_small_linear_static_ok != 0: up to 16 tokens of up to 3072 elements (16384 in
+ * all, rounded up to 512 each), at most 8192 outputs but for four tokens of 1024, and parameters inside the range of its short division (|step| in 2^-20 .. 2^20, finite clip values, quotients and
+ * zero point under 10^6).
+ */
+int fmsmo_small_linear_static_ok(int64_t M, int64_t N, int64_t K, float step, float zp, float clip_lo, float clip_hi);
+int fmsmo_small_linear_i8_static(const void* x, int x_dtype, int64_t ldx, float step, float zp, int sym, float clip_lo,
+                                 float clip_hi, float a_scale, const int8_t* w, int64_t ldw, const float* w_scale,
+                                 int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue, void* y, int y_dtype,
+                                 int64_t ldy, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------
  * 4. Chunked reduced-precision accumulation ("chunk-truncate") matmuls.

@@ -177,3 +177,86 @@ def test_what_is_left_to_the_two_calls():
     assert not lib.fmsmo_small_linear_ok(1, 4096, 5377, 0) and not lib.fmsmo_small_linear_ok(9, 64, 512, 0)
     assert not lib.fmsmo_small_linear_ok(2, 8200, 1024, 0) and lib.fmsmo_small_linear_ok(2, 8200, 4096, 0)
     assert not lib.fmsmo_small_linear_ok(1, 4096, 2048, 1) and lib.fmsmo_small_linear_ok(1, 4096, 4096, 1)
+
+
+PARAMS = [(7 / 255, -109.0, 0, -3.0, 4.0), (0.0123, 0.0, 1, -1.5, 1.5), (2.0 ** -20, -0.5, 0, -0.25, 0.5), (300.0, 3.25, 1, -6e4, 6e4)]
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("par", PARAMS)
+def test_static_codes_in_fp32(dev, dt, par):
+    """The kernel with the short division (contiguous rows) against the one with the IEEE division (rows of another stride), on every
+    16-bit pattern, and both against torch on the CPU."""
+    from fms_mo_amd import _lib as L
+    from fms_mo_amd import kernels as kn
+
+    step, zp, sym, lo, hi = par
+    x = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dt).reshape(64, 1024)
+    wide = torch.zeros(64, 1032, dtype=dt, device=dev)
+    wide[:, :1024] = x.to(dev)
+    args = (L.SQ_FMO, torch.float32, step, zp, sym, lo, hi)
+    q = kn.quant_act_i8_static_t(x.to(dev), *args)
+    assert torch.equal(q, kn.quant_act_i8_static_t(wide[:, :1024], *args))
+    f = torch.tensor
+    t = x.float().clamp(lo, hi) / f(step) - f(zp)
+    ok = ~torch.isnan(x.float())  # (the kernels take NaN for the lower clip value)
+    want = (torch.round(t) - (128 - sym)).nan_to_num(0).to(torch.int32).to(torch.int8)
+    assert torch.equal(q.cpu()[ok], want[ok])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 16), (1, 100, 2064), (3, 23, 528), (4, 9000, 1024), (8, 300, 2048), (16, 4100, 640), (2, 72, 3072)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_int8_with_the_static_quantizer(dev, M, N, K, dt):
+    from fms_mo_amd import _lib as L
+    from fms_mo_amd import kernels as kn
+
+    x = (3 * torch.randn(M, K, generator=gen(41))).to(dt).to(dev)
+    x[0, 1], x[0, K - 1], x[M - 1, 3] = float("inf"), -float("inf"), float("nan")
+    w = torch.randint(-127, 128, (N, K), generator=gen(42), dtype=torch.int8).to(dev)
+    sw, b = (torch.rand(N, generator=gen(43)) * 1e-3).to(dev), torch.randn(N, generator=gen(44)).to(dt).to(dev)
+    for step, zp, sym, lo, hi in PARAMS[:2]:
+        assert L.load().fmsmo_small_linear_static_ok(M, N, K, step, zp, lo, hi)
+        q = kn.quant_act_i8_static_t(x, L.SQ_FMO, torch.float32, step, zp, sym, lo, hi)
+        want = kn.gemm_i8_dq(q, w, torch.tensor([0.0274], device=dev), sw, b, out_dtype=torch.float16, exact_ref=True)
+        y = torch.empty(M, N, dtype=torch.float16, device=dev)
+        L.call("fmsmo_small_linear_i8_static", x.data_ptr(), kn._dt(x), K, step, zp, sym, lo, hi, 0.0274, w.data_ptr(), K,
+               sw.data_ptr(), N, b.data_ptr(), kn._dt(b), L.EPI_REF_F16, y.data_ptr(), 0, N, M, N, K,
+               torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,K", [(2, 640), (50, 1040), (3, 4096)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_forward_of_a_static_linear(dev, M, K, bias, monkeypatch):
+    """The native forward against the general one, before and after the module's parameters are written to."""
+    import types
+
+    from fms_mo_amd import _lib, kernels
+    from fms_mo_amd.modules.linear import QLinear, QLinearINT8Deploy
+
+    q = QLinear(K, 200, bias=bias, num_bits_feature=8, qa_mode="maxmin", num_bits_weight=8, qw_mode="maxperCh",
+                qcfg={"smoothq": False}, device=dev).to(dev).bfloat16()
+    q.quantize_weight.float(), q.quantize_feature.float()
+    with torch.no_grad():
+        q.quantize_weight.clip_val.copy_(q.weight.abs().amax(dim=1))
+        q.quantize_feature.clip_valn.fill_(-3.0), q.quantize_feature.clip_val.fill_(4.0)
+    m = QLinearINT8Deploy.from_fms_mo(q.eval()).bfloat16()
+    x = torch.randn(M, K, generator=gen(51)).bfloat16().to(dev)
+    stub = types.SimpleNamespace(**{n: (lambda *a: None) for n in dir(_lib.host()) if not n.startswith("_")})
+
+    def general():
+        with monkeypatch.context() as c:
+            c.setattr(_lib, "_host", stub), c.setattr(kernels, "_H", stub)
+            return m(x)
+
+    m(x)  # (the parameters are read)
+    assert _lib.host().deploy_i8(m.__dict__, x, QLinearINT8Deploy, __import__("fms_mo_amd.modules.linear", fromlist=["x"])._OWN_METHODS) is not None
+    assert torch.equal(m(x), general())
+    m.input_scale.mul_(2)
+    assert torch.equal(m(x), general())
+    m.cvs[0] = m.cvs[0] * 0.5
+    assert torch.equal(m(x), general())
+    m.quant_stepsize = m.quant_stepsize * 3
+    assert torch.equal(m(x), general()) and torch.equal(m(x), general())
+    m.qa_fmo_mo_qfunc = lambda t: torch.zeros(t.shape, dtype=torch.int8, device=t.device)
+    assert torch.equal(m(x), general())
