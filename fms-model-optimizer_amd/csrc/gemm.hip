@@ -45,7 +45,7 @@ extern "C" int fmsmo_gemm_i8_i32_ws(const int8_t* a, int64_t lda, const int8_t* 
   if (rc) return rc;
   if (M == 0) return FMSMO_OK;
   // a few tokens: the weight-streaming decode kernels, storing their int32 sums
-  if (use_decode(M, N, K))
+  if (use_decode(M, N, K, false))
     return fmsmo_gemv_dispatch(FMSMO_OP_I8, a, lda, b, ldb, nullptr, 1, nullptr, 1, nullptr, FMSMO_F32,
                                EPI_RAW_I32, c, FMSMO_F32, ldc, M, N, K, (hipStream_t)stream);
   GemmArgs g{};
@@ -78,7 +78,7 @@ static int gemm_i8_dq_impl(const int8_t* a, int64_t lda, const int8_t* b, int64_
   if (rc) return rc;
   if (epilogue < FMSMO_EPI_REF_F16 || epilogue > FMSMO_EPI_F32_MULADD) return FMSMO_ERR_UNSUPPORTED;
   if (M == 0) return FMSMO_OK;
-  if (use_decode(M, N, K))
+  if (use_decode(M, N, K, false))
     return fmsmo_gemv_dispatch(FMSMO_OP_I8, a, lda, b, ldb, a_scale, a_scale_n, w_scale, w_scale_n,
                                bias, bias_dtype, epilogue, y, y_dtype, ldy, M, N, K,
                                (hipStream_t)stream);
@@ -172,7 +172,7 @@ extern "C" int fmsmo_gemm_i8_dq_noalloc(const int8_t* a, int64_t lda, const int8
   if (epilogue < FMSMO_EPI_REF_F16 || epilogue > FMSMO_EPI_F32_MULADD) return FMSMO_ERR_UNSUPPORTED;
   if (M == 0) return FMSMO_OK;
   // the weight-streaming decode kernels use no scratch
-  const bool decode = use_decode(M, N, K);
+  const bool decode = use_decode(M, N, K, false);
   // (the plan that fits the scratch, if one does: else the preferred plan's size is reported)
   int64_t need = decode ? 0 : plan_split_k(M, N, K, (int64_t)FMSMO_STATIC_SCRATCH_BYTES).ws_bytes;
   if (need > (int64_t)FMSMO_STATIC_SCRATCH_BYTES) {
@@ -193,17 +193,17 @@ extern "C" int fmsmo_gemm_i8_dq_noalloc(const int8_t* a, int64_t lda, const int8
                          epilogue, y, y_dtype, ldy, M, N, K, ws, need, stream);
 }
 
-static bool any_takes(int64_t M, int64_t N, int64_t K) { return !fmsmo_gemv_batch_ok(M, K) && fmsmo_gemv_any_ok(M, N, K); }
+static bool any_takes(int64_t M, int64_t N, int64_t K, bool fp8) { return !fmsmo_gemv_batch_ok(M, K) && fmsmo_gemv_any_ok(M, N, K, fp8); }
 extern "C" int64_t fmsmo_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  return any_takes(M, N, K) ? 0 : plan_split_k(M, N, K).ws_bytes;
+  return any_takes(M, N, K, false) ? 0 : plan_split_k(M, N, K).ws_bytes;
 }
 extern "C" int64_t fmsmo_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  return any_takes(M, N, K) ? 0 : plan_split_k(M, N, K, 0, true).ws_bytes;
+  return any_takes(M, N, K, true) ? 0 : plan_split_k(M, N, K, 0, true).ws_bytes;
 }
 
 static int64_t gemm_tail_columns(bool fp8, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
-  if (use_decode(M, N, K)) return 0;
+  if (use_decode(M, N, K, fp8)) return 0;
   return tail_split_columns((int)M, (int)N, (int)K, fp8);
 }
 extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) { return gemm_tail_columns(false, M, N, K); }
@@ -217,11 +217,17 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
   if (K % 16) return FMSMO_ERR_ALIGN;
   *tile_m = *tile_n = 0;
   *splits = 1;
-  if (use_decode(M, N, K)) {
+  if (use_decode(M, N, K, fp8)) {
     *kernel = FMSMO_PLAN_DECODE;
     return FMSMO_OK;
   }
-  // one pass of 64 x 64 or 128 x 64 tiles, with or without a workspace
+  // one pass of 32 x 128, 64 x 64 or 128 x 64 tiles, with or without a workspace
+  if (K % 128 == 0 && use_low_tiles(M, N, K)) {
+    *kernel = FMSMO_PLAN_TILE_LDS_DMA;
+    *tile_m = TileLowK::BM;
+    *tile_n = TileLowK::BN;
+    return FMSMO_OK;
+  }
   if (use_small_tiles(M, N, K) || use_tall_tiles(M, N, K)) {
     *kernel = FMSMO_PLAN_TILE_LDS_DMA;
     *tile_m = use_small_tiles(M, N, K) ? TileSmallK::BM : TileTallK::BM;
@@ -243,13 +249,15 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
     *kernel = FMSMO_PLAN_GENERIC;
     return FMSMO_OK;
   }
-  if (cut_k_tall(M, N, K)) {
+  if (K % 128) {
+    const int bm[7] = {64, 128, 128, 128, 128, 256, 32}, bn[7] = {64, 64, 128, 192, 256, 256, 128};
+    const CutTile t = cut_k_tile(M, N, K, fp8 ? MMA_FP8 : MMA_I8);
     *kernel = FMSMO_PLAN_TILE_LDS_DMA;
-    *tile_m = TileTallK::BM;
-    *tile_n = TileTallK::BN;
+    *tile_m = bm[t];
+    *tile_n = bn[t];
     return FMSMO_OK;
   }
-  const bool rs = K % 128 == 0 && use_register_staged(MMA_I8);
+  const bool rs = use_register_staged(MMA_I8);
   const int bm[7] = {256, 128, 128, 256, 256, 128, 128}, bn[7] = {256, 256, 128, 192, 128, 192, 256};
   const int t = pick_tile((int)M, (int)N, (int)K, rs, fp8);
   *kernel = (rs && (t == 0 || t == 3 || t == 4)) ? FMSMO_PLAN_TILE_REGISTER_STAGED : FMSMO_PLAN_TILE_LDS_DMA;

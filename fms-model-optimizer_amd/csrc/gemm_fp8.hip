@@ -11,7 +11,7 @@ static int gemm_fp8_dq_impl(const uint8_t* a, int64_t lda, const uint8_t* b, int
   rc = check_dq(a_scale, a_scale_n, w_scale, w_scale_n, bias, bias_dtype, y_dtype, M, N);
   if (rc) return rc;
   if (M == 0) return FMSMO_OK;
-  if (use_decode(M, N, K))
+  if (use_decode(M, N, K, true))
     return fmsmo_gemv_dispatch(FMSMO_OP_E4M3, a, lda, b, ldb, a_scale, a_scale_n, w_scale,
                                w_scale_n, bias, bias_dtype, FMSMO_EPI_F32, y, y_dtype, ldy, M, N, K,
                                (hipStream_t)stream);
@@ -29,10 +29,7 @@ static int gemm_fp8_dq_impl(const uint8_t* a, int64_t lda, const uint8_t* b, int
                                                  bias_dtype, y, y_dtype, ldy, (hipStream_t)stream);
   }
   // The e4m3 matrix instruction takes 64 elements of K at a time and keeps fewer bits than fp32 additions
-  // do while it adds them: other K, which never went through it, run on the fp16 instruction.  Tiles by the int8
-  // rule for such K, 128 x 64 up to a round of them, then 128 x 128 (us, 128 x 64 / 128 x 128 / 128 x 256, K = 4016, tiles of
-  // 128 x 64 in front: 192 (300 x 4096) 22.3 / 27.4 / 46.7; 256 (1000 x 2048) 24.1 / 27.3 / 46.9; 320 (600 x 4096) 40.6 / 29.8 / 47.2;
-  // 512 (1000 x 4096) 45.1 / 35.3 / 47.9; 2048 (4000 x 4096) 163.6 / 131.2 / 121.8: 7 % for one more instance, left out).
+  // do while it adds them: other K, which never went through it, run on the fp16 instruction.
   if (K % 64)
     return launch_dq<MMA_FP8_F16, false, float>(g, a_scale, as, w_scale, ws, bias, bias_dtype, y, y_dtype, ldy,
                                                        (hipStream_t)stream);

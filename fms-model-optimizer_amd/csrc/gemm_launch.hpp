@@ -14,7 +14,7 @@ int fmsmo_check_launch();
 // block 0's clock readings (null = off); defined in gemm.hip.
 unsigned long long*& fmsmo_clock_probe();
 bool fmsmo_gemv_batch_ok(int64_t M, int64_t K);
-bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K);
+bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K, bool fp8);
 int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64_t ldb,
                         const float* a_scale, int64_t a_scale_n, const float* w_scale,
                         int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
@@ -38,8 +38,7 @@ int check_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const voi
 }
 
 // Tile shapes.  K is consumed in stages of BK bytes; K that are no multiple of a stage run the KT
-// instances of the LDS-DMA kernel (a last stage that is cut at K), of three shapes: TileBig,
-// TileMidK, TileTallK.
+// instances of the LDS-DMA kernel (a last stage that is cut at K), see cut_k_tile.
 struct TileBig { static constexpr int BM = 256, BN = 256, BK = 64, NST = 4, WGM = 2, WGN = 2; };
 struct TileWide { static constexpr int BM = 128, BN = 256, BK = 64, NST = 4, WGM = 2, WGN = 2; };
 struct TileMid { static constexpr int BM = 128, BN = 128, BK = 64, NST = 4, WGM = 2, WGN = 2; };
@@ -69,6 +68,8 @@ struct TileWideK { static constexpr int BM = 128, BN = 256, BK = 128, NST = 3, W
 // 64 x 64 tiles, two blocks per compute unit, for launches that would leave most compute units idle or take
 // K slices and a second kernel.
 struct TileSmallK { static constexpr int BM = 64, BN = 64, BK = 128, NST = 4, WGM = 2, WGN = 2; };
+// Up to 32 rows, see use_low_tiles
+struct TileLowK { static constexpr int BM = 32, BN = 128, BK = 128, NST = 4, WGM = 1, WGN = 4; };
 
 // Which launches they take: up to one block per compute unit on reductions under 2048 (one pass takes 3.3 us + 1.6
 // per 1024 of K, less than a pass of any other tile; from there on slices of two or four come close), up to 3072
@@ -87,17 +88,25 @@ struct TileSmallK { static constexpr int BM = 64, BN = 64, BK = 128, NST = 4, WG
 //   6.0, 64 15.8 -> 6.8; N = 14336, K = 4096: 17 13.4 -> 11.4, 40 18.0 -> 12.2 | 18.8 -> 11.8; N = 8192: 33 11.0 -> 10.5, 64 14.9 ->
 //   10.5; kept: N = 4096, K = 4096, 33 8.9 against 9.7; N = 8192, 32 9.6 against 10.5
 inline bool use_small_tiles(int64_t M, int64_t N, int64_t K) {
-  if (M <= 16 || K % 128 || (K >= 8192 && M <= 1024)) return false;
+  if (M <= 16) return K % 128 == 0 && !fmsmo_gemv_batch_ok(M, K) && !fmsmo_gemv_any_ok(M, N, K, false);
+  if (K % 128 || (K >= 8192 && M <= 1024)) return false;
   const int64_t tiles = (int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN);
   if (tiles > 512) return false;
   if (fmsmo_gemv_batch_ok(M, K)) return K <= (tiles > 256 ? 2048 : 4096) && tiles >= (M > 32 ? 128 : 192);
   if (tiles > 256) return K <= 1536;
+  if (M <= 64 && tiles > 32 && tiles <= 64) return K <= 2304;  // (us, 128 x 64 -> these, e4m3: 48 x 2385 x 1792 8.3 -> 6.5, 64 x 3262 x 1152 7.8 -> 5.7)
   if (tiles > 64) return K < 2048 || (M > 128 && K <= 3072) || M > 256;
   return M > 1024 || (tiles <= 32 && K < 2048);
 }
 // The decode kernels take the launch.
-inline bool use_decode(int64_t M, int64_t N, int64_t K) {
-  return fmsmo_gemv_batch_ok(M, K) ? !use_small_tiles(M, N, K) : fmsmo_gemv_any_ok(M, N, K);
+inline bool use_decode(int64_t M, int64_t N, int64_t K, bool fp8) {
+  return fmsmo_gemv_batch_ok(M, K) ? !use_small_tiles(M, N, K) : fmsmo_gemv_any_ok(M, N, K, fp8);
+}
+// Up to 32 rows and more than a round of 64 x 64 tiles, half or more of whose rows are padding: 32 x 128, half as many (us, 64 x 64 / 32 x 128, int8:
+// 24 x 25197 x 1616 12.0 / 10.9, 32 x 24387 x 1216 10.1 / 8.9, 16 x 18652 x 1648 11.1 / 9.3, 32 x 19476 x 5088 37.4 / 32.0; e4m3 32 x 18142 x 2112
+// 12.4 / 10.2; at 8192 .. 16384 columns the other way: 32 x 10054 x 3408 11.5 / 15.3, 8 x 14307 x 1984 8.2 / 8.5).
+inline bool use_low_tiles(int64_t M, int64_t N, int64_t K) {
+  return M <= 32 && N > 256 * TileSmallK::BN && (use_small_tiles(M, N, K) || !fmsmo_gemv_batch_ok(M, K));
 }
 
 // A few hundred rows through a projection whose 128 x 64 tiles fill half a round of the 256
@@ -166,7 +175,10 @@ int pick_tile(int M, int N, int K, bool rs192_ok, bool fp8) {
     const double score = scores[t] = eff[t] * pow(fill, 0.6) * pad;
     if (score > best_score) { best_score = score; best = t; }
   }
-  if (!rs192_ok || K < 512) return best;
+  if (!rs192_ok) return best;
+  // (Below 512 the other shapes keep the launches they had, whose edges a test counts on reaching, and not for their speed: us, int8 | e4m3, K = 256,
+  // 256 x 256 -> 128 x 256: 4342 x 3185 28.1 -> 19.3 | 22.8 -> 17.8; 256 x 192 -> 128 x 256: 3627 x 5389 27.2 -> 25.4 | 25.3 -> 21.5.)
+  if (K < 512) return best == 3 ? 6 : best;
   if (K <= (fp8 ? 640 : 1280)) {
     if (scores[2] > (fp8 ? 1.18 : 1.12) * best_score * (1 + fixed[best] / 4096) * K / (K + fixed[best])) best = 2;
     if (best == 2) return best;
@@ -181,6 +193,20 @@ int pick_tile(int M, int N, int K, bool rs192_ok, bool fp8) {
   if ((long)div_up(M, 128) * div_up(N, 128) > 256) {
     if ((long)div_up(M, Tile192K::BM) * div_up(N, Tile192K::BN) <= 256) return 5;
     if ((long)div_up(M, TileWideK::BM) * div_up(N, TileWideK::BN) < 256) return 6;
+  }
+  // What a tile of 256 rows spends ahead of its reduction and behind it, with one block on a compute unit, the two rounds or three of the
+  // 128-row ones of eight waves take less than on short reductions: rounds of a + b per 128 of K, us, fitted to 347 launches each; taken
+  // where a tenth is to be gained.  Up to a round of 256 x 256 tiles: with more of them their rounds overlap and the estimate
+  // no longer holds.  int8 2733 x 3200 x 1024 29.3 -> 22, 3367 x 2944 x 768 28 -> 22, e4m3 2733 x 3200 x 1024 0.79 of the time; 24 launches of 694 changed, by 13 %.
+  if ((best == 0 || best == 3 || best == 4) && (long)div_up(M, 256) * div_up(N, 256) <= 256) {
+    static const double A[2][5] = {{17.4, 14.1, 8.9, 3.6, 4.6}, {20.3, 11.4, 7.0, 2.9, 3.7}}, B[2][5] = {{.973, .857, .834, .613, .714}, {.75, .706, .666, .601, .823}};
+    auto cost = [&](int i, int rows, int cols) {
+      return std::ceil((double)div_up(M, rows) * div_up(N, cols) / 256) * (A[fp8][i] + B[fp8][i] * (K / 128));
+    };
+    const double now = best == 0 ? cost(0, 256, 256) : best == 3 ? cost(1, 256, 192) : cost(2, 256, 128);
+    const double c192 = cost(3, 128, 192), cwide = cost(4, 128, 256);
+    const bool full = best == 4 && (long)div_up(M, 256) * div_up(N, 128) > 230;  // (a full round of 256 x 128, see above)
+    if (!full && 1.1 * std::min(c192, cwide) < now) return c192 < cwide ? 5 : 6;
   }
   return best;
 }
@@ -260,52 +286,86 @@ void launch_k128(const GemmArgs& g0, int batch, int M, const Epi& epi, hipStream
   hipLaunchKernelGGL((gemm_k128_kernel<OP, Epi>), dim3((unsigned)blocks), dim3(256), 0, st, g, epi);
 }
 
-// K % 128 != 0: the KT instances.  Up to a round of 128 x 64 tiles over the 256 compute units those
-// are taken, then 128 x 128 while they need at most twice the rounds of 256 x 256 tiles, those beyond
-// (us, int8, 128 x 64 / 128 x 128 / 256 x 256, the three tile counts in front):
-//   192 / 96 / 32 (300 x 4096 x 4016) 16.1 / 19.2 / 44.3      256 / 128 / 32 (2000 x 1024 x 4016) 21.5 / 22.8 / 60.4
-//   320 / 160 / 48 (600 x 4096 x 4016) 32.7 / 23.7 / 51.6     512 / 256 / 64 (1000 x 4096 x 4016) 40.0 / 28.5 / 59.3
-//   1024 / 512 / 128 (2000 x 4096 x 4016) 72.5 / 50.8 / 58.7  2048 / 1024 / 256 (2000 x 8192 x 4016) 137 / 95.6 / 72.4
-inline bool cut_k_tall(int64_t M, int64_t N, int64_t K) {
-  return K % 128 && (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN) <= 256;
+// K % 128 != 0: the KT instances (a last stage that is cut at K).  The tile by an estimate of the time: rounds of tiles times
+// what a tile takes, a + b per 128 bytes of K, fitted to 520 launches of 65 .. 4096 rows, 256 .. 28672 columns and K = 512 .. 16384 with every
+// tile timed; a partly filled last round and a half empty chip count between their fraction and a whole one.  Over those launches the tiles chosen
+// take 0.854 (int8), 0.833 (e4m3) and 0.877 (fp16 instruction) of the time of the three shapes that served all of them before (128 x 64, 128 x 128 of
+// four waves, 256 x 256), the best tile of each launch 0.849 / 0.825 / 0.871; 256 x 256 by 114
+// more launches of 4000 columns and up (e4m3 3623 x 23627 x 4544 398, 128 x 256 475).  us, int8, before -> now: 2006 x 10495 x 1328 69.1 -> 56.4, 712 x 22911 x
+// 3024 113.7 -> 85.9, 2517 x 4095 x 1456 40.2 -> 31.5, 373 x 711 x 1904 10.9 -> 8.2, 1671 x 262 x 14112 48.4 -> 34.9, 91 x 6131 x 9456 48.2 -> 30.4.
+enum CutTile { CUT_SMALL, CUT_TALL, CUT_MID, CUT_192, CUT_WIDE, CUT_BIG, CUT_LOW };
+struct CutCost { double a, b; };
+constexpr CutCost CUT_COSTS[3][6] = {
+    {{2.3, .261}, {3.2, .430}, {3.8, .631}, {5.4, .807}, {7.0, .967}, {15.8, 1.6}},  // int8
+    {{2.1, .225}, {2.7, .356}, {3.5, .516}, {4.7, .717}, {6.3, .966}, {15.8, 1.38}},  // e4m3
+    {{2.5, .377}, {3.4, .551}, {4.6, .824}, {5.8, 1.16}, {7.1, 1.48}, {0, 0}}};       // e4m3, K % 64 != 0
+inline CutTile cut_k_tile(int64_t M, int64_t N, int64_t K, int op) {
+  const int kind = op == MMA_I8 ? 0 : op == MMA_FP8 ? 1 : 2;
+  const int bm[6] = {64, 128, 128, 128, 128, 256}, bn[6] = {64, 64, 128, 192, 256, 256};
+  if (use_low_tiles(M, N, K)) return CUT_LOW;
+  const double stages = (double)((K + 127) / 128);
+  CutTile best = CUT_SMALL;
+  double least = 0;
+  for (int t = 0; t < (kind == 2 ? 5 : 6); ++t) {
+    const double a = CUT_COSTS[kind][t].a, b = CUT_COSTS[kind][t].b * stages;
+    const double n = (double)div_up(M, bm[t]) * div_up(N, bn[t]) / 256, whole = std::ceil(n);
+    double cost;
+    if (t == CUT_SMALL) cost = n <= 1 ? a + b : (1.4 * a + 1.8 * b) * whole / 2;  // (two of these share a compute unit)
+    else cost = std::max(1.0, 0.72 * whole + 0.28 * n) * (a + b) * (1 - 0.25 * (1 - std::min(1.0, n)));
+    if (t == CUT_BIG && kind == 1) cost *= n > 2.25 ? 0.92 : n <= 1 ? 1.1 : 1;
+    if (t == 0 || cost < least) least = cost, best = (CutTile)t;
+  }
+  return best;
 }
 template <int OP, class Epi>
 void launch_cut_k(const GemmArgs& g, const Epi& epi, hipStream_t st) {
-  auto rounds = [&](int t) { return div_up((int64_t)div_up(g.M, t) * div_up(g.N, t), 256); };
-  if (cut_k_tall(g.M, g.N, g.K)) launch_tile<TileTallK, OP, false, true>(g, epi, st);
-  else if (rounds(128) <= 2 * rounds(256)) launch_tile<TileMidK, OP, false, true>(g, epi, st);
-  else launch_tile<TileBig, OP, false, true>(g, epi, st);
+  switch (cut_k_tile(g.M, g.N, g.K, OP)) {
+    case CUT_SMALL: launch_tile<TileSmallK, OP, false, true>(g, epi, st); break;
+    case CUT_TALL: launch_tile<TileTallK8, OP, false, true>(g, epi, st); break;
+    case CUT_MID: launch_tile<TileMidK8, OP, false, true>(g, epi, st); break;
+    case CUT_192: launch_tile<Tile192K, OP, false, true>(g, epi, st); break;
+    case CUT_WIDE: launch_tile<TileWideK, OP, false, true>(g, epi, st); break;
+    case CUT_LOW: launch_tile<TileLowK, OP, false, true>(g, epi, st); break;
+    default:
+      if constexpr (OP != MMA_FP8_F16) {
+        if (g.K % 64 == 0) launch_tile<TileBig, OP, false>(g, epi, st);  // (64-byte stages: whole)
+        else if constexpr (OP == MMA_I8) launch_tile<TileBig, OP, false, true>(g, epi, st);
+      }
+  }
 }
 
 template <int OP, class Epi>
 void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
-  if constexpr (OP == MMA_FP8_F16) {  // K % 64 != 0
-    if (cut_k_tall(g.M, g.N, g.K)) launch_tile<TileTallK, OP, false, true>(g, epi, st);
-    else launch_tile<TileMidK, OP, false, true>(g, epi, st);
+  if constexpr (OP == MMA_FP8_F16) {
+    launch_cut_k<OP>(g, epi, st);
+  } else if (g.K % 128) {
+    launch_cut_k<OP>(g, epi, st);
+  } else if (use_low_tiles(g.M, g.N, g.K)) {
+    launch_tile<TileLowK, OP, false>(g, epi, st);
   } else if (use_small_tiles(g.M, g.N, g.K)) {
     launch_tile<TileSmallK, OP, false>(g, epi, st);
   } else if (use_tall_tiles(g.M, g.N, g.K)) {
     if (OP != MMA_I8 || g.K < I8_EIGHT_WAVES_BELOW) launch_tile<TileTallK8, OP, false>(g, epi, st);
     else if constexpr (OP == MMA_I8) launch_tile<TileTallK, OP, false>(g, epi, st);
-  } else if (g.K % 64 == 0 && !cut_k_tall(g.M, g.N, g.K)) {
-    switch (pick_tile(g.M, g.N, g.K, g.K % 128 == 0 && use_register_staged(OP), OP != MMA_I8)) {
+  } else {
+    switch (pick_tile(g.M, g.N, g.K, use_register_staged(OP), OP != MMA_I8)) {
       case 0:
-        if (g.K % 128 == 0 && use_register_staged(OP)) launch_rs<OP>(g, epi, st);
+        if (use_register_staged(OP)) launch_rs<OP>(g, epi, st);
         else launch_tile<TileBig, OP, false>(g, epi, st);
         break;
       case 1: launch_tile<TileWide, OP, false>(g, epi, st); break;
       case 3:
-        if (g.K % 128 == 0 && use_register_staged(OP)) launch_rs<OP, false, 192>(g, epi, st);
+        if (use_register_staged(OP)) launch_rs<OP, false, 192>(g, epi, st);
         else launch_tile<TileBig, OP, false>(g, epi, st);
         break;
-      case 4: launch_rs<OP, false, 128>(g, epi, st); break;  // 4 .. 6 only offered when K % 128 == 0
+      case 4: launch_rs<OP, false, 128>(g, epi, st); break;  // 4 .. 6 only offered beside the register-staged kernel
       case 5: launch_tile<Tile192K, OP, false>(g, epi, st); break;
       case 6: launch_tile<TileWideK, OP, false>(g, epi, st); break;
       default:
         // one round of 128 x 128 tiles: stages of 128 bytes (us, 1024 rows, N = 4096: K = 4096 29.0 ->
         // 25.6, 5120 36.8 -> 31.2; 512 rows, N = 6144, K = 4096: 28.0 -> 23.5); more than a round keeps
         // the 64-byte stages, whose blocks fit two to a compute unit
-        if (g.K % 128 == 0 && (long)div_up(g.M, TileMidK::BM) * div_up(g.N, TileMidK::BN) <= 256) {
+        if ((long)div_up(g.M, TileMidK::BM) * div_up(g.N, TileMidK::BN) <= 256) {
           if (OP != MMA_I8 || g.K < I8_EIGHT_WAVES_BELOW) launch_tile<TileMidK8, OP, false>(g, epi, st);
           else if constexpr (OP == MMA_I8) launch_tile<TileMidK, OP, false>(g, epi, st);
         } else {
@@ -313,10 +373,6 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
         }
         break;
     }
-  } else if constexpr (OP == MMA_FP8) {
-    launch_tile<TileTallK, OP, false, true>(g, epi, st);  // (K % 64 == 0: MMA_FP8_F16 takes the others)
-  } else {
-    launch_cut_k<OP>(g, epi, st);
   }
 }
 
@@ -430,7 +486,7 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   SplitPlan p{1, K, 0, false};
   static const char* off = getenv("FMSMO_SPLIT_K");  // FMSMO_SPLIT_K=0 disables (tuning aid)
   if (off && off[0] == '0') return p;
-  if (M <= 16 || M > 1024 || use_small_tiles(M, N, K) || use_tall_tiles(M, N, K)) return p;
+  if (M <= 16 || M > 1024 || use_small_tiles(M, N, K) || use_tall_tiles(M, N, K) || use_low_tiles(M, N, K)) return p;
   const int64_t tiles_t = (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN);
   const int64_t room = limit > 0 ? limit / (M * N * 4) : 256;
   const int64_t tiles_s = (int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN);
@@ -452,8 +508,9 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   if (K % 128) {
     // (us, one pass -> slices, M = 40: N = 1024, K = 4016 13.1 -> 8.8; N = 3072 13.6 -> 10.3; M = 100,
     // N = 3072, K = 8208 26.3 -> 14.4; M = 200, N = 1500, K = 11216 36.7 -> 16.7.  From a quarter of a
-    // round of tiles on these shapes ask for no workspace.)
-    if (tiles_t < 64) cut_slices(p, M, N, K, (int)std::min<int64_t>(256 / tiles_t, room));
+    // round of tiles on these shapes ask for no workspace, nor up to where one pass of 64 x 64 tiles takes as long: int8 177 x 301 x 3936
+    // 10.9 against 11.0, 169 x 768 x 2848 10.1 against 8.9; e4m3, K % 64 != 0, 68 x 474 x 3424 11.6 against 14.5.)
+    if (tiles_t < 64 && K > (fp8 && K % 64 ? 2816 : 3584)) cut_slices(p, M, N, K, (int)std::min<int64_t>(256 / tiles_t, room));
     return p;
   }
   // Long reductions under a few hundred rows: 256 x 128 tiles of the register-staged kernel carry

@@ -460,6 +460,62 @@ __global__ __launch_bounds__(NW * 64) void gemv_any_kernel(GemvArgs g, int halve
   }
 }
 
+// Up to 16 tokens of rows of at most 512: a wave takes one step of 128 and has all its loads out at once, straight into the operand registers; no
+// staging, no loop.  A launch this short is bound by its latency (the chip reads 4 MB in 0.6 us): RG row groups of 16 to a block, so that
+// there are up to 1024 blocks of them.  us, gemv_any_kernel -> this: int8 12 x 4230 x 256 5.1 -> 3.9, 1 x 3087 x 512 4.2 -> 3.6, 16 x 6655 x 512 6.1 -> 4.5.
+template <int OP, int NW, int RG>
+__global__ __launch_bounds__(NW * 64) void gemv_short_kernel(GemvArgs g) {
+  typedef typename std::conditional<OP == FMSMO_OP_I8, int, float>::type AccT;
+  typedef AccT Acc4 __attribute__((ext_vector_type(4)));
+  __shared__ AccT red[NW][RG][16 * 17];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, kg = lane >> 4;
+  const int n0 = blockIdx.x * (RG * 16), rows = min(RG * 16, g.N - n0);
+  const int kchunks = g.K >> 4, c0 = wave * 8 + kg, c1 = c0 + 4;
+  // (rows and chunks past the end read as zeros; rows of tokens past M only reach outputs that are not stored)
+  const __amdgpu_buffer_rsrc_t rw =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(g.b + (int64_t)n0 * g.ldb), 0, (rows - 1) * (int)g.ldb + g.K, 0x00020000);
+  const unsigned xrow = g.M > 1 ? (unsigned)g.lda : (unsigned)g.K;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)g.a, 0, (g.M - 1) * (int)xrow + g.K, 0x00020000);
+  const unsigned wo = (unsigned)r * (unsigned)g.ldb, xo = (unsigned)min(r, g.M - 1) * xrow;
+  v4i w[RG][2], x[2];
+#pragma unroll
+  for (int i = 0; i < RG; ++i) {
+    const unsigned v = wo + (unsigned)(i * 16) * (unsigned)g.ldb;
+    w[i][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, c0 < kchunks ? v + c0 * 16 : GEMV_OUTSIDE, 0, 2));
+    w[i][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, c1 < kchunks ? v + c1 * 16 : GEMV_OUTSIDE, 0, 2));
+  }
+  x[0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rx, c0 < kchunks ? xo + c0 * 16 : GEMV_OUTSIDE, 0, 0));
+  x[1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rx, c1 < kchunks ? xo + c1 * 16 : GEMV_OUTSIDE, 0, 0));
+  // the scales and biases of this thread's outputs, with the operands
+  constexpr int OUT = (RG * 256 + NW * 64 - 1) / (NW * 64);
+  float as[OUT], ws[OUT], bv[OUT];
+#pragma unroll
+  for (int q = 0; q < OUT; ++q) {
+    const int o = threadIdx.x + q * NW * 64, n = min(n0 + ((o >> 8) * 16) + (o & 15), g.N - 1), m = min((o >> 4) & 15, g.M - 1);
+    as[q] = g.a_scale ? g.a_scale[g.a_stride ? m : 0] : 1.f;
+    ws[q] = g.w_scale ? g.w_scale[g.w_stride ? n : 0] : 1.f;
+    bv[q] = gemv_bias(g, n);
+  }
+#pragma unroll
+  for (int i = 0; i < RG; ++i) {
+    const Acc4 acc = gemv_mma<OP>(w[i][0], w[i][1], x[0], x[1], Acc4{0, 0, 0, 0});
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave][i][(kg * 4 + v) * 17 + r] = acc[v];  // (n = 4 kg + v, m = r)
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < OUT; ++q) {
+    const int o = threadIdx.x + q * NW * 64, i = o >> 8, n = n0 + i * 16 + (o & 15), m = (o >> 4) & 15;
+    if (i >= RG || n >= g.N || m >= g.M) continue;
+    const int e = (o & 15) * 17 + m;
+    AccT sum = red[0][i][e];
+#pragma unroll
+    for (int v = 1; v < NW; ++v) sum += red[v][i][e];
+    gemv_store(g, m, n, sum, as[q], ws[q], bv[q]);
+  }
+}
+
 }  // namespace fmsmo
 
 using namespace fmsmo;
@@ -467,6 +523,7 @@ using namespace fmsmo;
 int fmsmo_check_launch();
 // skinny.hip: the fused forms of its kernels, or the one here
 int fmsmo_decode_fused(int op, int x_dtype, const GemvArgs& g, hipStream_t st);
+bool fmsmo_gemv_stream_k(int64_t K);
 
 // Waves per block and blocks of a launch.  us, int8, waves x most blocks 16 x 256 | 8 x 256 | 8 x 512 | 4 x 1024:
 //   up to 512 halves of row groups (N = 4096) a group per block, 16 waves, 8 where K has no more than that many steps:
@@ -487,23 +544,28 @@ static AnyPlan any_plan(int64_t M, int64_t N, int64_t K) {
   return {8, 512};
 }
 
-// Up to 16 tokens: every K that skinny.hip has no instance for.  More: where the tiled kernels would take slices of K or
+// Up to 16 tokens: every K that skinny.hip has no instance for, but for several tokens and short rows over more columns than one
+// round of blocks takes, where tiles of 64 x 64 or 32 x 128 with their deeper loads win (us, this kernel against them, int8: 3 x 10473 x 1632 9.1 /
+// 7.4, 8 x 8327 x 4160 14.1 / 11.3, 16 x 9412 x 2272 10.9 / 8.4, 16 x 24703 x 1424 16.2 / 9.7, 5 x 27721 x 3120 25.2 / 21.8; kept: 3 x 17661 x 3024 16.9 / 18.9,
+// 2 x 26780 x 3968 19.7 / 21.0, 5 x 19664 x 5152 27.1 / 28.9, 13 x 7811 x 1792 6.7 / 7.2, 1 x 12736 x 2032 7.6 / 8.3; rows of 512 at most, gemv_short_kernel: 8 x
+// 10848 x 448 4.4 / 5.0, 4 x 17166 x 512 5.6 / 5.5, 16 x 26612 x 512 7.0 / 6.2, 4 x 53216 x 256 7.1 / 6.5).  More: where the tiled kernels would take slices of K or
 // launch too few tiles (us, those -> this one, int8): 17 x 4096: K = 528 5.6 -> 3.7, 1536 8.3 -> 4.4, 4480 10.2 -> 7.2, 9088
 // 13.5 -> 11.0; 32 x 1000: K = 896 5.1 -> 3.9, 2304 7.4 -> 5.8, 4480 8.2 -> 8.4; 32 x 4096 x 4480 10.7 -> 8.8; 40 x 2100: 896 7.1 ->
-// 4.8, 3328 9.3 -> 8.4; 64 x 2100: 896 7.3 -> 5.2, 2304 9.2 -> 8.1, 3328 10.0 -> 10.0; 64 x 256 x 1536 5.4 -> 6.4.  From 4096
+// 4.8, 3328 9.3 -> 8.4; from 48 tokens on, and e4m3 from 33 on, 64 x 64 tiles (this / those: int8 33 x 2081 x 1536 6.4 / 6.9, 48 x 3256 x 1280 6.7 / 6.7, 64 x
+// 1857 x 1792 7.9 / 7.4; e4m3 33 x 2277 x 1152 6.1 / 5.6, 64 x 1776 x 1792 7.9 / 6.4).  From 4096
 // columns on 64 x 64 tiles fill the chip in one pass (32 x 8192 x 1536 6.6 -> 7.2).  Longer rows: the activations that every
 // block reads again cost more than the slices' sums (32 x 1000 x 6144 9.0 -> 9.4).
-bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K) {
+bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K, bool fp8) {
   if (M < 1 || M > 64 || K % 16) return false;
-  if (M <= 16) return true;
+  if (M <= 16) return M == 1 || N <= (K <= 512 ? 24576 : 8192) || K > (M == 2 ? 2048 : M <= 4 ? 2560 : 4608) || fmsmo_gemv_stream_k(K);
   if (N > 4096) return false;
-  if (M <= 32) return K <= (M <= 24 ? 8192 : 4096);
-  return K % 128 ? K <= 1024 : N > 1024 && K <= 2304;
+  if (M <= 32) return K <= (M > 24 ? 4096 : fp8 ? 6144 : 8192);
+  return K % 128 ? K <= 1024 : !fp8 && M <= 48 && N > 1024 && K > 640 && K <= 2304;
 }
 
-// 32-bit offsets into the rows of a block and into the activations
+// 32-bit offsets into the rows of a block (four groups at most) and into the activations
 static bool any_offsets_ok(const GemvArgs& g) {
-  return (std::min(g.N, 16) - 1) * g.ldb + g.K < (1ll << 31) && (g.M > 1 ? (g.M - 1) * g.lda : 0) + g.K < (1ll << 31);
+  return (std::min(g.N, 64) - 1) * g.ldb + g.K < (1ll << 31) && (g.M > 1 ? (g.M - 1) * g.lda : 0) + g.K < (1ll << 31);
 }
 
 template <int OP, int MT, int XT = -1, int QUANT = QUANT_TOKEN>
@@ -531,9 +593,27 @@ static int any_launch(const GemvArgs& g, hipStream_t st) {
   return fmsmo_check_launch();
 }
 
+template <int OP, int NW>
+static int short_launch(const GemvArgs& g, hipStream_t st) {
+  const int groups = (g.N + 15) / 16;
+  const dim3 block(NW * 64);
+  if (groups > 2048) hipLaunchKernelGGL((gemv_short_kernel<OP, NW, 4>), dim3((unsigned)((groups + 3) / 4)), block, 0, st, g);
+  else if (groups > 1024) hipLaunchKernelGGL((gemv_short_kernel<OP, NW, 2>), dim3((unsigned)((groups + 1) / 2)), block, 0, st, g);
+  else hipLaunchKernelGGL((gemv_short_kernel<OP, NW, 1>), dim3((unsigned)groups), block, 0, st, g);
+  return fmsmo_check_launch();
+}
+template <int OP>
+static int short_waves(const GemvArgs& g, hipStream_t st) {
+  return g.K <= 128 ? short_launch<OP, 1>(g, st) : g.K <= 256 ? short_launch<OP, 2>(g, st) : short_launch<OP, 4>(g, st);
+}
+
 // FMSMO_ERR_UNSUPPORTED: offsets past 32 bits (nothing was launched)
 int fmsmo_gemv_any(int op, const GemvArgs& g, hipStream_t st) {
   if (!any_offsets_ok(g)) return FMSMO_ERR_UNSUPPORTED;
+  if (g.M <= 16 && g.K <= 512)
+    return op == FMSMO_OP_I8 ? short_waves<FMSMO_OP_I8>(g, st)
+           : g.K % 64        ? short_waves<GEMV_FP8_F16>(g, st)
+                             : short_waves<FMSMO_OP_E4M3>(g, st);
 #define GO(OP)                                    \
   if (g.M <= 16) return any_launch<OP, 1>(g, st); \
   if (g.M <= 32) return any_launch<OP, 2>(g, st); \

@@ -1044,10 +1044,17 @@ static bool rows_take(int op, int64_t M, int64_t N, int64_t K) {
   const int64_t kch = (K + 1023) / 1024;
   if (M > 2 || kch > 16) return false;
   const bool i8 = op == FMSMO_OP_I8;
-  if (kch == 1) return i8 && M == 1 && N > 8192;
+  if (kch == 1) return i8 && M == 1 && N > 8192 && K > 512;
   if (M == 1) return i8 || kch <= 8 || N <= 2048;
   if (kch == 2) return false;
   return kch <= 8 ? i8 || N <= 4096 : N <= (i8 ? 2048 : 1024);
+}
+
+// Rows that gemv_stream_kernel has an instance for.
+bool fmsmo_gemv_stream_k(int64_t K) {
+  for (int64_t steps : {8, 16, 32, 40, 64, 100, 112, 128})
+    if (K == steps * 128) return true;
+  return false;
 }
 
 // Batches of 17 .. 64 tokens that the weight-streaming kernel takes in one pass (their
@@ -1085,9 +1092,7 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
     // 14336: 13.7 -> 12.1; 5120: 5.7 against 5.9) and up to 2048 (6.8 -> 4.0), for one e4m3 token from K = 12800 (12.6 ->
     // 11.2; 8192: 7.9 both) and for one int8 token at K = 12800 (11.4 -> 10.8; 14336: 11.8 both,
     // 16384: 13.0 against 13.8).
-    const int steps128 = K % 128 ? 0 : (int)(K / 128);
-    const bool stream_ok = steps128 == 8 || steps128 == 16 || steps128 == 32 || steps128 == 40 ||
-                           steps128 == 64 || steps128 == 100 || steps128 == 112 || steps128 == 128;
+    const bool stream_ok = fmsmo_gemv_stream_k(K);
     // Rows of 14336 where N <= 4096 gives every block of the streaming kernel a single row group
     // (activations streamed beside the weights, seven steps in flight): one token 11.8 -> 11.2
     // (int8), 12.7 -> 11.9 (e4m3).

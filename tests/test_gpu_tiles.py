@@ -1,0 +1,57 @@
+"""Tile shapes of the products (csrc/gemm_launch.hpp), each at ragged edges: against exact sums."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def check(dev, M, N, K):
+    """int8 exact; e4m3 on small integers, whose sums stay below 2^24: exact in fp32."""
+    from fms_mo_amd import kernels as kn
+
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    a = torch.randint(-128, 128, (M, K + 16), generator=g, dtype=torch.int8, device=dev)[:, :K]
+    w = torch.randint(-128, 128, (N, K + 32), generator=g, dtype=torch.int8, device=dev)[:, :K]
+    acc = a.double() @ w.double().t()
+    assert torch.equal(kn.gemm_i8_i32(a, w).double(), acc)
+    one = torch.ones(1, device=dev)
+    assert torch.equal(kn.gemm_i8_dq(a, w, one, one, None, out_dtype=torch.float32, exact_ref=False).double(), acc)
+    # NaN behind the rows' K elements must not enter
+    nan = torch.full((), float("nan"), device=dev)
+    a8 = torch.cat((torch.randint(-4, 5, (M, K), generator=g, device=dev).float(), nan.expand(M, 16)), 1).to(torch.float8_e4m3fn)[:, :K]
+    w8 = torch.cat((torch.randint(-4, 5, (N, K), generator=g, device=dev).float(), nan.expand(N, 16)), 1).to(torch.float8_e4m3fn)[:, :K]
+    y = kn.gemm_fp8_dq(a8, w8, one, one, None, out_dtype=torch.float32)
+    assert torch.equal(y.double(), a8.double() @ w8.double().t())
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (65, 33, 528), (129, 4100, 1088), (200, 5000, 976), (193, 4801, 1088),         # 64 x 64, 128 x 64
+    (1025, 2050, 528), (1000, 2060, 704), (1300, 6000, 528), (1290, 3990, 704),     # 128 x 128, 128 x 192
+    (1210, 5142, 848), (1234, 5861, 832), (4000, 4090, 1040), (4010, 4080, 1088)])  # 128 x 256, 256 x 256 (int8)
+def test_last_stage_cut_at_k(dev, M, N, K):
+    from fms_mo_amd import kernels as kn
+
+    tile = {65: (64, 64), 193: (128, 64), 1000: (128, 128), 1290: (128, 192), 1234: (128, 256), 4010: (256, 256)}.get(M)
+    if tile and K % 64 == 0:
+        assert kn.gemm_plan(M, N, K)[1:3] == tile
+    check(dev, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (2733, 3200, 1024, (128, 192)), (3367, 2941, 768, (128, 192)), (2050, 2310, 896, (128, 192)), (3627, 5389, 256, (128, 256))])
+def test_short_reductions_in_tiles_of_128_rows(dev, M, N, K, tile):
+    from fms_mo_amd import kernels as kn
+
+    assert kn.gemm_plan(M, N, K)[1:3] == tile
+    check(dev, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (2, 8200, 272, None), (13, 8300, 640, (64, 64)), (16, 16384, 640, (64, 64)),                    # a few tokens, many columns
+    (5, 17001, 528, None), (3, 16500, 704, (32, 128)), (16, 20000, 640, (32, 128)), (32, 16450, 1152, (32, 128)), (17, 16387, 1024, (32, 128))])
+def test_a_few_rows_over_many_columns(dev, M, N, K, tile):
+    from fms_mo_amd import kernels as kn
+
+    if tile:
+        assert kn.gemm_plan(M, N, K)[1:3] == tile
+    check(dev, M, N, K)
