@@ -4,45 +4,77 @@
 
 namespace {
 
-// A few dozen rows per expert: the weights bound the launch, and small tiles make the blocks that stream them.
-// Two blocks of either fit a compute unit.
-struct Tile64 { static constexpr int BM = 64, BN = 64, BK = 128, NST = 4, WGM = 2, WGN = 2; };
-struct Tile32 { static constexpr int BM = 32, BN = 128, BK = 128, NST = 4, WGM = 1, WGN = 4; };
+// A hundred rows per expert: the columns of a 128 x 128 tile, half its rows
+struct TileHalfK { static constexpr int BM = 64, BN = 128, BK = 128, NST = 3, WGM = 2, WGN = 4; };
 
-// The tile by an estimate of the time: rounds of tiles (the host knows rows and experts, not their split:
-// every expert's last tile is taken to be half full) times what a tile takes, a + b per 128 bytes of K as
-// measured.  256 x 256 (persistent blocks) where the others are not clearly ahead.
-// us, 256 x 256 | 128 x 128, 128-byte stages | 128 x 128, 64-byte stages | 64 x 64 | 32 x 128  (experts, rows, N, K):
-//   4, 153, 3840, 1024  19.0 | 9.9 | 9.7 | 6.9 | 7.2         4, 172, 1792, 6912   64.7 | 24.1 | 29.0 | 16.3 | 16.4
-//   16, 164, 8192, 1024 39.5 | 35.6 | 27.3 | 30.9 | 24.5     8, 1445, 2560, 1152  26.1 | 20.1 | 14.2 | 19.6 | 17.3
-//   8, 1445, 1152, 1280 34.3 | 11.0 | 10.9 | 8.7 | 9.7       4, 1387, 3968, 4096  58.5 | 36.9 | 40.7 | 44.5 | 52.3
-//   16, 1336, 1664, 5632 67.6 | 29.3 | 30.3 | 39.1 | 43.2    8, 2652, 4352, 2176  69.1 | 48.2 | 49.4 | 59.7 | 63.6
-//   16, 1992, 1280, 11136 106.7 | 54.1 | 61.5 | 58.3 | 72.4  4, 1387, 8192, 3968  61.2 | 64.1 | 67.9 | 85.5 | 102.9
-//   8, 4772, 2560, 12672 175 | 234 | 254 | 325 | 377         8, 8192, 4096, 14336 537 | 636 | 724 | 1012 | 1331
+// The tile: rounds of tiles times what a tile takes as measured, 256 x 256 (persistent blocks) where the others are not clearly ahead (below 1024
+// and K % 128 != 0 no more than that).  The host knows rows and experts, not their split, and takes every expert's last tile to be half full.
 // A launch takes a round at least, however few its tiles (taken as half a one, up to a dozen tiles went to 256 x 256; us,
 // -> as now: 4, 9, 130, 256 8.8 -> 3.9; 7, 949, 59, 448 24.7 -> 9.0; of 60 such launches all faster, 13.8 -> 6.2 in the mean).
-enum GroupedTile { G_BIG, G_MIDK, G_MID, G_64, G_32 };
+// From K = 1024 on a finer estimate, for rows that fall on the experts alike, may choose another tile where a tenth is to be gained.  With n the tiles
+// per compute unit and s the stages of 128 bytes: one block to a unit, max(1, w ceil(n) + (1 - w) n) rounds of a + b s, of which a chip filled to n < 1
+// saves c (1 - n); two to a unit, the second one slows the first's stages by 1 + q; the mean over n 4 % and 1 % less and 6 % more, for the step at whole rounds.
+// Parameters fitted to two thirds of 960 launches with every tile timed (4, 8, 16 experts, 128 .. 8192 rows, K and N of hidden sizes 1024 .. 4096 and
+// intermediate ones to 14336): 0.93 of the time of the rounds alone, the best tile of each 0.91 (two runs of one tile differ by 0.03).
+// us, before -> now (experts, rows, N, K): 16, 7145, 1408, 1024 36.8 -> 22.6; 8, 547, 2688, 5120 37.1 -> 23.3; 16, 2005, 3328,
+// 5632 112 -> 72.8; 4, 1310, 3328, 7040 61.0 -> 41.1; 8, 675, 5376, 2432 35.6 -> 22.5.  900 random launches 0.92 of the time, 25 of them slower by 3 % or more (16, 2674, 2048, 9856 100 -> 130).
+enum GroupedTile { G_BIG, G_MID, G_WIDEK, G_MIDK, G_HALF, G_64, G_32, G_TILES };
+struct GroupedCost { int bm, bn, units, threads; double a, b, c, w, q; };
+constexpr GroupedCost GROUPED_COSTS[G_TILES] = {
+    {256, 256, 1, 256, 15.66, 1.154, 0, .941, 0},    {128, 128, 2, 256, 2.315, .840, 0, .721, .409}, {128, 256, 1, 512, 5.578, .775, .254, .871, 0},
+    {128, 128, 1, 512, 4.728, .460, .407, .982, 0}, {64, 128, 2, 512, 3.774, .422, 0, .554, .440},  {64, 64, 2, 256, .501, .243, 0, .610, 1.831},
+    {32, 128, 2, 256, 1.680, .291, 0, .996, 1.344}};
 GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t K) {
   const double slabs = (double)K / 128;
   auto tiles = [&](int bm, int bn) {
     const double per = std::max(1.0, (double)rows / ((double)experts * bm) + 0.5);
     return (rows < experts ? (double)rows : experts * per) * div_up(N, bn);
   };
-  const double t256 = tiles(256, 256) / 256, t128 = tiles(128, 128);
-  const double big = 0.5 * (std::max(1.0, std::ceil(t256 - 0.05)) + std::ceil(t256 + 0.05)) * (1.6 * slabs + 9);
-  double best = 0.95 * big;
-  GroupedTile pick = G_BIG;
-  auto offer = [&](GroupedTile t, int bm, int bn, double cost) {
-    // one block per possible tile, 256 threads each: a launch holds less than 2^32 threads (the persistent blocks do not grow)
-    if (((rows + bm - 1) / bm + experts) * div_up(N, bn) >= (1 << 24)) return;
-    if (cost < best) best = cost, pick = t;
+  // one block per possible tile: a launch holds less than 2^32 threads (the persistent blocks do not grow)
+  auto fits = [&](GroupedTile t) {
+    const GroupedCost& p = GROUPED_COSTS[t];
+    return t == G_BIG || ((rows + p.bm - 1) / p.bm + experts) * div_up(N, p.bn) < (1ll << 32) / p.threads;
   };
-  offer(G_MID, 128, 128, std::max(1.0, t128 / 512) * (1.2 * slabs + 6));
+  const double t256 = tiles(256, 256) / 256, t128 = tiles(128, 128);
+  GroupedTile pick = G_BIG;
+  double best = 0.95 * 0.5 * (std::max(1.0, std::ceil(t256 - 0.05)) + std::ceil(t256 + 0.05)) * (1.6 * slabs + 9);
+  auto offer = [&](GroupedTile t, double cost) {
+    if (cost < best && fits(t)) best = cost, pick = t;
+  };
+  offer(G_MID, std::max(1.0, t128 / 512) * (1.2 * slabs + 6));
   if (K % 128) return pick;  // (the others take whole 128-byte stages)
-  offer(G_MIDK, 128, 128, std::ceil(t128 / 256) * ((t128 <= 512 ? 0.5 : 0.6) * slabs + 5));
-  offer(G_64, 64, 64, std::max(1.0, tiles(64, 64) / 512) * (0.4 * slabs + 5));
-  offer(G_32, 32, 128, std::max(1.0, tiles(32, 128) / 512) * (0.45 * slabs + 5));
-  return pick;
+  offer(G_MIDK, std::ceil(t128 / 256) * ((t128 <= 512 ? 0.5 : 0.6) * slabs + 5));
+  offer(G_64, std::max(1.0, tiles(64, 64) / 512) * (0.4 * slabs + 5));
+  offer(G_32, std::max(1.0, tiles(32, 128) / 512) * (0.45 * slabs + 5));
+  if (K < 1024) return pick;
+  const double mean = (double)rows / experts;  // rows of an expert, of a standard deviation of sqrt(mean)
+  auto below = [](double x) { return 0.5 * std::erfc(-x * M_SQRT1_2); };
+  auto estimate = [&](GroupedTile t) {
+    const GroupedCost& p = GROUPED_COSTS[t];
+    const double m = mean / p.bm, dev = std::sqrt(mean) / p.bm;
+    double per = mean > 8 ? 1 : 1 - std::exp(-mean);  // row tiles of an expert: of the k-th there is one where its rows pass k bm
+    if (dev > 0.5) per = m + 0.5;
+    else for (int k = 1; k < m + 4 * dev; ++k) per += below((m - k) / dev);
+    const double n0 = experts * per * div_up(N, p.bn) / 256, a = p.a, b = p.b * slabs;
+    double sum = 0;
+    for (const double u : {0.96, 0.99, 1.06}) {
+      const double n = u * n0, y = p.w * std::ceil(n) + (1 - p.w) * n;
+      if (p.units == 1) sum += std::max(1.0, y) * (1 - p.c * (1 - std::min(1.0, n))) * (a + b);
+      else if (n <= 1) sum += a + b;
+      else if (n <= 2) sum += a * (1 + .4 * (y - 1)) + b * (1 + p.q * (y - 1));
+      else sum += (1.4 * a + b * (1 + p.q)) * y / 2;
+    }
+    return sum / 3 + 2;
+  };
+  GroupedTile other = pick;
+  const double present = estimate(pick);
+  double least = present;
+  for (int i = G_BIG; i < G_TILES; ++i) {
+    const GroupedTile t = (GroupedTile)i;
+    const double cost = estimate(t);
+    if (cost < least && fits(t)) least = cost, other = t;
+  }
+  return 1.1 * least < present ? other : pick;
 }
 
 bool big_is_persistent(int64_t K) { return K % 128 == 0 && use_register_staged(MMA_I8); }
@@ -56,10 +88,12 @@ int launch_grouped(const GemmArgs& g0, const float* a_scale, const float* w_scal
   auto rows_of = [&](int bm) { return div_up(g.M, bm) + g.num_experts; };  // upper bound on the row tiles
   auto run = [&](const auto& epi) {
     switch (t) {
-      case G_MIDK: g.grid_m = rows_of(TileMidK::BM); launch_tile<TileMidK, MMA_I8, true>(g, epi, st); break;
+      case G_WIDEK: g.grid_m = rows_of(TileWideK::BM); launch_tile<TileWideK, MMA_I8, true>(g, epi, st); break;
+      case G_MIDK: g.grid_m = rows_of(TileMidK8::BM); launch_tile<TileMidK8, MMA_I8, true>(g, epi, st); break;
+      case G_HALF: g.grid_m = rows_of(TileHalfK::BM); launch_tile<TileHalfK, MMA_I8, true>(g, epi, st); break;
       case G_MID: g.grid_m = rows_of(TileMid::BM); launch_tile<TileMid, MMA_I8, true>(g, epi, st); break;
-      case G_64: g.grid_m = rows_of(Tile64::BM); launch_tile<Tile64, MMA_I8, true>(g, epi, st); break;
-      case G_32: g.grid_m = rows_of(Tile32::BM); launch_tile<Tile32, MMA_I8, true>(g, epi, st); break;
+      case G_64: g.grid_m = rows_of(TileSmallK::BM); launch_tile<TileSmallK, MMA_I8, true>(g, epi, st); break;
+      case G_32: g.grid_m = rows_of(TileLowK::BM); launch_tile<TileLowK, MMA_I8, true>(g, epi, st); break;
       default:
         g.grid_m = rows_of(256);
         if (big_is_persistent(g.K)) launch_rs<MMA_I8, true>(g, epi, st);
@@ -118,8 +152,8 @@ extern "C" int fmsmo_grouped_gemm_plan(int num_experts, int64_t total_rows, int6
   if (K % 64) return FMSMO_ERR_ALIGN;
   const GroupedTile t = pick_grouped_tile(num_experts, total_rows, N, K);
   *kernel = t == G_BIG && big_is_persistent(K) ? FMSMO_PLAN_TILE_REGISTER_STAGED : FMSMO_PLAN_TILE_LDS_DMA;
-  *tile_m = t == G_BIG ? 256 : t == G_64 ? Tile64::BM : t == G_32 ? Tile32::BM : TileMid::BM;
-  *tile_n = t == G_BIG ? 256 : t == G_64 ? Tile64::BN : t == G_32 ? Tile32::BN : TileMid::BN;
+  *tile_m = GROUPED_COSTS[t].bm;
+  *tile_n = GROUPED_COSTS[t].bn;
   *stage = t == G_MID || (t == G_BIG && *kernel == FMSMO_PLAN_TILE_LDS_DMA) ? 64 : 128;
   return FMSMO_OK;
 }

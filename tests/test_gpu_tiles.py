@@ -55,3 +55,27 @@ def test_a_few_rows_over_many_columns(dev, M, N, K, tile):
     if tile:
         assert kn.gemm_plan(M, N, K)[1:3] == tile
     check(dev, M, N, K)
+
+
+@pytest.mark.parametrize("counts,N,K,tile", [
+    ([0, 3, 90, 1, 65, 41, 0, 6], 4270, 2048, (64, 128)),
+    ([1, 63, 64, 65, 0, 5, 128, 129, 40, 0, 2, 70, 90, 30, 7, 33], 2102, 1664, (64, 128)),
+    ([129, 1, 697], 4145, 1664, (128, 256)), ([128, 257, 255, 256, 0, 300], 3500, 1280, (128, 256)),
+    ([569, 0, 129], 1999, 2048, (128, 128))])
+def test_grouped_tiles_of_eight_waves(dev, counts, N, K, tile):
+    """int8: exact; experts without rows, with one, and on either side of a tile."""
+    from fms_mo_amd import kernels as kn
+
+    E, T = len(counts), sum(counts)
+    assert kn.grouped_gemm_plan(E, T, N, K)[1:3] == tile
+    g = torch.Generator(device=dev).manual_seed(N)
+    a = torch.randint(-128, 128, (T, K), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-128, 128, (E, N, K), generator=g, dtype=torch.int8, device=dev)
+    off = torch.tensor([0] + counts, device=dev).cumsum(0).to(torch.int32)
+    y = kn.grouped_gemm_i8_dq(a, w, off, torch.ones(T, device=dev), torch.ones(E, N, device=dev), None, out_dtype=torch.float32,
+                              exact_ref=False)
+    lo = 0
+    for e, c in enumerate(counts):  # (integer sums, rounded once to fp32)
+        want = (a[lo:lo + c].double() @ w[e].double().t()).float()
+        assert torch.equal(y[lo:lo + c], want), e
+        lo += c
