@@ -245,6 +245,12 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
     *splits = plan.splits;
     return FMSMO_OK;
   }
+  if (const FewRows few = a_few_rows(M, N, K)) {
+    *kernel = FMSMO_PLAN_TILE_LDS_DMA;
+    *tile_m = few == FEW_SMALL ? TileSmallK::BM : TileTallK::BM;
+    *tile_n = TileTallK::BN;
+    return FMSMO_OK;
+  }
   if (K % 64) {
     *kernel = FMSMO_PLAN_GENERIC;
     return FMSMO_OK;

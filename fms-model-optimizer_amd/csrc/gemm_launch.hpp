@@ -286,6 +286,16 @@ void launch_k128(const GemmArgs& g0, int batch, int M, const Epi& epi, hipStream
   hipLaunchKernelGGL((gemm_k128_kernel<OP, Epi>), dim3((unsigned)blocks), dim3(256), 0, st, g, epi);
 }
 
+// Up to 256 rows in one pass beside use_small_tiles and use_tall_tiles: 64 x 64 tiles up to a round of them, 128 x 64 ones up to a round (us, slices or 128 x
+// 128 tiles before -> these, 64 x 64: int8 64 x 8461 x 2816 15.2 -> 9.5, 100 x 5021 x 3200 14.1 -> 10.2, 128 x 1808 x 2176 10.5 -> 8.1, 24 x 8696 x 6016 24.4 ->
+// 19.5, 24 x 10874 x 7936 30.9 -> 25.0, 64 x 6923 x 3200 13.3 -> 10.1; 128 x 64: e4m3 100 x 8924 x 2816 16.9 -> 10.3, 100 x 11835 x 3584 21.7 -> 15.5).
+enum FewRows { FEW_NONE, FEW_SMALL, FEW_TALL };
+inline FewRows a_few_rows(int64_t M, int64_t N, int64_t K) {
+  if (M > 256 || K % 128) return FEW_NONE;
+  if ((int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN) <= 256) return K < 8192 ? FEW_SMALL : FEW_NONE;
+  return (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN) <= 256 ? FEW_TALL : FEW_NONE;
+}
+
 // K % 128 != 0: the KT instances (a last stage that is cut at K).  The tile by an estimate of the time: rounds of tiles times
 // what a tile takes, a + b per 128 bytes of K, fitted to 520 launches of 65 .. 4096 rows, 256 .. 28672 columns and K = 512 .. 16384 with every
 // tile timed; a partly filled last round and a half empty chip count between their fraction and a whole one.  Over those launches the tiles chosen
@@ -347,6 +357,9 @@ void launch_any(const GemmArgs& g, const Epi& epi, hipStream_t st) {
   } else if (use_tall_tiles(g.M, g.N, g.K)) {
     if (OP != MMA_I8 || g.K < I8_EIGHT_WAVES_BELOW) launch_tile<TileTallK8, OP, false>(g, epi, st);
     else if constexpr (OP == MMA_I8) launch_tile<TileTallK, OP, false>(g, epi, st);
+  } else if (const FewRows few = a_few_rows(g.M, g.N, g.K)) {
+    if (few == FEW_SMALL) launch_tile<TileSmallK, OP, false>(g, epi, st);
+    else launch_tile<TileTallK8, OP, false>(g, epi, st);
   } else {
     switch (pick_tile(g.M, g.N, g.K, use_register_staged(OP), OP != MMA_I8)) {
       case 0:
@@ -490,6 +503,12 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   const int64_t tiles_t = (int64_t)div_up(M, TileTallK::BM) * div_up(N, TileTallK::BN);
   const int64_t room = limit > 0 ? limit / (M * N * 4) : 256;
   const int64_t tiles_s = (int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN);
+  // Up to 256 rows one pass of the tiles of a_few_rows takes less than slices and their sums do: of 33 64 x 64 tiles or more below K = 4096, of 129 or more
+  // below 8192 (where slices of 128 x 64 tiles would be but two), of more than a round always.  (int8 at K = 2048, up to 128 tiles, and 4096, where tests
+  // count on slices, keeps them, and not for their speed.)
+  if (M <= 256 && K % 128 == 0 && (tiles_s > 256 || (tiles_s > (fp8 || K > 2048 ? 32 : 128) && K >= 2048 && K < 4096) ||
+                                   (M <= 128 && tiles_s > 128 && tiles_t > 64 && K < 8192 && K >= (fp8 ? 4096 : 4224))))
+    return p;
   if (K % 128 == 0 && tiles_s <= 32 && K > 2048) {
     // Few tiles: slices on 64 x 64 ones, four (eight of a long reduction: from then on the partial sums cost more
     // than a shorter pass saves).  us, slices of 128 x 64 tiles -> these, M = 100, N = 1024: K = 3072 8.7 -> 6.9, 4096 9.2 ->

@@ -79,3 +79,14 @@ def test_grouped_tiles_of_eight_waves(dev, counts, N, K, tile):
         want = (a[lo:lo + c].double() @ w[e].double().t()).float()
         assert torch.equal(y[lo:lo + c], want), e
         lo += c
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (100, 1100, 2176, (64, 64)), (64, 8461, 2816, (64, 64)), (128, 8190, 4224, (64, 64)), (200, 700, 3968, (64, 64)),
+    (65, 8300, 2816, (128, 64)), (100, 8924, 8320, (128, 64)), (130, 5470, 4224, (128, 64)), (100, 16000, 9344, (128, 64))])
+def test_a_few_hundred_rows_in_one_pass(dev, M, N, K, tile):
+    from fms_mo_amd import kernels as kn
+
+    for fp8 in (False, True):
+        assert kn.gemm_plan(M, N, K, with_workspace=True, fp8=fp8)[1:] == (*tile, 1)
+    check(dev, M, N, K)
