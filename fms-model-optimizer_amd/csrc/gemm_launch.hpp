@@ -314,22 +314,29 @@ inline CutTile cut_k_tile(int64_t M, int64_t N, int64_t K, int op) {
   const int bm[6] = {64, 128, 128, 128, 128, 256}, bn[6] = {64, 64, 128, 192, 256, 256};
   if (use_low_tiles(M, N, K)) return CUT_LOW;
   const double stages = (double)((K + 127) / 128);
-  CutTile best = CUT_SMALL;
-  double least = 0;
+  CutTile best = CUT_BIG;
+  double least = HUGE_VAL;
   for (int t = 0; t < (kind == 2 ? 5 : 6); ++t) {
     const double a = CUT_COSTS[kind][t].a, b = CUT_COSTS[kind][t].b * stages;
     const double n = (double)div_up(M, bm[t]) * div_up(N, bn[t]) / 256, whole = std::ceil(n);
+    // (two 64 x 64 tiles to a unit on a long reduction: int8 314 x 5681 x 15312 103, 128 x 128 92)
+    if (t == CUT_SMALL && n > 1 && K >= 8192) continue;
     double cost;
     if (t == CUT_SMALL) cost = n <= 1 ? a + b : (1.4 * a + 1.8 * b) * whole / 2;  // (two of these share a compute unit)
     else cost = std::max(1.0, 0.72 * whole + 0.28 * n) * (a + b) * (1 - 0.25 * (1 - std::min(1.0, n)));
     if (t == CUT_BIG && kind == 1) cost *= n > 2.25 ? 0.92 : n <= 1 ? 1.1 : 1;
-    if (t == 0 || cost < least) least = cost, best = (CutTile)t;
+    if (cost < least) least = cost, best = (CutTile)t;
   }
   return best;
 }
 template <int OP, class Epi>
 void launch_cut_k(const GemmArgs& g, const Epi& epi, hipStream_t st) {
-  switch (cut_k_tile(g.M, g.N, g.K, OP)) {
+  const CutTile t = cut_k_tile(g.M, g.N, g.K, OP);
+  if constexpr (OP == MMA_I8) {  // (long reductions on four waves, as with whole stages)
+    if (t == CUT_TALL && g.K >= I8_EIGHT_WAVES_BELOW) return launch_tile<TileTallK, OP, false, true>(g, epi, st);
+    if (t == CUT_MID && g.K >= I8_EIGHT_WAVES_BELOW) return launch_tile<TileMidK, OP, false, true>(g, epi, st);
+  }
+  switch (t) {
     case CUT_SMALL: launch_tile<TileSmallK, OP, false, true>(g, epi, st); break;
     case CUT_TALL: launch_tile<TileTallK8, OP, false, true>(g, epi, st); break;
     case CUT_MID: launch_tile<TileMidK8, OP, false, true>(g, epi, st); break;
