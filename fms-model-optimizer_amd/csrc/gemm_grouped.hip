@@ -11,7 +11,7 @@ struct TileHalfK { static constexpr int BM = 64, BN = 128, BK = 128, NST = 3, WG
 // and K % 128 != 0 no more than that).  The host knows rows and experts, not their split, and takes every expert's last tile to be half full.
 // A launch takes a round at least, however few its tiles (taken as half a one, up to a dozen tiles went to 256 x 256; us,
 // -> as now: 4, 9, 130, 256 8.8 -> 3.9; 7, 949, 59, 448 24.7 -> 9.0; of 60 such launches all faster, 13.8 -> 6.2 in the mean).
-// From K = 1024 on a finer estimate, for rows that fall on the experts alike, may choose another tile where a tenth is to be gained.  With n the tiles
+// From K = 1024 on a finer estimate, for rows that fall on the experts alike, may choose another tile where an eighth is to be gained (a tenth: 4, 3055, 3584, 1664 unevenly split 9 % slower).  With n the tiles
 // per compute unit and s the stages of 128 bytes: one block to a unit, max(1, w ceil(n) + (1 - w) n) rounds of a + b s, of which a chip filled to n < 1
 // saves c (1 - n); two to a unit, the second one slows the first's stages by 1 + q; the mean over n 4 % and 1 % less and 6 % more, for the step at whole rounds.
 // Parameters fitted to two thirds of 960 launches with every tile timed (4, 8, 16 experts, 128 .. 8192 rows, K and N of hidden sizes 1024 .. 4096 and
@@ -74,7 +74,7 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
     const double cost = estimate(t);
     if (cost < least && fits(t)) least = cost, other = t;
   }
-  return 1.1 * least < present ? other : pick;
+  return 1.15 * least < present ? other : pick;
 }
 
 bool big_is_persistent(int64_t K) { return K % 128 == 0 && use_register_staged(MMA_I8); }
