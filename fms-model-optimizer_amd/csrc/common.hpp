@@ -61,6 +61,12 @@ __device__ __forceinline__ float load_as_f32(const void* p, size_t i) {
   else if constexpr (T == FMSMO_BF16) return bf16_to_f32(((const u16*)p)[i]);
   else return ((const float*)p)[i];
 }
+// Element i of an array of dtype dt, known at run time.
+__device__ __forceinline__ float scalar_f32(const void* p, int dt, int64_t i = 0) {
+  return dt == FMSMO_F16    ? f16_to_f32(((const u16*)p)[i])
+         : dt == FMSMO_BF16 ? bf16_to_f32(((const u16*)p)[i])
+                            : ((const float*)p)[i];
+}
 template <int T>
 __device__ __forceinline__ void store_from_f32(void* p, size_t i, float v) {
   if constexpr (T == FMSMO_F16) ((u16*)p)[i] = f32_to_f16(v);

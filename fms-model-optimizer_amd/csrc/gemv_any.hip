@@ -400,7 +400,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_any_kernel(GemvArgs g, int halve
     else units_fp8<XT, NW, UPW>(g, U, qcur, xq, xs, xsc, xred);
     __syncthreads();
     if constexpr (!STATIC) gemv_put_scales(g, xsc);
-    as = STATIC ? g.a_value : xsc[em];
+    as = !STATIC ? xsc[em] : g.a_src ? scalar_f32(g.a_src, g.a_src_dtype) : g.a_value;
   } else {
     as = g.a_scale ? g.a_scale[g.a_stride ? em : 0] : 1.f;
   }
@@ -708,10 +708,10 @@ extern "C" int fmsmo_small_linear_static_ok(int64_t M, int64_t N, int64_t K, flo
   return K <= 3072 && M * ((K + UNIT - 1) / UNIT) <= 32 && (N <= 8192 || (M <= 4 && K <= 1024)) &&
          static_fmo32_ok(clip_lo, clip_hi, step, zp);
 }
-extern "C" int fmsmo_small_linear_i8_static(const void* x, int x_dtype, int64_t ldx, float step, float zp, int sym, float clip_lo,
-                                            float clip_hi, float a_scale, const int8_t* w, int64_t ldw, const float* w_scale,
-                                            int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue, void* y,
-                                            int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream) {
+static int small_linear_static(const void* x, int x_dtype, int64_t ldx, float step, float zp, int sym, float clip_lo,
+                               float clip_hi, float a_value, const void* a_src, int a_src_dtype, const int8_t* w, int64_t ldw,
+                               const float* w_scale, int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue, void* y,
+                               int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream) {
   if (!x || !w || !w_scale || !y) return FMSMO_ERR_NULL;
   if (M <= 0 || N <= 0 || K <= 0 || (M > 1 && ldx < K) || ldw < K || ldy < N) return FMSMO_ERR_SHAPE;
   if (w_scale_n != 1 && w_scale_n != N) return FMSMO_ERR_SHAPE;
@@ -729,8 +729,25 @@ extern "C" int fmsmo_small_linear_i8_static(const void* x, int x_dtype, int64_t 
   g.y = y; g.y_dtype = y_dtype; g.ldy = ldy;
   g.x16 = (const u16*)x; g.ldx = ldx;
   g.q_lo = clip_lo; g.q_hi = clip_hi; g.q_step = step; g.q_rcp = 1.0f / step; g.q_zp = zp; g.q_shift = 128 - (sym ? 1 : 0);
-  g.a_value = a_scale;
+  g.a_value = a_value; g.a_src = a_src; g.a_src_dtype = a_src_dtype;
   if (!any_offsets_ok(g)) return FMSMO_ERR_UNSUPPORTED;
   return x_dtype == FMSMO_F16 ? any_launch<FMSMO_OP_I8, 1, FMSMO_F16, QUANT_STATIC>(g, (hipStream_t)stream)
                               : any_launch<FMSMO_OP_I8, 1, FMSMO_BF16, QUANT_STATIC>(g, (hipStream_t)stream);
+}
+extern "C" int fmsmo_small_linear_i8_static(const void* x, int x_dtype, int64_t ldx, float step, float zp, int sym, float clip_lo,
+                                            float clip_hi, float a_scale, const int8_t* w, int64_t ldw, const float* w_scale,
+                                            int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue, void* y,
+                                            int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream) {
+  return small_linear_static(x, x_dtype, ldx, step, zp, sym, clip_lo, clip_hi, a_scale, nullptr, 0, w, ldw, w_scale, w_scale_n,
+                             bias, bias_dtype, epilogue, y, y_dtype, ldy, M, N, K, stream);
+}
+extern "C" int fmsmo_small_linear_i8_static_scale(const void* x, int x_dtype, int64_t ldx, float step, float zp, int sym,
+                                                  float clip_lo, float clip_hi, const void* a_scale, int a_scale_dtype,
+                                                  const int8_t* w, int64_t ldw, const float* w_scale, int64_t w_scale_n,
+                                                  const void* bias, int bias_dtype, int epilogue, void* y, int y_dtype,
+                                                  int64_t ldy, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream) {
+  if (!a_scale) return FMSMO_ERR_NULL;
+  if (a_scale_dtype < 0 || a_scale_dtype > 2) return FMSMO_ERR_UNSUPPORTED;
+  return small_linear_static(x, x_dtype, ldx, step, zp, sym, clip_lo, clip_hi, 0.0f, a_scale, a_scale_dtype, w, ldw, w_scale,
+                             w_scale_n, bias, bias_dtype, epilogue, y, y_dtype, ldy, M, N, K, stream);
 }

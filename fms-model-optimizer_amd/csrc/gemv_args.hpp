@@ -27,9 +27,11 @@ struct GemvArgs {
   int saturate;
   float* a_scale_out;   // [M] per-token scales (written by block 0), or NULL
   // static per-tensor quantizer (see fmsmo_quant_act_i8_static_t, FMSMO_SQ_FMO in fp32): clip values, step and its
-  // reciprocal, zero point, 128 - sym, and the scale that the sums are dequantized with
+  // reciprocal, zero point, 128 - sym, and the scale that the sums are dequantized with: read from a_src, or a_value
   float q_lo, q_hi, q_step, q_rcp, q_zp, a_value;
   int q_shift;
+  const void* a_src;    // scalar of a_src_dtype, or NULL
+  int a_src_dtype;
   float* clips;         // [2][M] the clip values they stand for, scale * 127 and its negative, or NULL
 };
 
@@ -48,9 +50,7 @@ __device__ __forceinline__ void gemv_put_scales(const GemvArgs& g, const float* 
 // bias of output column n (no bias: -0, whose addition changes nothing, not even the sign of a zero product)
 __device__ __forceinline__ float gemv_bias(const GemvArgs& g, int n) {
   if (!g.bias) return -0.f;
-  return g.bias_dtype == FMSMO_F16 ? f16_to_f32(((const u16*)g.bias)[n])
-         : g.bias_dtype == FMSMO_BF16 ? bf16_to_f32(((const u16*)g.bias)[n])
-                                      : ((const float*)g.bias)[n];
+  return scalar_f32(g.bias, g.bias_dtype, n);
 }
 
 // y[m, n] from a sum over K, its token and weight scales and its bias

@@ -26,9 +26,9 @@ namespace {
 #define ENTRIES(X)                                                                                       \
   X(fmsmo_quant_act_i8_pertoken) X(fmsmo_quant_act_i8_static) X(fmsmo_quant_act_i8_static_t)             \
   X(fmsmo_quant_act_fp8_pertoken) X(fmsmo_quant_act_fp8_dynamic) X(fmsmo_quant_act_fp8_tensor)           \
-  X(fmsmo_quant_act_i8_pertoken_clips) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
+  X(fmsmo_quant_act_i8_static_scale) X(fmsmo_quant_act_i8_pertoken_clips) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
-  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_small_linear_ok) X(fmsmo_small_linear_i8) X(fmsmo_small_linear_fp8) X(fmsmo_small_linear_static_ok) X(fmsmo_small_linear_i8_static) X(fmsmo_grouped_gemm_i8_dq)                   \
+  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_small_linear_ok) X(fmsmo_small_linear_i8) X(fmsmo_small_linear_fp8) X(fmsmo_small_linear_static_ok) X(fmsmo_small_linear_i8_static_scale) X(fmsmo_grouped_gemm_i8_dq)                   \
   X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq) X(fmsmo_matmul_chunk_workspace_bytes)    \
   X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_parts_first) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
   X(fmsmo_bmm_qa_i8) X(fmsmo_bmm_i8_zp)
@@ -544,9 +544,9 @@ PyObject* kept_for(PyObject* kept, const at::Tensor& t) {
 // The parameters of the static quantizer that the Python side keeps for activations of dtype xt beside the buffers they were read from
 // (QLinearINT8Deploy._static_params); false where one of those is another tensor or was written to since.
 struct StaticParams {
-  double scale = 0, step = 0, qzp = 0, lo = 0, hi = 0;
+  double step = 0, qzp = 0, lo = 0, hi = 0;
   at::ScalarType T = at::kFloat;
-  const at::Tensor* scale_t = nullptr;  // the scale as fp32 on the device
+  const at::Tensor* scale = nullptr;  // the buffer input_scale itself, one element
 };
 bool static_params(PyObject* self, PyObject* buffers, at::ScalarType xt, StaticParams* p) {
   PyObject *kept = item(self, k__sp_kept), *cvs = item(self, k_cvs);
@@ -562,17 +562,17 @@ bool static_params(PyObject* self, PyObject* buffers, at::ScalarType xt, StaticP
     if (!t || !same_stamp(PyTuple_GET_ITEM(stamps, i + 1), *t)) return false;
     if (i == 0 && t->numel() != 1) return false;
   }
-  const char* names[5] = {"scale", "step", "qzp", "lo", "hi"};
-  double* to[5] = {&p->scale, &p->step, &p->qzp, &p->lo, &p->hi};
-  for (int i = 0; i < 5; ++i) {
+  const char* names[4] = {"step", "qzp", "lo", "hi"};
+  double* to[4] = {&p->step, &p->qzp, &p->lo, &p->hi};
+  for (int i = 0; i < 4; ++i) {
     PyObject* v = PyDict_GetItemString(found, names[i]);
     if (!v || !PyFloat_Check(v)) return false;
     *to[i] = PyFloat_AS_DOUBLE(v);
   }
-  PyObject *T = PyDict_GetItemString(found, "T"), *st = PyDict_GetItemString(found, "scale_t");
-  if (!T || !dtype_arg(T, &p->T) || !st) return false;
-  p->scale_t = vec32(st, 1);
-  return p->scale_t != nullptr;
+  PyObject* T = PyDict_GetItemString(found, "T");
+  if (!T || !dtype_arg(T, &p->T)) return false;
+  p->scale = plain(of[0]);
+  return code_of(p->scale->scalar_type()) >= 0 && !p->scale->requires_grad();
 }
 
 // Is a method of the class, or of this instance, another function than the one that came with it?
@@ -644,24 +644,35 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     PyObject* sym = item(self, k_useSymAct);
     StaticParams p;
     if (smooth || native != Py_False || !sym || !plain_product() || other(k_qa_fmo_mo_qfunc, 6) || other(k__static_params, 7) ||
-        !static_params(self, buffers, xt, &p) || !here(x.t, p.scale_t))
+        !static_params(self, buffers, xt, &p) || !here(x.t, p.scale))
       return none();
-    const at::Tensor own_scale = *p.scale_t;
+    // The launches read the module's own buffer, as the general path does: a copy of it that the module kept could be
+    // freed under a graph that was captured with its address, and a number would not follow the buffer when one is replayed.
+    const at::Tensor own_scale = *p.scale;
+    const int sdt = code_of(own_scale.scalar_type());
     const int sy = PyObject_IsTrue(sym) == 1;
     at::Tensor y = out_like(*x.t, w.rows, ot);
     if (p.T == at::kFloat && w.rows * w.ld < (1ll << 31) &&
         p_fmsmo_small_linear_static_ok(x.rows, w.rows, x.cols, (float)p.step, (float)p.qzp, (float)p.lo, (float)p.hi)) {
-      if (!LAUNCH(fmsmo_small_linear_i8_static, x.p, code_of(xt), x.ld, (float)p.step, (float)p.qzp, sy, (float)p.lo, (float)p.hi,
-                  (float)p.scale, (const int8_t*)w.p, w.ld, (const float*)ws->data_ptr(), ws->numel(), b.p, b.dt,
+      if (!LAUNCH(fmsmo_small_linear_i8_static_scale, x.p, code_of(xt), x.ld, (float)p.step, (float)p.qzp, sy, (float)p.lo,
+                  (float)p.hi, (const void*)own_scale.data_ptr(), sdt, (const int8_t*)w.p, w.ld, (const float*)ws->data_ptr(), ws->numel(), b.p, b.dt,
                   FMSMO_EPI_REF_F16, y.data_ptr(), code_of(ot), w.rows, x.rows, w.rows, x.cols, stream_of(*x.t)))
         return nullptr;
       return wrap(y);
     }
-    at::Tensor q = empty({x.rows, x.cols}, at::kChar, *x.t);
-    if (!LAUNCH(fmsmo_quant_act_i8_static_t, x.p, code_of(xt), x.ld, FMSMO_SQ_FMO, code_of(p.T), (float)p.step, (float)p.qzp, sy,
-                (float)p.lo, (float)p.hi, (int8_t*)q.data_ptr(), x.cols, x.rows, x.cols, stream_of(*x.t)))
-      return nullptr;
-    if (!run_gemm_i8((const char*)q.data_ptr(), x.cols, w, (const float*)own_scale.data_ptr(), 1, *ws, b, FMSMO_EPI_REF_F16, y,
+    at::Tensor q = empty({x.rows, x.cols}, at::kChar, *x.t), s = own_scale;
+    if (sdt == FMSMO_F32) {
+      if (!LAUNCH(fmsmo_quant_act_i8_static_t, x.p, code_of(xt), x.ld, FMSMO_SQ_FMO, code_of(p.T), (float)p.step, (float)p.qzp,
+                  sy, (float)p.lo, (float)p.hi, (int8_t*)q.data_ptr(), x.cols, x.rows, x.cols, stream_of(*x.t)))
+        return nullptr;
+    } else {
+      s = empty({1}, at::kFloat, *x.t);
+      if (!LAUNCH(fmsmo_quant_act_i8_static_scale, x.p, code_of(xt), x.ld, FMSMO_SQ_FMO, code_of(p.T), (float)p.step,
+                  (float)p.qzp, sy, (float)p.lo, (float)p.hi, (int8_t*)q.data_ptr(), x.cols,
+                  (const void*)own_scale.data_ptr(), sdt, (float*)s.data_ptr(), x.rows, x.cols, stream_of(*x.t)))
+        return nullptr;
+    }
+    if (!run_gemm_i8((const char*)q.data_ptr(), x.cols, w, (const float*)s.data_ptr(), 1, *ws, b, FMSMO_EPI_REF_F16, y,
                      x.rows, x.cols))
       return nullptr;
     return wrap(y);

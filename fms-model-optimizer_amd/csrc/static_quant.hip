@@ -14,12 +14,21 @@ namespace fmsmo {
 struct StaticArgs {
   float scale, zp, sym, lo, hi;
   int mode;
+  const void* s_in;  // a scale of s_dtype that is to be written to s_out as fp32, or NULL
+  int s_dtype;
+  float* s_out;
 };
+// (A product behind the quantizer reads its scale as fp32.  A launch of its own for the one conversion takes 2 us, and
+// a copy kept on the host's side would not follow the buffer in a replayed graph.)
+__device__ __forceinline__ void put_scale(const StaticArgs& p) {
+  if (p.s_in && blockIdx.x == 0 && threadIdx.x == 0) *p.s_out = scalar_f32(p.s_in, p.s_dtype);
+}
 
 template <int XT, int T>
 __global__ __launch_bounds__(256) void quant_i8_static_t_kernel(const void* __restrict__ x, int64_t ldx,
                                                                 StaticArgs p, int8_t* __restrict__ q,
                                                                 int64_t ldq, int M, int K) {
+  put_scale(p);
   const int cpr = K / AQ_VEC;
   const int64_t total = (int64_t)M * cpr;
   for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < total; c += (int64_t)gridDim.x * 256) {
@@ -72,6 +81,7 @@ template <int T, int MODE>
 __global__ __launch_bounds__(256) void quant_i8_static16_kernel(const u16* __restrict__ x, StaticArgs p,
                                                                 float rcp_scale, int8_t* __restrict__ q,
                                                                 int64_t nchunks) {
+  put_scale(p);
   const float nz = opaque_neg_zero();
   auto rnd2 = [](float& a, float& b) {
     const uint32_t w = pack16<T>(a, b);
@@ -132,6 +142,7 @@ __global__ __launch_bounds__(256) void quant_i8_static16_kernel(const u16* __res
 template <int XT>
 __global__ __launch_bounds__(256) void quant_i8_static_fmo32_kernel(const u16* __restrict__ x, StaticArgs p, float rcp,
                                                                     int8_t* __restrict__ q, int64_t nchunks) {
+  put_scale(p);
   const float nz = opaque_neg_zero();
   const int shift = 128 - (int)p.sym;
   for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)gridDim.x * 256) {
@@ -390,10 +401,9 @@ int check_rows(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K) {
 }
 }  // namespace
 
-extern "C" int fmsmo_quant_act_i8_static_t(const void* x, int x_dtype, int64_t ldx, int mode,
-                                           int compute_dtype, float scale, float zp, int sym,
-                                           float clip_lo, float clip_hi, int8_t* q, int64_t ldq,
-                                           int64_t M, int64_t K, fmsmo_stream_t stream) {
+static int static_t_impl(const void* x, int x_dtype, int64_t ldx, int mode, int compute_dtype, float scale, float zp,
+                         int sym, float clip_lo, float clip_hi, int8_t* q, int64_t ldq, const void* scale_in,
+                         int scale_dtype, float* scale_out, int64_t M, int64_t K, fmsmo_stream_t stream) {
   int rc = check_rows(x, x_dtype, ldx, M, K);
   if (rc) return rc;
   if (!q) return FMSMO_ERR_NULL;
@@ -404,7 +414,7 @@ extern "C" int fmsmo_quant_act_i8_static_t(const void* x, int x_dtype, int64_t l
   // torch's promotion of x's dtype with the scale's: x's own dtype or fp32
   if (compute_dtype != FMSMO_F32 && compute_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
   if (M == 0) return FMSMO_OK;
-  StaticArgs p{scale, zp, (float)(sym ? 1 : 0), clip_lo, clip_hi, mode};
+  StaticArgs p{scale, zp, (float)(sym ? 1 : 0), clip_lo, clip_hi, mode, scale_in, scale_dtype, scale_out};
   dim3 grid(grid_for(M, K)), block(256);
   hipStream_t st = (hipStream_t)stream;
   // 16-bit compute dtype, contiguous rows, a divisor that is a finite non-zero value of that dtype
@@ -453,6 +463,23 @@ extern "C" int fmsmo_quant_act_i8_static_t(const void* x, int x_dtype, int64_t l
   }
 #undef LAUNCH
   return fmsmo_check_launch();
+}
+
+extern "C" int fmsmo_quant_act_i8_static_t(const void* x, int x_dtype, int64_t ldx, int mode,
+                                           int compute_dtype, float scale, float zp, int sym,
+                                           float clip_lo, float clip_hi, int8_t* q, int64_t ldq,
+                                           int64_t M, int64_t K, fmsmo_stream_t stream) {
+  return static_t_impl(x, x_dtype, ldx, mode, compute_dtype, scale, zp, sym, clip_lo, clip_hi, q, ldq, nullptr, 0, nullptr,
+                       M, K, stream);
+}
+extern "C" int fmsmo_quant_act_i8_static_scale(const void* x, int x_dtype, int64_t ldx, int mode, int compute_dtype,
+                                               float scale, float zp, int sym, float clip_lo, float clip_hi, int8_t* q,
+                                               int64_t ldq, const void* scale_in, int scale_dtype, float* scale_out,
+                                               int64_t M, int64_t K, fmsmo_stream_t stream) {
+  if (!scale_in || !scale_out) return FMSMO_ERR_NULL;
+  if (scale_dtype < 0 || scale_dtype > 2) return FMSMO_ERR_UNSUPPORTED;
+  return static_t_impl(x, x_dtype, ldx, mode, compute_dtype, scale, zp, sym, clip_lo, clip_hi, q, ldq, scale_in, scale_dtype,
+                       scale_out, M, K, stream);
 }
 
 extern "C" int fmsmo_quant_act_i8_dynamic(const void* x, int x_dtype, int64_t ldx,

@@ -17,11 +17,6 @@ namespace fmsmo {
 __device__ __forceinline__ float round_dyn(float v, int t) {
   return t == FMSMO_F16 ? round_to<FMSMO_F16>(v) : t == FMSMO_BF16 ? round_to<FMSMO_BF16>(v) : v;
 }
-__device__ __forceinline__ float load_dyn(const void* p, int t, size_t i) {
-  return t == FMSMO_F16 ? f16_to_f32(((const u16*)p)[i])
-         : t == FMSMO_BF16 ? bf16_to_f32(((const u16*)p)[i])
-                           : ((const float*)p)[i];
-}
 
 // 8 consecutive elements of a dtype known at run time, widened to fp32
 __device__ __forceinline__ void load8_dyn(const void* p, int t, size_t i, float (&v)[8]) {
@@ -47,7 +42,7 @@ __global__ __launch_bounds__(256) void quant_weight_i8_kernel(
     int8_t* __restrict__ q, int64_t ldq, int32_t* __restrict__ row_sum, int K) {
   __shared__ int red[4];
   const int row = blockIdx.x;
-  const float c = load_dyn(coef, coef_dtype, coef_stride ? row : 0);
+  const float c = scalar_f32(coef, coef_dtype, coef_stride ? row : 0);
   int sum = 0;
   constexpr int U = 4;  // 16-byte groups in flight per thread
   typedef typename std::conditional<WT == FMSMO_F32, float4, uint4>::type Raw;
@@ -129,7 +124,7 @@ __global__ __launch_bounds__(256) void quant_weight_div32_kernel(
   bool plain = true;
 #pragma unroll
   for (int r = 0; r < WQ_ROWS; ++r) {
-    c[r] = load_dyn(coef, coef_dtype, coef_stride ? row0 + min(r, nr - 1) : 0);
+    c[r] = scalar_f32(coef, coef_dtype, coef_stride ? row0 + min(r, nr - 1) : 0);
     plain = plain && c[r] >= 0x1p-90f && c[r] <= 0x1p90f;
     rc[r] = rcp_refined(c[r]);
     lim[r] = 127.25f * c[r];
@@ -310,7 +305,7 @@ __global__ __launch_bounds__(256) void deploy_vectors_kernel(
     w_scale[n] = ws;
     w_zp[n] = 0;
     corr[n] = c;
-    const float nb = bias ? load_dyn(bias, bias_dtype, n) - c : -c;
+    const float nb = bias ? scalar_f32(bias, bias_dtype, n) - c : -c;
     store_from_f32<WT>(new_bias, n, nb);
   }
   if (b == kb && threadIdx.x == 0) {
@@ -345,7 +340,7 @@ __global__ __launch_bounds__(256) void zero_shift_bias_kernel(
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
   if (lane == 0) {
-    const float b = bias ? load_dyn(bias, bias_dtype, row) : 0.0f;
+    const float b = bias ? scalar_f32(bias, bias_dtype, row) : 0.0f;
     const float ws = w_scale[w_scale_n > 1 ? row : 0];
     out[row] = b + (offset + a_meta[1]) * (float)sum * a_meta[0] * ws;
   }

@@ -36,6 +36,7 @@ SIGNATURES = {
     "fmsmo_quant_act_i8_pertoken_clips": [_P, _I, _L, _I, _I, _P, _L, _P, _P, _L, _L, _P],
     "fmsmo_quant_act_i8_static": [_P, _I, _L, _F, _I, _I, _P, _L, _L, _L, _P],
     "fmsmo_quant_act_i8_static_t": [_P, _I, _L, _I, _I, _F, _F, _I, _F, _F, _P, _L, _L, _L, _P],
+    "fmsmo_quant_act_i8_static_scale": [_P, _I, _L, _I, _I, _F, _F, _I, _F, _F, _P, _L, _P, _I, _P, _L, _L, _P],
     "fmsmo_quant_act_i8_dynamic": [_P, _I, _L, _P, _I, _I, _I, _P, _L, _P, _L, _L, _P],
     "fmsmo_fake_quant_fp8": [_P, _I, _L, _I, _P, _P, _L, _P, _L, _P, _P, _L, _L, _P],
     "fmsmo_quant_act_i8_mulscale": [_P, _I, _L, _P, _P, _I, _I, _I, _P, _L, _P, _L, _L, _P],
@@ -54,6 +55,8 @@ SIGNATURES = {
     "fmsmo_decode_linear_i8": [_P, _I, _L, _P, _I, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_small_linear_i8": [_P, _I, _L, _P, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _P, _P, _L, _L, _L, _P],
     "fmsmo_small_linear_i8_static": [_P, _I, _L, _F, _F, _I, _F, _F, _F, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L, _L, _L, _L, _P],
+    "fmsmo_small_linear_i8_static_scale": [_P, _I, _L, _F, _F, _I, _F, _F, _P, _I, _P, _L, _P, _L, _P, _I, _I, _P, _I, _L,
+                                           _L, _L, _L, _P],
     "fmsmo_small_linear_fp8": [_P, _I, _L, _P, _L, _P, _L, _P, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_decode_linear_fp8": [_P, _I, _L, _P, _L, _P, _L, _P, _I, _P, _I, _L, _P, _L, _L, _L, _P],
     "fmsmo_matmul_chunk_i8": [_P, _L, _P, _L, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I, _P],

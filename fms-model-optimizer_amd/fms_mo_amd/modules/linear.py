@@ -614,8 +614,7 @@ class QLinearINT8Deploy(nn.Linear):
                 p.update(T=quot.dtype, lo=float(cvn.to(clamped.dtype).reshape(-1)[0]),
                          hi=float(cv.to(clamped.dtype).reshape(-1)[0]),
                          step=float(self.quant_stepsize.reshape(-1)[0]),
-                         qzp=float(self.quant_zero_point.reshape(-1)[0]),
-                         scale_t=self.input_scale.detach().float().reshape(-1).contiguous())
+                         qzp=float(self.quant_zero_point.reshape(-1)[0]))
             self._sp_kept = kept = _Kept((stamp, p, [t.detach() for t in tensors]))
         return kept[1]
 

@@ -181,6 +181,13 @@ int fmsmo_quant_act_i8_static_t(const void* x, int x_dtype, int64_t ldx, int mod
                                 int compute_dtype, float scale, float zp, int sym, float clip_lo,
                                 float clip_hi, int8_t* q, int64_t ldq, int64_t M, int64_t K,
                                 fmsmo_stream_t stream);
+/*
+ * The same, and *scale_out = the scalar scale_in of scale_dtype as fp32, for a product behind it that dequantizes with a
+ * 16-bit buffer (nothing is written where M == 0).
+ */
+int fmsmo_quant_act_i8_static_scale(const void* x, int x_dtype, int64_t ldx, int mode, int compute_dtype, float scale, float zp,
+                                    int sym, float clip_lo, float clip_hi, int8_t* q, int64_t ldq, const void* scale_in,
+                                    int scale_dtype, float* scale_out, int64_t M, int64_t K, fmsmo_stream_t stream);
 
 /*
  * Dynamic symmetric int8 quantizers whose abs-max is taken over the whole tensor or per column
@@ -532,6 +539,12 @@ int fmsmo_small_linear_i8_static(const void* x, int x_dtype, int64_t ldx, float 
                                  float clip_hi, float a_scale, const int8_t* w, int64_t ldw, const float* w_scale,
                                  int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue, void* y, int y_dtype,
                                  int64_t ldy, int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream);
+/* The same with the scale read on the device: a_scale points to a scalar of a_scale_dtype. */
+int fmsmo_small_linear_i8_static_scale(const void* x, int x_dtype, int64_t ldx, float step, float zp, int sym, float clip_lo,
+                                       float clip_hi, const void* a_scale, int a_scale_dtype, const int8_t* w, int64_t ldw,
+                                       const float* w_scale, int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
+                                       void* y, int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K,
+                                       fmsmo_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------
  * 4. Chunked reduced-precision accumulation ("chunk-truncate") matmuls.
