@@ -832,14 +832,24 @@ class QLinearINT8Deploy(nn.Linear):
 
     def _w_scale_f32(self):
         """``w_scale`` as the contiguous fp32 vector the kernels read, converted once (the buffer
-        is fp16 in a deployed ``.half()`` module; converting it in every forward costs a launch)."""
+        is fp16 in a deployed ``.half()`` module; converting it in every forward costs a launch).  A copy that stays
+        of the same size is written to in place when the buffer changes: a captured graph may hold its address."""
         ws = self.w_scale
         if torch.compiler.is_compiling():
             return ws.float().reshape(-1)
         stamp = _stamp(ws)
         kept = getattr(self, "_ws_kept", None)
         if not kept or kept[0] != stamp:
-            self._ws_kept = kept = _Kept((stamp, ws.detach().float().reshape(-1).contiguous(), ws.detach()))
+            with torch.inference_mode(False), torch.no_grad():
+                f = ws.detach().float().reshape(-1).contiguous()
+                if f.is_cuda and torch.cuda.is_current_stream_capturing():
+                    return f    # (part of the graph: it holds nothing before a replay)
+                own = kept[1] if kept and kept[1].data_ptr() != kept[2].data_ptr() else None
+                if own is not None and f.data_ptr() != ws.data_ptr() and own.shape == f.shape and own.device == f.device:
+                    f = own.copy_(f)
+                if f.is_cuda:   # (whichever stream reads it next)
+                    torch.cuda.current_stream(f.device).synchronize()
+            self._ws_kept = kept = _Kept((stamp, f, ws.detach()))
         return kept[1]
 
     def _set_input_scale(self, s):

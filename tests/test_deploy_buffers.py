@@ -62,6 +62,24 @@ def test_a_buffer_in_the_memory_of_the_one_before(name):
         in_the_place_of(m, name, torch.full_like(m._buffers[name], 2))
 
 
+def test_the_copy_of_the_weight_scale_stays_where_it_is():
+    """A captured graph may hold its address: a change of the buffer is written to the copy, not to another one."""
+    m = deployed()
+    kept = m._w_scale_f32()
+    for change in (lambda: m.w_scale.mul_(0.5), lambda: in_the_place_of(m, "w_scale", m.w_scale.clone() * 2),
+                   lambda: setattr(m, "w_scale", m.w_scale.bfloat16())):
+        change()
+        with torch.inference_mode():
+            assert m._w_scale_f32() is kept
+        assert kept.tolist() == m.w_scale.float().tolist() and not kept.is_inference()
+    m.w_scale = m.w_scale.float()
+    assert m._w_scale_f32().data_ptr() == m.w_scale.data_ptr() != kept.data_ptr()
+    was = m.w_scale
+    m.w_scale = (was * 2).half()       # (another tensor's memory is never written to)
+    before = was.clone()
+    assert m._w_scale_f32().tolist() == m.w_scale.float().tolist() and torch.equal(was, before)
+
+
 def test_copies_and_pickles_ask_for_themselves():
     m = deployed()
     m._w_scale_f32(), m._smoothq_active()

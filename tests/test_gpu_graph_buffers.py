@@ -59,3 +59,33 @@ def test_replay_of_a_static_forward_reads_the_scale_of_the_module(dev, M, K, dty
         graph.replay()
         assert torch.equal(y, m(x)), i
         del held
+
+
+@pytest.mark.parametrize("M", [1, 40])
+def test_replay_of_a_dynamic_forward_follows_the_scale_of_the_weights(dev, M):
+    """w_scale of 16 bits: the fp32 copy that the products read."""
+    from fms_mo_amd.modules.linear import QLinear, QLinearINT8Deploy
+
+    q = QLinear(1024, 300, bias=True, num_bits_feature=8, qa_mode="pertokenmax", num_bits_weight=8, qw_mode="maxperCh",
+                qcfg={"smoothq": False}, device=dev).to(dev).half()
+    q.quantize_weight.float()
+    with torch.no_grad():
+        q.quantize_weight.clip_val.copy_(q.weight.abs().amax(dim=1))
+    m = QLinearINT8Deploy.from_fms_mo(q.eval(), use_dynamic_max_act_Qfunc=-1, recalc_clipvals=False).half()
+    x = torch.randn(M, 1024, generator=torch.Generator().manual_seed(M)).half().to(dev)
+    graph, y = captured(m, x)
+    for i in range(3):
+        m.w_scale.mul_(2)
+        want = m(x)
+        held = fill_freed_memory(dev)
+        graph.replay()
+        assert torch.equal(y, want) and torch.equal(m(x), want), i
+        del held
+    m.w_scale.mul_(0.25)
+    late = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(late):  # the buffer changed since the last eager call: converted inside the graph, kept by nobody
+        z = m(x)
+    want = m(x)
+    assert torch.equal(want, m(x)) and not torch.equal(want, y)
+    late.replay()
+    assert torch.equal(z, want)
