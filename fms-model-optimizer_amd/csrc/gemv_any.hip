@@ -14,9 +14,13 @@
 
 namespace fmsmo {
 
-// K % 64 != 0, e4m3: codes widened to fp16 (exact), products on the fp16 instruction, whose sums keep what fp32
-// additions keep (the e4m3 instruction, which takes 64 elements and more at a time, does not)
+// e4m3 on the fp16 instruction: codes widened to fp16 (exact), sums that keep what fp32 additions keep, which those of the
+// e4m3 instruction, 64 elements and more at a time, do not
 constexpr int GEMV_FP8_F16 = 6;
+// It serves K % 64 != 0, as on the tiles, and one and two tokens of rows from 1024 on, whose other kernel adds in fp32: the weights'
+// traffic bounds these (us, e4m3 instruction | this, one token, N = 3072 / 16384: K = 11008 10.7 / 36.7 | 10.9 / 37.1; two tokens,
+// 1408 4.3 / 8.0 | 4.4 / 8.5, 4608 - / 16.2 | - / 17.4).
+static bool e4m3_on_fp16(const GemvArgs& g) { return g.K % 64 || (g.M <= 2 && g.K >= 1024); }
 // per token (int8: with divisors of the 16-bit dtype, or none), with fp32 divisors, static per tensor
 enum { QUANT_TOKEN, QUANT_TOKEN_F32S, QUANT_STATIC };
 constexpr unsigned GEMV_OUTSIDE = 0x80000000u;  // past the end of every descriptor made here
@@ -308,6 +312,19 @@ __device__ __forceinline__ Acc4 gemv_mma(v4i w0, v4i w1, v4i x0, v4i x1, Acc4 ac
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(widen_fp8(w1[2], w1[3]), widen_fp8(x1[2], x1[3]), acc, 0, 0, 0);
   }
 }
+// The waves' parts of a sum in pairs, and pairs of pairs: a rounding per level, where one after the other takes one per wave
+// (e4m3, one token, 4096 x 11008, error in the 2-norm 7.3e-8 -> 5.6e-8, the row kernel's 5.5e-8).
+template <int NW, class F>
+__device__ __forceinline__ auto sum_waves(const F& part) {
+  decltype(part(0)) p[NW];
+#pragma unroll
+  for (int w = 0; w < NW; ++w) p[w] = part(w);
+#pragma unroll
+  for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+    for (int w = 0; w + d < NW; w += 2 * d) p[w] += p[w + d];
+  return p[0];
+}
 
 // XT >= 0: the activations are x16 (of that dtype), UPW units of them per wave quantized by every block for itself, in
 // LDS, while the head of its weight stream is in flight, by the quantizer QUANT.
@@ -450,9 +467,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_any_kernel(GemvArgs g, int halve
     static_assert(MT == 1 || (NW * 64) % 256 == 0, "outputs of a thread must share its column");
     for (int e = threadIdx.x; e < 256 * MT; e += NW * 64) {
       const int n = row_lo + gi * 16 + ((e >> 4) & 15), m = (e >> 8) * 16 + (e & 15);
-      AccT sum = red[gi & 1][0][e];
-#pragma unroll
-      for (int w = 1; w < NW; ++w) sum += red[gi & 1][w][e];
+      const AccT sum = sum_waves<NW>([&](int w) { return red[gi & 1][w][e]; });
       float am = as;
       if (MT > 1) am = g.a_scale ? g.a_scale[g.a_stride ? min(m, g.M - 1) : 0] : 1.f;
       if (n < row_hi && m < g.M) gemv_store(g, m, n, sum, am, ws, bv);
@@ -509,9 +524,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_short_kernel(GemvArgs g) {
     const int o = threadIdx.x + q * NW * 64, i = o >> 8, n = n0 + i * 16 + (o & 15), m = (o >> 4) & 15;
     if (i >= RG || n >= g.N || m >= g.M) continue;
     const int e = (o & 15) * 17 + m;
-    AccT sum = red[0][i][e];
-#pragma unroll
-    for (int v = 1; v < NW; ++v) sum += red[v][i][e];
+    const AccT sum = sum_waves<NW>([&](int v) { return red[v][i][e]; });
     gemv_store(g, m, n, sum, as[q], ws[q], bv[q]);
   }
 }
@@ -557,6 +570,7 @@ static AnyPlan any_plan(int64_t M, int64_t N, int64_t K) {
 // block reads again cost more than the slices' sums (32 x 1000 x 6144 9.0 -> 9.4).
 bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K, bool fp8) {
   if (M < 1 || M > 64 || K % 16) return false;
+  if (fp8 && M == 2 && K >= 1024 && K % 128 == 0) return true;  // (the tiles' e4m3 instruction keeps fewer bits)
   if (M <= 16) return M == 1 || N <= (K <= 512 ? 24576 : 8192) || K > (M == 2 ? 2048 : M <= 4 ? 2560 : 4608) || fmsmo_gemv_stream_k(K);
   if (N > 4096) return false;
   if (M <= 32) return K <= (M > 24 ? 4096 : fp8 ? 6144 : 8192);
@@ -612,14 +626,14 @@ int fmsmo_gemv_any(int op, const GemvArgs& g, hipStream_t st) {
   if (!any_offsets_ok(g)) return FMSMO_ERR_UNSUPPORTED;
   if (g.M <= 16 && g.K <= 512)
     return op == FMSMO_OP_I8 ? short_waves<FMSMO_OP_I8>(g, st)
-           : g.K % 64        ? short_waves<GEMV_FP8_F16>(g, st)
+           : e4m3_on_fp16(g) ? short_waves<GEMV_FP8_F16>(g, st)
                              : short_waves<FMSMO_OP_E4M3>(g, st);
 #define GO(OP)                                    \
   if (g.M <= 16) return any_launch<OP, 1>(g, st); \
   if (g.M <= 32) return any_launch<OP, 2>(g, st); \
   return any_launch<OP, 4>(g, st)
   if (op == FMSMO_OP_I8) { GO(FMSMO_OP_I8); }
-  if (g.K % 64) { GO(GEMV_FP8_F16); }
+  if (e4m3_on_fp16(g)) { GO(GEMV_FP8_F16); }
   GO(FMSMO_OP_E4M3);
 #undef GO
 }
@@ -630,7 +644,7 @@ static int any_fused(int op, const GemvArgs& g, hipStream_t st) {
     if (g.smooth && g.smooth_f32) return any_launch<FMSMO_OP_I8, 1, XT, QUANT_TOKEN_F32S>(g, st);
     return any_launch<FMSMO_OP_I8, 1, XT>(g, st);
   }
-  if (g.K % 64) return any_launch<GEMV_FP8_F16, 1, XT>(g, st);
+  if (e4m3_on_fp16(g)) return any_launch<GEMV_FP8_F16, 1, XT>(g, st);
   return any_launch<FMSMO_OP_E4M3, 1, XT>(g, st);
 }
 // the fused form; FMSMO_ERR_UNSUPPORTED: offsets past 32 bits, or more rows and elements than a block quantizes

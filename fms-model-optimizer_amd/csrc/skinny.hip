@@ -1037,15 +1037,17 @@ static void launch_gemv(const GemvArgs& g, hipStream_t st) {
 //     up to 1024 3.4 / 4.1 / - | 3.0 / 3.4 / -, but 20000 columns 6.4 | 7.2
 //   two tokens: 2048 4.1 / 4.4 / 6.0 | 4.0 / 4.2 / 5.9, 3072 3.6 / 4.7 / 6.5 | 4.4 / 4.9 / 7.3, 7168 4.5 / 6.5 / 12.9 | 6.1 / 7.0 / 11.8, 10240 4.7 / 8.3 / 17.6
 //     | 7.4 / 8.7 / 15.1
-//   e4m3 (twice the instructions per byte), one token: 7168 4.3 / 6.5 / 12.9 | 6.0 / 7.0 / 11.8, 10240 4.7 / 7.6 / 17.3 | 7.4 / 8.6 / 15.3, up to
-//     1024 3.7 / 4.5 / - | 3.1 / 3.4 / -; two: 3072 3.8 / 4.8 / 6.9 | 4.4 / 4.9 / 7.2, 7168 4.6 / 6.8 / 14.0 | 6.0 / 6.9 / 11.8, 10240 5.6 / 13.6 / 26.2 |
+//   e4m3 (twice the instructions per byte; both add in fp32), one token: 7168 4.3 / 6.5 / 12.9 | 6.0 / 7.0 / 11.8, 10240 4.7 / 7.6 / 17.3 | 7.4 / 8.6 /
+//     15.3, 1024 3.5 / 4.4 / - | 3.1 / 3.9 / -; two: 3072 3.8 / 4.8 / 6.9 | 4.4 / 4.9 / 7.2, 7168 4.6 / 6.8 / 14.0 | 6.0 / 6.9 / 11.8, 10240 5.6 / 13.6 / 26.2 |
 //     7.5 / 8.7 / 15.3
+//   e4m3, one token, N = 3072 / 4096 / 8320 / 12288 / 28672: 11008 9.4 / 12.6 / 20.6 / 28.3 / 56.7 | 10.9 / 12.4 / 23.8 / 33.0 / 55.9, 12928 11.7 / 13.4 / 23.2 /
+//     31.1 / 61.4 | 10.8 / 12.4 / 26.4 / 30.1 / 65.7; 1024, N = 8320 / 28672 5.4 / 8.8 | 5.7 / 10.5
 static bool rows_take(int op, int64_t M, int64_t N, int64_t K) {
   const int64_t kch = (K + 1023) / 1024;
   if (M > 2 || kch > 16) return false;
   const bool i8 = op == FMSMO_OP_I8;
-  if (kch == 1) return i8 && M == 1 && N > 8192 && K > 512;
-  if (M == 1) return i8 || kch <= 8 || N <= 2048;
+  if (kch == 1) return M == 1 && N > 8192 && (i8 ? K > 512 : K == 1024);
+  if (M == 1) return i8 || kch <= 8 || N <= 2048 || kch == 11 || kch == 13;
   if (kch == 2) return false;
   return kch <= 8 ? i8 || N <= 4096 : N <= (i8 ? 2048 : 1024);
 }
@@ -1148,7 +1150,8 @@ int fmsmo_gemv_dispatch(int op, const void* a, int64_t lda, const void* b, int64
   // G = 7).  FMSMO_GEMV_G overrides G for tuning.
   {
     static const int env_g = getenv("FMSMO_GEMV_G") ? atoi(getenv("FMSMO_GEMV_G")) : 0;
-    const int steps_total = K % 128 ? 0 : (int)(K / 128);
+    // (one e4m3 token of 1024 elements, like the longer ones that rows_take has, is added in fp32: gemv_any_kernel's form)
+    const int steps_total = K % 128 || (op == FMSMO_OP_E4M3 && M == 1 && K == 1024) ? 0 : (int)(K / 128);
     const int64_t groups = (N + 15) / 16;
     int NW = 0;
     if (steps_total && steps_total % 8 == 0) NW = 8;
@@ -1315,8 +1318,8 @@ static int decode_fused_launch(const GemvArgs& g, hipStream_t st) {
     return fmsmo_check_launch();
   }
   // (up to 1024 elements without divisors the weights' rows are too short for a wave each: us, e4m3, N = 1024 / 4096, rows -> these:
-  // K = 512 4.6 / 4.8 -> 3.6 / 3.7, 1024 4.5 / 4.7 -> 3.8 / 3.9; int8 4.5 -> 4.1, 4.5 -> 4.3)
-  const bool rows = g.M == 1 && !sf32 && g.K <= 8192 && (g.K > 1024 || g.smooth || (OP == FMSMO_OP_I8 && g.N > 8192));
+  // K = 512 4.6 / 4.8 -> 3.6 / 3.7, 1024 4.2 / 4.8 -> 3.9 / 4.6; int8 4.5 -> 4.1, 4.5 -> 4.3; over 8192 columns rows: e4m3, K = 1024, N = 8320 6.3 against 6.9)
+  const bool rows = g.M == 1 && !sf32 && g.K <= 8192 && (g.K > 1024 || g.smooth || (g.N > 8192 && (OP == FMSMO_OP_I8 || g.K == 1024)));
   const int rc = rows ? FMSMO_ERR_UNSUPPORTED : fmsmo_gemv_any_fused(OP, XT, g, st);
   return rc == FMSMO_ERR_UNSUPPORTED && g.M == 1 && !sf32 ? decode_rows_fused<OP, XT>(g, st) : rc;
 }

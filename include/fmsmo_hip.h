@@ -517,7 +517,7 @@ int fmsmo_decode_linear_fp8(const void* x, int x_dtype, int64_t ldx, const uint8
  * The same for any K that is a multiple of 16 where one launch is the better one (fmsmo_small_linear_ok != 0: one token of up to
  * 12288 elements, two to four up to 12288 in all, up to eight of 512, with at most 8192 outputs beyond one token, and every
  * shape above; fewer and shorter with fp32 divisors), else FMSMO_ERR_UNSUPPORTED.  Codes, scales and int8 results are those of the two
- * calls bit for bit.  clips (fp32 [2][M], may be NULL): the clip values as fmsmo_quant_act_i8_pertoken_clips
+ * calls bit for bit; e4m3 sums may be added in another order, by instructions that keep no fewer bits.  clips (fp32 [2][M], may be NULL): the clip values as fmsmo_quant_act_i8_pertoken_clips
  * writes them.  N * ldw < 2^31 for the shapes that the calls above refuse, otherwise as there.
  */
 int fmsmo_small_linear_ok(int64_t M, int64_t N, int64_t K, int smooth_f32);
