@@ -67,6 +67,11 @@ __device__ __forceinline__ float scalar_f32(const void* p, int dt, int64_t i = 0
          : dt == FMSMO_BF16 ? bf16_to_f32(((const u16*)p)[i])
                             : ((const float*)p)[i];
 }
+// The scalar at `at`, of dtype dt, from the aligned 32-bit word that holds it.
+__device__ __forceinline__ float scalar_of_word(uint32_t word, uintptr_t at, int dt) {
+  const u16 h = (u16)(word >> ((at & 2) * 8));
+  return dt == FMSMO_F16 ? f16_to_f32(h) : dt == FMSMO_BF16 ? bf16_to_f32(h) : __uint_as_float(word);
+}
 template <int T>
 __device__ __forceinline__ void store_from_f32(void* p, size_t i, float v) {
   if constexpr (T == FMSMO_F16) ((u16*)p)[i] = f32_to_f16(v);

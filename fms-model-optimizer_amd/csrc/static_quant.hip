@@ -19,19 +19,24 @@ struct StaticArgs {
   float* s_out;
 };
 // (A product behind the quantizer reads its scale as fp32.  A launch of its own for the one conversion takes 2 us, and
-// a copy kept on the host's side would not follow the buffer in a replayed graph.)
-__device__ __forceinline__ void put_scale(const StaticArgs& p) {
-  if (p.s_in && blockIdx.x == 0 && threadIdx.x == 0) *p.s_out = scalar_f32(p.s_in, p.s_dtype);
+// a copy kept on the host's side would not follow the buffer in a replayed graph.)  By one more block, the last: in front of
+// a block's own work the read would make the shortest launches longer.  Returns the blocks that quantize, 0 in the last one.
+__device__ __forceinline__ unsigned put_scale(const StaticArgs& p) {
+  if (!p.s_in) return gridDim.x;
+  if (blockIdx.x != gridDim.x - 1) return gridDim.x - 1;
+  if (threadIdx.x == 0) *p.s_out = scalar_f32(p.s_in, p.s_dtype);
+  return 0;
 }
 
 template <int XT, int T>
 __global__ __launch_bounds__(256) void quant_i8_static_t_kernel(const void* __restrict__ x, int64_t ldx,
                                                                 StaticArgs p, int8_t* __restrict__ q,
                                                                 int64_t ldq, int M, int K) {
-  put_scale(p);
+  const unsigned blocks = put_scale(p);
+  if (!blocks) return;
   const int cpr = K / AQ_VEC;
   const int64_t total = (int64_t)M * cpr;
-  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < total; c += (int64_t)gridDim.x * 256) {
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < total; c += (int64_t)blocks * 256) {
     const int64_t m = c / cpr;
     const int k = (int)(c - m * cpr) * AQ_VEC;
     float v[8];
@@ -81,14 +86,15 @@ template <int T, int MODE>
 __global__ __launch_bounds__(256) void quant_i8_static16_kernel(const u16* __restrict__ x, StaticArgs p,
                                                                 float rcp_scale, int8_t* __restrict__ q,
                                                                 int64_t nchunks) {
-  put_scale(p);
+  const unsigned blocks = put_scale(p);
+  if (!blocks) return;
   const float nz = opaque_neg_zero();
   auto rnd2 = [](float& a, float& b) {
     const uint32_t w = pack16<T>(a, b);
     a = cvt16<T>((u16)(w & 0xffff));
     b = cvt16<T>((u16)(w >> 16));
   };
-  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)gridDim.x * 256) {
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)blocks * 256) {
     const v4i raw = __builtin_nontemporal_load((const v4i*)(x + c * AQ_VEC));
     uint32_t code[4];
 #pragma unroll
@@ -142,10 +148,11 @@ __global__ __launch_bounds__(256) void quant_i8_static16_kernel(const u16* __res
 template <int XT>
 __global__ __launch_bounds__(256) void quant_i8_static_fmo32_kernel(const u16* __restrict__ x, StaticArgs p, float rcp,
                                                                     int8_t* __restrict__ q, int64_t nchunks) {
-  put_scale(p);
+  const unsigned blocks = put_scale(p);
+  if (!blocks) return;
   const float nz = opaque_neg_zero();
   const int shift = 128 - (int)p.sym;
-  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)gridDim.x * 256) {
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < nchunks; c += (int64_t)blocks * 256) {
     const v4i raw = __builtin_nontemporal_load((const v4i*)(x + c * AQ_VEC));
     uint32_t code[4];
 #pragma unroll
@@ -415,7 +422,7 @@ static int static_t_impl(const void* x, int x_dtype, int64_t ldx, int mode, int 
   if (compute_dtype != FMSMO_F32 && compute_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
   if (M == 0) return FMSMO_OK;
   StaticArgs p{scale, zp, (float)(sym ? 1 : 0), clip_lo, clip_hi, mode, scale_in, scale_dtype, scale_out};
-  dim3 grid(grid_for(M, K)), block(256);
+  dim3 grid((unsigned)grid_for(M, K) + (scale_in ? 1 : 0)), block(256);
   hipStream_t st = (hipStream_t)stream;
   // 16-bit compute dtype, contiguous rows, a divisor that is a finite non-zero value of that dtype
   // (inside 2^-60 .. 2^60 for bf16) and, for the formula that does not clamp its codes, clip values

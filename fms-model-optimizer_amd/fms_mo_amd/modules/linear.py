@@ -847,7 +847,8 @@ class QLinearINT8Deploy(nn.Linear):
                 own = kept[1] if kept and kept[1].data_ptr() != kept[2].data_ptr() else None
                 if own is not None and f.data_ptr() != ws.data_ptr() and own.shape == f.shape and own.device == f.device:
                     f = own.copy_(f)
-                if f.is_cuda:   # (whichever stream reads it next)
+                # complete before another stream is given it (the first forward waits in _smoothq_active, right behind)
+                if f.is_cuda and getattr(self, "_sq_kept", None):
                     torch.cuda.current_stream(f.device).synchronize()
             self._ws_kept = kept = _Kept((stamp, f, ws.detach()))
         return kept[1]
@@ -877,6 +878,8 @@ class QLinearINT8Deploy(nn.Linear):
         x2 = x if two_d else x.reshape(-1, K)
         if not x2.is_cuda:
             raise RuntimeError("fms_mo_amd.QLinearINT8Deploy runs on an AMD GPU only; there is no CPU path")
+        if not (torch.compiler.is_compiling() or getattr(self, "_ws_kept", None)):
+            self._w_scale_f32()
         use_sq = self._smoothq_active()
         plain = (self.useDynMaxQfunc == -1 and self.use_int_kernel
                  and not (K > self.chunk_size or self.truncate_lsb > 0)
