@@ -677,6 +677,7 @@ extern "C" int fmsmo_small_linear_ok(int64_t M, int64_t N, int64_t K, int smooth
 
 static int small_linear(int op, const void* x, int x_dtype, int64_t ldx, const void* smooth, int smooth_dtype, const void* w,
                         int64_t ldw, const float* w_scale, int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
+// (Those N = 4096 times had the product that streamed such K then; against the present ones and other N, see fmsmo_small_linear_better.)
                         void* y, int y_dtype, int64_t ldy, float* a_scale_out, float* clips, int64_t M, int64_t N, int64_t K,
                         fmsmo_stream_t stream) {
   if (!x || !w || !w_scale || !y) return FMSMO_ERR_NULL;
@@ -685,6 +686,36 @@ static int small_linear(int op, const void* x, int x_dtype, int64_t ldx, const v
   if (x_dtype != FMSMO_F16 && x_dtype != FMSMO_BF16) return FMSMO_ERR_UNSUPPORTED;
   const bool sf32 = smooth && smooth_dtype == FMSMO_F32;
   if (smooth && !sf32 && smooth_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
+// Where one launch is the better one of those it takes: 1.  2: where a second launch and its buffers cost the host 3 us, the calls that keep
+// the GPU longer but still take less of its time than two calls take of the host's (int8, whose results are the same bits either way).  Weights from HBM,
+// us on the GPU, one launch | two calls:
+//   int8, one token: 640 x 8208 8.7 | 7.3, 640 x 12288 10.1 | 7.2, 5504 x 12288 22.6 | 17.9, 4096 x 10240 12.4 | 12.6; up to K = 8192 0.5 .. 1.9 less,
+//     over 5504 columns and more down to the same
+//   e4m3, one token: 640 x 12288 10.5 | 9.0, 1024 x 9216 9.1 | 8.6, 2048 x 9216 10.4 | 10.2, 3072 x 9216 10.6 | 12.2; 7168 x 4352 12.8 | 11.1, 8192 x 6144 16.2 |
+//     14.0, 11008 x 7168 22.9 | 20.8, 11008 x 6144 17.3 | 17.6, 7168 x 3072 9.4 | 9.0
+//   two tokens, int8: 1024 x 3072 6.3 | 6.1, 256 x 4224 7.3 | 6.9, 4096 x 4224 8.8 | 9.5, 6144 x 3072 9.4 | 8.7, 6144 x 4224 13.2 | 10.9, 1024 x 6144 8.5 | 7.5; e4m3: 6144 x
+//     5376 15.1 | 13.8, 6144 x 4224 12.1 | 11.9, 1024 x 6144 8.7 | 7.8
+//   three, int8: 6144 x 3072 11.5 | 10.4, 6144 x 2304 10.2 | 9.6, 6144 x 1152 8.1 | 7.5; four: 6144 x 3072 12.9 | 10.7, 6144 x 1152 8.2 | 7.4, 6144 x 1024 6.8 | 6.9, 2048 x
+//     2048 6.6 | 5.9, 2048 x 2304 7.1 | 7.2; e4m3 6144 x 3072 11.5 | 9.7, 6144 x 2304 9.9 | 9.2; six, int8: 6144 x 256 6.2 | 5.0, 4096 x 256 4.7 | 4.8
+//   fp32 divisors: 1 x 6144 x 640 7.1 | 6.7, 2 x 4096 x 512 5.4 | 4.9, 2 x 6144 x 512 7.1 | 5.6, 2 x 6144 x 1024 7.3 | 7.1, 6 x 2048 x 256 5.9 | 4.7
+// (eager, weights in cache: int8 4 x 2048 x 1024 6.0 | 9.3, 6 x 256 x 6144 6.2 | 9.4 - 10.4, 1 x 11264 x 640 9.1 | 9.2 - 10.0; e4m3 1 x 4992 x 7168 10.9 | 9.6 - 10.0)
+extern "C" int fmsmo_small_linear_better(int fp8, int64_t M, int64_t N, int64_t K, int smooth_f32) {
+  if (!fmsmo_small_linear_ok(M, N, K, smooth_f32)) return 0;
+  if (smooth_f32 ? fmsmo_decode_linear_f32s_ok(M, K) : fmsmo_decode_linear_ok(M, K)) return 1;
+  if (smooth_f32) return M == 1 || (K > 512 && (M == 2 || N <= 4096)) ? 1 : 2;
+  if (fp8) {
+    if (M == 1) return K > 8192 ? N > 2048 : N <= 4096 || K <= (N > 8192 ? 6144 : 4096);
+    return N <= 4096 || K <= (M == 2 ? 4608 : M == 3 ? 4096 : 2304);
+  }
+  if (M == 1) return K <= 8192 ? 1 : N <= 2048 ? 2 : 0;
+  if (N > 4096) {
+    if (K > (M == 2 ? 3072 : 2304)) return 0;
+    return K <= (M == 2 ? 2048 : M <= 4 ? 1024 : 0) ? 1 : 2;
+  }
+  if (M == 2) return K <= (N > 2048 ? 4608 : 3072) ? 1 : 2;
+  return M == 4 && fmsmo_gemv_stream_k(K) && K > 1024 ? 2 : 1;
+}
+
   if (!fmsmo_small_linear_ok(M, N, K, sf32)) return FMSMO_ERR_UNSUPPORTED;
   if (N * ldw >= (fmsmo_decode_linear_ok(M, K) ? 1ll << 40 : 1ll << 31)) return FMSMO_ERR_UNSUPPORTED;
   if (y_dtype < 0 || y_dtype > 2 || (bias && (bias_dtype < 0 || bias_dtype > 2))) return FMSMO_ERR_UNSUPPORTED;

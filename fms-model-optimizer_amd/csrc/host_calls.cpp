@@ -28,7 +28,7 @@ namespace {
   X(fmsmo_quant_act_fp8_pertoken) X(fmsmo_quant_act_fp8_dynamic) X(fmsmo_quant_act_fp8_tensor)           \
   X(fmsmo_quant_act_i8_static_scale) X(fmsmo_quant_act_i8_pertoken_clips) X(fmsmo_gemm_i8_dq_ws) X(fmsmo_gemm_fp8_dq_ws) X(fmsmo_gemm_workspace_bytes)      \
   X(fmsmo_gemm_fp8_workspace_bytes) X(fmsmo_decode_linear_i8) X(fmsmo_decode_linear_fp8)                 \
-  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_small_linear_ok) X(fmsmo_small_linear_i8) X(fmsmo_small_linear_fp8) X(fmsmo_small_linear_static_ok) X(fmsmo_small_linear_i8_static_scale) X(fmsmo_grouped_gemm_i8_dq)                   \
+  X(fmsmo_decode_linear_ok) X(fmsmo_decode_linear_f32s_ok) X(fmsmo_small_linear_better) X(fmsmo_small_linear_i8) X(fmsmo_small_linear_fp8) X(fmsmo_small_linear_static_ok) X(fmsmo_small_linear_i8_static_scale) X(fmsmo_grouped_gemm_i8_dq)                   \
   X(fmsmo_matmul_chunk_i8_dq_ws) X(fmsmo_matmul_chunk_fp_dq) X(fmsmo_matmul_chunk_workspace_bytes)    \
   X(fmsmo_quant_i8_affine_sums) X(fmsmo_quant_i8_affine_pair) X(fmsmo_affine_sum_parts) X(fmsmo_affine_parts_first) X(fmsmo_affine_add_parts) X(fmsmo_bmm_qa_ok)   \
   X(fmsmo_bmm_qa_i8) X(fmsmo_bmm_i8_zp)
@@ -132,6 +132,13 @@ bool here(const T*... t) {
   return !c10::impl::TorchDispatchModeTLS::any_modes_set() && ((!t || t->get_device() == d) && ...);
 }
 void* stream_of(const at::Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+// part of a graph: its launches cost the host nothing when it is replayed
+bool capturing(const at::Tensor& t) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream_of(t), &s) == hipSuccess) return s == hipStreamCaptureStatusActive;
+  (void)hipGetLastError();
+  return false;
+}
 at::Tensor empty(at::IntArrayRef sizes, at::ScalarType st, const at::Tensor& like) {
   return at::empty(sizes, like.options().dtype(st).requires_grad(false));
 }
@@ -681,8 +688,9 @@ PyObject* deploy_i8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool f32s = smooth && sm.st == at::kFloat;
   const bool one = (!smooth || sm.st == xt || f32s) &&
                    (f32s ? p_fmsmo_decode_linear_f32s_ok(x.rows, x.cols) : p_fmsmo_decode_linear_ok(x.rows, x.cols));
-  const bool small = !one && (!smooth || sm.st == xt || f32s) && w.rows * w.ld < (1ll << 31) &&
-                     p_fmsmo_small_linear_ok(x.rows, w.rows, x.cols, f32s);
+  const int in_one = !one && (!smooth || sm.st == xt || f32s) && w.rows * w.ld < (1ll << 31)
+                         ? p_fmsmo_small_linear_better(0, x.rows, w.rows, x.cols, f32s) : 0;
+  const bool small = in_one == 1 || (in_one == 2 && !capturing(*x.t));
   if (one || smooth || small) s = empty({x.rows, 1}, at::kFloat, *x.t);
   if (one) {
     // decode step of a few tokens: quantizer and weight-streaming matmul in one launch
@@ -756,7 +764,7 @@ PyObject* fp8_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   at::Tensor y = out_like(*x.t, w.rows, xt);
   if (!per_tensor && floor == 1e-12 && !in_x && xt != at::kFloat &&
       (p_fmsmo_decode_linear_ok(x.rows, x.cols) ||
-       (w.rows * w.ld < (1ll << 31) && p_fmsmo_small_linear_ok(x.rows, w.rows, x.cols, 0)))) {
+       (w.rows * w.ld < (1ll << 31) && p_fmsmo_small_linear_better(1, x.rows, w.rows, x.cols, 0)))) {
     if (!LAUNCH(fmsmo_small_linear_fp8, x.p, code_of(xt), x.ld, (const uint8_t*)w.p, w.ld, wp, ws->numel(), b.p, b.dt,
                 y.data_ptr(), code_of(xt), w.rows, (float*)nullptr, x.rows, w.rows, x.cols, stream_of(*x.t)))
       return nullptr;

@@ -110,6 +110,7 @@ OTHER = {
     "fmsmo_decode_linear_ok": ([c_int64, c_int64], c_int),
     "fmsmo_decode_linear_f32s_ok": ([c_int64, c_int64], c_int),
     "fmsmo_small_linear_static_ok": ([c_int64, c_int64, c_int64, _F, _F, _F, _F], c_int),
+    "fmsmo_small_linear_better": ([c_int, c_int64, c_int64, c_int64, c_int], c_int),
     "fmsmo_small_linear_ok": ([c_int64, c_int64, c_int64, c_int], c_int),
     "fmsmo_gemm_tail_columns": ([c_int64, c_int64, c_int64], c_int64),
     "fmsmo_gemm_fp8_tail_columns": ([c_int64, c_int64, c_int64], c_int64),

@@ -514,13 +514,16 @@ int fmsmo_decode_linear_fp8(const void* x, int x_dtype, int64_t ldx, const uint8
                             int bias_dtype, void* y, int y_dtype, int64_t ldy, float* a_scale_out,
                             int64_t M, int64_t N, int64_t K, fmsmo_stream_t stream);
 /*
- * The same for any K that is a multiple of 16 where one launch is the better one (fmsmo_small_linear_ok != 0: one token of up to
+ * The same for any K that is a multiple of 16 (fmsmo_small_linear_ok != 0: one token of up to
  * 12288 elements, two to four up to 12288 in all, up to eight of 512, with at most 8192 outputs beyond one token, and every
  * shape above; fewer and shorter with fp32 divisors), else FMSMO_ERR_UNSUPPORTED.  Codes, scales and int8 results are those of the two
  * calls bit for bit; e4m3 sums may be added in another order, by instructions that keep no fewer bits.  clips (fp32 [2][M], may be NULL): the clip values as fmsmo_quant_act_i8_pertoken_clips
  * writes them.  N * ldw < 2^31 for the shapes that the calls above refuse, otherwise as there.
  */
 int fmsmo_small_linear_ok(int64_t M, int64_t N, int64_t K, int smooth_f32);
+/* Is one launch the better one (e4m3: fp8 != 0)?  0: no (also for shapes that fmsmo_small_linear_ok refuses), 1: yes, 2: where a launch costs
+ * host time, not in a graph. */
+int fmsmo_small_linear_better(int fp8, int64_t M, int64_t N, int64_t K, int smooth_f32);
 int fmsmo_small_linear_i8(const void* x, int x_dtype, int64_t ldx, const void* smooth, int smooth_dtype, const int8_t* w,
                           int64_t ldw, const float* w_scale, int64_t w_scale_n, const void* bias, int bias_dtype,
                           int epilogue, void* y, int y_dtype, int64_t ldy, float* a_scale_out, float* clips, int64_t M,

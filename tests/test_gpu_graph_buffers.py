@@ -89,3 +89,31 @@ def test_replay_of_a_dynamic_forward_follows_the_scale_of_the_weights(dev, M):
     assert torch.equal(want, m(x)) and not torch.equal(want, y)
     late.replay()
     assert torch.equal(z, want)
+
+
+@pytest.mark.parametrize("M,N,K,smooth", [(1, 640, 9216, False), (2, 256, 6144, False), (4, 1024, 2048, True), (6, 4112, 256, True)])
+def test_replay_of_what_is_one_launch_eagerly_and_two_in_a_graph(dev, M, N, K, smooth):
+    """The same bits and the same scales either way."""
+    from fms_mo_amd import _lib as L
+    from fms_mo_amd.modules.linear import QLinear, QLinearINT8Deploy
+
+    assert L.load().fmsmo_small_linear_better(0, M, N, K, 0) == 2
+    q = QLinear(K, N, bias=True, num_bits_feature=8, qa_mode="pertokenmax", num_bits_weight=8, qw_mode="maxperCh",
+                qcfg={"smoothq": smooth, "smoothq_alpha": 0.5}, device=dev).to(dev).half()
+    q.quantize_weight.float()
+    with torch.no_grad():
+        q.quantize_weight.clip_val.copy_(q.weight.abs().amax(dim=1))
+    if smooth:
+        q.smoothq_act_scale = torch.rand(K, device=dev) + 0.1
+        q.smoothq_alpha = torch.full((1,), 0.5, device=dev)
+    m = QLinearINT8Deploy.from_fms_mo(q.eval(), use_dynamic_max_act_Qfunc=-1, recalc_clipvals=False).half()
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half().to(dev)
+    graph, y = captured(m, x)
+    scale = m.input_scale
+    graph.replay()
+    want = m(x)
+    assert torch.equal(y, want) and torch.equal(scale, m.input_scale)
+    x.mul_(1.5)
+    graph.replay()
+    want = m(x)
+    assert torch.equal(y, want) and torch.equal(scale, m.input_scale)

@@ -1,0 +1,18 @@
+"""Where a dispatch has its lines, without a GPU: shapes on either side that were measured with the weights coming from memory."""
+import pytest
+
+from fms_mo_amd import _lib as L
+from fms_mo_amd import kernels
+
+
+@pytest.mark.parametrize("fp8,M,N,K,smooth_f32,better", [
+    (0, 1, 640, 8192, 0, 1), (0, 1, 640, 8208, 0, 2), (0, 1, 2064, 8208, 0, 0), (1, 1, 1024, 11008, 0, 0), (1, 1, 4096, 10240, 0, 1),
+    (1, 1, 7168, 4352, 0, 0), (1, 1, 4096, 4352, 0, 1), (1, 1, 11008, 6144, 0, 1), (1, 1, 11008, 7168, 0, 0),
+    (0, 2, 6144, 4224, 0, 0), (0, 2, 6144, 3072, 0, 2), (0, 2, 4096, 4224, 0, 1), (0, 2, 1024, 6144, 0, 2), (1, 2, 6144, 4224, 0, 1),
+    (1, 2, 6144, 6144, 0, 0), (0, 3, 6144, 3072, 0, 0), (1, 3, 6144, 3072, 0, 1), (0, 4, 6144, 1152, 0, 2), (0, 4, 4096, 3072, 0, 1),
+    (0, 4, 4096, 2048, 0, 2), (1, 4, 6144, 3072, 0, 0), (0, 6, 6144, 256, 0, 2), (0, 6, 4096, 256, 0, 1), (1, 8, 8192, 512, 0, 1),
+    (0, 2, 6144, 512, 1, 2), (0, 2, 6144, 1024, 1, 1), (0, 1, 6144, 1024, 1, 1), (0, 6, 2048, 256, 1, 2),
+    (0, 1, 28672, 4096, 1, 1), (0, 3, 4096, 14336, 0, 1), (1, 1, 8192, 8192, 0, 1),   # shapes of the streaming kernel and of whole rows
+    (0, 9, 64, 512, 0, 0), (0, 1, 4096, 16400, 0, 0), (0, 1, 4096, 5377, 0, 0)])      # not taken at all
+def test_one_launch_only_where_it_is_the_better_one(fp8, M, N, K, smooth_f32, better):
+    assert L.load().fmsmo_small_linear_better(fp8, M, N, K, smooth_f32) == better
