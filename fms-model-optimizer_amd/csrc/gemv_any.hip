@@ -564,21 +564,27 @@ static AnyPlan any_plan(int64_t M, int64_t N, int64_t K) {
   return {8, 512};
 }
 
-// Up to 16 tokens: every K that skinny.hip has no instance for, but for several tokens and short rows over more columns than one
-// round of blocks takes, where tiles of 64 x 64 or 32 x 128 with their deeper loads win (us, this kernel against them, int8: 3 x 10473 x 1632 9.1 /
-// 7.4, 8 x 8327 x 4160 14.1 / 11.3, 16 x 9412 x 2272 10.9 / 8.4, 16 x 24703 x 1424 16.2 / 9.7, 5 x 27721 x 3120 25.2 / 21.8; kept: 3 x 17661 x 3024 16.9 / 18.9,
-// 2 x 26780 x 3968 19.7 / 21.0, 5 x 19664 x 5152 27.1 / 28.9, 13 x 7811 x 1792 6.7 / 7.2, 1 x 12736 x 2032 7.6 / 8.3; rows of 512 at most, gemv_short_kernel: 8 x
-// 10848 x 448 4.4 / 5.0, 4 x 17166 x 512 5.6 / 5.5, 16 x 26612 x 512 7.0 / 6.2, 4 x 53216 x 256 7.1 / 6.5).  More: where the tiled kernels would take slices of K or
-// launch too few tiles (us, those -> this one, int8): 17 x 4096: K = 528 5.6 -> 3.7, 1536 8.3 -> 4.4, 4480 10.2 -> 7.2, 9088
-// 13.5 -> 11.0; 32 x 1000: K = 896 5.1 -> 3.9, 2304 7.4 -> 5.8, 4480 8.2 -> 8.4; 32 x 4096 x 4480 10.7 -> 8.8; 40 x 2100: 896 7.1 ->
-// 4.8, 3328 9.3 -> 8.4; from 48 tokens on, and e4m3 from 33 on, 64 x 64 tiles (this / those: int8 33 x 2081 x 1536 6.4 / 6.9, 48 x 3256 x 1280 6.7 / 6.7, 64 x
-// 1857 x 1792 7.9 / 7.4; e4m3 33 x 2277 x 1152 6.1 / 5.6, 64 x 1776 x 1792 7.9 / 6.4).  From 4096
-// columns on 64 x 64 tiles fill the chip in one pass (32 x 8192 x 1536 6.6 -> 7.2).  Longer rows: the activations that every
-// block reads again cost more than the slices' sums (32 x 1000 x 6144 9.0 -> 9.4).
+// Up to 16 tokens: every K that skinny.hip has no instance for, except short rows over more columns than one round of blocks takes, where tiles of
+// 64 x 64 or 32 x 128 with their deeper loads win.  us with the tokens' quantizer, weights from HBM, tiles | this kernel:
+//   up to 16384 columns: int8 2 x 9216 x 640 8.1 | 7.4, 4 x 14336 x 1152 10.4 | 10.3, 5 x 14336 x 1536 11.9 | 10.9, 5 x 11008 x 2816 16.1 | 13.7 (e4m3 16.5 | 13.6),
+//     16 x 9216 x 2816 14.9 | 14.7; K % 128 != 0 10 x 9216 x 3600 18.2 | 18.5, 16 x 9216 x 3600 18.3 | 20.2
+//   more: 5 x 24576 x 1536 14.0 | 14.4, 10 x 24576 x 2176 16.9 | 18.6, 10 x 24576 x 2816 19.8 | 20.2, 10 x 18944 x 4480 (e4m3) 26.4 | 25.9, 16 x 24576 x 3584 23.8 | 26.6;
+//     K % 128 != 0 5 x 18944 x 1616 16.4 | 14.9, 10 x 18944 x 3600 28.4 | 26.4, 16 x 18944 x 1616 16.8 | 16.8
+//   rows of 512 at most, gemv_short_kernel (products alone, weights in cache): 4 x 17166 x 512 5.5 | 5.6, 8 x 10848 x 448 5.0 | 4.4, 16 x 26612 x 512 6.2 | 7.0, 4 x 53216 x 256 6.5 | 7.1
+// More tokens: where the tiled kernels would take slices of K or launch too few tiles.  Products alone, weights in cache, tiles | this kernel, int8:
+//   17 x 4096: K = 528 5.6 | 3.7, 1536 8.3 | 4.4, 4480 10.2 | 7.2, 9088 13.5 | 11.0; 32 x 1000: 896 5.1 | 3.9, 2304 7.4 | 5.8, 4480 8.2 | 8.4; 32 x 4096 x 4480 10.7 | 8.8;
+//   40 x 2100: 896 7.1 | 4.8, 3328 9.3 | 8.4; from 48 tokens on, and e4m3 from 33 on, 64 x 64 tiles: 33 x 2081 x 1536 6.9 | 6.4, 48 x 3256 x 1280 6.7 | 6.7, 64 x 1857 x
+//   1792 7.4 | 7.9, e4m3 33 x 2277 x 1152 5.6 | 6.1, 64 x 1776 x 1792 6.4 | 7.9
+//   From 4096 columns on 64 x 64 tiles fill the chip in one pass (32 x 8192 x 1536 6.6 | 7.2).  Longer rows: the activations that every block reads
+//   again cost more than the slices' sums (32 x 1000 x 6144 9.0 | 9.4).
 bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K, bool fp8) {
   if (M < 1 || M > 64 || K % 16) return false;
   if (fp8 && M == 2 && K >= 1024 && K % 128 == 0) return true;  // (the tiles' e4m3 instruction keeps fewer bits)
-  if (M <= 16) return M == 1 || N <= (K <= 512 ? 24576 : 8192) || K > (M == 2 ? 2048 : M <= 4 ? 2560 : 4608) || fmsmo_gemv_stream_k(K);
+  if (M <= 16) {
+    if (M == 1 || N <= (K <= 512 ? 24576 : 8192) || fmsmo_gemv_stream_k(K)) return true;
+    if (M > 10 && (K % 128 || N > 16384)) return K > 4608;
+    return K > (N <= 16384 ? (M == 2 ? 512 : 1024) : K % 128 ? 1024 : 2304);
+  }
   if (N > 4096) return false;
   if (M <= 32) return K <= (M > 24 ? 4096 : fp8 ? 6144 : 8192);
   return K % 128 ? K <= 1024 : !fp8 && M <= 48 && N > 1024 && K > 640 && K <= 2304;

@@ -16,3 +16,13 @@ from fms_mo_amd import kernels
     (0, 9, 64, 512, 0, 0), (0, 1, 4096, 16400, 0, 0), (0, 1, 4096, 5377, 0, 0)])      # not taken at all
 def test_one_launch_only_where_it_is_the_better_one(fp8, M, N, K, smooth_f32, better):
     assert L.load().fmsmo_small_linear_better(fp8, M, N, K, smooth_f32) == better
+
+
+@pytest.mark.parametrize("M,N,K,decode", [
+    (5, 11008, 2816, True), (3, 10240, 2560, True), (16, 9088, 1664, True), (2, 12288, 640, True), (13, 8320, 640, False),
+    (4, 14336, 1024 - 128, False), (10, 24576, 2432, True), (10, 24576, 2176, False), (12, 24576, 2432, False), (16, 16384, 2816, True),
+    (5, 18944, 1616, True), (16, 9216, 3600, False), (10, 9216, 3600, True), (1, 28672, 528, True), (16, 24576, 5248, True)])
+def test_a_few_tokens_over_many_columns(M, N, K, decode):
+    for fp8 in (False, True):
+        assert (kernels.gemm_plan(M, N, K, fp8=fp8)[0] == L.PLAN_DECODE) is decode
+        assert K % 64 or kernels._workspace(M, N, K, "cpu", fp8) is None
