@@ -511,10 +511,14 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
   const int64_t room = limit > 0 ? limit / (M * N * 4) : 256;
   const int64_t tiles_s = (int64_t)div_up(M, TileSmallK::BM) * div_up(N, TileSmallK::BN);
   // Up to 256 rows one pass of the tiles of a_few_rows takes less than slices and their sums do: of 33 64 x 64 tiles or more below K = 4096, of 129 or more
-  // below 8192 (where slices of 128 x 64 tiles would be but two), of more than a round always.  (int8 at K = 2048, up to 128 tiles, and 4096, where tests
-  // count on slices, keeps them, and not for their speed.)
-  if (M <= 256 && K % 128 == 0 && (tiles_s > 256 || (tiles_s > (fp8 || K > 2048 ? 32 : 128) && K >= 2048 && K < 4096) ||
-                                   (M <= 128 && tiles_s > 128 && tiles_t > 64 && K < 8192 && K >= (fp8 ? 4096 : 4224))))
+  // below 6144 (where slices of 128 x 64 tiles would be but two), of more than a round always.  (int8 at K = 2048, up to 128 tiles, and 4096, where tests
+  // count on slices, keeps them, and not for their speed.)  With the weights from HBM a pass of few tiles has too few loads in flight: then below
+  // K = 3072 up to 64 rows, or up to 72 tiles, and below 3584 up to 128 tiles (us, one pass | slices, e4m3: 40 x 2176 x 3968 17.4 | 13.7, 40 x 4096 x 3072 15.3 |
+  // 13.8, 32 x 6784 x 3584 17.2 | 16.2, 64 x 2176 x 2560 14.2 | 13.8, 64 x 8192 x 2560 15.3 | 16.8, 80 x 2176 x 3328 15.5 | 14.3, 128 x 4096 x 3328 16.1 | 17.7, 80 x
+  // 5504 x 6912 26.7 | 23.8, 80 x 5504 x 4608 20.0 | 19.8, 128 x 5504 x 4608 20.6 | 21.2; int8 40 x 2176 x 3968 16.5 | 13.5, 64 x 4096 x 3584 16.1 | 15.5).
+  const int64_t one_pass_below = M > 128 || tiles_s > 128 ? 4096 : M <= 64 || tiles_s <= 72 ? 3072 : 3584;
+  if (M <= 256 && K % 128 == 0 && (tiles_s > 256 || (tiles_s > (fp8 || K > 2048 ? 32 : 128) && K >= 2048 && K < one_pass_below) ||
+                                   (M <= 128 && tiles_s > 128 && tiles_t > 64 && K < 6144 && K >= (fp8 ? 4096 : 4224))))
     return p;
   if (K % 128 == 0 && tiles_s <= 32 && K > 2048) {
     // Few tiles: slices on 64 x 64 ones, four (eight of a long reduction: from then on the partial sums cost more

@@ -26,3 +26,14 @@ def test_a_few_tokens_over_many_columns(M, N, K, decode):
     for fp8 in (False, True):
         assert (kernels.gemm_plan(M, N, K, fp8=fp8)[0] == L.PLAN_DECODE) is decode
         assert K % 64 or kernels._workspace(M, N, K, "cpu", fp8) is None
+
+
+@pytest.mark.parametrize("M,N,K,splits", [
+    (40, 2176, 3968, 3), (40, 4096, 3072, 3), (32, 6784, 3584, 2), (64, 4096, 3584, 3), (80, 2176, 3328, 3), (128, 4096, 3968, 3), (80, 5504, 6912, 2),
+    (64, 8192, 2560, 1), (64, 2176, 2560, 1), (64, 11008, 3584, 1), (128, 4096, 3328, 1), (128, 5504, 4608, 1), (200, 700, 3968, 1)])
+def test_slices_where_one_pass_has_too_few_loads_in_flight(M, N, K, splits):
+    for fp8 in (False, True):
+        plan = kernels.gemm_plan(M, N, K, with_workspace=True, fp8=fp8)
+        assert plan[3] == splits and (splits > 1 or plan[1:3] == (64, 64))
+        ws = kernels._workspace(M, N, K, "cpu", fp8)
+        assert (0 if ws is None else ws.numel()) == (splits * M * N * 4 if splits > 1 else 0)
