@@ -11,13 +11,14 @@ struct TileHalfK { static constexpr int BM = 64, BN = 128, BK = 128, NST = 3, WG
 // and K % 128 != 0 no more than that).  The host knows rows and experts, not their split, and takes every expert's last tile to be half full.
 // A launch takes a round at least, however few its tiles (taken as half a one, up to a dozen tiles went to 256 x 256; us,
 // -> as now: 4, 9, 130, 256 8.8 -> 3.9; 7, 949, 59, 448 24.7 -> 9.0; of 60 such launches all faster, 13.8 -> 6.2 in the mean).
-// From K = 1024 on a finer estimate, for rows that fall on the experts alike, may choose another tile where an eighth is to be gained (a tenth: 4, 3055, 3584, 1664 unevenly split 9 % slower).  With n the tiles
-// per compute unit and s the stages of 128 bytes: one block to a unit, max(1, w ceil(n) + (1 - w) n) rounds of a + b s, of which a chip filled to n < 1
-// saves c (1 - n); two to a unit, the second one slows the first's stages by 1 + q; the mean over n 4 % and 1 % less and 6 % more, for the step at whole rounds.
+// From K = 1024 on a finer estimate, for rows that fall on the experts alike, may choose another tile where 13 % are to be gained (with an eighth less
+// asked for, 4, 3055, 3584, 1664 unevenly split ran 9 % longer).  With n the tiles per compute unit and s the stages of 128 bytes: one block to a unit,
+// max(1, w ceil(n) + (1 - w) n) rounds of a + b s, of which a chip filled to n < 1 saves c (1 - n); two to a unit, the second one slows the first's
+// stages by 1 + q; the mean over n 4 % and 1 % less and 6 % more, for the step at whole rounds.
 // Parameters fitted to two thirds of 960 launches with every tile timed (4, 8, 16 experts, 128 .. 8192 rows, K and N of hidden sizes 1024 .. 4096 and
-// intermediate ones to 14336): 0.93 of the time of the rounds alone, the best tile of each 0.91 (two runs of one tile differ by 0.03).
-// us, before -> now (experts, rows, N, K): 16, 7145, 1408, 1024 36.8 -> 22.6; 8, 547, 2688, 5120 37.1 -> 23.3; 16, 2005, 3328,
-// 5632 112 -> 72.8; 4, 1310, 3328, 7040 61.0 -> 41.1; 8, 675, 5376, 2432 35.6 -> 22.5.  900 random launches 0.92 of the time, 25 of them slower by 3 % or more (16, 2674, 2048, 9856 100 -> 130).
+// intermediate ones to 14336), weights mostly in the last-level cache.  With weights from memory, over 1200 launches of those ranges: 0.927 of the time of the
+// rounds alone in the mean, 38 of them longer by 3 % or more, 7 by 8 % (two runs of one tile differ by up to that).  us, rounds alone -> now (experts, rows,
+// N, K): 8, 1643, 1152, 1792 18.4 -> 13.6; 16, 5405, 2048, 1280 34.1 -> 35.7; the longest 8, 166, 4096, 3712 28.0 -> 35.7 (64 x 64 -> 32 x 128).
 enum GroupedTile { G_BIG, G_MID, G_WIDEK, G_MIDK, G_HALF, G_64, G_32, G_TILES };
 struct GroupedCost { int bm, bn, units, threads; double a, b, c, w, q; };
 constexpr GroupedCost GROUPED_COSTS[G_TILES] = {
@@ -49,13 +50,22 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
   if (K < 1024) return pick;
   const double mean = (double)rows / experts;  // rows of an expert, of a standard deviation of sqrt(mean)
   auto below = [](double x) { return 0.5 * std::erfc(-x * M_SQRT1_2); };
-  auto estimate = [&](GroupedTile t) {
+  auto per_unit = [&](GroupedTile t) {  // tiles per compute unit
     const GroupedCost& p = GROUPED_COSTS[t];
     const double m = mean / p.bm, dev = std::sqrt(mean) / p.bm;
     double per = mean > 8 ? 1 : 1 - std::exp(-mean);  // row tiles of an expert: of the k-th there is one where its rows pass k bm
-    if (dev > 0.5) per = m + 0.5;
-    else for (int k = 1; k < m + 4 * dev; ++k) per += below((m - k) / dev);
-    const double n0 = experts * per * div_up(N, p.bn) / 256, a = p.a, b = p.b * slabs;
+    if (dev > 0.5) {
+      per = m + 0.5;
+    } else {
+      const int sure = (int)std::max(0.0, m - 6 * dev);
+      per += sure;
+      for (int k = sure + 1; k < m + 4 * dev; ++k) per += below((m - k) / dev);
+    }
+    return experts * per * div_up(N, p.bn) / 256;
+  };
+  auto estimate = [&](GroupedTile t) {
+    const GroupedCost& p = GROUPED_COSTS[t];
+    const double n0 = per_unit(t), a = p.a, b = p.b * slabs;
     double sum = 0;
     for (const double u : {0.96, 0.99, 1.06}) {
       const double n = u * n0, y = p.w * std::ceil(n) + (1 - p.w) * n;
@@ -66,11 +76,20 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
     }
     return sum / 3 + 2;
   };
+  // With the weights from memory a chip half of whose units have no tile streams them slower than the estimate has it: 64 x 64 tiles, which fill it, are
+  // left for 128 x 128 ones only from 0.55 of those per unit on, or under 16 MB of weights (3 launches, 0.92 .. 1.10), for 64 x 128 ones only beyond one per unit.
+  // us, 64 x 64 | 128 x 128: 4, 239, 3712, 10240 37.7 | 53.7, 4, 229, 3968, 7936 29.6 | 39.1, 4, 558, 1792, 9344 44.5 | 51.2, 8, 672, 2048, 2688 16.8 | 19.2;
+  // of 40 launches of 72 .. 128 tiles 27 ran longer, by up to 42 %, and 13 shorter, by up to 14 %; of 28 of 144 and more all but two ran shorter.
+  const bool streams = experts * N * K >= (16ll << 20);
+  auto starved = [&](GroupedTile t) {
+    return pick == G_64 && ((t == G_MIDK && streams && per_unit(t) <= 0.55) || (t == G_HALF && per_unit(t) <= 1));
+  };
   GroupedTile other = pick;
   const double present = estimate(pick);
   double least = present;
   for (int i = G_BIG; i < G_TILES; ++i) {
     const GroupedTile t = (GroupedTile)i;
+    if (t == G_MID || starved(t)) continue;  // (G_MID: offered above; as `other` it lost 7 % over five launches)
     const double cost = estimate(t);
     if (cost < least && fits(t)) least = cost, other = t;
   }

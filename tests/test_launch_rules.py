@@ -37,3 +37,11 @@ def test_slices_where_one_pass_has_too_few_loads_in_flight(M, N, K, splits):
         assert plan[3] == splits and (splits > 1 or plan[1:3] == (64, 64))
         ws = kernels._workspace(M, N, K, "cpu", fp8)
         assert (0 if ws is None else ws.numel()) == (splits * M * N * 4 if splits > 1 else 0)
+
+
+@pytest.mark.parametrize("experts,rows,N,K,tile", [
+    (4, 239, 3712, 10240, (64, 64)), (8, 672, 2048, 2688, (64, 64)), (16, 557, 2048, 11520, (64, 64)),     # 116 .. 256 larger tiles
+    (8, 1643, 1152, 1792, (128, 128)), (4, 1807, 1280, 6272, (128, 128)), (16, 2479, 1280, 9600, (64, 128)),   # more of them, or whole rounds
+    (16, 5405, 2048, 1280, (128, 256))])
+def test_grouped_tiles_that_leave_half_the_chip_idle(experts, rows, N, K, tile):
+    assert kernels.grouped_gemm_plan(experts, rows, N, K)[1:3] == tile
