@@ -603,19 +603,23 @@ static int any_launch(const GemvArgs& g, hipStream_t st) {
   // (fused: 64 units of 512 elements with 16 waves, which the host's rule keeps to, 32 with 8, 16 with 4)
   constexpr int UPW = XT >= 0 ? 4 : 1;
   const int units = g.M * ((g.K + UNIT - 1) / UNIT);
-  if constexpr (MT == 1) {
+  // Launches that no rule leads to have no instance: per-token int8 with its quantizer leaves N > 8192 to the row kernel, and with fp32
+  // divisors stops at K = 1024
+  constexpr bool TOKEN_I8 = XT >= 0 && OP == FMSMO_OP_I8 && QUANT != QUANT_STATIC;
+  if constexpr (MT == 1 && !TOKEN_I8) {
     if (p.nw == 4 && units <= 4 * UPW) {
       hipLaunchKernelGGL((gemv_any_kernel<OP, 4, MT, XT, UPW, QUANT>), grid, dim3(256), 0, st, g, halves);
       return fmsmo_check_launch();
     }
   }
-  if constexpr (MT <= 2) {
+  if constexpr (MT <= 2 && QUANT != QUANT_TOKEN_F32S) {
     if (p.nw == 16 || (XT >= 0 && units > 8 * UPW)) {
       if (XT >= 0 && units > 16 * UPW) return FMSMO_ERR_UNSUPPORTED;
       hipLaunchKernelGGL((gemv_any_kernel<OP, 16, MT, XT, UPW, QUANT>), grid, dim3(1024), 0, st, g, halves);
       return fmsmo_check_launch();
     }
   }
+  if (XT >= 0 && units > 8 * UPW) return FMSMO_ERR_UNSUPPORTED;
   hipLaunchKernelGGL((gemv_any_kernel<OP, 8, MT, XT, UPW, QUANT>), grid, dim3(512), 0, st, g, halves);
   return fmsmo_check_launch();
 }
@@ -673,6 +677,7 @@ int fmsmo_gemv_any_fused(int op, int x_dtype, const GemvArgs& g, hipStream_t st)
 // 5376 9.8 -> 10.7; four 1024 5.8 -> 4.9, 3072 7.7 -> 7.8; six 512 5.7 -> 4.8, 1024 5.9 -> 6.1; eight 512 5.7 -> 4.8, 1024 5.9 -> 6.3; N = 12000: three
 // tokens 640 7.4 -> 8.8, 2048 9.5 -> 10.5.  e4m3 and int8 without SmoothQuant: the same or up to 25 % better.  fp32 divisors: 1 x 1024 5.8 -> 5.7,
 // 4 x 512 5.7 -> 5.7, 1 x 2048 6.4 -> 7.4.
+// (Those N = 4096 times had the product that streamed such K then; against the present ones and other N, see fmsmo_small_linear_better.)
 extern "C" int fmsmo_small_linear_ok(int64_t M, int64_t N, int64_t K, int smooth_f32) {
   if (M < 1 || N < 1 || K < 16 || K % 16 || N >= (1 << 30)) return 0;
   if (smooth_f32 ? fmsmo_decode_linear_f32s_ok(M, K) : fmsmo_decode_linear_ok(M, K)) return 1;
@@ -681,17 +686,6 @@ extern "C" int fmsmo_small_linear_ok(int64_t M, int64_t N, int64_t K, int smooth
   return N <= 8192 && (M <= 4 ? M * K <= 12288 : M <= 8 && K <= 512);
 }
 
-static int small_linear(int op, const void* x, int x_dtype, int64_t ldx, const void* smooth, int smooth_dtype, const void* w,
-                        int64_t ldw, const float* w_scale, int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
-// (Those N = 4096 times had the product that streamed such K then; against the present ones and other N, see fmsmo_small_linear_better.)
-                        void* y, int y_dtype, int64_t ldy, float* a_scale_out, float* clips, int64_t M, int64_t N, int64_t K,
-                        fmsmo_stream_t stream) {
-  if (!x || !w || !w_scale || !y) return FMSMO_ERR_NULL;
-  if (M <= 0 || N <= 0 || K <= 0 || (M > 1 && ldx < K) || ldw < K || ldy < N) return FMSMO_ERR_SHAPE;
-  if (w_scale_n != 1 && w_scale_n != N) return FMSMO_ERR_SHAPE;
-  if (x_dtype != FMSMO_F16 && x_dtype != FMSMO_BF16) return FMSMO_ERR_UNSUPPORTED;
-  const bool sf32 = smooth && smooth_dtype == FMSMO_F32;
-  if (smooth && !sf32 && smooth_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
 // Where one launch is the better one of those it takes: 1.  2: where a second launch and its buffers cost the host 3 us, the calls that keep
 // the GPU longer but still take less of its time than two calls take of the host's (int8, whose results are the same bits either way).  Weights from HBM,
 // us on the GPU, one launch | two calls:
@@ -722,6 +716,16 @@ extern "C" int fmsmo_small_linear_better(int fp8, int64_t M, int64_t N, int64_t 
   return M == 4 && fmsmo_gemv_stream_k(K) && K > 1024 ? 2 : 1;
 }
 
+static int small_linear(int op, const void* x, int x_dtype, int64_t ldx, const void* smooth, int smooth_dtype, const void* w,
+                        int64_t ldw, const float* w_scale, int64_t w_scale_n, const void* bias, int bias_dtype, int epilogue,
+                        void* y, int y_dtype, int64_t ldy, float* a_scale_out, float* clips, int64_t M, int64_t N, int64_t K,
+                        fmsmo_stream_t stream) {
+  if (!x || !w || !w_scale || !y) return FMSMO_ERR_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || (M > 1 && ldx < K) || ldw < K || ldy < N) return FMSMO_ERR_SHAPE;
+  if (w_scale_n != 1 && w_scale_n != N) return FMSMO_ERR_SHAPE;
+  if (x_dtype != FMSMO_F16 && x_dtype != FMSMO_BF16) return FMSMO_ERR_UNSUPPORTED;
+  const bool sf32 = smooth && smooth_dtype == FMSMO_F32;
+  if (smooth && !sf32 && smooth_dtype != x_dtype) return FMSMO_ERR_UNSUPPORTED;
   if (!fmsmo_small_linear_ok(M, N, K, sf32)) return FMSMO_ERR_UNSUPPORTED;
   if (N * ldw >= (fmsmo_decode_linear_ok(M, K) ? 1ll << 40 : 1ll << 31)) return FMSMO_ERR_UNSUPPORTED;
   if (y_dtype < 0 || y_dtype > 2 || (bias && (bias_dtype < 0 || bias_dtype > 2))) return FMSMO_ERR_UNSUPPORTED;

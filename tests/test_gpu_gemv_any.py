@@ -11,7 +11,8 @@ def gen(seed):
 
 
 # (M, N, K): tiles of 16 tokens and their edges, half groups and single rows of weights, one 16-byte chunk of K up to many turns of
-# the waves, the limits of the 4-, 8- and 16-wave launches (K = 768 | 784, 1024 | 1040; N = 4096 | 4097, 8192 | 8200)
+# the waves, the limits of the 8- and 16-wave launches (K = 1024 | 1040; N = 4096 | 4097; N = 8200 at K = 768 and 784 goes to the tiles;
+# the 4-wave launches are those of WIDE below)
 SHAPES = [(1, 1, 16), (2, 7, 48), (3, 8, 128), (5, 9, 144), (16, 23, 528), (4, 1000, 640), (15, 8200, 768), (15, 8200, 784),
           (16, 4097, 1024), (16, 4096, 1040), (3, 300, 4224), (12, 700, 6032), (9, 520, 2432), (6, 9000, 6144), (2, 260, 7808),
           (1, 2060, 3072), (2, 2060, 9216), (1, 2060, 9232), (17, 40, 272), (24, 4096, 1168), (32, 513, 4080), (25, 100, 2240), (33, 65, 1008),
@@ -260,3 +261,45 @@ def test_forward_of_a_static_linear(dev, M, K, bias, monkeypatch):
     assert torch.equal(m(x), general()) and torch.equal(m(x), general())
     m.qa_fmo_mo_qfunc = lambda t: torch.zeros(t.shape, dtype=torch.int8, device=t.device)
     assert torch.equal(m(x), general())
+
+
+# More than 8192 columns: the launches of four waves (K <= 768), of two blocks and one per compute unit with several row groups each, and
+# of gemv_short_kernel with two and four groups to a block (K <= 512; more than 16384 and 32768 columns)
+WIDE = [(1, 8200, 640), (1, 8201, 720), (2, 8200, 640), (2, 9001, 768), (2, 8200, 784), (5, 11003, 2816), (10, 16391, 2432), (16, 8999, 1664),
+        (1, 8193, 9232), (4, 8200, 9216), (1, 16400, 272), (16, 20001, 512), (7, 17001, 16), (1, 32790, 496)]
+
+
+@pytest.mark.parametrize("M,N,K", WIDE)
+def test_sums_over_many_columns(dev, M, N, K):
+    from fms_mo_amd import _lib as L
+    from fms_mo_amd import kernels as kn
+
+    for fp8 in (False, True):
+        assert kn.gemm_plan(M, N, K, fp8=fp8)[0] == L.PLAN_DECODE
+    test_int8_sums_are_exact(dev, M, N, K)
+    test_e4m3_sums(dev, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 8200, 640), (16, 8201, 768)])
+def test_the_entry_point_of_the_decode_products_takes_four_waves_too(dev, M, N, K):
+    """fmsmo_gemv_i8_dq has no tiles to go to."""
+    from fms_mo_amd import _lib as L
+
+    a = torch.randint(-128, 128, (M, K), generator=gen(1), dtype=torch.int8)
+    w = torch.randint(-128, 128, (N, K), generator=gen(2), dtype=torch.int8)
+    ad, wd, one, y = a.to(dev), w.to(dev), torch.ones(1, device=dev), torch.empty(M, N, device=dev)
+    L.call("fmsmo_gemv_i8_dq", ad.data_ptr(), K, wd.data_ptr(), K, one.data_ptr(), 1, one.data_ptr(), 1, None, 0, L.EPI_F32, y.data_ptr(), 2, N,
+           M, N, K, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(y.cpu().double(), a.double() @ w.double().t())  # below 2^24: exact
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8200, 640), (1, 8201, 720), (1, 9000, 16)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_e4m3_with_its_quantizer_over_many_columns(dev, M, N, K, dt):
+    test_e4m3_with_its_quantizer(dev, M, N, K, dt)
+
+
+@pytest.mark.parametrize("M,N,K", [(4, 9000, 640), (1, 8201, 400), (3, 8195, 768)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_int8_with_the_static_quantizer_over_many_columns(dev, M, N, K, dt):
+    test_int8_with_the_static_quantizer(dev, M, N, K, dt)
