@@ -209,6 +209,21 @@ static int64_t gemm_tail_columns(bool fp8, int64_t M, int64_t N, int64_t K) {
 extern "C" int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K) { return gemm_tail_columns(false, M, N, K); }
 extern "C" int64_t fmsmo_gemm_fp8_tail_columns(int64_t M, int64_t N, int64_t K) { return gemm_tail_columns(true, M, N, K); }
 
+static void cut_tile_shape(bool fp8, int64_t M, int64_t N, int64_t K, int* tile_m, int* tile_n) {
+  static const int bm[7] = {64, 128, 128, 128, 128, 256, 32}, bn[7] = {64, 64, 128, 192, 256, 256, 128};
+  const CutTile t = cut_k_tile(M, N, K, !fp8 ? MMA_I8 : K % 64 ? MMA_FP8_F16 : MMA_FP8);
+  *tile_m = bm[t];
+  *tile_n = bn[t];
+}
+extern "C" int fmsmo_gemm_cut_tile(int fp8, int64_t M, int64_t N, int64_t K, int* tile_m, int* tile_n) {
+  if (!tile_m || !tile_n) return FMSMO_ERR_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return FMSMO_ERR_SHAPE;
+  if (K % 16) return FMSMO_ERR_ALIGN;
+  *tile_m = *tile_n = 0;
+  if (K % 128 && !use_decode(M, N, K, fp8)) cut_tile_shape(fp8, M, N, K, tile_m, tile_n);
+  return FMSMO_OK;
+}
+
 static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
                      int* tile_n, int* splits) {
   if (!kernel || !tile_m || !tile_n || !splits) return FMSMO_ERR_NULL;
@@ -252,15 +267,12 @@ static int gemm_plan(bool fp8, int64_t M, int64_t N, int64_t K, int with_workspa
     return FMSMO_OK;
   }
   if (K % 64) {
-    *kernel = FMSMO_PLAN_GENERIC;
+    *kernel = FMSMO_PLAN_GENERIC;  // (its tile: fmsmo_gemm_cut_tile)
     return FMSMO_OK;
   }
   if (K % 128) {
-    const int bm[7] = {64, 128, 128, 128, 128, 256, 32}, bn[7] = {64, 64, 128, 192, 256, 256, 128};
-    const CutTile t = cut_k_tile(M, N, K, fp8 ? MMA_FP8 : MMA_I8);
     *kernel = FMSMO_PLAN_TILE_LDS_DMA;
-    *tile_m = bm[t];
-    *tile_n = bn[t];
+    cut_tile_shape(fp8, M, N, K, tile_m, tile_n);
     return FMSMO_OK;
   }
   const bool rs = use_register_staged(MMA_I8);

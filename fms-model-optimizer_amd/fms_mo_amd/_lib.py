@@ -95,6 +95,7 @@ SIGNATURES = {
     "fmsmo_debug_mfma_loop": [_I, _P, _L, _I, _P, _P, _P],
     "fmsmo_gemm_plan": [_L, _L, _L, _I, _P, _P, _P, _P],
     "fmsmo_gemm_fp8_plan": [_L, _L, _L, _I, _P, _P, _P, _P],
+    "fmsmo_gemm_cut_tile": [_I, _L, _L, _L, _P, _P],
     "fmsmo_grouped_gemm_plan": [_I, _L, _L, _L, _P, _P, _P, _P],
 }
 OTHER = {

@@ -298,6 +298,15 @@ def gemm_plan(M, N, K, with_workspace=False, fp8=False):
     return tuple(o.value for o in out)
 
 
+def gemm_cut_tile(M, N, K, fp8=False):
+    """(tile_m, tile_n) of one pass over K that is no multiple of 128 (see fmsmo_gemm_cut_tile)."""
+    import ctypes
+
+    out = [ctypes.c_int(0) for _ in range(2)]
+    L.call("fmsmo_gemm_cut_tile", int(fp8), M, N, K, *[ctypes.byref(o) for o in out])
+    return tuple(o.value for o in out)
+
+
 def grouped_gemm_plan(experts, rows, N, K):
     """(kernel, tile_m, tile_n, bytes of K per stage) grouped_gemm_i8_dq uses for a shape; no GPU needed."""
     import ctypes

@@ -405,12 +405,14 @@ enum fmsmo_plan_kernel {
   FMSMO_PLAN_TILE_REGISTER_STAGED = 1,  /* MFMA tiles, 128-byte K slabs staged through registers */
   FMSMO_PLAN_TILE_LDS_DMA = 2,          /* MFMA tiles, 64-byte K stages loaded straight into LDS */
   FMSMO_PLAN_GENERIC = 3                /* K % 64 != 0: MFMA tiles as in 2 with a last stage cut at K
-                                           (the tile shape is not reported) */
+                                           (fmsmo_gemm_cut_tile reports the tile shape) */
 };
 int fmsmo_gemm_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
                     int* tile_n, int* splits);
 int fmsmo_gemm_fp8_plan(int64_t M, int64_t N, int64_t K, int with_workspace, int* kernel, int* tile_m,
                         int* tile_n, int* splits);
+/* The tile of one pass where a last stage is cut at K (K % 128 != 0; 0 x 0 for other K and for the decode kernels).  Host-only. */
+int fmsmo_gemm_cut_tile(int fp8, int64_t M, int64_t N, int64_t K, int* tile_m, int* tile_n);
 /* Columns that the single-pass *_dq GEMMs cut off the end of N and run as a second GEMM behind
    the first (0: the GEMM runs whole; fmsmo_gemm_plan describes the first, main part).  int8, e4m3.  Host-only. */
 int64_t fmsmo_gemm_tail_columns(int64_t M, int64_t N, int64_t K);

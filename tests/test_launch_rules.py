@@ -45,3 +45,18 @@ def test_slices_where_one_pass_has_too_few_loads_in_flight(M, N, K, splits):
     (16, 5405, 2048, 1280, (128, 256))])
 def test_grouped_tiles_that_leave_half_the_chip_idle(experts, rows, N, K, tile):
     assert kernels.grouped_gemm_plan(experts, rows, N, K)[1:3] == tile
+
+
+@pytest.mark.parametrize("M,N,K,i8,e4m3", [   # the sizes of test_gpu_tiles.test_last_stage_cut_at_k, and of a few rows over many columns
+    (65, 33, 528, (64, 64), (64, 64)), (129, 4100, 1088, (64, 64), (64, 64)), (200, 5000, 976, (128, 64), (128, 64)),
+    (193, 4801, 1088, (128, 64), (128, 64)), (1025, 2050, 528, (128, 128), (128, 128)), (1000, 2060, 704, (128, 128), (128, 128)),
+    (1300, 6000, 528, (128, 192), (128, 192)), (1290, 3990, 704, (128, 192), (128, 192)), (1210, 5142, 848, (128, 256), (128, 256)),
+    (1234, 5861, 832, (128, 256), (128, 256)), (4000, 4090, 1040, (256, 256), (128, 256)), (4010, 4080, 1088, (256, 256), (128, 256)),
+    (5, 17001, 528, (32, 128), (32, 128)), (32, 16450, 1136, (32, 128), (32, 128)),
+    (1, 17001, 528, (0, 0), (0, 0)), (4010, 4080, 1024, (0, 0), (0, 0))])                # decode kernel; whole stages
+def test_tiles_whose_last_stage_is_cut_at_k(M, N, K, i8, e4m3):
+    for fp8, tile in ((False, i8), (True, e4m3)):
+        assert kernels.gemm_cut_tile(M, N, K, fp8) == tile
+        assert K % 64 or K % 128 == 0 or kernels.gemm_plan(M, N, K, fp8=fp8)[1:3] == tile
+    with pytest.raises(L.FmsMoHipError):
+        kernels.gemm_cut_tile(0, N, K)
