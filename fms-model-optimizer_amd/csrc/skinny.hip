@@ -747,12 +747,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(GemvArgs g, int ha
     constexpr bool LAST = decltype(last_tag)::value;
     const int en = min(row_lo + gi * 16 + (int)((threadIdx.x >> 4) & 15), g.N - 1);
     const float ws = g.w_scale ? g.w_scale[g.w_stride ? en : 0] : 1.f;
-    float bv = -0.f;  // no bias: adding -0 changes nothing, not even the sign of a zero product
-    if (g.bias) {
-      bv = g.bias_dtype == FMSMO_F16 ? f16_to_f32(((const u16*)g.bias)[en])
-           : g.bias_dtype == FMSMO_BF16 ? bf16_to_f32(((const u16*)g.bias)[en])
-                                        : ((const float*)g.bias)[en];
-    }
+    const float bv = gemv_bias(g, en);
     Acc4 acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = Acc4{0, 0, 0, 0};
@@ -813,23 +808,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(GemvArgs g, int ha
 #pragma unroll
       for (int w = 1; w < NW; ++w) sum += red[gi % NRED][w][e];
       const int n = row_lo + gi * 16 + ((e >> 4) & 15), m = (e >> 8) * 16 + (e & 15);
-      if (n < row_hi && m < g.M) {
-        float out;
-        if (g.epi == FMSMO_EPI_REF_F16) {
-          const float sc = round_to<FMSMO_F16>(__fmul_rn(as_e, ws_e));
-          out = __fadd_rn(__fmul_rn((float)sum, sc), bv_e);
-          if (g.y_dtype != FMSMO_F32) out = round_to<FMSMO_F16>(out);
-        } else if (g.epi == FMSMO_EPI_F32_MULADD) {
-          out = __fadd_rn(__fmul_rn((float)sum, __fmul_rn(as_e, ws_e)), bv_e);
-        } else {
-          out = __fmaf_rn((float)sum, __fmul_rn(as_e, ws_e), bv_e);
-        }
-        const int64_t idx = (int64_t)m * g.ldy + n;
-        if (g.epi == EPI_RAW_I32) ((int*)g.y)[idx] = (int)sum;
-        else if (g.y_dtype == FMSMO_F16) ((u16*)g.y)[idx] = f32_to_f16(out);
-        else if (g.y_dtype == FMSMO_BF16) ((u16*)g.y)[idx] = f32_to_bf16(out);
-        else ((float*)g.y)[idx] = out;
-      }
+      if (n < row_hi && m < g.M) gemv_store(g, m, n, sum, as_e, ws_e, bv_e);
     };
     if constexpr (MT == 1) {
       if (threadIdx.x < 256) finish(threadIdx.x, as, ws, bv);
@@ -991,27 +970,7 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvArgs g) {
     const int n = n0 + eu;
     if ((lane & (SHARE - 1)) == 0 && n < g.N && em < g.M) {
       const float as = g.a_scale ? g.a_scale[g.a_stride ? em : 0] : 1.f, ws = g.w_scale ? g.w_scale[g.w_stride ? n : 0] : 1.f;
-      float bv = -0.f;  // no bias: adding -0 changes nothing, not even the sign of a zero product
-      if (g.bias) {
-        bv = g.bias_dtype == FMSMO_F16 ? f16_to_f32(((const u16*)g.bias)[n])
-             : g.bias_dtype == FMSMO_BF16 ? bf16_to_f32(((const u16*)g.bias)[n])
-                                          : ((const float*)g.bias)[n];
-      }
-      float out;
-      if (g.epi == FMSMO_EPI_REF_F16) {
-        const float sc = round_to<FMSMO_F16>(__fmul_rn(as, ws));
-        out = __fadd_rn(__fmul_rn((float)sum, sc), bv);
-        if (g.y_dtype != FMSMO_F32) out = round_to<FMSMO_F16>(out);
-      } else if (g.epi == FMSMO_EPI_F32_MULADD) {
-        out = __fadd_rn(__fmul_rn((float)sum, __fmul_rn(as, ws)), bv);
-      } else {
-        out = __fmaf_rn((float)sum, __fmul_rn(as, ws), bv);
-      }
-      const int64_t idx = (int64_t)em * g.ldy + n;
-      if (g.epi == EPI_RAW_I32) ((int*)g.y)[idx] = (int)sum;
-      else if (g.y_dtype == FMSMO_F16) ((u16*)g.y)[idx] = f32_to_f16(out);
-      else if (g.y_dtype == FMSMO_BF16) ((u16*)g.y)[idx] = f32_to_bf16(out);
-      else ((float*)g.y)[idx] = out;
+      gemv_store(g, em, n, sum, as, ws, gemv_bias(g, n));
     }
   }
 }
