@@ -77,12 +77,14 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
     return sum / 3 + 2;
   };
   // With the weights from memory a chip half of whose units have no tile streams them slower than the estimate has it: 64 x 64 tiles, which fill it, are
-  // left for 128 x 128 ones only from 0.55 of those per unit on, or under 16 MB of weights (3 launches, 0.92 .. 1.10), for 64 x 128 ones only beyond one per unit.
-  // us, 64 x 64 | 128 x 128: 4, 239, 3712, 10240 37.7 | 53.7, 4, 229, 3968, 7936 29.6 | 39.1, 4, 558, 1792, 9344 44.5 | 51.2, 8, 672, 2048, 2688 16.8 | 19.2;
-  // of 40 launches of 72 .. 128 tiles 29 ran longer, by up to 42 %, and 11 shorter, by up to 14 %; of 28 of 144 and more all but two ran shorter.
+  // left for 128 x 128 ones only beyond half a tile per unit, or under 16 MB of weights (3 launches, 0.92 .. 1.10), for 64 x 128 ones only beyond one per unit.
+  // us, 64 x 64 | 128 x 128: 4, 239, 3712, 10240 37.7 | 53.7, 4, 229, 3968, 7936 29.6 | 39.1, 4, 558, 1792, 9344 44.5 | 51.2; of 40 launches of 72 .. 128 tiles 29
+  // ran longer, by up to 42 %, and 11 shorter, by up to 14 %; of 28 of 144 and more all but two ran shorter.  Two 64 x 128 tiles of a unit stream long rows
+  // against each other: 128 x 128 | 64 x 128, 16, 932, 4096, 7168 98.5 | 130.1, 8, 1073, 2432, 9472 61.0 | 76.3, 8, 1182, 2176, 3712 31.1 | 33.0, 4, 541, 4864, 2688 38.4 | 26.5.
   const bool streams = experts * N * K >= (16ll << 20);
   auto starved = [&](GroupedTile t) {
-    return pick == G_64 && ((t == G_MIDK && streams && per_unit(t) <= 0.55) || (t == G_HALF && per_unit(t) <= 1));
+    if (pick == G_MIDK) return t == G_HALF && K > 3584;
+    return pick == G_64 && ((t == G_MIDK && streams && per_unit(t) <= 0.5) || (t == G_HALF && per_unit(t) <= 1));
   };
   GroupedTile other = pick;
   const double present = estimate(pick);
