@@ -566,7 +566,7 @@ static AnyPlan any_plan(int64_t M, int64_t N, int64_t K) {
 
 // Up to 16 tokens: every K that skinny.hip has no instance for, except short rows over more columns than one round of blocks takes, where tiles of
 // 64 x 64 or 32 x 128 with their deeper loads win.  us with the tokens' quantizer, weights from HBM, tiles | this kernel:
-//   up to 16384 columns: int8 2 x 9216 x 640 8.1 | 7.4, 4 x 14336 x 1152 10.4 | 10.3, 5 x 14336 x 1536 11.9 | 10.9, 5 x 11008 x 2816 16.1 | 13.7 (e4m3 16.5 | 13.6),
+//   up to 16384 columns: int8 2 x 9216 x 640 8.1 | 7.4, 5 x 9216 x 768 (e4m3) 8.8 | 8.1, 4 x 14336 x 1152 10.4 | 10.3, 5 x 14336 x 1536 11.9 | 10.9, 5 x 11008 x 2816 16.1 | 13.7 (e4m3 16.5 | 13.6),
 //     16 x 9216 x 2816 14.9 | 14.7; K % 128 != 0 10 x 9216 x 3600 18.2 | 18.5, 16 x 9216 x 3600 18.3 | 20.2
 //   more: 5 x 24576 x 1536 14.0 | 14.4, 10 x 24576 x 2176 16.9 | 18.6, 10 x 24576 x 2816 19.8 | 20.2, 10 x 18944 x 4480 (e4m3) 26.4 | 25.9, 16 x 24576 x 3584 23.8 | 26.6;
 //     K % 128 != 0 5 x 18944 x 1616 16.4 | 14.9, 10 x 18944 x 3600 28.4 | 26.4, 16 x 18944 x 1616 16.8 | 16.8
@@ -583,7 +583,7 @@ bool fmsmo_gemv_any_ok(int64_t M, int64_t N, int64_t K, bool fp8) {
   if (M <= 16) {
     if (M == 1 || N <= (K <= 512 ? 24576 : 8192) || fmsmo_gemv_stream_k(K)) return true;
     if (M > 10 && (K % 128 || N > 16384)) return K > 4608;
-    return K > (N <= 16384 ? (M == 2 ? 512 : 1024) : K % 128 ? 1024 : 2304);
+    return K > (N <= 16384 ? (M <= 10 ? 512 : 1024) : K % 128 ? 1024 : 2304);
   }
   if (N > 4096) return false;
   if (M <= 32) return K <= (M > 24 ? 4096 : fp8 ? 6144 : 8192);
@@ -697,12 +697,12 @@ extern "C" int fmsmo_small_linear_ok(int64_t M, int64_t N, int64_t K, int smooth
 //     5376 15.1 | 13.8, 6144 x 4224 12.1 | 11.9, 1024 x 6144 8.7 | 7.8
 //   three, int8: 6144 x 3072 11.5 | 10.4, 6144 x 2304 10.2 | 9.6, 6144 x 1152 8.1 | 7.5; four: 6144 x 3072 12.9 | 10.7, 6144 x 1152 8.2 | 7.4, 6144 x 1024 6.8 | 6.9, 2048 x
 //     2048 6.6 | 5.9, 2048 x 2304 7.1 | 7.2; e4m3 6144 x 3072 11.5 | 9.7, 6144 x 2304 9.9 | 9.2; six, int8: 6144 x 256 6.2 | 5.0, 4096 x 256 4.7 | 4.8
-//   fp32 divisors: 1 x 6144 x 640 7.1 | 6.7, 2 x 4096 x 512 5.4 | 4.9, 2 x 6144 x 512 7.1 | 5.6, 2 x 6144 x 1024 7.3 | 7.1, 6 x 2048 x 256 5.9 | 4.7
+//   fp32 divisors: 1 x 6793 x 512 7.0 | 5.5, 1 x 6144 x 640 7.1 | 6.7, 2 x 4096 x 512 5.4 | 4.9, 2 x 6144 x 512 7.1 | 5.6, 2 x 6144 x 1024 7.3 | 7.1, 6 x 2048 x 256 5.9 | 4.7
 // (eager, weights in cache: int8 4 x 2048 x 1024 6.0 | 9.3, 6 x 256 x 6144 6.2 | 9.4 - 10.4, 1 x 11264 x 640 9.1 | 9.2 - 10.0; e4m3 1 x 4992 x 7168 10.9 | 9.6 - 10.0)
 extern "C" int fmsmo_small_linear_better(int fp8, int64_t M, int64_t N, int64_t K, int smooth_f32) {
   if (!fmsmo_small_linear_ok(M, N, K, smooth_f32)) return 0;
   if (smooth_f32 ? fmsmo_decode_linear_f32s_ok(M, K) : fmsmo_decode_linear_ok(M, K)) return 1;
-  if (smooth_f32) return M == 1 || (K > 512 && (M == 2 || N <= 4096)) ? 1 : 2;
+  if (smooth_f32) return K > 512 && (M <= 2 || N <= 4096) ? 1 : 2;
   if (fp8) {
     if (M == 1) return K > 8192 ? N > 2048 : N <= 4096 || K <= (N > 8192 ? 6144 : 4096);
     return N <= 4096 || K <= (M == 2 ? 4608 : M == 3 ? 4096 : 2304);

@@ -11,7 +11,7 @@ from fms_mo_amd import kernels
     (0, 2, 6144, 4224, 0, 0), (0, 2, 6144, 3072, 0, 2), (0, 2, 4096, 4224, 0, 1), (0, 2, 1024, 6144, 0, 2), (1, 2, 6144, 4224, 0, 1),
     (1, 2, 6144, 6144, 0, 0), (0, 3, 6144, 3072, 0, 0), (1, 3, 6144, 3072, 0, 1), (0, 4, 6144, 1152, 0, 2), (0, 4, 4096, 3072, 0, 1),
     (0, 4, 4096, 2048, 0, 2), (1, 4, 6144, 3072, 0, 0), (0, 6, 6144, 256, 0, 2), (0, 6, 4096, 256, 0, 1), (1, 8, 8192, 512, 0, 1),
-    (0, 2, 6144, 512, 1, 2), (0, 2, 6144, 1024, 1, 1), (0, 1, 6144, 1024, 1, 1), (0, 6, 2048, 256, 1, 2),
+    (0, 2, 6144, 512, 1, 2), (0, 2, 6144, 1024, 1, 1), (0, 1, 6144, 1024, 1, 1), (0, 1, 6144, 512, 1, 2), (0, 6, 2048, 256, 1, 2),
     (0, 1, 28672, 4096, 1, 1), (0, 3, 4096, 14336, 0, 1), (1, 1, 8192, 8192, 0, 1),   # shapes of the streaming kernel and of whole rows
     (0, 9, 64, 512, 0, 0), (0, 1, 4096, 16400, 0, 0), (0, 1, 4096, 5377, 0, 0)])      # not taken at all
 def test_one_launch_only_where_it_is_the_better_one(fp8, M, N, K, smooth_f32, better):
@@ -20,7 +20,7 @@ def test_one_launch_only_where_it_is_the_better_one(fp8, M, N, K, smooth_f32, be
 
 @pytest.mark.parametrize("M,N,K,decode", [
     (5, 11008, 2816, True), (3, 10240, 2560, True), (16, 9088, 1664, True), (2, 12288, 640, True), (13, 8320, 640, False),
-    (4, 14336, 1024 - 128, False), (10, 24576, 2432, True), (10, 24576, 2176, False), (12, 24576, 2432, False), (16, 16384, 2816, True),
+    (12, 14336, 896, False), (5, 9216, 768, True), (10, 24576, 2432, True), (10, 24576, 2176, False), (12, 24576, 2432, False), (16, 16384, 2816, True),
     (5, 18944, 1616, True), (16, 9216, 3600, False), (10, 9216, 3600, True), (1, 28672, 528, True), (16, 24576, 5248, True)])
 def test_a_few_tokens_over_many_columns(M, N, K, decode):
     for fp8 in (False, True):
@@ -40,7 +40,8 @@ def test_slices_where_one_pass_has_too_few_loads_in_flight(M, N, K, splits):
 
 
 @pytest.mark.parametrize("experts,rows,N,K,tile", [
-    (4, 239, 3712, 10240, (64, 64)), (8, 672, 2048, 2688, (64, 64)), (16, 557, 2048, 11520, (64, 64)),     # 116 .. 256 larger tiles
+    (4, 239, 3712, 10240, (64, 64)), (4, 558, 1792, 9344, (64, 64)), (16, 557, 2048, 11520, (64, 64)),     # 112 .. 256 larger tiles
+    (16, 932, 4096, 7168, (128, 128)), (4, 541, 4864, 2688, (64, 128)),                                    # long rows, short ones
     (8, 1643, 1152, 1792, (128, 128)), (4, 1807, 1280, 6272, (128, 128)), (16, 2479, 1280, 9600, (64, 128)),   # more of them, or whole rounds
     (16, 5405, 2048, 1280, (128, 256))])
 def test_grouped_tiles_that_leave_half_the_chip_idle(experts, rows, N, K, tile):
