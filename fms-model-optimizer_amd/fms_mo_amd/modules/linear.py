@@ -840,12 +840,15 @@ class QLinearINT8Deploy(nn.Linear):
         stamp = _stamp(ws)
         kept = getattr(self, "_ws_kept", None)
         if not kept or kept[0] != stamp:
-            with torch.inference_mode(False), torch.no_grad():
-                f = ws.detach().float().reshape(-1).contiguous()
+            if torch.is_inference_mode_enabled():   # (a copy made in it could not be written to outside)
+                with torch.inference_mode(False):
+                    return self._w_scale_f32()
+            f = ws.detach().float().reshape(-1).contiguous()
+            if f.data_ptr() != ws.data_ptr():
                 if f.is_cuda and torch.cuda.is_current_stream_capturing():
                     return f    # (part of the graph: it holds nothing before a replay)
                 own = kept[1] if kept and kept[1].data_ptr() != kept[2].data_ptr() else None
-                if own is not None and f.data_ptr() != ws.data_ptr() and own.shape == f.shape and own.device == f.device:
+                if own is not None and own.shape == f.shape and own.device == f.device:
                     f = own.copy_(f)
                 # complete before another stream is given it (the first forward waits in _smoothq_active, right behind)
                 if f.is_cuda and getattr(self, "_sq_kept", None):
