@@ -548,18 +548,24 @@ bool fmsmo_gemv_stream_k(int64_t K);
 // Waves per block and blocks of a launch.  us, int8, waves x most blocks 16 x 256 | 8 x 256 | 8 x 512 | 4 x 1024:
 //   up to 512 halves of row groups (N = 4096) a group per block, 16 waves, 8 where K has no more than that many steps:
 //     1 x 3000: K = 1024 3.7 | 3.4, 2048 3.9 | 4.1, 7168 6.5 | 7.7; 16 x 3000: K = 2048 4.1 | 4.5, 8192 8.7 | 8.9
-//   more of them, several groups per block, whose ends two blocks per compute unit cover for each other:
-//     4 x 6144: K = 2048 5.4 | - | 5.1, 8192 11.4 | - | 10.7; 1 x 20000: K = 1024 9.4 | 9.1 | 7.2 | 7.8, 3072 15.1 | 17.1 |
-//     13.4 | 15.2; 2 x 26752 x 640 (e4m3) 11.8 | 11.1 | 8.0 | 7.5
-//   and one again on long rows: 1 x 20000 x 7168 25.5 | - | 26.0, 8192 27.5 | - | 29.1
+//   up to 1024 halves, several groups per block, whose ends two blocks per compute unit cover for each other:
+//     4 x 6144: K = 2048 5.4 | - | 5.1, 8192 11.4 | - | 10.7
+//   more of them a group per block again, whatever their number: a wave has one step of loads in flight, and up to four blocks of eight waves fit a unit.
+//     Weights from HBM, at most 512 blocks (K = 768: 1024) | a group per block: 4 x 9216: K = 768 5.7 | 4.9, 1280 7.1 | 5.9, 2816 10.3 | 8.4; 10 x 11776: 1536 7.9 | 6.6,
+//     2304 9.8 | 8.1; e4m3 2 x 9216 x 2304 9.7 | 7.7; 4 x 28672: K = 2560 0.93 of the time, 5376 0.90
+//     With the quantizer inside, which every block repeats, as before (static 3 x 16384 x 864 7.1 | 8.7, e4m3 1 x 24576 x 896 8.3 | 10.0).
+//   But on long rows, and from eleven tokens on beyond K = 2560, the activations that every block reads again weigh more: 4 x 9000 x 10880 1.08 of the
+//   time, 16 x 13000 x 5376 1.04; long rows as up to 512 halves: 1 x 20000 x 7168 25.5 | - | 26.0, 8192 27.5 | - | 29.1
 struct AnyPlan {
   int nw, blocks;
 };
-static AnyPlan any_plan(int64_t M, int64_t N, int64_t K) {
+static AnyPlan any_plan(int64_t M, int64_t N, int64_t K, bool fused) {
   const int64_t steps = (K + 127) / 128, halves = (N + 7) / 8;
   const bool wide = steps > 8 && M <= 32;  // (four tiles of tokens have no LDS for 16 waves' sums)
   if (halves <= 512) return {wide ? 16 : 8, 256};
-  if (M <= 16 && steps <= 6 && halves > 1024) return {4, 1024};
+  // (65536 blocks: a launch holds less than 2^32 threads)
+  if (!fused && halves > 1024 && K < 6144 && M <= (K <= 2560 ? 16 : 10)) return {steps <= 6 ? 4 : 8, (int)std::min<int64_t>((halves + 1) / 2, 65536)};
+  if (fused && M <= 16 && steps <= 6 && halves > 1024) return {4, 1024};
   if (wide && M <= 16 && K >= 6144 && halves > 1024) return {16, 256};
   return {8, 512};
 }
@@ -597,7 +603,7 @@ static bool any_offsets_ok(const GemvArgs& g) {
 
 template <int OP, int MT, int XT = -1, int QUANT = QUANT_TOKEN>
 static int any_launch(const GemvArgs& g, hipStream_t st) {
-  const AnyPlan p = any_plan(g.M, g.N, g.K);
+  const AnyPlan p = any_plan(g.M, g.N, g.K, XT >= 0);
   const int halves = (g.N + 7) / 8;
   const dim3 grid((unsigned)std::min(halves, p.blocks));
   // (fused: 64 units of 512 elements with 16 waves, which the host's rule keeps to, 32 with 8, 16 with 4)

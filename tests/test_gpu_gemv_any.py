@@ -303,3 +303,17 @@ def test_e4m3_with_its_quantizer_over_many_columns(dev, M, N, K, dt):
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_int8_with_the_static_quantizer_over_many_columns(dev, M, N, K, dt):
     test_int8_with_the_static_quantizer(dev, M, N, K, dt)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 8200, 640), (10, 9001, 2688), (10, 8207, 6016), (11, 8201, 2560), (11, 8201, 2688), (3, 1048605, 640)])
+def test_a_group_of_rows_per_block(dev, M, N, K):
+    """More than 8192 columns: a block per 16 of them, at the ends of the range, up to 65536 blocks, which own two groups in the last one's case."""
+    from fms_mo_amd import _lib as L
+
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    a = torch.randint(-64, 64, (M, K), generator=g, dtype=torch.int8, device=dev)
+    w = torch.randint(-32, 32, (N, K), generator=g, dtype=torch.int8, device=dev)
+    one, y = torch.ones(1, device=dev), torch.empty(M, N, device=dev)
+    L.call("fmsmo_gemv_i8_dq", a.data_ptr(), K, w.data_ptr(), K, one.data_ptr(), 1, one.data_ptr(), 1, None, 0, L.EPI_F32, y.data_ptr(), 2, N,
+           M, N, K, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(y.double(), a.double() @ w.double().t())  # sums below 2^24: exact
