@@ -16,9 +16,9 @@ struct TileHalfK { static constexpr int BM = 64, BN = 128, BK = 128, NST = 3, WG
 // max(1, w ceil(n) + (1 - w) n) rounds of a + b s, of which a chip filled to n < 1 saves c (1 - n); two to a unit, the second one slows the first's
 // stages by 1 + q; the mean over n 4 % and 1 % less and 6 % more, for the step at whole rounds.
 // Parameters fitted to two thirds of 960 launches with every tile timed (4, 8, 16 experts, 128 .. 8192 rows, K and N of hidden sizes 1024 .. 4096 and
-// intermediate ones to 14336), weights mostly in the last-level cache.  With weights from memory, over 1200 launches of those ranges: 0.927 of the time of the
-// rounds alone in the mean, 38 of them longer by 3 % or more, 7 by 8 % (two runs of one tile differ by up to that).  us, rounds alone -> now (experts, rows,
-// N, K): 8, 1643, 1152, 1792 18.4 -> 13.6; 16, 5405, 2048, 1280 34.1 -> 35.7; the longest 8, 166, 4096, 3712 28.0 -> 35.7 (64 x 64 -> 32 x 128).
+// intermediate ones to 14336), weights mostly in the last-level cache.  With weights from memory, over 1500 launches of those ranges: 0.917 of the time of the
+// rounds alone in the mean, 11 of them longer by 8 % or more, 6 of those on the same tile (two runs of one differ by up to that).  us, rounds alone -> now (experts, rows,
+// N, K): 8, 1643, 1152, 1792 18.4 -> 13.6; 16, 5405, 2048, 1280 34.1 -> 35.7; the longest 4, 552, 5120, 9984 64.3 -> 85.3 (128 x 128 -> 128 x 256).
 enum GroupedTile { G_BIG, G_MID, G_WIDEK, G_MIDK, G_HALF, G_64, G_32, G_TILES };
 struct GroupedCost { int bm, bn, units, threads; double a, b, c, w, q; };
 constexpr GroupedCost GROUPED_COSTS[G_TILES] = {
@@ -81,9 +81,12 @@ GroupedTile pick_grouped_tile(int64_t experts, int64_t rows, int64_t N, int64_t 
   // us, 64 x 64 | 128 x 128: 4, 239, 3712, 10240 37.7 | 53.7, 4, 229, 3968, 7936 29.6 | 39.1, 4, 558, 1792, 9344 44.5 | 51.2; of 40 launches of 72 .. 128 tiles 29
   // ran longer, by up to 42 %, and 11 shorter, by up to 14 %; of 28 of 144 and more all but two ran shorter.  Two 64 x 128 tiles of a unit stream long rows
   // against each other: 128 x 128 | 64 x 128, 16, 932, 4096, 7168 98.5 | 130.1, 8, 1073, 2432, 9472 61.0 | 76.3, 8, 1182, 2176, 3712 31.1 | 33.0, 4, 541, 4864, 2688 38.4 | 26.5.
+  // For 32 x 128 tiles they come with a third tile on a part of the units, the more so where an expert's rows fit one tile of either: 32 x 128 | 64 x 128, 16, 406, 5760,
+  // 4864 85.3 | 101.5, 16, 386, 4352, 6656 101 | 115, 16, 798, 4224, 6528 1.06 of the time; two to a unit, or more columns, the other way (8, 398, 7424, 5376 0.79, 16, 622, 5632, 5120 0.86).
   const bool streams = experts * N * K >= (16ll << 20);
   auto starved = [&](GroupedTile t) {
     if (pick == G_MIDK) return t == G_HALF && K > 3584;
+    if (pick == G_32) return t == G_HALF && streams && per_unit(t) > 2 && (per_unit(t) <= 2.25 || (mean <= 32 && per_unit(t) < 3));
     return pick == G_64 && ((t == G_MIDK && streams && per_unit(t) <= 0.5) || (t == G_HALF && per_unit(t) <= 1));
   };
   GroupedTile other = pick;

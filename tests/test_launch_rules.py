@@ -61,3 +61,10 @@ def test_tiles_whose_last_stage_is_cut_at_k(M, N, K, i8, e4m3):
         assert K % 64 or K % 128 == 0 or kernels.gemm_plan(M, N, K, fp8=fp8)[1:3] == tile
     with pytest.raises(L.FmsMoHipError):
         kernels.gemm_cut_tile(0, N, K)
+
+
+@pytest.mark.parametrize("experts,rows,N,K,tile", [
+    (16, 406, 5760, 4864, (32, 128)), (16, 386, 4352, 6656, (32, 128)), (16, 590, 4480, 6528, (32, 128)),   # a third tile on a part of the units
+    (8, 398, 7424, 5376, (64, 128)), (16, 469, 7168, 4096, (64, 128)), (16, 622, 5632, 5120, (64, 128))])   # two at most, or more rows or columns
+def test_grouped_tiles_of_experts_with_few_rows(experts, rows, N, K, tile):
+    assert kernels.grouped_gemm_plan(experts, rows, N, K)[1:3] == tile
