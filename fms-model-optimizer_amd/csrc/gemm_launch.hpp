@@ -540,7 +540,11 @@ inline SplitPlan plan_split_k(int64_t M, int64_t N, int64_t K, int64_t limit = 0
     // N = 3072, K = 8208 26.3 -> 14.4; M = 200, N = 1500, K = 11216 36.7 -> 16.7.  From a quarter of a
     // round of tiles on these shapes ask for no workspace, nor up to where one pass of 64 x 64 tiles takes as long: int8 177 x 301 x 3936
     // 10.9 against 11.0, 169 x 768 x 2848 10.1 against 8.9; e4m3, K % 64 != 0, 68 x 474 x 3424 11.6 against 14.5.)
-    if (tiles_t < 64 && K > (fp8 && K % 64 ? 2816 : 3584)) cut_slices(p, M, N, K, (int)std::min<int64_t>(256 / tiles_t, room));
+    // With the weights from HBM up to 128 rows over more than 24 such tiles begin earlier (int8, one pass | slices: 41 x 3467 x 3120 18.8 | 15.8, 44 x 1673 x 3424 17.2 | 13.9,
+    // 123 x 2739 x 3504 21.0 | 19.0, up to 64 rows over more than 36 47 x 2369 x 2960 16.7 | 15.1, 56 x 3671 x 2544 17.8 | 16.7; 35 x 3278 x 2448 1.04; in one pass 47 x
+    // 2090 x 2704 0.91 of the time, 109 x 866 x 3264 0.83).
+    const int64_t above = fp8 ? (K % 64 ? 2816 : 3584) : M <= 64 && tiles_t > 36 ? 2496 : M <= 128 && tiles_t > 24 ? 3072 : 3584;
+    if (tiles_t < 64 && K > above) cut_slices(p, M, N, K, (int)std::min<int64_t>(256 / tiles_t, room));
     return p;
   }
   // Long reductions under a few hundred rows: 256 x 128 tiles of the register-staged kernel carry

@@ -68,3 +68,12 @@ def test_tiles_whose_last_stage_is_cut_at_k(M, N, K, i8, e4m3):
     (8, 398, 7424, 5376, (64, 128)), (16, 469, 7168, 4096, (64, 128)), (16, 622, 5632, 5120, (64, 128))])   # two at most, or more rows or columns
 def test_grouped_tiles_of_experts_with_few_rows(experts, rows, N, K, tile):
     assert kernels.grouped_gemm_plan(experts, rows, N, K)[1:3] == tile
+
+
+@pytest.mark.parametrize("M,N,K,splits", [
+    (41, 3467, 3120, 3), (44, 1673, 3424, 3), (123, 2739, 3504, 3), (109, 866, 3264, 1), (226, 1395, 3424, 1), (47, 2369, 2960, 2), (56, 3671, 2544, 2), (35, 3278, 2448, 1),
+    (47, 2090, 2704, 1), (128, 1601, 3600, 3)])
+def test_slices_of_int8_reductions_that_are_cut_at_k(M, N, K, splits):
+    assert kernels.gemm_plan(M, N, K, with_workspace=True)[3] == splits
+    ws = kernels._workspace(M, N, K, "cpu", False)
+    assert (0 if ws is None else ws.numel()) == (splits * M * N * 4 if splits > 1 else 0)
